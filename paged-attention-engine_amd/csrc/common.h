@@ -54,16 +54,34 @@ __device__ __forceinline__ float act_of(float z, int kind) {
   return z / (1.0f + expf(-z));
 }
 
+// Reductions over a wavefront by a butterfly: every lane meets the lane 32, 16, 8, 4, 2 and 1 away, in this
+// order, and all lanes end with the same value.  No step goes through LDS (a shuffle does, about 100 clocks
+// each): the halves and the rows of 16 lanes change places by v_permlane32_swap and v_permlane16_swap; within a
+// row the lanes are rotated by 8, 4, 2 and 1, which brings the partner or a lane that by then holds the
+// partner's value.
+template <int ROTATE>
+__device__ __forceinline__ float row_rotated(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + ROTATE, 0xf, 0xf, true));
+}
+
+template <typename Op>
+__device__ __forceinline__ float wave_reduce(float v, Op op) {
+  const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = op(__uint_as_float(halves[0]), __uint_as_float(halves[1]));
+  const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = op(__uint_as_float(rows[0]), __uint_as_float(rows[1]));
+  v = op(v, row_rotated<8>(v));
+  v = op(v, row_rotated<4>(v));
+  v = op(v, row_rotated<2>(v));
+  return op(v, row_rotated<1>(v));
+}
+
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int off = PAE_WAVE / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, PAE_WAVE);
-  return v;
+  return wave_reduce(v, [](float a, float b) { return a + b; });
 }
 
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int off = PAE_WAVE / 2; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, PAE_WAVE));
-  return v;
+  return wave_reduce(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
 // Sum over a block of `NW` wavefronts in a fixed order: lanes by butterfly,
