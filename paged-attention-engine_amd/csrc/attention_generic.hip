@@ -1,6 +1,8 @@
-// Causal attention over the paged cache, one wavefront per (token, query head).
+// Causal attention over the paged cache in float32 arithmetic, two kernels that compute the same bits: one wavefront per
+// (token, query head) for any size, and a workgroup for the query heads of one key/value head and
+// a few tokens, which brings the keys and values to LDS once for all of them (below).
 //
-// This is the kernel every size goes through in float32 and the one bfloat16
+// These are the kernels every size goes through in float32 and the ones bfloat16
 // falls back to when the matrix-core kernels do not take a shape.  A step's
 // tokens are flat: token t belongs to sequence tok_seq[t] and stands at
 // positions[t]; its keys are the cache slots of positions start..pos of that
@@ -119,6 +121,307 @@ __global__ void paged_attention_generic_kernel(
   }
 }
 
+// The same for float32 rows that can be read four numbers at a time: a workgroup of four wavefronts takes up to 16 (token,
+// query head) rows that share a key/value head, and walks the chunks of 64 keys that any of them
+// sees.  A chunk's keys and values come to LDS once, by 16-byte loads, the next chunk's on their way
+// meanwhile; a wavefront computes up to four rows together, lane = key for the scores, lane = feature for
+// the sums, so that a key or value read from LDS serves four rows.  Every row does the operations of the
+// kernel above in its order and over its own keys only: the bits are the same, and a row never touches a
+// key it does not see.
+//
+// What bound the kernel above: every lane read its own key row number by number (64 rows of 512 bytes, a
+// load instruction per number), and every (token, head) read the keys and values again.  Measured, 12 heads over 2
+// of 128, float32: three prompts of 601 tokens in all 700 -> 68 us, a token each behind them 55 -> 37 us.  What is
+// left is the chain of a workgroup's chunks, 6 us each.  Loads under conditions (keys beside those in sight) had
+// the compiler wait for each in turn: 140 us for the prompts.  Eight wavefronts of two rows against four of four: 43
+// against 69 us a launch.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+#define PAE_ROWS_WAVES 8
+#define PAE_ROWS_EACH 2
+#define PAE_ROWS_MOST (PAE_ROWS_WAVES * PAE_ROWS_EACH)
+
+template <int MAXD>  // keys and values at most 64 * MAXD wide
+__global__ __launch_bounds__(PAE_WAVE * PAE_ROWS_WAVES) void paged_attention_rows_kernel(
+    float* __restrict__ out, int64_t out_stride, const float* __restrict__ q, int64_t q_stride,
+    const float* __restrict__ k_cache, const float* __restrict__ v_cache, const int* __restrict__ positions,
+    const int* __restrict__ tok_seq, const int* __restrict__ block_tables, int max_blocks, int bs, int num_tokens,
+    int nh, int nkv, int hd, int vd, float scale, int window, float cap, const float* __restrict__ sinks,
+    int chunked, const float* __restrict__ slopes, const float* __restrict__ gate, int64_t gate_stride,
+    int gate_per_head, int toks, int heads_each) {
+  constexpr int FOURS = 16 * MAXD / PAE_ROWS_WAVES;  // that a thread brings of a chunk's keys, and of its values
+  extern __shared__ float lds[];
+  const int kst = hd + 4, vst = vd + 4;  // row strides that spread a quad's reads and writes over the banks
+  float* k_lds = lds;                    // [64 keys][kst]
+  float* v_lds = lds + PAE_WAVE * kst;   // [64 keys][vst]
+  float* p_lds = v_lds + PAE_WAVE * vst; // [wavefront][row][64]
+  float* q_lds = p_lds + PAE_ROWS_MOST * PAE_WAVE;  // [row][hd]
+  const int tid = threadIdx.x, lane = tid % PAE_WAVE;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / PAE_WAVE);
+  const int g = nh / nkv;
+  const int parts = (g + heads_each - 1) / heads_each;
+  const int kvh = blockIdx.y / parts, head0 = (blockIdx.y % parts) * heads_each;
+  const int heads = min(heads_each, g - head0);
+  const int t0 = blockIdx.x * toks;
+  p_lds += wave * PAE_ROWS_EACH * PAE_WAVE;
+
+  // the wavefront's rows: row = token of the tile * heads + head
+  int tok[PAE_ROWS_EACH], head[PAE_ROWS_EACH], pos[PAE_ROWS_EACH], start[PAE_ROWS_EACH];
+  float acc[PAE_ROWS_EACH][MAXD], m[PAE_ROWS_EACH], l[PAE_ROWS_EACH];
+  bool live[PAE_ROWS_EACH];
+#pragma unroll
+  for (int i = 0; i < PAE_ROWS_EACH; ++i) {
+    const int row = wave + i * PAE_ROWS_WAVES;
+    live[i] = row < toks * heads && t0 + row / heads < num_tokens;
+    tok[i] = live[i] ? t0 + row / heads : t0;
+    head[i] = kvh * g + head0 + row % heads;
+    pos[i] = __builtin_amdgcn_readfirstlane(positions[tok[i]]);
+    start[i] = window <= 0 ? 0 : (chunked ? pos[i] - pos[i] % window : (pos[i] - window + 1 > 0 ? pos[i] - window + 1 : 0));
+    m[i] = -INFINITY;
+    l[i] = 0.f;
+#pragma unroll
+    for (int d = 0; d < MAXD; ++d) acc[i][d] = 0.f;
+  }
+
+  // the tile's queries, and which fours of a chunk a thread brings
+  for (int c = tid; c < toks * heads * (hd / 4); c += PAE_WAVE * PAE_ROWS_WAVES) {
+    const int row = c / (hd / 4), d = (c % (hd / 4)) * 4;
+    const int t = min(t0 + row / heads, num_tokens - 1);
+    const float* src = q + (int64_t)t * q_stride + (int64_t)(kvh * g + head0 + row % heads) * hd + d;
+    *(float4*)(q_lds + row * hd + d) = make_float4(src[0], src[1], src[2], src[3]);
+  }
+  // (threads without a four of their own bring the last one again)
+  const int span = min(bs, PAE_WAVE);  // keys of a chunk that lie in one page; a power of two
+  int k_key[FOURS], k_dim[FOURS], v_key[FOURS], v_dim[FOURS];
+#pragma unroll
+  for (int u = 0; u < FOURS; ++u) {
+    const int c = tid + u * PAE_WAVE * PAE_ROWS_WAVES;
+    const int ck = min(c, PAE_WAVE * hd / 4 - 1), cv = min(c, PAE_WAVE * vd / 4 - 1);
+    k_key[u] = ck / (hd / 4);
+    k_dim[u] = (ck % (hd / 4)) * 4;
+    // neighbouring threads take a feature's run of keys within a page, then the next feature
+    v_key[u] = cv / (span / 4 * vd) * span + cv % (span / 4) * 4;
+    v_dim[u] = cv % (span / 4 * vd) / (span / 4);
+  }
+
+  // tokens of one sequence at a time (neighbours in a step mostly are); the first barrier below is behind the queries, too
+  int at = t0;
+  const int t_end = min(t0 + toks, num_tokens);
+  while (at < t_end) {
+    const int s = __builtin_amdgcn_readfirstlane(tok_seq[at]);
+    int low = 0x7fffffff, high = -1, next = at;
+    for (; next < t_end && __builtin_amdgcn_readfirstlane(tok_seq[next]) == s; ++next) {
+      const int p = __builtin_amdgcn_readfirstlane(positions[next]);
+      const int first = window <= 0 ? 0 : (chunked ? p - p % window : (p - window + 1 > 0 ? p - window + 1 : 0));
+      low = min(low, first);
+      high = max(high, p);
+    }
+    const int* table = block_tables + (int64_t)s * max_blocks;
+    // A chunk's keys and values, four numbers at a time (keys [key][feature], values [page][feature][offset]); what a
+    // thread brings lies at the same places of every chunk.
+    // No load stands under a condition: pages before and behind those in sight are read as the nearest one in
+    // sight, and what lies beside the keys in sight is never looked at.
+    const int page_low = low / bs, page_high = high / bs;
+    f32x4 k_reg[FOURS], v_reg[FOURS];
+    auto fetch = [&](int base) {
+      const int page0 = base / bs, off0 = base % bs;
+      int k_page[FOURS], v_page[FOURS];
+#pragma unroll
+      for (int u = 0; u < FOURS; ++u) {
+        k_page[u] = table[min(max(page0 + k_key[u] / span, page_low), page_high)];
+        v_page[u] = table[min(max(page0 + v_key[u] / span, page_low), page_high)];
+      }
+#pragma unroll
+      for (int u = 0; u < FOURS; ++u)
+        k_reg[u] = *(const f32x4*)(k_cache + (((int64_t)k_page[u] * nkv + kvh) * bs + off0 + k_key[u] % span) * hd + k_dim[u]);
+#pragma unroll
+      for (int u = 0; u < FOURS; ++u)
+        v_reg[u] = *(const f32x4*)(v_cache + (((int64_t)v_page[u] * nkv + kvh) * vd + v_dim[u]) * bs + off0 + v_key[u] % span);
+    };
+    const int base0 = (low / PAE_WAVE) * PAE_WAVE;
+    fetch(base0);
+    for (int base = base0; base <= high; base += PAE_WAVE) {
+      __syncthreads();  // the chunk before has been read
+#pragma unroll
+      for (int u = 0; u < FOURS; ++u) *(f32x4*)(k_lds + k_key[u] * kst + k_dim[u]) = k_reg[u];
+#pragma unroll
+      for (int u = 0; u < FOURS; ++u) {
+        float* v = v_lds + v_key[u] * vst + v_dim[u];
+        v[0] = v_reg[u].x;
+        v[vst] = v_reg[u].y;
+        v[2 * vst] = v_reg[u].z;
+        v[3 * vst] = v_reg[u].w;
+      }
+      __syncthreads();
+      if (base + PAE_WAVE <= high) fetch(base + PAE_WAVE);
+      bool on[PAE_ROWS_EACH];
+      bool any = false, whole = true;
+#pragma unroll
+      for (int i = 0; i < PAE_ROWS_EACH; ++i) {
+        on[i] = live[i] && tok[i] >= at && tok[i] < next && base <= pos[i] && base + PAE_WAVE > start[i];
+        any = any || on[i];
+        whole = whole && (!live[i] || (on[i] && start[i] <= base && pos[i] >= base + PAE_WAVE - 1));
+      }
+      if (!any) continue;
+      // scores: the lane's key against every row
+      float dot[PAE_ROWS_EACH];
+      int q_row[PAE_ROWS_EACH];
+#pragma unroll
+      for (int i = 0; i < PAE_ROWS_EACH; ++i) {
+        dot[i] = 0.f;
+        q_row[i] = live[i] ? (wave + i * PAE_ROWS_WAVES) * hd : 0;
+      }
+      const float* kr = k_lds + lane * kst;
+#pragma unroll 4
+      for (int d = 0; d < hd; d += 4) {
+        const float4 k4 = *(const float4*)(kr + d);
+#pragma unroll
+        for (int i = 0; i < PAE_ROWS_EACH; ++i) {
+          const float4 q4 = *(const float4*)(q_lds + q_row[i] + d);
+          dot[i] = fmaf(q4.x, k4.x, dot[i]);
+          dot[i] = fmaf(q4.y, k4.y, dot[i]);
+          dot[i] = fmaf(q4.z, k4.z, dot[i]);
+          dot[i] = fmaf(q4.w, k4.w, dot[i]);
+        }
+      }
+      const int key = base + lane;
+      float sc[PAE_ROWS_EACH], m_new[PAE_ROWS_EACH], p[PAE_ROWS_EACH], sum[PAE_ROWS_EACH];
+#pragma unroll
+      for (int i = 0; i < PAE_ROWS_EACH; ++i) {
+        sc[i] = dot[i] * scale;
+        if (slopes) sc[i] -= slopes[head[i]] * (float)(pos[i] - key);
+        if (cap > 0.f) sc[i] = cap * tanhf(sc[i] / cap);
+        if (!(key >= start[i] && key <= pos[i])) sc[i] = -INFINITY;
+        m_new[i] = wave_max(sc[i]);
+      }
+#pragma unroll
+      for (int i = 0; i < PAE_ROWS_EACH; ++i) {  // the rows' reductions side by side; rows that are not on keep what they have
+        m_new[i] = fmaxf(m[i], m_new[i]);
+        p[i] = key >= start[i] && key <= pos[i] ? expf(sc[i] - m_new[i]) : 0.f;
+        sum[i] = wave_sum(p[i]);
+      }
+#pragma unroll
+      for (int i = 0; i < PAE_ROWS_EACH; ++i) {
+        if (!on[i]) continue;
+        const float alpha = expf(m[i] - m_new[i]);
+        l[i] = l[i] * alpha + sum[i];
+        m[i] = m_new[i];
+        p_lds[i * PAE_WAVE + lane] = p[i];
+#pragma unroll
+        for (int d = 0; d < MAXD; ++d) acc[i][d] *= alpha;
+      }
+      // sums: the lane's features over the keys in order (the wavefront's own p: no barrier, its LDS operations are in order)
+      __builtin_amdgcn_wave_barrier();
+      if (whole) {
+#pragma unroll 2
+        for (int j = 0; j < PAE_WAVE; j += 4) {
+          float v[4][MAXD];
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int d = 0; d < MAXD; ++d) v[u][d] = v_lds[(j + u) * vst + min(lane + d * PAE_WAVE, vd - 1)];
+#pragma unroll
+          for (int i = 0; i < PAE_ROWS_EACH; ++i) {
+            if (!live[i]) continue;
+            const float4 p4 = *(const float4*)(p_lds + i * PAE_WAVE + j);
+#pragma unroll
+            for (int d = 0; d < MAXD; ++d) {
+              acc[i][d] = fmaf(p4.x, v[0][d], acc[i][d]);
+              acc[i][d] = fmaf(p4.y, v[1][d], acc[i][d]);
+              acc[i][d] = fmaf(p4.z, v[2][d], acc[i][d]);
+              acc[i][d] = fmaf(p4.w, v[3][d], acc[i][d]);
+            }
+          }
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < PAE_ROWS_EACH; ++i) {
+          if (!on[i]) continue;
+          const int first = max(0, start[i] - base), last = min(PAE_WAVE - 1, pos[i] - base);
+          auto add = [&](int j, float p) {
+#pragma unroll
+            for (int d = 0; d < MAXD; ++d)
+              if (lane + d * PAE_WAVE < vd) acc[i][d] = fmaf(p, v_lds[j * vst + lane + d * PAE_WAVE], acc[i][d]);
+          };
+          int j = first;
+#pragma unroll 1
+          for (; j <= last && j % 4; ++j) add(j, p_lds[i * PAE_WAVE + j]);
+#pragma unroll 1
+          for (; j + 3 <= last; j += 4) {
+            const float4 p4 = *(const float4*)(p_lds + i * PAE_WAVE + j);
+            float v[4][MAXD];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+              for (int d = 0; d < MAXD; ++d) v[u][d] = v_lds[(j + u) * vst + min(lane + d * PAE_WAVE, vd - 1)];
+#pragma unroll
+            for (int d = 0; d < MAXD; ++d) {
+              acc[i][d] = fmaf(p4.x, v[0][d], acc[i][d]);
+              acc[i][d] = fmaf(p4.y, v[1][d], acc[i][d]);
+              acc[i][d] = fmaf(p4.z, v[2][d], acc[i][d]);
+              acc[i][d] = fmaf(p4.w, v[3][d], acc[i][d]);
+            }
+          }
+#pragma unroll 1
+          for (; j <= last; ++j) add(j, p_lds[i * PAE_WAVE + j]);
+        }
+      }
+    }
+    at = next;
+  }
+#pragma unroll
+  for (int i = 0; i < PAE_ROWS_EACH; ++i) {
+    if (!live[i]) continue;
+    float* o = out + (int64_t)tok[i] * out_stride + (int64_t)head[i] * vd;
+    float keep = 1.f;
+    if (sinks) {
+      const float sink = sinks[head[i]];
+      const float m_all = fmaxf(m[i], sink);
+      keep = expf(m[i] - m_all);
+      l[i] = l[i] * keep + expf(sink - m_all);
+    }
+    const float inv = keep / l[i];
+#pragma unroll
+    for (int d = 0; d < MAXD; ++d) {
+      const int f = lane + d * PAE_WAVE;
+      if (f < vd) {
+        float v = acc[i][d] * inv;
+        if (gate) v *= 1.0f / (1.0f + expf(-gate[(int64_t)tok[i] * gate_stride + (gate_per_head ? head[i] : (int64_t)head[i] * vd + f)]));
+        o[f] = v;
+      }
+    }
+  }
+}
+
+// Whether the rows kernel takes a call: rows and pages that can be read four numbers at a time, and a chunk's keys and values
+// in half a compute unit's LDS (heads of up to 128 wide) or at least in all of it.
+static bool rows_kernel_takes(const void* k_cache, const void* v_cache, int bs, int hd, int vd, int shared_kv) {
+  return !shared_kv && bs % 4 == 0 && (bs >= PAE_WAVE ? bs % PAE_WAVE == 0 : PAE_WAVE % bs == 0) && hd % 4 == 0 && vd <= 256 &&
+         hd <= 256 && (uintptr_t)k_cache % 16 == 0 && (uintptr_t)v_cache % 16 == 0;
+}
+
+static int launch_rows(float* out, int64_t out_stride, const float* q, int64_t q_stride, const float* k_cache,
+                       const float* v_cache, const int* positions, const int* tok_seq, const int* block_tables,
+                       int max_blocks, int bs, int num_tokens, int nh, int nkv, int hd, int vd, float scale, int window,
+                       float cap, const float* sinks, int chunked, const float* slopes, const float* gate,
+                       int64_t gate_stride, int gate_per_head, hipStream_t stream) {
+  const int g = nh / nkv;
+  const int heads_each = g < PAE_ROWS_MOST ? g : PAE_ROWS_MOST;
+  const int parts = (g + heads_each - 1) / heads_each;
+  // several tokens share a workgroup's keys where there are workgroups enough (decode steps: a token each)
+  const int toks = (int64_t)num_tokens * nkv * parts >= 512 ? PAE_ROWS_MOST / heads_each : 1;
+  const dim3 grid((num_tokens + toks - 1) / toks, nkv * parts);
+  const size_t lds = (size_t)(PAE_WAVE * (hd + 4 + vd + 4) + PAE_ROWS_MOST * (PAE_WAVE + hd)) * sizeof(float);
+#define PAE_LAUNCH(MAXD)                                                                                           do {                                                                                                               if (lds > 65536) {                                                                                                 const hipError_t err = hipFuncSetAttribute((const void*)paged_attention_rows_kernel<MAXD>,                                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);                if (err != hipSuccess) return pae_fail("attention: %zu bytes of LDS refused: %s", lds, hipGetErrorString(err));     }                                                                                                                paged_attention_rows_kernel<MAXD><<<grid, PAE_WAVE * PAE_ROWS_WAVES, lds, stream>>>(                                 out, out_stride, q, q_stride, k_cache, v_cache, positions, tok_seq, block_tables, max_blocks, bs,                num_tokens, nh, nkv, hd, vd, scale, window, cap, sinks, chunked, slopes, gate, gate_stride,                      gate_per_head, toks, heads_each);                                                                          } while (0)
+  const int wide = hd > vd ? hd : vd;
+  if (wide <= 64) PAE_LAUNCH(1);
+  else if (wide <= 128) PAE_LAUNCH(2);
+  else if (wide <= 192) PAE_LAUNCH(3);
+  else PAE_LAUNCH(4);
+#undef PAE_LAUNCH
+  return pae_check_launch("paged_attention_rows");
+}
+
 template <typename T>
 static int launch_generic(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k_cache,
                           const void* v_cache, const int* positions, const int* tok_seq,
@@ -161,6 +464,10 @@ extern "C" int pae_paged_attention_masked(int dtype, void* out, int64_t out_stri
   PAE_REQUIRE(cap >= 0.f, "attention: negative score cap %g", (double)cap);
   PAE_REQUIRE(nh <= 65535, "attention: %d query heads exceed the grid", nh);
   if (num_tokens <= 0) return 0;
+  if (dtype == PAE_F32 && rows_kernel_takes(k_cache, v_cache, bs, hd, vd, shared_kv) && nkv <= 65535)
+    return launch_rows((float*)out, out_stride, (const float*)q, q_stride, (const float*)k_cache, (const float*)v_cache, positions,
+                       tok_seq, block_tables, max_blocks, bs, num_tokens, nh, nkv, hd, vd, scale, window, cap, sinks, chunked,
+                       slopes, (const float*)gate, gate_stride, gate_per_head, stream);
   if (dtype == PAE_F32)
     return launch_generic<float>(out, out_stride, q, q_stride, k_cache, v_cache, positions, tok_seq, block_tables,
                                  max_blocks, bs, num_tokens, nh, nkv, hd, vd, scale, window, cap, sinks, chunked, slopes, gate,

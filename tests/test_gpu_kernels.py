@@ -86,6 +86,32 @@ def test_gemm_plain(dtype, M, N, K_):
         assert torch.equal(one[0], out[M - 1])
 
 
+@pytest.mark.parametrize("N,K_", [(15, 4), (17, 508), (130, 512), (64, 516), (200, 1040), (33, 4100), (16, 5002), (1536, 8960),
+                                  (40000, 1030)])
+def test_gemm_plain_adds_in_one_order(N, K_):
+    """Every kernel and every way to share k out gives a row the same bits: few rows (up to 16, 32 and 64), tiles of 64 and
+    of 128 rows, one workgroup a tile or several, rows read by fours or one by one; and the error against 64
+    bits is that of 512 products added in a row: 512 roundings of half a unit in the last place, of the
+    sum of the products' sizes, most of which cancel (a quarter of it bounds what is seen by far)."""
+    torch.manual_seed(N + K_)
+    a, w, b = torch.randn(300, K_), torch.randn(N, K_), torch.randn(N)
+    want = a.double() @ w.double().t() + b.double()
+    bound = 512 * 2.0 ** -24 * 0.25 * float((a.double().abs() @ w.double().abs().t()).max())
+    a, w, b = a.to(DEV), w.to(DEV), b.to(DEV)
+    spread = torch.zeros(300, K_ + 1, device=DEV)  # rows that do not begin on 16 bytes
+    spread[:, :K_] = a
+    first = None
+    for M in (1, 16, 17, 33, 64, 65, 128, 129, 300):
+        out = torch.full((M, N), float("nan"), device=DEV)
+        K().gemm_plain(out, a[300 - M:], w, b)
+        first = out if first is None else first
+        assert torch.equal(out[-1], first[0]), M
+        assert (out.double().cpu() - want[300 - M:]).abs().max() <= bound, M
+        one_by_one = torch.full((M, N), float("nan"), device=DEV)
+        K().gemm_plain(one_by_one, spread[300 - M:, :K_], w, b)
+        assert torch.equal(one_by_one, out), M
+
+
 @pytest.mark.parametrize("M", [1, 8, 17, 64])
 @pytest.mark.parametrize("N,K_", [(2048, 1536), (1536, 8960), (50, 72), (777, 64), (96, 200),
                                   # about 256 workgroups of 5, 6, 7 and 8 wavefronts of 16 weight rows (above 16 rows of A)
@@ -824,3 +850,51 @@ def test_sampling_kernel():
     for u in (0.0, 1e-7, 0.25, 0.5, 0.75, 0.999999):
         K().sample(tokens[:1], d_row, torch.tensor([0.9], device=DEV), torch.tensor([u], device=DEV))
         assert int(tokens[0]) == plain.sample_from_logits(row[0], 0.9, u)
+
+
+@pytest.mark.parametrize("nh,nkv,hd,vd,bs", [(12, 2, 128, 128, 16), (4, 4, 16, 24, 8), (20, 1, 64, 64, 64), (3, 1, 256, 200, 4),
+                                             (8, 2, 36, 256, 128), (18, 9, 128, 64, 16)])
+@pytest.mark.parametrize("window,chunked,cap,extras", [(0, False, 0.0, False), (37, False, 20.0, True), (64, True, 0.0, True),
+                                                       (1, False, 0.0, False)])
+def test_float32_attention_kernels_give_the_same_bits(nh, nkv, hd, vd, bs, window, chunked, cap, extras):
+    """The kernel that brings a chunk of keys to LDS for several rows against the kernel with one wavefront per (token, head)
+    (which takes pools that do not begin on 16 bytes): runs of tokens of several sequences side by side, single
+    tokens between them, lengths at and beside multiples of 64, few rows and many; pages before a
+    window given back; keys and values that nobody may see are NaN."""
+    lib = K()
+    torch.manual_seed(nh + hd + window)
+    for runs in ([(1, 1), (64, 1), (65, 1), (130, 1)], [(63, 63), (200, 130), (1, 1), (129, 64), (300, 200), (5, 5)]):
+        blocks = sum(-(-n // bs) for n, _ in runs) + 1
+        order = (torch.randperm(blocks - 1) + 1).tolist()
+        width = max(-(-n // bs) for n, _ in runs)
+        tables = torch.full((len(runs), width), -1, dtype=torch.int32)
+        positions, tok_seq = [], []
+        k_pool, v_pool = torch.full((blocks, nkv, bs, hd), float("nan")), torch.full((blocks, nkv, vd, bs), float("nan"))
+        for s, (n, new) in enumerate(runs):
+            first_seen = max(0, n - new - window + 1) if window and not chunked else 0
+            for page in range(-(-n // bs)):
+                block = order.pop()
+                if (page + 1) * bs <= first_seen:
+                    continue  # given back
+                tables[s, page] = block
+                here = min(bs, n - page * bs)
+                k_pool[block, :, :here] = torch.randn(nkv, here, hd)
+                v_pool[block, :, :, :here] = torch.randn(nkv, vd, here)
+            positions += list(range(n - new, n))
+            tok_seq += [s] * new
+        T = len(positions)
+        q = torch.randn(T, nh * hd, device=DEV)
+        slopes = torch.rand(nh, device=DEV) * 0.1 if extras else None
+        sinks = torch.randn(nh, device=DEV) if extras else None
+        gate = torch.randn(T, nh * vd, device=DEV) if extras else None
+        outs = []
+        for shift in (0, 1):  # floats by which the pools stand off a 16-byte boundary
+            kc = torch.empty(k_pool.numel() + 4, device=DEV)[shift:shift + k_pool.numel()].view(k_pool.shape).copy_(k_pool)
+            vc = torch.empty(v_pool.numel() + 4, device=DEV)[shift:shift + v_pool.numel()].view(v_pool.shape).copy_(v_pool)
+            out = torch.full((T, nh * vd), float("nan"), device=DEV)
+            lib.paged_attention_masked(out, q, kc, vc, torch.tensor(positions, dtype=torch.int32, device=DEV),
+                                       torch.tensor(tok_seq, dtype=torch.int32, device=DEV), tables.to(DEV), nh, nkv, hd, vd,
+                                       hd ** -0.5, window, chunked, slopes, gate, softcap=cap, sinks=sinks)
+            outs.append(out)
+        assert bool(torch.isfinite(outs[1]).all())
+        assert torch.equal(outs[0], outs[1]), runs
