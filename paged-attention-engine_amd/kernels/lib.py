@@ -68,6 +68,8 @@ def _declare(lib) -> None:
         "pae_scaled_rows": [P, P, P, I, F, I, I, P],
         "pae_skinny_ticket_slots": [I, I],
         "pae_gemm_skinny_act": [P, L, P, L, P, P, I, I, I, I, I, P, P, I, P],
+        "pae_gemm_plain_splits": [I, I, I],
+        "pae_gemm_plain_shared": [I, I, P, L, L, P, L, L, P, L, P, I, I, I, I, I, I, P, P],
         "pae_gemm_plain": [I, I, P, L, P, L, P, P, I, I, I, I, P],
         "pae_gemm_skinny_gated": [P, L, P, L, P, I, I, I, I, P, P, I, P],
         "pae_paged_attention_generic": [I, P, L, P, L, P, P, P, P, P, I, I, I, I, I, I, F, I, P],
@@ -979,7 +981,7 @@ def gemm_skinny_rope(q_out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, bias
 
 
 def gemm_plain(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None) -> None:
-    """out[M, N] = a[M, K] @ w[N, K]^T (+ bias), float32 accumulation in k order."""
+    """out[M, N] = a[M, K] @ w[N, K]^T (+ bias), float32 accumulation in an order that depends on k alone."""
     _not_while_recording("gemm_plain")
     _gpu(out, a, w, bias)
     M, K = a.shape
@@ -989,12 +991,17 @@ def gemm_plain(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, bias: Option
     if bias is not None:
         assert bias.numel() == N
     bp, bf = _param(bias)
-    _check(library().pae_gemm_plain(code_of(a.dtype), code_of(out.dtype), out.data_ptr(), out.stride(0),
-                                    a.data_ptr(), a.stride(0), w.data_ptr(), bp, bf, M, N, K, _stream()))
+    lib = library()
+    splits = lib.pae_gemm_plain_splits(M, N, K)
+    # the sums of every 512 of k, where a tile's k is shared over workgroups
+    sums = torch.empty((-(-K // 512), M, N), dtype=torch.float32, device=out.device) if splits > 1 else None
+    _check(lib.pae_gemm_plain_shared(code_of(a.dtype), code_of(out.dtype), out.data_ptr(), out.stride(0), 0,
+                                     a.data_ptr(), a.stride(0), 0, w.data_ptr(), 0, bp, bf, M, N, K, 1, splits,
+                                     _ptr(sums), _stream()))
 
 
 def gemm_plain_heads(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor) -> None:
-    """One product per head: out[:, h, :] = a[:, h, :] @ w[h]^T, float32 accumulation in k order.
+    """One product per head: out[:, h, :] = a[:, h, :] @ w[h]^T, float32 accumulation in an order that depends on k alone.
     `a` [M, B, K] and `out` [M, B, N] are views whose last dimension is contiguous (heads of wider
     rows, say); `w` [B, N, K] is contiguous."""
     _not_while_recording("gemm_plain_heads")

@@ -3,9 +3,9 @@
 The reference calls F.linear on weights stored (out_features, in_features)
 (engine/model.py:303-305,315,318-320).  Here:
 
-  float32    this engine's own product kernel: float32 fused multiply-adds in k
-             order, no reduced-precision matrix mode, each row independent of the
-             batch;
+  float32    this engine's own product kernels on the float32 matrix cores: products
+             and sums in full 32-bit, in an order that depends on k alone, each row
+             independent of the batch;
   bfloat16   up to 64 rows (decode steps, small portions): the weight-streaming
              matrix-core kernel, which reads W once; more rows: the platform's
              matrix library, as the reference's products go to its library.
