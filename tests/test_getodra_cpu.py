@@ -171,6 +171,9 @@ def test_work_lists_of_latent_attention():
     # pieces of 64 tokens, those with the most keys first, by their row in the table of pages
     assert formed["tiles"] == ([1, 326, 8, 1, 262, 64, 0, 129, 2, 0, 65, 64, 1, 198, 64, 0, 1, 64, 1, 134, 64], 3)
     assert latent_tiles(shape, 1, 2)["runs"][0][:4] == [3, 332, 2, 0]  # without the other kind every run is here
+    # under a window of 40 a run behind 100 rows sees them from position 61 on, in the fourth page of 16
+    seen = expanded_runs(StepShape((7,), (0,), (130,), (100,), 16), 128, 40)
+    assert seen["pages"][0][:8] == [0, 48, 16, 0, 0, 64, 16, 0] and seen["page_table"] == ([-1] * 3 + list(range(12)), 15)
     assert expanded_runs(StepShape((7,), (0,), (5,), (9,), 16), 128) == {"pages": ([], 4), "page_table": ([], 1), "tiles": ([], 3)}
 
 

@@ -333,6 +333,56 @@ def test_latent_attention_from_projected_rows_to_heads(dtype, H, D, R, V, C, dim
         assert err <= bound, f"key {key} of {first_seen}..{last}: {err} > {bound}"
 
 
+@pytest.mark.parametrize("H,D,R,V,C", [(3, 64, 0, 64, 64), (12, 128, 64, 128, 512), (2, 32, 16, 32, 96), (5, 128, 0, 128, 128)])
+@pytest.mark.parametrize("window,sinks", [(0, True), (1, False), (33, True), (64, False), (200, True)])
+def test_latent_attention_over_long_runs_under_a_window_and_with_sinks(H, D, R, V, C, window, sinks):
+    """The heads' keys and values formed for runs of tokens against the softmax in 64 bits: windows within a page of 16, over
+    several and beyond the run, pages in front of the window given back (-1 in the table, NaN where they were), two
+    sequences of which one begins behind cached rows, and a sink per head.  bfloat16 rounds the queries, the heads'
+    keys and values, the weights and the result: a few times 2^-8 of the largest value."""
+    from paged_attention_engine_amd.parts import StepShape
+    from paged_attention_engine_amd.parts.latent import expanded_runs
+
+    K = _K()
+    gen = torch.Generator().manual_seed(H + window)
+    bf = lambda t: t.to(torch.bfloat16)
+    bs, scale, runs = 16, 0.2 * D ** -0.5, [(0, 150), (301, 130)]  # (rows cached before, new rows)
+    w_uk, w_uv = bf(randn(gen, H * D, C, scale=C ** -0.5)), bf(randn(gen, H * V, C, scale=C ** -0.5))
+    sink = torch.randn(H, generator=gen) if sinks else None
+    width = max(-(-(a + n) // bs) for a, n in runs)
+    pool = torch.full((2 * width + 1, bs, C + R), float("nan"), dtype=torch.bfloat16)
+    tables = torch.full((2, width), -1, dtype=torch.int32)
+    order, q_rows, want = torch.randperm(2 * width, generator=gen).add(1).tolist(), [], []
+    for s, (past, n) in enumerate(runs):
+        c, shared = bf(randn(gen, past + n, C)), bf(randn(gen, past + n, max(R, 1)))[:, :R]
+        first = max(0, past - window + 1) // bs if window else 0
+        for page in range(first, -(-(past + n) // bs)):
+            tables[s, page] = order.pop()
+            here = min(bs, past + n - page * bs)
+            pool[tables[s, page], :here] = torch.cat([c, shared], -1)[page * bs:page * bs + here]
+        q = bf(randn(gen, n, H, D + R, scale=2.0))
+        q_rows.append(q.view(n, -1))
+        k = torch.cat([bf(c.double() @ w_uk.double().T).view(-1, H, D), shared[:, None].expand(-1, H, -1)], -1).double()
+        v = bf(c.double() @ w_uv.double().T).view(-1, H, V).double()
+        score = torch.einsum("ihd,jhd->hij", q.double(), k) * scale
+        i, j = torch.arange(past, past + n)[:, None], torch.arange(past + n)
+        score = score.masked_fill((j > i) | ((i - j >= window) if window else (j < 0)), -math.inf)
+        if sinks:
+            score = torch.cat([score, sink.double()[:, None, None].expand(-1, n, 1)], -1)
+        want.append(torch.einsum("hij,jhv->ihv", torch.softmax(score, -1)[..., :past + n], v).reshape(n, -1))
+    lists = expanded_runs(StepShape((0, 1), (0, 150), (150, 130), (0, 301), bs), 128, window)
+    assert all(at >= max(0, past - window + 1) // 16 * 16 if window else True
+               for (row, at, _, _), past in ((p, runs[p[0]][0]) for p in zip(*[iter(lists["pages"][0])] * 4)))
+    dev = lambda name: torch.tensor(lists[name][0], dtype=torch.int32, device=DEV).view(-1, lists[name][1])
+    positions = torch.cat([torch.arange(a, a + n) for a, n in runs]).to(torch.int32).to(DEV)
+    out = torch.full((280, H * V), float("nan"), dtype=torch.bfloat16, device=DEV)
+    K.latent_expanded(out, torch.cat(q_rows).to(DEV), pool.to(DEV), torch.cat([w_uk, w_uv]).to(DEV), dev("pages"), dev("page_table"),
+                      dev("tiles"), positions, tables.to(DEV), None, 1.0, H, D, R, 0, True, V, C, scale, None, window,
+                      None if sink is None else sink.to(DEV))
+    want = torch.cat(want)
+    assert float((out.cpu().double() - want).abs().max()) <= 2e-2 * float(want.abs().max())
+
+
 def test_rotating_pairs_by_hand():
     """Pair (1, 0) at position 3 with dims 2 turns by 3 radians; features behind `dims` pass unchanged."""
     x = torch.tensor([[[1.0, 0.0, 9.0, 8.0]]], dtype=torch.float64)
