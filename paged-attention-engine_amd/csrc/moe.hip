@@ -20,6 +20,7 @@
 // they are the kernels for steps of a few rows.
 #include "common.h"
 #include "api.h"
+#include "tile_gemm.h"
 
 template <typename T>
 __global__ __launch_bounds__(256) void project_f32_kernel(float* __restrict__ out, int64_t ldo, const T* __restrict__ A,
@@ -302,8 +303,8 @@ extern "C" int pae_moe_down(int dtype, float* out, const void* act, const void* 
 //                       of a token are float32 partial sums that the stream's next norm adds in order
 // each in three kernels by the step's size: moe_few_tiles (up to 512 pairs), moe_tiles_gate_up / moe_tiles_down (up to
 // 4,096), moe_big_tiles (above).
-typedef __attribute__((ext_vector_type(4))) float f32x4;
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+using tile_gemm::bf16x8;
+using tile_gemm::f32x4;
 
 __global__ __launch_bounds__(1024) void moe_sort_kernel(const int* __restrict__ chosen, int pairs, int experts, int tile_rows,
                                                         int* __restrict__ order, int4* __restrict__ tiles, int max_tiles) {
@@ -334,8 +335,10 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(const int* __restrict__ 
   }
   for (int e = threadIdx.x; e < experts; e += 1024)
     for (int j = 0; j * tile_rows < count[e]; ++j)
-      tiles[first_tile[e] + j] = make_int4(e, start[e] + j * tile_rows, min(tile_rows, count[e] - j * tile_rows), 0);
+      tiles[first_tile[e] + j] = make_int4(e, start[e] + j * tile_rows, min(tile_rows, count[e] - j * tile_rows),
+                                           j << 16 | ((count[e] + tile_rows - 1) / tile_rows & 0xffff));
   for (int i = *total + threadIdx.x; i < max_tiles; i += 1024) tiles[i] = make_int4(0, 0, 0, 0);
+  if (threadIdx.x == 0) tiles[max_tiles] = make_int4(*total, 0, 0, 0);
 }
 
 // A wavefront holds MT tiles of 16 rows by NT tiles of 16 features: MT + NT (2 NT with gate and up) operand loads
@@ -562,99 +565,64 @@ __global__ __launch_bounds__(256) void moe_few_tiles_kernel(bf16_t* __restrict__
 }
 
 // The same two products for prompts, where an expert sees hundreds of tokens: a workgroup takes a tile of 128 rows
-// and 128 features with gate and up (or 256 output features of the down product), and its operands pass through LDS:
-// every 64 of k, the 256 threads fetch 128 rows of activations and 256 rows of weights, a whole 128-byte line a row, into
-// registers while the step before is multiplied, and then write them to LDS (rows 144 bytes apart, so that the 16-byte
-// reads of a wavefront's lanes fall on all banks).  The four wavefronts are two by two: 64 rows by 64 features with gate
-// and up (or 128 features), 64 matrix instructions for 24 reads of LDS a step.  Two barriers a step.
-#define MOE_BIG_ROWS 128
-#define MOE_BIG_K 64
-#define MOE_LDS_STRIDE 72  // bf16 from a row of 64 to the next in LDS
+// and 128 features with gate and up (or 256 output features of the down product) through the loop of tile_gemm.h.
+// What bounds it: the rate at which a compute unit takes lines in (tile_gemm.h), so what a workgroup's neighbours
+// on the die bring to its L2 counts, and padding: experts see a few hundred rows each.  Measured, 3,001 tokens by four of 32
+// experts, 1,536 x 2,240 (165 and 83 GFLOP): with operands through registers, two barriers a stage of 64 of k and
+// one workgroup's features after another 594 and 298 us; through tile_gemm.h 382 and 172; with an expert's
+// tiles side by side on one die 318 and 140 (three quarters of the lines from L2); with the loads spread among
+// the products 306 and 127 us (540 and 650 TFLOP/s).
+#define MOE_BIG_ROWS tile_gemm::BM
+#define MOE_BIG_K tile_gemm::BK
 template <bool GATED>
-__global__ __launch_bounds__(256) void moe_big_tiles_kernel(bf16_t* __restrict__ act_out, float* __restrict__ y,
-                                                            const bf16_t* __restrict__ a_rows, int64_t lda,
-                                                            const bf16_t* __restrict__ w_first, const bf16_t* __restrict__ w_second,
-                                                            const int* __restrict__ order, const float* __restrict__ weights,
-                                                            const int4* __restrict__ tiles, int top, int num_tokens, int K,
-                                                            int N, int act_kind) {
+__global__ __launch_bounds__(256, 1) void moe_big_tiles_kernel(bf16_t* __restrict__ act_out, float* __restrict__ y,
+                                                               const bf16_t* __restrict__ a_rows, int64_t lda,
+                                                               const bf16_t* __restrict__ w_first, const bf16_t* __restrict__ w_second,
+                                                               const int* __restrict__ order, const float* __restrict__ weights,
+                                                               const int4* __restrict__ tiles, int max_tiles, int top,
+                                                               int num_tokens, int K, int N, int act_kind) {
   // GATED: a_rows = x (row of a pair = its token), w_first / w_second = gate / up [E][N][K], N = the experts' width;
   // else: a_rows = act in sorted order, w_first = down [E][N][K], N = the hidden width
-  __shared__ __attribute__((aligned(16))) bf16_t lds_a[MOE_BIG_ROWS * MOE_LDS_STRIDE];
-  __shared__ __attribute__((aligned(16))) bf16_t lds_w[256 * MOE_LDS_STRIDE];
-  const int4 tile = tiles[blockIdx.x];  // (expert, first sorted row, rows, unused)
-  if (tile.z <= 0) return;
+  extern __shared__ __attribute__((aligned(16))) char big_lds[];
   constexpr int FEATURES = GATED ? 128 : 256;  // output features a workgroup takes
-  const int n_base = blockIdx.y * FEATURES;
-  const int tid = threadIdx.x, lane = tid % PAE_WAVE, wave = tid / PAE_WAVE;
+  // Workgroups i, i + 8, i + 16, ... run on one die: they take an eighth of the work in a row, in which an expert's
+  // tiles of one block of features follow one another, so that what they share comes to the die's L2 once.
+  const int blocks = (N + FEATURES - 1) / FEATURES, total = tiles[max_tiles].x * blocks;
+  const int per = (total + 7) / 8, place = blockIdx.x / 8 < per ? blockIdx.x % 8 * per + blockIdx.x / 8 : total;
+  if (place >= total) return;
+  const int some = place / blocks, mine = tiles[some].w;  // a tile of the expert, its number among the expert's << 16 | how many
+  const int first = some - (mine >> 16), within = place - first * blocks;
+  const int4 tile = tiles[first + within % (mine & 0xffff)];  // (expert, first sorted row, rows, as above)
+  const int n_base = within / (mine & 0xffff) * FEATURES;
+  const int tid = threadIdx.x, lane = tid % PAE_WAVE, wave = __builtin_amdgcn_readfirstlane(tid / PAE_WAVE);
   const int col = lane % 16, kg = lane / 16;
   const int wr = wave / 2, wc = wave % 2;
-  // what this thread fetches: 16 bytes (piece tid % 8) of rows tid / 8 + 32 j
-  const int piece = tid % 8, frow = tid / 8;
-  const bf16_t* a_src[4];
-  const bf16_t* w_src[8];
+  tile_gemm::Source src;
+  src.a = reinterpret_cast<const char*>(a_rows);
+  // W's 256 rows in LDS: gated, the first 128 are gate's features (the first two wavefronts bring them), the rest up's
+  const bf16_t* w = (GATED && wave >= 2) ? w_second : w_first;
+  src.w = reinterpret_cast<const char*>(w + (int64_t)__builtin_amdgcn_readfirstlane(tile.x) * N * K);
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int r = frow + 32 * j;
+  for (int j = 0; j < tile_gemm::A_LOADS; ++j) {
+    const int r = (wave * tile_gemm::A_LOADS + j) * 8 + lane / 8;
     const int sorted = tile.y + (r < tile.z ? r : 0);
-    const int64_t row = GATED ? order[sorted] / top : sorted;
-    a_src[j] = a_rows + row * lda + 8 * piece;
+    src.a_off[j] = (uint32_t)((GATED ? order[sorted] / top : sorted) * lda * 2) + tile_gemm::piece_of(lane, r);
   }
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const int r = frow + 32 * j;  // row of the 256 in LDS: gated, the first 128 are gate's features, the rest up's
-    const int n = min(n_base + (GATED ? r % 128 : r), N - 1);
-    const bf16_t* w = (GATED && r >= 128) ? w_second : w_first;
-    w_src[j] = w + ((int64_t)tile.x * N + n) * K + 8 * piece;
+  for (int j = 0; j < tile_gemm::W_LOADS; ++j) {
+    const int r = (wave * tile_gemm::W_LOADS + j) * 8 + lane / 8;
+    src.w_off[j] = (uint32_t)min(n_base + (GATED ? r % 128 : r), N - 1) * (uint32_t)(K * 2) + tile_gemm::piece_of(lane, r);
   }
   f32x4 acc[4][8];
+  int w_row[8];
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt)
+  for (int nt = 0; nt < 8; ++nt) {
+    // gated: groups 0..3 are gate's features wc * 64 + 16 nt, groups 4..7 the same features of up
+    w_row[nt] = GATED ? (nt / 4) * 128 + wc * 64 + 16 * (nt % 4) : wc * 128 + 16 * nt;
 #pragma unroll
-    for (int nt = 0; nt < 8; ++nt) acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  bf16x8 fa[4], fw[8];
-  auto fetch = [&](int k) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) fa[j] = *reinterpret_cast<const bf16x8*>(a_src[j] + k);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) fw[j] = *reinterpret_cast<const bf16x8*>(w_src[j] + k);
-  };
-  auto stage = [&]() {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) *reinterpret_cast<bf16x8*>(&lds_a[(frow + 32 * j) * MOE_LDS_STRIDE + 8 * piece]) = fa[j];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) *reinterpret_cast<bf16x8*>(&lds_w[(frow + 32 * j) * MOE_LDS_STRIDE + 8 * piece]) = fw[j];
-  };
-  auto multiply = [&]() {
-#pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      bf16x8 a[4], w[8];
-#pragma unroll
-      for (int mt = 0; mt < 4; ++mt)
-        a[mt] = *reinterpret_cast<const bf16x8*>(&lds_a[(wr * 64 + 16 * mt + col) * MOE_LDS_STRIDE + 32 * half + 8 * kg]);
-#pragma unroll
-      for (int nt = 0; nt < 8; ++nt) {
-        // gated: tiles 0..3 are gate's features wc * 64 + 16 nt, tiles 4..7 the same features of up
-        const int row = GATED ? (nt / 4) * 128 + wc * 64 + 16 * (nt % 4) + col : wc * 128 + 16 * nt + col;
-        w[nt] = *reinterpret_cast<const bf16x8*>(&lds_w[row * MOE_LDS_STRIDE + 32 * half + 8 * kg]);
-      }
-#pragma unroll
-      for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-        for (int nt = 0; nt < 8; ++nt) acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[nt], a[mt], acc[mt][nt], 0, 0, 0);
-    }
-  };
-  fetch(0);
-  stage();
-  __syncthreads();
-  const int steps = K / MOE_BIG_K;
-  for (int s = 1; s < steps; ++s) {
-    fetch(MOE_BIG_K * s);  // on its way while the step before is multiplied
-    multiply();
-    __syncthreads();       // everyone has read the step before
-    stage();
-    __syncthreads();
+    for (int mt = 0; mt < 4; ++mt) acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  multiply();
+  tile_gemm::run(acc, big_lds, src, K / MOE_BIG_K, w_row);
   // a lane holds features 16 nt + 4 kg .. + 3 (of its wavefront's) of the row wr * 64 + 16 mt + col
 #pragma unroll
   for (int mt = 0; mt < 4; ++mt) {
@@ -664,10 +632,13 @@ __global__ __launch_bounds__(256) void moe_big_tiles_kernel(bf16_t* __restrict__
       bf16_t* o = act_out + (int64_t)(tile.y + r) * N;
 #pragma unroll
       for (int nt = 0; nt < 4; ++nt) {
-        const int f = n_base + wc * 64 + 16 * nt + 4 * kg;
+        const int f = n_base + wc * 64 + 16 * nt + 4 * kg;  // N is a multiple of 64: all four or none
+        if (f < N) {
+          bf16_t four[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (f + i < N) o[f + i] = __float2bfloat16(act_of(acc[mt][nt][i], act_kind) * acc[mt][nt + 4][i]);
+          for (int i = 0; i < 4; ++i) four[i] = __float2bfloat16(act_of(acc[mt][nt][i], act_kind) * acc[mt][nt + 4][i]);
+          *reinterpret_cast<uint2*>(o + f) = *reinterpret_cast<const uint2*>(four);
+        }
       }
     } else {
       const int pair = order[tile.y + r];
@@ -676,18 +647,19 @@ __global__ __launch_bounds__(256) void moe_big_tiles_kernel(bf16_t* __restrict__
 #pragma unroll
       for (int nt = 0; nt < 8; ++nt) {
         const int n = n_base + wc * 128 + 16 * nt + 4 * kg;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (n + i < N) o[n + i] = weight * acc[mt][nt][i];
+        if (n < N) *reinterpret_cast<f32x4*>(o + n) = weight * acc[mt][nt];
       }
     }
   }
 }
 
 // rows a tile holds for a step of that many pairs: 16 while an expert sees a few tokens, 64 in portions, 128 in prompts
-static int moe_tile_rows(int pairs, int hidden, int inter) {
+// (whose kernel reckons with 32-bit byte offsets within the rows and within an expert's weights)
+static int moe_tile_rows(int pairs, int hidden, int inter, int64_t row_bytes) {
   if (pairs <= 512) return 16;
-  return (pairs > 4096 && hidden % MOE_BIG_K == 0 && inter % MOE_BIG_K == 0) ? MOE_BIG_ROWS : 64;
+  const int64_t widest = row_bytes > (int64_t)inter * 2 ? row_bytes : (int64_t)inter * 2;
+  return (pairs > 4096 && hidden % MOE_BIG_K == 0 && inter % MOE_BIG_K == 0 && pairs * widest < (1ll << 32) &&
+          (int64_t)hidden * inter * 2 < (1ll << 32)) ? MOE_BIG_ROWS : 64;
 }
 extern "C" int pae_moe_tile_rows(int pairs) { return pairs <= 512 ? 16 : (pairs <= 4096 ? 64 : MOE_BIG_ROWS); }
 extern "C" int pae_moe_max_tiles(int pairs, int experts) {
@@ -696,7 +668,7 @@ extern "C" int pae_moe_max_tiles(int pairs, int experts) {
 }
 extern "C" int pae_moe_tiles_supported(int hidden, int inter) { return hidden % 32 == 0 && inter % 32 == 0; }
 
-// `order` int32 [pairs], `tiles` int32 [pae_moe_max_tiles][4], `act` bfloat16 [pairs][inter] are work space;
+// `order` int32 [pairs], `tiles` int32 [pae_moe_max_tiles + 1][4], `act` bfloat16 [pairs][inter] are work space;
 // y float32 [top][num_tokens][hidden] receives every pair's weighted output.
 extern "C" int pae_moe_experts_tiles(float* y, const void* x, int64_t ldx, const void* gate_w, const void* up_w,
                                      const void* down_w, const int* chosen, const float* weights, int num_tokens, int top,
@@ -707,7 +679,7 @@ extern "C" int pae_moe_experts_tiles(float* y, const void* x, int64_t ldx, const
   PAE_REQUIRE(ldx >= hidden && ldx % 8 == 0, "experts: row stride %lld", (long long)ldx);
   if (num_tokens <= 0) return 0;
   const int pairs = num_tokens * top;
-  const int tile_rows = moe_tile_rows(pairs, hidden, inter), max_tiles = pae_moe_max_tiles(pairs, experts);
+  const int tile_rows = moe_tile_rows(pairs, hidden, inter, ldx * 2), max_tiles = pae_moe_max_tiles(pairs, experts);
   moe_sort_kernel<<<1, 1024, (size_t)(4 * experts + 1) * sizeof(int), stream>>>(chosen, pairs, experts, tile_rows, order,
                                                                                (int4*)tiles, max_tiles);
 #define MOE_TILES(MT, UP_NT, DOWN_NT)                                                                                      \
@@ -732,13 +704,17 @@ extern "C" int pae_moe_experts_tiles(float* y, const void* x, int64_t ldx, const
                                                                inter, hidden, act_kind);
   } else if (tile_rows == 64) MOE_TILES(4, 2, 4);
   else {
-    dim3 up_grid(max_tiles, (inter + 127) / 128), down_grid(max_tiles, (hidden + 255) / 256);
-    PAE_REQUIRE(up_grid.y <= 65535 && down_grid.y <= 65535, "experts: widths %d, %d exceed the grid", hidden, inter);
-    moe_big_tiles_kernel<true><<<up_grid, 256, 0, stream>>>((bf16_t*)act, nullptr, (const bf16_t*)x, ldx, (const bf16_t*)gate_w,
-                                                            (const bf16_t*)up_w, order, weights, (const int4*)tiles, top,
+    const int64_t up_grid = (int64_t)max_tiles * ((inter + 127) / 128) + 7, down_grid = (int64_t)max_tiles * ((hidden + 255) / 256) + 7;
+    PAE_REQUIRE(up_grid < (1ll << 31) && down_grid < (1ll << 31), "experts: widths %d, %d exceed the grid", hidden, inter);
+    for (const void* kernel : {(const void*)moe_big_tiles_kernel<true>, (const void*)moe_big_tiles_kernel<false>}) {
+      const hipError_t err = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, tile_gemm::LDS_BYTES);
+      PAE_REQUIRE(err == hipSuccess, "experts: %d bytes of LDS refused: %s", tile_gemm::LDS_BYTES, hipGetErrorString(err));
+    }
+    moe_big_tiles_kernel<true><<<up_grid, 256, tile_gemm::LDS_BYTES, stream>>>((bf16_t*)act, nullptr, (const bf16_t*)x, ldx, (const bf16_t*)gate_w,
+                                                            (const bf16_t*)up_w, order, weights, (const int4*)tiles, max_tiles, top,
                                                             num_tokens, hidden, inter, act_kind);
-    moe_big_tiles_kernel<false><<<down_grid, 256, 0, stream>>>(nullptr, y, (const bf16_t*)act, inter, (const bf16_t*)down_w,
-                                                               nullptr, order, weights, (const int4*)tiles, top, num_tokens,
+    moe_big_tiles_kernel<false><<<down_grid, 256, tile_gemm::LDS_BYTES, stream>>>(nullptr, y, (const bf16_t*)act, inter, (const bf16_t*)down_w,
+                                                               nullptr, order, weights, (const int4*)tiles, max_tiles, top, num_tokens,
                                                                inter, hidden, act_kind);
   }
 #undef MOE_TILES

@@ -1919,7 +1919,7 @@ def moe_experts(x: torch.Tensor, gate_w: torch.Tensor, up_w: torch.Tensor, down_
     if x.dtype == torch.bfloat16 and lib.pae_moe_tiles_supported(H, F) and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0:
         parts = torch.empty((top, T, H), dtype=torch.float32, device=x.device)
         order = torch.empty(T * top, dtype=torch.int32, device=x.device)
-        tiles = torch.empty((lib.pae_moe_max_tiles(T * top, E), 4), dtype=torch.int32, device=x.device)
+        tiles = torch.empty((lib.pae_moe_max_tiles(T * top, E) + 1, 4), dtype=torch.int32, device=x.device)
         _check(lib.pae_moe_experts_tiles(parts.data_ptr(), x.data_ptr(), x.stride(0), gate_w.data_ptr(), up_w.data_ptr(),
                                          down_w.data_ptr(), chosen.data_ptr(), weights.data_ptr(), T, top, E, H, F,
                                          ACTIVATIONS[activation], order.data_ptr(), tiles.data_ptr(), act.data_ptr(),

@@ -438,3 +438,33 @@ def test_few_features_summed_in_float32(dtype):
     bias = torch.randn(7, generator=gen)
     got = K().project_f32(a.to(DEV), w.to(DEV), bias.to(DEV))
     close(got, a.double() @ w.double().T + bias.double(), 1e-5, "float32 sums")
+
+
+@pytest.mark.parametrize("H,F", [(64, 64), (128, 192), (192, 128), (256, 320), (320, 64), (64, 256), (576, 448)])
+def test_experts_of_prompts_on_large_tiles(H, F):
+    """Steps of over 4,096 pairs at widths in multiples of 64: one to nine stages of 64 of k in either product, features that end
+    inside a workgroup's 128 or 256, experts with one row, with 127, 128 and 129, with one tile and with many, and with none; the
+    rows of x wider apart than they are long.  Against float32 products of the same bfloat16 numbers, the activations rounded
+    between them as the kernels do: bfloat16 rounding of what lies between (2^-8) and float32 sums."""
+    gen = torch.Generator().manual_seed(H + F)
+    counts = [1, 127, 128, 129, 0, 640, 3300, 0, 37]
+    E, top = len(counts), 1
+    T = sum(counts)
+    chosen = torch.tensor([e for e, n in enumerate(counts) for _ in range(n)], dtype=torch.int32)[torch.randperm(T, generator=gen)]
+    x = torch.randn((T, H + 8), generator=gen).to(torch.bfloat16)[:, :H]
+    gate, up = ((torch.randn((E, F, H), generator=gen) * H ** -0.5).to(torch.bfloat16) for _ in range(2))
+    down = (torch.randn((E, H, F), generator=gen) * F ** -0.5).to(torch.bfloat16)
+    weights = torch.rand((T, top), generator=gen) + 0.5
+    want = torch.zeros((T, H))
+    for e in range(E):
+        rows = (chosen == e).nonzero()[:, 0]
+        h = x[rows].float()
+        act = (torch.nn.functional.silu(h @ gate[e].float().T) * (h @ up[e].float().T)).to(torch.bfloat16).float()
+        want[rows] = weights[rows] * (act @ down[e].float().T)
+    device_x = torch.empty((T, H + 8), dtype=torch.bfloat16, device=DEV)[:, :H].copy_(x)
+    got = K().moe_experts(device_x, gate.to(DEV), up.to(DEV), down.to(DEV), chosen[:, None].contiguous().to(DEV), weights.to(DEV))
+    close(got.sum(0), want.double(), 1.5e-2, f"experts {H} {F}")
+    # every expert twice a row, with weights that add up to the same
+    both = K().moe_experts(device_x, gate.to(DEV), up.to(DEV), down.to(DEV), chosen[:, None].expand(-1, 2).contiguous().to(DEV),
+                           torch.cat([weights * 0.25, weights * 0.75], -1).contiguous().to(DEV))
+    close(both.sum(0), want.double(), 1.5e-2, f"experts twice {H} {F}")
