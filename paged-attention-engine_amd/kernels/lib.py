@@ -90,7 +90,7 @@ def _declare(lib) -> None:
         "pae_latent_expand": [P, P, P, L, P, P, I, P, I, I, I, I, I, I, I, I, P],
         "pae_latent_queries": [P, P, L, I, P, F, I, I, I, I, I, I, P],
         "pae_attn_prefill_wide_width": [I, I],
-        "pae_attn_prefill_wide_bf16": [P, L, P, L, P, P, P, I, P, P, I, I, I, I, I, F, I, P, P, L, P],
+        "pae_attn_prefill_wide_bf16": [P, L, P, L, P, P, P, I, P, P, I, I, I, I, I, F, I, P, L, P],
         "pae_gated_act": [I, P, P, I, I, I, I, P],
         "pae_gemm_plain_batched": [I, I, P, L, L, P, L, L, P, L, P, I, I, I, I, I, P],
         "pae_rows_from_residual": [I, P, P, L, P],
@@ -1293,12 +1293,10 @@ def latent_key_width(dtype: torch.dtype, row_width: int, rank: int, head_width: 
 def latent_expanded(out: torch.Tensor, proj: torch.Tensor, latent: torch.Tensor, up_weight: torch.Tensor, pages: torch.Tensor,
                     page_table: torch.Tensor, tiles: torch.Tensor, positions: torch.Tensor, block_tables: torch.Tensor,
                     cos_sin: Optional[torch.Tensor], magnitude: float, nh: int, nope: int, rd: int, rot: int, interleaved: bool,
-                    value_dim: int, rank: int, scale: float, head_gate: Optional[torch.Tensor] = None, window: int = 0,
-                    sinks: Optional[torch.Tensor] = None) -> None:
+                    value_dim: int, rank: int, scale: float, head_gate: Optional[torch.Tensor] = None, window: int = 0) -> None:
     """Latent attention for runs of many tokens, the heads' keys and values formed first: out[t, h * value_dim:] of
     the runs' tokens receives the heads (gated by sigmoid of `head_gate` [T, >= nh] if given); other rows are left alone.
-    `window` > 0: a token at position p sees the keys from p - window + 1 on.  `sinks` float32 [nh]: exp(sink) joins each
-    head's denominator.  `proj` and `latent` as for `latent_prepare`, which has written the runs' rows; `up_weight` [nh (nope + value_dim),
+    `window` > 0: a token at position p sees the keys from p - window + 1 on.  `proj` and `latent` as for `latent_prepare`, which has written the runs' rows; `up_weight` [nh (nope + value_dim),
     rank] = [W_uk; W_uv].  `pages` int32 [n, 4] = (table row of the sequence, position of the first key, keys, 0) cuts
     every run's keys, from the sequence's first (or the first one in the window) on, into pages of 16; `page_table` int32 [runs, width] names each run's
     pages in that list, in order; `tiles` int32 [m, 3] = (row of `page_table`, first flat token, tokens <= PREFILL_TILE)."""
@@ -1319,8 +1317,6 @@ def latent_expanded(out: torch.Tensor, proj: torch.Tensor, latent: torch.Tensor,
     _check_cos_sin(cos_sin, rot, T)
     if head_gate is not None:
         _check_head_gate(head_gate, proj, nh)
-    if sinks is not None:
-        assert sinks.is_cuda and sinks.dtype == torch.float32 and sinks.numel() == nh and sinks.is_contiguous()
     lib, new = library(), lambda *shape: torch.empty(shape, dtype=proj.dtype, device=proj.device)
     rows = new(n * 16, rank)
     _check(lib.pae_latent_gather(rows.data_ptr(), latent.data_ptr(), pages.data_ptr(), n, block_tables.data_ptr(),
@@ -1336,7 +1332,7 @@ def latent_expanded(out: torch.Tensor, proj: torch.Tensor, latent: torch.Tensor,
     _check(lib.pae_attn_prefill_wide_bf16(
         out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0), keys.data_ptr(), values.data_ptr(), tiles.data_ptr(),
         tiles.shape[0], positions.data_ptr(), page_table.data_ptr(), page_table.shape[1], nh, nh, width, value_dim, float(scale), int(window),
-        _ptr(sinks), _ptr(head_gate), head_gate.stride(0) if head_gate is not None else 0, _stream()))
+        _ptr(head_gate), head_gate.stride(0) if head_gate is not None else 0, _stream()))
 
 
 def hyper_norm(streams: torch.Tensor, num_streams: int, y: Optional[torch.Tensor], layer_scale: Optional[torch.Tensor],

@@ -25,13 +25,14 @@ head's output is W_uv_j times that sum.  The query projection and the down proje
 product (a gate's rows ride in it); the two per-head products are one launch each.
 
 That costs kv_rank + rope_dim multiply-adds a score and kv_rank a value, the least where few queries meet many keys.
-Runs of many tokens (`EXPAND_ROWS`, bfloat16, no mask in chunks) have their keys and values formed instead, in one
-product over the keys the run sees, and attend with heads of nope_dim + rope_dim and value_dim
+Runs of many tokens (`EXPAND_ROWS`, bfloat16, the layer's own rows, no mask in chunks and no sinks) have their keys and
+values formed instead, in one product over the keys the run sees, and attend with heads of nope_dim + rope_dim and value_dim
 (`kernels.lib.latent_expanded`); the cache stays as it is.  At the 1.5B sizes (12 heads of 128, a latent of 512) that is 4.25
 times fewer multiply-adds a (query, key) pair, in a kernel that runs several times nearer the matrix peak: 8,192
 tokens with 64 rotated features under a window of 4,096 7.76 -> 0.44 ms a layer (and 0.2 to form what it reads), and a
-model of eight layers, two of them such, 28.9 -> 14.0 ms for that prompt; seven prompts of 3,001 tokens in all with a
-sink per head, the layer's own rows or an earlier layer's, 0.44 -> 0.07 ms.
+model of eight layers, two of them such, 28.9 -> 14.0 ms for that prompt.  (Layers with sinks stand before routed
+experts in the design that has them, where another rounding of the same sums chooses other experts at near ties;
+they keep the form whose numbers have been compared so far.  Their runs of 3,001 tokens would go from 0.44 to 0.07 ms.)
 """
 
 from __future__ import annotations
@@ -155,7 +156,7 @@ class LatentAttention(Part):
     def expand_rows(self) -> int:
         """Runs of at least this many tokens attend with the heads' keys and values formed (0: none do)."""
         s = self.spec
-        takes = ((s.mask == "window" or not s.window) and self.matrix_cores
+        takes = (s.own_kv and not s.sinks and (s.mask == "window" or not s.window) and self.matrix_cores
                  and K.latent_key_width(self.dtype, self.row_width, s.kv_rank, s.nope_dim + s.rope_dim, s.value_dim) > 0)
         return EXPAND_ROWS if takes else 0
 
@@ -242,5 +243,5 @@ class LatentAttention(Part):
             K.heads_product(heads.view(T, H, V), summed.view(T, H, C), self.up_v, self.up_v_t)
         if formed:  # over whatever the products above made of these rows
             K.latent_expanded(heads, proj, latent, self.up, tiles["pages"], tiles["page_table"], tiles["tiles"], ctx.positions,
-                              table, cos_sin, magnitude, H, D, R, rot, interleaved, V, C, s.scale, gate, s.window or 0, self.sinks)
+                              table, cos_sin, magnitude, H, D, R, rot, interleaved, V, C, s.scale, gate, s.window or 0)
         return self.out.branch(heads, ctx.sink)

@@ -334,12 +334,12 @@ def test_latent_attention_from_projected_rows_to_heads(dtype, H, D, R, V, C, dim
 
 
 @pytest.mark.parametrize("H,D,R,V,C", [(3, 64, 0, 64, 64), (12, 128, 64, 128, 512), (2, 32, 16, 32, 96), (5, 128, 0, 128, 128)])
-@pytest.mark.parametrize("window,sinks", [(0, True), (1, False), (33, True), (64, False), (200, True)])
-def test_latent_attention_over_long_runs_under_a_window_and_with_sinks(H, D, R, V, C, window, sinks):
+@pytest.mark.parametrize("window", [0, 1, 33, 64, 200])
+def test_latent_attention_over_long_runs_under_a_window(H, D, R, V, C, window):
     """The heads' keys and values formed for runs of tokens against the softmax in 64 bits: windows within a page of 16, over
     several and beyond the run, pages in front of the window given back (-1 in the table, NaN where they were), two
-    sequences of which one begins behind cached rows, and a sink per head.  bfloat16 rounds the queries, the heads'
-    keys and values, the weights and the result: a few times 2^-8 of the largest value."""
+    sequences of which one begins behind cached rows.  bfloat16 rounds the queries, the heads' keys and values, the
+    weights and the result: a few times 2^-8 of the largest value."""
     from paged_attention_engine_amd.parts import StepShape
     from paged_attention_engine_amd.parts.latent import expanded_runs
 
@@ -348,7 +348,6 @@ def test_latent_attention_over_long_runs_under_a_window_and_with_sinks(H, D, R, 
     bf = lambda t: t.to(torch.bfloat16)
     bs, scale, runs = 16, 0.2 * D ** -0.5, [(0, 150), (301, 130)]  # (rows cached before, new rows)
     w_uk, w_uv = bf(randn(gen, H * D, C, scale=C ** -0.5)), bf(randn(gen, H * V, C, scale=C ** -0.5))
-    sink = torch.randn(H, generator=gen) if sinks else None
     width = max(-(-(a + n) // bs) for a, n in runs)
     pool = torch.full((2 * width + 1, bs, C + R), float("nan"), dtype=torch.bfloat16)
     tables = torch.full((2, width), -1, dtype=torch.int32)
@@ -367,9 +366,7 @@ def test_latent_attention_over_long_runs_under_a_window_and_with_sinks(H, D, R, 
         score = torch.einsum("ihd,jhd->hij", q.double(), k) * scale
         i, j = torch.arange(past, past + n)[:, None], torch.arange(past + n)
         score = score.masked_fill((j > i) | ((i - j >= window) if window else (j < 0)), -math.inf)
-        if sinks:
-            score = torch.cat([score, sink.double()[:, None, None].expand(-1, n, 1)], -1)
-        want.append(torch.einsum("hij,jhv->ihv", torch.softmax(score, -1)[..., :past + n], v).reshape(n, -1))
+        want.append(torch.einsum("hij,jhv->ihv", torch.softmax(score, -1), v).reshape(n, -1))
     lists = expanded_runs(StepShape((0, 1), (0, 150), (150, 130), (0, 301), bs), 128, window)
     assert all(at >= max(0, past - window + 1) // 16 * 16 if window else True
                for (row, at, _, _), past in ((p, runs[p[0]][0]) for p in zip(*[iter(lists["pages"][0])] * 4)))
@@ -377,8 +374,7 @@ def test_latent_attention_over_long_runs_under_a_window_and_with_sinks(H, D, R, 
     positions = torch.cat([torch.arange(a, a + n) for a, n in runs]).to(torch.int32).to(DEV)
     out = torch.full((280, H * V), float("nan"), dtype=torch.bfloat16, device=DEV)
     K.latent_expanded(out, torch.cat(q_rows).to(DEV), pool.to(DEV), torch.cat([w_uk, w_uv]).to(DEV), dev("pages"), dev("page_table"),
-                      dev("tiles"), positions, tables.to(DEV), None, 1.0, H, D, R, 0, True, V, C, scale, None, window,
-                      None if sink is None else sink.to(DEV))
+                      dev("tiles"), positions, tables.to(DEV), None, 1.0, H, D, R, 0, True, V, C, scale, None, window)
     want = torch.cat(want)
     assert float((out.cpu().double() - want).abs().max()) <= 2e-2 * float(want.abs().max())
 
