@@ -381,3 +381,73 @@ def test_routing_chooses_by_score_plus_correction_and_weighs_by_score(case):
     if top < E:  # the correction matters: without it other experts are chosen for many tokens
         plainly, _ = K().moe_route(logits.to(DEV), 1, 1, top, 1.0)
         assert (plainly.cpu().long().sort(-1).values != want_chosen.sort(-1).values).any(-1).float().mean() > 0.1
+
+
+def _placed(t, aligned):
+    """A contiguous copy on the device that begins on 16 bytes, or one element behind."""
+    room = torch.empty(t.numel() + 8, dtype=t.dtype, device=DEV)
+    view = room[0 if aligned else 1:][: t.numel()].view(t.shape)
+    return view.copy_(t)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H", [4, 1020, 1024, 1028, 2048, 2052, 4096, 4100])
+@pytest.mark.parametrize("parts", [1, 5, 6])
+def test_norms_with_all_loads_up_front_give_the_bits_of_the_general_ones(dtype, H, parts):
+    """Widths at the edges of what a thread holds and pieces up to one too many (the same kernel on both sides then): the
+    weights of one call begin on 16 bytes, those of the other one element behind, which the general kernels take."""
+    from paged_attention_engine_amd.kernels import lib
+
+    gen = torch.Generator().manual_seed(H + parts)
+    T = 3
+    x, w, w2 = (torch.randn(n, H, generator=gen) for n in (T, 1, 1))
+    a, p, one = torch.randn(T, H, generator=gen).to(dtype), torch.randn(parts, T, H, generator=gen), torch.randn(H, generator=gen).to(dtype)
+    got = []
+    for aligned in (True, False):
+        put, weight = (lambda t: _placed(t, True)), (lambda t: _placed(t, aligned))
+        res, normed, rows = put(x), put(torch.zeros(T, H, dtype=dtype)), put(torch.zeros(T, H, dtype=dtype))
+        lib.norm_join(res, [(put(a), 0.7), (put(p), 1.0)] + ([(put(one), 1.3)] if parts == 1 else []), weight(w[0]), 1e-5, weight(w2[0]), 1e-6,
+                      normed, rows)
+        res2, out1, out2 = put(x), put(torch.zeros(T, H, dtype=dtype)), put(torch.zeros(T, H, dtype=dtype))
+        lib.sum_norm2(res2, [(put(p), 0.3), (put(a), 1.1)], weight(w[0]), weight(w2[0].to(dtype)), 1e-5, out1, out2)
+        got.append([t.cpu() for t in (res, normed, rows, res2, out1, out2)])
+    for one_way, other in zip(*got):
+        assert torch.isfinite(one_way.float()).all() and torch.equal(one_way, other)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,G,D,V", [(1, 1, 8, 8), (12, 2, 128, 128), (16, 4, 128, 64), (40, 24, 64, 64), (3, 0, 40, 40), (63, 1, 128, 128), (64, 1, 128, 128)])
+@pytest.mark.parametrize("rot_share,interleaved,per_head", [(0.0, False, True), (0.5, False, True), (1.0, True, True), (1.0, False, False)])
+def test_rows_by_chunks_are_prepared_as_number_by_number(dtype, H, G, D, V, rot_share, interleaved, per_head):
+    """Up to 256, 512 and 1,024 chunks of 16 bytes a row and beyond, whole and part rotation in both pairings: rows
+    that begin on 16 bytes against the same rows one element behind.  With a norm per head the bits are the same;
+    one sum over a projection is formed in another order.  Its squares are positive: each of the (up to 40 + 8) additions one
+    behind the other moves it by 2^-24 at most, the root by half of that, under 2^-18 of every normalised value; a
+    rotated one is a sum of two such, each up to the largest of all.  bfloat16 adds a rounding, 2^-8 of the value."""
+    from paged_attention_engine_amd.kernels import lib
+
+    gen = torch.Generator().manual_seed(H * 7 + D)
+    T, bs, rot = 3, 16, int(D * rot_share) // 2 * 2
+    width = (H + G) * D + G * V
+    x = torch.randn(T, width, generator=gen).to(dtype)
+    angles = torch.randn(T, max(rot // 2, 1), generator=gen)
+    cos_sin = torch.stack([angles.cos(), angles.sin()], -1).contiguous().to(DEV) if rot else None
+    qw, kw = (torch.randn(n * (1 if per_head else h), generator=gen).to(DEV) for n, h in ((D, H), (D, max(G, 1))))
+    ints = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    positions, seqs, tables = ints([0, 17, 5]), ints([0, 1, 2]), ints([[0, 1], [2, 3], [4, 5]])
+    got = []
+    for aligned in (True, False):
+        room = torch.zeros(T * (width + 8) + 8, dtype=dtype, device=DEV)
+        stride = -(-width // 8) * 8
+        rows = room[0 if aligned else 1:][: T * stride].view(T, stride)[:, :width]
+        rows.copy_(x)
+        k, v = (torch.zeros(6, G, *s, dtype=dtype, device=DEV) if G else None for s in ((bs, D), (V, bs)))
+        lib.qk_norm_rotate_store(rows, H, G, D, V, qw, kw if G else None, 1e-5, rot, interleaved, cos_sin, 1.1, positions,
+                                 seqs if G else None, tables if G else None, bs, k, v, per_head=per_head, temperature=(0.2, 4))
+        got.append([t.cpu() for t in (rows, k, v) if t is not None])
+    for one_way, other in zip(*got):
+        if per_head:
+            assert torch.equal(one_way, other)
+        else:
+            tol = 2.0 ** -8 * other.float().abs() if dtype == torch.bfloat16 else 0.0
+            assert ((one_way.float() - other.float()).abs() <= tol + 2.0 ** -17 * other.float().abs().max()).all()
