@@ -92,19 +92,44 @@ extern "C" int pae_project_f32(int dtype, float* out, int64_t ldo, const void* A
 
 #define MOE_MAX_PER_LANE 16  // experts a lane holds: up to 1,024 experts
 
+// The larger of two (number, place), the lower place of equal numbers, over a wavefront: in every lane.
+__device__ __forceinline__ void wave_best(float& best, int& at) {
+  auto meet = [&](float other, int other_at) {
+    if (other > best || (other == best && other_at < at)) {
+      best = other;
+      at = other_at;
+    }
+  };
+  {
+    const auto v = __builtin_amdgcn_permlane32_swap(__float_as_uint(best), __float_as_uint(best), false, false);
+    const auto p = __builtin_amdgcn_permlane32_swap((unsigned)at, (unsigned)at, false, false);
+    best = __uint_as_float(v[0]);
+    at = (int)p[0];
+    meet(__uint_as_float(v[1]), (int)p[1]);
+  }
+  {
+    const auto v = __builtin_amdgcn_permlane16_swap(__float_as_uint(best), __float_as_uint(best), false, false);
+    const auto p = __builtin_amdgcn_permlane16_swap((unsigned)at, (unsigned)at, false, false);
+    best = __uint_as_float(v[0]);
+    at = (int)p[0];
+    meet(__uint_as_float(v[1]), (int)p[1]);
+  }
+  meet(row_rotated<8>(best), __float_as_int(row_rotated<8>(__int_as_float(at))));
+  meet(row_rotated<4>(best), __float_as_int(row_rotated<4>(__int_as_float(at))));
+  meet(row_rotated<2>(best), __float_as_int(row_rotated<2>(__int_as_float(at))));
+  meet(row_rotated<1>(best), __float_as_int(row_rotated<1>(__int_as_float(at))));
+}
+
+// One token's routing by one wavefront: `z` its logits (memory or LDS), `lds` [E] scores, [groups] group scores, and with
+// a bias [E] what experts are compared by; `chosen` and `weights` its [top + shared_pieces] results.
 template <int PER_LANE>
-__global__ __launch_bounds__(PAE_WAVE) void moe_route_kernel(const float* __restrict__ logits, int E, int groups, int keep,
-                                                             int top, float scale, const float* __restrict__ choice_bias,
-                                                             int64_t ldz, int among_chosen, int shared_pieces,
-                                                             int* __restrict__ chosen, float* __restrict__ weights) {
-  extern __shared__ float lds[];  // [E] scores, [groups] group scores, and with a bias [E] what experts are compared by
+__device__ __forceinline__ void route_token(const float* z, float* lds, int E, int groups, int keep, int top, float scale,
+                                            const float* __restrict__ choice_bias, int among_chosen, int shared_pieces,
+                                            int* __restrict__ chosen, float* __restrict__ weights) {
   float* score = lds;
   float* group_score = lds + E;
   float* rank = choice_bias ? group_score + groups : score;
-  const int64_t t = blockIdx.x;
-  const int lane = threadIdx.x;
-  const float* z = logits + t * ldz;
-  const int places = top + shared_pieces;
+  const int lane = threadIdx.x % PAE_WAVE;
   float top_z = -INFINITY;
   for (int e = lane; e < E; e += PAE_WAVE) top_z = fmaxf(top_z, z[e]);
   top_z = wave_max(top_z);
@@ -140,6 +165,8 @@ __global__ __launch_bounds__(PAE_WAVE) void moe_route_kernel(const float* __rest
       if (before < keep) mine[j] = rank[e];
     }
   }
+  float kept = 0.f;
+  int kept_at = 0;
   float first = 0.f, total = 0.f;  // among_chosen: the largest chosen logit, and the sum of exponentials against it
   for (int r = 0; r < top; ++r) {
     float best = -INFINITY;
@@ -150,39 +177,91 @@ __global__ __launch_bounds__(PAE_WAVE) void moe_route_kernel(const float* __rest
         best = mine[j];
         at = lane + PAE_WAVE * j;
       }
-    for (int off = PAE_WAVE / 2; off > 0; off >>= 1) {
-      const float other = __shfl_xor(best, off, PAE_WAVE);
-      const int other_at = __shfl_xor(at, off, PAE_WAVE);
-      if (other > best || (other == best && other_at < at)) {
-        best = other;
-        at = other_at;
-      }
-    }
+    wave_best(best, at);
     if (at >= E) at = 0;  // no logit compares (not a number): an index that exists
     if (r == 0) first = best;
-    if (among_chosen) total += expf(best - first);
-    if (lane == 0) {
-      chosen[t * places + r] = at;
-      weights[t * places + r] = among_chosen ? expf(best - first) : score[at] / sum * scale;
+    const float e = among_chosen ? expf(best - first) : 0.f;
+    total += e;
+    if (lane == r % PAE_WAVE) {  // held until the sum is known; more than 64 choices are written as they come
+      kept_at = at;
+      kept = among_chosen ? e : score[at] / sum * scale;
+      if (top > PAE_WAVE) {
+        chosen[r] = kept_at;
+        weights[r] = kept;
+      }
     }
 #pragma unroll
     for (int j = 0; j < PER_LANE; ++j)
       if (lane + PAE_WAVE * j == at) mine[j] = -INFINITY;
   }
+  if (top <= PAE_WAVE && lane < top) {
+    chosen[lane] = kept_at;
+    weights[lane] = among_chosen ? kept / total * scale : kept;
+  }
+  if (top > PAE_WAVE && among_chosen)  // each lane its own numbers of the loop above
+    for (int r = lane; r < top; r += PAE_WAVE) weights[r] = weights[r] / total * scale;
   if (lane != 0) return;
-  if (among_chosen)  // this lane's own numbers of the loop above, brought to their sum
-    for (int r = 0; r < top; ++r) weights[t * places + r] = weights[t * places + r] / total * scale;
   for (int p = 0; p < shared_pieces; ++p) {
-    chosen[t * places + top + p] = E + p;
-    weights[t * places + top + p] = 1.0f / (1.0f + expf(-z[E]));
+    chosen[top + p] = E + p;
+    weights[top + p] = 1.0f / (1.0f + expf(-z[E]));
   }
 }
 
-extern "C" int pae_moe_route(const float* logits, int num_tokens, int experts, int groups, int keep, int top, float scale,
-                             const float* choice_bias, int64_t ldz, int among_chosen, int shared_pieces, int* chosen,
-                             float* weights, hipStream_t stream) {
-  PAE_REQUIRE(ldz >= experts + (shared_pieces > 0 ? 1 : 0) && shared_pieces >= 0, "routing: rows of %lld logits for %d experts and %d shared pieces",
-              (long long)ldz, experts, shared_pieces);
+template <int PER_LANE>
+__global__ __launch_bounds__(PAE_WAVE) void moe_route_kernel(const float* __restrict__ logits, int E, int groups, int keep,
+                                                             int top, float scale, const float* __restrict__ choice_bias,
+                                                             int64_t ldz, int among_chosen, int shared_pieces,
+                                                             int* __restrict__ chosen, float* __restrict__ weights) {
+  extern __shared__ float lds[];
+  const int64_t t = blockIdx.x, places = top + shared_pieces;
+  route_token<PER_LANE>(logits + t * ldz, lds, E, groups, keep, top, scale, choice_bias, among_chosen, shared_pieces,
+                        chosen + t * places, weights + t * places);
+}
+
+// Logits and routing of a token in one workgroup, for steps of a few tokens (two launches of a few microseconds' work
+// before): the sums of project_f32_wide_kernel, five outputs of a wavefront on their way together, to LDS, then the
+// first wavefront routes.  7 rows, 32 experts, 1,536 wide: 7.0 + 5.8 -> 7.9 us.
+template <typename T, int PER_LANE>
+__global__ __launch_bounds__(512) void moe_choose_kernel(const T* __restrict__ A, int64_t lda, const T* __restrict__ W,
+                                                         const void* __restrict__ bias, int b_is_f32, int N, int K, int E,
+                                                         int groups, int keep, int top, float scale,
+                                                         const float* __restrict__ choice_bias, int among_chosen,
+                                                         int shared_pieces, int* __restrict__ chosen,
+                                                         float* __restrict__ weights) {
+  constexpr int VEC = 16 / sizeof(T), OUTS = 5;  // (eight wavefronts: up to 40 outputs side by side)
+  struct alignas(16) Chunk { T v[VEC]; };
+  extern __shared__ float lds[];  // [N] logits, then route_token's
+  const int64_t t = blockIdx.x, places = top + shared_pieces;
+  const int wave = threadIdx.x / PAE_WAVE, lane = threadIdx.x % PAE_WAVE;
+  const T* a = A + t * lda;
+  for (int first = wave * OUTS; first < N; first += 8 * OUTS) {
+    float sum[OUTS];
+#pragma unroll
+    for (int o = 0; o < OUTS; ++o) sum[o] = 0.f;
+    for (int k = lane * VEC; k < K; k += PAE_WAVE * VEC) {
+      const Chunk x = *reinterpret_cast<const Chunk*>(a + k);
+      Chunk y[OUTS];
+#pragma unroll
+      for (int o = 0; o < OUTS; ++o) y[o] = *reinterpret_cast<const Chunk*>(W + (int64_t)min(first + o, N - 1) * K + k);
+#pragma unroll
+      for (int o = 0; o < OUTS; ++o)
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) sum[o] = fmaf(to_f32(x.v[i]), to_f32(y[o].v[i]), sum[o]);
+    }
+#pragma unroll
+    for (int o = 0; o < OUTS; ++o) {
+      sum[o] = wave_sum(sum[o]);
+      if (lane == 0 && first + o < N) lds[first + o] = sum[o] + (bias ? load_param(bias, b_is_f32, first + o) : 0.f);
+    }
+  }
+  __syncthreads();
+  if (wave > 0) return;  // (a barrier counts the wavefronts that are left)
+  route_token<PER_LANE>(lds, lds + N, E, groups, keep, top, scale, choice_bias, among_chosen, shared_pieces,
+                        chosen + t * places, weights + t * places);
+}
+
+static int check_route(int experts, int groups, int keep, int top, const float* choice_bias, int among_chosen, int shared_pieces) {
+  PAE_REQUIRE(shared_pieces >= 0, "routing: %d shared pieces", shared_pieces);
   PAE_REQUIRE(!among_chosen || (groups == 1 && !choice_bias), "routing: a softmax over the chosen logits goes with one group and no choice bias");
   PAE_REQUIRE(experts > 0 && experts <= PAE_WAVE * MOE_MAX_PER_LANE, "routing: %d experts (1..%d)", experts,
               PAE_WAVE * MOE_MAX_PER_LANE);
@@ -190,6 +269,50 @@ extern "C" int pae_moe_route(const float* logits, int num_tokens, int experts, i
               groups, experts, keep);
   PAE_REQUIRE(top > 0 && top <= keep * (experts / groups), "routing: %d experts chosen of %d that can be", top,
               keep * (experts / groups));
+  return 0;
+}
+
+// Whether pae_moe_choose takes rows of A: a few (above, the two kernels by themselves have workgroups enough), read 16 bytes
+// at a time.
+extern "C" int pae_moe_choose_takes(int dtype, const void* A, int64_t lda, const void* W, int M, int K) {
+  const int vec = dtype == PAE_F32 ? 4 : 8;
+  return M <= 256 && K % vec == 0 && lda % vec == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0;
+}
+
+// pae_project_f32 and pae_moe_route in one launch: W [experts (+ 1 with shared pieces)][K], bias or null.
+extern "C" int pae_moe_choose(int dtype, const void* A, int64_t lda, const void* W, const void* bias, int b_is_f32, int M,
+                              int K, int experts, int groups, int keep, int top, float scale, const float* choice_bias,
+                              int among_chosen, int shared_pieces, int* chosen, float* weights, hipStream_t stream) {
+  if (int rc = check_route(experts, groups, keep, top, choice_bias, among_chosen, shared_pieces)) return rc;
+  PAE_REQUIRE(dtype == PAE_F32 || dtype == PAE_BF16, "routing: unknown dtype code %d", dtype);
+  PAE_REQUIRE(K > 0 && lda >= K && pae_moe_choose_takes(dtype, A, lda, W, M, K), "routing: %d rows of %d, %lld apart", M, K, (long long)lda);
+  if (M <= 0) return 0;
+  const int N = experts + (shared_pieces > 0 ? 1 : 0);
+  const size_t lds = (size_t)(N + experts + groups + (choice_bias ? experts : 0)) * sizeof(float);
+#define MOE_CHOOSE(T, PER_LANE)                                                                                       \
+  moe_choose_kernel<T, PER_LANE><<<M, 512, lds, stream>>>((const T*)A, lda, (const T*)W, bias, b_is_f32, N, K, experts, \
+                                                          groups, keep, top, scale, choice_bias, among_chosen,        \
+                                                          shared_pieces, chosen, weights)
+#define MOE_CHOOSE_ANY(T)                               \
+  if (experts <= PAE_WAVE) MOE_CHOOSE(T, 1);            \
+  else if (experts <= 4 * PAE_WAVE) MOE_CHOOSE(T, 4);   \
+  else MOE_CHOOSE(T, MOE_MAX_PER_LANE);
+  if (dtype == PAE_F32) {
+    MOE_CHOOSE_ANY(float)
+  } else {
+    MOE_CHOOSE_ANY(bf16_t)
+  }
+#undef MOE_CHOOSE_ANY
+#undef MOE_CHOOSE
+  return pae_check_launch("moe_choose");
+}
+
+extern "C" int pae_moe_route(const float* logits, int num_tokens, int experts, int groups, int keep, int top, float scale,
+                             const float* choice_bias, int64_t ldz, int among_chosen, int shared_pieces, int* chosen,
+                             float* weights, hipStream_t stream) {
+  PAE_REQUIRE(ldz >= experts + (shared_pieces > 0 ? 1 : 0) && shared_pieces >= 0, "routing: rows of %lld logits for %d experts and %d shared pieces",
+              (long long)ldz, experts, shared_pieces);
+  if (int rc = check_route(experts, groups, keep, top, choice_bias, among_chosen, shared_pieces)) return rc;
   if (num_tokens <= 0) return 0;
   const size_t lds = (size_t)(experts + groups + (choice_bias ? experts : 0)) * sizeof(float);
 #define MOE_ROUTE(PER_LANE)                                                                                            \
@@ -501,7 +624,11 @@ __global__ __launch_bounds__(256) void moe_tiles_down_kernel(float* __restrict__
 // one tile of 16 features and take a quarter of k each, leave their sums in LDS, and the first adds them in wavefront
 // order (a wavefront per 16 features and the whole of k was measured against it: 35 + 22 us against 25 + 14 at one
 // token, 85 + 57 against 67 + 39 at eight).  The order of adding is a function of the sizes alone.
-template <bool GATED>
+//
+// In steps of up to 32 tokens and 256 pairs (LISTED) no sorting comes first: a workgroup belongs to an expert (blockIdx.x), a
+// block of features and a sixteen of its rows (blockIdx.z), and looks its pairs up itself, in their order (two
+// barriers, against a launch of 6 us and the same trip to memory for the tile); activations lie at their pair's number.
+template <bool GATED, bool LISTED>
 __global__ __launch_bounds__(256) void moe_few_tiles_kernel(bf16_t* __restrict__ act_out, float* __restrict__ y,
                                                             const bf16_t* __restrict__ a_rows, int64_t lda,
                                                             const bf16_t* __restrict__ w_first, const bf16_t* __restrict__ w_second,
@@ -509,16 +636,38 @@ __global__ __launch_bounds__(256) void moe_few_tiles_kernel(bf16_t* __restrict__
                                                             const int4* __restrict__ tiles, int top, int num_tokens, int K,
                                                             int N, int act_kind) {
   __shared__ f32x4 parts[3][2][PAE_WAVE];
-  const int4 tile = tiles[blockIdx.x];  // (expert, first sorted row, rows <= 16, unused)
+  __shared__ int pair_of[16], of_wave[4];
   const int lane = threadIdx.x % PAE_WAVE, wave = threadIdx.x / PAE_WAVE;
   const int col = lane % 16, kg = lane / 16;
   const int n0 = blockIdx.y * 16;
-  if (tile.z <= 0 || n0 >= N) return;
+  int4 tile;  // (expert, first sorted row, rows <= 16, unused)
+  if (LISTED) {  // order: the pairs' experts
+    const bool mine = (int)threadIdx.x < num_tokens * top && order[threadIdx.x] == (int)blockIdx.x;
+    const uint64_t found = __ballot(mine);
+    if (lane == 0) of_wave[wave] = __popcll(found);
+    __syncthreads();
+    int before = 0, all = 0;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      if (w < wave) before += of_wave[w];
+      all += of_wave[w];
+    }
+    const int place = before + __popcll(found & ((1ull << lane) - 1)) - (int)blockIdx.z * 16;
+    if (mine && place >= 0 && place < 16) pair_of[place] = threadIdx.x;
+    tile = make_int4(blockIdx.x, 0, min(16, all - (int)blockIdx.z * 16), 0);
+    if (tile.z <= 0) return;
+    __syncthreads();
+  } else {
+    tile = tiles[blockIdx.x];
+    if (tile.z <= 0) return;
+  }
+  if (n0 >= N) return;
+  const int sorted = LISTED ? pair_of[col < tile.z ? col : 0] : tile.y + (col < tile.z ? col : 0);
+  const int pair = LISTED ? sorted : order[sorted];  // where a result goes: row `sorted` of the activations, the pair's of y
   const int64_t w_row = (int64_t)tile.x * N + min(n0 + col, N - 1);
   const bf16_t* w1 = w_first + w_row * K + 8 * kg;
   const bf16_t* w2 = GATED ? w_second + w_row * K + 8 * kg : nullptr;
-  const int sorted = tile.y + (col < tile.z ? col : 0);
-  const bf16_t* a = a_rows + (int64_t)(GATED ? order[sorted] / top : sorted) * lda + 8 * kg;
+  const bf16_t* a = a_rows + (int64_t)(GATED ? pair / top : sorted) * lda + 8 * kg;
   const int steps = K / 32, per = (steps + 3) / 4;
   const int first = wave * per, last = min(steps, first + per);
   f32x4 s1 = {0.f, 0.f, 0.f, 0.f}, s2 = {0.f, 0.f, 0.f, 0.f};
@@ -550,12 +699,11 @@ __global__ __launch_bounds__(256) void moe_few_tiles_kernel(bf16_t* __restrict__
   }
   const int n = n0 + 4 * kg;  // a lane holds features n .. n + 3 of the row col
   if (GATED) {
-    bf16_t* o = act_out + (int64_t)(tile.y + col) * N + n;
+    bf16_t* o = act_out + (int64_t)sorted * N + n;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
       if (n + i < N) o[i] = __float2bfloat16(act_of(s1[i], act_kind) * s2[i]);
   } else {
-    const int pair = order[tile.y + col];
     const float weight = weights[pair];
     float* o = y + ((int64_t)(pair % top) * num_tokens + pair / top) * N + n;
 #pragma unroll
@@ -679,6 +827,18 @@ extern "C" int pae_moe_experts_tiles(float* y, const void* x, int64_t ldx, const
   PAE_REQUIRE(ldx >= hidden && ldx % 8 == 0, "experts: row stride %lld", (long long)ldx);
   if (num_tokens <= 0) return 0;
   const int pairs = num_tokens * top;
+  if (num_tokens <= 32 && pairs <= 256) {
+    // (an odd number of columns, so that an expert's workgroups go round the eight dies and not all to one)
+    const dim3 up_grid(experts | 1, (inter + 15) / 16, (num_tokens + 15) / 16), down_grid(experts | 1, (hidden + 15) / 16, (num_tokens + 15) / 16);
+    PAE_REQUIRE(up_grid.y <= 65535 && down_grid.y <= 65535, "experts: widths %d, %d exceed the grid", hidden, inter);
+    moe_few_tiles_kernel<true, true><<<up_grid, 256, 0, stream>>>((bf16_t*)act, nullptr, (const bf16_t*)x, ldx, (const bf16_t*)gate_w,
+                                                                  (const bf16_t*)up_w, chosen, weights, nullptr, top,
+                                                                  num_tokens, hidden, inter, act_kind);
+    moe_few_tiles_kernel<false, true><<<down_grid, 256, 0, stream>>>(nullptr, y, (const bf16_t*)act, inter, (const bf16_t*)down_w,
+                                                                     nullptr, chosen, weights, nullptr, top, num_tokens,
+                                                                     inter, hidden, act_kind);
+    return pae_check_launch("moe_experts_few");
+  }
   const int tile_rows = moe_tile_rows(pairs, hidden, inter, ldx * 2), max_tiles = pae_moe_max_tiles(pairs, experts);
   moe_sort_kernel<<<1, 1024, (size_t)(4 * experts + 1) * sizeof(int), stream>>>(chosen, pairs, experts, tile_rows, order,
                                                                                (int4*)tiles, max_tiles);
@@ -696,10 +856,10 @@ extern "C" int pae_moe_experts_tiles(float* y, const void* x, int64_t ldx, const
   if (tile_rows == 16) {
     dim3 up_grid(max_tiles, (inter + 15) / 16), down_grid(max_tiles, (hidden + 15) / 16);
     PAE_REQUIRE(up_grid.y <= 65535 && down_grid.y <= 65535, "experts: widths %d, %d exceed the grid", hidden, inter);
-    moe_few_tiles_kernel<true><<<up_grid, 256, 0, stream>>>((bf16_t*)act, nullptr, (const bf16_t*)x, ldx, (const bf16_t*)gate_w,
+    moe_few_tiles_kernel<true, false><<<up_grid, 256, 0, stream>>>((bf16_t*)act, nullptr, (const bf16_t*)x, ldx, (const bf16_t*)gate_w,
                                                             (const bf16_t*)up_w, order, weights, (const int4*)tiles, top,
                                                             num_tokens, hidden, inter, act_kind);
-    moe_few_tiles_kernel<false><<<down_grid, 256, 0, stream>>>(nullptr, y, (const bf16_t*)act, inter, (const bf16_t*)down_w,
+    moe_few_tiles_kernel<false, false><<<down_grid, 256, 0, stream>>>(nullptr, y, (const bf16_t*)act, inter, (const bf16_t*)down_w,
                                                                nullptr, order, weights, (const int4*)tiles, top, num_tokens,
                                                                inter, hidden, act_kind);
   } else if (tile_rows == 64) MOE_TILES(4, 2, 4);

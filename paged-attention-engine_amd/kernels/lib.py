@@ -119,6 +119,8 @@ def _declare(lib) -> None:
         "pae_moe_gate_up": [I, P, P, L, P, P, P, I, I, I, I, I, P],
         "pae_moe_down": [I, P, P, P, P, P, I, I, I, I, P],
         "pae_moe_tile_rows": [I],
+        "pae_moe_choose_takes": [I, P, L, P, I, I],
+        "pae_moe_choose": [I, P, L, P, P, I, I, I, I, I, I, I, F, P, I, I, P, P, P],
         "pae_moe_max_tiles": [I, I],
         "pae_moe_tiles_supported": [I, I],
         "pae_moe_experts_tiles": [P, P, L, P, P, P, P, P, I, I, I, I, I, I, P, P, P, P],
@@ -1891,6 +1893,30 @@ def moe_route(logits: torch.Tensor, groups: int, keep: int, top: int, scale: flo
     _check(library().pae_moe_route(logits.data_ptr(), T, E, int(groups), int(keep), int(top), float(scale),
                                    _ptr(choice_bias), logits.stride(0), 1 if among_chosen else 0, int(shared_pieces),
                                    chosen.data_ptr(), weights.data_ptr(), _stream()))
+    return chosen, weights
+
+
+def moe_choose(x: torch.Tensor, router: torch.Tensor, bias: Optional[torch.Tensor], groups: int, keep: int, top: int, scale: float,
+               choice_bias: Optional[torch.Tensor] = None, among_chosen: bool = False, shared_pieces: int = 0):
+    """`moe_route` of `project_f32(x, router, bias)`: in one launch for a few rows, the same bits."""
+    _not_while_recording("moe_choose")
+    _gpu(x, router, bias, choice_bias)
+    T, K = x.shape
+    lib = library()
+    assert x.dim() == 2 and x.stride(1) == 1 and router.dim() == 2 and router.is_contiguous() and router.shape[1] == K and router.dtype == x.dtype
+    if not lib.pae_moe_choose_takes(code_of(x.dtype), x.data_ptr(), x.stride(0), router.data_ptr(), T, K):
+        return moe_route(project_f32(x, router, bias), groups, keep, top, scale, choice_bias, among_chosen, shared_pieces)
+    E = router.shape[0] - (1 if shared_pieces else 0)
+    if bias is not None:
+        assert bias.numel() == router.shape[0] and bias.is_contiguous()
+    if choice_bias is not None:
+        assert choice_bias.dtype == torch.float32 and choice_bias.numel() == E and choice_bias.is_contiguous()
+    bp, bf = _param(bias)
+    chosen = torch.empty((T, top + shared_pieces), dtype=torch.int32, device=x.device)
+    weights = torch.empty((T, top + shared_pieces), dtype=torch.float32, device=x.device)
+    _check(lib.pae_moe_choose(code_of(x.dtype), x.data_ptr(), x.stride(0), router.data_ptr(), bp, bf, T, K, E, int(groups),
+                              int(keep), int(top), float(scale), _ptr(choice_bias), 1 if among_chosen else 0,
+                              int(shared_pieces), chosen.data_ptr(), weights.data_ptr(), _stream()))
     return chosen, weights
 
 

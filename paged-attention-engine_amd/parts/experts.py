@@ -122,9 +122,8 @@ class Experts(Part):
     def forward(self, ctx, x):
         s = self.spec
         x = plain_rows(x)
-        logits = K.project_f32(x, self.router, self.router_bias)
-        chosen, weights = K.moe_route(logits, s.groups, s.groups_kept, s.top, s.route_scale, self.choice_bias,
-                                      s.weights_over == "chosen", self.shared_pieces)
+        chosen, weights = K.moe_choose(x, self.router, self.router_bias, s.groups, s.groups_kept, s.top, s.route_scale,
+                                       self.choice_bias, s.weights_over == "chosen", self.shared_pieces)
         if self.routing_tap is not None:
             self.routing_tap(chosen[:, :s.top], weights[:, :s.top])
         return K.moe_experts(x, self.gate, self.up, self.down, chosen, weights, s.activation)

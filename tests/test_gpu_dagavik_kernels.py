@@ -468,3 +468,45 @@ def test_experts_of_prompts_on_large_tiles(H, F):
     both = K().moe_experts(device_x, gate.to(DEV), up.to(DEV), down.to(DEV), chosen[:, None].expand(-1, 2).contiguous().to(DEV),
                            torch.cat([weights * 0.25, weights * 0.75], -1).contiguous().to(DEV))
     close(both.sum(0), want.double(), 1.5e-2, f"experts twice {H} {F}")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("E,groups,keep,top,among,bias,shared", [(32, 4, 2, 4, False, False, 0), (33, 1, 1, 3, True, True, 1),
+                                                                 (70, 7, 3, 5, False, True, 0), (300, 1, 1, 8, True, False, 2), (1, 1, 1, 1, False, False, 0)])
+def test_choosing_in_one_launch_gives_the_bits_of_two(dtype, E, groups, keep, top, among, bias, shared):
+    """Logits and routing by one workgroup a token against the projection and the routing by themselves: outputs that do not fill a
+    wavefront's eight, widths that end inside a trip, 1 to 256 tokens, rows wider apart than they are long, equal logits."""
+    lib = K()
+    gen = torch.Generator().manual_seed(E)
+    for T, H in ((1, 8), (7, 1536), (33, 520), (256, 64)):
+        x = torch.empty((T, H + 8), dtype=dtype, device=DEV)[:, :H].copy_(torch.randn((T, H), generator=gen))
+        router = (torch.randn((E + (1 if shared else 0), H), generator=gen) * H ** -0.5).to(dtype).to(DEV)
+        if E > 4:
+            router[3] = router[1]  # two experts with the same logits
+        b = torch.randn(router.shape[0], generator=gen).to(DEV) if among else None
+        if b is not None and E > 4:
+            b[3] = b[1]
+        choice = torch.randn(E, generator=gen).mul_(0.01).to(DEV) if bias and not among else None
+        options = (groups, keep, top, 1.7, choice, among, shared)
+        assert lib.library().pae_moe_choose_takes(lib.code_of(dtype), x.data_ptr(), x.stride(0), router.data_ptr(), T, H)
+        got, want = lib.moe_choose(x, router, b, *options), lib.moe_route(lib.project_f32(x, router, b), *options)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]), (T, H)
+
+
+@pytest.mark.parametrize("T,E,top", [(1, 5, 3), (7, 33, 4), (16, 2, 2), (17, 2, 2), (32, 3, 3), (32, 40, 8)])
+def test_experts_of_a_few_tokens_by_lists_of_their_own(T, E, top):
+    """Steps of up to 32 tokens and 256 pairs, where every workgroup looks its expert's pairs up itself: experts that all
+    tokens chose (two sixteens of rows), experts that none did; against the same tokens inside a step of more pairs,
+    which are sorted first: the same bits."""
+    gen = torch.Generator().manual_seed(T + E)
+    H, F = 96, 160
+    gate, up = ((torch.randn((E, F, H), generator=gen) * 0.2).to(torch.bfloat16).to(DEV) for _ in range(2))
+    down = (torch.randn((E, H, F), generator=gen) * 0.2).to(torch.bfloat16).to(DEV)
+    x = torch.randn((300, H), generator=gen).to(torch.bfloat16).to(DEV)
+    chosen = torch.stack([torch.randperm(E, generator=gen)[:top] for _ in range(300)]).to(torch.int32).to(DEV)
+    weights = torch.rand((300, top), generator=gen).to(DEV)
+    few = K().moe_experts(x[:T], gate, up, down, chosen[:T].contiguous(), weights[:T].contiguous())
+    n = max(33, 256 // top + 1)  # more than 256 pairs or 32 tokens, at most 512 pairs: the same kernel behind the sort
+    assert n * top <= 512
+    many = K().moe_experts(x[:n], gate, up, down, chosen[:n].contiguous(), weights[:n].contiguous())
+    assert torch.equal(few, many[:, :T])
