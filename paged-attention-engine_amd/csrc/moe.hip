@@ -623,7 +623,10 @@ __global__ __launch_bounds__(256) void moe_tiles_down_kernel(float* __restrict__
 // tokens and its weights are streamed exactly once: a tile is up to 16 rows, and the four wavefronts of a workgroup share
 // one tile of 16 features and take a quarter of k each, leave their sums in LDS, and the first adds them in wavefront
 // order (a wavefront per 16 features and the whole of k was measured against it: 35 + 22 us against 25 + 14 at one
-// token, 85 + 57 against 67 + 39 at eight).  The order of adding is a function of the sizes alone.
+// token, 85 + 57 against 67 + 39 at eight).  The order of adding is a function of the sizes alone.  A wavefront asks for
+// four steps of 32 at once and works on the four before: a row's lines are whole in one batch (a step has half of
+// each), and 4 to 8 KB of a wavefront are on their way (7 tokens by four of 32 experts, 1,536 x 2,240, 267 and 133 MB
+// of weights: 63.6 + 36.0 -> 59.3 + 34.7 us, of 4 tokens 49.7 + 31.7 -> 44.6 + 26.2; the weights' stream bounds it).
 //
 // In steps of up to 32 tokens and 256 pairs (LISTED) no sorting comes first: a workgroup belongs to an expert (blockIdx.x), a
 // block of features and a sixteen of its rows (blockIdx.z), and looks its pairs up itself, in their order (two
@@ -635,6 +638,7 @@ __global__ __launch_bounds__(256) void moe_few_tiles_kernel(bf16_t* __restrict__
                                                             const int* __restrict__ order, const float* __restrict__ weights,
                                                             const int4* __restrict__ tiles, int top, int num_tokens, int K,
                                                             int N, int act_kind) {
+  constexpr int BATCH = 4;
   __shared__ f32x4 parts[3][2][PAE_WAVE];
   __shared__ int pair_of[16], of_wave[4];
   const int lane = threadIdx.x % PAE_WAVE, wave = threadIdx.x / PAE_WAVE;
@@ -671,20 +675,43 @@ __global__ __launch_bounds__(256) void moe_few_tiles_kernel(bf16_t* __restrict__
   const int steps = K / 32, per = (steps + 3) / 4;
   const int first = wave * per, last = min(steps, first + per);
   f32x4 s1 = {0.f, 0.f, 0.f, 0.f}, s2 = {0.f, 0.f, 0.f, 0.f};
-  if (first < last) {
-    bf16x8 ca = *reinterpret_cast<const bf16x8*>(a + 32 * first), c1 = *reinterpret_cast<const bf16x8*>(w1 + 32 * first), c2;
-    if (GATED) c2 = *reinterpret_cast<const bf16x8*>(w2 + 32 * first);
-    for (int st = first + 1; st < last; ++st) {
-      const bf16x8 na = *reinterpret_cast<const bf16x8*>(a + 32 * st), n1 = *reinterpret_cast<const bf16x8*>(w1 + 32 * st);
-      bf16x8 n2;
-      if (GATED) n2 = *reinterpret_cast<const bf16x8*>(w2 + 32 * st);
-      s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c1, ca, s1, 0, 0, 0);
-      if (GATED) s2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c2, ca, s2, 0, 0, 0);
-      ca = na; c1 = n1;
-      if (GATED) c2 = n2;
+  const auto load = [](const bf16_t* p) { return *reinterpret_cast<const bf16x8*>(p); };
+  bf16x8 ca[BATCH], c1[BATCH], c2[BATCH], na[BATCH], n1[BATCH], n2[BATCH];
+  const int batches = (last - first) / BATCH;
+  if (batches > 0) {
+#pragma unroll
+    for (int i = 0; i < BATCH; ++i) {
+      c1[i] = load(w1 + 32 * (first + i));
+      if (GATED) c2[i] = load(w2 + 32 * (first + i));
     }
-    s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c1, ca, s1, 0, 0, 0);
-    if (GATED) s2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c2, ca, s2, 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < BATCH; ++i) ca[i] = load(a + 32 * (first + i));
+  }
+  for (int b = 0; b < batches; ++b) {
+    const int next = first + BATCH * min(b + 1, batches - 1);  // (the last batch asks for its own lines again)
+#pragma unroll
+    for (int i = 0; i < BATCH; ++i) {
+      n1[i] = load(w1 + 32 * (next + i));
+      if (GATED) n2[i] = load(w2 + 32 * (next + i));
+    }
+#pragma unroll
+    for (int i = 0; i < BATCH; ++i) na[i] = load(a + 32 * (next + i));
+    __builtin_amdgcn_sched_barrier(0);  // (asked for before the products, or the loads would sink behind them)
+#pragma unroll
+    for (int i = 0; i < BATCH; ++i) {
+      s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c1[i], ca[i], s1, 0, 0, 0);
+      if (GATED) s2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c2[i], ca[i], s2, 0, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < BATCH; ++i) {
+      ca[i] = na[i]; c1[i] = n1[i];
+      if (GATED) c2[i] = n2[i];
+    }
+  }
+  for (int st = first + batches * BATCH; st < last; ++st) {
+    const bf16x8 x = load(a + 32 * st), g = load(w1 + 32 * st);
+    s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(g, x, s1, 0, 0, 0);
+    if (GATED) s2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(load(w2 + 32 * st), x, s2, 0, 0, 0);
   }
   if (wave > 0) {
     parts[wave - 1][0][lane] = s1;

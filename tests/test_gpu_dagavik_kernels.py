@@ -510,3 +510,24 @@ def test_experts_of_a_few_tokens_by_lists_of_their_own(T, E, top):
     assert n * top <= 512
     many = K().moe_experts(x[:n], gate, up, down, chosen[:n].contiguous(), weights[:n].contiguous())
     assert torch.equal(few, many[:, :T])
+
+
+@pytest.mark.parametrize("H,F", [(32, 512), (512, 32), (480, 544), (1568, 736), (2240, 96)])
+def test_experts_of_a_few_tokens_at_the_edges_of_a_batch_of_k(H, F):
+    """Four wavefronts share k in steps of 32, four steps to a batch: fewer than a batch each, whole batches, steps left over, a
+    last wavefront with less than the others.  Against 64 bits: products of bfloat16 numbers summed in float32, the
+    activations rounded once to bfloat16 (2^-8 of a number with random signs, so a few times 2^-8 of the largest sum)."""
+    gen = torch.Generator().manual_seed(H + F)
+    E, T, top = 3, 5, 2
+    gate, up = ((torch.randn((E, F, H), generator=gen) * H ** -0.5).to(torch.bfloat16) for _ in range(2))
+    down = (torch.randn((E, H, F), generator=gen) * F ** -0.5).to(torch.bfloat16)
+    x = torch.randn((T, H), generator=gen).to(torch.bfloat16)
+    chosen = torch.stack([torch.randperm(E, generator=gen)[:top] for _ in range(T)]).to(torch.int32)
+    weights = torch.rand((T, top), generator=gen)
+    got = K().moe_experts(x.to(DEV), gate.to(DEV), up.to(DEV), down.to(DEV), chosen.to(DEV), weights.to(DEV)).cpu().double().sum(0)
+    want = torch.zeros(T, H, dtype=torch.float64)
+    for t in range(T):
+        for e, w in zip(chosen[t].tolist(), weights[t].tolist()):
+            g, u = gate[e].double() @ x[t].double(), up[e].double() @ x[t].double()
+            want[t] += w * (down[e].double() @ (g * torch.sigmoid(g) * u))
+    assert float((got - want).abs().max()) <= 4 * 2.0 ** -8 * float(want.abs().max())
