@@ -18,6 +18,8 @@
 
 #define CONV_THREADS 128
 #define CONV_PER_THREAD 8  // head widths up to CONV_THREADS * CONV_PER_THREAD
+#define CONV_ROWS 8        // rows of a prompt that a wavefront takes
+#define CONV_ROWS_FROM 256 // steps of fewer rows leave most of the chip idle by wavefronts of eight
 
 // seq_runs[s] = (first flat row, rows in this step, tokens held before the step, unused)
 // One workgroup per (token, head): the q heads, then the k heads, then the v heads.
@@ -94,6 +96,120 @@ __global__ __launch_bounds__(CONV_THREADS) void conv_norm_store_kernel(
   }
 }
 
+// The same bits for the many rows of a prompt: a wavefront takes one head of eight consecutive rows, lane i its features i and
+// i + 64 (head widths up to 128).  The kernel above reads every row once per tap and every weight once per row, a
+// number a thread, and waits for each; here the rows, the TAPS - 1 before them and the weights are asked for at once,
+// a row's inputs are taken from registers, and eight values of a feature go to a page of V in one store where they lie
+// together.  Inputs from before the step come from the state, in the first TAPS - 1 rows of a run only.
+// Measured, 8,192 rows, 12 + 2 + 2 heads of 128, four taps: 146 -> 35 us (queries and keys, or 12 query heads only: 94 -> 27); 67 MB move, and issuing the
+// sums and norms bounds it now.
+template <typename T, int TAPS>
+__global__ __launch_bounds__(256) void conv_norm_store_rows_kernel(
+    const T* __restrict__ proj, int64_t row_stride, T* __restrict__ q_out, int64_t q_stride,
+    const int* __restrict__ tok_seq, const int* __restrict__ positions, const int4* __restrict__ seq_runs,
+    const int* __restrict__ slots, const float* __restrict__ conv_w, const float* __restrict__ conv_tail,
+    int64_t tail_slot_stride, int num_tokens, int nh, int nkv, int hd, int vd, int norm_heads, float eps,
+    const int* __restrict__ block_tables, int max_blocks, int bs, T* __restrict__ k_cache, T* __restrict__ v_cache) {
+  constexpr int ROWS = CONV_ROWS, N = 2;
+  struct alignas(16) Eight { T v[ROWS]; };
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / PAE_WAVE), lane = threadIdx.x % PAE_WAVE;
+  const int t0 = ((int)blockIdx.x * 4 + wave) * ROWS, seg = blockIdx.y;
+  if (t0 >= num_tokens) return;
+  const int C = nh * hd + nkv * (hd + vd);
+  const bool is_q = seg < nh, is_v = seg >= nh + nkv;
+  const int width = is_v ? vd : hd;
+  const int c0 = is_v ? (nh + nkv) * hd + (seg - nh - nkv) * vd : seg * hd;
+  T x[ROWS + TAPS - 1][N];
+  float w[N][TAPS];
+  int seq[ROWS], pos[ROWS], first[ROWS];
+  int64_t block[ROWS];
+#pragma unroll
+  for (int r = 0; r < ROWS + TAPS - 1; ++r) {
+    const int64_t row = min(max(t0 - (TAPS - 1) + r, 0), num_tokens - 1);
+#pragma unroll
+    for (int n = 0; n < N; ++n) x[r][n] = proj[row * row_stride + c0 + min(lane + PAE_WAVE * n, width - 1)];
+  }
+#pragma unroll
+  for (int n = 0; n < N; ++n)
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j) w[n][j] = conv_w[(int64_t)(c0 + min(lane + PAE_WAVE * n, width - 1)) * TAPS + j];
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r) {
+    const int t = min(t0 + r, num_tokens - 1);
+    seq[r] = tok_seq[t];
+    pos[r] = positions[t];
+  }
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r) {
+    first[r] = seq_runs[seq[r]].x;
+    block[r] = is_q ? 0 : block_tables[(int64_t)seq[r] * max_blocks + pos[r] / bs];
+  }
+  const int rows = min(ROWS, num_tokens - t0);
+  T kept[ROWS][N];
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r) {
+    const int in_step = min(t0 + r, num_tokens - 1) - first[r];  // rows of this sequence before this one in the step
+    float mine[N], ss[N];
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+      const int i = lane + PAE_WAVE * n;
+      float sum = 0.f;
+#pragma unroll
+      for (int j = 0; j < TAPS; ++j) {
+        const int back = TAPS - 1 - j;  // tap j weighs the input `back` tokens ago
+        float in = to_f32(x[r + j][n]);
+        if (back > in_step)
+          in = conv_tail[(int64_t)slots[seq[r]] * tail_slot_stride + (int64_t)(TAPS - 1 - (back - in_step)) * C + c0 + min(i, width - 1)];
+        sum = fmaf(w[n][j], in, sum);
+      }
+      mine[n] = i < width ? sum : 0.f;
+      ss[n] = fmaf(mine[n], mine[n], 0.f);
+    }
+    float inv = 1.f;
+    if (norm_heads && !is_v) {  // (the halves of a head are added as the two wavefronts' sums above)
+      float total = 0.f;
+      total += wave_sum(ss[0]);
+      total += wave_sum(ss[1]);
+      inv = 1.0f / sqrtf(total / (float)hd + eps);
+    }
+#pragma unroll
+    for (int n = 0; n < N; ++n) kept[r][n] = from_f32<T>(is_v ? mine[n] : mine[n] * inv);
+  }
+  if (is_v) {
+    const int off = pos[0] % bs;
+    T* head = v_cache + (int64_t)(seg - nh - nkv) * vd * bs;
+    if (rows == ROWS && seq[0] == seq[ROWS - 1] && pos[ROWS - 1] - pos[0] == ROWS - 1 && off % ROWS == 0 && bs % ROWS == 0) {
+#pragma unroll
+      for (int n = 0; n < N; ++n) {
+        const int i = lane + PAE_WAVE * n;
+        if (i >= width) continue;
+        Eight all;
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) all.v[r] = kept[r][n];
+        *reinterpret_cast<Eight*>(head + block[0] * nkv * (int64_t)vd * bs + (int64_t)i * bs + off) = all;
+      }
+      return;
+    }
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+      for (int n = 0; n < N; ++n) {
+        const int i = lane + PAE_WAVE * n;
+        if (r < rows && i < width) head[block[r] * nkv * (int64_t)vd * bs + (int64_t)i * bs + pos[r] % bs] = kept[r][n];
+      }
+    return;
+  }
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r) {
+    if (r >= rows) break;
+    T* dst = is_q ? q_out + (int64_t)(t0 + r) * q_stride + (int64_t)seg * hd
+                  : k_cache + ((block[r] * nkv + (seg - nh)) * bs + pos[r] % bs) * hd;
+#pragma unroll
+    for (int n = 0; n < N; ++n)
+      if (lane + PAE_WAVE * n < width) dst[lane + PAE_WAVE * n] = kept[r][n];
+  }
+}
+
 // The state's last taps - 1 inputs moved on by the step's rows: entry j of the new tail is the input
 // at (end of step) - keep + j, a row of this step or an entry further on in the old tail (read before
 // any entry at or above it is written: j ascends).
@@ -135,9 +251,21 @@ extern "C" int pae_conv_norm_store(int dtype, const void* proj, int64_t row_stri
   if (num_tokens <= 0) return 0;
   dim3 grid(num_tokens, nh + 2 * nkv);
   dim3 tail_grid((unsigned)((C + 255) / 256), num_seqs);
+  // many rows, heads that two numbers a lane hold, the usual numbers of taps: by wavefronts of eight rows
+  const bool by_rows = num_tokens >= CONV_ROWS_FROM && hd <= 2 * PAE_WAVE && vd <= 2 * PAE_WAVE && taps >= 2 && taps <= 4 &&
+                       (uintptr_t)v_cache % 16 == 0;
+  const dim3 rows_grid((num_tokens + 4 * CONV_ROWS - 1) / (4 * CONV_ROWS), nh + 2 * nkv);
+#define CONV_ROWS_LAUNCH(T, TAPS)                                                                                         \
+  conv_norm_store_rows_kernel<T, TAPS><<<rows_grid, 256, 0, stream>>>(                                                    \
+      (const T*)proj, row_stride, (T*)q_out, q_stride, tok_seq, positions, (const int4*)seq_runs, slots, conv_w,          \
+      conv_tail, tail_slot_stride, num_tokens, nh, nkv, hd, vd, norm_heads, eps, block_tables, max_blocks, bs,            \
+      (T*)k_cache, (T*)v_cache)
 #define CONV_LAUNCH(T)                                                                                                  \
   do {                                                                                                                  \
-    conv_norm_store_kernel<T><<<grid, CONV_THREADS, 0, stream>>>(                                                       \
+    if (by_rows && taps == 2) CONV_ROWS_LAUNCH(T, 2);                                                                   \
+    else if (by_rows && taps == 3) CONV_ROWS_LAUNCH(T, 3);                                                              \
+    else if (by_rows) CONV_ROWS_LAUNCH(T, 4);                                                                           \
+    else conv_norm_store_kernel<T><<<grid, CONV_THREADS, 0, stream>>>(                                                       \
         (const T*)proj, row_stride, (T*)q_out, q_stride, tok_seq, positions, (const int4*)seq_runs, slots, conv_w,      \
         conv_tail, tail_slot_stride, taps, nh, nkv, hd, vd, norm_heads, eps, block_tables, max_blocks, bs, (T*)k_cache, \
         (T*)v_cache);                                                                                                   \
@@ -149,5 +277,6 @@ extern "C" int pae_conv_norm_store(int dtype, const void* proj, int64_t row_stri
   else if (dtype == PAE_BF16) CONV_LAUNCH(bf16_t);
   else return pae_fail("conv_norm_store: unknown dtype code %d", dtype);
 #undef CONV_LAUNCH
+#undef CONV_ROWS_LAUNCH
   return pae_check_launch("conv_norm_store");
 }
