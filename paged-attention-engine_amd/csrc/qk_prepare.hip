@@ -104,7 +104,7 @@ __global__ __launch_bounds__(256) void qk_norm_rotate_store_kernel(
 // The same for rows that can be read 16 bytes at a time (head sizes in multiples of a chunk of 16 bytes, rows on such
 // boundaries): a thread has a chunk of neighbouring features of one head.  The row, the weights and the angles are all asked
 // for before the sums are known; the row goes to LDS in float32 once, where the sums per head and the other
-// half of a rotated pair find it.  On a few tokens the kernel above takes four trips to memory, number by number.
+// half of a rotated pair find it (the same bits).  On a few tokens the kernel above takes four trips to memory, number by number.
 // Measured, 12 query and 2 key heads of 128, bfloat16: 9 rows 11.5 -> 6.5 us, with one sum over each projection 10.5 -> 6.4.
 // (A row of more than 1,024 chunks or 64 KB in float32 stays above.)
 template <typename T, int TRIPS>  // at most 256 * TRIPS chunks of queries and keys
@@ -118,7 +118,7 @@ __global__ __launch_bounds__(256) void qk_norm_rotate_store_vec_kernel(
   constexpr int N = 16 / sizeof(T);
   struct alignas(16) Chunk { T v[N]; };
   extern __shared__ float row_lds[];  // [nh + nkv][hd] the row, [nh + nkv] what its heads are multiplied by
-  __shared__ float scratch[2][4];
+  __shared__ float scratch[4];
   const int t = blockIdx.x, tid = threadIdx.x;
   T* row = qkv + (int64_t)t * row_stride;
   const int nq = nh * hd, nk = nkv * hd, per = hd / N;  // chunks a head
@@ -158,7 +158,7 @@ __global__ __launch_bounds__(256) void qk_norm_rotate_store_vec_kernel(
     }
   }
   float inv_q = 1.f, inv_k = 1.f;
-  if (q_w && per_head) {
+  if (q_w) {
 #pragma unroll
     for (int r = 0; r < TRIPS; ++r) {
       const int c = tid + 256 * r;
@@ -167,41 +167,27 @@ __global__ __launch_bounds__(256) void qk_norm_rotate_store_vec_kernel(
         for (int i = 0; i < N; ++i) row_lds[c * N + i] = to_f32(x[r].v[i]);
     }
     __syncthreads();
-    // a wavefront a head in turn, lanes and order as in the kernel above: the same bits
-    const int wave = tid / PAE_WAVE, lane = tid % PAE_WAVE;
-    for (int h = wave; h < nh + nkv; h += 4) {
-      float ss = 0.f;
-      for (int i = lane; i < hd; i += PAE_WAVE) ss = fmaf(row_lds[h * hd + i], row_lds[h * hd + i], ss);
-      ss = wave_sum(ss);
-      if (lane == 0) head_inv[h] = 1.0f / sqrtf(ss / (float)hd + eps);
+    // the sums by the lanes and in the order of the kernel above: the same bits
+    if (per_head) {  // a wavefront a head in turn
+      const int wave = tid / PAE_WAVE, lane = tid % PAE_WAVE;
+      for (int h = wave; h < nh + nkv; h += 4) {
+        float ss = 0.f;
+        for (int i = lane; i < hd; i += PAE_WAVE) ss = fmaf(row_lds[h * hd + i], row_lds[h * hd + i], ss);
+        ss = wave_sum(ss);
+        if (lane == 0) head_inv[h] = 1.0f / sqrtf(ss / (float)hd + eps);
+      }
+    } else {  // one sum for all queries, one for all keys
+      float sq = 0.f, sk = 0.f;
+      for (int i = tid; i < nq; i += 256) sq = fmaf(row_lds[i], row_lds[i], sq);
+      for (int i = tid; i < nk; i += 256) sk = fmaf(row_lds[nq + i], row_lds[nq + i], sk);
+      sq = block_sum<4>(sq, scratch);
+      inv_q = 1.0f / sqrtf(sq / (float)nq + eps);
+      if (nk) {
+        sk = block_sum<4>(sk, scratch);
+        inv_k = 1.0f / sqrtf(sk / (float)nk + eps);
+      }
     }
     __syncthreads();
-  } else if (q_w) {  // one sum for all queries, one for all keys
-    float sq = 0.f, sk = 0.f;
-#pragma unroll
-    for (int r = 0; r < TRIPS; ++r) {
-      const int c = tid + 256 * r;
-      float ss = 0.f;
-#pragma unroll
-      for (int i = 0; i < N; ++i) ss = fmaf(to_f32(x[r].v[i]), to_f32(x[r].v[i]), ss);
-      if (c < nh * per) sq += ss;
-      else if (c < chunks) sk += ss;
-    }
-    sq = wave_sum(sq);
-    sk = wave_sum(sk);
-    if (tid % PAE_WAVE == 0) {
-      scratch[0][tid / PAE_WAVE] = sq;
-      scratch[1][tid / PAE_WAVE] = sk;
-    }
-    __syncthreads();
-    sq = sk = 0.f;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      sq += scratch[0][v];
-      sk += scratch[1][v];
-    }
-    inv_q = 1.0f / sqrtf(sq / (float)nq + eps);
-    inv_k = nk ? 1.0f / sqrtf(sk / (float)nk + eps) : 1.f;
   }
   float value[TRIPS][N];  // normalised
 #pragma unroll
