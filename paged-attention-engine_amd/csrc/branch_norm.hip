@@ -10,6 +10,7 @@
 // float32 partial sums [parts][rows][hidden] of a product split along k, added here in order.
 #include "common.h"
 #include "api.h"
+#include "row_pieces.h"
 
 template <typename T>
 __global__ void rows_from_residual_kernel(T* __restrict__ out, const float* __restrict__ residual, int64_t n) {
@@ -124,6 +125,52 @@ __global__ __launch_bounds__(256) void norm_scale_add_vec_kernel(float* __restri
   }
 }
 
+// The same bits for up to seven parts and widths up to 1,024 * TRIPS: the kernel above waits for one part before it asks for the
+// next, and for the weight number by number; here all of them are asked for as raw bits.  One row of 1,536:
+// 5.0 -> 4.1 us; six rows 6.2 -> 4.8 us.
+template <typename T, int TRIPS>
+__global__ __launch_bounds__(256) void norm_scale_add_few_trips_kernel(float* __restrict__ residual, row_pieces::Pieces pieces,
+                                                                       const void* __restrict__ weight, int w_is_f32, float eps,
+                                                                       float scale, T* __restrict__ next, int hidden) {
+  __shared__ float scratch[4];
+  const int64_t base = (int64_t)blockIdx.x * hidden;
+  uint4 raw[TRIPS][row_pieces::PIECES], raw_r[TRIPS], raw_w[TRIPS];
+  int at[TRIPS];
+#pragma unroll
+  for (int c = 0; c < TRIPS; ++c) {
+    const int i = (threadIdx.x + 256 * c) * 4;
+    at[c] = i < hidden ? i : -1;
+    const int from = i < hidden ? i : 0;  // a thread beyond the row reads its start and adds nothing
+    row_pieces::ask_all<T>(pieces, blockIdx.x, from, raw[c]);
+    raw_r[c] = row_pieces::ask(residual, base + from, true);
+    raw_w[c] = row_pieces::ask(weight, from, w_is_f32);
+  }
+  float y[TRIPS][4];
+  float ss = 0.f;
+#pragma unroll
+  for (int c = 0; c < TRIPS; ++c) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) y[c][e] = 0.f;
+    row_pieces::add_all<T>(pieces, raw[c], y[c]);
+    if (at[c] >= 0)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) ss = fmaf(y[c][e], y[c][e], ss);
+  }
+  const float total = block_sum<4>(ss, scratch);
+  const float inv = 1.0f / sqrtf(total / (float)hidden + eps);
+#pragma unroll
+  for (int c = 0; c < TRIPS; ++c) {
+    if (at[c] < 0) continue;
+    float r[4], w[4];
+    row_pieces::numbers(raw_r[c], true, r);
+    row_pieces::numbers(raw_w[c], w_is_f32, w);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) r[e] = r[e] + scale * (y[c][e] * inv * w[e]);
+    row_pieces::put4(residual + base + at[c], r);
+    if (next) row_pieces::put4(next + base + at[c], r);
+  }
+}
+
 extern "C" int pae_norm_scale_add(int dtype, float* residual, const void* y, int parts, int64_t part_stride,
                                   const void* weight, int w_is_f32, float eps, float scale, void* next, int num_rows,
                                   int hidden, hipStream_t stream) {
@@ -132,6 +179,28 @@ extern "C" int pae_norm_scale_add(int dtype, float* residual, const void* y, int
   if (num_rows == 0) return 0;
   const size_t lds = hidden <= 8192 ? (size_t)hidden * sizeof(float) : 0;
   if (hidden % 4 == 0 && hidden <= 4096 && part_stride % 4 == 0 && (dtype == PAE_F32 || dtype == PAE_BF16)) {
+    const int f32 = parts > 0 || dtype == PAE_F32, count = parts > 0 ? parts : 1;
+    const int64_t row_stride = hidden;
+    const float one = 1.f;
+    auto aligned = [](const void* p) { return (uintptr_t)p % 16 == 0; };
+    row_pieces::Pieces pieces;
+    if (aligned(residual) && aligned(y) && aligned(weight) && aligned(next) &&
+        row_pieces::flatten(pieces, 1, &y, &f32, &count, &part_stride, &row_stride, &one)) {
+#define SCALE_ADD_TRIPS(T, TRIPS) \
+  norm_scale_add_few_trips_kernel<T, TRIPS><<<num_rows, 256, 0, stream>>>(residual, pieces, weight, w_is_f32, eps, scale, (T*)next, hidden)
+#define SCALE_ADD_FEW(T)                          \
+  if (hidden <= 1024) SCALE_ADD_TRIPS(T, 1);      \
+  else if (hidden <= 2048) SCALE_ADD_TRIPS(T, 2); \
+  else SCALE_ADD_TRIPS(T, 4);
+      if (dtype == PAE_F32) {
+        SCALE_ADD_FEW(float)
+      } else {
+        SCALE_ADD_FEW(bf16_t)
+      }
+#undef SCALE_ADD_FEW
+#undef SCALE_ADD_TRIPS
+      return pae_check_launch("norm_scale_add");
+    }
     if (dtype == PAE_F32)
       norm_scale_add_vec_kernel<float><<<num_rows, 256, 0, stream>>>(residual, y, parts, part_stride, weight, w_is_f32,
                                                                      eps, scale, (float*)next, hidden);
