@@ -628,114 +628,137 @@ __global__ __launch_bounds__(256) void moe_tiles_down_kernel(float* __restrict__
 // each), and 4 to 8 KB of a wavefront are on their way (7 tokens by four of 32 experts, 1,536 x 2,240, 267 and 133 MB
 // of weights: 63.6 + 36.0 -> 59.3 + 34.7 us, of 4 tokens 49.7 + 31.7 -> 44.6 + 26.2; the weights' stream bounds it).
 //
-// In steps of up to 32 tokens and 256 pairs (LISTED) no sorting comes first: a workgroup belongs to an expert (blockIdx.x), a
-// block of features and a sixteen of its rows (blockIdx.z), and looks its pairs up itself, in their order (two
-// barriers, against a launch of 6 us and the same trip to memory for the tile); activations lie at their pair's number.
-template <bool GATED, bool LISTED>
+// In steps of up to 32 tokens and 256 pairs no sorting comes first: a workgroup looks its expert's pairs up itself, in their
+// order (two barriers, against a launch of 6 us, 30 with 256 experts, and the same trip to memory for the tile);
+// activations lie at their pair's number.  Nothing is assumed about how often a token names an expert: routing names one
+// several times where no logit compares.
+//   BY_PAIR    blockIdx.x is a pair; the workgroup takes the sixteen of its expert's pairs that begins with it, if one does
+//   BY_EXPERT  blockIdx.x is an expert; the workgroups along blockIdx.z take its sixteens in turn
+// What either costs over the weights' stream is its workgroups without work, so the list with fewer of them is taken:
+// pairs up to the number of experts, else experts.
+enum { SORTED, BY_PAIR, BY_EXPERT };
+template <bool GATED, int LIST>
 __global__ __launch_bounds__(256) void moe_few_tiles_kernel(bf16_t* __restrict__ act_out, float* __restrict__ y,
                                                             const bf16_t* __restrict__ a_rows, int64_t lda,
                                                             const bf16_t* __restrict__ w_first, const bf16_t* __restrict__ w_second,
                                                             const int* __restrict__ order, const float* __restrict__ weights,
-                                                            const int4* __restrict__ tiles, int top, int num_tokens, int K,
-                                                            int N, int act_kind) {
+                                                            const int4* __restrict__ tiles, int experts, int top, int num_tokens,
+                                                            int K, int N, int act_kind) {
   constexpr int BATCH = 4;
   __shared__ f32x4 parts[3][2][PAE_WAVE];
-  __shared__ int pair_of[16], of_wave[4];
+  __shared__ int pair_of[16];
+  __shared__ uint64_t of_wave[4];
   const int lane = threadIdx.x % PAE_WAVE, wave = threadIdx.x / PAE_WAVE;
   const int col = lane % 16, kg = lane / 16;
   const int n0 = blockIdx.y * 16;
   int4 tile;  // (expert, first sorted row, rows <= 16, unused)
-  if (LISTED) {  // order: the pairs' experts
-    const bool mine = (int)threadIdx.x < num_tokens * top && order[threadIdx.x] == (int)blockIdx.x;
-    const uint64_t found = __ballot(mine);
-    if (lane == 0) of_wave[wave] = __popcll(found);
-    __syncthreads();
-    int before = 0, all = 0;
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      if (w < wave) before += of_wave[w];
-      all += of_wave[w];
-    }
-    const int place = before + __popcll(found & ((1ull << lane) - 1)) - (int)blockIdx.z * 16;
-    if (mine && place >= 0 && place < 16) pair_of[place] = threadIdx.x;
-    tile = make_int4(blockIdx.x, 0, min(16, all - (int)blockIdx.z * 16), 0);
-    if (tile.z <= 0) return;
-    __syncthreads();
-  } else {
+  int place = -1, from = 0, all = 0;  // this thread's pair among its expert's, where the sixteen begins, how many there are
+  if (LIST == SORTED) {
     tile = tiles[blockIdx.x];
     if (tile.z <= 0) return;
+  } else {  // order: the pairs' experts
+    const int self = blockIdx.x, pairs = num_tokens * top;
+    const int expert = LIST == BY_PAIR ? order[min(self, pairs - 1)] : self;
+    const bool mine = (int)threadIdx.x < pairs && order[threadIdx.x] == expert;
+    const uint64_t found = __ballot(mine);
+    if (lane == 0) of_wave[wave] = found;
+    __syncthreads();
+    int before = 0;  // of the expert's pairs, those of the wavefronts before
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const uint64_t there = of_wave[w];
+      const int ahead = self - w * PAE_WAVE;  // of the wavefront's pairs, those before the workgroup's own
+      if (w < wave) before += __popcll(there);
+      if (LIST == BY_PAIR) from += __popcll(ahead >= PAE_WAVE ? there : ahead > 0 ? there & ((1ull << ahead) - 1) : 0);
+      all += __popcll(there);
+    }
+    if (LIST == BY_EXPERT) from = blockIdx.z * 16;
+    if ((LIST == BY_PAIR && self >= pairs) || from % 16 || from >= all || (unsigned)expert >= (unsigned)experts) return;
+    if (mine) place = before + __popcll(found & ((1ull << lane) - 1));
+    tile = make_int4(expert, 0, 0, 0);
   }
   if (n0 >= N) return;
-  const int sorted = LISTED ? pair_of[col < tile.z ? col : 0] : tile.y + (col < tile.z ? col : 0);
-  const int pair = LISTED ? sorted : order[sorted];  // where a result goes: row `sorted` of the activations, the pair's of y
-  const int64_t w_row = (int64_t)tile.x * N + min(n0 + col, N - 1);
-  const bf16_t* w1 = w_first + w_row * K + 8 * kg;
-  const bf16_t* w2 = GATED ? w_second + w_row * K + 8 * kg : nullptr;
-  const bf16_t* a = a_rows + (int64_t)(GATED ? pair / top : sorted) * lda + 8 * kg;
-  const int steps = K / 32, per = (steps + 3) / 4;
-  const int first = wave * per, last = min(steps, first + per);
-  f32x4 s1 = {0.f, 0.f, 0.f, 0.f}, s2 = {0.f, 0.f, 0.f, 0.f};
-  const auto load = [](const bf16_t* p) { return *reinterpret_cast<const bf16x8*>(p); };
-  bf16x8 ca[BATCH], c1[BATCH], c2[BATCH], na[BATCH], n1[BATCH], n2[BATCH];
-  const int batches = (last - first) / BATCH;
-  if (batches > 0) {
-#pragma unroll
-    for (int i = 0; i < BATCH; ++i) {
-      c1[i] = load(w1 + 32 * (first + i));
-      if (GATED) c2[i] = load(w2 + 32 * (first + i));
+  while (true) {  // (once, but BY_EXPERT)
+    if (LIST != SORTED) {
+      tile.z = min(16, all - from);
+      if (place >= from && place < from + 16) pair_of[place - from] = threadIdx.x;
+      __syncthreads();
     }
+    const int sorted = LIST != SORTED ? pair_of[col < tile.z ? col : 0] : tile.y + (col < tile.z ? col : 0);
+    const int pair = LIST != SORTED ? sorted : order[sorted];  // where a result goes: row `sorted` of the activations, the pair's of y
+    const int64_t w_row = (int64_t)tile.x * N + min(n0 + col, N - 1);
+    const bf16_t* w1 = w_first + w_row * K + 8 * kg;
+    const bf16_t* w2 = GATED ? w_second + w_row * K + 8 * kg : nullptr;
+    const bf16_t* a = a_rows + (int64_t)(GATED ? pair / top : sorted) * lda + 8 * kg;
+    const int steps = K / 32, per = (steps + 3) / 4;
+    const int first = wave * per, last = min(steps, first + per);
+    f32x4 s1 = {0.f, 0.f, 0.f, 0.f}, s2 = {0.f, 0.f, 0.f, 0.f};
+    const auto load = [](const bf16_t* p) { return *reinterpret_cast<const bf16x8*>(p); };
+    bf16x8 ca[BATCH], c1[BATCH], c2[BATCH], na[BATCH], n1[BATCH], n2[BATCH];
+    const int batches = (last - first) / BATCH;
+    if (batches > 0) {
 #pragma unroll
-    for (int i = 0; i < BATCH; ++i) ca[i] = load(a + 32 * (first + i));
-  }
-  for (int b = 0; b < batches; ++b) {
-    const int next = first + BATCH * min(b + 1, batches - 1);  // (the last batch asks for its own lines again)
+      for (int i = 0; i < BATCH; ++i) {
+        c1[i] = load(w1 + 32 * (first + i));
+        if (GATED) c2[i] = load(w2 + 32 * (first + i));
+      }
 #pragma unroll
-    for (int i = 0; i < BATCH; ++i) {
-      n1[i] = load(w1 + 32 * (next + i));
-      if (GATED) n2[i] = load(w2 + 32 * (next + i));
+      for (int i = 0; i < BATCH; ++i) ca[i] = load(a + 32 * (first + i));
     }
+    for (int b = 0; b < batches; ++b) {
+      const int next = first + BATCH * min(b + 1, batches - 1);  // (the last batch asks for its own lines again)
 #pragma unroll
-    for (int i = 0; i < BATCH; ++i) na[i] = load(a + 32 * (next + i));
-    __builtin_amdgcn_sched_barrier(0);  // (asked for before the products, or the loads would sink behind them)
+      for (int i = 0; i < BATCH; ++i) {
+        n1[i] = load(w1 + 32 * (next + i));
+        if (GATED) n2[i] = load(w2 + 32 * (next + i));
+      }
 #pragma unroll
-    for (int i = 0; i < BATCH; ++i) {
-      s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c1[i], ca[i], s1, 0, 0, 0);
-      if (GATED) s2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c2[i], ca[i], s2, 0, 0, 0);
+      for (int i = 0; i < BATCH; ++i) na[i] = load(a + 32 * (next + i));
+      __builtin_amdgcn_sched_barrier(0);  // (asked for before the products, or the loads would sink behind them)
+#pragma unroll
+      for (int i = 0; i < BATCH; ++i) {
+        s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c1[i], ca[i], s1, 0, 0, 0);
+        if (GATED) s2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(c2[i], ca[i], s2, 0, 0, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < BATCH; ++i) {
+        ca[i] = na[i]; c1[i] = n1[i];
+        if (GATED) c2[i] = n2[i];
+      }
     }
-#pragma unroll
-    for (int i = 0; i < BATCH; ++i) {
-      ca[i] = na[i]; c1[i] = n1[i];
-      if (GATED) c2[i] = n2[i];
+    for (int st = first + batches * BATCH; st < last; ++st) {
+      const bf16x8 x = load(a + 32 * st), g = load(w1 + 32 * st);
+      s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(g, x, s1, 0, 0, 0);
+      if (GATED) s2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(load(w2 + 32 * st), x, s2, 0, 0, 0);
     }
-  }
-  for (int st = first + batches * BATCH; st < last; ++st) {
-    const bf16x8 x = load(a + 32 * st), g = load(w1 + 32 * st);
-    s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(g, x, s1, 0, 0, 0);
-    if (GATED) s2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(load(w2 + 32 * st), x, s2, 0, 0, 0);
-  }
-  if (wave > 0) {
-    parts[wave - 1][0][lane] = s1;
-    if (GATED) parts[wave - 1][1][lane] = s2;
-  }
-  __syncthreads();
-  if (wave > 0 || col >= tile.z) return;
+    if (wave > 0) {
+      parts[wave - 1][0][lane] = s1;
+      if (GATED) parts[wave - 1][1][lane] = s2;
+    }
+    __syncthreads();
+    if (wave == 0 && col < tile.z) {
 #pragma unroll
-  for (int w = 0; w < 3; ++w) {
-    s1 += parts[w][0][lane];
-    if (GATED) s2 += parts[w][1][lane];
-  }
-  const int n = n0 + 4 * kg;  // a lane holds features n .. n + 3 of the row col
-  if (GATED) {
-    bf16_t* o = act_out + (int64_t)sorted * N + n;
+      for (int w = 0; w < 3; ++w) {
+        s1 += parts[w][0][lane];
+        if (GATED) s2 += parts[w][1][lane];
+      }
+      const int n = n0 + 4 * kg;  // a lane holds features n .. n + 3 of the row col
+      if (GATED) {
+        bf16_t* o = act_out + (int64_t)sorted * N + n;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (n + i < N) o[i] = __float2bfloat16(act_of(s1[i], act_kind) * s2[i]);
-  } else {
-    const float weight = weights[pair];
-    float* o = y + ((int64_t)(pair % top) * num_tokens + pair / top) * N + n;
+        for (int i = 0; i < 4; ++i)
+          if (n + i < N) o[i] = __float2bfloat16(act_of(s1[i], act_kind) * s2[i]);
+      } else {
+        const float weight = weights[pair];
+        float* o = y + ((int64_t)(pair % top) * num_tokens + pair / top) * N + n;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (n + i < N) o[i] = weight * s1[i];
+        for (int i = 0; i < 4; ++i)
+          if (n + i < N) o[i] = weight * s1[i];
+      }
+    }
+    from += 16 * gridDim.z;
+    if (LIST != BY_EXPERT || from >= all) return;
+    // (every wavefront has read its pairs, and the first one reads the sums before it comes to the next barrier)
   }
 }
 
@@ -855,15 +878,24 @@ extern "C" int pae_moe_experts_tiles(float* y, const void* x, int64_t ldx, const
   if (num_tokens <= 0) return 0;
   const int pairs = num_tokens * top;
   if (num_tokens <= 32 && pairs <= 256) {
-    // (an odd number of columns, so that an expert's workgroups go round the eight dies and not all to one)
-    const dim3 up_grid(experts | 1, (inter + 15) / 16, (num_tokens + 15) / 16), down_grid(experts | 1, (hidden + 15) / 16, (num_tokens + 15) / 16);
+    const bool by_pair = pairs <= experts;
+    // (an odd number of columns, so that a column's workgroups go round the eight dies and not all to one)
+    const dim3 up_grid((by_pair ? pairs : experts) | 1, (inter + 15) / 16, by_pair ? 1 : (num_tokens + 15) / 16);
+    const dim3 down_grid(up_grid.x, (hidden + 15) / 16, up_grid.z);
     PAE_REQUIRE(up_grid.y <= 65535 && down_grid.y <= 65535, "experts: widths %d, %d exceed the grid", hidden, inter);
-    moe_few_tiles_kernel<true, true><<<up_grid, 256, 0, stream>>>((bf16_t*)act, nullptr, (const bf16_t*)x, ldx, (const bf16_t*)gate_w,
-                                                                  (const bf16_t*)up_w, chosen, weights, nullptr, top,
-                                                                  num_tokens, hidden, inter, act_kind);
-    moe_few_tiles_kernel<false, true><<<down_grid, 256, 0, stream>>>(nullptr, y, (const bf16_t*)act, inter, (const bf16_t*)down_w,
-                                                                     nullptr, chosen, weights, nullptr, top, num_tokens,
-                                                                     inter, hidden, act_kind);
+#define MOE_LISTED(LIST)                                                                                                         \
+  moe_few_tiles_kernel<true, LIST><<<up_grid, 256, 0, stream>>>((bf16_t*)act, nullptr, (const bf16_t*)x, ldx,                    \
+                                                                (const bf16_t*)gate_w, (const bf16_t*)up_w, chosen, weights,     \
+                                                                nullptr, experts, top, num_tokens, hidden, inter, act_kind);     \
+  moe_few_tiles_kernel<false, LIST><<<down_grid, 256, 0, stream>>>(nullptr, y, (const bf16_t*)act, inter, (const bf16_t*)down_w, \
+                                                                   nullptr, chosen, weights, nullptr, experts, top, num_tokens,  \
+                                                                   inter, hidden, act_kind)
+    if (by_pair) {
+      MOE_LISTED(BY_PAIR);
+    } else {
+      MOE_LISTED(BY_EXPERT);
+    }
+#undef MOE_LISTED
     return pae_check_launch("moe_experts_few");
   }
   const int tile_rows = moe_tile_rows(pairs, hidden, inter, ldx * 2), max_tiles = pae_moe_max_tiles(pairs, experts);
@@ -883,12 +915,12 @@ extern "C" int pae_moe_experts_tiles(float* y, const void* x, int64_t ldx, const
   if (tile_rows == 16) {
     dim3 up_grid(max_tiles, (inter + 15) / 16), down_grid(max_tiles, (hidden + 15) / 16);
     PAE_REQUIRE(up_grid.y <= 65535 && down_grid.y <= 65535, "experts: widths %d, %d exceed the grid", hidden, inter);
-    moe_few_tiles_kernel<true, false><<<up_grid, 256, 0, stream>>>((bf16_t*)act, nullptr, (const bf16_t*)x, ldx, (const bf16_t*)gate_w,
-                                                            (const bf16_t*)up_w, order, weights, (const int4*)tiles, top,
-                                                            num_tokens, hidden, inter, act_kind);
-    moe_few_tiles_kernel<false, false><<<down_grid, 256, 0, stream>>>(nullptr, y, (const bf16_t*)act, inter, (const bf16_t*)down_w,
-                                                               nullptr, order, weights, (const int4*)tiles, top, num_tokens,
-                                                               inter, hidden, act_kind);
+    moe_few_tiles_kernel<true, SORTED><<<up_grid, 256, 0, stream>>>((bf16_t*)act, nullptr, (const bf16_t*)x, ldx, (const bf16_t*)gate_w,
+                                                                    (const bf16_t*)up_w, order, weights, (const int4*)tiles, experts,
+                                                                    top, num_tokens, hidden, inter, act_kind);
+    moe_few_tiles_kernel<false, SORTED><<<down_grid, 256, 0, stream>>>(nullptr, y, (const bf16_t*)act, inter, (const bf16_t*)down_w,
+                                                                       nullptr, order, weights, (const int4*)tiles, experts, top,
+                                                                       num_tokens, inter, hidden, act_kind);
   } else if (tile_rows == 64) MOE_TILES(4, 2, 4);
   else {
     const int64_t up_grid = (int64_t)max_tiles * ((inter + 127) / 128) + 7, down_grid = (int64_t)max_tiles * ((hidden + 255) / 256) + 7;

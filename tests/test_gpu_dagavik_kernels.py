@@ -531,3 +531,53 @@ def test_experts_of_a_few_tokens_at_the_edges_of_a_batch_of_k(H, F):
             g, u = gate[e].double() @ x[t].double(), up[e].double() @ x[t].double()
             want[t] += w * (down[e].double() @ (g * torch.sigmoid(g) * u))
     assert float((got - want).abs().max()) <= 4 * 2.0 ** -8 * float(want.abs().max())
+
+
+def _no_numbers(count):
+    """Fills the memory that the allocator hands out next for that many float32 numbers."""
+    kept = [torch.full((count,), float("nan"), device=DEV) for _ in range(64)]
+    del kept
+
+
+@pytest.mark.parametrize("chosen", [
+    [[0] * 4] * 4 + [[0, 1, 2, 3], [2, 0, 4, 1], [3, 4, 0, 2]],          # an expert with sixteen pairs of four tokens, and more
+    [[3, 3]] * 16, [[3, 3]] * 17, [[2] * 8] * 32, [[1] * 15] * 17,       # 32, 34, 256 and 255 pairs of one expert
+    [[1, 1, 2, 2], [2, 1, 2, 1], [0, 0, 0, 4]], [[4] * 200], [[0, 4] * 64, [4, 4] * 64]])
+def test_experts_of_a_few_tokens_named_more_than_once(chosen):
+    """A token may name an expert more than once (routing does so where no logit compares): more pairs of an expert than a step
+    has tokens, each with its own weight, against the same tokens inside a step of more pairs, which are sorted first:
+    the same bits.  The memory that the results come to holds no numbers before."""
+    gen = torch.Generator().manual_seed(len(chosen))
+    E, H, F = 5, 96, 160
+    T, top = len(chosen), len(chosen[0])
+    gate, up = ((torch.randn((E, F, H), generator=gen) * 0.2).to(torch.bfloat16).to(DEV) for _ in range(2))
+    down = (torch.randn((E, H, F), generator=gen) * 0.2).to(torch.bfloat16).to(DEV)
+    n = max(T, 256 // top + 1)
+    assert T <= 32 and T * top <= 256 < n * top <= 512
+    x = torch.randn((n, H), generator=gen).to(torch.bfloat16).to(DEV)
+    rows = torch.cat([torch.tensor(chosen), torch.randint(0, E, (n - T, top), generator=gen)]).to(torch.int32).to(DEV)
+    weights = torch.rand((n, top), generator=gen).to(DEV)
+    got = []
+    for count in (T, n):
+        _no_numbers(top * count * H)
+        got.append(K().moe_experts(x[:count], gate, up, down, rows[:count].contiguous(), weights[:count].contiguous()))
+    assert torch.equal(got[0], got[1][:, :T])
+
+
+def test_a_token_that_is_no_number_leaves_its_neighbours_alone():
+    """Routing gives a token whose logits do not compare expert 0 as often as it chooses: the other tokens' choices, weights and
+    experts are those of a step in which that token is an ordinary one."""
+    gen = torch.Generator().manual_seed(2)
+    E, H, F, T, top = 32, 96, 160, 32, 8
+    router = (torch.randn((E, H), generator=gen) * 0.2).to(torch.bfloat16).to(DEV)
+    gate, up = ((torch.randn((E, F, H), generator=gen) * 0.2).to(torch.bfloat16).to(DEV) for _ in range(2))
+    down = (torch.randn((E, H, F), generator=gen) * 0.2).to(torch.bfloat16).to(DEV)
+    x = torch.randn((T, H), generator=gen).to(torch.bfloat16).to(DEV)
+    hurt = x.clone()
+    hurt[:5] = float("nan")
+    got = []
+    for rows in (x, hurt):
+        chosen, weights = K().moe_choose(rows, router, None, 1, 1, top, 1.0)
+        _no_numbers(top * T * H)
+        got.append((chosen[5:], weights[5:], K().moe_experts(rows, gate, up, down, chosen, weights)[:, 5:]))
+    assert all(torch.equal(a, b) for a, b in zip(*got)) and torch.isfinite(got[0][2]).all()
