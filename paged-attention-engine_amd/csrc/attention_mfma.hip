@@ -351,17 +351,20 @@ __global__ __launch_bounds__(256, 1) void attn_prefill_split_kernel(
   const int lrow = lane / 4, lgrp = lane % 4;
   const int fetch_from = ((lane % 16) * 4 + lane / 16) * 4;
   bf16x8 kf[2][HD / 32], vf[VD / 16];
-  auto page_of = [&](int key0, int p) -> int64_t {  // in units of one head's page
+  // The first unit begins up to 31 keys before the first one that is seen: sixteens of keys that lie wholly before it are read as the
+  // one that holds it, whose page is the sequence's own.  (Their weights are zero, but the table may hold no page there any
+  // more, -1, and zero times what lies in another sequence's page may be no number.)
+  const int first_16 = (BIASED ? first_visible(pos0, window, chunked) : (window > 0 && pos0 - window + 1 > 0) ? pos0 - window + 1 : 0) / 16 * 16;
+  auto key_read = [&](int key0, int p) {
     const int key = key0 + 16 * p;
-    const int kc = key <= hi ? key : key0;  // a tile past the end repeats the first one (all of it is masked)
-    // a page the window has passed was given back (its entry is -1): all its keys are masked, read page 0
-    return (int64_t)max(table[kc / bs], 0) * nkv + kvh;
+    return max(key <= hi ? key : key0, first_16);  // a tile past the end repeats the first one (all of it is masked)
   };
+  auto page_of = [&](int kc) -> int64_t { return (int64_t)max(table[kc / bs], 0) * nkv + kvh; };  // in units of one head's page
   auto load_keys = [&](int key0) {
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
-      const int key = key0 + 16 * p, kc = key <= hi ? key : key0;
-      const bf16_t* kp = k_cache + page_of(key0, p) * (bs * HD) + (int64_t)(kc % bs) * HD;
+      const int kc = key_read(key0, p);
+      const bf16_t* kp = k_cache + page_of(kc) * (bs * HD) + (int64_t)(kc % bs) * HD;
 #pragma unroll
       for (int j = 0; j < HD / 32; ++j) kf[p][j] = *reinterpret_cast<const bf16x8*>(kp + lrow * HD + 32 * j + 8 * lgrp);
     }
@@ -370,8 +373,8 @@ __global__ __launch_bounds__(256, 1) void attn_prefill_split_kernel(
     const bf16_t* vp[2];
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
-      const int key = key0 + 16 * p, kc = key <= hi ? key : key0;
-      vp[p] = v_cache + page_of(key0, p) * (bs * VD) + kc % bs;
+      const int kc = key_read(key0, p);
+      vp[p] = v_cache + page_of(kc) * (bs * VD) + kc % bs;
     }
 #pragma unroll
     for (int t = 0; t < VD / 16; ++t)  // in the order of their use

@@ -414,6 +414,61 @@ def test_latent_attention_over_long_runs_under_a_window(H, D, R, V, C, window):
     assert float((out.cpu().double() - want).abs().max()) <= 2e-2 * float(want.abs().max())
 
 
+@pytest.mark.parametrize("window", [1, 17, 18, 190, 200])
+def test_runs_under_a_window_meet_no_numbers_of_another_run(window):
+    """Two runs whose heads' keys and values are formed, the first one's first rows infinite: the second, whose first keys in sight
+    lie in the second half of 32 (or not), gives the bits it gives beside a first run of numbers."""
+    from paged_attention_engine_amd.parts import StepShape
+    from paged_attention_engine_amd.parts.latent import expanded_runs
+
+    K = _K()
+    gen = torch.Generator().manual_seed(window)
+    H, D, R, V, C, bs, runs = 3, 64, 32, 64, 64, 16, [(0, 130), (301, 130)]  # (rows cached before, new rows)
+    up = randn(gen, H * (D + V), C, scale=C ** -0.5).to(torch.bfloat16).to(DEV)
+    width = max(-(-(a + n) // bs) for a, n in runs)
+    tables = torch.randperm(2 * width, generator=gen).view(2, width).to(torch.int32)
+    pool = randn(gen, 2 * width, bs, C + R).to(torch.bfloat16)
+    q = randn(gen, 260, H * (D + R)).to(torch.bfloat16).to(DEV)
+    lists = expanded_runs(StepShape((0, 1), (0, 130), (130, 130), (0, 301), bs), 128, window)
+    dev = lambda name: torch.tensor(lists[name][0], dtype=torch.int32, device=DEV).view(-1, lists[name][1])
+    positions = torch.cat([torch.arange(a, a + n) for a, n in runs]).to(torch.int32).to(DEV)
+    tables[1, :(301 - window + 1) // bs] = -1  # given back
+    got = []
+    for first in (None, math.inf, math.nan):
+        if first is not None:
+            pool[tables[0, 0]] = first
+        out = torch.full((260, H * V), float("nan"), dtype=torch.bfloat16, device=DEV)
+        K.latent_expanded(out, q, pool.to(DEV), up, dev("pages"), dev("page_table"), dev("tiles"), positions, tables.to(DEV), None,
+                          1.0, H, D, R, 0, True, V, C, D ** -0.5, None, window)
+        got.append(out[130:])
+    assert torch.isfinite(got[0].float()).all() and torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
+
+
+@pytest.mark.parametrize("bs,window", [(16, 17), (16, 100), (32, 100)])
+@pytest.mark.parametrize("chunked,slopes", [(False, False), (True, True), (False, True)])
+def test_prompts_under_a_window_meet_no_numbers_of_the_pool_s_first_page(bs, window, chunked, slopes):
+    """A run whose first pages were given back (their places in the table are -1), while the pool's first page holds another
+    request's infinities."""
+    K = _K()
+    gen = torch.Generator().manual_seed(window)
+    H, G, D, past, n = 4, 2, 64, 309, 70
+    width = -(-(past + n) // bs)
+    kc, vc = (randn(gen, width + 1, G, *shape).to(torch.bfloat16).to(DEV) for shape in ((bs, D), (D, bs)))
+    tables = torch.arange(1, width + 1, dtype=torch.int32).view(1, -1)
+    tables[0, :(past // window * window if chunked else past - window + 1) // bs] = -1
+    q = randn(gen, n, H * D).to(torch.bfloat16).to(DEV)
+    tiles = torch.tensor([(0, at, min(K.PREFILL_TILE, n - at)) for at in range(0, n, K.PREFILL_TILE)], dtype=torch.int32, device=DEV)
+    positions = torch.arange(past, past + n, dtype=torch.int32, device=DEV)
+    bias = torch.rand(H, generator=gen).to(DEV) * 0.1 if slopes else None
+    got = []
+    for first in (0.0, math.inf, math.nan):
+        kc[0], vc[0] = first, first
+        out = torch.full((n, H * D), float("nan"), dtype=torch.bfloat16, device=DEV)
+        K.attn_prefill(out, q, kc, vc, tiles, positions, tables.to(DEV), H, G, D, D ** -0.5, window, chunked=chunked, slopes=bias)
+        got.append(out)
+    assert torch.isfinite(got[0].float()).all() and torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
+
+
 def test_rotating_pairs_by_hand():
     """Pair (1, 0) at position 3 with dims 2 turns by 3 radians; features behind `dims` pass unchanged."""
     x = torch.tensor([[[1.0, 0.0, 9.0, 8.0]]], dtype=torch.float64)
