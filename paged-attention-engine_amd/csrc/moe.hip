@@ -624,9 +624,10 @@ __global__ __launch_bounds__(256) void moe_tiles_down_kernel(float* __restrict__
 // one tile of 16 features and take a quarter of k each, leave their sums in LDS, and the first adds them in wavefront
 // order (a wavefront per 16 features and the whole of k was measured against it: 35 + 22 us against 25 + 14 at one
 // token, 85 + 57 against 67 + 39 at eight).  The order of adding is a function of the sizes alone.  A wavefront asks for
-// four steps of 32 at once and works on the four before: a row's lines are whole in one batch (a step has half of
-// each), and 4 to 8 KB of a wavefront are on their way (7 tokens by four of 32 experts, 1,536 x 2,240, 267 and 133 MB
-// of weights: 63.6 + 36.0 -> 59.3 + 34.7 us, of 4 tokens 49.7 + 31.7 -> 44.6 + 26.2; the weights' stream bounds it).
+// two steps of 32 at once and works on the two before: a row's lines are whole in one batch (a step has half of
+// each), and five wavefronts a SIMD or more are resident.  Four steps at once take 128 registers where two take 80, and the chip then
+// has too few wavefronts: 8 tokens by four of 32 experts, 1,536 x 2,240, both products, one step 112, two 94, four 101 us; 16 by
+// eight of 128, 2,048 x 768, 179, 158 and 186; 24 by eight of 256, 2,048 x 512, 196, 181 and 216.  The weights' stream bounds it.
 //
 // In steps of up to 32 tokens and 256 pairs no sorting comes first: a workgroup looks its expert's pairs up itself, in their
 // order (two barriers, against a launch of 6 us, 30 with 256 experts, and the same trip to memory for the tile);
@@ -635,7 +636,8 @@ __global__ __launch_bounds__(256) void moe_tiles_down_kernel(float* __restrict__
 //   BY_PAIR    blockIdx.x is a pair; the workgroup takes the sixteen of its expert's pairs that begins with it, if one does
 //   BY_EXPERT  blockIdx.x is an expert; the workgroups along blockIdx.z take its sixteens in turn
 // What either costs over the weights' stream is its workgroups without work, so the list with fewer of them is taken:
-// pairs up to the number of experts, else experts.
+// pairs up to the number of experts, else experts.  Sorted / by pair / by expert: 1 token by eight of 256 68 / 21 / 33 us, 16 by eight of
+// 128 164 / 158 / 157, 16 by four of 32 117 / 116 / 112, 32 by four of 32 138 / 146 / 132.
 enum { SORTED, BY_PAIR, BY_EXPERT };
 template <bool GATED, int LIST>
 __global__ __launch_bounds__(256) void moe_few_tiles_kernel(bf16_t* __restrict__ act_out, float* __restrict__ y,
@@ -644,7 +646,7 @@ __global__ __launch_bounds__(256) void moe_few_tiles_kernel(bf16_t* __restrict__
                                                             const int* __restrict__ order, const float* __restrict__ weights,
                                                             const int4* __restrict__ tiles, int experts, int top, int num_tokens,
                                                             int K, int N, int act_kind) {
-  constexpr int BATCH = 4;
+  constexpr int BATCH = 2;
   __shared__ f32x4 parts[3][2][PAE_WAVE];
   __shared__ int pair_of[16];
   __shared__ uint64_t of_wave[4];
