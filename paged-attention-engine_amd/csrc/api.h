@@ -202,6 +202,7 @@ int pae_project_f32(int dtype, float* out, int64_t ldo, const void* A, int64_t l
 int pae_moe_route(const float* logits, int num_tokens, int experts, int groups, int keep, int top, float scale,
                   const float* choice_bias, int64_t ldz, int among_chosen, int shared_pieces, int* chosen, float* weights,
                   hipStream_t stream);
+int pae_moe_choose_pays(int dtype, int N, int K);
 int pae_moe_choose_takes(int dtype, const void* A, int64_t lda, const void* W, int M, int K);
 int pae_moe_choose(int dtype, const void* A, int64_t lda, const void* W, const void* bias, int b_is_f32, int M, int K,
                    int experts, int groups, int keep, int top, float scale, const float* choice_bias, int among_chosen,

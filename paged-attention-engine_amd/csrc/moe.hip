@@ -279,6 +279,12 @@ extern "C" int pae_moe_choose_takes(int dtype, const void* A, int64_t lda, const
   return M <= 256 && K % vec == 0 && lda % vec == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0;
 }
 
+// Whether it is ahead of the two launches for a router of N rows of K: all of them pass one workgroup, which has up to 40 outputs
+// on their way side by side, where the projection by itself spreads them over N / 4 workgroups.  One launch / two, 12 rows: 32 x 1,536 in
+// bfloat16 8.6 / 9.1 us, 40 x 1,536 8.9 / 9.4, 32 x 2,560 9.2 / 9.5, 41 x 1,536 9.9 / 9.6, 64 x 1,024 10.6 / 10.0, 8 x 7,168 10.6 / 10.3, 128 x
+// 2,048 19.3 / 14.2, 256 x 7,168 66 / 25.
+extern "C" int pae_moe_choose_pays(int dtype, int N, int K) { return N <= 40 && (int64_t)K * (dtype == PAE_F32 ? 4 : 2) <= 5120; }
+
 // pae_project_f32 and pae_moe_route in one launch: W [experts (+ 1 with shared pieces)][K], bias or null.
 extern "C" int pae_moe_choose(int dtype, const void* A, int64_t lda, const void* W, const void* bias, int b_is_f32, int M,
                               int K, int experts, int groups, int keep, int top, float scale, const float* choice_bias,

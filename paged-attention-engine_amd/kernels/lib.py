@@ -118,6 +118,7 @@ def _declare(lib) -> None:
         "pae_token_gate": [I, P, P, L, P, P, I, I, I, P],
         "pae_moe_gate_up": [I, P, P, L, P, P, P, I, I, I, I, I, P],
         "pae_moe_down": [I, P, P, P, P, P, I, I, I, I, P],
+        "pae_moe_choose_pays": [I, I, I],
         "pae_moe_tile_rows": [I],
         "pae_moe_choose_takes": [I, P, L, P, I, I],
         "pae_moe_choose": [I, P, L, P, P, I, I, I, I, I, I, I, F, P, I, I, P, P, P],
@@ -1898,14 +1899,24 @@ def moe_route(logits: torch.Tensor, groups: int, keep: int, top: int, scale: flo
 
 def moe_choose(x: torch.Tensor, router: torch.Tensor, bias: Optional[torch.Tensor], groups: int, keep: int, top: int, scale: float,
                choice_bias: Optional[torch.Tensor] = None, among_chosen: bool = False, shared_pieces: int = 0):
-    """`moe_route` of `project_f32(x, router, bias)`: in one launch for a few rows, the same bits."""
+    """`moe_route` of `project_f32(x, router, bias)`: in one launch for a few rows and a small router, the same bits."""
+    _not_while_recording("moe_choose")
+    lib = library()
+    code = code_of(x.dtype)
+    if not (lib.pae_moe_choose_pays(code, *router.shape)
+            and lib.pae_moe_choose_takes(code, x.data_ptr(), x.stride(0), router.data_ptr(), *x.shape)):
+        return moe_route(project_f32(x, router, bias), groups, keep, top, scale, choice_bias, among_chosen, shared_pieces)
+    return moe_choose_at_once(x, router, bias, groups, keep, top, scale, choice_bias, among_chosen, shared_pieces)
+
+
+def moe_choose_at_once(x: torch.Tensor, router: torch.Tensor, bias: Optional[torch.Tensor], groups: int, keep: int, top: int,
+                       scale: float, choice_bias: Optional[torch.Tensor] = None, among_chosen: bool = False, shared_pieces: int = 0):
+    """The one launch of `moe_choose`, for rows that `pae_moe_choose_takes`."""
     _not_while_recording("moe_choose")
     _gpu(x, router, bias, choice_bias)
     T, K = x.shape
     lib = library()
     assert x.dim() == 2 and x.stride(1) == 1 and router.dim() == 2 and router.is_contiguous() and router.shape[1] == K and router.dtype == x.dtype
-    if not lib.pae_moe_choose_takes(code_of(x.dtype), x.data_ptr(), x.stride(0), router.data_ptr(), T, K):
-        return moe_route(project_f32(x, router, bias), groups, keep, top, scale, choice_bias, among_chosen, shared_pieces)
     E = router.shape[0] - (1 if shared_pieces else 0)
     if bias is not None:
         assert bias.numel() == router.shape[0] and bias.is_contiguous()

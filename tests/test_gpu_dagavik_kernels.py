@@ -493,6 +493,21 @@ def test_choosing_in_one_launch_gives_the_bits_of_two(dtype, E, groups, keep, to
         assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]), (T, H)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("E,top,shared", [(40, 4, 0), (39, 3, 1), (41, 5, 0), (300, 8, 2), (1024, 70, 0)])
+def test_choosing_at_once_gives_the_bits_of_two_launches_for_any_router(dtype, E, top, shared):
+    """The one launch itself, also for routers that `moe_choose` leaves to two: outputs that the wavefronts take in one trip, in
+    two and in many, more choices than lanes."""
+    lib = K()
+    gen = torch.Generator().manual_seed(E)
+    for T, H in ((1, 64), (5, 1032)):
+        x = torch.randn((T, H), generator=gen).to(dtype).to(DEV)
+        router = (torch.randn((E + (1 if shared else 0), H), generator=gen) * H ** -0.5).to(dtype).to(DEV)
+        options = (1, 1, top, 1.7, None, True, shared)
+        got, want = lib.moe_choose_at_once(x, router, None, *options), lib.moe_route(lib.project_f32(x, router, None), *options)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]), (T, H)
+
+
 @pytest.mark.parametrize("T,E,top", [(1, 5, 3), (7, 33, 4), (16, 2, 2), (17, 2, 2), (32, 3, 3), (32, 40, 8)])
 def test_experts_of_a_few_tokens_by_lists_of_their_own(T, E, top):
     """Steps of up to 32 tokens and 256 pairs, where every workgroup looks its expert's pairs up itself: experts that all
