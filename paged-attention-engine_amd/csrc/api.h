@@ -209,7 +209,7 @@ int pae_moe_choose(int dtype, const void* A, int64_t lda, const void* W, const v
                    int shared_pieces, int* chosen, float* weights, hipStream_t stream);
 int pae_moe_gate_up(int dtype, void* act, const void* x, int64_t ldx, const void* gate_w, const void* up_w,
                     const int* chosen, int num_tokens, int top, int hidden, int inter, int act_kind, hipStream_t stream);
-int pae_moe_tile_rows(int pairs);
+int pae_moe_tile_rows(int pairs, int hidden, int inter, int64_t row_bytes);
 int pae_moe_max_tiles(int pairs, int experts);
 int pae_moe_tiles_supported(int hidden, int inter);
 int pae_moe_experts_tiles(float* y, const void* x, int64_t ldx, const void* gate_w, const void* up_w, const void* down_w,

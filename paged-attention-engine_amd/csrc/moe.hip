@@ -861,13 +861,13 @@ __global__ __launch_bounds__(256, 1) void moe_big_tiles_kernel(bf16_t* __restric
 
 // rows a tile holds for a step of that many pairs: 16 while an expert sees a few tokens, 64 in portions, 128 in prompts
 // (whose kernel reckons with 32-bit byte offsets within the rows and within an expert's weights)
-static int moe_tile_rows(int pairs, int hidden, int inter, int64_t row_bytes) {
+// (and counts an expert's tiles in 15 bits)
+extern "C" int pae_moe_tile_rows(int pairs, int hidden, int inter, int64_t row_bytes) {
   if (pairs <= 512) return 16;
   const int64_t widest = row_bytes > (int64_t)inter * 2 ? row_bytes : (int64_t)inter * 2;
-  return (pairs > 4096 && hidden % MOE_BIG_K == 0 && inter % MOE_BIG_K == 0 && pairs * widest < (1ll << 32) &&
+  return (pairs > 4096 && pairs <= 0x7fff * MOE_BIG_ROWS && hidden % MOE_BIG_K == 0 && inter % MOE_BIG_K == 0 && pairs * widest < (1ll << 32) &&
           (int64_t)hidden * inter * 2 < (1ll << 32)) ? MOE_BIG_ROWS : 64;
 }
-extern "C" int pae_moe_tile_rows(int pairs) { return pairs <= 512 ? 16 : (pairs <= 4096 ? 64 : MOE_BIG_ROWS); }
 extern "C" int pae_moe_max_tiles(int pairs, int experts) {
   const int rows = pairs <= 512 ? 16 : 64;  // the smallest tiles such a step may get: the most tiles there can be
   return (pairs + rows - 1) / rows + experts;
@@ -906,7 +906,7 @@ extern "C" int pae_moe_experts_tiles(float* y, const void* x, int64_t ldx, const
 #undef MOE_LISTED
     return pae_check_launch("moe_experts_few");
   }
-  const int tile_rows = moe_tile_rows(pairs, hidden, inter, ldx * 2), max_tiles = pae_moe_max_tiles(pairs, experts);
+  const int tile_rows = pae_moe_tile_rows(pairs, hidden, inter, ldx * 2), max_tiles = pae_moe_max_tiles(pairs, experts);
   moe_sort_kernel<<<1, 1024, (size_t)(4 * experts + 1) * sizeof(int), stream>>>(chosen, pairs, experts, tile_rows, order,
                                                                                (int4*)tiles, max_tiles);
 #define MOE_TILES(MT, UP_NT, DOWN_NT)                                                                                      \

@@ -119,7 +119,7 @@ def _declare(lib) -> None:
         "pae_moe_gate_up": [I, P, P, L, P, P, P, I, I, I, I, I, P],
         "pae_moe_down": [I, P, P, P, P, P, I, I, I, I, P],
         "pae_moe_choose_pays": [I, I, I],
-        "pae_moe_tile_rows": [I],
+        "pae_moe_tile_rows": [I, I, I, L],
         "pae_moe_choose_takes": [I, P, L, P, I, I],
         "pae_moe_choose": [I, P, L, P, P, I, I, I, I, I, I, I, F, P, I, I, P, P, P],
         "pae_moe_max_tiles": [I, I],
