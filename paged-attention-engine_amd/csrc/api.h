@@ -31,15 +31,14 @@ int pae_rope_kv_write(int dtype, void* qkv, int64_t row_stride, int num_tokens, 
 int pae_swiglu(int dtype, void* out, const void* x, int num_tokens, int inter, int block, hipStream_t stream);
 int pae_gated_act(int dtype, void* out, const void* x, int num_tokens, int inter, int block, int kind,
                   hipStream_t stream);  // act(gate) * up, act by code: 0 gelu (erf), 1 gelu (tanh), 2 silu
-int pae_gemm_plain_splits(int M, int N, int K);  // shares of k that pae_gemm_plain_shared is best called with
+int64_t pae_gemm_plain_scratch(int M, int N, int K);  // floats of scratch memory that pae_gemm_plain_shared is best called with
+void pae_gemm_plain_part(int M, int N, int K, int shared, int* part);  // rows and columns that one pass of its launches makes
 int pae_gemm_plain_shared(int in_dtype, int out_dtype, void* C, int64_t ldc, int64_t batch_c, const void* A, int64_t lda,
                           int64_t batch_a, const void* W, int64_t batch_w, const void* bias, int b_is_f32, int M, int N,
-                          int K, int batch, int splits, float* scratch, hipStream_t stream);
+                          int K, int batch, float* scratch, hipStream_t stream);
 int pae_gemm_plain_batched(int in_dtype, int out_dtype, void* C, int64_t ldc, int64_t batch_c, const void* A, int64_t lda,
                            int64_t batch_a, const void* W, int64_t batch_w, const void* bias, int b_is_f32, int M, int N,
                            int K, int batch, hipStream_t stream);
-int pae_gemm_plain(int in_dtype, int out_dtype, void* C, int64_t ldc, const void* A, int64_t lda, const void* W,
-                   const void* bias, int b_is_f32, int M, int N, int K, hipStream_t stream);
 int pae_gemm_skinny(int epilogue, void* out, int64_t ldc, const void* A, int64_t lda, const void* W,
                     const void* bias, int b_is_f32, int M, int N, int K, int splits, int64_t part_stride,
                     float* ticket_parts, int* ticket_counters, const float* row_stats, int row_stat_tiles,

@@ -362,17 +362,55 @@ __global__ __launch_bounds__(256) void gemm_plain_sum_kernel(TC* __restrict__ C,
 // Over how many workgroups the blocks of k of one tile are shared: 1 where the tiles fill the chip by themselves or
 // there is one block only.  A share costs its sums a way to memory and back and the launch that adds them (about
 // 4 us), so that up to 64 rows a workgroup's wavefronts take up to GP_FEW_WAVES blocks side by side first.
-extern "C" int pae_gemm_plain_splits(int M, int N, int K) {
+static int splits_of(int M, int N, int K) {
   const int blocks = (K + GP_BLOCK - 1) / GP_BLOCK;
   if (M <= 0 || blocks == 1) return 1;
   if (M <= GP_FEW_ROWS) {
     if (blocks <= GP_FEW_WAVES || (N + 15) / 16 >= 512) return 1;
-    return (blocks + GP_FEW_WAVES - 1) / GP_FEW_WAVES;
+    const int want = (blocks + GP_FEW_WAVES - 1) / GP_FEW_WAVES;
+    return want < 65535 ? want : 65535;
   }
   const int64_t tiles = (int64_t)((M + GP_TILE - 1) / GP_TILE) * ((N + GP_TILE - 1) / GP_TILE);
   if (tiles >= GP_ROUND) return 1;
   const int want = (int)((GP_ROUND + tiles - 1) / tiles);
   return want < blocks ? want : blocks;
+}
+
+// Rows and columns of C that one pass of launches makes.  A product with shared blocks of k keeps their sums, whatever the
+// number of shares: up to GP_SCRATCH floats (128 MiB) at once, more rows or columns than that one after the other, the longer side of C
+// cut into equal parts (all at once, a product of 2,000 x 512 x 18,944 would keep 152 MB; cut it takes 428 us instead of 380; one of
+// 200 x 3,584 x 18,944 keeps 106 MB).  And a grid's threads along x are counted in 32 bits.
+#define GP_SCRATCH (32 << 20)
+struct GpPart {
+  int rows, cols;
+};
+static GpPart part_of(int M, int N, int K, bool shared) {
+  const int64_t blocks = (K + GP_BLOCK - 1) / GP_BLOCK;
+  auto cut = [](int whole, int64_t most) {  // equal parts of at most `most`, in multiples of a tile
+    const int64_t tiles = (whole + GP_TILE - 1) / GP_TILE, fit = most / GP_TILE > 0 ? most / GP_TILE : 1, parts = (tiles + fit - 1) / fit;
+    return parts == 1 ? whole : (int)((tiles + parts - 1) / parts * GP_TILE);
+  };
+  GpPart part = {M, cut(N, 1 << 26)};
+  if (shared && splits_of(M, N, K) > 1 && blocks * M * N > GP_SCRATCH) {
+    if (N >= M) part.cols = cut(N, GP_SCRATCH / (blocks * M));
+    else part.rows = cut(M, GP_SCRATCH / (blocks * N));
+  }
+  part.rows = cut(part.rows, (int64_t)0xffffff / ((part.cols + GP_TILE - 1) / GP_TILE) * GP_TILE);
+  return part;
+}
+
+// part_of, for who wants to look: part[0] rows by part[1] columns.
+extern "C" void pae_gemm_plain_part(int M, int N, int K, int shared, int* part) {
+  const GpPart p = part_of(M, N, K, shared != 0);
+  part[0] = p.rows;
+  part[1] = p.cols;
+}
+
+// Floats of scratch memory that pae_gemm_plain_shared is best called with (0: none).
+extern "C" int64_t pae_gemm_plain_scratch(int M, int N, int K) {
+  if (M <= 0 || N <= 0 || K <= 0 || splits_of(M, N, K) == 1) return 0;
+  const GpPart part = part_of(M, N, K, true);
+  return (int64_t)((K + GP_BLOCK - 1) / GP_BLOCK) * part.rows * part.cols;
 }
 
 template <typename TA, typename TC, bool VEC>
@@ -407,48 +445,49 @@ static int launch_plain(void* C, int64_t ldc, int64_t batch_c, const void* A, in
 
 // in_dtype: operands; out_dtype: C.  Supported: f32->f32, bf16->bf16, bf16->f32.
 // `batch` products at once (one per head, say): product b reads A + b batch_a and W + b batch_w and
-// writes C + b batch_c, with the same leading dimensions; no bias then.  `splits` (pae_gemm_plain_splits; 1: none):
-// over how many workgroups a tile's k is shared, with room for ceil(K / 512) * M * N floats in `scratch`.
+// writes C + b batch_c, with the same leading dimensions; no bias then.  `scratch`: pae_gemm_plain_scratch floats for one product,
+// whose k may then be shared over workgroups, or null.
 extern "C" int pae_gemm_plain_shared(int in_dtype, int out_dtype, void* C, int64_t ldc, int64_t batch_c, const void* A,
                                      int64_t lda, int64_t batch_a, const void* W, int64_t batch_w, const void* bias,
-                                     int b_is_f32, int M, int N, int K, int batch, int splits, float* scratch,
-                                     hipStream_t stream) {
+                                     int b_is_f32, int M, int N, int K, int batch, float* scratch, hipStream_t stream) {
   PAE_REQUIRE(M >= 0 && N > 0 && K > 0, "gemm: bad sizes M=%d N=%d K=%d", M, N, K);
   PAE_REQUIRE(batch >= 1 && batch <= 65535 && (batch == 1 || !bias), "gemm: %d products at once (1..65535, no bias)", batch);
   PAE_REQUIRE(lda >= K && ldc >= N, "gemm: leading dimensions lda=%lld ldc=%lld too small for K=%d N=%d",
               (long long)lda, (long long)ldc, K, N);
-  PAE_REQUIRE(splits >= 1 && splits <= (K + GP_BLOCK - 1) / GP_BLOCK && splits <= 65535 && (splits == 1 || (scratch && batch == 1)),
-              "gemm: %d shares of k (one product at a time, at most a share per 512, with scratch memory)", splits);
+  PAE_REQUIRE(batch == 1 || !scratch, "gemm: shares of k go with one product at a time, not with %d", batch);
+  PAE_REQUIRE((in_dtype == PAE_F32 && out_dtype == PAE_F32) || (in_dtype == PAE_BF16 && (out_dtype == PAE_BF16 || out_dtype == PAE_F32)),
+              "gemm: unsupported dtype pair in=%d out=%d", in_dtype, out_dtype);
   if (M == 0) return 0;
   PAE_REQUIRE(M <= 65535 * 64, "gemm: M=%d exceeds the grid", M);
-  PAE_REQUIRE((int64_t)((M + 63) / 64) * ((N + 63) / 64) <= 0x7fffffff, "gemm: M=%d x N=%d exceeds the grid", M, N);
-  PAE_REQUIRE(splits == 1 || M <= 65535, "gemm: M=%d rows with shares of k", M);
-  if (splits == 1) scratch = nullptr;
   // four numbers at a time: 16 bytes in float32, 8 in bfloat16
-  const int elem = in_dtype == PAE_F32 ? 4 : 2;
+  const int elem = in_dtype == PAE_F32 ? 4 : 2, out_elem = out_dtype == PAE_F32 ? 4 : 2;
   const bool vec = K % 4 == 0 && lda % 4 == 0 && (batch == 1 || (batch_a % 4 == 0 && batch_w % 4 == 0)) &&
                    (uintptr_t)A % (4 * elem) == 0 && (uintptr_t)W % (4 * elem) == 0;
-#define GP_GO(TA, TC)                                                                                            \
-  return vec ? launch_plain<TA, TC, true>(C, ldc, batch_c, A, lda, batch_a, W, batch_w, bias, b_is_f32, M, N, K, \
-                                          batch, scratch, splits, stream)                                        \
-             : launch_plain<TA, TC, false>(C, ldc, batch_c, A, lda, batch_a, W, batch_w, bias, b_is_f32, M, N, K, \
-                                           batch, scratch, splits, stream)
-  if (in_dtype == PAE_F32 && out_dtype == PAE_F32) GP_GO(float, float);
-  if (in_dtype == PAE_BF16 && out_dtype == PAE_BF16) GP_GO(bf16_t, bf16_t);
-  if (in_dtype == PAE_BF16 && out_dtype == PAE_F32) GP_GO(bf16_t, float);
+  const GpPart part = part_of(M, N, K, scratch != nullptr);
+  for (int64_t n0 = 0; n0 < N; n0 += part.cols)
+    for (int64_t m0 = 0; m0 < M; m0 += part.rows) {
+      const int rows = (int)(M - m0 < part.rows ? M - m0 : part.rows), cols = (int)(N - n0 < part.cols ? N - n0 : part.cols);
+      char* c = (char*)C + (m0 * ldc + n0) * out_elem;
+      const char* a = (const char*)A + m0 * lda * elem;
+      const char* w = (const char*)W + n0 * K * elem;
+      const char* b = bias ? (const char*)bias + n0 * (b_is_f32 ? 4 : 2) : nullptr;
+      const int splits = scratch ? splits_of(rows, cols, K) : 1;
+      float* sums = splits > 1 ? scratch : nullptr;
+#define GP_GO(TA, TC)                                                                                                    \
+  (vec ? launch_plain<TA, TC, true>(c, ldc, batch_c, a, lda, batch_a, w, batch_w, b, b_is_f32, rows, cols, K, batch, sums, \
+                                    splits, stream)                                                                      \
+       : launch_plain<TA, TC, false>(c, ldc, batch_c, a, lda, batch_a, w, batch_w, b, b_is_f32, rows, cols, K, batch,    \
+                                     sums, splits, stream))
+      const int rc = in_dtype == PAE_F32 ? GP_GO(float, float) : out_dtype == PAE_BF16 ? GP_GO(bf16_t, bf16_t) : GP_GO(bf16_t, float);
 #undef GP_GO
-  return pae_fail("gemm: unsupported dtype pair in=%d out=%d", in_dtype, out_dtype);
+      if (rc) return rc;
+    }
+  return 0;
 }
 
 extern "C" int pae_gemm_plain_batched(int in_dtype, int out_dtype, void* C, int64_t ldc, int64_t batch_c, const void* A,
                                       int64_t lda, int64_t batch_a, const void* W, int64_t batch_w, const void* bias,
                                       int b_is_f32, int M, int N, int K, int batch, hipStream_t stream) {
   return pae_gemm_plain_shared(in_dtype, out_dtype, C, ldc, batch_c, A, lda, batch_a, W, batch_w, bias, b_is_f32, M, N, K,
-                               batch, 1, nullptr, stream);
-}
-
-extern "C" int pae_gemm_plain(int in_dtype, int out_dtype, void* C, int64_t ldc, const void* A, int64_t lda,
-                              const void* W, const void* bias, int b_is_f32, int M, int N, int K,
-                              hipStream_t stream) {
-  return pae_gemm_plain_batched(in_dtype, out_dtype, C, ldc, 0, A, lda, 0, W, 0, bias, b_is_f32, M, N, K, 1, stream);
+                               batch, nullptr, stream);
 }

@@ -68,9 +68,7 @@ def _declare(lib) -> None:
         "pae_scaled_rows": [P, P, P, I, F, I, I, P],
         "pae_skinny_ticket_slots": [I, I],
         "pae_gemm_skinny_act": [P, L, P, L, P, P, I, I, I, I, I, P, P, I, P],
-        "pae_gemm_plain_splits": [I, I, I],
-        "pae_gemm_plain_shared": [I, I, P, L, L, P, L, L, P, L, P, I, I, I, I, I, I, P, P],
-        "pae_gemm_plain": [I, I, P, L, P, L, P, P, I, I, I, I, P],
+        "pae_gemm_plain_shared": [I, I, P, L, L, P, L, L, P, L, P, I, I, I, I, I, P, P],
         "pae_gemm_skinny_gated": [P, L, P, L, P, I, I, I, I, P, P, I, P],
         "pae_paged_attention_generic": [I, P, L, P, L, P, P, P, P, P, I, I, I, I, I, I, F, I, P],
         "pae_paged_attention_capped": [I, P, L, P, L, P, P, P, P, P, I, I, I, I, I, I, I, F, I, F, P, P],
@@ -118,9 +116,9 @@ def _declare(lib) -> None:
         "pae_token_gate": [I, P, P, L, P, P, I, I, I, P],
         "pae_moe_gate_up": [I, P, P, L, P, P, P, I, I, I, I, I, P],
         "pae_moe_down": [I, P, P, P, P, P, I, I, I, I, P],
-        "pae_moe_choose_pays": [I, I, I],
         "pae_moe_tile_rows": [I, I, I, L],
         "pae_moe_choose_takes": [I, P, L, P, I, I],
+        "pae_moe_choose_pays": [I, I, I],
         "pae_moe_choose": [I, P, L, P, P, I, I, I, I, I, I, I, F, P, I, I, P, P, P],
         "pae_moe_max_tiles": [I, I],
         "pae_moe_tiles_supported": [I, I],
@@ -155,6 +153,10 @@ def _declare(lib) -> None:
         fn.restype = c_int
     lib.pae_skinny_ticket_floats.argtypes = [I, I, I]
     lib.pae_skinny_ticket_floats.restype = c_int64
+    lib.pae_gemm_plain_scratch.argtypes = [I, I, I]
+    lib.pae_gemm_plain_scratch.restype = c_int64
+    lib.pae_gemm_plain_part.argtypes = [I, I, I, I, P]
+    lib.pae_gemm_plain_part.restype = None
     lib.pae_delta_rule_work_floats.argtypes = [I, I, I, I, I, I]
     lib.pae_delta_rule_work_floats.restype = c_int64
     lib.pae_matrix_memory_work_floats.argtypes = [I, I, I, I, I]
@@ -995,12 +997,12 @@ def gemm_plain(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, bias: Option
         assert bias.numel() == N
     bp, bf = _param(bias)
     lib = library()
-    splits = lib.pae_gemm_plain_splits(M, N, K)
-    # the sums of every 512 of k, where a tile's k is shared over workgroups
-    sums = torch.empty((-(-K // 512), M, N), dtype=torch.float32, device=out.device) if splits > 1 else None
+    # the sums of every 512 of k, where a tile's k is shared over workgroups (up to 128 MiB)
+    floats = lib.pae_gemm_plain_scratch(M, N, K)
+    sums = torch.empty(floats, dtype=torch.float32, device=out.device) if floats else None
     _check(lib.pae_gemm_plain_shared(code_of(a.dtype), code_of(out.dtype), out.data_ptr(), out.stride(0), 0,
-                                     a.data_ptr(), a.stride(0), 0, w.data_ptr(), 0, bp, bf, M, N, K, 1, splits,
-                                     _ptr(sums), _stream()))
+                                     a.data_ptr(), a.stride(0), 0, w.data_ptr(), 0, bp, bf, M, N, K, 1, _ptr(sums),
+                                     _stream()))
 
 
 def gemm_plain_heads(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor) -> None:

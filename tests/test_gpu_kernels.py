@@ -112,6 +112,23 @@ def test_gemm_plain_adds_in_one_order(N, K_):
         assert torch.equal(one_by_one, out), M
 
 
+@pytest.mark.parametrize("M,N,K_", [(300, 2100, 30000), (2100, 300, 30000)])
+def test_gemm_plain_in_parts_gives_the_bits_of_the_whole(M, N, K_):
+    """Products whose blocks' sums do not fit the scratch memory at once are made in parts, along the columns or along the rows:
+    the bits of the same rows and columns by themselves."""
+    torch.manual_seed(M)
+    a, w, b = torch.randn(M, K_, device=DEV), torch.randn(N, K_, device=DEV), torch.randn(N, device=DEV)
+    floats = K().library().pae_gemm_plain_scratch(M, N, K_)
+    assert 0 < floats < -(-K_ // 512) * M * N
+    out = torch.full((M, N + 4), float("nan"), device=DEV)
+    K().gemm_plain(out[:, :N], a, w, b)
+    assert bool(out[:, N:].isnan().all())
+    for rows, cols in (((0, 65), (0, N)), ((M - 1, M), (0, N)), ((0, M), (N - 70, N)), ((0, M), (0, 1))):
+        one = torch.full((rows[1] - rows[0], cols[1] - cols[0]), float("nan"), device=DEV)
+        K().gemm_plain(one, a[rows[0]:rows[1]], w[cols[0]:cols[1]], b[cols[0]:cols[1]].clone())
+        assert torch.equal(one, out[rows[0]:rows[1], cols[0]:cols[1]])
+
+
 @pytest.mark.parametrize("M", [1, 8, 17, 64])
 @pytest.mark.parametrize("N,K_", [(2048, 1536), (1536, 8960), (50, 72), (777, 64), (96, 200),
                                   # about 256 workgroups of 5, 6, 7 and 8 wavefronts of 16 weight rows (above 16 rows of A)

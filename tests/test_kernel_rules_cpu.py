@@ -1,9 +1,38 @@
 """The rules by which the kernel library chooses a route for a call, and the memory it asks for: plain host code, asked here
 without a GPU."""
 
+import ctypes
+
+import pytest
 import torch
 
 from paged_attention_engine_amd.kernels import lib as K
+
+
+def part_of(M, N, K_, shared=True):
+    part = (ctypes.c_int * 2)()
+    K.library().pae_gemm_plain_part(M, N, K_, int(shared), ctypes.addressof(part))
+    return tuple(part)
+
+
+@pytest.mark.parametrize("M,N,K_", [(200, 3584, 18944), (601, 3584, 18944), (800, 3584, 18944), (601, 2048, 11008), (2000, 512, 18944),
+                                    (3000, 512, 18944), (24000, 64, 18944), (65, 24000, 18944), (64, 8000, 53248), (100, 100, 2000000)])
+def test_memory_for_the_sums_of_shared_products_is_bounded(M, N, K_):
+    """At most 128 MiB, or one row or column of tiles where its sums are more than that; every part of the product fits it."""
+    blocks, (rows, cols) = -(-K_ // 512), part_of(M, N, K_)
+    floats = K.library().pae_gemm_plain_scratch(M, N, K_)
+    assert floats <= max(32 << 20, blocks * 64 * min(M, N))
+    assert 0 < rows <= M and 0 < cols <= N and (rows == M or rows % 64 == 0) and (cols == N or cols % 64 == 0)
+    assert floats in (0, blocks * rows * cols)
+
+
+@pytest.mark.parametrize("M,N,K_", [(4194240, 16448, 1), (4194240, 4096, 64), (70000, 1 << 20, 1), (1, 1 << 30, 4), (64, 2000000000, 1)])
+@pytest.mark.parametrize("shared", [False, True])
+def test_products_of_any_size_fit_a_grid(M, N, K_, shared):
+    """A grid's threads along x are counted in 32 bits: 256 a tile of 64 x 64, up to 512 a sixteen of columns of few rows."""
+    rows, cols = part_of(M, N, K_, shared)
+    assert 0 < rows <= M and 0 < cols <= N
+    assert (-(-rows // 64) * -(-cols // 64) * 256 if rows > 64 else -(-cols // 16) * 512) < 1 << 32
 
 
 def test_routers_that_one_workgroup_reads_are_small():
