@@ -36,7 +36,7 @@
 #define GP_FEW_ROWS 64
 #define GP_FEW_WAVES 8
 #define GP_TILE 64    // rows of either side of a tile
-#define GP_ROUND 768  // tiles that give every compute unit three
+#define GP_UNITS 256  // compute units
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -362,17 +362,23 @@ __global__ __launch_bounds__(256) void gemm_plain_sum_kernel(TC* __restrict__ C,
 // Over how many workgroups the blocks of k of one tile are shared: 1 where the tiles fill the chip by themselves or
 // there is one block only.  A share costs its sums a way to memory and back and the launch that adds them (about
 // 4 us), so that up to 64 rows a workgroup's wavefronts take up to GP_FEW_WAVES blocks side by side first.
+// Up to 64 rows a compute unit works through its workgroups in rounds, and shares pay where they leave fewer rounds of the whole
+// k; with more rows, up to one and a half tiles a compute unit.  Measured without shares / with them: 3 rows of 11,008 by 128 sixteens of
+// weight rows (2 rounds of a third) 36.1 / 30.1 us, of 16,384 by 192 (3 of a quarter) 50.0 / 44.3, of 8,192 by 192 (2 of a half)
+// 27.0 / 28.6, of 11,008 by 256 (3 of a third) 44.8 / 49.3; 320 tiles 392 / 299 (601 x 2,048 x 11,008), 376 669 / 632 (3,000 x 512 x
+// 18,944), 416 397 / 433 (800 x 2,048 x 11,008), 658 258 / 288 (3,000 x 896 x 4,864), 728 992 / 1,121 (800 x 3,584 x 18,944).
 static int splits_of(int M, int N, int K) {
   const int blocks = (K + GP_BLOCK - 1) / GP_BLOCK;
   if (M <= 0 || blocks == 1) return 1;
   if (M <= GP_FEW_ROWS) {
-    if (blocks <= GP_FEW_WAVES || (N + 15) / 16 >= 512) return 1;
-    const int want = (blocks + GP_FEW_WAVES - 1) / GP_FEW_WAVES;
-    return want < 65535 ? want : 65535;
+    if (blocks <= GP_FEW_WAVES) return 1;
+    const int64_t sixteens = (N + 15) / 16, shares = (blocks + GP_FEW_WAVES - 1) / GP_FEW_WAVES;
+    const int64_t rounds = (sixteens + GP_UNITS - 1) / GP_UNITS, rounds_of_shares = (sixteens * shares + GP_UNITS - 1) / GP_UNITS;
+    return rounds_of_shares < rounds * shares && shares <= 65535 ? (int)shares : 1;
   }
   const int64_t tiles = (int64_t)((M + GP_TILE - 1) / GP_TILE) * ((N + GP_TILE - 1) / GP_TILE);
-  if (tiles >= GP_ROUND) return 1;
-  const int want = (int)((GP_ROUND + tiles - 1) / tiles);
+  if (2 * tiles >= 3 * GP_UNITS) return 1;
+  const int want = (int)((3 * GP_UNITS + tiles - 1) / tiles);  // three workgroups a compute unit
   return want < blocks ? want : blocks;
 }
 
