@@ -128,20 +128,20 @@ __global__ __launch_bounds__(256) void norm_scale_add_vec_kernel(float* __restri
 // The same bits for up to seven parts and widths up to 1,024 * TRIPS: the kernel above waits for one part before it asks for the
 // next, and for the weight number by number; here all of them are asked for as raw bits.  One row of 1,536:
 // 5.0 -> 4.1 us; six rows 6.2 -> 4.8 us.
-template <typename T, int TRIPS>
+template <typename T, int TRIPS, int MOST>
 __global__ __launch_bounds__(256) void norm_scale_add_few_trips_kernel(float* __restrict__ residual, row_pieces::Pieces pieces,
                                                                        const void* __restrict__ weight, int w_is_f32, float eps,
                                                                        float scale, T* __restrict__ next, int hidden) {
   __shared__ float scratch[4];
   const int64_t base = (int64_t)blockIdx.x * hidden;
-  uint4 raw[TRIPS][row_pieces::PIECES], raw_r[TRIPS], raw_w[TRIPS];
+  uint4 raw[TRIPS][MOST], raw_r[TRIPS], raw_w[TRIPS];
   int at[TRIPS];
 #pragma unroll
   for (int c = 0; c < TRIPS; ++c) {
     const int i = (threadIdx.x + 256 * c) * 4;
     at[c] = i < hidden ? i : -1;
     const int from = i < hidden ? i : 0;  // a thread beyond the row reads its start and adds nothing
-    row_pieces::ask_all<T>(pieces, blockIdx.x, from, raw[c]);
+    row_pieces::ask_all<T, MOST>(pieces, blockIdx.x, from, raw[c]);
     raw_r[c] = row_pieces::ask(residual, base + from, true);
     raw_w[c] = row_pieces::ask(weight, from, w_is_f32);
   }
@@ -151,7 +151,7 @@ __global__ __launch_bounds__(256) void norm_scale_add_few_trips_kernel(float* __
   for (int c = 0; c < TRIPS; ++c) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) y[c][e] = 0.f;
-    row_pieces::add_all<T>(pieces, raw[c], y[c]);
+    row_pieces::add_all<T, MOST>(pieces, raw[c], y[c]);
     if (at[c] >= 0)
 #pragma unroll
       for (int e = 0; e < 4; ++e) ss = fmaf(y[c][e], y[c][e], ss);
@@ -184,20 +184,30 @@ extern "C" int pae_norm_scale_add(int dtype, float* residual, const void* y, int
     const float one = 1.f;
     auto aligned = [](const void* p) { return (uintptr_t)p % 16 == 0; };
     row_pieces::Pieces pieces;
-    if (aligned(residual) && aligned(y) && aligned(weight) && aligned(next) &&
+    // (three parts and more, the kernel above / this one: 1,024 rows of 1,536 13.0 / 13.9 us, 2,048 of 3,584 27.4 / 28.9; 3,000 of 1,536 19.6 /
+    // 18.8, 4,096 of 3,584 68.6 / 60.0)
+    if ((num_rows < 512 || num_rows > 2560 || count <= row_pieces::FEW) && aligned(residual) && aligned(y) && aligned(weight) && aligned(next) &&
         row_pieces::flatten(pieces, 1, &y, &f32, &count, &part_stride, &row_stride, &one)) {
-#define SCALE_ADD_TRIPS(T, TRIPS) \
-  norm_scale_add_few_trips_kernel<T, TRIPS><<<num_rows, 256, 0, stream>>>(residual, pieces, weight, w_is_f32, eps, scale, (T*)next, hidden)
-#define SCALE_ADD_FEW(T)                          \
-  if (hidden <= 1024) SCALE_ADD_TRIPS(T, 1);      \
-  else if (hidden <= 2048) SCALE_ADD_TRIPS(T, 2); \
-  else SCALE_ADD_TRIPS(T, 4);
+#define SCALE_ADD_TRIPS(T, TRIPS, MOST) \
+  norm_scale_add_few_trips_kernel<T, TRIPS, MOST><<<num_rows, 256, 0, stream>>>(residual, pieces, weight, w_is_f32, eps, scale, (T*)next, hidden)
+#define SCALE_ADD_MOST(T, MOST)                         \
+  if (hidden <= 1024) SCALE_ADD_TRIPS(T, 1, MOST);      \
+  else if (hidden <= 2048) SCALE_ADD_TRIPS(T, 2, MOST); \
+  else if (hidden <= 3072) SCALE_ADD_TRIPS(T, 3, MOST); \
+  else SCALE_ADD_TRIPS(T, 4, MOST);
+#define SCALE_ADD_FEW(T)                  \
+  if (pieces.count <= row_pieces::FEW) {  \
+    SCALE_ADD_MOST(T, row_pieces::FEW)    \
+  } else {                                \
+    SCALE_ADD_MOST(T, row_pieces::PIECES) \
+  }
       if (dtype == PAE_F32) {
         SCALE_ADD_FEW(float)
       } else {
         SCALE_ADD_FEW(bf16_t)
       }
 #undef SCALE_ADD_FEW
+#undef SCALE_ADD_MOST
 #undef SCALE_ADD_TRIPS
       return pae_check_launch("norm_scale_add");
     }

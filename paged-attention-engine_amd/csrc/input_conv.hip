@@ -249,7 +249,7 @@ __global__ __launch_bounds__(256) void norm_join_conv_few_trips_kernel(
     const int i = (threadIdx.x + 256 * c) * 4;
     at[c] = i < hidden ? i : -1;
     const int from = i < hidden ? i : 0;  // a thread beyond the row reads its start and adds nothing
-    row_pieces::ask_all<T>(pieces, t, from, raw[c]);
+    row_pieces::ask_all<T, row_pieces::PIECES>(pieces, t, from, raw[c]);
     raw_r[c] = row_pieces::ask(residual, base + from, true);
     raw_w[c] = row_pieces::ask(weight, from, w_is_f32);
 #pragma unroll
@@ -266,7 +266,7 @@ __global__ __launch_bounds__(256) void norm_join_conv_few_trips_kernel(
   for (int c = 0; c < TRIPS; ++c) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) y[c][e] = past[c][e] = 0.f;
-    row_pieces::add_all<T>(pieces, raw[c], y[c]);
+    row_pieces::add_all<T, row_pieces::PIECES>(pieces, raw[c], y[c]);
 #pragma unroll
     for (int j = 0; j < KEEP; ++j) {  // oldest first: tap j weighs the input KEEP - j tokens ago
       float w[4], in[4];

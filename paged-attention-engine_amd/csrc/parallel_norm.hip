@@ -99,7 +99,7 @@ __global__ __launch_bounds__(256) void sum_norm2_kernel(float* __restrict__ resi
 
 // The same bits for widths in multiples of four up to 1,024 * TRIPS, with everything the row needs asked for at once
 // (row_pieces.h) and held in registers.  7 rows of 1,536, the experts' four parts and two more terms: 12.1 -> 7.4 us.
-template <typename T, int TRIPS>
+template <typename T, int TRIPS, int MOST>
 __global__ __launch_bounds__(256) void sum_norm2_few_trips_kernel(float* __restrict__ residual, row_pieces::Pieces pieces,
                                                                   const void* __restrict__ w1, int w1_is_f32,
                                                                   const void* __restrict__ w2, int w2_is_f32, float eps,
@@ -108,7 +108,7 @@ __global__ __launch_bounds__(256) void sum_norm2_few_trips_kernel(float* __restr
   __shared__ float scratch[4];
   const int64_t src = rows ? rows[blockIdx.x] : blockIdx.x;
   float* x = residual + src * hidden;
-  uint4 raw[TRIPS][row_pieces::PIECES], raw_x[TRIPS], raw1[TRIPS], raw2[TRIPS];
+  uint4 raw[TRIPS][MOST], raw_x[TRIPS], raw1[TRIPS], raw2[TRIPS];
   int at[TRIPS];
 #pragma unroll
   for (int c = 0; c < TRIPS; ++c) {
@@ -116,7 +116,7 @@ __global__ __launch_bounds__(256) void sum_norm2_few_trips_kernel(float* __restr
     at[c] = i < hidden ? i : -1;
     const int from = i < hidden ? i : 0;  // a thread beyond the row reads its start and adds nothing
     raw_x[c] = row_pieces::ask(x, from, true);
-    row_pieces::ask_all<T>(pieces, src, from, raw[c]);
+    row_pieces::ask_all<T, MOST>(pieces, src, from, raw[c]);
     if (out1) raw1[c] = row_pieces::ask(w1, from, w1_is_f32);
     if (out2) raw2[c] = row_pieces::ask(w2, from, w2_is_f32);
   }
@@ -125,7 +125,7 @@ __global__ __launch_bounds__(256) void sum_norm2_few_trips_kernel(float* __restr
 #pragma unroll
   for (int c = 0; c < TRIPS; ++c) {
     row_pieces::numbers(raw_x[c], true, v[c]);
-    row_pieces::add_all<T>(pieces, raw[c], v[c]);
+    row_pieces::add_all<T, MOST>(pieces, raw[c], v[c]);
     if (at[c] < 0) continue;
 #pragma unroll
     for (int e = 0; e < 4; ++e) ss = fmaf(v[c][e], v[c][e], ss);
@@ -183,19 +183,27 @@ extern "C" int pae_sum_norm2(int dtype, float* residual, int num_terms, const vo
   row_pieces::Pieces pieces;
   if (vec && hidden <= 4096 && aligned(out1) && aligned(out2) && (!out1 || aligned(w1)) && (!out2 || aligned(w2)) &&
       row_pieces::flatten(pieces, terms.count, terms.ptr, terms.is_f32, terms.parts, terms.part_stride, row_stride, terms.scale)) {
-#define SUM_NORM2_TRIPS(T, TRIPS)                                                                                     \
-  sum_norm2_few_trips_kernel<T, TRIPS><<<num_rows, 256, 0, stream>>>(residual, pieces, w1, w1_is_f32, w2, w2_is_f32, eps, \
+#define SUM_NORM2_TRIPS(T, TRIPS, MOST)                                                                                         \
+  sum_norm2_few_trips_kernel<T, TRIPS, MOST><<<num_rows, 256, 0, stream>>>(residual, pieces, w1, w1_is_f32, w2, w2_is_f32, eps, \
                                                                      rows, (T*)out1, (T*)out2, hidden, rows ? 0 : write_residual)
-#define SUM_NORM2_FEW(T)                          \
-  if (hidden <= 1024) SUM_NORM2_TRIPS(T, 1);      \
-  else if (hidden <= 2048) SUM_NORM2_TRIPS(T, 2); \
-  else SUM_NORM2_TRIPS(T, 4);
+#define SUM_NORM2_MOST(T, MOST)                         \
+  if (hidden <= 1024) SUM_NORM2_TRIPS(T, 1, MOST);      \
+  else if (hidden <= 2048) SUM_NORM2_TRIPS(T, 2, MOST); \
+  else if (hidden <= 3072) SUM_NORM2_TRIPS(T, 3, MOST); \
+  else SUM_NORM2_TRIPS(T, 4, MOST);
+#define SUM_NORM2_FEW(T)                  \
+  if (pieces.count <= row_pieces::FEW) {  \
+    SUM_NORM2_MOST(T, row_pieces::FEW)    \
+  } else {                                \
+    SUM_NORM2_MOST(T, row_pieces::PIECES) \
+  }
     if (dtype == PAE_F32) {
       SUM_NORM2_FEW(float)
     } else {
       SUM_NORM2_FEW(bf16_t)
     }
 #undef SUM_NORM2_FEW
+#undef SUM_NORM2_MOST
 #undef SUM_NORM2_TRIPS
     return pae_check_launch("sum_norm2");
   }

@@ -5,13 +5,14 @@
 // On a few rows such a kernel's time is its trips to memory, one behind the other: a piece's type and number are known at
 // run time only, and a load whose value is converted under a condition is waited for there.  So all pieces are
 // asked for at once as raw bits, the weights with them, and converted and added when all are there.  Up to
-// PIECES pieces and 4,096 columns; the general kernels take the rest.
+// PIECES pieces and 4,096 columns; the general kernels take the rest.  Kernels are built for up to FEW pieces and for up to PIECES
+// (MOST): room for all seven is registers, 156 to 172 of them at four trips, which many rows of few pieces then lack wavefronts for.
 #pragma once
 #include "common.h"
 
 namespace row_pieces {
 
-constexpr int PIECES = 7;
+constexpr int PIECES = 7, FEW = 2;
 
 struct Pieces {
   const void* ptr[PIECES];
@@ -66,19 +67,19 @@ __device__ __forceinline__ void put4(bf16_t* p, const float (&v)[4]) {
 }
 
 // The pieces of a row's columns i .. i + 3 as raw bits.  T: the activation type.
-template <typename T>
-__device__ __forceinline__ void ask_all(const Pieces& pieces, int64_t row, int i, uint4 (&raw)[PIECES]) {
+template <typename T, int MOST>
+__device__ __forceinline__ void ask_all(const Pieces& pieces, int64_t row, int i, uint4 (&raw)[MOST]) {
 #pragma unroll
-  for (int k = 0; k < PIECES; ++k)
+  for (int k = 0; k < MOST; ++k)
     if (k < pieces.count) raw[k] = ask(pieces.ptr[k], row * pieces.row_stride[k] + i, sizeof(T) == 4 || pieces.is_f32[k]);
 }
 
 // sum[e] += scale_j * (the pieces of term j, added in order), terms in order.
-template <typename T>
-__device__ __forceinline__ void add_all(const Pieces& pieces, const uint4 (&raw)[PIECES], float (&sum)[4]) {
+template <typename T, int MOST>
+__device__ __forceinline__ void add_all(const Pieces& pieces, const uint4 (&raw)[MOST], float (&sum)[4]) {
   float term[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int k = 0; k < PIECES; ++k)
+  for (int k = 0; k < MOST; ++k)
     if (k < pieces.count) {
       float v[4];
       numbers(raw[k], sizeof(T) == 4 || pieces.is_f32[k], v);

@@ -141,7 +141,7 @@ __global__ __launch_bounds__(256) void norm_join_kernel(float* __restrict__ resi
 // The same bits for widths in multiples of four up to 1,024 * TRIPS, with everything the row needs asked for at once
 // (row_pieces.h) and held in registers: one trip to memory, the two sums, the stores.  8 rows of 1,536, two
 // bfloat16 terms: 8.1 -> 5.4 us.
-template <typename T, int TRIPS>
+template <typename T, int TRIPS, int MOST>
 __global__ __launch_bounds__(256) void norm_join_few_trips_kernel(float* __restrict__ residual, row_pieces::Pieces pieces,
                                                                   const void* __restrict__ w_out, int w_out_is_f32, float eps,
                                                                   const void* __restrict__ w_next, int w_next_is_f32,
@@ -149,14 +149,14 @@ __global__ __launch_bounds__(256) void norm_join_few_trips_kernel(float* __restr
                                                                   int hidden) {
   __shared__ float scratch[4];
   const int64_t base = (int64_t)blockIdx.x * hidden;
-  uint4 raw[TRIPS][row_pieces::PIECES], raw_x[TRIPS], raw_out[TRIPS], raw_next[TRIPS];
+  uint4 raw[TRIPS][MOST], raw_x[TRIPS], raw_out[TRIPS], raw_next[TRIPS];
   int at[TRIPS];
 #pragma unroll
   for (int c = 0; c < TRIPS; ++c) {
     const int i = (threadIdx.x + 256 * c) * 4;
     at[c] = i < hidden ? i : -1;
     const int from = i < hidden ? i : 0;  // a thread beyond the row reads its start and adds nothing
-    row_pieces::ask_all<T>(pieces, blockIdx.x, from, raw[c]);
+    row_pieces::ask_all<T, MOST>(pieces, blockIdx.x, from, raw[c]);
     raw_x[c] = row_pieces::ask(residual, base + from, true);
     if (w_out) raw_out[c] = row_pieces::ask(w_out, from, w_out_is_f32);
     if (normed) raw_next[c] = row_pieces::ask(w_next, from, w_next_is_f32);
@@ -168,7 +168,7 @@ __global__ __launch_bounds__(256) void norm_join_few_trips_kernel(float* __restr
     row_pieces::numbers(raw_x[c], true, x[c]);
 #pragma unroll
     for (int e = 0; e < 4; ++e) y[c][e] = 0.f;
-    row_pieces::add_all<T>(pieces, raw[c], y[c]);
+    row_pieces::add_all<T, MOST>(pieces, raw[c], y[c]);
     if (at[c] >= 0)
 #pragma unroll
       for (int e = 0; e < 4; ++e) ss = fmaf(y[c][e], y[c][e], ss);
@@ -240,19 +240,27 @@ extern "C" int pae_norm_join(int dtype, float* residual, int num_terms, const vo
   row_pieces::Pieces pieces;
   if (vec && hidden <= 4096 && (!w_out || (uintptr_t)w_out % 16 == 0) && (!normed || (uintptr_t)w_next % 16 == 0) &&
       row_pieces::flatten(pieces, terms.count, terms.ptr, terms.is_f32, terms.parts, terms.part_stride, terms.row_stride, terms.scale)) {
-#define NORM_JOIN_TRIPS(T, TRIPS)                                                                                   \
-  norm_join_few_trips_kernel<T, TRIPS><<<num_rows, 256, 0, stream>>>(residual, pieces, w_out, w_out_is_f32, eps, w_next, \
+#define NORM_JOIN_TRIPS(T, TRIPS, MOST)                                                                                        \
+  norm_join_few_trips_kernel<T, TRIPS, MOST><<<num_rows, 256, 0, stream>>>(residual, pieces, w_out, w_out_is_f32, eps, w_next, \
                                                                      w_next_is_f32, eps_next, (T*)normed, (T*)rows, hidden)
-#define NORM_JOIN_FEW(T)                          \
-  if (hidden <= 1024) NORM_JOIN_TRIPS(T, 1);      \
-  else if (hidden <= 2048) NORM_JOIN_TRIPS(T, 2); \
-  else NORM_JOIN_TRIPS(T, 4);
+#define NORM_JOIN_MOST(T, MOST)                         \
+  if (hidden <= 1024) NORM_JOIN_TRIPS(T, 1, MOST);      \
+  else if (hidden <= 2048) NORM_JOIN_TRIPS(T, 2, MOST); \
+  else if (hidden <= 3072) NORM_JOIN_TRIPS(T, 3, MOST); \
+  else NORM_JOIN_TRIPS(T, 4, MOST);
+#define NORM_JOIN_FEW(T)                  \
+  if (pieces.count <= row_pieces::FEW) {  \
+    NORM_JOIN_MOST(T, row_pieces::FEW)    \
+  } else {                                \
+    NORM_JOIN_MOST(T, row_pieces::PIECES) \
+  }
     if (dtype == PAE_F32) {
       NORM_JOIN_FEW(float)
     } else {
       NORM_JOIN_FEW(bf16_t)
     }
 #undef NORM_JOIN_FEW
+#undef NORM_JOIN_MOST
 #undef NORM_JOIN_TRIPS
     return pae_check_launch("norm_join");
   }

@@ -418,6 +418,30 @@ def test_norms_with_all_loads_up_front_give_the_bits_of_the_general_ones(dtype, 
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H", [1024, 2048, 3072, 3076, 4096])
+@pytest.mark.parametrize("T,parts", [(2, 1), (2, 2), (2, 3), (600, 1), (600, 3), (2600, 3)])
+def test_norms_of_few_pieces_and_many_rows_give_the_bits_of_the_general_ones(dtype, H, T, parts):
+    """Up to two pieces and more, widths at the edges of three and four trips, many rows of several parts: weights on 16 bytes and
+    one element behind, as above."""
+    from paged_attention_engine_amd.kernels import lib
+
+    torch.manual_seed(H + T + parts)
+    x, p, w = torch.randn(T, H), torch.randn(parts, T, H), torch.randn(H)
+    y = torch.randn(T, H).to(dtype)
+    got = []
+    for aligned in (True, False):
+        weight = _placed(w.to(DEV), aligned)
+        streams, rows = [_placed(x.to(DEV), True) for _ in range(4)], [torch.zeros(T, H, dtype=dtype, device=DEV) for _ in range(6)]
+        lib.norm_join(streams[0], [(p.to(DEV), 0.7)], weight, 1e-5, weight, 1e-6, rows[0], rows[1])
+        lib.sum_norm2(streams[1], [(p.to(DEV), 0.3)], weight, weight, 1e-5, rows[2], rows[3])
+        lib.norm_scale_add(streams[2], p.to(DEV), weight, 1e-5, 0.6, rows[4])
+        lib.norm_scale_add(streams[3], y.to(DEV), weight, 1e-5, 0.6, rows[5])
+        got.append([t.cpu() for t in streams + rows])
+    for one_way, other in zip(*got):
+        assert torch.isfinite(one_way.float()).all() and torch.equal(one_way, other)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("H,G,D,V", [(1, 1, 8, 8), (12, 2, 128, 128), (16, 4, 128, 64), (40, 24, 64, 64), (3, 0, 40, 40), (63, 1, 128, 128), (64, 1, 128, 128)])
 @pytest.mark.parametrize("rot_share,interleaved,per_head", [(0.0, False, True), (0.5, False, True), (1.0, True, True), (1.0, False, False)])
 def test_rows_by_chunks_are_prepared_as_number_by_number(dtype, H, G, D, V, rot_share, interleaved, per_head):
