@@ -19,7 +19,8 @@
 #define CONV_THREADS 128
 #define CONV_PER_THREAD 8  // head widths up to CONV_THREADS * CONV_PER_THREAD
 #define CONV_ROWS 8        // rows of a prompt that a wavefront takes
-#define CONV_ROWS_FROM 256 // steps of fewer rows leave most of the chip idle by wavefronts of eight
+#define CONV_ROWS_FROM 256 // rows of a step, and (row, head) pairs, from which wavefronts of eight rows are ahead: fewer pairs than
+#define CONV_PAIRS_FROM 8192  // these leave some of the chip's 1,024 vector units without a wavefront
 
 // seq_runs[s] = (first flat row, rows in this step, tokens held before the step, unused)
 // One workgroup per (token, head): the q heads, then the k heads, then the v heads.
@@ -251,8 +252,10 @@ extern "C" int pae_conv_norm_store(int dtype, const void* proj, int64_t row_stri
   if (num_tokens <= 0) return 0;
   dim3 grid(num_tokens, nh + 2 * nkv);
   dim3 tail_grid((unsigned)((C + 255) / 256), num_seqs);
-  // many rows, heads that two numbers a lane hold, the usual numbers of taps: by wavefronts of eight rows
-  const bool by_rows = num_tokens >= CONV_ROWS_FROM && hd <= 2 * PAE_WAVE && vd <= 2 * PAE_WAVE && taps >= 2 && taps <= 4 &&
+  // many rows, heads that two numbers a lane hold, the usual numbers of taps: by wavefronts of eight rows.  Row by row / by eight
+  // rows: 384 rows of 16 heads of 128 9.7 / 10.4 us, 512 11.0 / 10.3; 1,024 of 6 heads of 64 8.6 / 10.1, 1,536 10.8 / 10.1; 256 of
+  // 36 heads of 128 11.9 / 10.2
+  const bool by_rows = num_tokens >= CONV_ROWS_FROM && (int64_t)num_tokens * (nh + 2 * nkv) >= CONV_PAIRS_FROM && hd <= 2 * PAE_WAVE && vd <= 2 * PAE_WAVE && taps >= 2 && taps <= 4 &&
                        (uintptr_t)v_cache % 16 == 0;
   const dim3 rows_grid((num_tokens + 4 * CONV_ROWS - 1) / (4 * CONV_ROWS), nh + 2 * nkv);
 #define CONV_ROWS_LAUNCH(T, TAPS)                                                                                         \

@@ -159,13 +159,14 @@ def test_convolution_norm_and_store_whole_and_cut_anywhere(dtype, H, G, D, V, ta
 @pytest.mark.parametrize("H,G,D,V,taps,bs", [(2, 2, 16, 24, 3, 16), (3, 1, 128, 128, 4, 16), (1, 2, 65, 127, 2, 8), (2, 1, 40, 64, 4, 4),
                                              (4, 0, 64, 64, 3, 16)])
 def test_convolution_and_store_of_many_rows_give_the_bits_of_few(dtype, H, G, D, V, taps, bs):
-    """A step of 301 rows (by wavefronts of eight) against the same sequences one step each (fewer than 256 rows: row by
-    row): runs that begin and end inside eight rows, inputs from the state, pages shorter than eight rows or entered off
-    their start."""
+    """A step of over 8,192 (row, head) pairs (by wavefronts of eight rows) against the same sequences in steps of their own of up to
+    200 rows (row by row): runs that begin and end inside eight rows, inputs from the state, pages shorter than eight rows
+    or entered off their start."""
     K = _K()
     gen = torch.Generator().manual_seed(D + taps)
-    lens, pasts = (131, 1, 9, 160), (0, 5, 16, 3)
+    lens, pasts = (131, 1, 9, 1910), (0, 5, 16, 3)
     T, S, C = sum(lens), len(lens), H * D + G * (D + V)
+    assert T * (H + 2 * G) >= 8192
     rows, conv = randn(gen, T, C + 8).to(dtype).to(DEV), randn(gen, C, taps, scale=0.6).float().to(DEV)
     width = max(-(-(a + n) // bs) for a, n in zip(pasts, lens))
     tables = torch.randperm(S * width, generator=gen).to(torch.int32).view(S, width).to(DEV)
@@ -175,15 +176,19 @@ def test_convolution_and_store_of_many_rows_give_the_bits_of_few(dtype, H, G, D,
     ints = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
     positions = torch.cat([torch.arange(a, a + n) for a, n in zip(pasts, lens)]).to(torch.int32).to(DEV)
     got = []
-    for steps in ([range(S)], [[s] for s in range(S)]):
+    # steps of (sequence, its first row in the step, rows)
+    pieces = [[(s, at, min(200, lens[s] - at))] for s in range(S) for at in range(0, lens[s], 200)]
+    for steps in ([[(s, 0, lens[s]) for s in range(S)]], pieces):
         kc, vc = (torch.zeros(S * width, max(G, 1), *shape, dtype=dtype, device=DEV) for shape in ((bs, D), (V, bs)))
         state, q = tail.to(DEV), torch.zeros(T, H * D, dtype=dtype, device=DEV)
         for step in steps:
-            a, b = starts[step[0]], starts[step[-1]] + lens[step[-1]]
-            seqs = torch.cat([torch.full((lens[s],), i) for i, s in enumerate(step)]).to(torch.int32).to(DEV)
-            runs = runs_tensor([(starts[s] - a, lens[s], pasts[s]) for s in step])
-            own = tables[step[0]:step[-1] + 1].contiguous()
-            K.conv_norm_store(rows[a:b], q[a:b], seqs, positions[a:b].contiguous(), runs, ints(list(step)), conv, state, taps, H, G, D, V,
+            a = starts[step[0][0]] + step[0][1]
+            b = starts[step[-1][0]] + step[-1][1] + step[-1][2]
+            seqs = torch.cat([torch.full((n,), i) for i, (_, _, n) in enumerate(step)]).to(torch.int32).to(DEV)
+            runs = runs_tensor([(starts[s] + at - a, n, pasts[s] + at) for s, at, n in step])
+            live = [s for s, _, _ in step]
+            own = tables[live[0]:live[-1] + 1].contiguous()
+            K.conv_norm_store(rows[a:b], q[a:b], seqs, positions[a:b].contiguous(), runs, ints(live), conv, state, taps, H, G, D, V,
                               True, 1e-5, own if G else None, bs, kc if G else None, vc if G else None)
         got.append([t.cpu() for t in (q, kc, vc, state)])
     for many, few in zip(*got):
