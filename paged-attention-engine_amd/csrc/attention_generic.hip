@@ -121,20 +121,20 @@ __global__ void paged_attention_generic_kernel(
   }
 }
 
-// The same for float32 rows that can be read four numbers at a time: a workgroup of four wavefronts takes up to 16 (token,
+// The same for float32 rows that can be read four numbers at a time: a workgroup of eight wavefronts takes up to 16 (token,
 // query head) rows that share a key/value head, and walks the chunks of 64 keys that any of them
 // sees.  A chunk's keys and values come to LDS once, by 16-byte loads, the next chunk's on their way
-// meanwhile; a wavefront computes up to four rows together, lane = key for the scores, lane = feature for
-// the sums, so that a key or value read from LDS serves four rows.  Every row does the operations of the
+// meanwhile; a wavefront computes up to two rows together, lane = key for the scores, lane = feature for
+// the sums, so that a key or value read from LDS serves two rows.  Every row does the operations of the
 // kernel above in its order and over its own keys only: the bits are the same, and a row never touches a
 // key it does not see.
 //
 // What bound the kernel above: every lane read its own key row number by number (64 rows of 512 bytes, a
 // load instruction per number), and every (token, head) read the keys and values again.  Measured, 12 heads over 2
-// of 128, float32: three prompts of 601 tokens in all 700 -> 68 us, a token each behind them 55 -> 37 us.  What is
-// left is the chain of a workgroup's chunks, 6 us each.  Loads under conditions (keys beside those in sight) had
-// the compiler wait for each in turn: 140 us for the prompts.  Eight wavefronts of two rows against four of four: 43
-// against 69 us a launch.
+// of 128, float32: three prompts of 601 tokens in all 262 -> 58 us, a token each behind them 92 -> 27, one prompt of 601 tokens 647 ->
+// 117, eight single tokens at 4,096 1,551 -> 338.  What is left is the chain of a workgroup's chunks, 5 us each.  Loads
+// under conditions (keys beside those in sight) had the compiler wait for each in turn (twice the time for prompts), and
+// four wavefronts of four rows instead of eight of two took half as long again.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 #define PAE_ROWS_WAVES 8
@@ -394,7 +394,7 @@ __global__ __launch_bounds__(PAE_WAVE * PAE_ROWS_WAVES) void paged_attention_row
 }
 
 // Whether the rows kernel takes a call: rows and pages that can be read four numbers at a time, and a chunk's keys and values
-// in half a compute unit's LDS (heads of up to 128 wide) or at least in all of it.
+// in a compute unit's LDS (150 KB at heads of 256).
 static bool rows_kernel_takes(const void* k_cache, const void* v_cache, int bs, int hd, int vd, int shared_kv) {
   return !shared_kv && bs % 4 == 0 && (bs >= PAE_WAVE ? bs % PAE_WAVE == 0 : PAE_WAVE % bs == 0) && hd % 4 == 0 && vd <= 256 &&
          hd <= 256 && (uintptr_t)k_cache % 16 == 0 && (uintptr_t)v_cache % 16 == 0;
@@ -412,7 +412,17 @@ static int launch_rows(float* out, int64_t out_stride, const float* q, int64_t q
   const int toks = (int64_t)num_tokens * nkv * parts >= 512 ? PAE_ROWS_MOST / heads_each : 1;
   const dim3 grid((num_tokens + toks - 1) / toks, nkv * parts);
   const size_t lds = (size_t)(PAE_WAVE * (hd + 4 + vd + 4) + PAE_ROWS_MOST * (PAE_WAVE + hd)) * sizeof(float);
-#define PAE_LAUNCH(MAXD)                                                                                           do {                                                                                                               if (lds > 65536) {                                                                                                 const hipError_t err = hipFuncSetAttribute((const void*)paged_attention_rows_kernel<MAXD>,                                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);                if (err != hipSuccess) return pae_fail("attention: %zu bytes of LDS refused: %s", lds, hipGetErrorString(err));     }                                                                                                                paged_attention_rows_kernel<MAXD><<<grid, PAE_WAVE * PAE_ROWS_WAVES, lds, stream>>>(                                 out, out_stride, q, q_stride, k_cache, v_cache, positions, tok_seq, block_tables, max_blocks, bs,                num_tokens, nh, nkv, hd, vd, scale, window, cap, sinks, chunked, slopes, gate, gate_stride,                      gate_per_head, toks, heads_each);                                                                          } while (0)
+#define PAE_LAUNCH(MAXD)                                                                                              \
+  do {                                                                                                                \
+    if (lds > 65536) {                                                                                                \
+      const hipError_t err = hipFuncSetAttribute((const void*)paged_attention_rows_kernel<MAXD>,                      \
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);               \
+      if (err != hipSuccess) return pae_fail("attention: %zu bytes of LDS refused: %s", lds, hipGetErrorString(err)); \
+    }                                                                                                                 \
+    paged_attention_rows_kernel<MAXD><<<grid, PAE_WAVE * PAE_ROWS_WAVES, lds, stream>>>(                              \
+        out, out_stride, q, q_stride, k_cache, v_cache, positions, tok_seq, block_tables, max_blocks, bs, num_tokens, \
+        nh, nkv, hd, vd, scale, window, cap, sinks, chunked, slopes, gate, gate_stride, gate_per_head, toks, heads_each); \
+  } while (0)
   const int wide = hd > vd ? hd : vd;
   if (wide <= 64) PAE_LAUNCH(1);
   else if (wide <= 128) PAE_LAUNCH(2);

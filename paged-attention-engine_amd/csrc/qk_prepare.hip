@@ -106,7 +106,7 @@ __global__ __launch_bounds__(256) void qk_norm_rotate_store_kernel(
 // for before the sums are known; the row goes to LDS in float32 once, where the sums per head and the other
 // half of a rotated pair find it (the same bits).  On a few tokens the kernel above takes four trips to memory, number by number.
 // Measured, 12 query and 2 key heads of 128, bfloat16: 9 rows 11.5 -> 6.5 us, with one sum over each projection 10.5 -> 6.4.
-// (A row of more than 1,024 chunks or 64 KB in float32 stays above.)
+// (A row of more than 1,024 chunks stays above; 1,024 are at most 32 KB in float32.)
 template <typename T, int TRIPS>  // at most 256 * TRIPS chunks of queries and keys
 __global__ __launch_bounds__(256) void qk_norm_rotate_store_vec_kernel(
     T* __restrict__ qkv, int64_t row_stride, int nh, int nkv, int hd, int vd, const void* __restrict__ q_w,
@@ -259,8 +259,8 @@ extern "C" int pae_qk_norm_rotate_store(int dtype, void* qkv, int64_t row_stride
   const int chunk = dtype == PAE_F32 ? 4 : 8, elem = dtype == PAE_F32 ? 4 : 2;
   const int64_t chunks = (int64_t)(nh + nkv) * hd / chunk;
   const size_t wide_lds = ((size_t)(nh + nkv) * hd + nh + nkv) * sizeof(float);
-  if (hd % chunk == 0 && row_stride % chunk == 0 && (uintptr_t)qkv % 16 == 0 && (uintptr_t)k_cache % 16 == 0 && wide_lds <= 65536 &&
-      chunks <= 1024 && (uintptr_t)cos_sin % 8 == 0 && (!q_w || ((uintptr_t)q_w % 16 == 0 && (uintptr_t)k_w % 16 == 0)) && (dtype == PAE_F32 || dtype == PAE_BF16)) {
+  if (hd % chunk == 0 && row_stride % chunk == 0 && (uintptr_t)qkv % 16 == 0 && (uintptr_t)k_cache % 16 == 0 && chunks <= 1024 &&
+      (uintptr_t)cos_sin % 8 == 0 && (!q_w || ((uintptr_t)q_w % 16 == 0 && (uintptr_t)k_w % 16 == 0)) && (dtype == PAE_F32 || dtype == PAE_BF16)) {
 #define QK_VEC(T, TRIPS)                                                                                                   \
   qk_norm_rotate_store_vec_kernel<T, TRIPS><<<num_tokens, 256, wide_lds, stream>>>(                                        \
       (T*)qkv, row_stride, nh, nkv, hd, vd, q_w, k_w, w_is_f32, eps, rot, interleaved, cos_sin, magnitude, positions,      \

@@ -29,7 +29,8 @@ constexpr int LDS_BYTES = STAGES * STAGE_BYTES;
 constexpr int A_LOADS = BM / 8 / 4, W_LOADS = BN / 8 / 4;  // of 8 rows, that a wavefront makes a stage
 
 // One load of 64 lanes x 16 bytes to LDS at `lds` (the same in every lane), lane by lane in a row.  It is not a load to the
-// compiler: the waits for it are written below.
+// compiler: the waits for it are written below.  It sets m0, which cannot be named as changed (the compiler reserves it): kernels
+// that use this must have nothing else that goes through m0, as the compiler's own loads to LDS, indexed register moves or messages do.
 __device__ __forceinline__ void load_to_lds(uint32_t lds, uint32_t offset, const void* base) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds), "v"(offset), "s"(base) : "memory");
 }

@@ -89,8 +89,8 @@ def test_gemm_plain(dtype, M, N, K_):
 @pytest.mark.parametrize("N,K_", [(15, 4), (17, 508), (130, 512), (64, 516), (200, 1040), (33, 4100), (16, 5002), (1536, 8960),
                                   (40000, 1030)])
 def test_gemm_plain_adds_in_one_order(N, K_):
-    """Every kernel and every way to share k out gives a row the same bits: few rows (up to 16, 32 and 64), tiles of 64 and
-    of 128 rows, one workgroup a tile or several, rows read by fours or one by one; and the error against 64
+    """Every kernel and every way to share k out gives a row the same bits: few rows (up to 16, 32 and 64), tiles of 64
+    rows, one workgroup a tile or several, rows read by fours or one by one; and the error against 64
     bits is that of 512 products added in a row: 512 roundings of half a unit in the last place, of the
     sum of the products' sizes, most of which cancel (a quarter of it bounds what is seen by far)."""
     torch.manual_seed(N + K_)
