@@ -351,20 +351,24 @@ __global__ __launch_bounds__(256, 1) void attn_prefill_split_kernel(
   const int lrow = lane / 4, lgrp = lane % 4;
   const int fetch_from = ((lane % 16) * 4 + lane / 16) * 4;
   bf16x8 kf[2][HD / 32], vf[VD / 16];
-  // The first unit begins up to 31 keys before the first one that is seen: sixteens of keys that lie wholly before it are read as the
-  // one that holds it, whose page is the sequence's own.  (Their weights are zero, but the table may hold no page there any
-  // more, -1, and zero times what lies in another sequence's page may be no number.)
+  // The first unit begins up to 31 keys before the first one that is seen, and a page that lies wholly before it was given
+  // back (its entry is -1): such keys are read as the sixteen that holds the first one seen, which is the sequence's own.  (Their
+  // weights are zero, but zero times what lies in another sequence's page may be no number.)
   const int first_16 = (BIASED ? first_visible(pos0, window, chunked) : (window > 0 && pos0 - window + 1 > 0) ? pos0 - window + 1 : 0) / 16 * 16;
-  auto key_read = [&](int key0, int p) {
+  const int first_page = max(table[first_16 / bs], 0);
+  auto sixteen_of = [&](int key0, int p, int& offset) -> int64_t {  // in units of one head's page; keys 16 p .. of the unit begin there
     const int key = key0 + 16 * p;
-    return max(key <= hi ? key : key0, first_16);  // a tile past the end repeats the first one (all of it is masked)
+    const int kc = key <= hi ? key : key0;  // a tile past the end repeats the first one (all of it is masked)
+    const int page = table[kc / bs];
+    offset = BS == 16 ? 0 : (page < 0 ? first_16 : kc) % bs;
+    return (int64_t)(page < 0 ? first_page : page) * nkv + kvh;
   };
-  auto page_of = [&](int kc) -> int64_t { return (int64_t)max(table[kc / bs], 0) * nkv + kvh; };  // in units of one head's page
   auto load_keys = [&](int key0) {
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
-      const int kc = key_read(key0, p);
-      const bf16_t* kp = k_cache + page_of(kc) * (bs * HD) + (int64_t)(kc % bs) * HD;
+      int offset;
+      const bf16_t* kp = k_cache + sixteen_of(key0, p, offset) * (bs * HD);
+      kp += (int64_t)offset * HD;
 #pragma unroll
       for (int j = 0; j < HD / 32; ++j) kf[p][j] = *reinterpret_cast<const bf16x8*>(kp + lrow * HD + 32 * j + 8 * lgrp);
     }
@@ -373,8 +377,9 @@ __global__ __launch_bounds__(256, 1) void attn_prefill_split_kernel(
     const bf16_t* vp[2];
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
-      const int kc = key_read(key0, p);
-      vp[p] = v_cache + page_of(kc) * (bs * VD) + kc % bs;
+      int offset;
+      vp[p] = v_cache + sixteen_of(key0, p, offset) * (bs * VD);
+      vp[p] += offset;
     }
 #pragma unroll
     for (int t = 0; t < VD / 16; ++t)  // in the order of their use
