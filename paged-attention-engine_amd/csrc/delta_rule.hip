@@ -193,6 +193,13 @@ __global__ __launch_bounds__(256) void delta_recurrence_kernel(
 // lane keeps the read-outs of the tokens of its number until the chunk's end instead of a store by one lane a step.  What
 // bounds it now is the issue of a step's 52 vector instructions by the one wavefront a SIMD has.  Measured, 12 heads
 // of 128 x 128: 2,048 tokens of one sequence 544 -> 307 us (the same bits).
+//
+// Steps in which no run can hold a whole chunk (decoding) have a kernel without the unrolled part (WHOLE off): that takes 130 to 148
+// registers where the loop by tokens takes 75 to 90, and with many sequences, whose states' way from memory and back is the
+// time, wavefronts are then missing (the whole delta step for 64 sequences of one token 48.8 us with it, 43.0 without; with 28 heads
+// 91 and 75).  The host knows a step's tokens and sequences, not its longest run: many runs of 3 to 15 tokens side by side pay for the
+// chunk that none of them fills (64 of three 46 -> 55 us).  Unrolling two or four tokens at a time takes 111 to 130
+// registers and half of what a long run gains (2,048 tokens 352 us all 16, 434 four, 442 two, 611 before).
 template <int L>
 __device__ __forceinline__ float group_sum(float v) {
   v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, true));  // lanes (1, 0, 3, 2) of a quad
@@ -202,7 +209,7 @@ __device__ __forceinline__ float group_sum(float v) {
   return v;
 }
 
-template <int R, int L, int CH, bool CHANNEL, bool DELTA>
+template <int R, int L, int CH, bool CHANNEL, bool DELTA, bool WHOLE>
 __global__ __launch_bounds__(16 * L) void delta_recurrence_group_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v, const float* __restrict__ beta,
     const float* __restrict__ decay, const int4* __restrict__ seq_runs, const int* __restrict__ slots,
@@ -337,7 +344,7 @@ __global__ __launch_bounds__(16 * L) void delta_recurrence_group_kernel(
     __syncthreads();
     if (first + CH < run.y) fetch(first + CH);
     const int n = min(CH, run.y - first);
-    if (n == CH) {
+    if (WHOLE && n == CH) {
       Token cur = token(0);
       float kept[CH / L];  // lane `sub` keeps the read-outs of tokens sub, sub + L, ... until the chunk's end
 #pragma unroll
@@ -351,8 +358,40 @@ __global__ __launch_bounds__(16 * L) void delta_recurrence_group_kernel(
 #pragma unroll
         for (int j = 0; j < CH / L; ++j) out[((int64_t)(run.x + first + j * L + sub) * H + h) * V + col] = kept[j];
     } else {
-      for (int i = 0; i < n; ++i) {
-        const float o = step(token(i));
+      for (int i = 0; i < n; ++i) {  // (a number is read where it is used: what waits for its use is registers)
+        const float* kt = s_k + i * DP;
+        const float* qt = s_q + i * DP;
+        const float dec = s_bd[CH + i], b = s_bd[i], vt = s_v[i * 16 + tid / L];
+        float kr[R], dot = 0.f, o = 0.f;
+#pragma unroll
+        for (int r4 = 0; r4 < R / 4; ++r4) {
+          const f32x4 k4 = *reinterpret_cast<const f32x4*>(kt + r4 * (4 * L) + sub * 4);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) kr[4 * r4 + e] = k4[e];
+        }
+#pragma unroll
+        for (int r4 = 0; r4 < R / 4; ++r4) {
+          f32x4 d4 = {dec, dec, dec, dec};
+          if (CHANNEL) d4 = *reinterpret_cast<const f32x4*>(s_dec + i * DP + r4 * (4 * L) + sub * 4);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) S[4 * r4 + e] *= d4[e];
+        }
+        if (DELTA) {
+#pragma unroll
+          for (int r = 0; r < R; ++r) dot = fmaf(S[r], kr[r], dot);
+          dot = group_sum<L>(dot);
+        }
+        const float u = DELTA ? b * (vt - dot) : b * vt;
+#pragma unroll
+        for (int r4 = 0; r4 < R / 4; ++r4) {
+          const f32x4 q4 = *reinterpret_cast<const f32x4*>(qt + r4 * (4 * L) + sub * 4);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            S[4 * r4 + e] = fmaf(kr[4 * r4 + e], u, S[4 * r4 + e]);
+            o = fmaf(S[4 * r4 + e], q4[e], o);
+          }
+        }
+        o = group_sum<L>(o);
         if (live && sub == 0) out[((int64_t)(run.x + first + i) * H + h) * V + col] = o;
       }
     }
@@ -405,18 +444,24 @@ int pae_launch_gated_norm(int dtype, const float* o, const void* gates, int64_t 
 static int lanes_per_column(int D, int R);
 void pae_launch_recurrence(const float* q, const float* k, const float* v, const float* beta, const float* decay,
                            const int4* runs, const int* slots, float* state, int64_t state_slot_stride, int G, int H,
-                           int D, int V, int num_seqs, int channel_decay, int delta, float* o, hipStream_t stream);
+                           int D, int V, int num_tokens, int num_seqs, int channel_decay, int delta, float* o, hipStream_t stream);
 
 // The recurrence over a step's rows for every (sequence, head, column of S).  `channel_decay`: `decay` is
 // [T][H][D] instead of [T][H]; `delta` off: u = beta v (a state that only adds; with `channel_decay` only).
 void pae_launch_recurrence(const float* q, const float* k, const float* v, const float* beta, const float* decay,
                            const int4* runs, const int* slots, float* state, int64_t state_slot_stride, int G, int H,
-                           int D, int V, int num_seqs, int channel_decay, int delta, float* o, hipStream_t stream) {
+                           int D, int V, int num_tokens, int num_seqs, int channel_decay, int delta, float* o, hipStream_t stream) {
   dim3 group_grid((V + 15) / 16, H, num_seqs);
   // (rows a lane, lanes a column, tokens a chunk)
-#define GROUP_AS(R, L, CH, CHANNEL, DELTA)                                                                        \
-  delta_recurrence_group_kernel<R, L, CH, CHANNEL, DELTA><<<group_grid, 16 * L, 0, stream>>>(                     \
+#define GROUP_OF(R, L, CH, CHANNEL, DELTA, WHOLE)                                                                 \
+  delta_recurrence_group_kernel<R, L, CH, CHANNEL, DELTA, WHOLE><<<group_grid, 16 * L, 0, stream>>>(              \
       q, k, v, beta, decay, runs, slots, state, state_slot_stride, G, H, D, V, o)
+  // (runs of a token at least, the longest has at most the step's tokens less one for each of the others)
+#define GROUP_AS(R, L, CH, CHANNEL, DELTA)                                              \
+  do {                                                                                  \
+    if (num_tokens - num_seqs + 1 < CH) GROUP_OF(R, L, CH, CHANNEL, DELTA, false);      \
+    else GROUP_OF(R, L, CH, CHANNEL, DELTA, true);                                      \
+  } while (0)
 #define GROUP(R, L, CH)                                       \
   do {                                                        \
     if (channel_decay && delta) GROUP_AS(R, L, CH, true, true);      \
@@ -436,6 +481,7 @@ void pae_launch_recurrence(const float* q, const float* k, const float* v, const
   }
 #undef GROUP
 #undef GROUP_AS
+#undef GROUP_OF
 }
 
 static int lanes_per_column(int D, int R) {
@@ -483,7 +529,7 @@ extern "C" int pae_delta_rule_step(int dtype, const void* proj, int64_t row_stri
   if (taps > 1)                                                                                                         \
     delta_conv_tail_kernel<T><<<tail_grid, 256, 0, stream>>>((const T*)proj, row_stride, runs, slots, conv_tail,        \
                                                              tail_slot_stride, taps, (int)C);                           \
-  pae_launch_recurrence(q, k, v, beta, decay, runs, slots, state, state_slot_stride, G, H, D, V, num_seqs,              \
+  pae_launch_recurrence(q, k, v, beta, decay, runs, slots, state, state_slot_stride, G, H, D, V, num_tokens, num_seqs,  \
                         channel_decay, 1, o, stream);                                                                   \
   delta_gated_norm_kernel<T><<<norm_grid, PAE_WAVE, 0, stream>>>(o, (const T*)gate_in, gate_stride, gate_sigmoid,       \
                                                                  norm_w, w_is_f32, norm_eps, H, V, (T*)out)

@@ -23,7 +23,7 @@
 
 void pae_launch_recurrence(const float* q, const float* k, const float* v, const float* beta, const float* decay,
                            const int4* runs, const int* slots, float* state, int64_t state_slot_stride, int G, int H,
-                           int D, int V, int num_seqs, int channel_decay, int delta, float* o, hipStream_t stream);
+                           int D, int V, int num_tokens, int num_seqs, int channel_decay, int delta, float* o, hipStream_t stream);
 int pae_launch_gated_norm(int dtype, const float* o, const void* gates, int64_t gate_stride, int gate_sigmoid,
                           const void* weight, int w_is_f32, float eps, int num_tokens, int H, int V, void* out,
                           hipStream_t stream);
@@ -88,7 +88,7 @@ extern "C" int pae_linear_attention_step(int dtype, const void* proj, int64_t ro
   else
     gla_prepare_kernel<bf16_t><<<token_heads, 128, 0, stream>>>((const bf16_t*)proj, row_stride, (const bf16_t*)z_in, z_stride,
                                                                 z_bias, bias_is_f32, 1.0f / tau, H, D, V, q, k, v, decay, ones);
-  pae_launch_recurrence(q, k, v, ones, decay, runs, slots, state, state_slot_stride, H, H, D, V, num_seqs, 1, 0, o, stream);
+  pae_launch_recurrence(q, k, v, ones, decay, runs, slots, state, state_slot_stride, H, H, D, V, num_tokens, num_seqs, 1, 0, o, stream);
   const int code = pae_launch_gated_norm(dtype, o, gate_in, gate_stride, gate_sigmoid, norm_w, w_is_f32, norm_eps,
                                          num_tokens, H, V, out, stream);
   if (code) return code;

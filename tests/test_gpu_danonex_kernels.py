@@ -331,3 +331,37 @@ def test_the_few_row_product_with_an_activation_on_its_sums(rows, kind):
         K.gemm_skinny_act(out, a.to(DEV), w.to(DEV), kind, splits)
         err = (out.double().cpu() - want).abs().max()
         assert float(err) <= 2.0 ** -8 * float(want.abs().max()), (splits, float(err))
+
+
+@pytest.mark.parametrize("channel", [False, True])
+@pytest.mark.parametrize("D,V", [(16, 24), (32, 32), (64, 20), (128, 128), (200, 48)])
+def test_the_delta_rule_of_whole_chunks_gives_the_bits_of_token_by_token(D, V, channel):
+    """Runs of up to two chunks of 32 (or 16) tokens and a remainder in one step, where whole chunks are worked through unrolled, against
+    the same tokens in steps in which no run can hold a chunk, which have a kernel without that part; beside a single token,
+    and with as many tokens as make a chunk possible and one less."""
+    from paged_attention_engine_amd.kernels import lib
+
+    gen = torch.Generator().manual_seed(D + V)
+    G, H, taps, T = 2, 4, 4, 78
+    C, nd = 2 * G * D + H * V, H * D if channel else H
+    put = lambda *shape: torch.randn(*shape, generator=gen).to("cuda:0")
+    proj, gate, beta, decay, conv, state0 = put(T + 1, C), put(T + 1, H * V), put(T + 1, H), put(T + 1, nd), put(C, taps), put(2, H, V, D)
+    a_log, dt, norm = put(H), put(nd), put(V)
+    got = []
+    for steps in ((T,), (31, 32, 15), (15,) * 5 + (3,), (15, 16, 17, 30)):
+        tail, state, out = torch.zeros(2, taps - 1, C, device="cuda:0"), state0.clone(), torch.full((T + 1, H * V), float("nan"), device="cuda:0")
+        at = 0
+        for n in steps:
+            lone = at == 0  # the other sequence brings its one token with the first step
+            rows = torch.tensor(([T] if lone else []) + list(range(at, at + n)), device="cuda:0")
+            runs = ([[0, 1, 0, 0]] if lone else []) + [[int(lone), n, at, 0]]
+            ints = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda:0")
+            here = torch.empty(len(rows), H * V, device="cuda:0")
+            lib.delta_rule_step(proj[rows], here, ints(([0] if lone else []) + [len(runs) - 1] * n), ints(([0] if lone else []) + list(range(at, at + n))),
+                                ints(runs), ints(([1] if lone else []) + [0]), conv, tail, state, a_log, dt, norm, G, H, D, V, taps, 1e-6, 1e-6,
+                                gate[rows], beta[rows], decay[rows], channel)
+            out[rows] = here
+            at += n
+        got.append((out, state, tail))
+    for one_way in got[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(got[0], one_way)) and torch.isfinite(got[0][0]).all()
