@@ -463,10 +463,10 @@ extern "C" int pae_gemm_plain_shared(int in_dtype, int out_dtype, void* C, int64
   PAE_REQUIRE(lda >= K && ldc >= N, "gemm: leading dimensions lda=%lld ldc=%lld too small for K=%d N=%d",
               (long long)lda, (long long)ldc, K, N);
   PAE_REQUIRE(batch == 1 || !scratch, "gemm: shares of k go with one product at a time, not with %d", batch);
-  PAE_REQUIRE((in_dtype == PAE_F32 && out_dtype == PAE_F32) || (in_dtype == PAE_BF16 && (out_dtype == PAE_BF16 || out_dtype == PAE_F32)),
-              "gemm: unsupported dtype pair in=%d out=%d", in_dtype, out_dtype);
   if (M == 0) return 0;
   PAE_REQUIRE(M <= 65535 * 64, "gemm: M=%d exceeds the grid", M);
+  PAE_REQUIRE((in_dtype == PAE_F32 && out_dtype == PAE_F32) || (in_dtype == PAE_BF16 && (out_dtype == PAE_BF16 || out_dtype == PAE_F32)),
+              "gemm: unsupported dtype pair in=%d out=%d", in_dtype, out_dtype);
   // four numbers at a time: 16 bytes in float32, 8 in bfloat16
   const int elem = in_dtype == PAE_F32 ? 4 : 2, out_elem = out_dtype == PAE_F32 ? 4 : 2;
   const bool vec = K % 4 == 0 && lda % 4 == 0 && (batch == 1 || (batch_a % 4 == 0 && batch_w % 4 == 0)) &&

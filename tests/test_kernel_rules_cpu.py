@@ -48,3 +48,8 @@ def test_large_tiles_of_experts_are_counted_in_fifteen_bits():
     assert [rows(n, 1536, 2240, 3072) for n in (512, 513, 4096, 4097, 12004)] == [16, 64, 64, 128, 128]
     assert rows(0x7fff * 128, 64, 64, 128) == 128 and rows(0x7fff * 128 + 1, 64, 64, 128) == 64
     assert rows(1 << 20, 4096, 2240, 8192) == 64 and rows(8192, 1536, 2240 + 32, 3072) == 64
+
+
+def test_a_product_of_no_rows_is_done_whatever_its_types():
+    for pair in ((0, 0), (1, 1), (1, 0), (0, 1)):
+        assert K.library().pae_gemm_plain_shared(*pair, None, 8, 0, None, 8, 0, None, 0, None, 0, 0, 8, 8, 1, None, None) == 0
