@@ -132,7 +132,8 @@ __global__ void paged_attention_generic_kernel(
 // What bound the kernel above: every lane read its own key row number by number (64 rows of 512 bytes, a
 // load instruction per number), and every (token, head) read the keys and values again.  Measured, 12 heads over 2
 // of 128, float32: three prompts of 601 tokens in all 262 -> 58 us, a token each behind them 92 -> 27, one prompt of 601 tokens 647 ->
-// 117, eight single tokens at 4,096 1,551 -> 338.  What is left is the chain of a workgroup's chunks, 5 us each.  Loads
+// 117, eight single tokens at 4,096 1,551 -> 338; 8 heads over 2 of 256, where six of 256 registers do not fit and lie in memory, 399 -> 77,
+// 177 -> 47, 900 -> 132, 2,534 -> 521.  What is left is the chain of a workgroup's chunks, 5 us each.  Loads
 // under conditions (keys beside those in sight) had the compiler wait for each in turn (twice the time for prompts), and
 // four wavefronts of four rows instead of eight of two took half as long again.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -215,6 +216,10 @@ __global__ __launch_bounds__(PAE_WAVE * PAE_ROWS_WAVES) void paged_attention_row
       const int first = window <= 0 ? 0 : (chunked ? p - p % window : (p - window + 1 > 0 ? p - window + 1 : 0));
       low = min(low, first);
       high = max(high, p);
+    }
+    if (high < low) {  // tokens that see no key, position -1: their table need not name a page
+      at = next;
+      continue;
     }
     const int* table = block_tables + (int64_t)s * max_blocks;
     // A chunk's keys and values, four numbers at a time (keys [key][feature], values [page][feature][offset]); what a

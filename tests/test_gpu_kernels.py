@@ -749,6 +749,25 @@ def test_generic_attention(dtype, nh, nkv, hd, bs, window):
     assert (got - want).abs().max() <= (1e-5 if dtype == "float32" else 3e-2)
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_generic_attention_of_a_token_that_sees_no_key(dtype):
+    # position -1 under a table that names no page, alone in its sequence, beside a token with keys: no number, and no page is read
+    nh, nkv, hd, bs = 4, 2, 32, 16
+    torch.manual_seed(3)
+    kp, vp = torch.randn(2, nkv, bs, hd).to(DT[dtype]), torch.randn(2, nkv, hd, bs).to(DT[dtype])
+    q = torch.randn(3, nh, hd).to(DT[dtype])
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    out = torch.zeros(3, nh * hd, dtype=DT[dtype], device=DEV)
+    K().paged_attention_generic(out, q.view(3, -1).to(DEV), kp.to(DEV), vp.to(DEV), i32([20, -1, 20]), i32([0, 1, 0]),
+                                i32([[1, 0], [-1, -1]]), nh, nkv, hd, hd ** -0.5, 0)
+    keys = torch.cat([kp[1].transpose(0, 1), kp[0].transpose(0, 1)])  # [position][kv head][hd]
+    values = torch.cat([vp[1].permute(2, 0, 1), vp[0].permute(2, 0, 1)])
+    for t in (0, 2):
+        want = reference_attention(q[t].float(), keys.float(), values.float(), 20, hd ** -0.5, 0).reshape(-1)
+        assert (out[t].double().cpu() - want).abs().max() <= (1e-5 if dtype == "float32" else 3e-2)
+    assert torch.isnan(out[1]).all()
+
+
 MFMA_SHAPES = [(12, 2, 128, 16, 0), (14, 2, 64, 16, 0), (4, 4, 32, 16, 0), (16, 1, 96, 32, 0),
                (7, 1, 256, 16, 0), (12, 2, 128, 16, 100), (6, 3, 64, 32, 33), (5, 1, 160, 16, 0)]
 
