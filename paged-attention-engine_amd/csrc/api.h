@@ -39,6 +39,9 @@ int pae_gemm_plain_shared(int in_dtype, int out_dtype, void* C, int64_t ldc, int
 int pae_gemm_plain_batched(int in_dtype, int out_dtype, void* C, int64_t ldc, int64_t batch_c, const void* A, int64_t lda,
                            int64_t batch_a, const void* W, int64_t batch_w, const void* bias, int b_is_f32, int M, int N,
                            int K, int batch, hipStream_t stream);
+int pae_gemm_wide_plan(int mode, int act, int M, int N, int K, int ranges);  // shape | ranges of k << 8, or -1: the platform library
+int pae_gemm_wide(int mode, int act, int plan, void* out, int64_t ldc, const void* a, int64_t lda, const void* w, const void* bias,
+                  int b_is_f32, int M, int N, int K, hipStream_t stream);
 int pae_gemm_skinny(int epilogue, void* out, int64_t ldc, const void* A, int64_t lda, const void* W,
                     const void* bias, int b_is_f32, int M, int N, int K, int splits, int64_t part_stride,
                     float* ticket_parts, int* ticket_counters, const float* row_stats, int row_stat_tiles,

@@ -1,0 +1,349 @@
+// bfloat16 products with many rows, C = A W^T, on the matrix cores: the loops of wide_gemm.h, with what follows a product in the
+// epilogue: a bias and an activation, a gated activation, or the sums of a range of k as they are.
+//
+// A launch is either the tiles of 256 x 256 as long as they fill rounds of the chip's 256 compute units, then what is left over
+// of them whole, in halves or in quarters, where these still make one round; or, where that leaves too many units
+// idle, smaller tiles throughout, whose k may be cut into ranges that leave float32 sums of their own.  Which one is the
+// least of what the shapes' measured times say (pae_gemm_wide_plan).
+//
+// Measured beside the platform library's product (weights from memory, us; rows x features x k):
+//     2,048 x 17,920 x  1,536   library 111 and 22 for the gate behind it    here with the gate 100
+//     2,048 x  1,536 x  8,960           71                                   66
+//     2,048 x  2,048 x  1,536           19                                   15
+//     6,030 x 37,888 x  3,584        1,209 and 117 for the gate              1,176 with the gate
+//     6,030 x  3,584 x 18,944        1,041                                   600
+//       601 x  1,536 x  8,960           36                                   24 in three ranges of k
+//       200 x  1,536 x  1,536           20                                   8
+#include "wide_gemm.h"
+#include "api.h"
+
+#include <type_traits>
+
+using wide_gemm::bf16x4;
+using wide_gemm::bf16x8;
+using wide_gemm::f32x4;
+using wide_gemm::Large;
+using wide_gemm::Tile;
+
+namespace {
+
+constexpr int UNITS = 256, DIES = 8, NO_ACT = -1;
+
+struct Product {
+  void* out;  // bfloat16 [M][ldc], or float32 [split][M][ldc]
+  int64_t ldc;
+  const char* a;  // rows of lda bytes
+  const char* w;  // rows of ldw bytes
+  int64_t lda, ldw;
+  const void* bias;
+  int b_is_f32;
+  int M, N, stages, splits;
+  int row_tiles, col_tiles, strip;
+  int whole;  // tiles of 256 x 256 that are run as such
+};
+
+// Workgroups i, i + 8, i + 16, ... run on one die: they take an eighth of `count` in a row, so that tiles that share
+// rows of A or W find them in their die's L2.
+__device__ __forceinline__ int in_row(int i, int count) {
+  const int q = count / DIES, r = count % DIES, die = i % DIES;
+  return die * q + min(die, r) + i / DIES;
+}
+
+// Tile `id` of row_tiles x col_tiles: strips of `strip` row tiles, column by column.
+__device__ __forceinline__ void place_of(int id, int row_tiles, int col_tiles, int strip, int& tm, int& tn) {
+  const int s = id / (strip * col_tiles), in = id - s * strip * col_tiles, rows = min(strip, row_tiles - s * strip);
+  tm = s * strip + in % rows;
+  tn = in / rows;
+}
+
+// What an activation reads: the sum as a product kept in bfloat16 holds it.  So a product with its activation is the same bits as the
+// product and the activation's kernel behind it, which make it where there is no plan, and a near tie among a later
+// layer's experts falls the same way whichever of the two ran.
+__device__ __forceinline__ float rounded(float sum) { return (float)(__bf16)sum; }
+
+// acc[i][x][e] of a wavefront: row row0 + 16 i + lane % 16 by W row n0 + dealt_row(x, 4 (lane / 16) + e).
+// ACT: the activation's code (common.h), NO_ACT none; a template's argument, as code for all of them at every element is more than
+// the instruction cache holds (2,048 rows by 17,920 features: 150 us instead of 115).
+template <int MODE, int ACT, int MT, int X>
+__device__ __forceinline__ void finish(const Product& p, const f32x4 (&acc)[MT][X], int row0, int n0, int split) {
+  const int lane = threadIdx.x % PAE_WAVE, col = lane % 16, kg = lane / 16;
+  if constexpr (MODE == wide_gemm::GATED) {
+    static_assert(X == 2 || X == 4, "4 or 8 neighbouring features a lane");
+    const int f = n0 / 2 + kg * (2 * X);
+    if (f >= p.N / 2) return;  // N / 2 is a multiple of 8
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const int row = row0 + 16 * i + col;
+      if (row >= p.M) continue;
+      bf16_t* o = (bf16_t*)p.out + row * p.ldc + f;
+      __bf16 v[2 * X];
+#pragma unroll
+      for (int x = 0; x < X; x += 2)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[2 * x + e] = (__bf16)(act_of(rounded(acc[i][x][e]), ACT) * rounded(acc[i][x + 1][e]));
+      if constexpr (X == 4) *reinterpret_cast<bf16x8*>(o) = *reinterpret_cast<const bf16x8*>(v);
+      else *reinterpret_cast<bf16x4*>(o) = *reinterpret_cast<const bf16x4*>(v);
+    }
+  } else if constexpr (MODE == wide_gemm::SUMS) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const int row = row0 + 16 * i + col;
+      if (row >= p.M) continue;
+      float* o = (float*)p.out + ((int64_t)split * p.M + row) * p.ldc;
+#pragma unroll
+      for (int x = 0; x < X; ++x) {
+        const int n = n0 + 16 * x + 4 * kg;
+        if (n < p.N) *reinterpret_cast<f32x4*>(o + n) = acc[i][x];
+      }
+    }
+  } else {
+    f32x4 bias[X];
+    if (p.bias) {
+#pragma unroll
+      for (int x = 0; x < X; ++x)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          bias[x][e] = load_param(p.bias, p.b_is_f32, min(n0 + wide_gemm::dealt_row<MODE, X>(x, 4 * kg + e), p.N - 1));
+    }
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const int row = row0 + 16 * i + col;
+      if (row >= p.M) continue;
+      bf16_t* o = (bf16_t*)p.out + row * p.ldc;
+      f32x4 z[X];
+#pragma unroll
+      for (int x = 0; x < X; ++x)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) z[x][e] = ACT == NO_ACT ? acc[i][x][e] : rounded(acc[i][x][e]);
+      if (p.bias) {
+#pragma unroll
+        for (int x = 0; x < X; ++x) z[x] += bias[x];
+      }
+      __bf16 v[4 * X];
+#pragma unroll
+      for (int x = 0; x < X; ++x)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[4 * x + e] = (__bf16)(ACT == NO_ACT ? z[x][e] : act_of(z[x][e], ACT));
+#pragma unroll
+      for (int x = 0; x < X; x += 2) {
+        const int n = n0 + 16 * x + (x + 1 < X ? 8 : 4) * kg;
+        if (n >= p.N) continue;  // N is a multiple of 8
+        if (x + 1 < X) *reinterpret_cast<bf16x8*>(o + n) = *reinterpret_cast<const bf16x8*>(v + 4 * x);
+        else *reinterpret_cast<bf16x4*>(o + n) = *reinterpret_cast<const bf16x4*>(v + 4 * x);
+      }
+    }
+  }
+}
+
+// The tile of T at rows m0.. and W rows n0..; stages [first, first + stages) of k.
+template <int MODE, int ACT, typename T>
+__device__ __forceinline__ void small_tile(const Product& p, char* lds, int m0, int n0, int first, int stages, int split) {
+  const int lane = threadIdx.x % PAE_WAVE;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PAE_WAVE);
+  typename T::Source src;
+  src.a = p.a + m0 * p.lda + (int64_t)first * wide_gemm::ROW_BYTES;
+  src.w = p.w + n0 * p.ldw + (int64_t)first * wide_gemm::ROW_BYTES;
+#pragma unroll
+  for (int j = 0; j < T::A_LOADS; ++j) {
+    const int q = (wave * T::A_LOADS + j) * 8 + lane / 8;
+    src.a_off[j] = (uint32_t)min(q, p.M - 1 - m0) * (uint32_t)p.lda + wide_gemm::piece_of(lane, q);
+  }
+#pragma unroll
+  for (int j = 0; j < T::W_LOADS; ++j) {
+    const int q = (wave * T::W_LOADS + j) * 8 + lane / 8;
+    const int n = q / T::PN * T::PN + wide_gemm::dealt_row<MODE, T::X>(q % T::PN / 16, q % 16);
+    src.w_off[j] = (uint32_t)min(n, p.N - 1 - n0) * (uint32_t)p.ldw + wide_gemm::piece_of(lane, q);
+  }
+  f32x4 acc[T::MT][T::X];
+#pragma unroll
+  for (int i = 0; i < T::MT; ++i)
+#pragma unroll
+    for (int x = 0; x < T::X; ++x) acc[i][x] = f32x4{0.f, 0.f, 0.f, 0.f};
+  T::run(acc, lds, src, stages);
+  finish<MODE, ACT>(p, acc, m0 + wave / T::WN * T::PM, n0 + wave % T::WN * T::PN, split);
+}
+
+using Half = Tile<128, 256, 2, 4, 3>;     // of a tile of 256 x 256, by the same eight wavefronts
+using Quarter = Tile<128, 128, 2, 4, 4>;
+
+// parts: into how many each tile behind the whole ones is cut (1, 2 or 4)
+template <int MODE, int ACT, int PARTS>
+__global__ __launch_bounds__(512, 2) void wide_large_kernel(Product p) {
+  extern __shared__ __attribute__((aligned(16))) char wide_lds[];
+  const int lane = threadIdx.x % PAE_WAVE;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PAE_WAVE);
+  int tm, tn;
+  if (PARTS > 1 && (int)blockIdx.x >= p.whole) {
+    const int rest = (p.row_tiles * p.col_tiles - p.whole) * PARTS, at = in_row(blockIdx.x - p.whole, rest);
+    place_of(p.whole + at / PARTS, p.row_tiles, p.col_tiles, p.strip, tm, tn);
+    const int m0 = tm * 256 + at % PARTS / (PARTS / 2) * 128, n0 = tn * 256 + (PARTS == 4 ? at % 2 * 128 : 0);
+    if (m0 >= p.M || n0 >= p.N) return;
+    small_tile<MODE, ACT, typename std::conditional<PARTS == 4, Quarter, Half>::type>(p, wide_lds, m0, n0, 0, p.stages, 0);
+    return;
+  }
+  place_of(in_row(blockIdx.x, p.whole), p.row_tiles, p.col_tiles, p.strip, tm, tn);
+  const int m0 = tm * 256, n0 = tn * 256;
+  Large::Source src;
+  src.a = p.a + m0 * p.lda;
+  src.w = p.w + n0 * p.ldw;
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int q = (wave * 2 + j) * 8 + lane / 8;
+      src.a_off[h][j] = (uint32_t)min(Large::a_row(h, q), p.M - 1 - m0) * (uint32_t)p.lda + wide_gemm::piece_of(lane, q);
+      src.w_off[h][j] = (uint32_t)min(Large::w_row<MODE>(h, q), p.N - 1 - n0) * (uint32_t)p.ldw + wide_gemm::piece_of(lane, q);
+    }
+  f32x4 acc[Large::MT][Large::X];
+#pragma unroll
+  for (int i = 0; i < Large::MT; ++i)
+#pragma unroll
+    for (int x = 0; x < Large::X; ++x) acc[i][x] = f32x4{0.f, 0.f, 0.f, 0.f};
+  Large::run(acc, wide_lds, src, p.stages);
+  finish<MODE, ACT>(p, acc, m0 + wave / Large::WN * Large::PM, n0 + wave % Large::WN * Large::PN, 0);
+}
+
+// One shape of smaller tiles throughout; the ranges of k lie one after another.  (Never all 512 registers for a wavefront: the
+// compiler would put part of the sums into the accumulation file and move them to and fro.)
+template <int MODE, int ACT, typename T>
+__global__ __launch_bounds__(T::WAVES * 64, 2) void wide_small_kernel(Product p) {
+  extern __shared__ __attribute__((aligned(16))) char wide_lds[];
+  const int tiles = p.row_tiles * p.col_tiles;
+  int id = in_row(blockIdx.x, tiles * p.splits), tm, tn;
+  const int split = id / tiles;
+  id -= split * tiles;
+  place_of(id, p.row_tiles, p.col_tiles, p.strip, tm, tn);
+  const int first = (int)((int64_t)p.stages * split / p.splits), last = (int)((int64_t)p.stages * (split + 1) / p.splits);
+  small_tile<MODE, ACT, T>(p, wide_lds, tm * T::BM, tn * T::BN, first, last - first, split);
+}
+
+template <typename K>
+int launch(K kernel, const Product& p, int64_t blocks, int threads, int lds, hipStream_t stream) {
+  const hipError_t err = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  PAE_REQUIRE(err == hipSuccess, "wide product: %d bytes of LDS refused: %s", lds, hipGetErrorString(err));
+  kernel<<<(unsigned)blocks, threads, lds, stream>>>(p);
+  return pae_check_launch("gemm_wide");
+}
+
+int64_t tiles_of(int M, int N, int bm, int bn) { return (int64_t)((M + bm - 1) / bm) * ((N + bn - 1) / bn); }
+
+template <int MODE, int ACT, typename T>
+int launch_small(Product p, hipStream_t stream) {
+  p.row_tiles = (p.M + T::BM - 1) / T::BM;
+  p.col_tiles = (p.N + T::BN - 1) / T::BN;
+  p.strip = 8;
+  PAE_REQUIRE((int64_t)p.row_tiles * p.col_tiles * p.splits < (1ll << 30), "wide product: too many tiles");
+  return launch(wide_small_kernel<MODE, ACT, T>, p, (int64_t)p.row_tiles * p.col_tiles * p.splits, T::WAVES * 64, T::LDS_BYTES, stream);
+}
+
+template <int MODE, int ACT>
+int launch_large(Product p, hipStream_t stream) {
+  p.row_tiles = (p.M + 255) / 256;
+  p.col_tiles = (p.N + 255) / 256;
+  p.strip = 8;
+  const int64_t tiles = (int64_t)p.row_tiles * p.col_tiles;
+  PAE_REQUIRE(tiles < (1ll << 28), "wide product: too many tiles");
+  const int rest = (int)(tiles % UNITS), parts = rest == 0 || rest > UNITS / 2 ? 1 : rest > UNITS / 4 ? 2 : 4;
+  p.whole = (int)(parts == 1 ? tiles : tiles - rest);
+  constexpr int LDS = Large::LDS_BYTES > Half::LDS_BYTES ? Large::LDS_BYTES : Half::LDS_BYTES;
+  static_assert(Quarter::LDS_BYTES <= LDS, "room for every part");
+  if (parts == 1) return launch(wide_large_kernel<MODE, ACT, 1>, p, tiles, 512, Large::LDS_BYTES, stream);
+  if (parts == 2) return launch(wide_large_kernel<MODE, ACT, 2>, p, p.whole + 2 * rest, 512, LDS, stream);
+  return launch(wide_large_kernel<MODE, ACT, 4>, p, p.whole + 4 * rest, 512, LDS, stream);
+}
+
+enum { SHAPE_LARGE, SHAPE_128_256, SHAPE_128_128, SHAPE_128_96, SHAPE_64_128, SHAPE_64_64, SHAPES };
+
+// Microseconds of a product in a shape, from times of all shapes at 14 sizes of weights (896 to 18,944 of k) by 24 row counts
+// from 72 to 8,192, which this meets within 11 to 13 % (root mean square): a round of tiles costs its start and end and so much a
+// stage.  The least of them is on average 1 % behind the fastest shape.
+double shape_time(int shape, int M, int N, int K, int splits) {
+  const double stages = K / 64.0 / splits;
+  struct Cost { int bm, bn, blocks; double launch, round, stage, part; };  // part: a stage of a last round that half the units' places or fewer take
+  static const Cost cost[SHAPES] = {{256, 256, 1, 0.0, 3.5, 1.35, 0.0},  {128, 256, 1, 0.0, 2.9, 0.73, 0.73}, {128, 128, 1, 0.0, 2.4, 0.46, 0.46},
+                                    {128, 96, 1, 0.3, 2.4, 0.39, 0.39}, {64, 128, 2, 2.5, 0.0, 0.62, 0.33},  {64, 64, 2, 2.9, 0.0, 0.38, 0.21}};
+  const Cost& c = cost[shape];
+  const int64_t tiles = tiles_of(M, N, c.bm, c.bn) * splits, places = (int64_t)UNITS * c.blocks;
+  const int64_t rest = tiles % places;
+  double last = 0.0;
+  if (rest) last = c.round + stages * (shape == SHAPE_LARGE ? (rest > UNITS / 2 ? c.stage : rest > UNITS / 4 ? 0.77 : 0.40) : rest > places / 2 ? c.stage : c.part);
+  return c.launch + tiles / places * (c.round + stages * c.stage) + last;
+}
+
+template <int MODE, int ACT>
+int run_shape(int shape, const Product& p, hipStream_t stream) {
+  constexpr bool PAIRS = MODE == wide_gemm::GATED;
+  switch (shape) {
+    case SHAPE_LARGE:
+      if constexpr (MODE != wide_gemm::SUMS) return launch_large<MODE, ACT>(p, stream);
+      break;
+    case SHAPE_128_256: return launch_small<MODE, ACT, Tile<128, 256, 2, 4, 3>>(p, stream);
+    case SHAPE_128_128: return launch_small<MODE, ACT, Tile<128, 128, 2, 2, 4>>(p, stream);
+    case SHAPE_128_96:
+      if constexpr (!PAIRS) return launch_small<MODE, ACT, Tile<128, 96, 2, 2, 4>>(p, stream);
+      break;
+    case SHAPE_64_128: return launch_small<MODE, ACT, Tile<64, 128, 2, 2, 3>>(p, stream);
+    case SHAPE_64_64: return launch_small<MODE, ACT, Tile<64, 64, 2, 2, 4>>(p, stream);
+  }
+  return pae_fail("wide product: shape %d does not take mode %d", shape, MODE);
+}
+
+}  // namespace
+
+// The shape for a product, in the low byte, and its ranges of k behind that.  `mode` as for pae_gemm_wide; `ranges` != 0: the
+// product may leave float32 sums of ranges of k for a caller that reads them again (counted at 4.5 TB/s against one bfloat16
+// result).  -1: the platform library, for a product without an activation that no shape here fills the chip with: from
+// 30 us on and below 0.95 PFLOP/s by the times above the library, which shares such products out over k, was ahead of
+// these shapes two times in three (6,030 x 1,536 x 8,960 141 against 160 us, 2,048 x 4,608 x 3,584 59 against 68).
+extern "C" int pae_gemm_wide_plan(int mode, int act, int M, int N, int K, int ranges) {
+  static const int CUTS[] = {2, 3, 4, 6, 8};
+  int best = SHAPE_LARGE, cuts = 1;
+  double least = 1e30;
+  for (int shape = 0; shape < SHAPES; ++shape) {
+    if ((shape == SHAPE_128_96 && mode == wide_gemm::GATED) || (shape == SHAPE_LARGE && K < 128)) continue;
+    const double t = shape_time(shape, M, N, K, 1);
+    if (t < least) least = t, best = shape;
+  }
+  for (int shape = SHAPE_LARGE + 1; ranges && shape < SHAPES; ++shape)
+    for (int n : CUTS) {
+      if (K < 1024 * n) break;  // (k of 1,536 in two ranges: 8.2 -> 7.8 us at best, and slower from 900 rows on)
+      const double t = shape_time(shape, M, N, K, n) + (4.0 * n - 2.0) * M * N / 4.5e6;
+      if (t < least) least = t, best = shape, cuts = n;
+    }
+  if (mode == wide_gemm::PLAIN && act == NO_ACT && least > 30.0 && 2.0 * M * N * K / least < 0.95e9) return -1;
+  return best | cuts << 8;
+}
+
+// C = A W^T for A [M, K] (rows of lda numbers), W [N, K]; K a multiple of 64, N of 16.  mode 0: bfloat16 [M, N] of act(A W^T + bias), act
+// -1 (none), 0 or 3; 1: bfloat16 [M, N / 2] of act(gate) * other, W's rows in blocks of 8 of the one and of the
+// other, act 1 or 2; 2: float32 [ranges, M, N] of the sums over ranges of k.  Operands begin at multiples of 16 bytes.
+extern "C" int pae_gemm_wide(int mode, int act, int plan, void* out, int64_t ldc, const void* a, int64_t lda, const void* w, const void* bias,
+                             int b_is_f32, int M, int N, int K, hipStream_t stream) {
+  const int shape = plan & 255, ranges = plan >> 8;
+  PAE_REQUIRE(M > 0 && N > 0 && N % 16 == 0 && K > 0 && K % 64 == 0, "wide product: bad sizes M=%d N=%d K=%d", M, N, K);
+  PAE_REQUIRE(plan >= 0 && shape < SHAPES && ranges >= 1 && ranges <= K / 64 && (mode == wide_gemm::SUMS || ranges == 1) && (shape != SHAPE_LARGE || K >= 128),
+              "wide product: plan %d for mode %d and K=%d", plan, mode, K);
+  PAE_REQUIRE(lda >= 0 && lda % 8 == 0 && lda < (1 << 22) && K < (1 << 22), "wide product: rows of %lld numbers", (long long)lda);  // 256 rows in 32 bits
+  PAE_REQUIRE(ldc % (mode == wide_gemm::SUMS ? 4 : 8) == 0 && ((uintptr_t)out | (uintptr_t)a | (uintptr_t)w) % 16 == 0, "wide product: operands must lie at multiples of 16 bytes");
+  Product p;
+  p.out = out;
+  p.ldc = ldc;
+  p.a = (const char*)a;
+  p.lda = lda * 2;
+  p.w = (const char*)w;
+  p.ldw = (int64_t)K * 2;
+  p.bias = bias;
+  p.b_is_f32 = b_is_f32;
+  p.M = M;
+  p.N = N;
+  p.stages = K / 64;
+  p.splits = ranges;
+  p.row_tiles = p.col_tiles = p.strip = p.whole = 0;
+  if (mode == wide_gemm::SUMS) return run_shape<wide_gemm::SUMS, NO_ACT>(shape, p, stream);
+  if (mode == wide_gemm::PLAIN && act == NO_ACT) return run_shape<wide_gemm::PLAIN, NO_ACT>(shape, p, stream);
+  if (mode == wide_gemm::PLAIN && act == 0) return run_shape<wide_gemm::PLAIN, 0>(shape, p, stream);
+  if (mode == wide_gemm::PLAIN && act == 3) return run_shape<wide_gemm::PLAIN, 3>(shape, p, stream);
+  if (mode == wide_gemm::GATED && act == 1) return run_shape<wide_gemm::GATED, 1>(shape, p, stream);
+  if (mode == wide_gemm::GATED && act == 2) return run_shape<wide_gemm::GATED, 2>(shape, p, stream);
+  return pae_fail("wide product: mode %d with activation %d", mode, act);
+}

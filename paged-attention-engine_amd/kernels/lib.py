@@ -64,6 +64,8 @@ def _declare(lib) -> None:
         "pae_swiglu": [I, P, P, I, I, I, P],
         "pae_gemm_skinny": [I, P, L, P, L, P, P, I, I, I, I, I, L, P, P, P, I, F, P, L, P, I, P, P],
         "pae_gemm_skinny_rope": [P, L, P, L, P, P, I, I, I, I, I, I, I, P, P, P, P, I, I, P, P, I, P, P, P, I, F, P],
+        "pae_gemm_wide_plan": [I, I, I, I, I, I],
+        "pae_gemm_wide": [I, I, I, P, L, P, L, P, P, I, I, I, I, P],
         "pae_embedding_rows": [I, P, P, P, I, I, I, F, P, P, I, P, P],
         "pae_scaled_rows": [P, P, P, I, F, I, I, P],
         "pae_skinny_ticket_slots": [I, I],
@@ -820,6 +822,58 @@ def gemm_skinny_gated(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, kind:
 CHECK_TICKET_SUMS = os.environ.get("PAE_CHECK_TICKETS", "") == "sums"
 
 
+# Products of more rows than the few-row kernels take (csrc/gemm_wide.hip).  `plan`: how one is made, as `wide_plan` gives it.
+WIDE_PLAIN, WIDE_GATED, WIDE_SUMS = 0, 1, 2
+WIDE_ACTIVATIONS = {WIDE_PLAIN: ("gelu", "relu2"), WIDE_GATED: ("gelu_tanh", "silu")}  # those that the product's epilogue knows
+_WIDE_STRIDE = 1 << 22
+
+
+def wide_plan(a: torch.Tensor, w: torch.Tensor, mode: int = WIDE_PLAIN, kind: Optional[str] = None, ranges: bool = False) -> Optional[int]:
+    """How `gemm_wide` makes this product, or None: sizes or operands it does not take, or that the platform's library is
+    ahead at.  `ranges`: the product may leave float32 sums of ranges of k (plan >> 8 says how many)."""
+    if (a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or a.shape[0] <= SKINNY_MAX_ROWS or w.shape[0] % 16 or w.shape[1] % 64
+            or w.shape[0] == 0 or w.shape[1] == 0 or a.stride(1) != 1 or a.stride(0) % 8 or not w.is_contiguous()
+            or a.data_ptr() % 16 or w.data_ptr() % 16 or a.stride(0) >= _WIDE_STRIDE or w.shape[1] >= _WIDE_STRIDE):
+        return None
+    if kind is not None and kind not in WIDE_ACTIVATIONS[mode]:
+        return None
+    plan = library().pae_gemm_wide_plan(mode, -1 if kind is None else ACTIVATIONS[kind], a.shape[0], w.shape[0], w.shape[1], 1 if ranges else 0)
+    return None if plan < 0 else plan
+
+
+def gemm_wide(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, plan: int, bias: Optional[torch.Tensor] = None,
+              kind: Optional[str] = None, mode: int = WIDE_PLAIN) -> None:
+    """By mode: out [M, N] = act(A W^T + bias), act by name or none; out [M, N / 2] = act(gate) * up for W's rows in blocks of 8 of
+    the gate and 8 of the other factor; float32 out [ranges, M, N] = the sums over `plan`'s ranges of k.  A sum is
+    float32; an activation reads it rounded to bfloat16, as `activation`, `swiglu` and `gated_act` behind a product do, and is
+    worked out in float32."""
+    _not_while_recording("gemm_wide")
+    _gpu(out, a, w, bias)
+    M, K = a.shape
+    N = w.shape[0]
+    assert w.shape == (N, K) and w.is_contiguous() and a.stride(1) == 1 and out.is_contiguous()
+    if mode == WIDE_SUMS:
+        assert out.shape == (plan >> 8, M, N) and out.dtype == torch.float32 and bias is None and kind is None
+    else:
+        assert out.shape == (M, N // 2 if mode == WIDE_GATED else N) and out.dtype == a.dtype
+        assert mode == WIDE_PLAIN or (bias is None and kind is not None)
+    assert bias is None or bias.shape == (N,)
+    bp, bf = _param(bias)
+    _check(library().pae_gemm_wide(mode, -1 if kind is None else ACTIVATIONS[kind], plan, out.data_ptr(), out.shape[-1], a.data_ptr(),
+                                   a.stride(0), w.data_ptr(), bp, bf, M, N, K, _stream()))
+
+
+def product_of_rows(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """x W^T in x's dtype for many rows: by `gemm_wide` or, where that does not take it or is behind, by the platform's library."""
+    out = torch.empty((x.shape[0], w.shape[0]), dtype=x.dtype, device=x.device)
+    plan = wide_plan(x, w)
+    if plan is None:
+        torch.mm(x, w.t(), out=out)
+    else:
+        gemm_wide(out, x, w, plan)
+    return out
+
+
 def _check_ticket_sums(out, before, a, w, bias, epilogue, splits, row_scale, following) -> None:
     again = before if before is not None else torch.empty_like(out)
     follow = None
@@ -1326,7 +1380,7 @@ def latent_expanded(out: torch.Tensor, proj: torch.Tensor, latent: torch.Tensor,
     rows = new(n * 16, rank)
     _check(lib.pae_latent_gather(rows.data_ptr(), latent.data_ptr(), pages.data_ptr(), n, block_tables.data_ptr(),
                                  block_tables.shape[1], bs, rank, rank + rd, _stream()))
-    up = torch.mm(rows, up_weight.t())
+    up = product_of_rows(rows, up_weight)
     keys, values = new(n, nh, 16, width), new(n, nh, value_dim, 16)
     _check(lib.pae_latent_expand(keys.data_ptr(), values.data_ptr(), up.data_ptr(), up.stride(0), latent.data_ptr(),
                                  pages.data_ptr(), n, block_tables.data_ptr(), block_tables.shape[1], bs, nh, nope, rd,

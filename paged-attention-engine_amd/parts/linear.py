@@ -7,9 +7,9 @@ The reference calls F.linear on weights stored (out_features, in_features)
              and sums in full 32-bit, in an order that depends on k alone, each row
              independent of the batch;
   bfloat16   up to 64 rows (decode steps, small portions): the weight-streaming
-             matrix-core kernel, which reads W once; more rows: the platform's
-             matrix library, as the reference's products go to its library.
-             Both accumulate in float32.
+             matrix-core kernel, which reads W once; more rows: this engine's tiled
+             kernels, or the platform's matrix library where it is ahead or the sizes are none
+             of theirs.  All accumulate in float32.
 """
 
 from __future__ import annotations
@@ -42,13 +42,17 @@ class Linear:
     def graph_max_rows(self):
         return rows_a_graph_may_hold(self.weight.dtype, self.in_features)
 
-    def _library(self, x: torch.Tensor, with_bias: bool = True) -> torch.Tensor:
-        out = torch.empty((x.shape[0], self.out_features), dtype=x.dtype, device=x.device)
+    def _many_rows(self, x: torch.Tensor, with_bias: bool = True) -> torch.Tensor:
+        """The product of more rows than the few-row kernel takes."""
         bias = self.bias if with_bias else None
         if bias is None:
-            torch.mm(x, self.weight.t(), out=out)
-        else:
+            return K.product_of_rows(x, self.weight)
+        out = torch.empty((x.shape[0], self.out_features), dtype=x.dtype, device=x.device)
+        plan = K.wide_plan(x, self.weight)
+        if plan is None:
             torch.addmm(bias if bias.dtype == x.dtype else bias.to(x.dtype), x, self.weight.t(), out=out)
+        else:
+            K.gemm_wide(out, x, self.weight, plan, bias)
         return out
 
     def __call__(self, x) -> torch.Tensor:
@@ -69,16 +73,16 @@ class Linear:
             out = torch.empty((M, self.out_features), dtype=x.dtype, device=x.device)
             K.gemm_skinny(out, x, self.weight, self.bias, K.EPI_BF16)
             return out
-        return self._library(x)
+        return self._many_rows(x)
 
     def without_bias(self, x) -> Optional[torch.Tensor]:
-        """The product without its bias where that is the cheaper call (the matrix library's plain
-        product, many rows), for a caller that adds the bias in a kernel of its own that follows
-        anyway; None where the bias costs nothing (this engine's own products)."""
+        """The product of many rows without its bias, for a caller that adds the bias in float32 in a
+        kernel of its own that follows anyway (the matrix library's plain product is the cheaper call); None
+        for few rows, whose product adds it to its float32 sums."""
         if (self.bias is None or isinstance(x, OwedRows) or x.dtype != torch.bfloat16 or x.shape[0] == 0
                 or K.skinny_supported(x, self.weight)):
             return None
-        return self._library(x, with_bias=False)
+        return self._many_rows(x, with_bias=False)
 
     def branch(self, x: torch.Tensor, sink=None, bias_terms: bool = False):
         """The product as a residual branch's output: [M, N] in x's dtype (few rows with a bias: k ranges
@@ -112,6 +116,11 @@ class Linear:
             out = torch.empty((x.shape[0], self.out_features), dtype=x.dtype, device=x.device)
             K.gemm_skinny(out, x, self.weight, self.bias, K.EPI_BF16,
                           K.whole_sum_splits(self.out_features, self.in_features, x.shape[0]))
+            return out
+        plan = K.wide_plan(x, self.weight, K.WIDE_SUMS, ranges=True) if sink is not None and self.bias is None else None
+        if plan is not None and plan >> 8 > 1:
+            out = torch.empty((plan >> 8, x.shape[0], self.out_features), dtype=torch.float32, device=x.device)
+            K.gemm_wide(out, x, self.weight, plan, mode=K.WIDE_SUMS)
             return out
         return self(x)
 

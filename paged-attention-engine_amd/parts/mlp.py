@@ -62,6 +62,8 @@ class SwiGLU(Part):
         """`x`: normalised activations, or `OwedRows` (the gated product then pays their scale)."""
         act = torch.empty((x.shape[0], self.spec.intermediate_size), dtype=x.dtype, device=x.device)
         rows = x.rows if isinstance(x, OwedRows) else x
+        plan = (K.wide_plan(x, self.gate_up.weight, K.WIDE_GATED, self.spec.activation)
+                if self.block and not isinstance(x, OwedRows) else None)
         if self.silu and self.block and x.shape[0] and K.skinny_supported(rows, self.gate_up.weight):
             splits = K.whole_sum_splits(2 * self.spec.intermediate_size, self.spec.hidden_size, x.shape[0])
             K.gemm_skinny(act, rows, self.gate_up.weight, None, K.EPI_SWIGLU, splits,
@@ -70,6 +72,8 @@ class SwiGLU(Part):
             # another activation: the same product and layout, the activation by name in its epilogue
             splits = K.whole_sum_splits(2 * self.spec.intermediate_size, self.spec.hidden_size, x.shape[0])
             K.gemm_skinny_gated(act, rows, self.gate_up.weight, self.spec.activation, splits)
+        elif plan is not None:
+            K.gemm_wide(act, x, self.gate_up.weight, plan, kind=self.spec.activation, mode=K.WIDE_GATED)
         elif self.silu:
             K.swiglu(act, self.gate_up(plain_rows(x)), self.block)
         else:
@@ -109,13 +113,18 @@ class DenseFeedForward(Part):
         self.down = Linear(self.matrix(weights[prefix + s.down_name + s.weight_suffix]), bias(s.down_name))
 
     def forward(self, ctx, x):
-        """Up to 64 rows the activation runs in the up product's epilogue, on its float32 sums; above,
-        the platform library's product is followed by the activation kernel, which adds the bias first."""
+        """The activation runs in the up product's epilogue (up to 64 rows on its float32 sums) where the product's kernel knows
+        it; elsewhere a product of many rows is followed by the activation kernel, which adds the bias first: the
+        same bits as the epilogue of many rows."""
         x = plain_rows(x)
+        plan = K.wide_plan(x, self.up.weight, K.WIDE_PLAIN, self.spec.activation)
         if x.shape[0] and K.skinny_supported(x, self.up.weight):
             act = torch.empty((x.shape[0], self.spec.intermediate_size), dtype=x.dtype, device=x.device)
             splits = K.whole_sum_splits(self.spec.intermediate_size, self.spec.hidden_size, x.shape[0])
             K.gemm_skinny_act(act, x, self.up.weight, self.spec.activation, splits, self.up.bias)
+        elif plan is not None:
+            act = torch.empty((x.shape[0], self.spec.intermediate_size), dtype=x.dtype, device=x.device)
+            K.gemm_wide(act, x, self.up.weight, plan, self.up.bias, self.spec.activation)
         else:
             act = self.up.without_bias(x)
             bias = self.up.bias if act is not None else None

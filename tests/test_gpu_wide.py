@@ -1,0 +1,164 @@
+"""Products of many rows (csrc/gemm_wide.hip) against the same in 64 bits, over every tile shape: edges and remainders of
+tiles in rows and features, the fewest stages of k, what is left over behind whole rounds of tiles in halves and quarters, operands that are
+rows of wider ones.  A sum's order depends on k alone, so every shape gives the same bits."""
+
+import pytest
+import torch
+
+from paged_attention_engine_amd.kernels import lib as K
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = range(6)
+GATED_SHAPES = (0, 1, 2, 4, 5)
+SUMS_SHAPES = (1, 2, 3, 4, 5)
+GUARD = 64  # rows behind the result, which must stay as they are
+
+# rows, features, k
+SIZES = [(65, 16, 128), (64 + 1, 48, 192), (127, 144, 128), (128, 256, 256), (129, 272, 320), (255, 1168, 128), (257, 528, 448),
+         (300, 96, 1536), (513, 1552, 896),
+         (513, 21856, 128),   # 3 x 86 tiles of 256 x 256: two left over behind a round, in quarters, and the last of them 96 wide
+         (1100, 17920, 128),  # 5 x 70: 94 left over, in halves, rows that end inside a half
+         (2048, 17920, 192)]  # 8 x 70: 48 left over, in quarters
+
+
+def operands(M, N, k, seed=0, wider=0):
+    gen = torch.Generator(device="cuda").manual_seed(seed + M + N + k)
+    a = torch.randn(M, k + wider, generator=gen, device="cuda").to(torch.bfloat16)[:, :k]
+    w = (torch.randn(N, k, generator=gen, device="cuda") * k ** -0.5).to(torch.bfloat16)
+    return a, w
+
+
+def guarded(M, N, dtype, lead=None):
+    whole = torch.full(((lead or 1) * M + GUARD, N), 7.0, device="cuda", dtype=dtype)
+    out = whole[:(lead or 1) * M]
+    return (out.view(lead, M, N) if lead else out), whole[(lead or 1) * M:]
+
+
+def exact(a, w):
+    """The product in 64 bits and a bound of the float32 sums' error: k additions, each within half a place (2^-24) of
+    a partial sum, which is at most the sum of magnitudes."""
+    ref = a.double() @ w.double().T
+    return ref, w.shape[1] * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T)
+
+
+def check(got, ref, err):
+    """`err`: of what is rounded to bfloat16 at the end (half a place of its 8 bits: 2^-8)."""
+    rounding = 2.0 ** -8 * (ref.abs() + err) if got.dtype == torch.bfloat16 else 0.0
+    off = (got.double() - ref).abs() - (err + rounding) * 1.001
+    assert float(off.max()) <= 0.0, float(off.max())
+
+
+@pytest.mark.parametrize("M,N,k", SIZES)
+def test_product(M, N, k):
+    a, w = operands(M, N, k)
+    ref, err = exact(a, w)
+    first = None
+    for shape in SHAPES:
+        out, behind = guarded(M, N, torch.bfloat16)
+        K.gemm_wide(out, a, w, shape | 1 << 8)
+        check(out, ref, err)
+        assert bool((behind == 7.0).all())
+        first = out if first is None else first
+        assert torch.equal(out, first), shape
+
+
+@pytest.mark.parametrize("M,N,k", [(65, 16, 128), (129, 272, 320), (513, 1552, 896), (513, 21856, 128)])
+@pytest.mark.parametrize("kind", [None, "gelu", "relu2"])
+def test_bias_and_activation(M, N, k, kind):
+    a, w = operands(M, N, k, 1, wider=24)
+    bias = torch.randn(N, device="cuda")
+    for b in (bias, bias.to(torch.bfloat16)):
+        ref, err = exact(a, w)
+        if kind is not None:  # the activation reads the sum rounded to bfloat16
+            err = err + 2.0 ** -8 * (ref.abs() + err)
+        ref = ref + b.double()
+        err = err + 2.0 ** -24 * (ref.abs() + err)
+        if kind == "gelu":  # its slope is at most 1.13; erff and what is around it: a few places
+            ref, err = torch.nn.functional.gelu(ref), 1.13 * err + 8 * 2.0 ** -24 * (ref.abs() + 1.0)
+        elif kind == "relu2":
+            ref, err = torch.relu(ref).pow(2), (2 * ref.abs() + err) * err + 2.0 ** -23 * (ref.abs() + err).pow(2)
+        for shape in SHAPES:
+            out, behind = guarded(M, N, torch.bfloat16)
+            K.gemm_wide(out, a, w, shape | 1 << 8, b, kind)
+            check(out, ref, err)
+            assert bool((behind == 7.0).all())
+
+
+@pytest.mark.parametrize("M,N,k", [(65, 16, 128), (129, 272, 320), (257, 528, 448), (513, 21856, 128), (1100, 17920, 128)])
+@pytest.mark.parametrize("kind", ["silu", "gelu_tanh"])
+def test_gated(M, N, k, kind):
+    a, w = operands(M, N, k, 2, wider=8)
+    ref, err = exact(a, w)
+    err = err + 2.0 ** -8 * (ref.abs() + err)  # both factors are read rounded to bfloat16
+    pair, off = ref.view(M, N // 16, 2, 8), err.view(M, N // 16, 2, 8)
+    g, u, dg, du = (t.reshape(M, N // 2) for t in (pair[:, :, 0], pair[:, :, 1], off[:, :, 0], off[:, :, 1]))
+    act = torch.nn.functional.silu(g) if kind == "silu" else torch.nn.functional.gelu(g, approximate="tanh")
+    # both slopes are at most 1.13; expf, tanhf and what is around them: within 2^-20 of the argument's size
+    da = 1.13 * dg + 2.0 ** -20 * (g.abs() + 1.0) * (1.0 + dg)
+    ref, err = act * u, act.abs() * du + (u.abs() + du) * da + 2.0 ** -24 * (act * u).abs()
+    for shape in GATED_SHAPES:
+        out, behind = guarded(M, N // 2, torch.bfloat16)
+        K.gemm_wide(out, a, w, shape | 1 << 8, kind=kind, mode=K.WIDE_GATED)
+        check(out, ref, err)
+        assert bool((behind == 7.0).all())
+
+
+@pytest.mark.parametrize("M,N,k,ranges", [(65, 16, 64, 1), (129, 272, 320, 2), (257, 528, 448, 7), (513, 1552, 896, 3)])
+def test_sums_of_ranges(M, N, k, ranges):
+    a, w = operands(M, N, k, 3)
+    at = [k // 64 * i // ranges * 64 for i in range(ranges + 1)]
+    for shape in SUMS_SHAPES:
+        out, behind = guarded(M, N, torch.float32, ranges)
+        K.gemm_wide(out, a, w, shape | ranges << 8, mode=K.WIDE_SUMS)
+        for i in range(ranges):
+            check(out[i], *exact(a[:, at[i]:at[i + 1]], w[:, at[i]:at[i + 1]]))
+        assert bool((behind == 7.0).all())
+
+
+@pytest.mark.parametrize("M,N,k", [(129, 272, 320), (1100, 17920, 128)])
+def test_same_bits_as_two_kernels(M, N, k):
+    a, w = operands(M, N, k, 5)
+    product = torch.empty((M, N), device="cuda", dtype=torch.bfloat16)
+    K.gemm_wide(product, a, w, 2 | 1 << 8)
+    bias = torch.randn(N, device="cuda")
+    for kind in K.WIDE_ACTIVATIONS[K.WIDE_PLAIN]:
+        want, got = product.clone(), torch.empty_like(product)
+        K.activation(want, kind, bias)
+        K.gemm_wide(got, a, w, 0 | 1 << 8, bias, kind)
+        assert torch.equal(got, want), kind
+    for kind in K.WIDE_ACTIVATIONS[K.WIDE_GATED]:
+        want, got = (torch.empty((M, N // 2), device="cuda", dtype=torch.bfloat16) for _ in range(2))
+        (K.swiglu if kind == "silu" else lambda o, x, block: K.gated_act(o, x, kind, block))(want, product, 8)
+        K.gemm_wide(got, a, w, 0 | 1 << 8, kind=kind, mode=K.WIDE_GATED)
+        assert torch.equal(got, want), kind
+
+
+def test_which_products_are_taken():
+    a, w = operands(100, 1536, 1536)
+    assert K.wide_plan(a, w) is not None
+    plan = K.wide_plan(a, operands(100, 1536, 8960)[1], K.WIDE_SUMS, ranges=True)
+    assert plan >> 8 > 1  # few tiles and much of k
+    for bad in (a[:64], a.float(), a[:, 1:], a.t()):
+        assert K.wide_plan(bad, w) is None
+    wide = operands(100, 1536, 1544)[0]
+    assert K.wide_plan(wide[:, :1536], w) is not None  # rows of a wider matrix
+    assert K.wide_plan(wide[:, 4:1540], w) is None     # that begin between two multiples of 16 bytes
+    assert K.wide_plan(operands(100, 1536, 96)[0], operands(100, 1536, 96)[1]) is None
+    assert K.wide_plan(a, w[:1530]) is None
+    assert K.wide_plan(a, w, K.WIDE_GATED, "gelu") is None and K.wide_plan(a, w, K.WIDE_GATED, "silu") is not None
+
+
+def test_linear_with_odd_operands():
+    """Products that the tiles do not take go to the library, with the same meaning."""
+    from paged_attention_engine_amd.parts.linear import Linear
+
+    for M, N, k in ((70, 1530, 200), (70, 50, 96), (100, 256, 256)):
+        a, w = operands(M, N, k, 4)
+        bias = torch.randn(N, device="cuda")
+        ref, err = exact(a, w)
+        for b in (None, bias):
+            want = ref if b is None else ref + b.to(torch.bfloat16).double()
+            got = Linear(w, None if b is None else b.to(torch.bfloat16))(a)
+            # (the library may round the product before it adds the bias)
+            check(got, want, err + 2.0 ** -7 * ref.abs())
