@@ -4,62 +4,213 @@
 // W is stored (out_features, in_features) row-major as in the checkpoint, the
 // layout F.linear takes in the reference (engine/model.py:303-305,315,318-320).
 //
-// Products run on the float32 matrix cores (v_mfma_f32_16x16x4_f32: products and sums in full
-// 32-bit).  k is cut into slabs of 16, of which one instruction takes the j-th number of every
-// four (j = 0..3 in turn: a lane reads four neighbouring k at once), and into blocks of 512 whose
-// sums are then added up in order (with rows of 30,000 terms one running sum loses a digit more
-// than the block sums do).  Every kernel here adds in this order, so that the value of an output
-// element does not depend on M, on the tile it falls in, on how the blocks are shared out
-// or on which other rows share the launch.
+// Products run on the bfloat16 matrix cores (v_mfma_f32_16x16x32_bf16).  A float32 number is the sum of three bfloat16 numbers that hold
+// its 24 bits, and of the nine products of two numbers' parts the six that reach a float32 product's last bit are
+// added in float32; the three left out are below 2^-25 of the product.  bfloat16 numbers are one part and take one product.  The
+// float32 instructions (v_mfma_f32_16x16x4_f32), which these replace, add up four products at a time and give 154 TFLOP/s on the
+// whole chip; six of the others do the work at up to 230.  A slab's products are a sum of their own before they join the others'.  Error
+// against 64 bits (root mean square, share of the result's; normal operands): k 1,536 4.1e-7 before, 1.0e-7 now; 8,960 4.1e-7 and
+// 1.6e-7; 18,944 4.2e-7 and 2.1e-7; bfloat16 operands 1.7e-7 and 0.9e-7.
+// (A number below 2^-110 loses what its parts have below 2^-133, the smallest bfloat16.)
 //
-// Why three kernels.  Up to 64 rows the weights' way from memory is the time: `few` gives 16 weight
+// k is cut into slabs of 32, one set of instructions each, and into blocks of 512 whose sums are then added up in
+// order (with rows of 30,000 terms one running sum loses a digit more than the block sums do).  Every kernel here adds in this
+// order, so that the value of an output element does not depend on M, on the tile it falls in, on how
+// the blocks are shared out or on which other rows share the launch.
+//
+// Why three kernels.  Up to 32 rows the weights' way from memory is the time: `few` gives 16 weight
 // rows to a workgroup whose wavefronts take a block of k each, nothing staged (a wavefront reads 16
-// rows x 64 bytes an instruction).  With more rows the matrix cores are: `tiles` stages 32 of k of 64
-// rows of either side through LDS, two buffers that take turns.  Where a launch has too
+// rows x 64 bytes an instruction).  With more rows the matrix cores are: `tiles` takes the numbers apart once and stages the
+// parts of 32 of k through LDS, two buffers that take turns.  Where a launch has too
 // few tiles for the chip the blocks of k are shared out over workgroups as well (`splits`): the
 // block sums go to scratch memory and `sum` adds them in order.
-// Measured, weights from HBM, 2,048 / 1,536 / 17,920 x 1,536 and 1,536 x 8,960 (the kernel before this one, 64 x 64 tiles of
-// multiply-adds on the vector ALU, took 240 ms of a pass of three requests of 601 tokens in all and four steps behind
-// them at the 1.5B sizes; these take 25):
-//   3 rows     6.6, 6.6, 25.1 (4.4 TB/s), 21.9 us
-//   601 rows   50, 37, 311 (106 TFLOP/s), 184 us
-//   2,048      115, 87, 970 (116 TFLOP/s), 478 us (118 of the 154 that the chip gives)
-// Tried: tiles of 128 x 128, 128 x 64 (the accumulators and block totals of a wavefront then leave one or two of
-// them a SIMD: 377 and 326 us for the third product at 601 rows), 16 and 64 of k a stage (329, 322 us).  In `few`
+// Measured, weights from HBM, 2,048 / 1,536 / 17,920 x 1,536 and 1,536 x 8,960, before (float32 instructions, tiles of 64 x 64) and now:
+//   3 rows     8.2, 9.0, 24.0 (4.6 TB/s), 22 us, and the same now
+//   64 rows    18, 18, 76, 64 us                 15, 15, 52, 25
+//   300 rows   27, 27, 173, 95                   25, 23, 142, 81
+//   601 rows   48, 37, 306 (108 TFLOP/s), 185    40, 31, 256 (129 TFLOP/s), 128
+//   2,048      117, 88, 967, 473                 98, 74, 666 (169), 379
+// Tried: W's rows from memory straight to the registers they are multiplied from (a wavefront's load then touches 16 lines, and what
+// a slab needs took 2.4 us to arrive); numbers taken apart with conversions and dot products (see half_parts_of); loads under a condition
+// (see load8_anyhow);
+// all six products straight into the running sums (601 x 17,920 x 1,536 226 us, but an error of 3.4e-7 that leans to one side: a model's
+// logits were 1.8e-6 off instead of 1.5e-6).  In `few`
 // the compiler moves the loads of a batch down to where they are used unless it is told not to (sched_barrier): 18.8
 // against 15.3 us a launch in the step.
 #include "common.h"
 #include "api.h"
 
 #define GP_BLOCK 512  // k of a block whose sum is formed before it joins the total
-#define GP_SLAB 16    // k of four instructions
-#define GP_FEW_ROWS 64
+#define GP_SLAB 32    // k of one instruction
+#define GP_FEW_ROWS 32  // (64 where rows are read number by number)
 #define GP_FEW_WAVES 8
-#define GP_TILE 64    // rows of either side of a tile
+#define GP_TILE 64    // parts of a product are cut in multiples of it
 #define GP_UNITS 256  // compute units
+#define GP_LARGE_WHOLE 160  // large tiles from which on none is shared
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ f32x4 load4(const float* p) { return *(const f32x4*)p; }
-__device__ __forceinline__ f32x4 load4(const bf16_t* p) {
-  const uint2 v = *(const uint2*)p;
-  return f32x4{__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16),
-               __uint_as_float(v.y & 0xffff0000u)};
-}
-// Four numbers of a row from k on, zeros from `end` on; number by number.
+// Eight numbers of a row's slab as they lie in memory: lane group (or thread of four) q holds the fours at 4 q and at 16 + 4 q, so that
+// the four that read a row side by side ask for 64 bytes in a row.  Which of an instruction's k a number stands at is free as
+// long as both sides agree.
 template <typename T>
-__device__ __forceinline__ f32x4 load4_to(const T* row, int k, int end) {
-  f32x4 v;
+struct Eight;
+template <>
+struct Eight<float> {
+  f32x4 v[2];
+};
+template <>
+struct Eight<bf16_t> {
+  uint2 v[2];
+};
+// Group q's of the slab at k; rows may be read four numbers at a time.
+__device__ __forceinline__ void load8(Eight<float>& e, const float* row, int k, int q) {
+  e.v[0] = *(const f32x4*)(row + k + q * 4);
+  e.v[1] = *(const f32x4*)(row + k + 16 + q * 4);
+}
+__device__ __forceinline__ void load8(Eight<bf16_t>& e, const bf16_t* row, int k, int q) {
+  e.v[0] = *(const uint2*)(row + k + q * 4);
+  e.v[1] = *(const uint2*)(row + k + 16 + q * 4);
+}
+// The same with zeros from `end` on; four numbers at a time (FOURS: `end` is a multiple of four) or one.
+template <bool FOURS>
+__device__ __forceinline__ void load8_to(Eight<float>& e, const float* row, int k, int q, int end) {
 #pragma unroll
-  for (int u = 0; u < 4; ++u) v[u] = k + u < end ? to_f32(row[k + u]) : 0.f;
-  return v;
+  for (int h = 0; h < 2; ++h) {
+    const int at = k + 16 * h + q * 4;
+    if (FOURS) {
+      e.v[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (at < end) e.v[h] = *(const f32x4*)(row + at);
+    } else {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) e.v[h][u] = at + u < end ? row[at + u] : 0.f;
+    }
+  }
+}
+template <bool FOURS>
+__device__ __forceinline__ void load8_to(Eight<bf16_t>& e, const bf16_t* row, int k, int q, int end) {
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int at = k + 16 * h + q * 4;
+    if (FOURS) {
+      e.v[h] = uint2{0u, 0u};
+      if (at < end) e.v[h] = *(const uint2*)(row + at);
+    } else {
+      uint32_t w[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) w[u] = at + u < end ? ((const uint16_t*)row)[at + u] : 0u;
+      e.v[h] = uint2{w[0] | w[1] << 16, w[2] | w[3] << 16};
+    }
+  }
 }
 
-// One slab: four instructions, the j-th numbers of the lanes' fours.
-__device__ __forceinline__ f32x4 slab(f32x4 acc, f32x4 a, f32x4 b) {
+// The same without a condition around a load (one makes the compiler wait for every load on its way): what lies from `end` on is
+// read elsewhere in the row, and `cut` makes it zero when it is there.
+template <bool FOURS>
+__device__ __forceinline__ void load8_anyhow(Eight<float>& e, const float* row, int k, int q, int end) {
 #pragma unroll
-  for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], b[j], acc, 0, 0, 0);
-  return acc;
+  for (int h = 0; h < 2; ++h) {
+    const int at = k + 16 * h + q * 4;
+    if (FOURS) {
+      e.v[h] = *(const f32x4*)(row + min(at, end - 4));
+    } else {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) e.v[h][u] = row[min(at + u, end - 1)];
+    }
+  }
+}
+template <bool FOURS>
+__device__ __forceinline__ void load8_anyhow(Eight<bf16_t>& e, const bf16_t* row, int k, int q, int end) {
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int at = k + 16 * h + q * 4;
+    if (FOURS) {
+      e.v[h] = *(const uint2*)(row + min(at, end - 4));
+    } else {
+      uint32_t w[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) w[u] = ((const uint16_t*)row)[min(at + u, end - 1)];
+      e.v[h] = uint2{w[0] | w[1] << 16, w[2] | w[3] << 16};
+    }
+  }
+}
+__device__ __forceinline__ void cut(Eight<float>& e, int k, int q, int end) {
+#pragma unroll
+  for (int u = 0; u < 8; ++u)
+    if (k + u / 4 * 16 + q * 4 + u % 4 >= end) e.v[u / 4][u % 4] = 0.f;
+}
+__device__ __forceinline__ void cut(Eight<bf16_t>& e, int k, int q, int end) {
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int left = end - (k + 16 * h + q * 4);  // numbers of the four that there are
+    e.v[h].x &= left >= 2 ? ~0u : left == 1 ? 0xffffu : 0u;
+    e.v[h].y &= left >= 4 ? ~0u : left == 3 ? 0xffffu : 0u;
+  }
+}
+
+// The eight as sums of bfloat16 numbers, largest part first: three of them hold a float32's 24 bits.  The first is the nearest
+// (so that the products left out below have either sign), the second what its first eight bits are of the rest, and the
+// differences are exact.  Additions and masks and not v_cvt_pk_bf16_f32 and v_dot2c_f32_bf16, which do it in half the
+// instructions: beside a matrix instruction of 17 clocks two of the former are free, but one of the latter makes it 35.
+template <typename T>
+struct Parts {
+  static constexpr int P = sizeof(T) == 4 ? 3 : 1;
+  u32x4 p[P];
+};
+__device__ __forceinline__ uint32_t upper_halves(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); }
+// Half h of the eight: four numbers.
+__device__ __forceinline__ void half_parts_of(Parts<float>& o, const Eight<float>& e, int h) {
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const float a = e.v[h][2 * i], b = e.v[h][2 * i + 1];
+    const uint32_t a0 = __float_as_uint(a) + 0x8000u, b0 = __float_as_uint(b) + 0x8000u;
+    const float a1 = a - __uint_as_float(a0 & 0xffff0000u), b1 = b - __uint_as_float(b0 & 0xffff0000u);
+    const float a2 = a1 - __uint_as_float(__float_as_uint(a1) & 0xffff0000u), b2 = b1 - __uint_as_float(__float_as_uint(b1) & 0xffff0000u);
+    o.p[0][2 * h + i] = upper_halves(a0, b0);
+    o.p[1][2 * h + i] = upper_halves(__float_as_uint(a1), __float_as_uint(b1));
+    o.p[2][2 * h + i] = upper_halves(__float_as_uint(a2), __float_as_uint(b2));
+  }
+}
+__device__ __forceinline__ void half_parts_of(Parts<bf16_t>& o, const Eight<bf16_t>& e, int h) {
+  o.p[0][2 * h] = e.v[h].x;
+  o.p[0][2 * h + 1] = e.v[h].y;
+}
+template <typename T>
+__device__ __forceinline__ void parts_of(Parts<T>& o, const Eight<T>& e) {
+  half_parts_of(o, e, 0);
+  half_parts_of(o, e, 1);
+}
+
+__device__ __forceinline__ f32x4 mfma(u32x4 a, u32x4 w, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, w), c, 0, 0, 0);
+}
+
+// A slab's sum, which then joins the others'.  float32: the six products of parts that reach its 24 bits, small ones first.
+__device__ __forceinline__ f32x4 slab(const Parts<float>& a, const Parts<float>& w) {
+  f32x4 t = mfma(a.p[2], w.p[0], f32x4{0.f, 0.f, 0.f, 0.f});
+  t = mfma(a.p[0], w.p[2], t);
+  t = mfma(a.p[1], w.p[1], t);
+  t = mfma(a.p[1], w.p[0], t);
+  t = mfma(a.p[0], w.p[1], t);
+  return mfma(a.p[0], w.p[0], t);
+}
+__device__ __forceinline__ f32x4 slab(const Parts<bf16_t>& a, const Parts<bf16_t>& w) { return mfma(a.p[0], w.p[0], f32x4{0.f, 0.f, 0.f, 0.f}); }
+
+// A result that is not finite is formed again from the numbers themselves: an infinity has no parts (its remainder is no
+// number), nor have the last few numbers below the largest, whose nearest first part is infinite.  A number by itself, as
+// it should never be needed; the blocks' sums are added as ever.
+__device__ __forceinline__ bool is_finite(float v) { return fabsf(v) <= 3.402823466e38f; }
+__device__ __attribute__((noinline)) float formed_again(const float* a, const float* w, int K) {
+  float total = 0.f;
+  for (int k = 0; k < K && total == total; k += GP_BLOCK) {
+    float sum = 0.f;
+    const int end = min(K, k + GP_BLOCK);
+    for (int i = k; i < end && sum == sum; ++i) sum = fmaf(a[i], w[i], sum);
+    total += sum;
+  }
+  return total;
 }
 
 // Up to 16 * MT rows: blockIdx.x 16 weight rows, blockIdx.y the product of the batch, blockIdx.z a share of
@@ -84,7 +235,7 @@ __global__ __launch_bounds__(64 * GP_FEW_WAVES) void gemm_plain_few_kernel(
   const TA* a_row[MT];
 #pragma unroll
   for (int i = 0; i < MT; ++i) a_row[i] = A + (int64_t)min(i * 16 + r, M - 1) * lda;
-  constexpr int U = MT == 1 ? 4 : 2;  // slabs whose loads are on their way together, twice
+  constexpr int U = MT == 1 ? 2 : 1;  // slabs whose loads are on their way together, twice
   constexpr int TOTALS = (16 * MT * 16) / PAE_WAVE;
   float total[TOTALS];  // thread t: outputs t, t + threads, ...
 #pragma unroll
@@ -102,22 +253,28 @@ __global__ __launch_bounds__(64 * GP_FEW_WAVES) void gemm_plain_few_kernel(
       if (steady) {
         // two batches take turns; no load stands under a condition of its own
         struct Batch {
-          f32x4 w[U], a[U][MT];
+          Eight<TA> w[U], a[U][MT];
         } b0, b1;
         auto fetch = [&](Batch& b, int at) {
 #pragma unroll
           for (int u = 0; u < U; ++u) {
-            b.w[u] = load4(w_row + at + u * GP_SLAB + kq * 4);
+            load8(b.w[u], w_row, at + u * GP_SLAB, kq);
 #pragma unroll
-            for (int i = 0; i < MT; ++i) b.a[u][i] = load4(a_row[i] + at + u * GP_SLAB + kq * 4);
+            for (int i = 0; i < MT; ++i) load8(b.a[u][i], a_row[i], at + u * GP_SLAB, kq);
           }
           __builtin_amdgcn_sched_barrier(0);
         };
         auto multiply = [&](const Batch& b) {
 #pragma unroll
-          for (int u = 0; u < U; ++u)
+          for (int u = 0; u < U; ++u) {
+            Parts<TA> w, a;
+            parts_of(w, b.w[u]);
 #pragma unroll
-            for (int i = 0; i < MT; ++i) acc[i] = slab(acc[i], b.a[u][i], b.w[u]);
+            for (int i = 0; i < MT; ++i) {
+              parts_of(a, b.a[u][i]);
+              acc[i] += slab(a, w);
+            }
+          }
           __builtin_amdgcn_sched_barrier(0);
         };
         constexpr int STEP = GP_SLAB * U;
@@ -141,9 +298,16 @@ __global__ __launch_bounds__(64 * GP_FEW_WAVES) void gemm_plain_few_kernel(
         k += batches * STEP;
       }
       for (; k < end; k += GP_SLAB) {
-        const f32x4 w = load4_to(w_row, k + kq * 4, end);
+        Eight<TA> raw;
+        Parts<TA> w, a;
+        load8_to<VEC>(raw, w_row, k, kq, end);
+        parts_of(w, raw);
 #pragma unroll
-        for (int i = 0; i < MT; ++i) acc[i] = slab(acc[i], load4_to(a_row[i], k + kq * 4, end), w);
+        for (int i = 0; i < MT; ++i) {
+          load8_to<VEC>(raw, a_row[i], k, kq, end);
+          parts_of(a, raw);
+          acc[i] += slab(a, w);
+        }
       }
     }
     if (scratch) {  // this block's sums to memory; another kernel adds them up
@@ -179,25 +343,33 @@ __global__ __launch_bounds__(64 * GP_FEW_WAVES) void gemm_plain_few_kernel(
     const int o = threadIdx.x + i * blockDim.x, m = o / 16, n = n0 + o % 16;
     if (o < MT * 256 && m < M && n < N) {
       float v = total[i];
+      if constexpr (Parts<TA>::P > 1) {
+        if (!is_finite(v)) v = formed_again(A + m * lda, W + (int64_t)n * K, K);
+      }
       if (bias) v += load_param(bias, b_is_f32, n);
       C[(int64_t)m * ldc + n] = from_f32<TC>(v);
     }
   }
 }
 
-// Tiles of BM x BN, four wavefronts of BM/2 x BN/2.  blockIdx.x: the tiles, those of one column of tiles (the same weights)
+// Tiles of BM rows of A by BN of W, WM x WN wavefronts.  blockIdx.x: the tiles, those of one column of tiles (the same weights)
 // next to each other on one die; blockIdx.y: the product of the batch; blockIdx.z: a share of the blocks of k.
-// A row's 16 numbers of a slab lie in LDS as four fours, at places turned by the row so that the 16 rows
-// a wavefront reads a four of fall into different banks.
-template <typename TA, typename TC, int BM, int BN, int SLABS, bool VEC>
-__global__ __launch_bounds__(256) void gemm_plain_tiles_kernel(
+// What bounds it is the matrix cores' six instructions a slab of float32 and, not far behind, LDS, which takes in 192 bytes a row
+// and slab and gives them to WN or WM wavefronts; a thread takes three eights a slab apart (26 instructions a half; one eight in
+// tiles of 64 x 64) between its products.  A row of 32 numbers of one part, 64 bytes, lies in LDS as four eights, at places turned by the row so
+// that the 16 rows that a wavefront reads an eight of fall into different banks.
+template <typename TA, typename TC, int BM, int BN, int WM, int WN, bool VEC, bool SHARED>
+__global__ __launch_bounds__(64 * WM * WN, 2) void gemm_plain_tiles_kernel(
     TC* __restrict__ C, int64_t ldc, const TA* __restrict__ A, int64_t lda, const TA* __restrict__ W,
     const void* __restrict__ bias, int b_is_f32, int M, int N, int K, int64_t batch_c, int64_t batch_a,
     int64_t batch_w, float* __restrict__ scratch) {
   C += blockIdx.y * batch_c;
   A += blockIdx.y * batch_a;
   W += blockIdx.y * batch_w;
-  __shared__ f32x4 a_lds[2][SLABS][BM * 4], w_lds[2][SLABS][BN * 4];
+  constexpr int THREADS = 64 * WM * WN, P = Parts<TA>::P, MT = BM / WM / 16, NT = BN / WN / 16;
+  constexpr int E = (BM + BN) * 4 / THREADS;  // eights that a thread brings
+  static_assert((BM + BN) * 4 % THREADS == 0, "whole eights");
+  extern __shared__ u32x4 parts_lds[];  // [2][P][BM + BN][4]
   const int tid = threadIdx.x, lane = tid % PAE_WAVE, r = lane % 16, kq = lane / 16;
   const int wave = __builtin_amdgcn_readfirstlane(tid / PAE_WAVE);
   const int tiles_m = (M + BM - 1) / BM;
@@ -205,144 +377,152 @@ __global__ __launch_bounds__(256) void gemm_plain_tiles_kernel(
   // workgroups i, i + 8, i + 16, ... run on one die: they take neighbouring tiles
   const int per = tiles / 8, rest = tiles % 8, die = blockIdx.x % 8;
   const int tile = die * per + min(die, rest) + blockIdx.x / 8;
-  const int m0 = (tile % tiles_m) * BM, n0 = (tile / tiles_m) * BN;
+  const int m_tile = (tile % tiles_m) * BM, n_tile = (tile / tiles_m) * BN;
+  const int m0 = m_tile + wave / WN * (BM / WM), n0 = n_tile + wave % WN * (BN / WN);
   const int blocks = (K + GP_BLOCK - 1) / GP_BLOCK;
   const int share = (blocks + gridDim.z - 1) / gridDim.z;
   const int block0 = blockIdx.z * share, block1 = min(blocks, block0 + share);
   if (block0 >= block1) return;
 
-  constexpr int CA = BM * 4 / 256, CW = BN * 4 / 256;  // fours that a thread brings of either side
-  const TA* a_src[CA];
-  const TA* w_src[CW];
-  int a_dst[CA], w_dst[CW];
+  const TA* src[E];
+  int dst[E];
 #pragma unroll
-  for (int i = 0; i < CA; ++i) {
-    const int c = tid + i * 256, row = c / 4;
-    a_src[i] = A + (int64_t)min(m0 + row, M - 1) * lda;
-    a_dst[i] = row * 4 + ((c % 4) ^ ((row >> 2) & 3));
+  for (int u = 0; u < E; ++u) {
+    const int c = tid + u * THREADS, row = c / 4;
+    src[u] = row < BM ? A + (int64_t)min(m_tile + row, M - 1) * lda : W + (int64_t)min(n_tile + row - BM, N - 1) * K;
+    dst[u] = row * 4 + ((c % 4) ^ ((row >> 1) & 3));
   }
+  const int at = r * 4 + (kq ^ ((r >> 1) & 3));  // of the lane's eight within 16 rows
+  const int a_at = wave / WN * (BM / WM) * 4 + at, w_at = (BM + wave % WN * (BN / WN)) * 4 + at;
+
+  f32x4 acc[MT][NT], total[SHARED ? 1 : MT][NT];
 #pragma unroll
-  for (int i = 0; i < CW; ++i) {
-    const int c = tid + i * 256, row = c / 4;
-    w_src[i] = W + (int64_t)min(n0 + row, N - 1) * K;
-    w_dst[i] = row * 4 + ((c % 4) ^ ((row >> 2) & 3));
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[i][j] = total[SHARED ? 0 : i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  Eight<TA> raw[E];
+  const int k_begin = block0 * GP_BLOCK;
+  auto fetch = [&](int u, int k) { load8_anyhow<VEC>(raw[u], src[u], k, tid % 4, K); };
+  auto parts_at = [&](int buf, int p) { return parts_lds + (buf * P + p) * ((BM + BN) * 4); };
+  auto store = [&](const Parts<TA>& part, int u, int buf) {
+#pragma unroll
+    for (int p = 0; p < P; ++p) parts_at(buf, p)[dst[u]] = part.p[p];
+  };
+#pragma unroll
+  for (int u = 0; u < E; ++u) fetch(u, k_begin);
+#pragma unroll
+  for (int u = 0; u < E; ++u) {
+    Parts<TA> part;
+    if (k_begin + GP_SLAB > K) cut(raw[u], k_begin, tid % 4, K);
+    parts_of(part, raw[u]);
+    store(part, u, 0);
+    fetch(u, k_begin + GP_SLAB);
   }
-  const int kc = (tid % 4) * 4;
-  constexpr int TM = BM / 32, TN = BN / 32;  // matrix tiles of a wavefront
-  const int wm = (wave / 2) * (BM / 2), wn = (wave % 2) * (BN / 2);
-  const int at = r * 4 + (kq ^ ((r >> 2) & 3));  // of the lane's four within a matrix tile's 16 rows
-
-  f32x4 acc[TM][TN], total[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = total[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  f32x4 a_reg[SLABS][CA], w_reg[SLABS][CW];
-  auto fetch = [&](int k) {
-    if (VEC && k + GP_SLAB * SLABS <= K) {
-#pragma unroll
-      for (int u = 0; u < SLABS; ++u) {
-#pragma unroll
-        for (int i = 0; i < CA; ++i) a_reg[u][i] = load4(a_src[i] + k + u * GP_SLAB + kc);
-#pragma unroll
-        for (int i = 0; i < CW; ++i) w_reg[u][i] = load4(w_src[i] + k + u * GP_SLAB + kc);
-      }
-    } else {  // zeros past the end add nothing
-#pragma unroll
-      for (int u = 0; u < SLABS; ++u) {
-#pragma unroll
-        for (int i = 0; i < CA; ++i) a_reg[u][i] = load4_to(a_src[i], k + u * GP_SLAB + kc, K);
-#pragma unroll
-        for (int i = 0; i < CW; ++i) w_reg[u][i] = load4_to(w_src[i], k + u * GP_SLAB + kc, K);
-      }
-    }
-  };
-  auto put = [&](int buf) {
-#pragma unroll
-    for (int u = 0; u < SLABS; ++u) {
-#pragma unroll
-      for (int i = 0; i < CA; ++i) a_lds[buf][u][a_dst[i]] = a_reg[u][i];
-#pragma unroll
-      for (int i = 0; i < CW; ++i) w_lds[buf][u][w_dst[i]] = w_reg[u][i];
-    }
-  };
-  const int k_begin = block0 * GP_BLOCK, k_end = min(K, block1 * GP_BLOCK);
-  fetch(k_begin);
-  put(0);
   __syncthreads();
   int buf = 0;
   for (int block = block0; block < block1; ++block) {
     const int end = min(K, (block + 1) * GP_BLOCK);
-    for (int k = block * GP_BLOCK; k < end; k += GP_SLAB * SLABS) {
-      const bool more = k + GP_SLAB * SLABS < k_end;
-      if (more) fetch(k + GP_SLAB * SLABS);
+    for (int k = block * GP_BLOCK; k < end; k += GP_SLAB) {
+      // the products, and between them the parts of the next slab's numbers (behind the last slab: of what nobody reads)
+      Parts<TA> a[2], w[NT], part;
+      f32x4 sum[2][NT];
+      auto read_a = [&](int i) {
 #pragma unroll
-      for (int u = 0; u < SLABS; ++u) {
-        f32x4 a[TM], w[TN];
+        for (int p = 0; p < P; ++p) a[i % 2].p[p] = parts_at(buf, p)[a_at + i * 64];
+      };
+      read_a(0);
 #pragma unroll
-        for (int i = 0; i < TM; ++i) a[i] = a_lds[buf][u][(wm + i * 16) * 4 + at];
+      for (int j = 0; j < NT; ++j)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) w[j] = w_lds[buf][u][(wn + j * 16) * 4 + at];
+        for (int p = 0; p < P; ++p) w[j].p[p] = parts_at(buf, p)[w_at + j * 64];
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
+      for (int i = 0; i < MT; ++i) {
+        if (i + 1 < MT) read_a(i + 1);
+        constexpr int HALVES = 2 * E;
 #pragma unroll
-          for (int i = 0; i < TM; ++i)
+        for (int h = i * HALVES / MT; h < (i + 1) * HALVES / MT; ++h) {
+          if (h % 2 == 0 && k + 2 * GP_SLAB > K) cut(raw[h / 2], k + GP_SLAB, tid % 4, K);
+          half_parts_of(part, raw[h / 2], h % 2);
 #pragma unroll
-            for (int j = 0; j < TN; ++j)
-              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][q], w[j][q], acc[i][j], 0, 0, 0);
+          for (int p = 0; p < P; ++p)  // here and not where the compiler would have it: in one piece behind the products
+            asm volatile("" : "+v"(part.p[p][h % 2 * 2]), "+v"(part.p[p][h % 2 * 2 + 1]));
+          if (h % 2) {
+            store(part, h / 2, buf ^ 1);
+            fetch(h / 2, k + 2 * GP_SLAB);
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < NT; ++j) sum[i % 2][j] = slab(a[i % 2], w[j]);
+        if (i > 0) {  // the sums before these, which are done by now
+#pragma unroll
+          for (int j = 0; j < NT; ++j) acc[i > 0 ? i - 1 : 0][j] += sum[(i + 1) % 2][j];
+        }
+        __builtin_amdgcn_sched_barrier(0);
       }
-      if (more) {
-        put(buf ^ 1);
-        __syncthreads();
-        buf ^= 1;
-      }
+#pragma unroll
+      for (int j = 0; j < NT; ++j) acc[MT - 1][j] += sum[(MT - 1) % 2][j];
+      __syncthreads();
+      buf ^= 1;
     }
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+    for (int i = 0; i < MT; ++i)
 #pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        if (scratch) {
-          const int n = n0 + wn + j * 16 + r;
+      for (int j = 0; j < NT; ++j) {
+        if (SHARED) {
+          const int n = n0 + j * 16 + r, m = m0 + i * 16 + kq * 4;
+          float* p = scratch + ((int64_t)block * M + m) * N + n;
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int m = m0 + wm + i * 16 + kq * 4 + e;
-            if (m < M && n < N) scratch[((int64_t)block * M + m) * N + n] = acc[i][j][e];
-          }
+          for (int e = 0; e < 4; ++e, p += N)
+            if (m + e < M && n < N) *p = acc[i][j][e];
         } else {
-          total[i][j] += acc[i][j];
+          total[SHARED ? 0 : i][j] += acc[i][j];
         }
         acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
       }
   }
-  if (scratch) return;
+  if (SHARED) return;
+  bool whole = true;
 #pragma unroll
-  for (int j = 0; j < TN; ++j) {
-    const int n = n0 + wn + j * 16 + r;
+  for (int j = 0; j < NT; ++j) {
+    const int n = n0 + j * 16 + r;
     if (n >= N) continue;
     const float b = bias ? load_param(bias, b_is_f32, n) : 0.f;
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+    for (int i = 0; i < MT; ++i)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int m = m0 + wm + i * 16 + kq * 4 + e;
+        const int m = m0 + i * 16 + kq * 4 + e;
         if (m >= M) continue;
-        float v = total[i][j][e];
+        float v = total[SHARED ? 0 : i][j][e];
+        whole = whole && is_finite(v);
         if (bias) v += b;
         C[(int64_t)m * ldc + n] = from_f32<TC>(v);
       }
   }
+  if constexpr (P > 1) {
+    if (whole) return;
+    for (int o = 0; o < MT * NT * 4; ++o) {  // the sums are gone from the registers: what was stored is looked at
+      const int n = n0 + o % NT * 16 + r, m = m0 + o / (NT * 4) * 16 + kq * 4 + o / NT % 4;
+      if (m >= M || n >= N || is_finite(C[(int64_t)m * ldc + n])) continue;
+      float v = formed_again(A + m * lda, W + (int64_t)n * K, K);
+      if (bias) v += load_param(bias, b_is_f32, n);
+      C[(int64_t)m * ldc + n] = v;
+    }
+  }
 }
 
 // The block sums [blocks][M][N] added up in order.
-template <typename TC>
-__global__ __launch_bounds__(256) void gemm_plain_sum_kernel(TC* __restrict__ C, int64_t ldc,
+template <typename TA, typename TC>
+__global__ __launch_bounds__(256) void gemm_plain_sum_kernel(TC* __restrict__ C, int64_t ldc, const TA* __restrict__ A,
+                                                             int64_t lda, const TA* __restrict__ W,
                                                              const float* __restrict__ scratch,
                                                              const void* __restrict__ bias, int b_is_f32, int M,
-                                                             int N, int blocks) {
+                                                             int N, int K) {
   const int n = blockIdx.x * 256 + threadIdx.x;
   const int m = blockIdx.y;
   if (n >= N) return;
+  const int blocks = (K + GP_BLOCK - 1) / GP_BLOCK;
   const int64_t stride = (int64_t)M * N;
   const float* p = scratch + (int64_t)m * N + n;
   float total = 0.f;
@@ -355,18 +535,41 @@ __global__ __launch_bounds__(256) void gemm_plain_sum_kernel(TC* __restrict__ C,
     for (int u = 0; u < 8; ++u) total += v[u];
   }
   for (; b < blocks; ++b) total += p[b * stride];
+  if constexpr (Parts<TA>::P > 1) {
+    if (!is_finite(total)) total = formed_again(A + m * lda, W + (int64_t)n * K, K);
+  }
   if (bias) total += load_param(bias, b_is_f32, n);
   C[(int64_t)m * ldc + n] = from_f32<TC>(total);
 }
 
+// Tiles of 128 x 256 have the most products to a byte of LDS (M = N = 2,048 rows and 17,920 features of 1,536: 660 us against
+// 820 in tiles of 64 x 128), tiles of 64 x 64 let three workgroups a compute unit hide each other's waits and spread over the chip.  The
+// line lies at 200 pairs of a large tile and a block of k, of which a unit takes one at a time; a little over the chip's 256
+// leaves it a second round nearly empty.  Large / small: 65 x 17,920 x 1,536 (210 pairs) 53 / 62 us, 200 x 1,536 x 8,960 (216) 51 / 64, 450 x
+// 1,536 x 8,960 (432) 101 / 117, 601 x 17,920 x 1,536 (1,050) 249 / 275; 128 x 1,536 x 8,960 (108) 53 / 41, 601 x 2,048 x 1,536 (120) 46 /
+// 40, 65 x 2,048 x 1,536 (24) 40 / 14, 300 x 1,536 x 8,960 (324) 90 / 79, 2,048 x 1,536 x 1,536 (288) 94 / 74,
+// 400 x 17,920 x 1,536 (280 tiles) 254 / 187.
+struct GpShape {
+  int rows, cols;
+};
+static GpShape shape_of(int M, int N, int K) {
+  const int64_t tiles = (int64_t)((M + 127) / 128) * ((N + 255) / 256), pairs = tiles * ((K + GP_BLOCK - 1) / GP_BLOCK);
+  const int64_t groups = tiles >= GP_LARGE_WHOLE ? tiles : pairs;
+  const bool second_round = groups > GP_UNITS && groups <= GP_UNITS + GP_UNITS / 4 + 10;
+  return pairs >= 200 && !second_round ? GpShape{128, 256} : GpShape{64, 64};
+}
+static int64_t tiles_of(int M, int N, GpShape shape) {
+  return (int64_t)((M + shape.rows - 1) / shape.rows) * ((N + shape.cols - 1) / shape.cols);
+}
 // Over how many workgroups the blocks of k of one tile are shared: 1 where the tiles fill the chip by themselves or
 // there is one block only.  A share costs its sums a way to memory and back and the launch that adds them (about
-// 4 us), so that up to 64 rows a workgroup's wavefronts take up to GP_FEW_WAVES blocks side by side first.
-// Up to 64 rows a compute unit works through its workgroups in rounds, and shares pay where they leave fewer rounds of the whole
-// k; with more rows, up to one and a half tiles a compute unit.  Measured without shares / with them: 3 rows of 11,008 by 128 sixteens of
-// weight rows (2 rounds of a third) 36.1 / 30.1 us, of 16,384 by 192 (3 of a quarter) 50.0 / 44.3, of 8,192 by 192 (2 of a half)
-// 27.0 / 28.6, of 11,008 by 256 (3 of a third) 44.8 / 49.3; 320 tiles 392 / 299 (601 x 2,048 x 11,008), 376 669 / 632 (3,000 x 512 x
-// 18,944), 416 397 / 433 (800 x 2,048 x 11,008), 658 258 / 288 (3,000 x 896 x 4,864), 728 992 / 1,121 (800 x 3,584 x 18,944).
+// 4 us), so that up to 32 rows a workgroup's wavefronts take up to GP_FEW_WAVES blocks side by side first.
+// Few rows: a compute unit works through its workgroups in rounds, and shares pay where they leave fewer rounds of the whole
+// k.  Measured without shares / with them: 3 rows of 11,008 by 128 sixteens of weight rows (2 rounds of a third) 36.1 / 30.1 us, of
+// 16,384 by 192 (3 of a quarter) 50.0 / 44.3, of 8,192 by 192 (2 of a half) 27.0 / 28.6, of 11,008 by 256 (3 of a third) 44.8 / 49.3.
+// More rows: large tiles are shared up to 160 of them, for two rounds of the chip (300 x 17,920 x 1,536, 210 tiles, 122 / 146;
+// 200 x 17,920 x 1,536, 140 tiles, 128 / 109), small ones up to 500, for three workgroups a compute unit (601 x 2,048 x 1,536, 320
+// tiles, 44 / 40; 601 x 1,536 x 1,536, 240 tiles, the same both ways).
 static int splits_of(int M, int N, int K) {
   const int blocks = (K + GP_BLOCK - 1) / GP_BLOCK;
   if (M <= 0 || blocks == 1) return 1;
@@ -376,9 +579,10 @@ static int splits_of(int M, int N, int K) {
     const int64_t rounds = (sixteens + GP_UNITS - 1) / GP_UNITS, rounds_of_shares = (sixteens * shares + GP_UNITS - 1) / GP_UNITS;
     return rounds_of_shares < rounds * shares && shares <= 65535 ? (int)shares : 1;
   }
-  const int64_t tiles = (int64_t)((M + GP_TILE - 1) / GP_TILE) * ((N + GP_TILE - 1) / GP_TILE);
-  if (2 * tiles >= 3 * GP_UNITS) return 1;
-  const int want = (int)((3 * GP_UNITS + tiles - 1) / tiles);  // three workgroups a compute unit
+  const GpShape shape = shape_of(M, N, K);
+  const int64_t tiles = tiles_of(M, N, shape);
+  if (tiles >= (shape.rows == 128 ? GP_LARGE_WHOLE : 500)) return 1;
+  const int want = (int)(((shape.rows == 128 ? 2 : 3) * GP_UNITS + tiles - 1) / tiles);
   return want < blocks ? want : blocks;
 }
 
@@ -426,27 +630,45 @@ static int launch_plain(void* C, int64_t ldc, int64_t batch_c, const void* A, in
   const int blocks = (K + GP_BLOCK - 1) / GP_BLOCK;
 #define GP_ARGS                                                                                                  \
   (TC*)C, ldc, (const TA*)A, lda, (const TA*)W, bias, b_is_f32, M, N, K, batch_c, batch_a, batch_w, scratch
-  // (over 32 rows read number by number by one wavefront a workgroup: the tiles are faster, 64 x 130 x 511 67 -> 44 us; over
-  // five blocks of k they are not, 64 x 1,537 x 2,049 74 against 171)
-  if (M <= (VEC || blocks > 1 ? GP_FEW_ROWS : GP_FEW_ROWS / 2)) {
+  // Over 32 rows the tiles are faster (33 x 17,920 x 1,536 59 us against 48, 33 x 1,536 x 8,960 49 against 24, 33 x 1,536 x 1,536 16 against
+  // 14.5), except that rows read number by number stay with `few` up to 64 where there is more than a block of k (64 x 1,537 x 2,049 42 us)
+  if (M <= (VEC || blocks == 1 ? GP_FEW_ROWS : 2 * GP_FEW_ROWS)) {
     const int each = (blocks + splits - 1) / splits;
     const int waves = each < GP_FEW_WAVES ? each : GP_FEW_WAVES;
     const dim3 grid((N + 15) / 16, batch, splits);
 #define GP_FEW(MT)                                                                                               \
   gemm_plain_few_kernel<TA, TC, MT, VEC><<<grid, waves * PAE_WAVE, scratch ? 0 : waves * MT * 1024, stream>>>(GP_ARGS)
     if (M <= 16) GP_FEW(1);
-    else if (M <= 32) GP_FEW(2);
-    else GP_FEW(4);
+    else if (VEC || M <= 32) GP_FEW(2);
+    else GP_FEW(VEC ? 2 : 4);
 #undef GP_FEW
   } else {
-    const dim3 grid((unsigned)(((M + GP_TILE - 1) / GP_TILE) * (int64_t)((N + GP_TILE - 1) / GP_TILE)), batch, splits);
-    gemm_plain_tiles_kernel<TA, TC, GP_TILE, GP_TILE, 2, VEC><<<grid, 256, 0, stream>>>(GP_ARGS);
+    const GpShape shape = shape_of(M, N, K);
+    const dim3 grid((unsigned)tiles_of(M, N, shape), batch, splits);
+    constexpr int ROW = 2 * Parts<TA>::P * 64;  // bytes of LDS
+#define GP_TILES(BM, BN, WM, WN, SHARED)                                                                                  \
+  do {                                                                                                                    \
+    auto kernel = gemm_plain_tiles_kernel<TA, TC, BM, BN, WM, WN, VEC, SHARED>;                                           \
+    const hipError_t allowed =                                                                                            \
+        hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (BM + BN) * ROW);            \
+    PAE_REQUIRE(allowed == hipSuccess, "gemm: no %d bytes of LDS", (BM + BN) * ROW);                                      \
+    kernel<<<grid, 64 * WM * WN, (BM + BN) * ROW, stream>>>(GP_ARGS);                                                     \
+  } while (0)
+    if (shape.rows == 128) {
+      if (scratch) GP_TILES(128, 256, 1, 8, true);
+      else GP_TILES(128, 256, 1, 8, false);
+    } else {
+      if (scratch) GP_TILES(64, 64, 2, 4, true);
+      else GP_TILES(64, 64, 2, 4, false);
+    }
+#undef GP_TILES
   }
 #undef GP_ARGS
   if (scratch) {
     const int bad = pae_check_launch("gemm_plain");
     if (bad) return bad;
-    gemm_plain_sum_kernel<TC><<<dim3((N + 255) / 256, M), 256, 0, stream>>>((TC*)C, ldc, scratch, bias, b_is_f32, M, N, blocks);
+    gemm_plain_sum_kernel<TA, TC><<<dim3((N + 255) / 256, M), 256, 0, stream>>>((TC*)C, ldc, (const TA*)A, lda, (const TA*)W, scratch,
+                                                                                bias, b_is_f32, M, N, K);
   }
   return pae_check_launch("gemm_plain");
 }

@@ -112,6 +112,41 @@ def test_gemm_plain_adds_in_one_order(N, K_):
         assert torch.equal(one_by_one, out), M
 
 
+@pytest.mark.parametrize("M,N,K_", [(3, 40, 600), (40, 70, 31), (70, 200, 600), (64, 65, 100), (129, 90, 1537), (65, 1500, 17000),
+                                    (257, 18000, 520)])
+def test_gemm_plain_keeps_what_is_not_finite(M, N, K_):
+    """float32 numbers are taken apart for the product; infinities, numbers that are none and numbers so large that their first part would be
+    infinite give what they give in the numbers themselves, in every kernel (few rows; small and large tiles, shared k
+    or not), and nothing beside them changes.  Rows of small numbers keep their digits."""
+    torch.manual_seed(M)
+    a, w = torch.randn(M, K_, device=DEV), torch.randn(N, K_, device=DEV)
+    plain = torch.empty(M, N, device=DEV)
+    K().gemm_plain(plain, a, w)
+    top = torch.finfo(torch.float32).max
+    w[:, 5] = w[:, 5].sign() * 1e-3
+    a[M // 2, 5] = top
+    w[1, 3] = 0.0
+    a[0, 3] = float("inf")
+    a[M - 1, K_ - 1] = float("nan")
+    a[1] *= 2.0 ** -90
+    out = torch.empty(M, N, device=DEV)
+    K().gemm_plain(out, a, w)
+    want = (a.double() @ w.double().t())
+    assert bool(want[0].isinf().sum() == N - 1) and bool(want[0, 1].isnan()) and bool(want[M - 1].isnan().all())
+    assert torch.equal(out.isnan(), want.isnan()) and torch.equal(out.isinf(), want.isinf())
+    assert torch.equal(out[0][out[0].isinf()].sign().double(), want[0][want[0].isinf()].sign())
+    finite = torch.where(want.isfinite(), want, 0.0)
+    # as in the test above: 512 roundings of half a unit of the sum of the products' sizes, of which a quarter bounds what is seen
+    bound = 512 * 2.0 ** -24 * 0.25 * (torch.where(a.isfinite(), a, 0.0).double().abs() @ w.double().abs().t())
+    assert bool(((torch.where(out.isfinite(), out, 0.0).double() - finite).abs() <= bound + 1e-300).all())
+    clean = [m for m in range(M) if m not in (0, 1, M // 2, M - 1)]
+    if clean:  # the rows beside them, with the old numbers back in W
+        torch.manual_seed(M)
+        torch.randn(M, K_, device=DEV), w.copy_(torch.randn(N, K_, device=DEV))
+        K().gemm_plain(out, a, w)
+        assert torch.equal(out[clean], plain[clean])
+
+
 @pytest.mark.parametrize("M,N,K_", [(300, 2100, 30000), (2100, 300, 30000)])
 def test_gemm_plain_in_parts_gives_the_bits_of_the_whole(M, N, K_):
     """Products whose blocks' sums do not fit the scratch memory at once are made in parts, along the columns or along the rows:
