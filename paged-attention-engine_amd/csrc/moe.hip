@@ -20,7 +20,7 @@
 // they are the kernels for steps of a few rows.
 #include "common.h"
 #include "api.h"
-#include "tile_gemm.h"
+#include "wide_gemm.h"
 
 template <typename T>
 __global__ __launch_bounds__(256) void project_f32_kernel(float* __restrict__ out, int64_t ldo, const T* __restrict__ A,
@@ -432,8 +432,8 @@ extern "C" int pae_moe_down(int dtype, float* out, const void* act, const void* 
 //                       of a token are float32 partial sums that the stream's next norm adds in order
 // each in three kernels by the step's size: moe_few_tiles (up to 512 pairs), moe_tiles_gate_up / moe_tiles_down (up to
 // 4,096), moe_big_tiles (above).
-using tile_gemm::bf16x8;
-using tile_gemm::f32x4;
+using wide_gemm::bf16x8;
+using wide_gemm::f32x4;
 
 __global__ __launch_bounds__(1024) void moe_sort_kernel(const int* __restrict__ chosen, int pairs, int experts, int tile_rows,
                                                         int* __restrict__ order, int4* __restrict__ tiles, int max_tiles) {
@@ -771,17 +771,19 @@ __global__ __launch_bounds__(256) void moe_few_tiles_kernel(bf16_t* __restrict__
 }
 
 // The same two products for prompts, where an expert sees hundreds of tokens: a workgroup takes a tile of 128 rows
-// and 128 features with gate and up (or 256 output features of the down product) through the loop of tile_gemm.h.
-// What bounds it: the rate at which a compute unit takes lines in (tile_gemm.h), so what a workgroup's neighbours
+// and 128 features with gate and up (or 256 output features of the down product) through the loop of wide_gemm.h, eight wavefronts of
+// 64 x 64.  What bounds it: LDS and the lines that a compute unit takes in (wide_gemm.h), so what a workgroup's neighbours
 // on the die bring to its L2 counts, and padding: experts see a few hundred rows each.  Measured, 3,001 tokens by four of 32
 // experts, 1,536 x 2,240 (165 and 83 GFLOP): with operands through registers, two barriers a stage of 64 of k and
-// one workgroup's features after another 594 and 298 us; through tile_gemm.h 382 and 172; with an expert's
+// one workgroup's features after another 594 and 298 us; four wavefronts of 64 x 128 through LDS 382 and 172; with an expert's
 // tiles side by side on one die 318 and 140 (three quarters of the lines from L2); with the loads spread among
-// the products 306 and 127 us (540 and 650 TFLOP/s).
-#define MOE_BIG_ROWS tile_gemm::BM
-#define MOE_BIG_K tile_gemm::BK
+// the products 306 and 127 us (540 and 650 TFLOP/s); eight wavefronts of 64 x 64, two a
+// SIMD, 243 and 121 us (680 TFLOP/s both).
+typedef wide_gemm::Tile<128, 256, 2, 4, 3> MoeTile;
+#define MOE_BIG_ROWS MoeTile::BM
+#define MOE_BIG_K wide_gemm::BK
 template <bool GATED>
-__global__ __launch_bounds__(256, 1) void moe_big_tiles_kernel(bf16_t* __restrict__ act_out, float* __restrict__ y,
+__global__ __launch_bounds__(512, 1) void moe_big_tiles_kernel(bf16_t* __restrict__ act_out, float* __restrict__ y,
                                                                const bf16_t* __restrict__ a_rows, int64_t lda,
                                                                const bf16_t* __restrict__ w_first, const bf16_t* __restrict__ w_second,
                                                                const int* __restrict__ order, const float* __restrict__ weights,
@@ -800,60 +802,55 @@ __global__ __launch_bounds__(256, 1) void moe_big_tiles_kernel(bf16_t* __restric
   const int first = some - (mine >> 16), within = place - first * blocks;
   const int4 tile = tiles[first + within % (mine & 0xffff)];  // (expert, first sorted row, rows, as above)
   const int n_base = within / (mine & 0xffff) * FEATURES;
-  const int tid = threadIdx.x, lane = tid % PAE_WAVE, wave = __builtin_amdgcn_readfirstlane(tid / PAE_WAVE);
+  const int lane = threadIdx.x % PAE_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PAE_WAVE);
   const int col = lane % 16, kg = lane / 16;
-  const int wr = wave / 2, wc = wave % 2;
-  tile_gemm::Source src;
+  const int wm = wave / MoeTile::WN, wn = wave % MoeTile::WN;
+  MoeTile::Source src;
   src.a = reinterpret_cast<const char*>(a_rows);
-  // W's 256 rows in LDS: gated, the first 128 are gate's features (the first two wavefronts bring them), the rest up's
-  const bf16_t* w = (GATED && wave >= 2) ? w_second : w_first;
+  // A wavefront's 64 rows of W in LDS are, gated, 32 of gate's features and the same 32 of up's; a wavefront brings 32 rows
+  static_assert(MoeTile::W_LOADS * 8 == 32 && MoeTile::PN == 64, "a wavefront brings rows of one of the two");
+  const bf16_t* w = (GATED && wave % 2) ? w_second : w_first;
   src.w = reinterpret_cast<const char*>(w + (int64_t)__builtin_amdgcn_readfirstlane(tile.x) * N * K);
 #pragma unroll
-  for (int j = 0; j < tile_gemm::A_LOADS; ++j) {
-    const int r = (wave * tile_gemm::A_LOADS + j) * 8 + lane / 8;
+  for (int j = 0; j < MoeTile::A_LOADS; ++j) {
+    const int r = (wave * MoeTile::A_LOADS + j) * 8 + lane / 8;
     const int sorted = tile.y + (r < tile.z ? r : 0);
-    src.a_off[j] = (uint32_t)((GATED ? order[sorted] / top : sorted) * lda * 2) + tile_gemm::piece_of(lane, r);
+    src.a_off[j] = (uint32_t)((GATED ? order[sorted] / top : sorted) * lda * 2) + wide_gemm::piece_of(lane, r);
   }
 #pragma unroll
-  for (int j = 0; j < tile_gemm::W_LOADS; ++j) {
-    const int r = (wave * tile_gemm::W_LOADS + j) * 8 + lane / 8;
-    src.w_off[j] = (uint32_t)min(n_base + (GATED ? r % 128 : r), N - 1) * (uint32_t)(K * 2) + tile_gemm::piece_of(lane, r);
+  for (int j = 0; j < MoeTile::W_LOADS; ++j) {
+    const int r = (wave * MoeTile::W_LOADS + j) * 8 + lane / 8;
+    // gated: row q of group x (of two) holds feature q / 4 * 8 + x * 4 + q % 4 of the 32, so that a lane ends with 8 neighbours
+    const int q = r % 16, f = GATED ? r / 64 * 32 + q / 4 * 8 + r / 16 % 2 * 4 + q % 4 : r;
+    src.w_off[j] = (uint32_t)min(n_base + f, N - 1) * (uint32_t)(K * 2) + wide_gemm::piece_of(lane, r);
   }
-  f32x4 acc[4][8];
-  int w_row[8];
+  f32x4 acc[MoeTile::MT][MoeTile::X];
 #pragma unroll
-  for (int nt = 0; nt < 8; ++nt) {
-    // gated: groups 0..3 are gate's features wc * 64 + 16 nt, groups 4..7 the same features of up
-    w_row[nt] = GATED ? (nt / 4) * 128 + wc * 64 + 16 * (nt % 4) : wc * 128 + 16 * nt;
+  for (int mt = 0; mt < MoeTile::MT; ++mt)
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt) acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
-  tile_gemm::run(acc, big_lds, src, K / MOE_BIG_K, w_row);
-  // a lane holds features 16 nt + 4 kg .. + 3 (of its wavefront's) of the row wr * 64 + 16 mt + col
+    for (int x = 0; x < MoeTile::X; ++x) acc[mt][x] = f32x4{0.f, 0.f, 0.f, 0.f};
+  MoeTile::run(acc, big_lds, src, K / MOE_BIG_K);
+  // a lane holds rows 16 x + 4 kg .. + 3 (of its wavefront's of W in LDS) of the row wm * 64 + 16 mt + col
 #pragma unroll
-  for (int mt = 0; mt < 4; ++mt) {
-    const int r = wr * 64 + 16 * mt + col;
+  for (int mt = 0; mt < MoeTile::MT; ++mt) {
+    const int r = wm * MoeTile::PM + 16 * mt + col;
     if (r >= tile.z) continue;
     if (GATED) {
-      bf16_t* o = act_out + (int64_t)(tile.y + r) * N;
+      const int f = n_base + wn * 32 + 8 * kg;  // N is a multiple of 64: all eight or none
+      if (f < N) {
+        bf16_t eight[8];
 #pragma unroll
-      for (int nt = 0; nt < 4; ++nt) {
-        const int f = n_base + wc * 64 + 16 * nt + 4 * kg;  // N is a multiple of 64: all four or none
-        if (f < N) {
-          bf16_t four[4];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) four[i] = __float2bfloat16(act_of(acc[mt][nt][i], act_kind) * acc[mt][nt + 4][i]);
-          *reinterpret_cast<uint2*>(o + f) = *reinterpret_cast<const uint2*>(four);
-        }
+        for (int i = 0; i < 8; ++i) eight[i] = __float2bfloat16(act_of(acc[mt][i / 4][i % 4], act_kind) * acc[mt][2 + i / 4][i % 4]);
+        *reinterpret_cast<uint4*>(act_out + (int64_t)(tile.y + r) * N + f) = *reinterpret_cast<const uint4*>(eight);
       }
     } else {
       const int pair = order[tile.y + r];
       const float weight = weights[pair];
       float* o = y + ((int64_t)(pair % top) * num_tokens + pair / top) * N;
 #pragma unroll
-      for (int nt = 0; nt < 8; ++nt) {
-        const int n = n_base + wc * 128 + 16 * nt + 4 * kg;
-        if (n < N) *reinterpret_cast<f32x4*>(o + n) = weight * acc[mt][nt];
+      for (int x = 0; x < MoeTile::X; ++x) {
+        const int n = n_base + wn * MoeTile::PN + 16 * x + 4 * kg;
+        if (n < N) *reinterpret_cast<f32x4*>(o + n) = weight * acc[mt][x];
       }
     }
   }
@@ -934,13 +931,13 @@ extern "C" int pae_moe_experts_tiles(float* y, const void* x, int64_t ldx, const
     const int64_t up_grid = (int64_t)max_tiles * ((inter + 127) / 128) + 7, down_grid = (int64_t)max_tiles * ((hidden + 255) / 256) + 7;
     PAE_REQUIRE(up_grid < (1ll << 31) && down_grid < (1ll << 31), "experts: widths %d, %d exceed the grid", hidden, inter);
     for (const void* kernel : {(const void*)moe_big_tiles_kernel<true>, (const void*)moe_big_tiles_kernel<false>}) {
-      const hipError_t err = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, tile_gemm::LDS_BYTES);
-      PAE_REQUIRE(err == hipSuccess, "experts: %d bytes of LDS refused: %s", tile_gemm::LDS_BYTES, hipGetErrorString(err));
+      const hipError_t err = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, MoeTile::LDS_BYTES);
+      PAE_REQUIRE(err == hipSuccess, "experts: %d bytes of LDS refused: %s", MoeTile::LDS_BYTES, hipGetErrorString(err));
     }
-    moe_big_tiles_kernel<true><<<up_grid, 256, tile_gemm::LDS_BYTES, stream>>>((bf16_t*)act, nullptr, (const bf16_t*)x, ldx, (const bf16_t*)gate_w,
+    moe_big_tiles_kernel<true><<<up_grid, 512, MoeTile::LDS_BYTES, stream>>>((bf16_t*)act, nullptr, (const bf16_t*)x, ldx, (const bf16_t*)gate_w,
                                                             (const bf16_t*)up_w, order, weights, (const int4*)tiles, max_tiles, top,
                                                             num_tokens, hidden, inter, act_kind);
-    moe_big_tiles_kernel<false><<<down_grid, 256, tile_gemm::LDS_BYTES, stream>>>(nullptr, y, (const bf16_t*)act, inter, (const bf16_t*)down_w,
+    moe_big_tiles_kernel<false><<<down_grid, 512, MoeTile::LDS_BYTES, stream>>>(nullptr, y, (const bf16_t*)act, inter, (const bf16_t*)down_w,
                                                                nullptr, order, weights, (const int4*)tiles, max_tiles, top, num_tokens,
                                                                inter, hidden, act_kind);
   }
