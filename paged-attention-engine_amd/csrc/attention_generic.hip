@@ -133,7 +133,10 @@ __global__ void paged_attention_generic_kernel(
 // load instruction per number), and every (token, head) read the keys and values again.  Measured, 12 heads over 2
 // of 128, float32: three prompts of 601 tokens in all 262 -> 58 us, a token each behind them 92 -> 27, one prompt of 601 tokens 647 ->
 // 117, eight single tokens at 4,096 1,551 -> 338; 8 heads over 2 of 256, where six of 256 registers do not fit and lie in memory, 399 -> 77,
-// 177 -> 47, 900 -> 132, 2,534 -> 521.  What is left is the chain of a workgroup's chunks, 5 us each.  Loads
+// 177 -> 47, 900 -> 132, 2,534 -> 521.  What is left is the chain of a workgroup's chunks, 5 us each.  Where a workgroup has
+// eight rows or fewer (a token's heads, mostly) a wavefront takes one: the chain is a row's then, and registers are left to ask
+// LDS for more at once (a token at 4,096 330 -> 275 us, three at 250 25.6 -> 22.2, at heads of 64 18.6 -> 14.0; eight at 1,000, heads
+// of 256, 136 -> 114).  Loads
 // under conditions (keys beside those in sight) had the compiler wait for each in turn (twice the time for prompts), and
 // four wavefronts of four rows instead of eight of two took half as long again.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -142,7 +145,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 #define PAE_ROWS_EACH 2
 #define PAE_ROWS_MOST (PAE_ROWS_WAVES * PAE_ROWS_EACH)
 
-template <int MAXD>  // keys and values at most 64 * MAXD wide
+template <int MAXD, int EACH>  // keys and values at most 64 * MAXD wide; rows of a wavefront: one where eight rows are all there are
 __global__ __launch_bounds__(PAE_WAVE * PAE_ROWS_WAVES) void paged_attention_rows_kernel(
     float* __restrict__ out, int64_t out_stride, const float* __restrict__ q, int64_t q_stride,
     const float* __restrict__ k_cache, const float* __restrict__ v_cache, const int* __restrict__ positions,
@@ -164,14 +167,14 @@ __global__ __launch_bounds__(PAE_WAVE * PAE_ROWS_WAVES) void paged_attention_row
   const int kvh = blockIdx.y / parts, head0 = (blockIdx.y % parts) * heads_each;
   const int heads = min(heads_each, g - head0);
   const int t0 = blockIdx.x * toks;
-  p_lds += wave * PAE_ROWS_EACH * PAE_WAVE;
+  p_lds += wave * EACH * PAE_WAVE;
 
   // the wavefront's rows: row = token of the tile * heads + head
-  int tok[PAE_ROWS_EACH], head[PAE_ROWS_EACH], pos[PAE_ROWS_EACH], start[PAE_ROWS_EACH];
-  float acc[PAE_ROWS_EACH][MAXD], m[PAE_ROWS_EACH], l[PAE_ROWS_EACH];
-  bool live[PAE_ROWS_EACH];
+  int tok[EACH], head[EACH], pos[EACH], start[EACH];
+  float acc[EACH][MAXD], m[EACH], l[EACH];
+  bool live[EACH];
 #pragma unroll
-  for (int i = 0; i < PAE_ROWS_EACH; ++i) {
+  for (int i = 0; i < EACH; ++i) {
     const int row = wave + i * PAE_ROWS_WAVES;
     live[i] = row < toks * heads && t0 + row / heads < num_tokens;
     tok[i] = live[i] ? t0 + row / heads : t0;
@@ -259,29 +262,29 @@ __global__ __launch_bounds__(PAE_WAVE * PAE_ROWS_WAVES) void paged_attention_row
       }
       __syncthreads();
       if (base + PAE_WAVE <= high) fetch(base + PAE_WAVE);
-      bool on[PAE_ROWS_EACH];
+      bool on[EACH];
       bool any = false, whole = true;
 #pragma unroll
-      for (int i = 0; i < PAE_ROWS_EACH; ++i) {
+      for (int i = 0; i < EACH; ++i) {
         on[i] = live[i] && tok[i] >= at && tok[i] < next && base <= pos[i] && base + PAE_WAVE > start[i];
         any = any || on[i];
         whole = whole && (!live[i] || (on[i] && start[i] <= base && pos[i] >= base + PAE_WAVE - 1));
       }
       if (!any) continue;
       // scores: the lane's key against every row
-      float dot[PAE_ROWS_EACH];
-      int q_row[PAE_ROWS_EACH];
+      float dot[EACH];
+      int q_row[EACH];
 #pragma unroll
-      for (int i = 0; i < PAE_ROWS_EACH; ++i) {
+      for (int i = 0; i < EACH; ++i) {
         dot[i] = 0.f;
         q_row[i] = live[i] ? (wave + i * PAE_ROWS_WAVES) * hd : 0;
       }
       const float* kr = k_lds + lane * kst;
-#pragma unroll 4
+#pragma unroll(EACH == 1 && MAXD <= 2 ? 8 : 4)
       for (int d = 0; d < hd; d += 4) {
         const float4 k4 = *(const float4*)(kr + d);
 #pragma unroll
-        for (int i = 0; i < PAE_ROWS_EACH; ++i) {
+        for (int i = 0; i < EACH; ++i) {
           const float4 q4 = *(const float4*)(q_lds + q_row[i] + d);
           dot[i] = fmaf(q4.x, k4.x, dot[i]);
           dot[i] = fmaf(q4.y, k4.y, dot[i]);
@@ -290,9 +293,9 @@ __global__ __launch_bounds__(PAE_WAVE * PAE_ROWS_WAVES) void paged_attention_row
         }
       }
       const int key = base + lane;
-      float sc[PAE_ROWS_EACH], m_new[PAE_ROWS_EACH], p[PAE_ROWS_EACH], sum[PAE_ROWS_EACH];
+      float sc[EACH], m_new[EACH], p[EACH], sum[EACH];
 #pragma unroll
-      for (int i = 0; i < PAE_ROWS_EACH; ++i) {
+      for (int i = 0; i < EACH; ++i) {
         sc[i] = dot[i] * scale;
         if (slopes) sc[i] -= slopes[head[i]] * (float)(pos[i] - key);
         if (cap > 0.f) sc[i] = cap * tanhf(sc[i] / cap);
@@ -300,13 +303,13 @@ __global__ __launch_bounds__(PAE_WAVE * PAE_ROWS_WAVES) void paged_attention_row
         m_new[i] = wave_max(sc[i]);
       }
 #pragma unroll
-      for (int i = 0; i < PAE_ROWS_EACH; ++i) {  // the rows' reductions side by side; rows that are not on keep what they have
+      for (int i = 0; i < EACH; ++i) {  // the rows' reductions side by side; rows that are not on keep what they have
         m_new[i] = fmaxf(m[i], m_new[i]);
         p[i] = key >= start[i] && key <= pos[i] ? expf(sc[i] - m_new[i]) : 0.f;
         sum[i] = wave_sum(p[i]);
       }
 #pragma unroll
-      for (int i = 0; i < PAE_ROWS_EACH; ++i) {
+      for (int i = 0; i < EACH; ++i) {
         if (!on[i]) continue;
         const float alpha = expf(m[i] - m_new[i]);
         l[i] = l[i] * alpha + sum[i];
@@ -318,7 +321,7 @@ __global__ __launch_bounds__(PAE_WAVE * PAE_ROWS_WAVES) void paged_attention_row
       // sums: the lane's features over the keys in order (the wavefront's own p: no barrier, its LDS operations are in order)
       __builtin_amdgcn_wave_barrier();
       if (whole) {
-#pragma unroll 2
+#pragma unroll(EACH == 1 && MAXD <= 2 ? 4 : 2)
         for (int j = 0; j < PAE_WAVE; j += 4) {
           float v[4][MAXD];
 #pragma unroll
@@ -326,7 +329,7 @@ __global__ __launch_bounds__(PAE_WAVE * PAE_ROWS_WAVES) void paged_attention_row
 #pragma unroll
             for (int d = 0; d < MAXD; ++d) v[u][d] = v_lds[(j + u) * vst + min(lane + d * PAE_WAVE, vd - 1)];
 #pragma unroll
-          for (int i = 0; i < PAE_ROWS_EACH; ++i) {
+          for (int i = 0; i < EACH; ++i) {
             if (!live[i]) continue;
             const float4 p4 = *(const float4*)(p_lds + i * PAE_WAVE + j);
 #pragma unroll
@@ -340,7 +343,7 @@ __global__ __launch_bounds__(PAE_WAVE * PAE_ROWS_WAVES) void paged_attention_row
         }
       } else {
 #pragma unroll
-        for (int i = 0; i < PAE_ROWS_EACH; ++i) {
+        for (int i = 0; i < EACH; ++i) {
           if (!on[i]) continue;
           const int first = max(0, start[i] - base), last = min(PAE_WAVE - 1, pos[i] - base);
           auto add = [&](int j, float p) {
@@ -375,7 +378,7 @@ __global__ __launch_bounds__(PAE_WAVE * PAE_ROWS_WAVES) void paged_attention_row
     at = next;
   }
 #pragma unroll
-  for (int i = 0; i < PAE_ROWS_EACH; ++i) {
+  for (int i = 0; i < EACH; ++i) {
     if (!live[i]) continue;
     float* o = out + (int64_t)tok[i] * out_stride + (int64_t)head[i] * vd;
     float keep = 1.f;
@@ -417,16 +420,21 @@ static int launch_rows(float* out, int64_t out_stride, const float* q, int64_t q
   const int toks = (int64_t)num_tokens * nkv * parts >= 512 ? PAE_ROWS_MOST / heads_each : 1;
   const dim3 grid((num_tokens + toks - 1) / toks, nkv * parts);
   const size_t lds = (size_t)(PAE_WAVE * (hd + 4 + vd + 4) + PAE_ROWS_MOST * (PAE_WAVE + hd)) * sizeof(float);
-#define PAE_LAUNCH(MAXD)                                                                                              \
+#define PAE_LAUNCH_EACH(MAXD, EACH)                                                                                   \
   do {                                                                                                                \
     if (lds > 65536) {                                                                                                \
-      const hipError_t err = hipFuncSetAttribute((const void*)paged_attention_rows_kernel<MAXD>,                      \
+      const hipError_t err = hipFuncSetAttribute((const void*)paged_attention_rows_kernel<MAXD, EACH>,                \
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);               \
       if (err != hipSuccess) return pae_fail("attention: %zu bytes of LDS refused: %s", lds, hipGetErrorString(err)); \
     }                                                                                                                 \
-    paged_attention_rows_kernel<MAXD><<<grid, PAE_WAVE * PAE_ROWS_WAVES, lds, stream>>>(                              \
+    paged_attention_rows_kernel<MAXD, EACH><<<grid, PAE_WAVE * PAE_ROWS_WAVES, lds, stream>>>(                        \
         out, out_stride, q, q_stride, k_cache, v_cache, positions, tok_seq, block_tables, max_blocks, bs, num_tokens, \
         nh, nkv, hd, vd, scale, window, cap, sinks, chunked, slopes, gate, gate_stride, gate_per_head, toks, heads_each); \
+  } while (0)
+#define PAE_LAUNCH(MAXD)                                                     \
+  do {                                                                       \
+    if (toks * heads_each <= PAE_ROWS_WAVES) PAE_LAUNCH_EACH(MAXD, 1);       \
+    else PAE_LAUNCH_EACH(MAXD, PAE_ROWS_EACH);                               \
   } while (0)
   const int wide = hd > vd ? hd : vd;
   if (wide <= 64) PAE_LAUNCH(1);
@@ -434,6 +442,7 @@ static int launch_rows(float* out, int64_t out_stride, const float* q, int64_t q
   else if (wide <= 192) PAE_LAUNCH(3);
   else PAE_LAUNCH(4);
 #undef PAE_LAUNCH
+#undef PAE_LAUNCH_EACH
   return pae_check_launch("paged_attention_rows");
 }
 

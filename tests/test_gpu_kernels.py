@@ -969,3 +969,10 @@ def test_float32_attention_kernels_give_the_same_bits(nh, nkv, hd, vd, bs, windo
             outs.append(out)
         assert bool(torch.isfinite(outs[1]).all())
         assert torch.equal(outs[0], outs[1]), runs
+
+
+@pytest.mark.parametrize("nh,nkv,hd", [(8, 1, 64), (9, 1, 64), (16, 2, 192)])
+def test_float32_attention_of_eight_rows_a_workgroup_and_of_nine(nh, nkv, hd):
+    """Up to eight rows a wavefront of the kernel that shares a chunk takes one, from nine on two."""
+    test_float32_attention_kernels_give_the_same_bits(nh, nkv, hd, hd, 16, 0, False, 0.0, False)
+
