@@ -200,9 +200,12 @@ struct Tile {
 //     (1, 0)                    A half 1             A half 0 of t + 2
 //     (1, 1)                    W half 0 of t + 1    W half 1 of t + 2
 //
-// A half of the stage's rows is written again only two barriers or more behind the last products that wait for its reads, in both
-// halves of the wavefronts (the second runs one barrier behind the first); what a quarter reads has arrived because every
-// wavefront waited for its own loads of it before a barrier that lies in between.
+// A half of the stage's rows is written again only behind a barrier that all reads of it were answered before, in both halves of the
+// wavefronts (the second runs one barrier behind the first).  The first quarter's products wait for the reads of A half 0, the second's
+// for W half 1 and the third's for A half 1, each two barriers or more before the loads that write there.  W half 0 is read a quarter
+// early, and the second half's first products come in the very interval in which the first half's loads overwrite it: the reads
+// before the first quarter wait for it, which costs nothing (its four are older than A's eight, and LDS answers in order).
+// What a quarter reads has arrived because every wavefront waited for its own loads of it before a barrier that lies in between.
 struct Large {
   static constexpr int BM = 256, BN = 256, WM = 2, WN = 4, WAVES = 8, PM = 128, PN = 64, MT = 8, X = 4;
   static constexpr int HALF = 128 * ROW_BYTES, STAGE_BYTES = 4 * HALF, LDS_BYTES = 2 * STAGE_BYTES;
@@ -284,6 +287,7 @@ struct Large {
       constexpr int ONE = one_.value, TWO = two_.value;
       const uint32_t other = at ^ STAGE_BYTES;
       read_a(0, at);
+      asm volatile("s_waitcnt lgkmcnt(8)" ::: "memory");  // W half 0, whose rows the other half's next loads write: all but A's eight reads
       if (ONE) {
         load_a(1, other);
         forward();
@@ -314,6 +318,8 @@ struct Large {
       meet();
     };
     read_w(0, 0);
+    asm volatile("" ::: "memory");  // before the reads of A half 0, as that wait counts them
+    __builtin_amdgcn_sched_barrier(0);
     uint32_t at = 0;
     for (int left = stages; left > 2; --left) {
       stage(Number<1>(), Number<1>(), at);
