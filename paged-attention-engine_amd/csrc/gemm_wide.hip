@@ -256,18 +256,21 @@ enum { SHAPE_LARGE, SHAPE_128_256, SHAPE_128_128, SHAPE_128_96, SHAPE_64_128, SH
 
 // Microseconds of a product in a shape, from times of all shapes at 14 sizes of weights (896 to 18,944 of k) by 24 row counts
 // from 72 to 8,192, which this meets within 11 to 13 % (root mean square): a round of tiles costs its start and end and so much a
-// stage.  The least of them is on average 1 % behind the fastest shape.
+// stage.  The shapes of two workgroups a unit take a quarter longer a stage from 2,048 of k on, with weights from memory (64 x 64 at up
+// to one a unit: 0.16 to 0.20 up to k 1,536, 0.24 to 0.26 from 2,048 to 18,944; 64 x 128 0.32 and 0.40 to 0.43).  The least of all is on
+// average 1 % behind the fastest shape (300 x 4,608 x 3,584 24.8 us; without that quarter 64 x 128 was taken, 28.1).
 double shape_time(int shape, int M, int N, int K, int splits) {
   const double stages = K / 64.0 / splits;
   struct Cost { int bm, bn, blocks; double launch, round, stage, part; };  // part: a stage of a last round that half the units' places or fewer take
   static const Cost cost[SHAPES] = {{256, 256, 1, 0.0, 3.5, 1.35, 0.0},  {128, 256, 1, 0.0, 2.9, 0.73, 0.73}, {128, 128, 1, 0.0, 2.4, 0.46, 0.46},
                                     {128, 96, 1, 0.3, 2.4, 0.39, 0.39}, {64, 128, 2, 2.5, 0.0, 0.62, 0.33},  {64, 64, 2, 2.9, 0.0, 0.38, 0.21}};
   const Cost& c = cost[shape];
+  const double far = c.blocks == 2 && K >= 2048 * splits ? 1.25 : 1.0;
   const int64_t tiles = tiles_of(M, N, c.bm, c.bn) * splits, places = (int64_t)UNITS * c.blocks;
   const int64_t rest = tiles % places;
   double last = 0.0;
-  if (rest) last = c.round + stages * (shape == SHAPE_LARGE ? (rest > UNITS / 2 ? c.stage : rest > UNITS / 4 ? 0.77 : 0.40) : rest > places / 2 ? c.stage : c.part);
-  return c.launch + tiles / places * (c.round + stages * c.stage) + last;
+  if (rest) last = c.round + stages * (shape == SHAPE_LARGE ? (rest > UNITS / 2 ? c.stage : rest > UNITS / 4 ? 0.77 : 0.40) : far * (rest > places / 2 ? c.stage : c.part));
+  return c.launch + tiles / places * (c.round + stages * far * c.stage) + last;
 }
 
 template <int MODE, int ACT>
@@ -292,9 +295,13 @@ int run_shape(int shape, const Product& p, hipStream_t stream) {
 
 // The shape for a product, in the low byte, and its ranges of k behind that.  `mode` as for pae_gemm_wide; `ranges` != 0: the
 // product may leave float32 sums of ranges of k for a caller that reads them again (counted at 4.5 TB/s against one bfloat16
-// result).  -1: the platform library, for a product without an activation that no shape here fills the chip with: from
-// 30 us on and below 0.95 PFLOP/s by the times above the library, which shares such products out over k, was ahead of
-// these shapes two times in three (6,030 x 1,536 x 8,960 141 against 160 us, 2,048 x 4,608 x 3,584 59 against 68).
+// result).  -1: the platform library, which shares a product out over k, for one without an activation that no shape here fills
+// the chip with.  That is from 30 us on and below 0.95 PFLOP/s by the times above, where the library was ahead of
+// these shapes two times in three (6,030 x 1,536 x 8,960 141 against 160 us, 2,048 x 4,608 x 3,584 59 against 68); and from 48 stages of k
+// on where even tiles of 64 x 64 leave half the units idle, whose one chain of stages is then longer than the library's shares: up
+// to 64 tiles 0.84 to 1.83 times its time, 1.30 on average, and up to 128 0.85 to 1.26, 1.04 on average (128 x 896 x 4,864 23.9 against 13.1
+// us, 300 x 256 x 4,096 18.6 against 11.2, 65 x 16 x 8,192 22.4 against 8.3).  Up to 35 stages as few tiles are ahead (65 x 1,536 x 2,240 8.8
+// against 11.4), and so are 128 to 256 of them (0.84 on average).
 extern "C" int pae_gemm_wide_plan(int mode, int act, int M, int N, int K, int ranges) {
   static const int CUTS[] = {2, 3, 4, 6, 8};
   int best = SHAPE_LARGE, cuts = 1;
@@ -310,7 +317,9 @@ extern "C" int pae_gemm_wide_plan(int mode, int act, int M, int N, int K, int ra
       const double t = shape_time(shape, M, N, K, n) + (4.0 * n - 2.0) * M * N / 4.5e6;
       if (t < least) least = t, best = shape, cuts = n;
     }
-  if (mode == wide_gemm::PLAIN && act == NO_ACT && least > 30.0 && 2.0 * M * N * K / least < 0.95e9) return -1;
+  if (mode == wide_gemm::PLAIN && act == NO_ACT &&
+      ((least > 30.0 && 2.0 * M * N * K / least < 0.95e9) || (K >= 48 * 64 && tiles_of(M, N, 64, 64) <= UNITS / 2)))
+    return -1;
   return best | cuts << 8;
 }
 

@@ -53,3 +53,18 @@ def test_large_tiles_of_experts_are_counted_in_fifteen_bits():
 def test_a_product_of_no_rows_is_done_whatever_its_types():
     for pair in ((0, 0), (1, 1), (1, 0), (0, 1)):
         assert K.library().pae_gemm_plain_shared(*pair, None, 8, 0, None, 8, 0, None, 0, None, 0, 0, 8, 8, 1, None, None) == 0
+
+
+@pytest.mark.parametrize("M,N,K_", [(65, 896, 4864), (513, 896, 4864), (300, 256, 4096), (2048, 256, 4096), (65, 16, 8192), (4096, 64, 4096)])
+def test_products_of_few_tiles_and_much_of_k_go_to_the_library(M, N, K_):
+    """One chain of stages a tile takes longer there than the library's shares of k (1.2 to 2.7 times, with half the units idle or more); an
+    activation, or sums of ranges of k for a caller that adds them, are still made here, and so is what has less of k or more tiles."""
+    plan = K.library().pae_gemm_wide_plan
+    assert plan(K.WIDE_PLAIN, -1, M, N, K_, 0) == -1
+    assert plan(K.WIDE_PLAIN, 0, M, N, K_, 0) >= 0 and plan(K.WIDE_SUMS, -1, M, N, K_, 1) >> 8 >= 1
+    assert plan(K.WIDE_PLAIN, -1, M, N, 2240, 0) >= 0 and plan(K.WIDE_PLAIN, -1, 150, 4608, 3584, 0) >= 0
+
+
+def test_the_shape_of_a_product_between_one_and_two_small_tiles_a_unit():
+    """Rows of 2,048 numbers and more come slower to two workgroups a unit: 128 x 96 is ahead of 64 x 128 there (24.8 against 28.1 us)."""
+    assert K.library().pae_gemm_wide_plan(K.WIDE_PLAIN, -1, 300, 4608, 3584, 0) == 3 | 1 << 8
