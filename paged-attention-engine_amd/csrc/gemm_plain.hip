@@ -6,7 +6,8 @@
 //
 // Products run on the bfloat16 matrix cores (v_mfma_f32_16x16x32_bf16).  A float32 number is the sum of three bfloat16 numbers that hold
 // its 24 bits, and of the nine products of two numbers' parts the six that reach a float32 product's last bit are
-// added in float32; the three left out are below 2^-25 of the product.  bfloat16 numbers are one part and take one product.  The
+// added in float32; the three left out are below 2^-24 of the product, half a unit of its last place, of either sign (root mean square of
+// normal operands 2^-27.4).  bfloat16 numbers are one part and take one product.  The
 // float32 instructions (v_mfma_f32_16x16x4_f32), which these replace, add up four products at a time and give 154 TFLOP/s on the
 // whole chip; six of the others do the work at up to 230.  A slab's products are a sum of their own before they join the others'.  Error
 // against 64 bits (root mean square, share of the result's; normal operands): k 1,536 4.1e-7 before, 1.0e-7 now; 8,960 4.1e-7 and
@@ -150,9 +151,10 @@ __device__ __forceinline__ void cut(Eight<bf16_t>& e, int k, int q, int end) {
   }
 }
 
-// The eight as sums of bfloat16 numbers, largest part first: three of them hold a float32's 24 bits.  The first is the nearest
-// (so that the products left out below have either sign), the second what its first eight bits are of the rest, and the
-// differences are exact.  Additions and masks and not v_cvt_pk_bf16_f32 and v_dot2c_f32_bf16, which do it in half the
+// The eight as sums of bfloat16 numbers, largest part first: three of them hold a float32's 24 bits.  The first two are the
+// nearest, so that the products left out (of a second and a third part, and of two third parts) have either sign and are
+// below 2^-24 of the product; with the second part cut off instead they have the product's sign where a row meets itself, and reach
+// 2^-23.  The differences are exact.  Additions and masks and not v_cvt_pk_bf16_f32 and v_dot2c_f32_bf16, which do it in half the
 // instructions: beside a matrix instruction of 17 clocks two of the former are free, but one of the latter makes it 35.
 template <typename T>
 struct Parts {
@@ -166,10 +168,11 @@ __device__ __forceinline__ void half_parts_of(Parts<float>& o, const Eight<float
   for (int i = 0; i < 2; ++i) {
     const float a = e.v[h][2 * i], b = e.v[h][2 * i + 1];
     const uint32_t a0 = __float_as_uint(a) + 0x8000u, b0 = __float_as_uint(b) + 0x8000u;
-    const float a1 = a - __uint_as_float(a0 & 0xffff0000u), b1 = b - __uint_as_float(b0 & 0xffff0000u);
-    const float a2 = a1 - __uint_as_float(__float_as_uint(a1) & 0xffff0000u), b2 = b1 - __uint_as_float(__float_as_uint(b1) & 0xffff0000u);
+    const float ra = a - __uint_as_float(a0 & 0xffff0000u), rb = b - __uint_as_float(b0 & 0xffff0000u);
+    const uint32_t a1 = __float_as_uint(ra) + 0x8000u, b1 = __float_as_uint(rb) + 0x8000u;
+    const float a2 = ra - __uint_as_float(a1 & 0xffff0000u), b2 = rb - __uint_as_float(b1 & 0xffff0000u);
     o.p[0][2 * h + i] = upper_halves(a0, b0);
-    o.p[1][2 * h + i] = upper_halves(__float_as_uint(a1), __float_as_uint(b1));
+    o.p[1][2 * h + i] = upper_halves(a1, b1);
     o.p[2][2 * h + i] = upper_halves(__float_as_uint(a2), __float_as_uint(b2));
   }
 }

@@ -147,6 +147,59 @@ def test_gemm_plain_keeps_what_is_not_finite(M, N, K_):
         assert torch.equal(out[clean], plain[clean])
 
 
+def rounded_sums(K_):
+    """A bound of a float32 product's error against 64 bits, root mean square, as a share of the result's, for operands of either sign: a slab
+    of 32 of k is six instructions and the sum that it joins, seven roundings of partial sums, each evenly spread within half a
+    unit (2^-24 / sqrt(3)) of the sum so far, whose square grows with the slabs; and what six of nine products of parts leave out, 2^-27."""
+    slabs = -(-K_ // 32)
+    return 2.0 ** -24 * (7 * (slabs + 1) / 6) ** 0.5 + 2.0 ** -27
+
+
+# few rows (16, 32 and 64), small tiles and large ones, k shared or not, rows read by fours or one by one
+SIX_SIZES = [(3, 40, 32), (16, 100, 64), (3, 200, 512), (16, 900, 896), (30, 70, 1536), (40, 70, 1537), (70, 200, 64), (129, 90, 33),
+             (65, 1536, 1536), (65, 17920, 1536), (1100, 17920, 512)]
+
+
+@pytest.mark.parametrize("M,N,K_", SIX_SIZES)
+def test_gemm_plain_keeps_24_bits(M, N, K_):
+    """float32 products are of parts of 8 bits: sums without one of the six that count are 1.5 times this bound off or more."""
+    torch.manual_seed(M + N + K_)
+    a, w = torch.randn(M, K_, device=DEV), torch.randn(N, K_, device=DEV)
+    out = torch.empty(M, N, device=DEV)
+    K().gemm_plain(out, a, w)
+    want = a.double() @ w.double().t()
+    assert float((out.double() - want).norm() / want.norm()) <= rounded_sums(K_)
+
+
+@pytest.mark.parametrize("M,N,K_", SIX_SIZES)
+def test_gemm_plain_of_single_products(M, N, K_):
+    """Rows with one number: what is left out of a product is below 2^-24 of it; the last instruction is within a unit (2^-23) of what it
+    adds, and the four before it add up what has at most 2^-6 of the product's size."""
+    torch.manual_seed(M + N + K_)
+    a, w = torch.zeros(M, K_, device=DEV), torch.zeros(N, K_, device=DEV)
+    at = K_ // 2
+    a[:, at], w[:, at] = torch.randn(M, device=DEV), torch.randn(N, device=DEV)
+    hard = torch.tensor([1 + 2.0 ** -8 - 2.0 ** -23, 1 + 2.0 ** -8 - 2.0 ** -17, 1 + 2.0 ** -8 - 2.0 ** -16 - 2.0 ** -17], device=DEV)
+    a[:3, at], w[:3, at] = hard, hard
+    out = torch.empty(M, N, device=DEV)
+    K().gemm_plain(out, a, w)
+    want = a[:, at:at + 1].double() * w[:, at].double()
+    off = (out.double() - want) / want
+    assert float(off.abs().max()) <= (1 + 2 + 4 * 2 * 2.0 ** -6) * 2.0 ** -24
+
+
+@pytest.mark.parametrize("K_", [32, 64, 512])
+def test_gemm_plain_of_rows_by_themselves_leans_to_neither_side(K_):
+    """What is left out of a row's product with itself has either sign (its mean is below 2^-30); a part cut off and not rounded would lean by
+    2^-25 and more.  Half of that is allowed (the mean of 2,000 rows is 1e-9 off by chance)."""
+    torch.manual_seed(K_)
+    a = torch.randn(2000, K_, device=DEV)
+    out = torch.empty(2000, 2000, device=DEV)
+    K().gemm_plain(out, a, a)
+    want = a.double().pow(2).sum(1)
+    assert abs(float(((out.diagonal().double() - want) / want).mean())) <= 2.0 ** -26
+
+
 @pytest.mark.parametrize("M,N,K_", [(300, 2100, 30000), (2100, 300, 30000)])
 def test_gemm_plain_in_parts_gives_the_bits_of_the_whole(M, N, K_):
     """Products whose blocks' sums do not fit the scratch memory at once are made in parts, along the columns or along the rows:
