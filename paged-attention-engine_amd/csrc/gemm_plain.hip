@@ -12,7 +12,6 @@
 // whole chip; six of the others do the work at up to 230.  A slab's products are a sum of their own before they join the others'.  Error
 // against 64 bits (root mean square, share of the result's; normal operands): k 1,536 4.1e-7 before, 1.0e-7 now; 8,960 4.1e-7 and
 // 1.6e-7; 18,944 4.2e-7 and 2.1e-7; bfloat16 operands 1.7e-7 and 0.9e-7.
-// (A number below 2^-110 loses what its parts have below 2^-133, the smallest bfloat16.)
 //
 // k is cut into slabs of 32, one set of instructions each, and into blocks of 512 whose sums are then added up in
 // order (with rows of 30,000 terms one running sum loses a digit more than the block sums do).  Every kernel here adds in this
@@ -43,6 +42,7 @@
 
 #define GP_BLOCK 512  // k of a block whose sum is formed before it joins the total
 #define GP_SLAB 32    // k of one instruction
+#define GP_UP 65536.f  // float32 operands are taken times this, and sums of products divided by its square
 #define GP_FEW_ROWS 32  // (64 where rows are read number by number)
 #define GP_FEW_WAVES 8
 #define GP_TILE 64    // parts of a product are cut in multiples of it
@@ -75,39 +75,8 @@ __device__ __forceinline__ void load8(Eight<bf16_t>& e, const bf16_t* row, int k
   e.v[0] = *(const uint2*)(row + k + q * 4);
   e.v[1] = *(const uint2*)(row + k + 16 + q * 4);
 }
-// The same with zeros from `end` on; four numbers at a time (FOURS: `end` is a multiple of four) or one.
-template <bool FOURS>
-__device__ __forceinline__ void load8_to(Eight<float>& e, const float* row, int k, int q, int end) {
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int at = k + 16 * h + q * 4;
-    if (FOURS) {
-      e.v[h] = f32x4{0.f, 0.f, 0.f, 0.f};
-      if (at < end) e.v[h] = *(const f32x4*)(row + at);
-    } else {
-#pragma unroll
-      for (int u = 0; u < 4; ++u) e.v[h][u] = at + u < end ? row[at + u] : 0.f;
-    }
-  }
-}
-template <bool FOURS>
-__device__ __forceinline__ void load8_to(Eight<bf16_t>& e, const bf16_t* row, int k, int q, int end) {
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int at = k + 16 * h + q * 4;
-    if (FOURS) {
-      e.v[h] = uint2{0u, 0u};
-      if (at < end) e.v[h] = *(const uint2*)(row + at);
-    } else {
-      uint32_t w[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) w[u] = at + u < end ? ((const uint16_t*)row)[at + u] : 0u;
-      e.v[h] = uint2{w[0] | w[1] << 16, w[2] | w[3] << 16};
-    }
-  }
-}
-
-// The same without a condition around a load (one makes the compiler wait for every load on its way): what lies from `end` on is
+// The same of a row that ends at `end`, four numbers at a time (FOURS: `end` is a multiple of four) or one, without a condition around
+// a load (one makes the compiler wait for every load on its way): what lies from `end` on is
 // read elsewhere in the row, and `cut` makes it zero when it is there.
 template <bool FOURS>
 __device__ __forceinline__ void load8_anyhow(Eight<float>& e, const float* row, int k, int q, int end) {
@@ -151,7 +120,9 @@ __device__ __forceinline__ void cut(Eight<bf16_t>& e, int k, int q, int end) {
   }
 }
 
-// The eight as sums of bfloat16 numbers, largest part first: three of them hold a float32's 24 bits.  The first two are the
+// The eight, times 2^16, as sums of bfloat16 numbers, largest part first: three of them hold a float32's 24 bits.  Times 2^16 the
+// smallest float32 is 2^-133, as is the smallest bfloat16, so that no number is too small for its parts (as they are, numbers below 2^-110 would
+// lose digits); sums of products are divided by 2^32 at the end.  The first two are the
 // nearest, so that the products left out (of a second and a third part, and of two third parts) have either sign and are
 // below 2^-24 of the product; with the second part cut off instead they have the product's sign where a row meets itself, and reach
 // 2^-23.  The differences are exact.  Additions and masks and not v_cvt_pk_bf16_f32 and v_dot2c_f32_bf16, which do it in half the
@@ -166,7 +137,7 @@ __device__ __forceinline__ uint32_t upper_halves(uint32_t a, uint32_t b) { retur
 __device__ __forceinline__ void half_parts_of(Parts<float>& o, const Eight<float>& e, int h) {
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
-    const float a = e.v[h][2 * i], b = e.v[h][2 * i + 1];
+    const float a = e.v[h][2 * i] * GP_UP, b = e.v[h][2 * i + 1] * GP_UP;
     const uint32_t a0 = __float_as_uint(a) + 0x8000u, b0 = __float_as_uint(b) + 0x8000u;
     const float ra = a - __uint_as_float(a0 & 0xffff0000u), rb = b - __uint_as_float(b0 & 0xffff0000u);
     const uint32_t a1 = __float_as_uint(ra) + 0x8000u, b1 = __float_as_uint(rb) + 0x8000u;
@@ -201,8 +172,12 @@ __device__ __forceinline__ f32x4 slab(const Parts<float>& a, const Parts<float>&
 }
 __device__ __forceinline__ f32x4 slab(const Parts<bf16_t>& a, const Parts<bf16_t>& w) { return mfma(a.p[0], w.p[0], f32x4{0.f, 0.f, 0.f, 0.f}); }
 
+// A sum of products of numbers times GP_UP, of the numbers themselves.
+template <typename T>
+__device__ __forceinline__ float sized(float v) { return sizeof(T) == 4 ? v * (1.f / GP_UP / GP_UP) : v; }
+
 // A result that is not finite is formed again from the numbers themselves: an infinity has no parts (its remainder is no
-// number), nor have the last few numbers below the largest, whose nearest first part is infinite.  A number by itself, as
+// number), nor have numbers from 2^112 on, and sums from 2^96 on are infinite times 2^32.  A number by itself, as
 // it should never be needed; the blocks' sums are added as ever.
 __device__ __forceinline__ bool is_finite(float v) { return fabsf(v) <= 3.402823466e38f; }
 __device__ __attribute__((noinline)) float formed_again(const float* a, const float* w, int K) {
@@ -303,11 +278,13 @@ __global__ __launch_bounds__(64 * GP_FEW_WAVES) void gemm_plain_few_kernel(
       for (; k < end; k += GP_SLAB) {
         Eight<TA> raw;
         Parts<TA> w, a;
-        load8_to<VEC>(raw, w_row, k, kq, end);
+        load8_anyhow<VEC>(raw, w_row, k, kq, K);
+        cut(raw, k, kq, K);
         parts_of(w, raw);
 #pragma unroll
         for (int i = 0; i < MT; ++i) {
-          load8_to<VEC>(raw, a_row[i], k, kq, end);
+          load8_anyhow<VEC>(raw, a_row[i], k, kq, K);
+          cut(raw, k, kq, K);
           parts_of(a, raw);
           acc[i] += slab(a, w);
         }
@@ -345,7 +322,7 @@ __global__ __launch_bounds__(64 * GP_FEW_WAVES) void gemm_plain_few_kernel(
   for (int i = 0; i < TOTALS; ++i) {
     const int o = threadIdx.x + i * blockDim.x, m = o / 16, n = n0 + o % 16;
     if (o < MT * 256 && m < M && n < N) {
-      float v = total[i];
+      float v = sized<TA>(total[i]);
       if constexpr (Parts<TA>::P > 1) {
         if (!is_finite(v)) v = formed_again(A + m * lda, W + (int64_t)n * K, K);
       }
@@ -497,7 +474,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_plain_tiles_kernel(
       for (int e = 0; e < 4; ++e) {
         const int m = m0 + i * 16 + kq * 4 + e;
         if (m >= M) continue;
-        float v = total[SHARED ? 0 : i][j][e];
+        float v = sized<TA>(total[SHARED ? 0 : i][j][e]);
         whole = whole && is_finite(v);
         if (bias) v += b;
         C[(int64_t)m * ldc + n] = from_f32<TC>(v);
@@ -538,6 +515,7 @@ __global__ __launch_bounds__(256) void gemm_plain_sum_kernel(TC* __restrict__ C,
     for (int u = 0; u < 8; ++u) total += v[u];
   }
   for (; b < blocks; ++b) total += p[b * stride];
+  total = sized<TA>(total);
   if constexpr (Parts<TA>::P > 1) {
     if (!is_finite(total)) total = formed_again(A + m * lda, W + (int64_t)n * K, K);
   }

@@ -6,16 +6,18 @@ import torch
 from tests.test_gpu_kernels import rounded_sums
 
 UPPER = -65536  # the bits of a float32's first half
+UP = 65536.0
 
 
 def parts_of(x):
-    """The parts in float64."""
+    """The parts in float64, of the number itself; the kernels hold them times 2^16."""
     bits, number = lambda t: t.contiguous().view(torch.int32), lambda t: t.view(torch.float32)
+    x = x * UP
     first = number((bits(x) + 0x8000) & UPPER)
     second = number((bits(x - first) + 0x8000) & UPPER)
     third = x - first - second
     assert torch.equal(number(bits(third) & UPPER), third)
-    return [t.double() for t in (first, second, third)]
+    return [t.double() / UP for t in (first, second, third)]
 
 
 SIX = [(0, 0), (0, 1), (1, 0), (1, 1), (0, 2), (2, 0)]
@@ -30,8 +32,8 @@ def off(a, w, kept):
 def test_numbers_are_their_parts():
     gen = torch.Generator().manual_seed(1)
     x = torch.randn(100000, generator=gen)
-    for scale in (0, 100, -60):
-        y = x * 2.0 ** scale
+    for scale in (0, 100, -60, -110, -126, -140, -149):
+        y = x * 2.0 ** scale if scale > -126 else x * 2.0 ** -100 * 2.0 ** (scale + 100)
         assert torch.equal(sum(parts_of(y)), y.double()), scale
 
 

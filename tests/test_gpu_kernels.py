@@ -200,6 +200,20 @@ def test_gemm_plain_of_rows_by_themselves_leans_to_neither_side(K_):
     assert abs(float(((out.diagonal().double() - want) / want).mean())) <= 2.0 ** -26
 
 
+@pytest.mark.parametrize("M,N,K_", SIX_SIZES)
+@pytest.mark.parametrize("scale", [-100, -112, -120, -126, -140])
+def test_gemm_plain_of_small_numbers(M, N, K_, scale):
+    """Numbers have their 24 bits down to the smallest float32 on both sides of a product (below 2^-126 as many as they have left)."""
+    torch.manual_seed(M + N + K_)
+    a, w = torch.randn(M, K_, device=DEV) * 2.0 ** -90 * 2.0 ** (scale + 90), torch.randn(N, K_, device=DEV) * 2.0 ** 60
+    out, other = torch.empty(M, N, device=DEV), torch.empty(N, M, device=DEV)
+    K().gemm_plain(out, a, w)
+    want = a.double() @ w.double().t()
+    assert float((out.double() - want).norm() / want.norm()) <= rounded_sums(K_)
+    K().gemm_plain(other, w, a)
+    assert float((other.double().t() - want).norm() / want.norm()) <= rounded_sums(K_)
+
+
 @pytest.mark.parametrize("M,N,K_", [(300, 2100, 30000), (2100, 300, 30000)])
 def test_gemm_plain_in_parts_gives_the_bits_of_the_whole(M, N, K_):
     """Products whose blocks' sums do not fit the scratch memory at once are made in parts, along the columns or along the rows:
