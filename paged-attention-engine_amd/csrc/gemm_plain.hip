@@ -621,7 +621,7 @@ static int launch_plain(void* C, int64_t ldc, int64_t batch_c, const void* A, in
   gemm_plain_few_kernel<TA, TC, MT, VEC><<<grid, waves * PAE_WAVE, scratch ? 0 : waves * MT * 1024, stream>>>(GP_ARGS)
     if (M <= 16) GP_FEW(1);
     else if (VEC || M <= 32) GP_FEW(2);
-    else GP_FEW(VEC ? 2 : 4);
+    else if constexpr (!VEC) GP_FEW(4);
 #undef GP_FEW
   } else {
     const GpShape shape = shape_of(M, N, K);
