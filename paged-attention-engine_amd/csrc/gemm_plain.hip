@@ -45,6 +45,8 @@
 #define GP_UP 65536.f  // float32 operands are taken times this, and sums of products divided by its square
 #define GP_FEW_ROWS 32  // (64 where rows are read number by number)
 #define GP_FEW_WAVES 8
+#define GP_FEW_MOST 12  // wavefronts of up to 16 rows, where blocks of k are spread
+#define GP_STAGED_ROWS 8
 #define GP_TILE 64    // parts of a product are cut in multiples of it
 #define GP_UNITS 256  // compute units
 #define GP_LARGE_WHOLE 160  // large tiles from which on none is shared
@@ -192,22 +194,30 @@ __device__ __attribute__((noinline)) float formed_again(const float* a, const fl
 }
 
 // Up to 16 * MT rows: blockIdx.x 16 weight rows, blockIdx.y the product of the batch, blockIdx.z a share of
-// the blocks of k, one block a wavefront at a time.  VEC: rows may be read four numbers at a time.
-template <typename TA, typename TC, int MT, bool VEC>
-__global__ __launch_bounds__(64 * GP_FEW_WAVES) void gemm_plain_few_kernel(
+// the blocks of k.  VEC: rows may be read four numbers at a time.  A block of k is one wavefront's; SPREAD: of
+// `parts` wavefronts, an equal range of its slabs each, whose sums meet in LDS one by one and are added in the order of k, the order
+// of a running sum.  STAGED: the rows' parts are made once for all wavefronts and lie in LDS.
+#define GP_SLABS (GP_BLOCK / GP_SLAB)
+__host__ __device__ constexpr int few_slots(bool spread) { return spread ? GP_SLABS : 1; }  // sums of a block in LDS
+template <typename TA, typename TC, int MT, bool VEC, bool SPREAD, bool STAGED>
+__global__ __launch_bounds__(64 * (SPREAD && MT <= 2 ? GP_FEW_MOST : GP_FEW_WAVES), 2) void gemm_plain_few_kernel(
     TC* __restrict__ C, int64_t ldc, const TA* __restrict__ A, int64_t lda, const TA* __restrict__ W,
     const void* __restrict__ bias, int b_is_f32, int M, int N, int K, int64_t batch_c, int64_t batch_a,
-    int64_t batch_w, float* __restrict__ scratch) {
+    int64_t batch_w, float* __restrict__ scratch, int parts) {
   C += blockIdx.y * batch_c;
   A += blockIdx.y * batch_a;
   W += blockIdx.y * batch_w;
-  extern __shared__ float part[];  // [wavefront][16 * MT][16]
-  const int waves = blockDim.x / PAE_WAVE;
+  extern __shared__ f32x4 sums_lds[];  // [block][slot][MT][lane]; STAGED: behind it u32x4 [block][slab][part][row][eight]
+  constexpr int SLOTS = few_slots(SPREAD), P = Parts<TA>::P;
+  if (!SPREAD) parts = 1;
+  const int waves = blockDim.x / PAE_WAVE, here = waves / parts;  // blocks side by side
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PAE_WAVE);
+  const int place = wave / parts, part_slabs = GP_SLABS / parts, slab0 = (wave - place * parts) * part_slabs;
   const int lane = threadIdx.x % PAE_WAVE, r = lane % 16, kq = lane / 16;
   const int n0 = blockIdx.x * 16;
   const int blocks = (K + GP_BLOCK - 1) / GP_BLOCK;
-  const int step = waves * gridDim.z;
+  const int step = here * gridDim.z;
+  u32x4* a_lds = (u32x4*)(sums_lds + here * SLOTS * MT * PAE_WAVE);
   // rows past the end are read as the last one and dropped
   const TA* w_row = W + (int64_t)min(n0 + r, N - 1) * K;
   const TA* a_row[MT];
@@ -220,102 +230,155 @@ __global__ __launch_bounds__(64 * GP_FEW_WAVES) void gemm_plain_few_kernel(
   for (int i = 0; i < TOTALS; ++i) total[i] = 0.f;
 
   for (int first = 0; first < blocks; first += step) {  // the same trips for every wavefront
-    const int block = first + blockIdx.z * waves + wave;
+    const int round = first + blockIdx.z * here, block = round + place;
+    int k = 0, end = 0;
+    if (block < blocks) {
+      k = block * GP_BLOCK + slab0 * GP_SLAB;
+      end = min(K, k + part_slabs * GP_SLAB);
+    }
+    struct Batch {
+      Eight<TA> w[U], a[U][STAGED ? 1 : MT];
+    } b0, b1;
+    constexpr int STEP = GP_SLAB * U;
+    int batches = VEC ? max(0, end - k) / STEP : 0;
+    auto fetch = [&](Batch& b, int at) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        load8(b.w[u], w_row, at + u * GP_SLAB, kq);
+        if constexpr (!STAGED) {
+#pragma unroll
+          for (int i = 0; i < MT; ++i) load8(b.a[u][i], a_row[i], at + u * GP_SLAB, kq);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    if (batches > 0) fetch(b0, k);
+    if constexpr (STAGED) {
+      const int k0 = round * GP_BLOCK, slabs = (min(K, k0 + here * GP_BLOCK) - k0 + GP_SLAB - 1) / GP_SLAB;
+      for (int e = threadIdx.x; e < M * slabs * 4; e += blockDim.x) {
+        const int row = e / (slabs * 4), slab = e / 4 - row * slabs, q = e % 4;
+        Eight<TA> raw;
+        load8_anyhow<VEC>(raw, A + (int64_t)row * lda, k0 + slab * GP_SLAB, q, K);
+        cut(raw, k0 + slab * GP_SLAB, q, K);
+        Parts<TA> made;
+        parts_of(made, raw);
+#pragma unroll
+        for (int p = 0; p < P; ++p) a_lds[((slab * P + p) * M + row) * 4 + q] = made.p[p];
+      }
+      __syncthreads();
+    }
     f32x4 acc[MT];
 #pragma unroll
     for (int i = 0; i < MT; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (block < blocks) {
-      int k = block * GP_BLOCK;
-      const int end = min(K, k + GP_BLOCK);
-      const int steady = VEC ? (end - k) / (GP_SLAB * U) : 0;
-      if (steady) {
-        // two batches take turns; no load stands under a condition of its own
-        struct Batch {
-          Eight<TA> w[U], a[U][MT];
-        } b0, b1;
-        auto fetch = [&](Batch& b, int at) {
+    f32x4* to = sums_lds + (place * SLOTS + slab0) * (MT * PAE_WAVE) + lane;
+    const u32x4* staged = a_lds + (place * GP_SLABS + slab0) * (P * 4 * M) + min(r, M - 1) * 4 + kq;
+    auto join = [&](const Parts<TA>& w, const Eight<TA>* a) {
 #pragma unroll
-          for (int u = 0; u < U; ++u) {
-            load8(b.w[u], w_row, at + u * GP_SLAB, kq);
+      for (int i = 0; i < MT; ++i) {
+        Parts<TA> made;
+        if constexpr (STAGED) {
 #pragma unroll
-            for (int i = 0; i < MT; ++i) load8(b.a[u][i], a_row[i], at + u * GP_SLAB, kq);
-          }
-          __builtin_amdgcn_sched_barrier(0);
-        };
-        auto multiply = [&](const Batch& b) {
-#pragma unroll
-          for (int u = 0; u < U; ++u) {
-            Parts<TA> w, a;
-            parts_of(w, b.w[u]);
-#pragma unroll
-            for (int i = 0; i < MT; ++i) {
-              parts_of(a, b.a[u][i]);
-              acc[i] += slab(a, w);
-            }
-          }
-          __builtin_amdgcn_sched_barrier(0);
-        };
-        constexpr int STEP = GP_SLAB * U;
-        int batches = steady;
-        fetch(b0, k);
-        while (batches >= 3) {
-          fetch(b1, k + STEP);
-          multiply(b0);
-          fetch(b0, k + 2 * STEP);
-          multiply(b1);
-          k += 2 * STEP;
-          batches -= 2;
-        }
-        if (batches == 2) {
-          fetch(b1, k + STEP);
-          multiply(b0);
-          multiply(b1);
+          for (int p = 0; p < P; ++p) made.p[p] = staged[p * 4 * M];
         } else {
-          multiply(b0);
+          parts_of(made, a[i]);
         }
-        k += batches * STEP;
+        if constexpr (!SPREAD) acc[i] += slab(made, w);
+        else to[i * PAE_WAVE] = f32x4{0.f, 0.f, 0.f, 0.f} + slab(made, w);
       }
-      for (; k < end; k += GP_SLAB) {
-        Eight<TA> raw;
-        Parts<TA> w, a;
-        load8_anyhow<VEC>(raw, w_row, k, kq, K);
-        cut(raw, k, kq, K);
-        parts_of(w, raw);
+      if (SPREAD) to += MT * PAE_WAVE;
+      if (STAGED) staged += P * 4 * M;
+    };
+    if (batches > 0) {
+      // two batches take turns; no load stands under a condition of its own
+      auto multiply = [&](const Batch& b) {
 #pragma unroll
-        for (int i = 0; i < MT; ++i) {
-          load8_anyhow<VEC>(raw, a_row[i], k, kq, K);
-          cut(raw, k, kq, K);
-          parts_of(a, raw);
-          acc[i] += slab(a, w);
+        for (int u = 0; u < U; ++u) {
+          Parts<TA> w;
+          parts_of(w, b.w[u]);
+          join(w, b.a[u]);
         }
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      while (batches >= 3) {
+        fetch(b1, k + STEP);
+        multiply(b0);
+        fetch(b0, k + 2 * STEP);
+        multiply(b1);
+        k += 2 * STEP;
+        batches -= 2;
+      }
+      if (batches == 2) {
+        fetch(b1, k + STEP);
+        multiply(b0);
+        multiply(b1);
+      } else {
+        multiply(b0);
+      }
+      k += batches * STEP;
+    }
+    for (; k < end; k += GP_SLAB) {
+      Eight<TA> w_raw, a_raw[MT];
+      load8_anyhow<VEC>(w_raw, w_row, k, kq, K);
+      if constexpr (!STAGED) {
+#pragma unroll
+        for (int i = 0; i < MT; ++i) load8_anyhow<VEC>(a_raw[i], a_row[i], k, kq, K);
+#pragma unroll
+        for (int i = 0; i < MT; ++i) cut(a_raw[i], k, kq, K);
+      }
+      cut(w_raw, k, kq, K);
+      Parts<TA> w;
+      parts_of(w, w_raw);
+      join(w, a_raw);
+    }
+    if constexpr (!SPREAD) {
+      if (scratch) {  // this block's sums to memory; another kernel adds them up
+        if (block < blocks && n0 + r < N) {
+#pragma unroll
+          for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const int m = i * 16 + kq * 4 + e;
+              if (m < M) scratch[((int64_t)block * M + m) * N + n0 + r] = acc[i][e];
+            }
+        }
+        if (STAGED) __syncthreads();
+        continue;
+      }
+      if (block < blocks) {
+#pragma unroll
+        for (int i = 0; i < MT; ++i) to[i * PAE_WAVE] = acc[i];
       }
     }
-    if (scratch) {  // this block's sums to memory; another kernel adds them up
-      if (block < blocks && n0 + r < N) {
-#pragma unroll
-        for (int i = 0; i < MT; ++i)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int m = i * 16 + kq * 4 + e;
-            if (m < M) scratch[((int64_t)block * M + m) * N + n0 + r] = acc[i][e];
-          }
-      }
-      continue;
-    }
-    float* mine = part + wave * (MT * 256);
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) mine[(i * 16 + kq * 4 + e) * 16 + r] = acc[i][e];
     __syncthreads();
-    const int here = min(waves, blocks - first);
+    // output o of lane (o / 64 % 4, o % 16), element o / 16 % 4
+    auto place_of = [&](int o) { return (o / 256 * PAE_WAVE + o / 64 % 4 * 16 + o % 16) * 4 + o / 16 % 4; };
+    float* sums = (float*)sums_lds;
+    const int there = min(here, blocks - round);
+    if constexpr (SPREAD) {  // the blocks' sums, a thread an output; they take the place of the first slabs'
+      for (int o = threadIdx.x; o < there * MT * 256; o += blockDim.x) {
+        const int v = o / (MT * 256), left = K - (round + v) * GP_BLOCK;
+        float* from = sums + v * (SLOTS * MT * 256) + place_of(o % (MT * 256));
+        float slab_sum[GP_SLABS], sum = 0.f;
+#pragma unroll
+        for (int j = 0; j < GP_SLABS; ++j) slab_sum[j] = from[j * (MT * 256)];
+#pragma unroll
+        for (int j = 0; j < GP_SLABS; ++j) sum += j * GP_SLAB < left ? slab_sum[j] : 0.f;
+        *from = sum;
+      }
+      __syncthreads();
+    }
 #pragma unroll
     for (int i = 0; i < TOTALS; ++i) {
-      const int o = threadIdx.x + i * blockDim.x;
-      if (o < MT * 256)
-        for (int v = 0; v < here; ++v) total[i] += part[v * (MT * 256) + o];
+      const int o = threadIdx.x + i * blockDim.x, m = o / 16, n = n0 + o % 16;
+      if (o >= MT * 256) continue;
+      const float* from = sums + place_of(o);
+      for (int v = 0; v < there; ++v) {
+        const float sum = from[v * (SLOTS * MT * 256)];
+        if (!scratch) total[i] += sum;
+        else if (m < M && n < N) scratch[((int64_t)(round + v) * M + m) * N + n] = sum;  // another kernel adds them up
+      }
     }
-    __syncthreads();
+    if (first + step < blocks) __syncthreads();
   }
   if (scratch) return;
 #pragma unroll
@@ -323,7 +386,7 @@ __global__ __launch_bounds__(64 * GP_FEW_WAVES) void gemm_plain_few_kernel(
     const int o = threadIdx.x + i * blockDim.x, m = o / 16, n = n0 + o % 16;
     if (o < MT * 256 && m < M && n < N) {
       float v = sized<TA>(total[i]);
-      if constexpr (Parts<TA>::P > 1) {
+      if constexpr (P > 1) {
         if (!is_finite(v)) v = formed_again(A + m * lda, W + (int64_t)n * K, K);
       }
       if (bias) v += load_param(bias, b_is_f32, n);
@@ -604,6 +667,34 @@ extern "C" int64_t pae_gemm_plain_scratch(int M, int N, int K) {
   return (int64_t)((K + GP_BLOCK - 1) / GP_BLOCK) * part.rows * part.cols;
 }
 
+// How few rows are worked on.  What a wavefront does for a slab is mostly taking numbers apart (8.5 instructions a number, eight of W
+// and eight of A for each lane), and small products leave most places for wavefronts empty.  So where a unit has room for it, a block's slabs are
+// spread over up to 8 wavefronts, and up to 8 rows, of which a wavefront alone would take 16 apart, are taken apart once for all.
+// Without either / spread / spread and staged, us: 3 x 512 x 512 7.5, 4.9, 4.6; 1 x 896 x 896 8.1, 6.2, 5.9; 1 x 1,536 x 1,536 8.5, 8.2, 6.9; 8
+// rows 8.6, 8.9, 8.3.  Staged alone: 1 x 17,920 x 1,536 25.2 / 23.8, 3 x 1,536 x 8,960 24.4 / 22.1.
+// The lines: more than two blocks side by side (three and four with staged rows, or where rows are read number by number and what
+// counts is loads on their way: 1 x 1,537 x 1,538 18.0 / 12.9) are enough for the four SIMDs (16 x 1,536 x 1,536 9.2, spread 9.8; 16 x 896 x 4,864 15.1,
+// 16.4); a thread of a workgroup stages four eights at most (8 x 9,728 x 896 13.0, staged 14.4; 6 x 3,584 x 3,584 14.6, staged 15.9); 128 of k are four
+// slabs (1 x 1,536 x 64 3.6, staged 3.8, spread 4.2).  `here` blocks lie side by side in each of `groups` workgroups.
+struct GpFew {
+  int parts;  // wavefronts a block is spread over
+  bool staged;
+};
+static GpFew few_of(int here, int mt, int M, int K, int64_t groups, bool three_parts, bool vec) {
+  const int rounds = (int)(groups < 16 * GP_UNITS ? (groups + GP_UNITS - 1) / GP_UNITS : 16), side = 16 / here > 1 ? 16 / here : 1;
+  const int fit = rounds < side ? rounds : side;  // workgroups that a unit holds side by side
+  GpFew few = {1, false};
+  const bool may_stage = three_parts && mt == 1 && M <= GP_STAGED_ROWS && K > 128;
+  for (int staged = may_stage; staged >= 0; --staged) {
+    int parts = 1;
+    if (K > 128 && here <= (staged || !vec ? 4 : 2) && fit * here * (GP_SLABS * mt + (staged ? 3 * M : 0)) <= 160)
+      while (parts < 8 && here * parts * 2 <= GP_FEW_MOST && fit * here * parts * 2 <= 16) parts *= 2;
+    few = GpFew{parts, staged != 0};
+    if (staged && M <= 4 * parts && fit * here * ((parts > 1 ? GP_SLABS : 1) + 3 * M) <= 160) break;
+  }
+  return few;
+}
+
 template <typename TA, typename TC, bool VEC>
 static int launch_plain(void* C, int64_t ldc, int64_t batch_c, const void* A, int64_t lda, int64_t batch_a,
                         const void* W, int64_t batch_w, const void* bias, int b_is_f32, int M, int N, int K, int batch,
@@ -615,14 +706,32 @@ static int launch_plain(void* C, int64_t ldc, int64_t batch_c, const void* A, in
   // 14.5), except that rows read number by number stay with `few` up to 64 where there is more than a block of k (64 x 1,537 x 2,049 42 us)
   if (M <= (VEC || blocks == 1 ? GP_FEW_ROWS : 2 * GP_FEW_ROWS)) {
     const int each = (blocks + splits - 1) / splits;
-    const int waves = each < GP_FEW_WAVES ? each : GP_FEW_WAVES;
+    const int here = each < GP_FEW_WAVES ? each : GP_FEW_WAVES;
     const dim3 grid((N + 15) / 16, batch, splits);
-#define GP_FEW(MT)                                                                                               \
-  gemm_plain_few_kernel<TA, TC, MT, VEC><<<grid, waves * PAE_WAVE, scratch ? 0 : waves * MT * 1024, stream>>>(GP_ARGS)
+#define GP_FEW_KERNEL(MT, SPREAD, STAGED)                                                                                 \
+  do {                                                                                                                    \
+    auto kernel = gemm_plain_few_kernel<TA, TC, MT, VEC, SPREAD, STAGED>;                                                 \
+    const int lds = here * (few_slots(SPREAD) * MT + (STAGED ? 3 * M : 0)) * 1024;                                        \
+    if (lds > 65536) {                                                                                                    \
+      const hipError_t allowed = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds); \
+      PAE_REQUIRE(allowed == hipSuccess, "gemm: no %d bytes of LDS", lds);                                                \
+    }                                                                                                                     \
+    kernel<<<grid, here * few.parts * PAE_WAVE, lds, stream>>>(GP_ARGS, few.parts);                                       \
+  } while (0)
+#define GP_FEW(MT)                                                                                                        \
+  do {                                                                                                                    \
+    constexpr bool CAN = MT == 1 && Parts<TA>::P == 3;                                                                    \
+    const GpFew few = few_of(here, MT, M, K, (int64_t)grid.x * batch * splits, Parts<TA>::P == 3, VEC);                        \
+    if (few.parts > 1 && few.staged) GP_FEW_KERNEL(MT, true, CAN);                                                        \
+    else if (few.parts > 1) GP_FEW_KERNEL(MT, true, false);                                                               \
+    else if (few.staged) GP_FEW_KERNEL(MT, false, CAN);                                                                   \
+    else GP_FEW_KERNEL(MT, false, false);                                                                                 \
+  } while (0)
     if (M <= 16) GP_FEW(1);
     else if (VEC || M <= 32) GP_FEW(2);
     else if constexpr (!VEC) GP_FEW(4);
 #undef GP_FEW
+#undef GP_FEW_KERNEL
   } else {
     const GpShape shape = shape_of(M, N, K);
     const dim3 grid((unsigned)tiles_of(M, N, shape), batch, splits);

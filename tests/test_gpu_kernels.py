@@ -214,6 +214,20 @@ def test_gemm_plain_of_small_numbers(M, N, K_, scale):
     assert float((other.double().t() - want).norm() / want.norm()) <= rounded_sums(K_)
 
 
+@pytest.mark.parametrize("N,K_", [(40, 128), (40, 132), (33, 896), (9728, 896), (130, 1536), (50, 2048), (50, 2052), (40, 1537), (900, 4864), (1536, 8960)])
+def test_gemm_plain_of_a_few_rows_has_the_bits_of_many(N, K_):
+    """A block of k by one wavefront or by several, rows taken apart by each or once for all, one workgroup or several, blocks that are not
+    full: the bits of tiles of 64 rows."""
+    torch.manual_seed(N + K_)
+    a, w = torch.randn(70, K_, device=DEV), torch.randn(N, K_, device=DEV)
+    want = torch.empty(70, N, device=DEV)
+    K().gemm_plain(want, a, w)
+    for M in (1, 2, 4, 5, 8, 9, 13, 16, 17, 32):
+        out = torch.full((M, N), float("nan"), device=DEV)
+        K().gemm_plain(out, a[:M], w)
+        assert torch.equal(out, want[:M]), M
+
+
 @pytest.mark.parametrize("M,N,K_", [(300, 2100, 30000), (2100, 300, 30000)])
 def test_gemm_plain_in_parts_gives_the_bits_of_the_whole(M, N, K_):
     """Products whose blocks' sums do not fit the scratch memory at once are made in parts, along the columns or along the rows:
