@@ -49,7 +49,6 @@
 #define GP_STAGED_ROWS 8
 #define GP_TILE 64    // parts of a product are cut in multiples of it
 #define GP_UNITS 256  // compute units
-#define GP_LARGE_WHOLE 160  // large tiles from which on none is shared
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -586,34 +585,50 @@ __global__ __launch_bounds__(256) void gemm_plain_sum_kernel(TC* __restrict__ C,
   C[(int64_t)m * ldc + n] = from_f32<TC>(total);
 }
 
-// Tiles of 128 x 256 have the most products to a byte of LDS (M = N = 2,048 rows and 17,920 features of 1,536: 660 us against
-// 820 in tiles of 64 x 128), tiles of 64 x 64 let three workgroups a compute unit hide each other's waits and spread over the chip.  The
-// line lies at 200 pairs of a large tile and a block of k, of which a unit takes one at a time; a little over the chip's 256
-// leaves it a second round nearly empty.  Large / small: 65 x 17,920 x 1,536 (210 pairs) 53 / 62 us, 200 x 1,536 x 8,960 (216) 51 / 64, 450 x
-// 1,536 x 8,960 (432) 101 / 117, 601 x 17,920 x 1,536 (1,050) 249 / 275; 128 x 1,536 x 8,960 (108) 53 / 41, 601 x 2,048 x 1,536 (120) 46 /
-// 40, 65 x 2,048 x 1,536 (24) 40 / 14, 300 x 1,536 x 8,960 (324) 90 / 79, 2,048 x 1,536 x 1,536 (288) 94 / 74,
-// 400 x 17,920 x 1,536 (280 tiles) 254 / 187.
-struct GpShape {
-  int rows, cols;
+// How a product of many rows is cut: into tiles of 128 x 256, which have the most products to a byte of LDS, or of 64 x 64, of which three
+// workgroups a compute unit hide each other's waits, and over how many workgroups the blocks of k of a tile are shared.
+//
+// The least of the times (us) that the two shapes and every number of shares would take, from times of both at 18 sizes of weights (16 to 17,920
+// features, 512 to 18,944 of k) by 20 row counts from 33 to 4,096 and up to eight numbers of shares, which this meets within 11 % (root mean
+// square) and whose fastest it is on average 1 % behind: a large tile has a unit to itself and takes 36 a block of k, small ones 11.6 a
+// block alone, 15.4 two to a unit and 20.5 three to a unit; where rows are read number by number 73 and 24, 43 and 63.  Shares cost the
+// launch that adds their sums, and the sums a way to memory and back.  Large / small, each with its best number of shares: 65 x 17,920 x 1,536 54 / 64 us, 1,500 x 17,920 x 1,536 542 / 676, 300 x
+// 17,920 x 1,536 137 / 145, 601 x 1,536 x 8,960 129 / 145, 4,096 x 1,536 x 8,960 717 / 853; 65 x 1,536 x 8,960 49 / 38, 1,024 x 896 x 4,864 123 / 85,
+// 601 x 1,536 x 1,536 47 / 32, 65 x 64 x 1,536 42 / 14.
+struct GpTiles {
+  int rows, cols, splits;
 };
-static GpShape shape_of(int M, int N, int K) {
-  const int64_t tiles = (int64_t)((M + 127) / 128) * ((N + 255) / 256), pairs = tiles * ((K + GP_BLOCK - 1) / GP_BLOCK);
-  const int64_t groups = tiles >= GP_LARGE_WHOLE ? tiles : pairs;
-  const bool second_round = groups > GP_UNITS && groups <= GP_UNITS + GP_UNITS / 4 + 10;
-  return pairs >= 200 && !second_round ? GpShape{128, 256} : GpShape{64, 64};
+static int64_t tiles_of(int M, int N, int rows, int cols) { return (int64_t)((M + rows - 1) / rows) * ((N + cols - 1) / cols); }
+static GpTiles tiles_plan(int M, int N, int K, bool shared) {
+  const int blocks = (K + GP_BLOCK - 1) / GP_BLOCK;
+  const int64_t large = tiles_of(M, N, 128, 256), small = tiles_of(M, N, 64, 64);
+  struct Cost {
+    double large, small[4];
+  };
+  static const Cost by_fours = {35.9, {0.0, 11.6, 15.4, 20.5}}, one_by_one = {73.0, {0.0, 24.0, 43.0, 63.0}};
+  const Cost& cost = K % 4 ? one_by_one : by_fours;
+  GpTiles best = {64, 64, 1};
+  double least = 1e30;
+  for (int z = 1, last = 0; z <= (shared ? blocks : 1); ++z) {
+    const int each = (blocks + z - 1) / z;  // blocks of a workgroup
+    if (each == last) continue;             // no more shares than they take
+    last = each;
+    if (z > 1 && large * (z - 1) > 4 * GP_UNITS && small * (z - 1) > 6 * GP_UNITS) break;  // more rounds of both
+    const double each_k = each * GP_BLOCK < K ? each : K / (double)GP_BLOCK;
+    const double sums = z > 1 ? 1.9 + 8.0 * blocks * M * N / 7.6e6 : 0.0;
+    const int64_t rest = (small * z) % (3 * GP_UNITS);
+    const double by_large = 5.8 + (large * z + GP_UNITS - 1) / GP_UNITS * cost.large * each_k + sums;
+    const double by_small = 0.7 + ((small * z) / (3 * GP_UNITS) * cost.small[3] + cost.small[(rest + GP_UNITS - 1) / GP_UNITS]) * each_k + sums;
+    if (by_large < least) least = by_large, best = GpTiles{128, 256, z};
+    if (by_small < least) least = by_small, best = GpTiles{64, 64, z};
+  }
+  return best;
 }
-static int64_t tiles_of(int M, int N, GpShape shape) {
-  return (int64_t)((M + shape.rows - 1) / shape.rows) * ((N + shape.cols - 1) / shape.cols);
-}
-// Over how many workgroups the blocks of k of one tile are shared: 1 where the tiles fill the chip by themselves or
-// there is one block only.  A share costs its sums a way to memory and back and the launch that adds them (about
-// 4 us), so that up to 32 rows a workgroup's wavefronts take up to GP_FEW_WAVES blocks side by side first.
+// Over how many workgroups the blocks of k of one tile are shared.  A share costs its sums a way to memory and back and the launch that adds
+// them (about 4 us), so that up to 32 rows a workgroup's wavefronts take up to GP_FEW_WAVES blocks side by side first.
 // Few rows: a compute unit works through its workgroups in rounds, and shares pay where they leave fewer rounds of the whole
 // k.  Measured without shares / with them: 3 rows of 11,008 by 128 sixteens of weight rows (2 rounds of a third) 36.1 / 30.1 us, of
 // 16,384 by 192 (3 of a quarter) 50.0 / 44.3, of 8,192 by 192 (2 of a half) 27.0 / 28.6, of 11,008 by 256 (3 of a third) 44.8 / 49.3.
-// More rows: large tiles are shared up to 160 of them, for two rounds of the chip (300 x 17,920 x 1,536, 210 tiles, 122 / 146;
-// 200 x 17,920 x 1,536, 140 tiles, 128 / 109), small ones up to 500, for three workgroups a compute unit (601 x 2,048 x 1,536, 320
-// tiles, 44 / 40; 601 x 1,536 x 1,536, 240 tiles, the same both ways).
 static int splits_of(int M, int N, int K) {
   const int blocks = (K + GP_BLOCK - 1) / GP_BLOCK;
   if (M <= 0 || blocks == 1) return 1;
@@ -623,11 +638,7 @@ static int splits_of(int M, int N, int K) {
     const int64_t rounds = (sixteens + GP_UNITS - 1) / GP_UNITS, rounds_of_shares = (sixteens * shares + GP_UNITS - 1) / GP_UNITS;
     return rounds_of_shares < rounds * shares && shares <= 65535 ? (int)shares : 1;
   }
-  const GpShape shape = shape_of(M, N, K);
-  const int64_t tiles = tiles_of(M, N, shape);
-  if (tiles >= (shape.rows == 128 ? GP_LARGE_WHOLE : 500)) return 1;
-  const int want = (int)(((shape.rows == 128 ? 2 : 3) * GP_UNITS + tiles - 1) / tiles);
-  return want < blocks ? want : blocks;
+  return tiles_plan(M, N, K, true).splits;
 }
 
 // Rows and columns of C that one pass of launches makes.  A product with shared blocks of k keeps their sums, whatever the
@@ -649,7 +660,7 @@ static GpPart part_of(int M, int N, int K, bool shared) {
     if (N >= M) part.cols = cut(N, GP_SCRATCH / (blocks * M));
     else part.rows = cut(M, GP_SCRATCH / (blocks * N));
   }
-  part.rows = cut(part.rows, (int64_t)0xffffff / ((part.cols + GP_TILE - 1) / GP_TILE) * GP_TILE);
+  part.rows = cut(part.rows, (int64_t)0x7fffff / ((part.cols + GP_TILE - 1) / GP_TILE) * GP_TILE);
   return part;
 }
 
@@ -733,8 +744,8 @@ static int launch_plain(void* C, int64_t ldc, int64_t batch_c, const void* A, in
 #undef GP_FEW
 #undef GP_FEW_KERNEL
   } else {
-    const GpShape shape = shape_of(M, N, K);
-    const dim3 grid((unsigned)tiles_of(M, N, shape), batch, splits);
+    const GpTiles shape = tiles_plan(M, N, K, splits > 1);
+    const dim3 grid((unsigned)tiles_of(M, N, shape.rows, shape.cols), batch, splits);
     constexpr int ROW = 2 * Parts<TA>::P * 64;  // bytes of LDS
 #define GP_TILES(BM, BN, WM, WN, SHARED)                                                                                  \
   do {                                                                                                                    \

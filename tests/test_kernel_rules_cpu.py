@@ -29,10 +29,10 @@ def test_memory_for_the_sums_of_shared_products_is_bounded(M, N, K_):
 @pytest.mark.parametrize("M,N,K_", [(4194240, 16448, 1), (4194240, 4096, 64), (70000, 1 << 20, 1), (1, 1 << 30, 4), (64, 2000000000, 1)])
 @pytest.mark.parametrize("shared", [False, True])
 def test_products_of_any_size_fit_a_grid(M, N, K_, shared):
-    """A grid's threads along x are counted in 32 bits: 256 a tile of 64 x 64, up to 512 a sixteen of columns of few rows."""
+    """A grid's threads along x are counted in 32 bits: up to 512 a tile of 64 x 64, up to 768 a sixteen of columns of few rows."""
     rows, cols = part_of(M, N, K_, shared)
     assert 0 < rows <= M and 0 < cols <= N
-    assert (-(-rows // 64) * -(-cols // 64) * 256 if rows > 64 else -(-cols // 16) * 512) < 1 << 32
+    assert (-(-rows // 64) * -(-cols // 64) * 512 if rows > 64 else -(-cols // 16) * 768) < 1 << 32
 
 
 def test_routers_that_one_workgroup_reads_are_small():
