@@ -828,9 +828,14 @@ WIDE_ACTIVATIONS = {WIDE_PLAIN: ("gelu", "relu2"), WIDE_GATED: ("gelu_tanh", "si
 _WIDE_STRIDE = 1 << 22
 
 
-def wide_plan(a: torch.Tensor, w: torch.Tensor, mode: int = WIDE_PLAIN, kind: Optional[str] = None, ranges: bool = False) -> Optional[int]:
-    """How `gemm_wide` makes this product, or None: sizes or operands it does not take, or that the platform's library is
-    ahead at.  `ranges`: the product may leave float32 sums of ranges of k (plan >> 8 says how many)."""
+def wide_plan(a: torch.Tensor, w: torch.Tensor, mode: int = WIDE_PLAIN, kind: Optional[str] = None, ranges: bool = False,
+              bias: Optional[torch.Tensor] = None) -> Optional[int]:
+    """How `gemm_wide` makes this product, or None: sizes or operands it does not take (among them those that the library refuses), or that
+    the platform's library is ahead at.  `ranges`: the product may leave float32 sums of ranges of k (plan >> 8 says how many)."""
+    if not a.is_cuda or a.device != w.device or a.dim() != 2 or w.dim() != 2 or a.shape[1] != w.shape[1]:
+        return None
+    if bias is not None and (bias.device != a.device or bias.dtype not in _CODE or bias.shape != (w.shape[0],) or not bias.is_contiguous()):
+        return None
     if (a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or a.shape[0] <= SKINNY_MAX_ROWS or w.shape[0] % 16 or w.shape[1] % 64
             or w.shape[0] == 0 or w.shape[1] == 0 or a.stride(1) != 1 or a.stride(0) % 8 or not w.is_contiguous()
             or a.data_ptr() % 16 or w.data_ptr() % 16 or a.stride(0) >= _WIDE_STRIDE or w.shape[1] >= _WIDE_STRIDE):

@@ -48,7 +48,7 @@ class Linear:
         if bias is None:
             return K.product_of_rows(x, self.weight)
         out = torch.empty((x.shape[0], self.out_features), dtype=x.dtype, device=x.device)
-        plan = K.wide_plan(x, self.weight)
+        plan = K.wide_plan(x, self.weight, bias=bias)
         if plan is None:
             torch.addmm(bias if bias.dtype == x.dtype else bias.to(x.dtype), x, self.weight.t(), out=out)
         else:

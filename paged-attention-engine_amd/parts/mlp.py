@@ -117,7 +117,7 @@ class DenseFeedForward(Part):
         it; elsewhere a product of many rows is followed by the activation kernel, which adds the bias first: the
         same bits as the epilogue of many rows."""
         x = plain_rows(x)
-        plan = K.wide_plan(x, self.up.weight, K.WIDE_PLAIN, self.spec.activation)
+        plan = K.wide_plan(x, self.up.weight, K.WIDE_PLAIN, self.spec.activation, bias=self.up.bias)
         if x.shape[0] and K.skinny_supported(x, self.up.weight):
             act = torch.empty((x.shape[0], self.spec.intermediate_size), dtype=x.dtype, device=x.device)
             splits = K.whole_sum_splits(self.spec.intermediate_size, self.spec.hidden_size, x.shape[0])

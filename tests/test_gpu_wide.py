@@ -162,3 +162,17 @@ def test_linear_with_odd_operands():
             got = Linear(w, None if b is None else b.to(torch.bfloat16))(a)
             # (the library may round the product before it adds the bias)
             check(got, want, err + 2.0 ** -7 * ref.abs())
+
+
+def test_linear_with_odd_biases():
+    """A bias that does not lie number by number, or is one number for all, goes to the library; shapes that do not fit are refused there."""
+    from paged_attention_engine_amd.parts.linear import Linear
+
+    a, w = operands(100, 256, 256, 6)
+    wide = torch.randn(2 * 256, device="cuda").to(torch.bfloat16)
+    for bias in (wide[::2], wide[:1], wide[:256].to(torch.float16)):
+        ref, err = exact(a, w)
+        want = ref + bias.to(torch.bfloat16).double()
+        check(Linear(w, bias)(a), want, err + 2.0 ** -7 * ref.abs())
+    with pytest.raises(RuntimeError):
+        Linear(w)(a[:, :128].contiguous())

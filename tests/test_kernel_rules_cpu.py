@@ -68,3 +68,15 @@ def test_products_of_few_tiles_and_much_of_k_go_to_the_library(M, N, K_):
 def test_the_shape_of_a_product_between_one_and_two_small_tiles_a_unit():
     """Rows of 2,048 numbers and more come slower to two workgroups a unit: 128 x 96 is ahead of 64 x 128 there (24.8 against 28.1 us)."""
     assert K.library().pae_gemm_wide_plan(K.WIDE_PLAIN, -1, 300, 4608, 3584, 0) == 3 | 1 << 8
+
+
+def test_products_of_many_rows_take_the_operands_that_the_library_takes():
+    """Tensors that are not the GPU's, and shapes that do not fit each other, are the library's, to work on or to refuse."""
+    from paged_attention_engine_amd.parts.linear import Linear
+
+    a, w, bias = (torch.randn(*shape).to(torch.bfloat16) for shape in ((70, 128), (64, 128), (64,)))
+    assert torch.equal(Linear(w)(a), torch.mm(a, w.t()))
+    assert torch.equal(Linear(w, bias)(a), torch.addmm(bias, a, w.t()))
+    for wrong in (a[:, :64].contiguous(), a[:, 0], a[None]):
+        with pytest.raises(RuntimeError):
+            Linear(w)(wrong)
