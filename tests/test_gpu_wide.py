@@ -137,7 +137,7 @@ def test_same_bits_as_two_kernels(M, N, k):
 def test_which_products_are_taken():
     a, w = operands(100, 1536, 1536)
     assert K.wide_plan(a, w) is not None
-    plan = K.wide_plan(a, operands(100, 1536, 8960)[1], K.WIDE_SUMS, ranges=True)
+    plan = K.wide_plan(*operands(100, 1536, 8960), K.WIDE_SUMS, ranges=True)
     assert plan >> 8 > 1  # few tiles and much of k
     for bad in (a[:64], a.float(), a[:, 1:], a.t()):
         assert K.wide_plan(bad, w) is None
