@@ -11,7 +11,9 @@
 // float32 instructions (v_mfma_f32_16x16x4_f32), which these replace, add up four products at a time and give 154 TFLOP/s on the
 // whole chip; six of the others do the work at up to 230.  A slab's products are a sum of their own before they join the others'.  Error
 // against 64 bits (root mean square, share of the result's; normal operands): k 1,536 4.1e-7 before, 1.0e-7 now; 8,960 4.1e-7 and
-// 1.6e-7; 18,944 4.2e-7 and 2.1e-7; bfloat16 operands 1.7e-7 and 0.9e-7.
+// 1.6e-7; 18,944 4.2e-7 and 2.1e-7; bfloat16 operands 1.7e-7 and 0.9e-7.  (Rows with one or two numbers only are further off than before, 3.5e-8
+// against 2.5e-8 and 3.3e-8 against 3.1e-8: the last of the six instructions does not always round to the nearest.  Adding it up apart from
+// the others mends that and takes tiles of 128 x 256 6 to 9 % longer.)
 //
 // k is cut into slabs of 32, one set of instructions each, and into blocks of 512 whose sums are then added up in
 // order (with rows of 30,000 terms one running sum loses a digit more than the block sums do).  Every kernel here adds in this
@@ -19,17 +21,19 @@
 // the blocks are shared out or on which other rows share the launch.
 //
 // Why three kernels.  Up to 32 rows the weights' way from memory is the time: `few` gives 16 weight
-// rows to a workgroup whose wavefronts take a block of k each, nothing staged (a wavefront reads 16
+// rows to a workgroup whose wavefronts take a block of k each, or a part of one where they are few (a wavefront reads 16
 // rows x 64 bytes an instruction).  With more rows the matrix cores are: `tiles` takes the numbers apart once and stages the
 // parts of 32 of k through LDS, two buffers that take turns.  Where a launch has too
-// few tiles for the chip the blocks of k are shared out over workgroups as well (`splits`): the
+// few tiles for the chip the blocks of k are shared out over workgroups as well: the
 // block sums go to scratch memory and `sum` adds them in order.
-// Measured, weights from HBM, 2,048 / 1,536 / 17,920 x 1,536 and 1,536 x 8,960, before (float32 instructions, tiles of 64 x 64) and now:
-//   3 rows     8.2, 9.0, 24.0 (4.6 TB/s), 22 us, and the same now
-//   64 rows    18, 18, 76, 64 us                 15, 15, 52, 25
-//   300 rows   27, 27, 173, 95                   25, 23, 142, 81
-//   601 rows   48, 37, 306 (108 TFLOP/s), 185    40, 31, 256 (129 TFLOP/s), 128
-//   2,048      117, 88, 967, 473                 98, 74, 666 (169), 379
+// Measured, weights from HBM, 2,048 / 1,536 / 17,920 x 1,536 and 1,536 x 8,960, with the float32 instruction in tiles of 64 x 64 and now:
+//   3 rows     6.9, 6.8, 26.3 (4.2 TB/s), 23 us      8.0, 7.9, 26.7, 22 us
+//   64 rows    18, 18, 78, 65                        17, 18, 46, 26
+//   300 rows   27, 27, 173, 96                       25, 24, 135, 85
+//   601 rows   51, 39, 332 (100 TFLOP/s), 188        43, 33, 264 (125 TFLOP/s), 131
+//   2,048      117, 90, 985, 488                     101, 79, 703 (160), 369
+// The nearest second part and the factor 2^16 are two of the 8.5 instructions that take a number apart: without them 601 rows take 253
+// and 127 us instead of 264 and 131.
 // Tried: W's rows from memory straight to the registers they are multiplied from (a wavefront's load then touches 16 lines, and what
 // a slab needs took 2.4 us to arrive); numbers taken apart with conversions and dot products (see half_parts_of); loads under a condition
 // (see load8_anyhow);
@@ -397,7 +401,7 @@ __global__ __launch_bounds__(64 * (SPREAD && MT <= 2 ? GP_FEW_MOST : GP_FEW_WAVE
 // Tiles of BM rows of A by BN of W, WM x WN wavefronts.  blockIdx.x: the tiles, those of one column of tiles (the same weights)
 // next to each other on one die; blockIdx.y: the product of the batch; blockIdx.z: a share of the blocks of k.
 // What bounds it is the matrix cores' six instructions a slab of float32 and, not far behind, LDS, which takes in 192 bytes a row
-// and slab and gives them to WN or WM wavefronts; a thread takes three eights a slab apart (26 instructions a half; one eight in
+// and slab and gives them to WN or WM wavefronts; a thread takes three eights a slab apart (34 instructions a half; one eight in
 // tiles of 64 x 64) between its products.  A row of 32 numbers of one part, 64 bytes, lies in LDS as four eights, at places turned by the row so
 // that the 16 rows that a wavefront reads an eight of fall into different banks.
 template <typename TA, typename TC, int BM, int BN, int WM, int WN, bool VEC, bool SHARED>

@@ -3,9 +3,10 @@
 The reference calls F.linear on weights stored (out_features, in_features)
 (engine/model.py:303-305,315,318-320).  Here:
 
-  float32    this engine's own product kernels on the float32 matrix cores: products
-             and sums in full 32-bit, in an order that depends on k alone, each row
-             independent of the batch;
+  float32    this engine's own product kernels: a number is taken apart into three bfloat16
+             numbers that hold its 24 bits, six products of parts are added in float32 by
+             the bfloat16 matrix cores (what they leave out of a product is below 2^-24 of it),
+             in an order that depends on k alone, each row independent of the batch;
   bfloat16   up to 64 rows (decode steps, small portions): the weight-streaming
              matrix-core kernel, which reads W once; more rows: this engine's tiled
              kernels, or the platform's matrix library where it is ahead or the sizes are none

@@ -117,7 +117,7 @@ def test_gemm_plain_adds_in_one_order(N, K_):
 def test_gemm_plain_keeps_what_is_not_finite(M, N, K_):
     """float32 numbers are taken apart for the product; infinities, numbers that are none and numbers so large that their first part would be
     infinite give what they give in the numbers themselves, in every kernel (few rows; small and large tiles, shared k
-    or not), and nothing beside them changes.  Rows of small numbers keep their digits."""
+    or not), and nothing beside them changes, a row of small numbers among it (whose digits test_gemm_plain_of_small_numbers looks at)."""
     torch.manual_seed(M)
     a, w = torch.randn(M, K_, device=DEV), torch.randn(N, K_, device=DEV)
     plain = torch.empty(M, N, device=DEV)
