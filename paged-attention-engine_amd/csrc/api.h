@@ -115,10 +115,13 @@ int pae_latent_queries(void* out, const void* proj, int64_t row_stride, int num_
                        float magnitude, int H, int D, int rd, int rot, int interleaved, int KD, hipStream_t stream);
 // prefill attention with value heads of their own width and a gate per token and head: see attention_mfma.hip
 int pae_attn_prefill_wide_width(int width, int vd);
+// which kernel takes a step's runs (0, or the query groups a workgroup: see attention_mfma.hip)
+int pae_attn_prefill_route(int nh, int hd, int vd, int bs, int num_tiles, int tokens, int max_blocks, int window);
 int pae_attn_prefill_wide_bf16(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k_cache,
                                const void* v_cache, const int* tiles, int num_tiles, const int* positions,
                                const int* block_tables, int max_blocks, int nh, int nkv, int hd, int vd, float scale,
-                               int window, const void* head_gate, int64_t head_gate_stride, hipStream_t stream);
+                               int window, const void* head_gate, int64_t head_gate_stride, int tokens, int route,
+                               hipStream_t stream);
 // rows [q | k | v]: RMS norm of q and of k over the whole projection, or head by head with one weight that the
 // heads share (`per_head`; weights null: none), rotation, cache write
 int pae_qk_norm_rotate_store(int dtype, void* qkv, int64_t row_stride, int num_tokens, int nh, int nkv, int hd, int vd,
@@ -239,7 +242,7 @@ int pae_attn_prefill_capped_bf16(void* out, int64_t out_stride, const void* q, i
                                  const void* v_cache, const int* tiles, int num_tiles, const int* positions,
                                  const int* block_tables, int max_blocks, int bs, int nh, int nkv, int hd, float scale,
                                  int window, float cap, const float* sinks, const void* head_gate,
-                                 int64_t head_gate_stride, hipStream_t stream);
+                                 int64_t head_gate_stride, int tokens, int route, hipStream_t stream);
 // the two with the window read as a chunk length (`chunked`), a bias by distance (`slopes` float32 [nh] or null:
 // score -= slopes[h] (position - key)) and a gate on the output (`gate` bfloat16 rows [token][nh * hd] or null)
 int pae_attn_decode_biased_bf16(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k_cache,
@@ -251,7 +254,7 @@ int pae_attn_prefill_biased_bf16(void* out, int64_t out_stride, const void* q, i
                                  const void* v_cache, const int* tiles, int num_tiles, const int* positions,
                                  const int* block_tables, int max_blocks, int bs, int nh, int nkv, int hd, float scale,
                                  int window, int chunked, const float* slopes, const void* gate, int64_t gate_stride,
-                                 hipStream_t stream);
+                                 int tokens, int route, hipStream_t stream);
 // A decode step's layers as one resident kernel (see decode_program.hip).
 // A caller builds a list of phases in host memory with the put functions (each returns the bytes of
 // LDS a quad of four wavefronts needs for the phase, or a negative code), copies it to the device and

@@ -16,6 +16,13 @@ __device__ __forceinline__ short bf16_bits(float x) {
   return *reinterpret_cast<const short*>(&h);
 }
 
+// The first key that position `pos` sees under a sliding window (0: none) or in chunks of `window`.
+__device__ __forceinline__ int first_visible(int pos, int window, int chunked) {
+  if (window <= 0) return 0;
+  if (chunked) return pos - pos % window;
+  return pos - window + 1 > 0 ? pos - window + 1 : 0;
+}
+
 // State of CT column tiles of one wavefront.
 template <int HD, int CT>
 struct AttnState {

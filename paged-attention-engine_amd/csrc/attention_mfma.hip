@@ -20,7 +20,8 @@
 //          and merge in LDS; a second small kernel merges the splits.  Splits
 //          start at multiples of the split length from position 0.
 // prefill: one workgroup per (up to 64 consecutive tokens of a sequence, query head), whose
-//          wavefronts share out the keys (see there).
+//          wavefronts share out the keys (see there); most runs of more than a few hundred tokens go to
+//          attention_prefill.hip, which shares them through LDS (`route_of` below has the rule).
 //
 // Masking is the reference's rule (engine/attention.py:474-487: key j visible iff
 // j <= position of the query) plus an optional window.  A column's result depends
@@ -32,6 +33,7 @@
 #include "common.h"
 #include "api.h"
 #include "attention_device.h"
+#include "attention_prefill.h"
 
 // ------------------------------------------------------------------ decode
 // Split s of a token covers keys [s * 64 TPW, (s + 1) * 64 TPW); wavefront w of its
@@ -43,12 +45,6 @@
 // for every workgroup and cost more than the second launch.)
 //   part_acc[((token * nkv + kvh) * max_splits + split) * g + head in group][HD]
 //   part_ml [ ... same index ... ][2] = (maximum in log2 units, sum)
-__device__ __forceinline__ int first_visible(int pos, int window, int chunked) {
-  if (window <= 0) return 0;
-  if (chunked) return pos - pos % window;
-  return pos - window + 1 > 0 ? pos - window + 1 : 0;
-}
-
 template <int HD, int TPW, bool CAPPED, bool BIASED>
 __global__ __launch_bounds__(256) void attn_decode_kernel(
     float* __restrict__ part_acc, float* __restrict__ part_ml, int max_splits,
@@ -263,7 +259,6 @@ typedef __attribute__((ext_vector_type(2))) float f32x2;
 typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
 typedef __attribute__((ext_vector_type(4))) int i32x4;
-#define RESCALE_STEP 8.0f
 
 // A register loaded in the order (row = lane / 4, group = lane % 4), in which a quad of lanes reads
 // contiguous bytes, moved to the matrix instruction's order (row = lane % 16, group = lane / 16).
@@ -274,8 +269,8 @@ __device__ __forceinline__ bf16x8 quad_to_mfma_order(bf16x8 x, int fetch_from) {
   return *reinterpret_cast<bf16x8*>(&raw);
 }
 
-// tiles[t] = (table row of the sequence, first flat token, number of tokens <= 64); blockIdx.z picks
-// the part of 16 CT tokens of the run that this workgroup takes.
+// tiles[t] = (table row of the sequence, first flat token, number of tokens <= 128); a workgroup takes
+// 16 CT of them, the last ones (which see the most keys) first.
 // BS: the page size if it is 16 (the value rows' offsets are then constants), or 0 for any other.
 // VD: the width of a value head, if it is not HD.
 // `head_gate` (null: none): one number a token and head, the head's output is multiplied by its sigmoid.
@@ -298,11 +293,13 @@ __global__ __launch_bounds__(256, 1) void attn_prefill_split_kernel(
   // keys and values in flight)
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PAE_WAVE), lane = threadIdx.x % PAE_WAVE;
   const int col = lane % 16, g4 = lane / 16;
-  const int head = blockIdx.x, kvh = head / (nh / nkv);
+  constexpr int PARTS = PREFILL_RUN / TOK;
+  const int head = blockIdx.x % nh, kvh = head / (nh / nkv);
+  const int tile = blockIdx.y, part = PARTS - 1 - blockIdx.x / nh;
   const float slope_over_scale = (BIASED && slopes) ? slopes[head] * inv_scale : 0.f;
-  const int seq_row = tiles[blockIdx.y * 3];
-  const int tok0 = tiles[blockIdx.y * 3 + 1] + blockIdx.z * TOK;
-  const int ntok = min(TOK, tiles[blockIdx.y * 3 + 2] - (int)blockIdx.z * TOK);
+  const int seq_row = tiles[tile * 3];
+  const int tok0 = tiles[tile * 3 + 1] + part * TOK;
+  const int ntok = min(TOK, tiles[tile * 3 + 2] - part * TOK);
   if (ntok <= 0) return;  // the whole workgroup
   const int* table = block_tables + (int64_t)seq_row * max_blocks;
   const int pos0 = positions[tok0];
@@ -702,15 +699,57 @@ extern "C" int pae_attn_decode_bf16(void* out, int64_t out_stride, const void* q
                                      max_blocks, bs, nh, nkv, hd, scale, window, 0.f, nullptr, nullptr, 0, part_acc, part_ml, stream);
 }
 
-// tiles[t] = (table row of the sequence, first flat token, number of tokens <= 64), heaviest runs
+// Which kernel takes a step's runs: 0 the one above, else the query groups of a workgroup of attention_prefill.hip.
+// Times in us, from graphs of one kernel over 130 steps (12, 14 and 28 heads of 64, 128 and 192 features, 1 to 8
+// sequences of 32 to 8,192 tokens); the choice is on average 1 % behind the fastest of the three.
+//   * 32-token workgroups that are one round of the chip and meet about a thousand keys: the kernel above, which has no
+//     LDS to fill before its first product (12 heads, 128 tokens: 7.7, two query groups 8.9; 512 tokens 10.5 and 11.3; 1,024
+//     tokens, 384 workgroups, 19.2 and 14.6; 64 tokens behind 3,000 28.4 and 25.3).
+//   * else two query groups where 64-token workgroups are one round, and for heads of 64 always (two of its workgroups fit a
+//     compute unit: 14 heads, 4,096 tokens 47.2, four groups 49.2);
+//   * else whichever ends sooner as a row of workgroups of (start and end + keys) dealt to 256 compute units, longest
+//     first: 12 heads of 128, one prompt of 2,048 tokens 27.0 (two) and 31.1 (four), of 8,192 237 and 213; 8 prompts of
+//     600 tokens in all, one round of four groups and two of two, 17.0 and 13.1.
+static int route_of(int nh, int hd, int vd, int bs, int num_tiles, int tokens, int max_blocks, int window) {
+  if (!attn_prefill_shared_takes(hd, vd, bs)) return 0;
+  const double runs = num_tiles;  // workgroups of 32 and 64 tokens, about: every run's last one is half full
+  const double few = nh * fmin(4 * runs, tokens / 32.0 + runs / 2), two = nh * fmin(2 * runs, tokens / 64.0 + runs / 2), four = nh * runs;
+  double keys = 16.0 * max_blocks;
+  if (window > 0) keys = fmin(keys, window + (double)PREFILL_RUN);
+  if (few <= 288 && keys <= 1024) return 0;
+  if (hd == 64 || two <= 256) return 2;
+  const double mean = tokens < keys ? keys - 0.5 * tokens : 0.5 * keys;
+  auto time = [&](double groups, double start, double per_key) {
+    const double longest = start + per_key * keys;
+    if (groups <= 256) return longest;
+    const double level = groups / 256 * (start + per_key * mean);
+    // up to two rounds: the shortest of the first round and the longest of the second, on one unit
+    const double stacked = groups <= 512 ? 2 * (start + per_key * (keys - 2 * (keys - mean) * 256 / groups)) : 0;
+    return fmax(longest, fmax(level, stacked));
+  };
+  return time(four, 10.0, 1 / 73.0) < time(two, 7.5, 1 / 128.0) ? 4 : 2;
+}
+
+extern "C" int pae_attn_prefill_route(int nh, int hd, int vd, int bs, int num_tiles, int tokens, int max_blocks, int window) {
+  return route_of(nh, hd, vd, bs, num_tiles, tokens, max_blocks, window);
+}
+
+static int check_route(const char* what, int route, int hd, int vd, int bs, const void* k, const void* v) {
+  PAE_REQUIRE(route <= 0 || ((route == 2 || route == 4) && attn_prefill_shared_takes(hd, vd, bs) && ((uintptr_t)k | (uintptr_t)v) % 16 == 0),
+              "%s: %d query groups a workgroup are not built for heads of %d and %d in pages of %d", what, route, hd, vd, bs);
+  return 0;
+}
+
+// tiles[t] = (table row of the sequence, first flat token, number of tokens <= 128), heaviest runs
 // first: workgroups start in the order of the grid, and the last to finish sets the time.
+// `tokens`: the step's rows, as many as the runs have or a few more.  `route`: what `route_of` says, or -1 to ask it.
 static int attn_prefill_any(void* out, int64_t out_stride, const void* q, int64_t q_stride,
                                           const void* k_cache, const void* v_cache, const int* tiles,
                                           int num_tiles, const int* positions, const int* block_tables,
                                           int max_blocks, int bs, int nh, int nkv, int hd, float scale, int window,
                                           float cap, const float* sinks, bool biased, int chunked, const float* slopes,
                                           const void* gate, int64_t gate_stride, const void* head_gate,
-                                          int64_t head_gate_stride, hipStream_t stream) {
+                                          int64_t head_gate_stride, int tokens, int route, hipStream_t stream) {
   if (int rc = check_common("attn_prefill", nh, nkv, hd, bs, max_blocks, window)) return rc;
   PAE_REQUIRE(!biased || cap == 0.f, "attn_prefill: a bias by distance and a score cap together are not built");
   PAE_REQUIRE(!biased || !slopes || scale > 0.f, "attn_prefill: a bias by distance needs a positive scale");
@@ -720,16 +759,26 @@ static int attn_prefill_any(void* out, int64_t out_stride, const void* q, int64_
               (long long)head_gate_stride);
   PAE_REQUIRE(num_tiles <= 65535, "attn_prefill: %d runs exceed the grid", num_tiles);
   if (num_tiles <= 0) return 0;
+  if (int rc = check_route("attn_prefill", route, hd, hd, bs, k_cache, v_cache)) return rc;
   const float scale_log2 = scale * LOG2E;
+  PAE_REQUIRE(cap >= 0.f && (cap == 0.f || scale > 0.f), "attn_prefill: bad score cap %g (scale %g)", (double)cap, (double)scale);
+  const float cap_over_scale = cap > 0.f ? cap / scale : 0.f, scale_over_cap = cap > 0.f ? scale / cap : 0.f;
+  // (pages that do not start on 16 bytes, which the loads to LDS need, stay here)
+  if (route < 0) route = ((uintptr_t)k_cache | (uintptr_t)v_cache) % 16 ? 0 : route_of(nh, hd, hd, bs, num_tiles, tokens, max_blocks, window);
+  if (route > 0) {
+    const PrefillArgs args = {(bf16_t*)out, out_stride, (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache,
+                              tiles, num_tiles, positions, block_tables, max_blocks, nh, nkv, scale_log2, window, cap_over_scale,
+                              scale_over_cap, sinks, chunked, slopes, slopes ? 1.0f / scale : 0.f, (const bf16_t*)gate, gate_stride,
+                              (const bf16_t*)head_gate, head_gate_stride};
+    return attn_prefill_shared(args, hd, hd, biased, route, stream);
+  }
   // Four column tiles (64 tokens) per workgroup up to head_dim 128, two above (registers).  Two also up to
   // head_dim 128 while the 64-token workgroups would not fill the chip's compute units: twice the
   // workgroups, each with half the arithmetic per 32 keys (1.5B heads: 512 tokens 16.4 -> 12.1 us, 1,024
   // tokens 22.0 -> 19.3; from 2,048 tokens on, 384 workgroups, four tiles are ahead: 40.5 against 47.0 us).
-  const bool halves = (int64_t)nh * num_tiles <= 256;
-  PAE_REQUIRE(cap >= 0.f && (cap == 0.f || scale > 0.f), "attn_prefill: bad score cap %g (scale %g)", (double)cap, (double)scale);
-  const float cap_over_scale = cap > 0.f ? cap / scale : 0.f, scale_over_cap = cap > 0.f ? scale / cap : 0.f;
+  const bool halves = (int64_t)nh * min(2 * num_tiles, tokens / 64 + (num_tiles + 1) / 2) <= 256;
 #define LAUNCH_CAPPED(HD, CT, BS, CAPPED, BIASED)                                                              \
-  attn_prefill_split_kernel<HD, CT, BS, CAPPED, BIASED><<<dim3(nh, num_tiles, 4 / CT), 256, 0, stream>>>(      \
+  attn_prefill_split_kernel<HD, CT, BS, CAPPED, BIASED><<<dim3(nh * (PREFILL_RUN / 16 / CT), num_tiles), 256, 0, stream>>>( \
       (bf16_t*)out, out_stride, (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache,    \
       tiles, positions, block_tables, max_blocks, bs, nh, nkv, scale_log2, window, cap_over_scale,             \
       scale_over_cap, sinks, chunked, slopes, slopes ? 1.0f / scale : 0.f, (const bf16_t*)gate, gate_stride, (const bf16_t*)head_gate, head_gate_stride)
@@ -766,10 +815,10 @@ extern "C" int pae_attn_prefill_capped_bf16(void* out, int64_t out_stride, const
                                           int num_tiles, const int* positions, const int* block_tables,
                                           int max_blocks, int bs, int nh, int nkv, int hd, float scale, int window,
                                           float cap, const float* sinks, const void* head_gate, int64_t head_gate_stride,
-                                          hipStream_t stream) {
+                                          int tokens, int route, hipStream_t stream) {
   return attn_prefill_any(out, out_stride, q, q_stride, k_cache, v_cache, tiles, num_tiles, positions, block_tables,
                           max_blocks, bs, nh, nkv, hd, scale, window, cap, sinks, false, 0, nullptr, nullptr, 0, head_gate,
-                          head_gate_stride, stream);
+                          head_gate_stride, tokens, route, stream);
 }
 
 extern "C" int pae_attn_prefill_biased_bf16(void* out, int64_t out_stride, const void* q, int64_t q_stride,
@@ -777,10 +826,10 @@ extern "C" int pae_attn_prefill_biased_bf16(void* out, int64_t out_stride, const
                                           int num_tiles, const int* positions, const int* block_tables,
                                           int max_blocks, int bs, int nh, int nkv, int hd, float scale, int window,
                                           int chunked, const float* slopes, const void* gate, int64_t gate_stride,
-                                          hipStream_t stream) {
+                                          int tokens, int route, hipStream_t stream) {
   return attn_prefill_any(out, out_stride, q, q_stride, k_cache, v_cache, tiles, num_tiles, positions, block_tables,
                           max_blocks, bs, nh, nkv, hd, scale, window, 0.f, nullptr, true, chunked, slopes, gate, gate_stride,
-                          nullptr, 0, stream);
+                          nullptr, 0, tokens, route, stream);
 }
 
 extern "C" int pae_attn_prefill_bf16(void* out, int64_t out_stride, const void* q, int64_t q_stride,
@@ -788,7 +837,8 @@ extern "C" int pae_attn_prefill_bf16(void* out, int64_t out_stride, const void* 
                                      const int* positions, const int* block_tables, int max_blocks, int bs, int nh,
                                      int nkv, int hd, float scale, int window, hipStream_t stream) {
   return pae_attn_prefill_capped_bf16(out, out_stride, q, q_stride, k_cache, v_cache, tiles, num_tiles, positions,
-                                      block_tables, max_blocks, bs, nh, nkv, hd, scale, window, 0.f, nullptr, nullptr, 0, stream);
+                                      block_tables, max_blocks, bs, nh, nkv, hd, scale, window, 0.f, nullptr, nullptr, 0,
+                                      num_tiles * PREFILL_RUN, -1, stream);
 }
 
 // Key widths `hd` (multiples of 32 up to 256) built for values `vd` wide: the smallest that holds `width` features, or 0.
@@ -806,15 +856,23 @@ extern "C" int pae_attn_prefill_wide_width(int width, int vd) {
 extern "C" int pae_attn_prefill_wide_bf16(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k_cache,
                                           const void* v_cache, const int* tiles, int num_tiles, const int* positions,
                                           const int* block_tables, int max_blocks, int nh, int nkv, int hd, int vd, float scale,
-                                          int window, const void* head_gate, int64_t head_gate_stride, hipStream_t stream) {
+                                          int window, const void* head_gate, int64_t head_gate_stride, int tokens, int route, hipStream_t stream) {
   if (int rc = check_common("attn_prefill_wide", nh, nkv, hd, 16, max_blocks, window)) return rc;
   PAE_REQUIRE(pae_attn_prefill_wide_width(hd, vd) == hd, "attn_prefill_wide: keys of %d with values of %d are not built", hd, vd);
   PAE_REQUIRE(out_stride >= (int64_t)nh * vd && q_stride >= (int64_t)nh * hd, "attn_prefill_wide: row strides too small");
   PAE_REQUIRE(!head_gate || head_gate_stride >= nh, "attn_prefill_wide: gate row stride %lld too small", (long long)head_gate_stride);
   PAE_REQUIRE(num_tiles <= 65535, "attn_prefill_wide: %d runs exceed the grid", num_tiles);
   if (num_tiles <= 0) return 0;
+  if (int rc = check_route("attn_prefill_wide", route, hd, vd, 16, k_cache, v_cache)) return rc;
+  if (route < 0) route = ((uintptr_t)k_cache | (uintptr_t)v_cache) % 16 ? 0 : route_of(nh, hd, vd, 16, num_tiles, tokens, max_blocks, window);
+  if (route > 0) {
+    const PrefillArgs args = {(bf16_t*)out, out_stride, (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache,
+                              tiles, num_tiles, positions, block_tables, max_blocks, nh, nkv, scale * LOG2E, window, 0.f, 0.f,
+                              nullptr, 0, nullptr, 0.f, nullptr, 0, (const bf16_t*)head_gate, head_gate_stride};
+    return attn_prefill_shared(args, hd, vd, false, route, stream);
+  }
 #define WIDE_LAUNCH(HD, CT, VD)                                                                                          \
-  attn_prefill_split_kernel<HD, CT, 16, false, false, VD><<<dim3(nh, num_tiles, 4 / CT), 256, 0, stream>>>(               \
+  attn_prefill_split_kernel<HD, CT, 16, false, false, VD><<<dim3(nh * (PREFILL_RUN / 16 / CT), num_tiles), 256, 0, stream>>>( \
       (bf16_t*)out, out_stride, (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, tiles,        \
       positions, block_tables, max_blocks, 16, nh, nkv, scale * LOG2E, window, 0.f, 0.f, nullptr, 0, nullptr, 0.f, nullptr, 0, \
       (const bf16_t*)head_gate, head_gate_stride)

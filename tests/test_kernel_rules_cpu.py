@@ -80,3 +80,16 @@ def test_products_of_many_rows_take_the_operands_that_the_library_takes():
     for wrong in (a[:, :64].contiguous(), a[:, 0], a[None]):
         with pytest.raises(RuntimeError):
             Linear(w)(wrong)
+
+
+def test_runs_of_a_prompt_choose_a_kernel_that_is_built_for_them():
+    """Heads, pages and run counts of any size get an answer, and other widths and pages the kernel for any shape."""
+    route = K.library().pae_attn_prefill_route
+    assert [route(12, 128, 128, 16, -(-n // 128), n, -(-n // 16), 0) for n in (2, 128, 512, 2048, 8192)] == [0, 0, 0, 2, 4]
+    assert route(12, 192, 128, 16, 42, 5000, 60, 0) == 4 and route(12, 192, 128, 16, 1, 128, 8, 0) == 0
+    for n in (2, 600, 5000, 1 << 22):
+        assert route(14, 64, 64, 16, -(-n // 128), n, -(-n // 16), 0) in (0, 2)
+        for hd, vd, bs in ((96, 96, 16), (256, 256, 16), (128, 128, 32), (64, 64, 48), (128, 64, 16), (256, 128, 16)):
+            assert route(12, hd, vd, bs, -(-n // 128), n, -(-n // bs), 0) == 0
+        for window in (0, 1, 64, 4096):
+            assert route(1, 128, 128, 16, -(-n // 128), n, 1 << 20, window) in (0, 2, 4)
