@@ -85,9 +85,10 @@ def latent_tiles(shape: StepShape, single: int, runs: int, expand: int = 0):
     return {"single": (one, 4), "runs": ([x for _, piece in many for x in piece], 4)}
 
 
-def expanded_runs(shape: StepShape, expand: int, window: int = 0):
-    """Work lists of `kernels.lib.latent_expanded` for the sequences that bring at least `expand` tokens.  Under a `window`
-    the pages begin with the one that holds the first key the run's first token sees; the places before it stay -1."""
+def expanded_runs(shape: StepShape, expand: int, window: int = 0, piece: int = 64):
+    """Work lists of `kernels.lib.latent_expanded` for the sequences that bring at least `expand` tokens, in pieces of up to
+    `piece` <= PREFILL_TILE tokens.  Under a `window` the pages begin with the one that holds the first key the run's first
+    token sees; the places before it stay -1."""
     pages, tables, pieces = [], [], []
     for row, (start, n, past) in enumerate(zip(shape.q_starts, shape.q_lens, shape.past_lens)):
         if n < expand:
@@ -96,8 +97,8 @@ def expanded_runs(shape: StepShape, expand: int, window: int = 0):
         skipped = max(0, past - window + 1) // 16 if window else 0
         for at in range(16 * skipped, keys, 16):
             pages += [row, at, min(16, keys - at), 0]
-        for at in range(0, n, K.PREFILL_TILE):
-            count = min(K.PREFILL_TILE, n - at)
+        for at in range(0, n, piece):
+            count = min(piece, n - at)
             pieces.append((past + at + count, (len(tables), start + at, count)))
         tables.append([-1] * skipped + list(range(first, len(pages) // 4)))
     pieces.sort(key=lambda piece: -piece[0])
@@ -161,7 +162,7 @@ class LatentAttention(Part):
     def step_lists(self, shape: StepShape):
         H = self.spec.num_heads
         lists = latent_tiles(shape, K.latent_attn_tokens(H, 1), K.latent_attn_tokens(H, 2), self.expand_rows)
-        return {**lists, **expanded_runs(shape, self.expand_rows, self.spec.window or 0)} if self.expand_rows else lists
+        return {**lists, **expanded_runs(shape, self.expand_rows, self.spec.window or 0, K.PREFILL_TILE)} if self.expand_rows else lists
 
     @property
     def expand_rows(self) -> int:
