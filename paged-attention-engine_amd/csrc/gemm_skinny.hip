@@ -20,7 +20,7 @@
 // makes a round trip through memory.
 #include "common.h"
 #include "api.h"
-#include "skinny_device.h"
+#include "gemm_stream.h"
 
 // MT: column tiles of 16 rows of A; RT: tiles of 16 weight rows per workgroup; SKINNY_U: k steps
 // of a wavefront whose loads are in flight together.  With more
@@ -415,6 +415,11 @@ static int launch_skinny(int epilogue, void* out, int64_t ldc, const void* A, in
   int k_per_split = (K + splits - 1) / splits;
   k_per_split = (k_per_split + 127) / 128 * 128;
   PAE_REQUIRE((int64_t)k_per_split * (splits - 1) < K, "gemm_skinny: %d k ranges are too many for K=%d", splits, K);
+  if (const int tiles = stream_tiles(epilogue, A, W, M, N, K, lda, splits)) {
+    const StreamProduct p{epilogue, out, ldc, (const bf16_t*)A, lda, (const bf16_t*)W, bias, b_is_f32, M, N, K, k_per_split,
+                          part_stride, rope, tickets, norm};
+    return launch_stream(p, tiles, splits, stream);
+  }
   // many weight rows and more than 16 rows of A: 128 weight rows a workgroup, activations through LDS
   // (measured at 1.5B/7B/72B layer sizes: ahead from about one workgroup per compute unit on, behind below)
   const int medium_groups = (N + 127) / 128;
@@ -592,9 +597,13 @@ extern "C" int pae_gemm_skinny_gated(void* out, int64_t ldc, const void* A, int6
 // Counters and scratch floats that `splits` k ranges of an [M, K] x [N, K]^T product need for their
 // tickets, whichever kernel takes the product (one counter per wavefront that ends with whole sums of
 // its own; its accumulators for every range).
-extern "C" int pae_skinny_ticket_slots(int M, int N) { return (N + 15) / 16 * ((M + 15) / 16); }
+extern "C" int pae_skinny_ticket_slots(int M, int N) {
+  const int slots = (N + 15) / 16 * ((M + 15) / 16), stream = stream_ticket_slots(M, N);
+  return slots > stream ? slots : stream;
+}
 extern "C" int64_t pae_skinny_ticket_floats(int M, int N, int splits) {
-  return (int64_t)((N + 127) / 128) * 8 * ((M + 15) / 16) * splits * 4 * PAE_WAVE;
+  const int64_t floats = (int64_t)((N + 127) / 128) * 8 * ((M + 15) / 16) * splits * 4 * PAE_WAVE, stream = stream_ticket_floats(M, N, splits);
+  return floats > stream ? floats : stream;
 }
 
 // q_out[M, nh * hd] = rotated queries of A * W^T (+ bias), W = [(nh + 2 nkv) * hd, K] holding the

@@ -69,6 +69,7 @@ def _declare(lib) -> None:
         "pae_embedding_rows": [I, P, P, P, I, I, I, F, P, P, I, P, P],
         "pae_scaled_rows": [P, P, P, I, F, I, I, P],
         "pae_skinny_ticket_slots": [I, I],
+        "pae_stream_ranges": [I, I, I],
         "pae_gemm_skinny_act": [P, L, P, L, P, P, I, I, I, I, I, P, P, I, P],
         "pae_gemm_plain_shared": [I, I, P, L, L, P, L, L, P, L, P, I, I, I, I, I, P, P],
         "pae_gemm_skinny_gated": [P, L, P, L, P, I, I, I, I, P, P, I, P],
@@ -680,7 +681,15 @@ def skinny_splits(N: int, K: int, M: int = 1) -> int:
         if M > SAME_ORDER_MAX_ROWS and 4 <= one_round <= 8 and K // one_round >= 1024:
             wanted = one_round
     k_per = -(-(-(-K // wanted)) // 128) * 128
-    return -(-K // k_per)
+    return _streamed_splits(N, K, M, -(-K // k_per))
+
+
+def _streamed_splits(N: int, K: int, M: int, splits: int) -> int:
+    """k ranges of a product of more than 16 rows that csrc/gemm_stream.hip takes (several ranges, or many weight rows), by its
+    times; else `splits`, which suit the other kernels."""
+    if M <= SAME_ORDER_MAX_ROWS or (splits == 1 and N <= 3072):
+        return splits
+    return library().pae_stream_ranges(M, N, K) or splits
 
 
 _UNITS = 0
@@ -977,6 +986,8 @@ def whole_sum_splits(N: int, K: int, M: int) -> int:
         # 15.2 / 20.4 against 13.1 / 14.1 / 20.9; gate/up likewise at all seven widths)
         return 1
     waves = -(-(-(-N // 16)) // 256)  # wavefronts of 16 weight rows a workgroup for at most 256 workgroups
+    if 32 < M <= SKINNY_MAX_ROWS and N > 3072:
+        return _streamed_splits(N, K, M, 1)
     if 5 <= waves <= 8 and -(-(-(-N // 16)) // waves) >= 216:
         # one workgroup per compute unit, nearly all units busy: one range (the launcher then takes the
         # kernel of `waves` wavefronts; 1.5B gate/up at 32 rows 19.1 -> 16.7 us, at 64 rows 23.4 -> 22.2)
@@ -984,19 +995,21 @@ def whole_sum_splits(N: int, K: int, M: int) -> int:
     if 128 <= groups < 256:
         # a couple of workgroups of 32 weight rows per compute unit: three ranges from 32
         # rows on (1.5B gate/up at 64 rows 27.2 -> 23.3 us, at 32 rows 20.2 -> 19.0 us; below, one range is ahead)
-        return 3 if M >= 32 and K >= 1536 else 1
-    if tiles <= 96 or groups >= 384:
+        return _streamed_splits(N, K, M, 3 if M >= 32 and K >= 1536 else 1)
+    if tiles <= 96:
         return 1
+    if groups >= 384:
+        return _streamed_splits(N, K, M, 1)
     if groups >= 256:
         wanted = -(-(768 if M > 48 else 512) // groups)
         if K // wanted < 512:
-            return 1
+            return _streamed_splits(N, K, M, 1)
     else:
         # (and no more than make about a thousand 32-row workgroups: 72B QKV at 32 / 64 rows, 320 tiles, six
         # ranges 44.6 / 56.8 us, three 40.3 / 52.9)
         wanted = min(8, max(1, (K + 640) // 1280), max(1, round(1000 / tiles)))
     k_per = -(-(-(-K // wanted)) // 128) * 128
-    return -(-K // k_per)
+    return _streamed_splits(N, K, M, -(-K // k_per))
 
 
 def skinny_rope_supported(a: torch.Tensor, w: torch.Tensor, hd: int, rot: int) -> bool:

@@ -93,3 +93,21 @@ def test_runs_of_a_prompt_choose_a_kernel_that_is_built_for_them():
             assert route(12, hd, vd, bs, -(-n // 128), n, -(-n // bs), 0) == 0
         for window in (0, 1, 64, 4096):
             assert route(1, 128, 128, 16, -(-n // 128), n, 1 << 20, window) in (0, 2, 4)
+
+
+@pytest.mark.parametrize("M", [17, 32, 33, 64])
+def test_ranges_of_streamed_products_fit_their_scratch(M):
+    """Ranges of whole stages that cover k, and room for the sums of whichever count of weight tiles a workgroup takes."""
+    lib = K.library()
+    for N in (16, 896, 1536, 3072, 3080, 4608, 10240, 37888, 131072):
+        for k in (64, 896, 1536, 8960, 18944):
+            ranges = lib.pae_stream_ranges(M, N, k)
+            if not ranges:
+                continue
+            per = -(-(-(-k // ranges)) // 128) * 128
+            assert 1 <= ranges <= 8 and per * (ranges - 1) < k and (ranges > 1 or N > 3072)
+            floats, slots = lib.pae_skinny_ticket_floats(M, N, ranges), lib.pae_skinny_ticket_slots(M, N)
+            for tiles in (2, 3, 4, 5, 6, 8, 10) if M > 32 else (2, 4, 6, 8, 10):
+                groups, mine = -(-N // (16 * tiles)), -(-(tiles if M > 32 else tiles // 2) // 2)
+                assert groups * 8 <= max(slots, 8) and groups * 8 * mine * ranges * 256 <= floats
+    assert [lib.pae_stream_ranges(m, 4608, k) for m, k in ((16, 3584), (65, 3584), (64, 3592))] == [0, 0, 0]
