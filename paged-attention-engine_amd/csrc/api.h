@@ -60,23 +60,25 @@ int pae_gemm_skinny_rope(void* q_out, int64_t ldq, const void* A, int64_t lda, c
                          const int* positions, const int* tok_seq, const int* block_tables, int max_blocks, int bs,
                          void* k_cache, void* v_cache, int splits, float* ticket_parts, int* ticket_counters,
                          const float* row_stats, int row_stat_tiles, float row_eps, hipStream_t stream);
+int64_t pae_paged_attention_scratch(int dtype, const void* k_cache, const void* v_cache, int max_blocks, int bs, int num_tokens, int nh,
+                                    int nkv, int hd, int vd, int shared_kv);
 int pae_paged_attention_generic(int dtype, void* out, int64_t out_stride, const void* q, int64_t q_stride,
                                 const void* k_cache, const void* v_cache, const int* positions,
                                 const int* tok_seq, const int* block_tables, int max_blocks, int bs,
                                 int num_tokens, int nh, int nkv, int hd, float scale, int window,
-                                hipStream_t stream);
+                                float* scratch, hipStream_t stream);
 // attention with values of their own width `vd`, a cap on the scores (0: none) and per-head sinks (null: none)
 int pae_paged_attention_capped(int dtype, void* out, int64_t out_stride, const void* q, int64_t q_stride,
                                const void* k_cache, const void* v_cache, const int* positions, const int* tok_seq,
                                const int* block_tables, int max_blocks, int bs, int num_tokens, int nh, int nkv, int hd,
-                               int vd, float scale, int window, float cap, const float* sinks, hipStream_t stream);
+                               int vd, float scale, int window, float cap, const float* sinks, float* scratch, hipStream_t stream);
 // the same with a mask in chunks, a bias by distance, an output gate, and values shared with the keys
 int pae_paged_attention_masked(int dtype, void* out, int64_t out_stride, const void* q, int64_t q_stride,
                                const void* k_cache, const void* v_cache, const int* positions, const int* tok_seq,
                                const int* block_tables, int max_blocks, int bs, int num_tokens, int nh, int nkv, int hd,
                                int vd, float scale, int window, float cap, const float* sinks, int chunked,
                                const float* slopes, const void* gate, int64_t gate_stride, int gate_per_head,
-                               int shared_kv, hipStream_t stream);
+                               int shared_kv, float* scratch, hipStream_t stream);
 // a stream kept as several copies joined by hyper-connections: see hyper.hip
 int pae_hyper_norm(int dtype, float* streams, int num_streams, const void* y, int parts, int64_t part_stride,
                    const void* ls, int ls_is_f32, const float* mix, const float* outw, const float* inw,

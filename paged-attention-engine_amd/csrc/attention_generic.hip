@@ -11,10 +11,12 @@
 // j <= query position and j < kv length) plus the window, which it lacks.
 // KV head j serves query heads j*g .. (j+1)*g-1 (engine/attention.py:72-74).
 //
-// Keys are walked in chunks of 64 aligned to multiples of 64 from position 0,
-// lane = key within the chunk, with an online softmax in float32.  What a
+// Keys are taken in chunks of 64 aligned to multiples of 64 from position 0,
+// lane = key within the chunk: every chunk's weights have the chunk's largest score for their reference, and the
+// chunks' sums are added in order, in float32 (`add_chunk`).  What a
 // (token, head) computes therefore depends on nothing but its own position:
-// not on how the step was cut, nor on what else is in the batch.
+// not on how the step was cut, nor on what else is in the batch, nor on whether a workgroup walks the chunks or
+// each chunk has one of its own (few tokens at many keys: `split_chunks`).
 //
 // Three things beyond the reference's attention, each switched by a parameter: values of their own
 // width `vd` (keys and queries stay `hd` wide), a cap on the scores (s <- cap * tanh(s / cap),
@@ -30,6 +32,39 @@
 // serves as key and as value: v_cache is then not read).
 #include "common.h"
 #include "api.h"
+
+// A chunk's sums (its largest score, the sum of its weights, the weighted values) onto those of the chunks before it.
+template <int MAXD>
+__device__ __forceinline__ void add_chunk(float (&acc)[MAXD], float& m, float& l, const float (&sum)[MAXD], float m_chunk, float l_chunk) {
+  const float m_new = fmaxf(m, m_chunk);
+  const float before = expf(m - m_new), now = expf(m_chunk - m_new);  // 0 and 1 on the first chunk (m = -inf)
+  l = l * before + l_chunk * now;
+  m = m_new;
+#pragma unroll
+  for (int i = 0; i < MAXD; ++i) acc[i] = acc[i] * before + sum[i] * now;
+}
+
+// The row's output from its sums: the sink joins the denominator, then the gate.
+template <typename T, int MAXD>
+__device__ __forceinline__ void finish_row(T* __restrict__ o, const float (&acc)[MAXD], float m, float l, int vd, int lane,
+                                           const float* __restrict__ sink, const T* __restrict__ gate, int gate_per_head) {
+  float keep = 1.f;  // what the sums keep when the sink raises the reference point
+  if (sink) {
+    const float m_all = fmaxf(m, *sink);
+    keep = expf(m - m_all);
+    l = l * keep + expf(*sink - m_all);
+  }
+  const float inv = keep / l;
+#pragma unroll
+  for (int i = 0; i < MAXD; ++i) {
+    const int d = lane + i * PAE_WAVE;
+    if (d < vd) {
+      float v = acc[i] * inv;
+      if (gate) v *= 1.0f / (1.0f + expf(-to_f32(gate[gate_per_head ? 0 : d])));
+      o[d] = from_f32<T>(v);
+    }
+  }
+}
 
 template <typename T, int MAXD>  // MAXD: output features per lane, value width <= 64 * MAXD
 __global__ void paged_attention_generic_kernel(
@@ -75,17 +110,16 @@ __global__ void paged_attention_generic_kernel(
       if (slopes) s -= slope * (float)(pos - key);
       if (cap > 0.f) s = cap * tanhf(s / cap);
     }
-    const float m_new = fmaxf(m, wave_max(s));  // finite: every chunk holds a valid key
-    const float p = valid ? expf(s - m_new) : 0.f;
-    const float alpha = expf(m - m_new);        // 0 on the first chunk (m = -inf)
-    l = l * alpha + wave_sum(p);
-    m = m_new;
+    const float m_chunk = wave_max(s);  // finite: every chunk holds a valid key
+    const float p = valid ? expf(s - m_chunk) : 0.f;
+    const float l_chunk = wave_sum(p);
     p_lds[lane] = p;
     __syncthreads();
     const int first = (start > base ? start - base : 0);
     const int last = (pos - base < PAE_WAVE - 1 ? pos - base : PAE_WAVE - 1);
+    float sum[MAXD];
 #pragma unroll
-    for (int i = 0; i < MAXD; ++i) acc[i] *= alpha;
+    for (int i = 0; i < MAXD; ++i) sum[i] = 0.f;
     for (int j = first; j <= last; ++j) {
       const float pj = p_lds[j];
       const int rj = __shfl(row, j, PAE_WAVE);
@@ -96,29 +130,14 @@ __global__ void paged_attention_generic_kernel(
 #pragma unroll
       for (int i = 0; i < MAXD; ++i) {
         const int d = lane + i * PAE_WAVE;
-        if (d < vd) acc[i] = fmaf(pj, to_f32(vr[(int64_t)d * step]), acc[i]);
+        if (d < vd) sum[i] = fmaf(pj, to_f32(vr[(int64_t)d * step]), sum[i]);
       }
     }
+    add_chunk<MAXD>(acc, m, l, sum, m_chunk, l_chunk);
     __syncthreads();
   }
-  T* o = out + (int64_t)t * out_stride + (int64_t)head * vd;
-  float keep = 1.f;  // what the sums keep when the sink raises the reference point
-  if (sinks) {
-    const float sink = sinks[head];
-    const float m_all = fmaxf(m, sink);
-    keep = expf(m - m_all);
-    l = l * keep + expf(sink - m_all);
-  }
-  const float inv = keep / l;
-#pragma unroll
-  for (int i = 0; i < MAXD; ++i) {
-    const int d = lane + i * PAE_WAVE;
-    if (d < vd) {
-      float v = acc[i] * inv;
-      if (gate) v *= 1.0f / (1.0f + expf(-to_f32(gate[(int64_t)t * gate_stride + (gate_per_head ? head : (int64_t)head * vd + d)])));
-      o[d] = from_f32<T>(v);
-    }
-  }
+  finish_row<T, MAXD>(out + (int64_t)t * out_stride + (int64_t)head * vd, acc, m, l, vd, lane, sinks ? sinks + head : nullptr,
+                      gate ? gate + (int64_t)t * gate_stride + (gate_per_head ? head : (int64_t)head * vd) : nullptr, gate_per_head);
 }
 
 // The same for float32 rows that can be read four numbers at a time: a workgroup of eight wavefronts takes up to 16 (token,
@@ -133,7 +152,8 @@ __global__ void paged_attention_generic_kernel(
 // load instruction per number), and every (token, head) read the keys and values again.  Measured, 12 heads over 2
 // of 128, float32: three prompts of 601 tokens in all 262 -> 58 us, a token each behind them 92 -> 27, one prompt of 601 tokens 647 ->
 // 117, eight single tokens at 4,096 1,551 -> 338; 8 heads over 2 of 256, where six of 256 registers do not fit and lie in memory, 399 -> 77,
-// 177 -> 47, 900 -> 132, 2,534 -> 521.  What is left is the chain of a workgroup's chunks, 5 us each.  Where a workgroup has
+// 177 -> 47, 900 -> 132, 2,534 -> 521.  What is left is the chain of a workgroup's chunks, 5 us each, which few tokens share out
+// (`split_chunks`).  Where a workgroup has
 // eight rows or fewer (a token's heads, mostly) a wavefront takes one: the chain is a row's then, and registers are left to ask
 // LDS for more at once (a token at 4,096 330 -> 275 us, three at 250 25.6 -> 22.2, at heads of 64 18.6 -> 14.0; eight at 1,000, heads
 // of 256, 136 -> 114).  Loads
@@ -144,15 +164,19 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 #define PAE_ROWS_WAVES 8
 #define PAE_ROWS_EACH 2
 #define PAE_ROWS_MOST (PAE_ROWS_WAVES * PAE_ROWS_EACH)
+#define SPLIT_GROUPS 128         // up to so many workgroups' chunks are shared out
+#define SPLIT_FLOATS (16 << 20)  // numbers that their sums may take: 64 MiB
 
-template <int MAXD, int EACH>  // keys and values at most 64 * MAXD wide; rows of a wavefront: one where eight rows are all there are
+// SPLIT: blockIdx.z is the only chunk of 64 keys the workgroup looks at, and every row's sums over it go to
+// `chunk_sums` [(token, head)][chunk][vd] and `chunk_ml` [(token, head)][chunk][2], for the kernel below to add up in the order of the chunks.
+template <int MAXD, int EACH, bool SPLIT>  // keys and values at most 64 * MAXD wide; rows of a wavefront: one where eight rows are all there are
 __global__ __launch_bounds__(PAE_WAVE * PAE_ROWS_WAVES) void paged_attention_rows_kernel(
     float* __restrict__ out, int64_t out_stride, const float* __restrict__ q, int64_t q_stride,
     const float* __restrict__ k_cache, const float* __restrict__ v_cache, const int* __restrict__ positions,
     const int* __restrict__ tok_seq, const int* __restrict__ block_tables, int max_blocks, int bs, int num_tokens,
     int nh, int nkv, int hd, int vd, float scale, int window, float cap, const float* __restrict__ sinks,
     int chunked, const float* __restrict__ slopes, const float* __restrict__ gate, int64_t gate_stride,
-    int gate_per_head, int toks, int heads_each) {
+    int gate_per_head, int toks, int heads_each, float* __restrict__ chunk_sums, float* __restrict__ chunk_ml) {
   constexpr int FOURS = 16 * MAXD / PAE_ROWS_WAVES;  // that a thread brings of a chunk's keys, and of its values
   extern __shared__ float lds[];
   const int kst = hd + 4, vst = vd + 4;  // row strides that spread a quad's reads and writes over the banks
@@ -246,9 +270,13 @@ __global__ __launch_bounds__(PAE_WAVE * PAE_ROWS_WAVES) void paged_attention_row
       for (int u = 0; u < FOURS; ++u)
         v_reg[u] = *(const f32x4*)(v_cache + (((int64_t)v_page[u] * nkv + kvh) * vd + v_dim[u]) * bs + off0 + v_key[u] % span);
     };
-    const int base0 = (low / PAE_WAVE) * PAE_WAVE;
+    const int base0 = SPLIT ? blockIdx.z * PAE_WAVE : (low / PAE_WAVE) * PAE_WAVE;
+    if (SPLIT && (base0 > high || base0 + PAE_WAVE <= low)) {
+      at = next;
+      continue;
+    }
     fetch(base0);
-    for (int base = base0; base <= high; base += PAE_WAVE) {
+    for (int base = base0; SPLIT ? base == base0 : base <= high; base += PAE_WAVE) {
       __syncthreads();  // the chunk before has been read
 #pragma unroll
       for (int u = 0; u < FOURS; ++u) *(f32x4*)(k_lds + k_key[u] * kst + k_dim[u]) = k_reg[u];
@@ -261,7 +289,7 @@ __global__ __launch_bounds__(PAE_WAVE * PAE_ROWS_WAVES) void paged_attention_row
         v[3 * vst] = v_reg[u].w;
       }
       __syncthreads();
-      if (base + PAE_WAVE <= high) fetch(base + PAE_WAVE);
+      if (!SPLIT && base + PAE_WAVE <= high) fetch(base + PAE_WAVE);
       bool on[EACH];
       bool any = false, whole = true;
 #pragma unroll
@@ -293,30 +321,25 @@ __global__ __launch_bounds__(PAE_WAVE * PAE_ROWS_WAVES) void paged_attention_row
         }
       }
       const int key = base + lane;
-      float sc[EACH], m_new[EACH], p[EACH], sum[EACH];
+      float sc[EACH], m_chunk[EACH], p[EACH], l_chunk[EACH], sum[EACH][MAXD];
 #pragma unroll
       for (int i = 0; i < EACH; ++i) {
         sc[i] = dot[i] * scale;
         if (slopes) sc[i] -= slopes[head[i]] * (float)(pos[i] - key);
         if (cap > 0.f) sc[i] = cap * tanhf(sc[i] / cap);
         if (!(key >= start[i] && key <= pos[i])) sc[i] = -INFINITY;
-        m_new[i] = wave_max(sc[i]);
+        m_chunk[i] = wave_max(sc[i]);
       }
 #pragma unroll
       for (int i = 0; i < EACH; ++i) {  // the rows' reductions side by side; rows that are not on keep what they have
-        m_new[i] = fmaxf(m[i], m_new[i]);
-        p[i] = key >= start[i] && key <= pos[i] ? expf(sc[i] - m_new[i]) : 0.f;
-        sum[i] = wave_sum(p[i]);
+        p[i] = key >= start[i] && key <= pos[i] ? expf(sc[i] - m_chunk[i]) : 0.f;
+        l_chunk[i] = wave_sum(p[i]);
       }
 #pragma unroll
       for (int i = 0; i < EACH; ++i) {
-        if (!on[i]) continue;
-        const float alpha = expf(m[i] - m_new[i]);
-        l[i] = l[i] * alpha + sum[i];
-        m[i] = m_new[i];
-        p_lds[i * PAE_WAVE + lane] = p[i];
+        if (on[i]) p_lds[i * PAE_WAVE + lane] = p[i];
 #pragma unroll
-        for (int d = 0; d < MAXD; ++d) acc[i][d] *= alpha;
+        for (int d = 0; d < MAXD; ++d) sum[i][d] = 0.f;
       }
       // sums: the lane's features over the keys in order (the wavefront's own p: no barrier, its LDS operations are in order)
       __builtin_amdgcn_wave_barrier();
@@ -334,10 +357,10 @@ __global__ __launch_bounds__(PAE_WAVE * PAE_ROWS_WAVES) void paged_attention_row
             const float4 p4 = *(const float4*)(p_lds + i * PAE_WAVE + j);
 #pragma unroll
             for (int d = 0; d < MAXD; ++d) {
-              acc[i][d] = fmaf(p4.x, v[0][d], acc[i][d]);
-              acc[i][d] = fmaf(p4.y, v[1][d], acc[i][d]);
-              acc[i][d] = fmaf(p4.z, v[2][d], acc[i][d]);
-              acc[i][d] = fmaf(p4.w, v[3][d], acc[i][d]);
+              sum[i][d] = fmaf(p4.x, v[0][d], sum[i][d]);
+              sum[i][d] = fmaf(p4.y, v[1][d], sum[i][d]);
+              sum[i][d] = fmaf(p4.z, v[2][d], sum[i][d]);
+              sum[i][d] = fmaf(p4.w, v[3][d], sum[i][d]);
             }
           }
         }
@@ -349,7 +372,7 @@ __global__ __launch_bounds__(PAE_WAVE * PAE_ROWS_WAVES) void paged_attention_row
           auto add = [&](int j, float p) {
 #pragma unroll
             for (int d = 0; d < MAXD; ++d)
-              if (lane + d * PAE_WAVE < vd) acc[i][d] = fmaf(p, v_lds[j * vst + lane + d * PAE_WAVE], acc[i][d]);
+              if (lane + d * PAE_WAVE < vd) sum[i][d] = fmaf(p, v_lds[j * vst + lane + d * PAE_WAVE], sum[i][d]);
           };
           int j = first;
 #pragma unroll 1
@@ -364,41 +387,71 @@ __global__ __launch_bounds__(PAE_WAVE * PAE_ROWS_WAVES) void paged_attention_row
               for (int d = 0; d < MAXD; ++d) v[u][d] = v_lds[(j + u) * vst + min(lane + d * PAE_WAVE, vd - 1)];
 #pragma unroll
             for (int d = 0; d < MAXD; ++d) {
-              acc[i][d] = fmaf(p4.x, v[0][d], acc[i][d]);
-              acc[i][d] = fmaf(p4.y, v[1][d], acc[i][d]);
-              acc[i][d] = fmaf(p4.z, v[2][d], acc[i][d]);
-              acc[i][d] = fmaf(p4.w, v[3][d], acc[i][d]);
+              sum[i][d] = fmaf(p4.x, v[0][d], sum[i][d]);
+              sum[i][d] = fmaf(p4.y, v[1][d], sum[i][d]);
+              sum[i][d] = fmaf(p4.z, v[2][d], sum[i][d]);
+              sum[i][d] = fmaf(p4.w, v[3][d], sum[i][d]);
             }
           }
 #pragma unroll 1
           for (; j <= last; ++j) add(j, p_lds[i * PAE_WAVE + j]);
         }
       }
+#pragma unroll
+      for (int i = 0; i < EACH; ++i) {
+        if (!on[i]) continue;
+        if (!SPLIT) {
+          add_chunk<MAXD>(acc[i], m[i], l[i], sum[i], m_chunk[i], l_chunk[i]);
+          continue;
+        }
+        const int64_t part = ((int64_t)tok[i] * nh + head[i]) * gridDim.z + blockIdx.z;
+        if (lane == 0) *reinterpret_cast<float2*>(chunk_ml + 2 * part) = make_float2(m_chunk[i], l_chunk[i]);
+#pragma unroll
+        for (int d = 0; d < MAXD; ++d)
+          if (lane + d * PAE_WAVE < vd) chunk_sums[part * vd + lane + d * PAE_WAVE] = sum[i][d];
+      }
     }
     at = next;
   }
+  if (SPLIT) return;
 #pragma unroll
-  for (int i = 0; i < EACH; ++i) {
-    if (!live[i]) continue;
-    float* o = out + (int64_t)tok[i] * out_stride + (int64_t)head[i] * vd;
-    float keep = 1.f;
-    if (sinks) {
-      const float sink = sinks[head[i]];
-      const float m_all = fmaxf(m[i], sink);
-      keep = expf(m[i] - m_all);
-      l[i] = l[i] * keep + expf(sink - m_all);
-    }
-    const float inv = keep / l[i];
+  for (int i = 0; i < EACH; ++i)
+    if (live[i])
+      finish_row<float, MAXD>(out + (int64_t)tok[i] * out_stride + (int64_t)head[i] * vd, acc[i], m[i], l[i], vd, lane, sinks ? sinks + head[i] : nullptr,
+                              gate ? gate + (int64_t)tok[i] * gate_stride + (gate_per_head ? head[i] : (int64_t)head[i] * vd) : nullptr, gate_per_head);
+}
+
+// A row's chunks, added in their order as the kernels above add them: one wavefront per (token, query head), eight chunks'
+// sums on their way together.
+template <int MAXD>
+__global__ __launch_bounds__(PAE_WAVE) void paged_attention_chunks_kernel(
+    float* __restrict__ out, int64_t out_stride, const float* __restrict__ chunk_sums, const float* __restrict__ chunk_ml, int chunks,
+    const int* __restrict__ positions, int nh, int vd, int window, const float* __restrict__ sinks, int chunked,
+    const float* __restrict__ gate, int64_t gate_stride, int gate_per_head) {
+  constexpr int AHEAD = 8;
+  const int t = blockIdx.x, head = blockIdx.y, lane = threadIdx.x, pos = positions[t];
+  const int start = window <= 0 ? 0 : (chunked ? pos - pos % window : (pos - window + 1 > 0 ? pos - window + 1 : 0));
+  const int64_t row = ((int64_t)t * nh + head) * chunks;
+  const int last = pos < 0 ? -1 : pos / PAE_WAVE;
+  float acc[MAXD], m = -INFINITY, l = 0.f;
 #pragma unroll
-    for (int d = 0; d < MAXD; ++d) {
-      const int f = lane + d * PAE_WAVE;
-      if (f < vd) {
-        float v = acc[i][d] * inv;
-        if (gate) v *= 1.0f / (1.0f + expf(-gate[(int64_t)tok[i] * gate_stride + (gate_per_head ? head[i] : (int64_t)head[i] * vd + f)]));
-        o[f] = v;
-      }
+  for (int i = 0; i < MAXD; ++i) acc[i] = 0.f;
+  for (int c0 = start / PAE_WAVE; c0 <= last; c0 += AHEAD) {
+    float2 ml[AHEAD];
+    float sum[AHEAD][MAXD];
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+      const int64_t part = row + min(c0 + u, last);
+      ml[u] = *reinterpret_cast<const float2*>(chunk_ml + 2 * part);
+#pragma unroll
+      for (int i = 0; i < MAXD; ++i) sum[u][i] = chunk_sums[part * vd + min(lane + i * PAE_WAVE, vd - 1)];
     }
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u)
+      if (c0 + u <= last) add_chunk<MAXD>(acc, m, l, sum[u], ml[u].x, ml[u].y);
   }
+  finish_row<float, MAXD>(out + (int64_t)t * out_stride + (int64_t)head * vd, acc, m, l, vd, lane, sinks ? sinks + head : nullptr,
+                          gate ? gate + (int64_t)t * gate_stride + (gate_per_head ? head : (int64_t)head * vd) : nullptr, gate_per_head);
 }
 
 // Whether the rows kernel takes a call: rows and pages that can be read four numbers at a time, and a chunk's keys and values
@@ -408,33 +461,62 @@ static bool rows_kernel_takes(const void* k_cache, const void* v_cache, int bs, 
          hd <= 256 && (uintptr_t)k_cache % 16 == 0 && (uintptr_t)v_cache % 16 == 0;
 }
 
+// Tokens that share a workgroup's keys, its heads of each, and the parts of a key/value head's query heads.  Several tokens where
+// there are workgroups enough (decode steps: a token each).
+static int rows_of_a_workgroup(int num_tokens, int nh, int nkv, int& heads_each, int& parts) {
+  const int g = nh / nkv;
+  heads_each = g < PAE_ROWS_MOST ? g : PAE_ROWS_MOST;
+  parts = (g + heads_each - 1) / heads_each;
+  return (int64_t)num_tokens * nkv * parts >= 512 ? PAE_ROWS_MOST / heads_each : 1;
+}
+
+// Chunks of keys that get workgroups of their own, or 1: a workgroup walks them.  Shared out where the walks would leave most of the
+// chip idle and the chunks are three or more (a token at 60 keys 9.5 and 11.3; 14 heads of 64 at 75 about 8 and 9): 12 heads over 2 of
+// 128, in us, walked and shared: three tokens at 200 keys 20.7 and 12.1, eight at 1,000 71 and 13.4, at
+// 4,000 278 and 49, 64 at 1,000 77 and 71 (128 workgroups), 40 tokens behind 2,000 142 and 85 (80); but a prompt of 200 tokens (400)
+// 33 and 44, 600 tokens 111 and 173: a workgroup's start and end, 5 us, then come once a chunk.
+static int split_chunks(int num_tokens, int nh, int nkv, int vd, int max_blocks, int bs) {
+  int heads_each, parts;
+  const int toks = rows_of_a_workgroup(num_tokens, nh, nkv, heads_each, parts);
+  const int64_t chunks = ((int64_t)max_blocks * bs + PAE_WAVE - 1) / PAE_WAVE;
+  const int64_t groups = (int64_t)((num_tokens + toks - 1) / toks) * nkv * parts;
+  if (chunks < 3 || chunks > 65535 || groups > SPLIT_GROUPS || (int64_t)num_tokens * nh * chunks * (vd + 2) > SPLIT_FLOATS) return 1;
+  return (int)chunks;
+}
+
 static int launch_rows(float* out, int64_t out_stride, const float* q, int64_t q_stride, const float* k_cache,
                        const float* v_cache, const int* positions, const int* tok_seq, const int* block_tables,
                        int max_blocks, int bs, int num_tokens, int nh, int nkv, int hd, int vd, float scale, int window,
                        float cap, const float* sinks, int chunked, const float* slopes, const float* gate,
-                       int64_t gate_stride, int gate_per_head, hipStream_t stream) {
-  const int g = nh / nkv;
-  const int heads_each = g < PAE_ROWS_MOST ? g : PAE_ROWS_MOST;
-  const int parts = (g + heads_each - 1) / heads_each;
-  // several tokens share a workgroup's keys where there are workgroups enough (decode steps: a token each)
-  const int toks = (int64_t)num_tokens * nkv * parts >= 512 ? PAE_ROWS_MOST / heads_each : 1;
-  const dim3 grid((num_tokens + toks - 1) / toks, nkv * parts);
+                       int64_t gate_stride, int gate_per_head, float* scratch, hipStream_t stream) {
+  int heads_each, parts;
+  const int toks = rows_of_a_workgroup(num_tokens, nh, nkv, heads_each, parts);
+  const int chunks = scratch ? split_chunks(num_tokens, nh, nkv, vd, max_blocks, bs) : 1;
+  float* part_ml = scratch;
+  float* part_sums = scratch ? scratch + (int64_t)2 * num_tokens * nh * chunks : nullptr;
+  const dim3 grid((num_tokens + toks - 1) / toks, nkv * parts, chunks);
   const size_t lds = (size_t)(PAE_WAVE * (hd + 4 + vd + 4) + PAE_ROWS_MOST * (PAE_WAVE + hd)) * sizeof(float);
-#define PAE_LAUNCH_EACH(MAXD, EACH)                                                                                   \
+#define PAE_LAUNCH_EACH(MAXD, EACH, SPLIT)                                                                            \
   do {                                                                                                                \
     if (lds > 65536) {                                                                                                \
-      const hipError_t err = hipFuncSetAttribute((const void*)paged_attention_rows_kernel<MAXD, EACH>,                \
+      const hipError_t err = hipFuncSetAttribute((const void*)paged_attention_rows_kernel<MAXD, EACH, SPLIT>,         \
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);               \
       if (err != hipSuccess) return pae_fail("attention: %zu bytes of LDS refused: %s", lds, hipGetErrorString(err)); \
     }                                                                                                                 \
-    paged_attention_rows_kernel<MAXD, EACH><<<grid, PAE_WAVE * PAE_ROWS_WAVES, lds, stream>>>(                        \
+    paged_attention_rows_kernel<MAXD, EACH, SPLIT><<<grid, PAE_WAVE * PAE_ROWS_WAVES, lds, stream>>>(                 \
         out, out_stride, q, q_stride, k_cache, v_cache, positions, tok_seq, block_tables, max_blocks, bs, num_tokens, \
-        nh, nkv, hd, vd, scale, window, cap, sinks, chunked, slopes, gate, gate_stride, gate_per_head, toks, heads_each); \
+        nh, nkv, hd, vd, scale, window, cap, sinks, chunked, slopes, gate, gate_stride, gate_per_head, toks, heads_each, \
+        part_sums, part_ml);                                                                                          \
   } while (0)
-#define PAE_LAUNCH(MAXD)                                                     \
-  do {                                                                       \
-    if (toks * heads_each <= PAE_ROWS_WAVES) PAE_LAUNCH_EACH(MAXD, 1);       \
-    else PAE_LAUNCH_EACH(MAXD, PAE_ROWS_EACH);                               \
+#define PAE_LAUNCH(MAXD)                                                                                              \
+  do {                                                                                                                \
+    if (chunks > 1) {                                                                                                 \
+      if (toks * heads_each <= PAE_ROWS_WAVES) PAE_LAUNCH_EACH(MAXD, 1, true);                                        \
+      else PAE_LAUNCH_EACH(MAXD, PAE_ROWS_EACH, true);                                                                \
+      paged_attention_chunks_kernel<MAXD><<<dim3(num_tokens, nh), PAE_WAVE, 0, stream>>>(                             \
+          out, out_stride, part_sums, part_ml, chunks, positions, nh, vd, window, sinks, chunked, gate, gate_stride, gate_per_head); \
+    } else if (toks * heads_each <= PAE_ROWS_WAVES) PAE_LAUNCH_EACH(MAXD, 1, false);                                  \
+    else PAE_LAUNCH_EACH(MAXD, PAE_ROWS_EACH, false);                                                                 \
   } while (0)
   const int wide = hd > vd ? hd : vd;
   if (wide <= 64) PAE_LAUNCH(1);
@@ -469,6 +551,16 @@ static int launch_generic(void* out, int64_t out_stride, const void* q, int64_t 
   return pae_check_launch("paged_attention_generic");
 }
 
+// Floats of scratch for the calls below (16-byte aligned), 0: none is used.  Without it a workgroup walks its chunks; the bits are the same.
+extern "C" int64_t pae_paged_attention_scratch(int dtype, const void* k_cache, const void* v_cache, int max_blocks, int bs, int num_tokens,
+                                               int nh, int nkv, int hd, int vd, int shared_kv) {
+  if (dtype != PAE_F32 || num_tokens <= 0 || nh <= 0 || nkv <= 0 || nh % nkv || nkv > 65535 || bs <= 0 || vd <= 0 ||
+      !rows_kernel_takes(k_cache, v_cache, bs, hd, vd, shared_kv))
+    return 0;
+  const int chunks = split_chunks(num_tokens, nh, nkv, vd, max_blocks, bs);
+  return chunks > 1 ? (int64_t)num_tokens * nh * chunks * (vd + 2) : 0;
+}
+
 extern "C" int pae_paged_attention_masked(int dtype, void* out, int64_t out_stride, const void* q,
                                           int64_t q_stride, const void* k_cache, const void* v_cache,
                                           const int* positions, const int* tok_seq,
@@ -476,7 +568,7 @@ extern "C" int pae_paged_attention_masked(int dtype, void* out, int64_t out_stri
                                           int num_tokens, int nh, int nkv, int hd, int vd, float scale,
                                           int window, float cap, const float* sinks, int chunked,
                                           const float* slopes, const void* gate, int64_t gate_stride, int gate_per_head,
-                                          int shared_kv, hipStream_t stream) {
+                                          int shared_kv, float* scratch, hipStream_t stream) {
   PAE_REQUIRE(nh > 0 && nkv > 0 && nh % nkv == 0, "attention: %d query heads over %d key/value heads", nh, nkv);
   PAE_REQUIRE(hd > 0 && hd <= 1024, "attention: head_dim %d is outside 1..1024", hd);
   PAE_REQUIRE(vd > 0 && vd <= 512, "attention: value width %d is outside 1..512", vd);
@@ -491,7 +583,7 @@ extern "C" int pae_paged_attention_masked(int dtype, void* out, int64_t out_stri
   if (dtype == PAE_F32 && rows_kernel_takes(k_cache, v_cache, bs, hd, vd, shared_kv) && nkv <= 65535)
     return launch_rows((float*)out, out_stride, (const float*)q, q_stride, (const float*)k_cache, (const float*)v_cache, positions,
                        tok_seq, block_tables, max_blocks, bs, num_tokens, nh, nkv, hd, vd, scale, window, cap, sinks, chunked,
-                       slopes, (const float*)gate, gate_stride, gate_per_head, stream);
+                       slopes, (const float*)gate, gate_stride, gate_per_head, scratch, stream);
   if (dtype == PAE_F32)
     return launch_generic<float>(out, out_stride, q, q_stride, k_cache, v_cache, positions, tok_seq, block_tables,
                                  max_blocks, bs, num_tokens, nh, nkv, hd, vd, scale, window, cap, sinks, chunked, slopes, gate,
@@ -508,11 +600,11 @@ extern "C" int pae_paged_attention_capped(int dtype, void* out, int64_t out_stri
                                           const int* positions, const int* tok_seq,
                                           const int* block_tables, int max_blocks, int bs,
                                           int num_tokens, int nh, int nkv, int hd, int vd, float scale,
-                                          int window, float cap, const float* sinks, hipStream_t stream) {
+                                          int window, float cap, const float* sinks, float* scratch, hipStream_t stream) {
   PAE_REQUIRE(vd > 0 && vd <= 256, "attention: value width %d is outside 1..256", vd);
   return pae_paged_attention_masked(dtype, out, out_stride, q, q_stride, k_cache, v_cache, positions, tok_seq,
                                     block_tables, max_blocks, bs, num_tokens, nh, nkv, hd, vd, scale, window, cap, sinks,
-                                    0, nullptr, nullptr, 0, 0, 0, stream);
+                                    0, nullptr, nullptr, 0, 0, 0, scratch, stream);
 }
 
 extern "C" int pae_paged_attention_generic(int dtype, void* out, int64_t out_stride, const void* q,
@@ -520,9 +612,9 @@ extern "C" int pae_paged_attention_generic(int dtype, void* out, int64_t out_str
                                            const int* positions, const int* tok_seq,
                                            const int* block_tables, int max_blocks, int bs,
                                            int num_tokens, int nh, int nkv, int hd, float scale,
-                                           int window, hipStream_t stream) {
+                                           int window, float* scratch, hipStream_t stream) {
   PAE_REQUIRE(hd > 0 && hd <= 256, "attention: head_dim %d is outside 1..256", hd);
   return pae_paged_attention_capped(dtype, out, out_stride, q, q_stride, k_cache, v_cache, positions, tok_seq,
                                     block_tables, max_blocks, bs, num_tokens, nh, nkv, hd, hd, scale, window, 0.f,
-                                    nullptr, stream);
+                                    nullptr, scratch, stream);
 }

@@ -65,7 +65,8 @@ class StepRunner:
     no real sequence ever holds), so it reads and writes nothing that anyone looks at; its
     logits are dropped."""
 
-    TABLE_ROUND = 64    # block tables of captured steps are padded to a multiple of this many pages
+    TABLE_ROUND = 64    # block tables of captured steps are padded to a multiple of this many pages,
+    SHORT_CONTEXT = 128  # but those of sequences up to so many tokens to this: kernels that share out keys then see that they are few
     MAX_GRAPHS = 24
 
     def __init__(self, model: Model, cache: CacheManager, use_graphs: bool = True,
@@ -205,7 +206,8 @@ class StepRunner:
         for tables in per_group:
             width = max(1, max(len(t) for t in tables))
             if decode_only:
-                width = -(-width // self.TABLE_ROUND) * self.TABLE_ROUND
+                short = max(1, self.SHORT_CONTEXT // cache.block_size)
+                width = short if width <= short else -(-width // self.TABLE_ROUND) * self.TABLE_ROUND
             widths.append(width)
 
         # index lists that parts asked for (their kernels' work lists), built from the step's shape

@@ -73,10 +73,10 @@ def _declare(lib) -> None:
         "pae_gemm_skinny_act": [P, L, P, L, P, P, I, I, I, I, I, P, P, I, P],
         "pae_gemm_plain_shared": [I, I, P, L, L, P, L, L, P, L, P, I, I, I, I, I, P, P],
         "pae_gemm_skinny_gated": [P, L, P, L, P, I, I, I, I, P, P, I, P],
-        "pae_paged_attention_generic": [I, P, L, P, L, P, P, P, P, P, I, I, I, I, I, I, F, I, P],
-        "pae_paged_attention_capped": [I, P, L, P, L, P, P, P, P, P, I, I, I, I, I, I, I, F, I, F, P, P],
+        "pae_paged_attention_generic": [I, P, L, P, L, P, P, P, P, P, I, I, I, I, I, I, F, I, P, P],
+        "pae_paged_attention_capped": [I, P, L, P, L, P, P, P, P, P, I, I, I, I, I, I, I, F, I, F, P, P, P],
         "pae_qk_norm_rotate_store": [I, P, L, I, I, I, I, I, P, P, I, F, I, I, P, F, P, P, P, I, I, P, P, I, I, F, I, P, L, F, P],
-        "pae_paged_attention_masked": [I, P, L, P, L, P, P, P, P, P, I, I, I, I, I, I, I, F, I, F, P, I, P, P, L, I, I, P],
+        "pae_paged_attention_masked": [I, P, L, P, L, P, P, P, P, P, I, I, I, I, I, I, I, F, I, F, P, I, P, P, L, I, I, P, P],
         "pae_hyper_norm": [I, P, I, P, I, L, P, I, P, P, P, P, I, F, P, P, I, I, I, P],
         "pae_hyper_spread": [P, P, I, I, I, P],
         "pae_hyper_collapse": [P, P, I, I, I, P],
@@ -157,6 +157,8 @@ def _declare(lib) -> None:
         fn.restype = c_int
     lib.pae_skinny_ticket_floats.argtypes = [I, I, I]
     lib.pae_skinny_ticket_floats.restype = c_int64
+    lib.pae_paged_attention_scratch.argtypes = [I, P, P, I, I, I, I, I, I, I, I]
+    lib.pae_paged_attention_scratch.restype = c_int64
     lib.pae_gemm_plain_scratch.argtypes = [I, I, I]
     lib.pae_gemm_plain_scratch.restype = c_int64
     lib.pae_gemm_plain_part.argtypes = [I, I, I, I, P]
@@ -1149,7 +1151,20 @@ def paged_attention_generic(out: torch.Tensor, q: torch.Tensor, k_cache: torch.T
     _check(library().pae_paged_attention_generic(
         code_of(q.dtype), out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0), k_cache.data_ptr(),
         v_cache.data_ptr(), positions.data_ptr(), tok_seq.data_ptr(), block_tables.data_ptr(),
-        block_tables.shape[1], bs, T, nh, nkv, hd, float(scale), int(window), _stream()))
+        block_tables.shape[1], bs, T, nh, nkv, hd, float(scale), int(window),
+        _ptr(_attention_scratch(q, k_cache, v_cache, block_tables, bs, nh, nkv, hd, hd)), _stream()))
+
+
+ATTENTION_SPLIT_GROUPS = 128  # workgroups whose chunks of keys are shared out, at most (a token and key/value head has one or more)
+
+
+def _attention_scratch(q, k_cache, v_cache, block_tables, bs: int, nh: int, nkv: int, hd: int, vd: int) -> Optional[torch.Tensor]:
+    """Room for the sums over chunks of keys, where the attention kernels for any shape share a row's chunks out (else None)."""
+    if q.dtype != torch.float32 or q.shape[0] * nkv > ATTENTION_SPLIT_GROUPS or block_tables.shape[1] * bs <= 128:
+        return None  # what the library would say, without the call
+    floats = library().pae_paged_attention_scratch(code_of(q.dtype), k_cache.data_ptr(), _ptr(v_cache), block_tables.shape[1], bs,
+                                                   q.shape[0], nh, nkv, hd, vd, 1 if v_cache is None else 0)
+    return torch.empty(floats, dtype=torch.float32, device=q.device) if floats else None
 
 
 def _check_pools_wide(k_cache, v_cache, nkv: int, bs: int, hd: int, vd: int) -> None:
@@ -1182,7 +1197,7 @@ def paged_attention_capped(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Te
         code_of(q.dtype), out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0), k_cache.data_ptr(),
         v_cache.data_ptr(), positions.data_ptr(), tok_seq.data_ptr(), block_tables.data_ptr(),
         block_tables.shape[1], bs, T, nh, nkv, hd, vd, float(scale), int(window), float(softcap), _ptr(sinks),
-        _stream()))
+        _ptr(_attention_scratch(q, k_cache, v_cache, block_tables, bs, nh, nkv, hd, vd)), _stream()))
 
 
 def _check_head_gate(gate: torch.Tensor, q: torch.Tensor, nh: int) -> None:
@@ -1233,7 +1248,7 @@ def paged_attention_masked(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Te
         _ptr(v_cache), positions.data_ptr(), tok_seq.data_ptr(), block_tables.data_ptr(),
         block_tables.shape[1], bs, T, nh, nkv, hd, vd, float(scale), int(window), float(softcap), _ptr(sinks),
         1 if chunked else 0, _ptr(slopes), _ptr(gate), gate_stride, 1 if head_gate is not None else 0,
-        1 if v_cache is None else 0, _stream()))
+        1 if v_cache is None else 0, _ptr(_attention_scratch(q, k_cache, v_cache, block_tables, bs, nh, nkv, hd, vd)), _stream()))
 
 
 def conv_norm_store(proj: torch.Tensor, q_out: torch.Tensor, tok_seq: torch.Tensor, positions: torch.Tensor,

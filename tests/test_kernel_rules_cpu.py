@@ -111,3 +111,17 @@ def test_ranges_of_streamed_products_fit_their_scratch(M):
                 groups, mine = -(-N // (16 * tiles)), -(-(tiles if M > 32 else tiles // 2) // 2)
                 assert groups * 8 <= max(slots, 8) and groups * 8 * mine * ranges * 256 <= floats
     assert [lib.pae_stream_ranges(m, 4608, k) for m, k in ((16, 3584), (65, 3584), (64, 3592))] == [0, 0, 0]
+
+
+@pytest.mark.parametrize("T,nh,nkv,hd,vd,blocks,bs", [(1, 12, 2, 128, 128, 64, 16), (64, 12, 2, 128, 128, 64, 16), (65, 12, 2, 128, 128, 64, 16),
+                                                      (3, 40, 1, 64, 64, 5, 16), (8, 16, 16, 64, 200, 3, 64), (1, 1, 1, 4, 4, 8, 16), (2, 8, 2, 256, 256, 6000, 16)])
+def test_scratch_of_shared_out_chunks(T, nh, nkv, hd, vd, blocks, bs):
+    """Every chunk's sums have room, within 64 MiB; what is not asked of the library has none; other types and pools use none."""
+    scratch = lambda *args: K.library().pae_paged_attention_scratch(*args)
+    floats, chunks = scratch(0, 256, 512, blocks, bs, T, nh, nkv, hd, vd, 0), -(-blocks * bs // 64)
+    assert floats in (0, T * nh * chunks * (vd + 2)) and floats <= 16 << 20
+    if T * nkv > K.ATTENTION_SPLIT_GROUPS or blocks * bs <= 128:
+        assert floats == 0
+    assert scratch(1, 256, 512, blocks, bs, T, nh, nkv, hd, vd, 0) == scratch(0, 260, 512, blocks, bs, T, nh, nkv, hd, vd, 0) == 0
+    assert scratch(0, 256, None, blocks, bs, T, nh, 1, hd, vd, 1) == 0
+    assert K.library().pae_paged_attention_scratch(0, 256, 512, 64, 16, 3, 12, 2, 128, 128, 0) == 3 * 12 * 16 * 130
