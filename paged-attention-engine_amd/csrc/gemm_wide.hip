@@ -3,7 +3,7 @@
 //
 // A launch is either the tiles of 256 x 256 as long as they fill rounds of the chip's 256 compute units, then what is left over
 // of them whole, in halves or in quarters, where these still make one round; or, where that leaves too many units
-// idle, smaller tiles throughout, whose k may be cut into ranges that leave float32 sums of their own.  Which one is the
+// idle, smaller tiles throughout; and of either k may be cut into ranges that leave float32 sums of their own.  Which one is the
 // least of what the shapes' measured times say (pae_gemm_wide_plan).
 //
 // Measured beside the platform library's product (weights from memory, us; rows x features x k):
@@ -13,6 +13,9 @@
 //     6,030 x 37,888 x  3,584        1,209 and 117 for the gate              1,176 with the gate
 //     6,030 x  3,584 x 18,944        1,041                                   600
 //       601 x  1,536 x  8,960           36                                   24 in three ranges of k
+//   With the norm that adds the ranges' sums, before them and now in tiles of 256 x 256 too:
+//     2,048 x  1,536 x  8,960           77.7                                 69.4 in five ranges
+//     2,500 x  2,048 x 11,008          134                                  107 in three
 //       200 x  1,536 x  1,536           20                                   8
 #include "wide_gemm.h"
 #include "api.h"
@@ -181,11 +184,18 @@ __global__ __launch_bounds__(512, 2) void wide_large_kernel(Product p) {
     small_tile<MODE, ACT, typename std::conditional<PARTS == 4, Quarter, Half>::type>(p, wide_lds, m0, n0, 0, p.stages, 0);
     return;
   }
-  place_of(in_row(blockIdx.x, p.whole), p.row_tiles, p.col_tiles, p.strip, tm, tn);
+  int id = in_row(blockIdx.x, MODE == wide_gemm::SUMS ? p.whole * p.splits : p.whole), split = 0, first = 0, stages = p.stages;
+  if (MODE == wide_gemm::SUMS) {  // the ranges of k lie one after another
+    split = id / p.whole;
+    id -= split * p.whole;
+    first = (int)((int64_t)p.stages * split / p.splits);
+    stages = (int)((int64_t)p.stages * (split + 1) / p.splits) - first;
+  }
+  place_of(id, p.row_tiles, p.col_tiles, p.strip, tm, tn);
   const int m0 = tm * 256, n0 = tn * 256;
   Large::Source src;
-  src.a = p.a + m0 * p.lda;
-  src.w = p.w + n0 * p.ldw;
+  src.a = p.a + m0 * p.lda + (int64_t)first * wide_gemm::ROW_BYTES;
+  src.w = p.w + n0 * p.ldw + (int64_t)first * wide_gemm::ROW_BYTES;
 #pragma unroll
   for (int h = 0; h < 2; ++h)
 #pragma unroll
@@ -199,8 +209,8 @@ __global__ __launch_bounds__(512, 2) void wide_large_kernel(Product p) {
   for (int i = 0; i < Large::MT; ++i)
 #pragma unroll
     for (int x = 0; x < Large::X; ++x) acc[i][x] = f32x4{0.f, 0.f, 0.f, 0.f};
-  Large::run(acc, wide_lds, src, p.stages);
-  finish<MODE, ACT>(p, acc, m0 + wave / Large::WN * Large::PM, n0 + wave % Large::WN * Large::PN, 0);
+  Large::run(acc, wide_lds, src, stages);
+  finish<MODE, ACT>(p, acc, m0 + wave / Large::WN * Large::PM, n0 + wave % Large::WN * Large::PN, split);
 }
 
 // One shape of smaller tiles throughout; the ranges of k lie one after another.  (Never all 512 registers for a wavefront: the
@@ -243,6 +253,11 @@ int launch_large(Product p, hipStream_t stream) {
   p.strip = 8;
   const int64_t tiles = (int64_t)p.row_tiles * p.col_tiles;
   PAE_REQUIRE(tiles < (1ll << 28), "wide product: too many tiles");
+  if constexpr (MODE == wide_gemm::SUMS) {
+    p.whole = (int)tiles;
+    PAE_REQUIRE(tiles * p.splits < (1ll << 30), "wide product: too many tiles");
+    return launch(wide_large_kernel<MODE, ACT, 1>, p, tiles * p.splits, 512, Large::LDS_BYTES, stream);
+  }
   const int rest = (int)(tiles % UNITS), parts = rest == 0 || rest > UNITS / 2 ? 1 : rest > UNITS / 4 ? 2 : 4;
   p.whole = (int)(parts == 1 ? tiles : tiles - rest);
   constexpr int LDS = Large::LDS_BYTES > Half::LDS_BYTES ? Large::LDS_BYTES : Half::LDS_BYTES;
@@ -259,6 +274,10 @@ enum { SHAPE_LARGE, SHAPE_128_256, SHAPE_128_128, SHAPE_128_96, SHAPE_64_128, SH
 // stage.  The shapes of two workgroups a unit take a quarter longer a stage from 2,048 of k on, with weights from memory (64 x 64 at up
 // to one a unit: 0.16 to 0.20 up to k 1,536, 0.24 to 0.26 from 2,048 to 18,944; 64 x 128 0.32 and 0.40 to 0.43).  The least of all is on
 // average 1 % behind the fastest shape (300 x 4,608 x 3,584 24.8 us; without that quarter 64 x 128 was taken, 28.1).
+// Ranges of k in tiles of 256 x 256: 1.15 us a stage where all tiles are one round and 1.45 behind that, where the chip's clock has gone down; with
+// the norm that adds the ranges' sums, at 7 widths by 15 row counts, the choice is 1.1 % behind the fastest (in us, without such tiles and with them:
+// 2,048 x 1,536 x 8,960 77.7 and 69.4 in five ranges, 3,000 x 1,536 x 8,960 111 and 90, 4,096 x 1,536 x 8,960 139 and 114, 2,500 x 2,048 x 11,008 134
+// and 107, 1,000 x 3,584 x 18,944 147 and 131, 2,048 x 3,584 x 18,944 269 and 234; but 6,000 x 3,584 x 18,944 681 whole and 702).
 double shape_time(int shape, int M, int N, int K, int splits) {
   const double stages = K / 64.0 / splits;
   struct Cost { int bm, bn, blocks; double launch, round, stage, part; };  // part: a stage of a last round that half the units' places or fewer take
@@ -269,6 +288,7 @@ double shape_time(int shape, int M, int N, int K, int splits) {
   const int64_t tiles = tiles_of(M, N, c.bm, c.bn) * splits, places = (int64_t)UNITS * c.blocks;
   const int64_t rest = tiles % places;
   double last = 0.0;
+  if (shape == SHAPE_LARGE && splits > 1) return (tiles + UNITS - 1) / UNITS * (c.round + stages * (tiles <= UNITS ? 1.15 : 1.45));
   if (rest) last = c.round + stages * (shape == SHAPE_LARGE ? (rest > UNITS / 2 ? c.stage : rest > UNITS / 4 ? 0.77 : 0.40) : far * (rest > places / 2 ? c.stage : c.part));
   return c.launch + tiles / places * (c.round + stages * far * c.stage) + last;
 }
@@ -277,9 +297,7 @@ template <int MODE, int ACT>
 int run_shape(int shape, const Product& p, hipStream_t stream) {
   constexpr bool PAIRS = MODE == wide_gemm::GATED;
   switch (shape) {
-    case SHAPE_LARGE:
-      if constexpr (MODE != wide_gemm::SUMS) return launch_large<MODE, ACT>(p, stream);
-      break;
+    case SHAPE_LARGE: return launch_large<MODE, ACT>(p, stream);
     case SHAPE_128_256: return launch_small<MODE, ACT, Tile<128, 256, 2, 4, 3>>(p, stream);
     case SHAPE_128_128: return launch_small<MODE, ACT, Tile<128, 128, 2, 2, 4>>(p, stream);
     case SHAPE_128_96:
@@ -294,7 +312,7 @@ int run_shape(int shape, const Product& p, hipStream_t stream) {
 }  // namespace
 
 // The shape for a product, in the low byte, and its ranges of k behind that.  `mode` as for pae_gemm_wide; `ranges` != 0: the
-// product may leave float32 sums of ranges of k for a caller that reads them again (counted at 4.5 TB/s against one bfloat16
+// product may leave float32 sums of ranges of k for a caller that reads them again (counted at 3.6 TB/s against one bfloat16
 // result).  -1: the platform library, which shares a product out over k, for one without an activation that no shape here fills
 // the chip with.  That is from 30 us on and below 0.95 PFLOP/s by the times above, where the library was ahead of
 // these shapes two times in three (6,030 x 1,536 x 8,960 141 against 160 us, 2,048 x 4,608 x 3,584 59 against 68); and from 48 stages of k
@@ -303,7 +321,7 @@ int run_shape(int shape, const Product& p, hipStream_t stream) {
 // us, 300 x 256 x 4,096 18.6 against 11.2, 65 x 16 x 8,192 22.4 against 8.3).  Up to 35 stages as few tiles are ahead (65 x 1,536 x 2,240 8.8
 // against 11.4), and so are 128 to 256 of them (0.84 on average).
 extern "C" int pae_gemm_wide_plan(int mode, int act, int M, int N, int K, int ranges) {
-  static const int CUTS[] = {2, 3, 4, 6, 8};
+  static const int CUTS[] = {2, 3, 4, 5, 6, 8};
   int best = SHAPE_LARGE, cuts = 1;
   double least = 1e30;
   for (int shape = 0; shape < SHAPES; ++shape) {
@@ -311,10 +329,10 @@ extern "C" int pae_gemm_wide_plan(int mode, int act, int M, int N, int K, int ra
     const double t = shape_time(shape, M, N, K, 1);
     if (t < least) least = t, best = shape;
   }
-  for (int shape = SHAPE_LARGE + 1; ranges && shape < SHAPES; ++shape)
+  for (int shape = SHAPE_LARGE; ranges && shape < SHAPES; ++shape)
     for (int n : CUTS) {
       if (K < 1024 * n) break;  // (k of 1,536 in two ranges: 8.2 -> 7.8 us at best, and slower from 900 rows on)
-      const double t = shape_time(shape, M, N, K, n) + (4.0 * n - 2.0) * M * N / 4.5e6;
+      const double t = shape_time(shape, M, N, K, n) + (4.0 * n - 2.0) * M * N / 3.6e6;
       if (t < least) least = t, best = shape, cuts = n;
     }
   if (mode == wide_gemm::PLAIN && act == NO_ACT &&
@@ -330,7 +348,7 @@ extern "C" int pae_gemm_wide(int mode, int act, int plan, void* out, int64_t ldc
                              int b_is_f32, int M, int N, int K, hipStream_t stream) {
   const int shape = plan & 255, ranges = plan >> 8;
   PAE_REQUIRE(M > 0 && N > 0 && N % 16 == 0 && K > 0 && K % 64 == 0, "wide product: bad sizes M=%d N=%d K=%d", M, N, K);
-  PAE_REQUIRE(plan >= 0 && shape < SHAPES && ranges >= 1 && ranges <= K / 64 && (mode == wide_gemm::SUMS || ranges == 1) && (shape != SHAPE_LARGE || K >= 128),
+  PAE_REQUIRE(plan >= 0 && shape < SHAPES && ranges >= 1 && ranges <= K / 64 && (mode == wide_gemm::SUMS || ranges == 1) && (shape != SHAPE_LARGE || K >= 128 * ranges),
               "wide product: plan %d for mode %d and K=%d", plan, mode, K);
   PAE_REQUIRE(lda >= 0 && lda % 8 == 0 && lda < (1 << 22) && K < (1 << 22), "wide product: rows of %lld numbers", (long long)lda);  // 256 rows in 32 bits
   PAE_REQUIRE(ldc % (mode == wide_gemm::SUMS ? 4 : 8) == 0 && ((uintptr_t)out | (uintptr_t)a | (uintptr_t)w) % 16 == 0, "wide product: operands must lie at multiples of 16 bytes");

@@ -116,6 +116,20 @@ def test_sums_of_ranges(M, N, k, ranges):
         assert bool((behind == 7.0).all())
 
 
+@pytest.mark.parametrize("M,N,k,ranges", [(65, 16, 128, 1), (129, 272, 320, 2), (257, 528, 448, 3), (513, 1552, 896, 7), (300, 4112, 1216, 4)])
+def test_sums_of_ranges_in_the_largest_tiles(M, N, k, ranges):
+    """Two stages a range and more, odd numbers of them, more tiles than one and ranges of unequal length."""
+    a, w = operands(M, N, k, 3)
+    at = [k // 64 * i // ranges * 64 for i in range(ranges + 1)]
+    out, behind = guarded(M, N, torch.float32, ranges)
+    K.gemm_wide(out, a, w, ranges << 8, mode=K.WIDE_SUMS)
+    for i in range(ranges):
+        check(out[i], *exact(a[:, at[i]:at[i + 1]], w[:, at[i]:at[i + 1]]))
+    assert bool((behind == 7.0).all())
+    with pytest.raises(K.KernelError):  # a range of one stage
+        K.gemm_wide(torch.empty((k // 64, M, N), device="cuda"), a, w, k // 64 << 8, mode=K.WIDE_SUMS)
+
+
 @pytest.mark.parametrize("M,N,k", [(129, 272, 320), (1100, 17920, 128)])
 def test_same_bits_as_two_kernels(M, N, k):
     a, w = operands(M, N, k, 5)
