@@ -42,6 +42,9 @@ int pae_gemm_plain_batched(int in_dtype, int out_dtype, void* C, int64_t ldc, in
 int pae_gemm_wide_plan(int mode, int act, int M, int N, int K, int ranges);  // shape | ranges of k << 8, or -1: the platform library
 int pae_gemm_wide(int mode, int act, int plan, void* out, int64_t ldc, const void* a, int64_t lda, const void* w, const void* bias,
                   int b_is_f32, int M, int N, int K, hipStream_t stream);
+int pae_gemm_wide_rope(int plan, void* out, int64_t ldc, const void* a, int64_t lda, const void* w, const void* bias, int b_is_f32, int M,
+                       int K, int nh, int nkv, int hd, int rot, const float* cos_sin, const int* positions, const int* tok_seq,
+                       const int* block_tables, int max_blocks, int bs, void* k_cache, void* v_cache, hipStream_t stream);
 int pae_gemm_skinny(int epilogue, void* out, int64_t ldc, const void* A, int64_t lda, const void* W,
                     const void* bias, int b_is_f32, int M, int N, int K, int splits, int64_t part_stride,
                     float* ticket_parts, int* ticket_counters, const float* row_stats, int row_stat_tiles,

@@ -6,6 +6,10 @@
 // idle, smaller tiles throughout; and of either k may be cut into ranges that leave float32 sums of their own.  Which one is the
 // least of what the shapes' measured times say (pae_gemm_wide_plan).
 //
+// An attention layer's projections are rotated and stored by the product as well (ROTATED), which then writes queries, keys and values once
+// where a kernel behind it read and wrote them again: 2,048 x 2,048 x 1,536 18.3 and 11.2 us behind it, 22.9 in one; 6,030 x 4,608 x 3,584
+// 160 and 45.6, 177 in one.  What the epilogue adds is the angles' and pages' way and the values' stores of 2 bytes.
+//
 // Measured beside the platform library's product (weights from memory, us; rows x features x k):
 //     2,048 x 17,920 x  1,536   library 111 and 22 for the gate behind it    here with the gate 100
 //     2,048 x  1,536 x  8,960           71                                   66
@@ -32,6 +36,17 @@ namespace {
 
 constexpr int UNITS = 256, DIES = 8, NO_ACT = -1;
 
+// Where the rows of a projection to query, key and value heads go, and how they are rotated (ROTATED).
+struct Heads {
+  const float* cos_sin;     // [M][rot / 2][2]
+  const int* positions;     // [M]
+  const int* tok_seq;       // [M] row of block_tables
+  const int* block_tables;  // [sequences][max_blocks]
+  bf16_t* k_cache;          // [block][key/value head][bs][hd]
+  bf16_t* v_cache;          // [block][key/value head][hd][bs]
+  int nh, nkv, hd, rot, max_blocks, bs;
+};
+
 struct Product {
   void* out;  // bfloat16 [M][ldc], or float32 [split][M][ldc]
   int64_t ldc;
@@ -43,7 +58,21 @@ struct Product {
   int M, N, stages, splits;
   int row_tiles, col_tiles, strip;
   int whole;  // tiles of 256 x 256 that are run as such
+  Heads heads;
 };
+
+// The row of W that a tile takes as its row n: of a rotated head's rows, in sixteens, 8 features and then the 8 they are rotated with.
+template <int MODE>
+__device__ __forceinline__ int w_row_of(const Product& p, int n) {
+  if (MODE != wide_gemm::ROTATED) return n;
+  const int head = n / p.heads.hd, f = n % p.heads.hd, half = p.heads.rot / 2;
+  if (head >= p.heads.nh + p.heads.nkv || f >= p.heads.rot) return n;
+  return head * p.heads.hd + (f % 16 < 8 ? f / 16 * 8 + f % 8 : half + f / 16 * 8 + f % 8);
+}
+
+// The first row of W that the tile from n0 on may take.
+template <int MODE>
+__device__ __forceinline__ int first_w_row(const Product& p, int n0) { return MODE == wide_gemm::ROTATED ? n0 / p.heads.hd * p.heads.hd : n0; }
 
 // Workgroups i, i + 8, i + 16, ... run on one die: they take an eighth of `count` in a row, so that tiles that share
 // rows of A or W find them in their die's L2.
@@ -86,6 +115,83 @@ __device__ __forceinline__ void finish(const Product& p, const f32x4 (&acc)[MT][
         for (int e = 0; e < 4; ++e) v[2 * x + e] = (__bf16)(act_of(rounded(acc[i][x][e]), ACT) * rounded(acc[i][x + 1][e]));
       if constexpr (X == 4) *reinterpret_cast<bf16x8*>(o) = *reinterpret_cast<const bf16x8*>(v);
       else *reinterpret_cast<bf16x4*>(o) = *reinterpret_cast<const bf16x4*>(v);
+    }
+  } else if constexpr (MODE == wide_gemm::ROTATED) {
+    static_assert(X == 2 || X == 4, "4 or 8 neighbouring features a lane");
+    // a lane's 2 X features of a row and, 8 rows of the tile behind them, those they are rotated with (or simply the next ones)
+    const Heads& h = p.heads;
+    const int at = kg * (2 * X), n = n0 + at / 8 * 16 + at % 8;  // tile row of the first
+    if (n >= p.N) return;
+    // (the same head in the whole part, and wholly turned or not: heads and what is rotated of them are multiples of 64 wide)
+    const int head = n0 / h.hd, f0 = n - head * h.hd, half = h.rot / 2;
+    const bool turned = head < h.nh + h.nkv && n0 - head * h.hd < h.rot, cached = head >= h.nh, value = head >= h.nh + h.nkv;
+    const int lo = turned ? f0 / 16 * 8 + f0 % 8 : f0, hi = turned ? lo + half : f0 + 8;
+    f32x4 bias[X];
+#pragma unroll
+    for (int x = 0; x < X; ++x)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) bias[x][e] = p.bias ? load_param(p.bias, p.b_is_f32, head * h.hd + (x % 2 ? hi : lo) + x / 2 * 4 + e) : 0.f;
+    constexpr int AT_ONCE = MT < 4 ? MT : 4;  // rows whose angles and pages are asked for together
+#pragma unroll
+    for (int i0 = 0; i0 < MT; i0 += AT_ONCE) {
+      f32x4 angles[AT_ONCE][X];  // (cosine, sine) of 2 X pairs
+      int64_t place[AT_ONCE];
+      if (turned) {
+#pragma unroll
+        for (int i = 0; i < AT_ONCE; ++i) {
+          const float* from = h.cos_sin + ((int64_t)min(row0 + 16 * (i0 + i) + col, p.M - 1) * half + lo) * 2;
+#pragma unroll
+          for (int x = 0; x < X; ++x) angles[i][x] = *reinterpret_cast<const f32x4*>(from + 4 * x);
+        }
+      }
+      if (cached) {
+        int pos[AT_ONCE], seq[AT_ONCE];
+#pragma unroll
+        for (int i = 0; i < AT_ONCE; ++i) {
+          const int row = min(row0 + 16 * (i0 + i) + col, p.M - 1);
+          pos[i] = h.positions[row];
+          seq[i] = h.tok_seq[row];
+        }
+#pragma unroll
+        for (int i = 0; i < AT_ONCE; ++i)
+          place[i] = ((int64_t)h.block_tables[(int64_t)seq[i] * h.max_blocks + pos[i] / h.bs] * h.nkv + (head - h.nh) % h.nkv) * ((int64_t)h.bs * h.hd) +
+                     (int64_t)(pos[i] % h.bs) * (value ? 1 : h.hd);
+      }
+#pragma unroll
+      for (int i = 0; i < AT_ONCE; ++i) {
+        const int row = row0 + 16 * (i0 + i) + col;
+        if (row >= p.M) continue;
+        // the projection is rounded to bfloat16 before the rotation, as where the two are separate kernels
+        __bf16 v[2][2 * X];
+#pragma unroll
+        for (int x = 0; x < X; ++x)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[x % 2][x / 2 * 4 + e] = (__bf16)(acc[i0 + i][x][e] + bias[x][e]);
+        if (turned) {
+#pragma unroll
+          for (int e = 0; e < 2 * X; ++e) {
+            const float a = (float)v[0][e], b = (float)v[1][e], c = angles[i][e / 2][2 * (e % 2)], s = angles[i][e / 2][2 * (e % 2) + 1];
+            v[0][e] = (__bf16)(a * c - b * s);
+            v[1][e] = (__bf16)(b * c + a * s);
+          }
+        }
+        if (value) {  // values lie the other way round
+          __bf16* values = (__bf16*)h.v_cache + place[i];
+#pragma unroll
+          for (int part = 0; part < 2; ++part)
+#pragma unroll
+            for (int e = 0; e < 2 * X; ++e) values[(int64_t)((part ? hi : lo) + e) * h.bs] = v[part][e];
+          continue;
+        }
+        bf16_t* o = cached ? h.k_cache + place[i] : (bf16_t*)p.out + row * p.ldc + (int64_t)head * h.hd;
+        if constexpr (X == 4) {
+          *reinterpret_cast<bf16x8*>(o + lo) = *reinterpret_cast<const bf16x8*>(v[0]);
+          *reinterpret_cast<bf16x8*>(o + hi) = *reinterpret_cast<const bf16x8*>(v[1]);
+        } else {
+          *reinterpret_cast<bf16x4*>(o + lo) = *reinterpret_cast<const bf16x4*>(v[0]);
+          *reinterpret_cast<bf16x4*>(o + hi) = *reinterpret_cast<const bf16x4*>(v[1]);
+        }
+      }
     }
   } else if constexpr (MODE == wide_gemm::SUMS) {
 #pragma unroll
@@ -145,7 +251,8 @@ __device__ __forceinline__ void small_tile(const Product& p, char* lds, int m0, 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PAE_WAVE);
   typename T::Source src;
   src.a = p.a + m0 * p.lda + (int64_t)first * wide_gemm::ROW_BYTES;
-  src.w = p.w + n0 * p.ldw + (int64_t)first * wide_gemm::ROW_BYTES;
+  const int w0 = first_w_row<MODE>(p, n0);
+  src.w = p.w + w0 * p.ldw + (int64_t)first * wide_gemm::ROW_BYTES;
 #pragma unroll
   for (int j = 0; j < T::A_LOADS; ++j) {
     const int q = (wave * T::A_LOADS + j) * 8 + lane / 8;
@@ -155,7 +262,7 @@ __device__ __forceinline__ void small_tile(const Product& p, char* lds, int m0, 
   for (int j = 0; j < T::W_LOADS; ++j) {
     const int q = (wave * T::W_LOADS + j) * 8 + lane / 8;
     const int n = q / T::PN * T::PN + wide_gemm::dealt_row<MODE, T::X>(q % T::PN / 16, q % 16);
-    src.w_off[j] = (uint32_t)min(n, p.N - 1 - n0) * (uint32_t)p.ldw + wide_gemm::piece_of(lane, q);
+    src.w_off[j] = (uint32_t)(w_row_of<MODE>(p, min(n0 + n, p.N - 1)) - w0) * (uint32_t)p.ldw + wide_gemm::piece_of(lane, q);
   }
   f32x4 acc[T::MT][T::X];
 #pragma unroll
@@ -195,14 +302,15 @@ __global__ __launch_bounds__(512, 2) void wide_large_kernel(Product p) {
   const int m0 = tm * 256, n0 = tn * 256;
   Large::Source src;
   src.a = p.a + m0 * p.lda + (int64_t)first * wide_gemm::ROW_BYTES;
-  src.w = p.w + n0 * p.ldw + (int64_t)first * wide_gemm::ROW_BYTES;
+  const int w0 = first_w_row<MODE>(p, n0);
+  src.w = p.w + w0 * p.ldw + (int64_t)first * wide_gemm::ROW_BYTES;
 #pragma unroll
   for (int h = 0; h < 2; ++h)
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int q = (wave * 2 + j) * 8 + lane / 8;
       src.a_off[h][j] = (uint32_t)min(Large::a_row(h, q), p.M - 1 - m0) * (uint32_t)p.lda + wide_gemm::piece_of(lane, q);
-      src.w_off[h][j] = (uint32_t)min(Large::w_row<MODE>(h, q), p.N - 1 - n0) * (uint32_t)p.ldw + wide_gemm::piece_of(lane, q);
+      src.w_off[h][j] = (uint32_t)(w_row_of<MODE>(p, min(n0 + Large::w_row<MODE>(h, q), p.N - 1)) - w0) * (uint32_t)p.ldw + wide_gemm::piece_of(lane, q);
     }
   f32x4 acc[Large::MT][Large::X];
 #pragma unroll
@@ -295,7 +403,7 @@ double shape_time(int shape, int M, int N, int K, int splits) {
 
 template <int MODE, int ACT>
 int run_shape(int shape, const Product& p, hipStream_t stream) {
-  constexpr bool PAIRS = MODE == wide_gemm::GATED;
+  constexpr bool PAIRS = MODE == wide_gemm::GATED || MODE == wide_gemm::ROTATED;
   switch (shape) {
     case SHAPE_LARGE: return launch_large<MODE, ACT>(p, stream);
     case SHAPE_128_256: return launch_small<MODE, ACT, Tile<128, 256, 2, 4, 3>>(p, stream);
@@ -341,11 +449,19 @@ extern "C" int pae_gemm_wide_plan(int mode, int act, int M, int N, int K, int ra
   return best | cuts << 8;
 }
 
+static int wide_product(int mode, int act, int plan, void* out, int64_t ldc, const void* a, int64_t lda, const void* w, const void* bias,
+                        int b_is_f32, int M, int N, int K, const Heads& heads, hipStream_t stream);
+
 // C = A W^T for A [M, K] (rows of lda numbers), W [N, K]; K a multiple of 64, N of 16.  mode 0: bfloat16 [M, N] of act(A W^T + bias), act
 // -1 (none), 0 or 3; 1: bfloat16 [M, N / 2] of act(gate) * other, W's rows in blocks of 8 of the one and of the
 // other, act 1 or 2; 2: float32 [ranges, M, N] of the sums over ranges of k.  Operands begin at multiples of 16 bytes.
 extern "C" int pae_gemm_wide(int mode, int act, int plan, void* out, int64_t ldc, const void* a, int64_t lda, const void* w, const void* bias,
                              int b_is_f32, int M, int N, int K, hipStream_t stream) {
+  return wide_product(mode, act, plan, out, ldc, a, lda, w, bias, b_is_f32, M, N, K, Heads{}, stream);
+}
+
+static int wide_product(int mode, int act, int plan, void* out, int64_t ldc, const void* a, int64_t lda, const void* w, const void* bias,
+                        int b_is_f32, int M, int N, int K, const Heads& heads, hipStream_t stream) {
   const int shape = plan & 255, ranges = plan >> 8;
   PAE_REQUIRE(M > 0 && N > 0 && N % 16 == 0 && K > 0 && K % 64 == 0, "wide product: bad sizes M=%d N=%d K=%d", M, N, K);
   PAE_REQUIRE(plan >= 0 && shape < SHAPES && ranges >= 1 && ranges <= K / 64 && (mode == wide_gemm::SUMS || ranges == 1) && (shape != SHAPE_LARGE || K >= 128 * ranges),
@@ -366,6 +482,8 @@ extern "C" int pae_gemm_wide(int mode, int act, int plan, void* out, int64_t ldc
   p.stages = K / 64;
   p.splits = ranges;
   p.row_tiles = p.col_tiles = p.strip = p.whole = 0;
+  p.heads = heads;
+  if (mode == wide_gemm::ROTATED) return run_shape<wide_gemm::ROTATED, NO_ACT>(shape, p, stream);
   if (mode == wide_gemm::SUMS) return run_shape<wide_gemm::SUMS, NO_ACT>(shape, p, stream);
   if (mode == wide_gemm::PLAIN && act == NO_ACT) return run_shape<wide_gemm::PLAIN, NO_ACT>(shape, p, stream);
   if (mode == wide_gemm::PLAIN && act == 0) return run_shape<wide_gemm::PLAIN, 0>(shape, p, stream);
@@ -373,4 +491,20 @@ extern "C" int pae_gemm_wide(int mode, int act, int plan, void* out, int64_t ldc
   if (mode == wide_gemm::GATED && act == 1) return run_shape<wide_gemm::GATED, 1>(shape, p, stream);
   if (mode == wide_gemm::GATED && act == 2) return run_shape<wide_gemm::GATED, 2>(shape, p, stream);
   return pae_fail("wide product: mode %d with activation %d", mode, act);
+}
+
+// A W^T + bias, W [(nh + 2 nkv) hd, K] the projections to query, key and value heads: query heads, their first `rot` features rotated in pairs
+// (i, i + rot / 2), to out [M, nh hd], key heads rotated likewise and value heads to their places in the pages, as pae_rope_kv_write
+// puts them.  `plan` as pae_gemm_wide_plan gives it for mode 1.  nkv may be 0: only queries.
+extern "C" int pae_gemm_wide_rope(int plan, void* out, int64_t ldc, const void* a, int64_t lda, const void* w, const void* bias, int b_is_f32,
+                                  int M, int K, int nh, int nkv, int hd, int rot, const float* cos_sin, const int* positions, const int* tok_seq,
+                                  const int* block_tables, int max_blocks, int bs, void* k_cache, void* v_cache, hipStream_t stream) {
+  PAE_REQUIRE(nh > 0 && nkv >= 0 && hd > 0 && hd % 64 == 0 && rot >= 0 && rot <= hd && rot % 64 == 0 && (rot == 0 || cos_sin),
+              "wide projection: heads of %d with %d features rotated", hd, rot);
+  PAE_REQUIRE(nkv == 0 || (bs > 0 && max_blocks > 0 && k_cache && v_cache && block_tables && tok_seq && positions),
+              "wide projection: the cache write needs tables and pools");
+  PAE_REQUIRE(ldc >= (int64_t)nh * hd && (uintptr_t)k_cache % 16 == 0 && (uintptr_t)cos_sin % 16 == 0 && (int64_t)(256 + hd) * K < (1ll << 31),
+              "wide projection: rows of %lld numbers, or operands between multiples of 16 bytes", (long long)ldc);
+  return wide_product(wide_gemm::ROTATED, NO_ACT, plan, out, ldc, a, lda, w, bias, b_is_f32, M, (nh + 2 * nkv) * hd, K,
+                      Heads{cos_sin, positions, tok_seq, block_tables, (bf16_t*)k_cache, (bf16_t*)v_cache, nh, nkv, hd, rot, max_blocks, bs}, stream);
 }

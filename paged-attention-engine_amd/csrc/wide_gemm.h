@@ -27,7 +27,8 @@
 // part are dealt so that its results leave in stores of 16 bytes a lane, 64 bytes in a row of the result: a lane ends with 8
 // neighbours of 32 in two groups (X: groups of 16 W rows; a single group left over: 4 of 16), with 4 of 16 where the sums leave as
 // float32, and for gated products, whose rows alternate in blocks of 8 of the gate and 8 of the other factor, with 2 X
-// neighbouring gates and the same features' other factors.
+// neighbouring gates and the same features' other factors.  Heads whose pairs of features are rotated are dealt likewise, 8 features
+// and the 8 they are rotated with.
 #pragma once
 #include "common.h"
 
@@ -54,12 +55,12 @@ struct Number {
 // The piece of 16 bytes that a lane brings of the LDS row `row` of its tile.
 __device__ __forceinline__ uint32_t piece_of(int lane, int row) { return (uint32_t)((lane % 8) ^ ((row >> 1) & 7)) * 16; }
 
-enum { PLAIN, GATED, SUMS };  // what leaves: bfloat16, act(gate) * other in bfloat16, float32
+enum { PLAIN, GATED, SUMS, ROTATED };  // what leaves: bfloat16, act(gate) * other in bfloat16, float32, heads with pairs of features rotated
 
 // The W row, among the PN of a wavefront's part, that row `r` of its group `x` of 16 (of X) holds.
 template <int MODE, int X>
 __device__ __forceinline__ int dealt_row(int x, int r) {
-  if (MODE == GATED) {
+  if (MODE == GATED || MODE == ROTATED) {
     const int feature = (r / 4) * (2 * X) + (x / 2) * 4 + r % 4;
     return (feature / 8) * 16 + feature % 8 + 8 * (x % 2);
   }

@@ -66,6 +66,7 @@ def _declare(lib) -> None:
         "pae_gemm_skinny_rope": [P, L, P, L, P, P, I, I, I, I, I, I, I, P, P, P, P, I, I, P, P, I, P, P, P, I, F, P],
         "pae_gemm_wide_plan": [I, I, I, I, I, I],
         "pae_gemm_wide": [I, I, I, P, L, P, L, P, P, I, I, I, I, P],
+        "pae_gemm_wide_rope": [I, P, L, P, L, P, P, I, I, I, I, I, I, I, P, P, P, P, I, I, P, P, P],
         "pae_embedding_rows": [I, P, P, P, I, I, I, F, P, P, I, P, P],
         "pae_scaled_rows": [P, P, P, I, F, I, I, P],
         "pae_skinny_ticket_slots": [I, I],
@@ -878,6 +879,39 @@ def gemm_wide(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, plan: int, bi
     bp, bf = _param(bias)
     _check(library().pae_gemm_wide(mode, -1 if kind is None else ACTIVATIONS[kind], plan, out.data_ptr(), out.shape[-1], a.data_ptr(),
                                    a.stride(0), w.data_ptr(), bp, bf, M, N, K, _stream()))
+
+
+def wide_rope_plan(a: torch.Tensor, w: torch.Tensor, hd: int, rot: int, bias: Optional[torch.Tensor] = None, cos_sin: Optional[torch.Tensor] = None,
+                   k_cache: Optional[torch.Tensor] = None) -> Optional[int]:
+    """How `gemm_wide_rope` makes this projection, or None: sizes or operands that it does not take."""
+    if hd % 64 or rot % 64 or any(t is not None and t.data_ptr() % 16 for t in (cos_sin, k_cache)) or (256 + hd) * a.shape[-1] >= 1 << 31:
+        return None
+    return wide_plan(a, w, WIDE_GATED, bias=bias)
+
+
+def gemm_wide_rope(q_out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], plan: int, nh: int, nkv: int, hd: int,
+                   rot: int, cos_sin: Optional[torch.Tensor], positions: torch.Tensor, tok_seq: Optional[torch.Tensor],
+                   block_tables: Optional[torch.Tensor], block_size: int, k_cache: Optional[torch.Tensor], v_cache: Optional[torch.Tensor]) -> None:
+    """`gemm_skinny_rope` for more rows: the projections to query, key and value heads, the queries rotated to `q_out` [M, nh * hd], keys
+    rotated and values to their cache slots (nkv 0: queries only).  `plan` as `wide_rope_plan` gives it."""
+    _not_while_recording("gemm_wide_rope")
+    _gpu(q_out, a, w, bias, cos_sin, positions, tok_seq, block_tables, k_cache, v_cache)
+    M, K = a.shape
+    assert w.shape == ((nh + 2 * nkv) * hd, K) and w.is_contiguous() and a.stride(1) == 1 and a.dtype == w.dtype == q_out.dtype == torch.bfloat16
+    assert q_out.shape == (M, nh * hd) and q_out.stride(1) == 1 and positions.dtype == torch.int32 and positions.numel() == M
+    assert bias is None or bias.shape == (w.shape[0],)
+    _check_cos_sin(cos_sin, rot, M)
+    max_blocks = 0
+    if nkv:
+        assert k_cache.dtype == v_cache.dtype == a.dtype and tok_seq.dtype == torch.int32 and tok_seq.numel() == M
+        assert block_tables.dtype == torch.int32 and block_tables.dim() == 2 and block_tables.is_contiguous()
+        _check_pools(k_cache, v_cache, nkv, block_size, hd)
+        max_blocks = block_tables.shape[1]
+    bp, bf = _param(bias)
+    _check(library().pae_gemm_wide_rope(
+        plan, q_out.data_ptr(), q_out.stride(0), a.data_ptr(), a.stride(0), w.data_ptr(), bp, bf, M, K, nh, nkv, hd, rot,
+        _ptr(cos_sin) if rot else None, positions.data_ptr(), _ptr(tok_seq), _ptr(block_tables), max_blocks, block_size, _ptr(k_cache),
+        _ptr(v_cache), _stream()))
 
 
 def product_of_rows(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:

@@ -320,7 +320,13 @@ class PagedAttention(Part):
                                ctx.positions, ctx.tok_seq, table, bs, k_cache, v_cache, splits,
                                row_scale=owed.row_scale if owed is not None else None)
             return q
-        # many rows: the library's plain product (its variant with a bias costs the host six times the
+        plan = K.wide_rope_plan(x, linear.weight, s.head_dim, rot, linear.bias, cos_sin, k_cache) if owed is None else None
+        if plan is not None:  # more rows, likewise
+            q = torch.empty((x.shape[0], s.num_heads * s.head_dim), dtype=x.dtype, device=x.device)
+            K.gemm_wide_rope(q, x, linear.weight, linear.bias, plan, s.num_heads, nkv, s.head_dim, rot, cos_sin, ctx.positions,
+                             ctx.tok_seq, table, bs, k_cache, v_cache)
+            return q
+        # other sizes: the library's plain product (its variant with a bias costs the host six times the
         # call), and the bias is added by the kernel that rotates and stores, which follows anyway
         qkv = linear.without_bias(x) if owed is None else None
         bias = linear.bias if qkv is not None else None

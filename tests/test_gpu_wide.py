@@ -190,3 +190,48 @@ def test_linear_with_odd_biases():
         check(Linear(w, bias)(a), want, err + 2.0 ** -7 * ref.abs())
     with pytest.raises(RuntimeError):
         Linear(w)(a[:, :128].contiguous())
+
+
+@pytest.mark.parametrize("M", [65, 130, 300])
+@pytest.mark.parametrize("nh,nkv,hd,rot,bs,bias,k", [(12, 2, 128, 128, 16, True, 192), (7, 1, 64, 64, 16, False, 128), (3, 3, 192, 64, 32, True, 128),
+                                                     (5, 1, 128, 64, 8, True, 128), (4, 0, 64, 64, 16, True, 128), (2, 2, 64, 0, 16, False, 128)])
+def test_projections_rotate_and_store(M, nh, nkv, hd, rot, bs, bias, k):
+    """In every tile shape: queries rotated, keys rotated and values in their pages, nothing beside them written."""
+    from tests.plain import qwen2_plain as plain
+
+    N = (nh + 2 * nkv) * hd
+    gen = torch.Generator().manual_seed(M + N)
+    a, w = torch.randn(M, k, generator=gen).bfloat16(), (torch.randn(N, k, generator=gen) * k ** -0.5).bfloat16()
+    b = torch.randn(N, generator=gen).bfloat16() if bias else None
+    positions = torch.arange(2, 2 + 2 * M, 2, dtype=torch.int32) // 3 * 2  # not one after another
+    positions, tok_seq = positions + torch.arange(M, dtype=torch.int32) % 2, torch.arange(M, dtype=torch.int32) % 7
+    blocks = int(positions.max()) // bs + 1
+    tables = torch.randperm(7 * blocks, generator=gen).int().view(7, blocks)
+    x = (a.double() @ w.double().t() + (b.double() if bias else 0.0)).bfloat16().double().view(M, -1, hd)
+    turned = x.clone()
+    if rot:
+        cos, sin = plain.rope_cos_sin(plain.rope_inv_freq(rot, 1e4, torch.float64), positions, torch.float64)
+        turned[..., :rot] = x[..., :rot] * cos[:, None] + plain.rotate_half(x[..., :rot]) * sin[:, None]
+    dev = lambda t: t.cuda() if t is not None else None
+    angles = K.rope_table(positions.cuda(), plain.rope_inv_freq(rot, 1e4).cuda()) if rot else None
+    # the projection's rounding may fall the other way (2^-7 of it), of each of a rotated pair, and the result is rounded
+    bound = 2.0 ** -7 * (x.abs().amax(-1, keepdim=True) * 1.5 + 0.01)
+    assert K.wide_rope_plan(dev(a), dev(w), hd, rot, dev(b)) is not None
+    for shape in GATED_SHAPES:
+        pools = [torch.full((7 * blocks, nkv, *s), 7.0, dtype=torch.bfloat16, device="cuda") for s in ((bs, hd), (hd, bs))] if nkv else [None, None]
+        q = torch.full((M, nh * hd + 8), 7.0, dtype=torch.bfloat16, device="cuda")
+        K.gemm_wide_rope(q[:, :nh * hd], dev(a), dev(w), dev(b), shape | 1 << 8, nh, nkv, hd, rot, angles, dev(positions), dev(tok_seq) if nkv else None,
+                         dev(tables) if nkv else None, bs, *pools)
+        assert ((q[:, :nh * hd].double().cpu().view(M, nh, hd) - turned[:, :nh]).abs() <= bound[:, :nh]).all()
+        assert bool((q[:, nh * hd:] == 7.0).all())
+        if not nkv:
+            continue
+        last = {(int(tok_seq[m]), int(positions[m])): m for m in range(M)}  # the rows whose slot no later row takes
+        pages, at = [int(tables[s, p // bs]) for s, p in last], [p % bs for _, p in last]
+        rows = list(last.values())
+        assert len(rows) == M
+        assert ((pools[0].cpu().double()[pages, :, at] - turned[rows, nh:nh + nkv]).abs() <= bound[rows, nh:nh + nkv]).all()
+        assert ((pools[1].cpu().double()[pages, :, :, at] - x[rows, nh + nkv:]).abs() <= bound[rows, nh + nkv:]).all()
+        kept = torch.ones(7 * blocks, bs, dtype=torch.bool)
+        kept[pages, at] = False
+        assert bool((pools[0].cpu().transpose(1, 2)[kept] == 7.0).all()) and bool((pools[1].cpu().permute(0, 3, 1, 2)[kept] == 7.0).all())
