@@ -126,8 +126,8 @@ int pae_attn_prefill_route(int nh, int hd, int vd, int bs, int num_tiles, int to
 int pae_attn_prefill_wide_bf16(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k_cache,
                                const void* v_cache, const int* tiles, int num_tiles, const int* positions,
                                const int* block_tables, int max_blocks, int nh, int nkv, int hd, int vd, float scale,
-                               int window, const void* head_gate, int64_t head_gate_stride, int tokens, int route,
-                               hipStream_t stream);
+                               int window, const float* sinks, const void* head_gate, int64_t head_gate_stride, int tokens,
+                               int route, hipStream_t stream);
 // rows [q | k | v]: RMS norm of q and of k over the whole projection, or head by head with one weight that the
 // heads share (`per_head`; weights null: none), rotation, cache write
 int pae_qk_norm_rotate_store(int dtype, void* qkv, int64_t row_stride, int num_tokens, int nh, int nkv, int hd, int vd,

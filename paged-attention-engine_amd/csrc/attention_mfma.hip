@@ -852,11 +852,12 @@ extern "C" int pae_attn_prefill_wide_width(int width, int vd) {
   return 0;
 }
 
-// `pae_attn_prefill_bf16` over pages of 16 with value heads of their own width and a gate per token and head.
+// `pae_attn_prefill_bf16` over pages of 16 with value heads of their own width, sinks and a gate per token and head.
 extern "C" int pae_attn_prefill_wide_bf16(void* out, int64_t out_stride, const void* q, int64_t q_stride, const void* k_cache,
                                           const void* v_cache, const int* tiles, int num_tiles, const int* positions,
                                           const int* block_tables, int max_blocks, int nh, int nkv, int hd, int vd, float scale,
-                                          int window, const void* head_gate, int64_t head_gate_stride, int tokens, int route, hipStream_t stream) {
+                                          int window, const float* sinks, const void* head_gate, int64_t head_gate_stride, int tokens,
+                                          int route, hipStream_t stream) {
   if (int rc = check_common("attn_prefill_wide", nh, nkv, hd, 16, max_blocks, window)) return rc;
   PAE_REQUIRE(pae_attn_prefill_wide_width(hd, vd) == hd, "attn_prefill_wide: keys of %d with values of %d are not built", hd, vd);
   PAE_REQUIRE(out_stride >= (int64_t)nh * vd && q_stride >= (int64_t)nh * hd, "attn_prefill_wide: row strides too small");
@@ -868,13 +869,13 @@ extern "C" int pae_attn_prefill_wide_bf16(void* out, int64_t out_stride, const v
   if (route > 0) {
     const PrefillArgs args = {(bf16_t*)out, out_stride, (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache,
                               tiles, num_tiles, positions, block_tables, max_blocks, nh, nkv, scale * LOG2E, window, 0.f, 0.f,
-                              nullptr, 0, nullptr, 0.f, nullptr, 0, (const bf16_t*)head_gate, head_gate_stride};
+                              sinks, 0, nullptr, 0.f, nullptr, 0, (const bf16_t*)head_gate, head_gate_stride};
     return attn_prefill_shared(args, hd, vd, false, route, stream);
   }
 #define WIDE_LAUNCH(HD, CT, VD)                                                                                          \
   attn_prefill_split_kernel<HD, CT, 16, false, false, VD><<<dim3(nh * (PREFILL_RUN / 16 / CT), num_tiles), 256, 0, stream>>>( \
       (bf16_t*)out, out_stride, (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache, tiles,        \
-      positions, block_tables, max_blocks, 16, nh, nkv, scale * LOG2E, window, 0.f, 0.f, nullptr, 0, nullptr, 0.f, nullptr, 0, \
+      positions, block_tables, max_blocks, 16, nh, nkv, scale * LOG2E, window, 0.f, 0.f, sinks, 0, nullptr, 0.f, nullptr, 0, \
       (const bf16_t*)head_gate, head_gate_stride)
 #define WIDE_CASE(HD, VD)                  \
   if (hd == HD && vd == VD) {              \

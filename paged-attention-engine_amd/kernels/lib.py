@@ -93,7 +93,7 @@ def _declare(lib) -> None:
         "pae_latent_queries": [P, P, L, I, P, F, I, I, I, I, I, I, P],
         "pae_attn_prefill_wide_width": [I, I],
         "pae_attn_prefill_route": [I, I, I, I, I, I, I, I],
-        "pae_attn_prefill_wide_bf16": [P, L, P, L, P, P, P, I, P, P, I, I, I, I, I, F, I, P, L, I, I, P],
+        "pae_attn_prefill_wide_bf16": [P, L, P, L, P, P, P, I, P, P, I, I, I, I, I, F, I, P, P, L, I, I, P],
         "pae_gated_act": [I, P, P, I, I, I, I, P],
         "pae_gemm_plain_batched": [I, I, P, L, L, P, L, L, P, L, P, I, I, I, I, I, P],
         "pae_rows_from_residual": [I, P, P, L, P],
@@ -1420,15 +1420,19 @@ def latent_key_width(dtype: torch.dtype, row_width: int, rank: int, head_width: 
 def latent_expanded(out: torch.Tensor, proj: torch.Tensor, latent: torch.Tensor, up_weight: torch.Tensor, pages: torch.Tensor,
                     page_table: torch.Tensor, tiles: torch.Tensor, positions: torch.Tensor, block_tables: torch.Tensor,
                     cos_sin: Optional[torch.Tensor], magnitude: float, nh: int, nope: int, rd: int, rot: int, interleaved: bool,
-                    value_dim: int, rank: int, scale: float, head_gate: Optional[torch.Tensor] = None, window: int = 0) -> None:
+                    value_dim: int, rank: int, scale: float, head_gate: Optional[torch.Tensor] = None, window: int = 0,
+                    sinks: Optional[torch.Tensor] = None) -> None:
     """Latent attention for runs of many tokens, the heads' keys and values formed first: out[t, h * value_dim:] of
     the runs' tokens receives the heads (gated by sigmoid of `head_gate` [T, >= nh] if given); other rows are left alone.
+    `sinks` float32 [nh]: exp(sink) joins each head's denominator.
     `window` > 0: a token at position p sees the keys from p - window + 1 on.  `proj` and `latent` as for `latent_prepare`, which has written the runs' rows; `up_weight` [nh (nope + value_dim),
     rank] = [W_uk; W_uv].  `pages` int32 [n, 4] = (table row of the sequence, position of the first key, keys, 0) cuts
     every run's keys, from the sequence's first (or the first one in the window) on, into pages of 16; `page_table` int32 [runs, width] names each run's
     pages in that list, in order; `tiles` int32 [m, 3] = (row of `page_table`, first flat token, tokens <= PREFILL_TILE)."""
     _not_while_recording("latent_expanded")
-    _gpu(out, proj, latent, up_weight, pages, page_table, tiles, positions, block_tables, cos_sin, head_gate)
+    _gpu(out, proj, latent, up_weight, pages, page_table, tiles, positions, block_tables, cos_sin, head_gate, sinks)
+    if sinks is not None:
+        assert sinks.dtype == torch.float32 and sinks.numel() == nh and sinks.is_contiguous()
     T, n, bs = proj.shape[0], pages.shape[0], latent.shape[1]
     width = latent_key_width(proj.dtype, latent.shape[2], rank, nope + rd, value_dim)
     assert width > 0 and latent.shape[2] == rank + rd and latent.is_contiguous() and latent.dtype == proj.dtype == out.dtype
@@ -1453,13 +1457,15 @@ def latent_expanded(out: torch.Tensor, proj: torch.Tensor, latent: torch.Tensor,
     _check(lib.pae_latent_expand(keys.data_ptr(), values.data_ptr(), up.data_ptr(), up.stride(0), latent.data_ptr(),
                                  pages.data_ptr(), n, block_tables.data_ptr(), block_tables.shape[1], bs, nh, nope, rd,
                                  value_dim, rank, width, _stream()))
-    q = new(T, nh * width)
-    _check(lib.pae_latent_queries(q.data_ptr(), proj.data_ptr(), proj.stride(0), T, _ptr(cos_sin) if rot else None,
-                                  float(magnitude), nh, nope, rd, rot, 1 if interleaved else 0, width, _stream()))
+    q = proj
+    if rd or nope != width or proj.stride(0) % 8 or proj.data_ptr() % 16:  # else the queries are rows as they are to be
+        q = new(T, nh * width)
+        _check(lib.pae_latent_queries(q.data_ptr(), proj.data_ptr(), proj.stride(0), T, _ptr(cos_sin) if rot else None,
+                                      float(magnitude), nh, nope, rd, rot, 1 if interleaved else 0, width, _stream()))
     _check(lib.pae_attn_prefill_wide_bf16(
         out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0), keys.data_ptr(), values.data_ptr(), tiles.data_ptr(),
         tiles.shape[0], positions.data_ptr(), page_table.data_ptr(), page_table.shape[1], nh, nh, width, value_dim, float(scale), int(window),
-        _ptr(head_gate), head_gate.stride(0) if head_gate is not None else 0, T, -1, _stream()))
+        _ptr(sinks), _ptr(head_gate), head_gate.stride(0) if head_gate is not None else 0, T, -1, _stream()))
 
 
 def hyper_norm(streams: torch.Tensor, num_streams: int, y: Optional[torch.Tensor], layer_scale: Optional[torch.Tensor],

@@ -25,7 +25,7 @@ head's output is W_uv_j times that sum.  The query projection and the down proje
 product (a gate's rows ride in it); the two per-head products are one launch each.
 
 That costs kv_rank + rope_dim multiply-adds a score and kv_rank a value, the least where few queries meet many keys.
-Runs of many tokens (`EXPAND_ROWS`, bfloat16, the layer's own rows, no mask in chunks and no sinks) have their keys and
+Runs of many tokens (`EXPAND_ROWS`, bfloat16, no mask in chunks) have their keys and
 values formed instead, in one product over the keys the run sees, and attend with heads of nope_dim + rope_dim and value_dim
 (`kernels.lib.latent_expanded`); the cache stays as it is.  At the 1.5B sizes (12 heads of 128, a latent of 512, 64 rotated
 features) that is 3.4 times fewer multiply-adds a (query, key) pair, in a kernel that runs several times nearer the matrix
@@ -40,10 +40,12 @@ average out over the keys); on random inputs whose softmax one or two keys domin
 0.0039 formed, because what a folded query's rounding does to such keys' scores is partly the same for all of them.  The model's
 logits are as far from 64 bits either way (ratio of the errors 1.000 over 18 prompts, 0.97 to 1.04 a prompt).
 
-Layers with sinks and layers that read an earlier layer's rows keep the folded form.  Nothing about sinks asks for it: the one
-design that has them puts such layers before routed experts, where another rounding chooses other experts at near
-ties, and there the logits' error rose on some prompts (0.0070 -> 0.0079, 0.0041 -> 0.0044, 0.0047 -> 0.0047).  Their
-runs of 3,001 tokens would go from 0.44 to 0.07 ms.
+Layers with sinks and layers that read an earlier layer's rows take the same two forms (the reader's keys and values are
+products of those rows with its own W_uk and W_uv).  The one design that has them puts such layers before routed experts, where
+another rounding chooses other experts at near ties, so that one prompt's error moves by up to a tenth either way: over 136
+batches of 900, 3,001 and 5,000 tokens the formed logits' error against 64 bits is 1.000 of the folded ones' (geometric mean;
+1.009 +- 0.008, 1.000 +- 0.017 and 0.972 +- 0.023 by size).  Two such layers in a model of eight, 7 runs of 3,001 tokens in all
+and 8 steps behind them: 17.23 -> 16.22 ms, the attention itself 0.46 -> 0.07 ms a layer.
 """
 
 from __future__ import annotations
@@ -168,7 +170,7 @@ class LatentAttention(Part):
     def expand_rows(self) -> int:
         """Runs of at least this many tokens attend with the heads' keys and values formed (0: none do)."""
         s = self.spec
-        takes = (s.own_kv and not s.sinks and (s.mask == "window" or not s.window) and self.matrix_cores
+        takes = ((s.mask == "window" or not s.window) and self.matrix_cores
                  and K.latent_key_width(self.dtype, self.row_width, s.kv_rank, s.nope_dim + s.rope_dim, s.value_dim) > 0)
         return EXPAND_ROWS if takes else 0
 
@@ -255,5 +257,5 @@ class LatentAttention(Part):
             K.heads_product(heads.view(T, H, V), summed.view(T, H, C), self.up_v, self.up_v_t)
         if formed:  # over whatever the products above made of these rows
             K.latent_expanded(heads, proj, latent, self.up, tiles["pages"], tiles["page_table"], tiles["tiles"], ctx.positions,
-                              table, cos_sin, magnitude, H, D, R, rot, interleaved, V, C, s.scale, gate, s.window or 0)
+                              table, cos_sin, magnitude, H, D, R, rot, interleaved, V, C, s.scale, gate, s.window or 0, self.sinks)
         return self.out.branch(heads, ctx.sink)

@@ -99,7 +99,7 @@ def test_prefill_by_shared_keys(hd, vd, route, kind, runs):
         hg = d(head_gate)
         assert K.library().pae_attn_prefill_wide_bf16(
             out.data_ptr(), out.stride(0), qd.data_ptr(), qd.stride(0), kd.data_ptr(), vd_.data_ptr(), td.data_ptr(), len(tiles),
-            pd.data_ptr(), bd.data_ptr(), bd.shape[1], nh, nkv, hd, vd, scale, window, hg.data_ptr() if hg is not None else None,
+            pd.data_ptr(), bd.data_ptr(), bd.shape[1], nh, nkv, hd, vd, scale, window, None, hg.data_ptr() if hg is not None else None,
             hg.stride(0) if hg is not None else 0, len(q), route, torch.cuda.current_stream().cuda_stream) == 0
     got = out[:, :nh * vd].double().cpu().view(-1, nh, vd)
     assert torch.isnan(out[:, nh * vd:]).all()
@@ -113,3 +113,44 @@ def test_prefill_by_shared_keys(hd, vd, route, kind, runs):
         g = torch.sigmoid(head_gate[:, :nh].double())[..., None]
         want, bound = want * g, bound * g
     assert ((got - want).abs() <= bound).all(), float(((got - want).abs() / bound).max())
+
+
+@pytest.mark.parametrize("R,V,window,pad", [(0, 128, 0, 0), (0, 128, 0, 1), (0, 64, 0, 0), (64, 128, 0, 0), (0, 128, 150, 0)])
+def test_formed_heads_with_sinks(R, V, window, pad):
+    """Latent attention with the heads formed, with sinks, against 64 bits.  Rows without a rotated part are the queries as they are
+    where they start on 16 bytes (`pad` 0)."""
+    from paged_attention_engine_amd.parts import StepShape
+    from paged_attention_engine_amd.parts.latent import expanded_runs
+
+    gen = torch.Generator().manual_seed(R + V + window)
+    H, D, C, bs, runs = 5, 128, 64, 16, [(0, 129), (37, 200)]  # (keys before, new rows)
+    bf = lambda x: x.to(torch.bfloat16)
+    randn = lambda *shape: torch.randn(*shape, generator=gen)
+    w_uk, w_uv, sinks = bf(randn(H * D, C) * C ** -0.5), bf(randn(H * V, C) * C ** -0.5), 3 * randn(H)
+    scale, T, past = (D + R) ** -0.5, sum(n for _, n in runs), [a for a, _ in runs]
+    width = max(-(-(a + n) // bs) for a, n in runs)
+    tables = torch.randperm(2 * width, generator=gen).view(2, width).to(torch.int32)
+    pool = bf(randn(2 * width, bs, C + R))
+    q = bf(randn(T, H * (D + R) + pad))
+    want, sizes, at = [], [], 0
+    for s, (a, n) in enumerate(runs):
+        rows = pool[tables[s].long()].reshape(-1, C + R)[:a + n].double()
+        k = torch.cat([bf(rows[:, :C] @ w_uk.double().T).double().view(-1, H, D), rows[:, None, C:].expand(-1, H, -1)], -1)
+        v = bf(rows[:, :C] @ w_uv.double().T).double().view(-1, H, V)
+        score = torch.einsum("ihd,jhd->hij", q[at:at + n, :H * (D + R)].double().view(n, H, D + R), k) * scale
+        i, j = torch.arange(a, a + n)[:, None], torch.arange(a + n)
+        score = score.masked_fill((j > i) | ((i - j >= window) if window else (j < 0)), -math.inf)
+        p = torch.softmax(torch.cat([score, sinks.double()[:, None, None].expand(-1, n, 1)], -1), -1)[..., :-1]
+        want.append(torch.einsum("hij,jhv->ihv", p, v).reshape(n, -1))
+        sizes.append(torch.einsum("hij,jhv->ihv", p, v.abs()).reshape(n, -1))
+        at += n
+    lists = expanded_runs(StepShape((0, 1), (0, runs[0][1]), tuple(n for _, n in runs), tuple(past), bs), 128, window, K.PREFILL_TILE)
+    dev = lambda name: torch.tensor(lists[name][0], dtype=torch.int32, device=DEV).view(-1, lists[name][1])
+    positions = torch.cat([torch.arange(a, a + n) for a, n in runs]).to(torch.int32).to(DEV)
+    out = torch.full((T, H * V), math.nan, dtype=torch.bfloat16, device=DEV)
+    K.latent_expanded(out, q.to(DEV), pool.to(DEV), torch.cat([w_uk, w_uv]).to(DEV), dev("pages"), dev("page_table"), dev("tiles"),
+                      positions, tables.to(DEV), None, 1.0, H, D, R, 0, True, V, C, scale, None, window, sinks.to(DEV))
+    want, sizes = torch.cat(want), torch.cat(sizes)
+    # the roundings of weights, their sum and the result as above; the keys' and values' own, which the oracle repeats, fall on the other
+    # side of a tie where the product's sum in 32 bits does: 2^-8 of one of 128 terms of a score, and of a value
+    assert ((out.cpu().double() - want).abs() <= 2.0 ** -8 * (2 * sizes + 2 * want.abs()) + 1e-3).all()
