@@ -181,6 +181,7 @@ int pae_linear_attention_step(int dtype, const void* proj, int64_t row_stride, c
                               int D, int V, float* state, int64_t state_slot_stride, const void* norm_w, int w_is_f32,
                               float norm_eps, float* work, void* out, hipStream_t stream);
 int64_t pae_linear_attention_work_floats(int num_tokens, int H, int D, int V);
+int pae_linear_attention_by_chunks(int num_tokens, int num_seqs, int D);
 // linear attention with a fixed decay per head over a step's projected rows: see fixed_decay.hip
 int pae_fixed_decay_chunk(int D);
 int pae_fixed_decay_step(int dtype, const void* proj, int64_t row_stride, const void* gate_in, int64_t gate_stride,

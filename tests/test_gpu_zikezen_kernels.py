@@ -331,6 +331,39 @@ def test_linear_attention_whole_and_in_steps_in_used_slots(dtype, shape):
     close(got[:20], want[:20], rel, f"the other {shape}")
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,D,V,lens", [(3, 64, 48, (176, 161)), (2, 128, 40, (1, 335)), (1, 68, 16, (160,)), (2, 48, 24, (320, 15)),
+                                        (1, 132, 9, (175, 160)), (1, 192, 32, (16, 17, 450)), (2, 256, 16, (161,)), (2, 4, 8, (330,)), (1, 32, 16, (337, 330)),
+                                        (1, 130, 6, (170,))])
+@pytest.mark.parametrize("z_mean,tau", [(2.0, 4.0), (-9.0, 0.25)])
+def test_linear_attention_by_chunks(dtype, H, D, V, lens, z_mean, tau):
+    """Runs long enough on average to go by chunks of 16 tokens: whole chunks and chunks of 1 and 15 tokens, runs of one chunk beside long ones, every
+    number of tiles a wavefront holds, full and not; decays near one and decays whose products over a chunk are zero in float32.  A
+    second step goes on from the first one's state token by token.  (130 features are no multiple of four: never by chunks.)"""
+    lib = K()
+    gen = torch.Generator().manual_seed(D + sum(lens))
+    eps, T, S, after = 1e-5, sum(lens), len(lens), 3
+    assert bool(lib.library().pae_linear_attention_by_chunks(T, S, D)) == (D != 130)
+    rows = T + after * S
+    proj, z, bias, norm = gla_inputs(gen, rows, H, D, V, dtype, z_mean)
+    starts = [sum(lens[:s]) for s in range(S)]
+    # a sequence's rows: those of the first step, then one in each of the others
+    own = [list(range(a, a + n)) + [T + i * S + s for i in range(after)] for s, (a, n) in enumerate(zip(starts, lens))]
+    want = torch.empty((rows, H * V), dtype=torch.float64)
+    for ids in own:
+        want[ids] = gla_plain(proj[ids], z[ids], bias, norm, H, D, V, tau, eps)
+    state = torch.randn((S + 1, H, V, D), device=DEV)
+    untouched = state[S].clone()
+    state[:S] = 0
+    slots = list(range(S))[::-1]
+    got = [gla_step(lib, proj, z, bias, norm, H, D, V, tau, eps, lens, (0,) * S, slots, state)]
+    for i in range(after):
+        got.append(gla_step(lib, proj, z, bias, norm, H, D, V, tau, eps, (1,) * S, [n + i for n in lens], slots, state, first_row=T + i * S))
+    # as for the steps above: float32 sums of up to a few hundred terms each, or one rounding of the result to 8 bits and its gate's
+    close(torch.cat(got), want, 3e-5 if dtype == torch.float32 else 1.5e-2, f"chunks {D} {lens}")
+    assert torch.equal(state[S], untouched)
+
+
 def test_linear_attention_keeps_what_it_was_told_to():
     """A value written once is read back 400 tokens later through decays close to one (a large temperature), and is gone
     when the decays are small (a temperature of one and inputs below zero)."""

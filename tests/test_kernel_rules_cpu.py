@@ -125,3 +125,14 @@ def test_scratch_of_shared_out_chunks(T, nh, nkv, hd, vd, blocks, bs):
     assert scratch(1, 256, 512, blocks, bs, T, nh, nkv, hd, vd, 0) == scratch(0, 260, 512, blocks, bs, T, nh, nkv, hd, vd, 0) == 0
     assert scratch(0, 256, None, blocks, bs, T, nh, 1, hd, vd, 1) == 0
     assert K.library().pae_paged_attention_scratch(0, 256, 512, 64, 16, 3, 12, 2, 128, 128, 0) == 3 * 12 * 16 * 130
+
+
+@pytest.mark.parametrize("T,S,D", [(1, 1, 128), (160, 1, 128), (319, 2, 64), (320, 2, 64), (320, 1, 32), (4000, 16, 256), (200, 1, 130), (500, 1, 260)])
+def test_scratch_of_linear_attention_by_chunks(T, S, D):
+    """Where a step goes by chunks, whatever its sequences, the scratch of its tokens has room for 16 factors a token and head."""
+    lib, H, V = K.library(), 3, 40
+    part = lambda n: -(-n // 4) * 4
+    rows = 3 * part(T * H * D) + 2 * part(T * H * V)
+    need = rows + part(T * H * (16 if lib.pae_linear_attention_by_chunks(T, S, D) else 1))
+    assert lib.pae_linear_attention_work_floats(T, H, D, V) >= need
+    assert not lib.pae_linear_attention_by_chunks(64, 64, D)
