@@ -239,7 +239,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_skinny_kernel(void* __restrict__
                                part_stride, rope, norm, scale, AHEAD ? &ahead : nullptr);
 }
 
-// The same product for 17..64 rows of A where there are many weight rows.  With several column
+// The same product for 17..64 rows of A where there are many weight rows, where gemm_stream.hip does not take it.  With several column
 // tiles the kernel above is held up by the activations, which every workgroup reads again for its
 // few weight rows, and by adding up its four wavefronts' sums.  Here a workgroup takes 64 RT weight
 // rows, 16 RT per wavefront over the whole k range, and reads each slab of the activations (128 wide

@@ -70,7 +70,7 @@ __global__ __launch_bounds__(128) void gla_prepare_kernel(const T* __restrict__ 
 // 130 ns, and the longest run sets the time; 16 tokens here take 0.85 us, the chain of a chunk's instructions and of its barrier.
 // (The places of a chunk's numbers are lane offsets behind a scalar base: reckoned in 64 bits by every lane a chunk took 1.4 us;
 // with what lies behind a run's end taken out where it is loaded, which waits for it there, 3.2.)  gla_chunk_prepare is bound by
-// its instructions, half of them the decays' logarithms and powers: 36 us for 2,047 tokens of 12 heads, 18 without the factors.
+// its instructions, half of them the decays' logarithms and powers: 36 us for 2,047 tokens of 12 heads, `gla_prepare`'s 25 without the factors.
 // Measured, the whole mixer with 12 heads of 128 x 128: a run of 2,047 tokens 308 -> 152 us, four of 2,047 in all 138 -> 96,
 // 16 of 4,000 220 -> 152.  Against 64 bits, 12 heads, float32 rows, runs of 300 and of 1,500 tokens: read-outs 2.38e-7 -> 2.24e-7
 // and 2.67e-7 -> 2.52e-7, states 2.10e-7 -> 2.00e-7 and 2.62e-7 -> 2.50e-7.

@@ -66,7 +66,8 @@ class StepRunner:
     logits are dropped."""
 
     TABLE_ROUND = 64    # block tables of captured steps are padded to a multiple of this many pages,
-    SHORT_CONTEXT = 128  # but those of sequences up to so many tokens to this: kernels that share out keys then see that they are few
+    SHORT_CONTEXT = 128  # but in float32 those of sequences up to so many tokens to this: its attention, which shares out keys by the
+    # tables' width, then sees that they are few (bfloat16's splits keys at fixed places, whatever the width)
     MAX_GRAPHS = 24
 
     def __init__(self, model: Model, cache: CacheManager, use_graphs: bool = True,
@@ -207,7 +208,7 @@ class StepRunner:
             width = max(1, max(len(t) for t in tables))
             if decode_only:
                 short = max(1, self.SHORT_CONTEXT // cache.block_size)
-                width = short if width <= short else -(-width // self.TABLE_ROUND) * self.TABLE_ROUND
+                width = short if width <= short and self.model.dtype == torch.float32 else -(-width // self.TABLE_ROUND) * self.TABLE_ROUND
             widths.append(width)
 
         # index lists that parts asked for (their kernels' work lists), built from the step's shape
