@@ -1057,3 +1057,35 @@ def test_float32_attention_of_eight_rows_a_workgroup_and_of_nine(nh, nkv, hd):
     """Up to eight rows a wavefront of the kernel that shares a chunk takes one, from nine on two."""
     test_float32_attention_kernels_give_the_same_bits(nh, nkv, hd, hd, 16, 0, False, 0.0, False)
 
+
+
+@pytest.mark.parametrize("nh,nkv,hd,bs", [(12, 2, 128, 16), (3, 1, 64, 8)])
+@pytest.mark.parametrize("silent", [0, 1, 2, 3])
+def test_float32_attention_with_a_chunk_of_scores_of_minus_infinity(nh, nkv, hd, bs, silent):
+    """Sixty-four keys (or the last one alone) whose scores overflow to minus infinity weigh nothing, wherever they stand: by the
+    kernel that shares a chunk, walked and shared out, and by the one with a wavefront per (token, head).  Sums of 250 float32
+    terms each: a few times 2^-24 of the largest value, 2e-5 with room."""
+    torch.manual_seed(7 + silent)
+    for n, new in ((193, 1), (193, 193), (250, 40)):
+        pages = -(-n // bs)
+        keys, values = torch.randn(n, nkv, hd), torch.randn(n, nkv, hd)
+        q = torch.randn(new, nh, hd)
+        q[..., 0], keys[..., 0] = 1e20, 0.0
+        keys[64 * silent:64 * silent + 64, :, 0] = -1e30
+        pad = lambda x: torch.cat([x, torch.full((pages * bs - n, nkv, hd), float("nan"))]).view(pages, bs, nkv, hd)
+        k_pool, v_pool = pad(keys).permute(0, 2, 1, 3).contiguous(), pad(values).permute(0, 2, 3, 1).contiguous()
+        at = torch.arange(n - new, n)
+        scores = torch.einsum("thd,khd->thk", q.double(), keys.double().repeat_interleave(nh // nkv, 1)) * hd ** -0.5
+        scores.masked_fill_(torch.arange(n) > at[:, None, None], -math.inf)
+        want = torch.einsum("thk,khd->thd", scores.softmax(-1), values.double().repeat_interleave(nh // nkv, 1)).reshape(new, nh * hd)
+        seen = at >= (64 if silent == 0 else 0)  # rows with a key whose score is a number
+        outs = []
+        for shift in (0, 1):
+            kc = torch.empty(k_pool.numel() + 4, device=DEV)[shift:shift + k_pool.numel()].view(k_pool.shape).copy_(k_pool)
+            vc = torch.empty(v_pool.numel() + 4, device=DEV)[shift:shift + v_pool.numel()].view(v_pool.shape).copy_(v_pool)
+            out = torch.empty((new, nh * hd), device=DEV)
+            K().paged_attention_generic(out, q.view(new, nh * hd).to(DEV), kc, vc, at.to(torch.int32).to(DEV),
+                                        torch.zeros(new, dtype=torch.int32, device=DEV),
+                                        torch.arange(pages, dtype=torch.int32, device=DEV)[None], nh, nkv, hd, hd ** -0.5, 0)
+            outs.append(out.cpu()[seen])
+        assert torch.equal(outs[0], outs[1]) and float((outs[0].double() - want[seen]).abs().max()) < 2e-5, (n, new)
