@@ -75,7 +75,7 @@ __global__ __launch_bounds__(128) void gla_prepare_kernel(const T* __restrict__ 
 // 16 of 4,000 220 -> 152.  Against 64 bits, 12 heads, float32 rows, runs of 300 and of 1,500 tokens: read-outs 2.38e-7 -> 2.24e-7
 // and 2.67e-7 -> 2.52e-7, states 2.10e-7 -> 2.00e-7 and 2.62e-7 -> 2.50e-7.
 //
-// What is infinite or NaN in a token's row reaches the read-outs of the chunk's earlier tokens as well (as a NaN, by a factor of 0).
+// What is infinite or NaN in a token's row reaches its own read-out and those behind it, as token by token.
 constexpr int GLA_CHUNK = 16;
 // Steps whose runs have that many tokens on average go by chunks; the host knows no run's length.  Both ways in us, 12 heads of 128:
 // one run of 96 24.7 and 26.6, 128 30.6 and 29.1, 160 36.5 and 31.7; 8 runs of 100 57.3 and 60.3, of 138 71.0 and 68.3; 28 heads, two
@@ -249,6 +249,17 @@ __global__ __launch_bounds__(256) void gla_chunks_kernel(const float* __restrict
     x.near = nc[(unsigned)(mine * GLA_CHUNK + 4 * g + wave)];
     return x;
   };
+  // Values that are infinite or NaN, among the tokens 4 g + wave, onto the read-outs of their own token and of those behind it (rare).
+  auto add_no_numbers = [&](float near, float vw, gla_x4& o) {
+    for (int from = 0; from < 4; ++from) {
+      const float value = __shfl(vw, 16 * from + m, PAE_WAVE);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float factor = __shfl(near, 16 * from + 4 * g + i, PAE_WAVE);
+        if (!__builtin_isfinite(value) && 4 * from + wave <= 4 * g + i) o[i] += factor * value;
+      }
+    }
+  };
   auto advance = [&](const Chunk& x, int first, int n, int turn) {
     // the chunk's own tokens: wavefront w takes those 4 g + w
     const float vw = wave == 0 ? x.v[0] : wave == 1 ? x.v[1] : wave == 2 ? x.v[2] : x.v[3];
@@ -257,7 +268,10 @@ __global__ __launch_bounds__(256) void gla_chunks_kernel(const float* __restrict
     for (int i = 0; i < 4; ++i)
 #pragma unroll
       for (int j = 0; j < TW; ++j) o[j % 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.q[j][i], S[j][i], o[j % 2], 0, 0, 0);
-    o[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.near, vw, o[1], 0, 0, 0);
+    // (the instruction multiplies the tokens behind a read-out's own by a factor of zero: what is no number among them goes apart)
+    const bool number = __builtin_isfinite(vw);
+    o[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.near, number ? vw : 0.f, o[1], 0, 0, 0);
+    if (__builtin_amdgcn_ballot_w64(!number) != 0) add_no_numbers(x.near, vw, o[1]);
 #pragma unroll
     for (int j = 0; j < TW; ++j) S[j] *= x.through[j];
 #pragma unroll

@@ -364,6 +364,32 @@ def test_linear_attention_by_chunks(dtype, H, D, V, lens, z_mean, tau):
     assert torch.equal(state[S], untouched)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("what", [float("nan"), float("inf"), -float("inf")])
+@pytest.mark.parametrize("which", ["v", "k", "z"])
+def test_what_is_no_number_in_a_token_stays_behind_the_tokens_before_it(dtype, what, which):
+    """By chunks as token by token: read-outs of earlier tokens, and all of another run's, keep their bits."""
+    H, D, V, lens = 2, 64, 40, (331, 205)
+    lib = K()
+    gen = torch.Generator().manual_seed(3)
+    T = sum(lens)
+    assert lib.library().pae_linear_attention_by_chunks(T, len(lens), D)
+    proj, z, bias, norm = gla_inputs(gen, T, H, D, V, dtype)
+    first = {"v": 2 * H * D, "k": H * D, "z": 0}[which]
+    for at in (0, 15, 16, 165, 200, 330):  # the first and the last token of a chunk, some between, one of the chunk that is not full
+        rows = []
+        for spoiled in (False, True):
+            p, g = proj.clone(), z.clone()
+            if spoiled:
+                (g if which == "z" else p)[at, first + 3] = what
+            state = torch.zeros((2, H, V, D), device=DEV)
+            rows.append(gla_step(lib, p, g, bias, norm, H, D, V, 4.0, 1e-5, lens, (0, 0), [1, 0], state).cpu())
+        clean, got = rows
+        assert torch.equal(got[:at], clean[:at]) and torch.equal(got[lens[0]:], clean[lens[0]:]), (at, which)
+        if which == "v" or math.isnan(what):
+            assert not bool(torch.isfinite(got[at:lens[0]].float()).all(1).any())  # the token's own and those behind it show it
+
+
 def test_linear_attention_keeps_what_it_was_told_to():
     """A value written once is read back 400 tokens later through decays close to one (a large temperature), and is gone
     when the decays are small (a temperature of one and inputs below zero)."""
