@@ -457,6 +457,7 @@ static int wide_product(int mode, int act, int plan, void* out, int64_t ldc, con
 // other, act 1 or 2; 2: float32 [ranges, M, N] of the sums over ranges of k.  Operands begin at multiples of 16 bytes.
 extern "C" int pae_gemm_wide(int mode, int act, int plan, void* out, int64_t ldc, const void* a, int64_t lda, const void* w, const void* bias,
                              int b_is_f32, int M, int N, int K, hipStream_t stream) {
+  PAE_REQUIRE(mode != wide_gemm::ROTATED, "wide product: heads that are rotated have an entry point of their own");
   return wide_product(mode, act, plan, out, ldc, a, lda, w, bias, b_is_f32, M, N, K, Heads{}, stream);
 }
 
@@ -483,7 +484,10 @@ static int wide_product(int mode, int act, int plan, void* out, int64_t ldc, con
   p.splits = ranges;
   p.row_tiles = p.col_tiles = p.strip = p.whole = 0;
   p.heads = heads;
-  if (mode == wide_gemm::ROTATED) return run_shape<wide_gemm::ROTATED, NO_ACT>(shape, p, stream);
+  if (mode == wide_gemm::ROTATED) {
+    PAE_REQUIRE(heads.hd > 0, "wide projection: heads of no width");
+    return run_shape<wide_gemm::ROTATED, NO_ACT>(shape, p, stream);
+  }
   if (mode == wide_gemm::SUMS) return run_shape<wide_gemm::SUMS, NO_ACT>(shape, p, stream);
   if (mode == wide_gemm::PLAIN && act == NO_ACT) return run_shape<wide_gemm::PLAIN, NO_ACT>(shape, p, stream);
   if (mode == wide_gemm::PLAIN && act == 0) return run_shape<wide_gemm::PLAIN, 0>(shape, p, stream);

@@ -136,3 +136,13 @@ def test_scratch_of_linear_attention_by_chunks(T, S, D):
     need = rows + part(T * H * (16 if lib.pae_linear_attention_by_chunks(T, S, D) else 1))
     assert lib.pae_linear_attention_work_floats(T, H, D, V) >= need
     assert not lib.pae_linear_attention_by_chunks(64, 64, D)
+
+
+def test_the_plain_entry_of_wide_products_refuses_rotated_heads():
+    """Mode 3 needs the heads' sizes and pools, which its own entry point brings; the places behind the operands are never read."""
+    lib = K.library()
+    plan = lib.pae_gemm_wide_plan(K.WIDE_GATED, -1, 128, 256, 128, 0)
+    assert lib.pae_gemm_wide(3, -1, plan, 1 << 20, 256, 1 << 20, 128, 1 << 20, None, 0, 128, 256, 128, None) != 0
+    assert "entry point of their own" in lib.pae_last_error().decode()
+    for hd in (0, 32, 80):
+        assert lib.pae_gemm_wide_rope(plan, 1 << 20, 256, 1 << 20, 128, 1 << 20, None, 0, 128, 128, 2, 0, hd, 0, None, None, None, None, 0, 16, None, None, None) != 0
