@@ -646,9 +646,10 @@ def skinny_supported(a: torch.Tensor, w: torch.Tensor) -> bool:
             and a.shape[1] % 8 == 0 and a.stride(0) % 8 == 0 and a.stride(1) == 1 and a.data_ptr() % 16 == 0)
 
 
-def skinny_splits(N: int, K: int, M: int = 1) -> int:
+def skinny_splits(N: int, K: int, M: int = 1, w: Optional[torch.Tensor] = None) -> int:
     """k ranges for a product whose consumer adds float32 partials: enough workgroups to fill the
-    chip (a workgroup takes 16 weight rows, or 32 and more with more than 8 rows of activations)."""
+    chip (a workgroup takes 16 weight rows, or 32 and more with more than 8 rows of activations).
+    `w`: the weights, where they are at hand (see `_streamed_splits`)."""
     rows = 32 if M > 8 else 16
     tiles = -(-N // rows)
     # (ranges of at least 1,024 of k: the 0.5B sizes at 8 rows, O 5.3 us in three ranges and 3.9 in one, down
@@ -684,13 +685,13 @@ def skinny_splits(N: int, K: int, M: int = 1) -> int:
         if M > SAME_ORDER_MAX_ROWS and 4 <= one_round <= 8 and K // one_round >= 1024:
             wanted = one_round
     k_per = -(-(-(-K // wanted)) // 128) * 128
-    return _streamed_splits(N, K, M, -(-K // k_per))
+    return _streamed_splits(N, K, M, -(-K // k_per), w)
 
 
-def _streamed_splits(N: int, K: int, M: int, splits: int) -> int:
+def _streamed_splits(N: int, K: int, M: int, splits: int, w: Optional[torch.Tensor]) -> int:
     """k ranges of a product of more than 16 rows that csrc/gemm_stream.hip takes (several ranges, or many weight rows), by its
-    times; else `splits`, which suit the other kernels."""
-    if M <= SAME_ORDER_MAX_ROWS or (splits == 1 and N <= 3072):
+    times; else, also for weights off 16 bytes, `splits`, which suit the other kernels."""
+    if M <= SAME_ORDER_MAX_ROWS or (splits == 1 and N <= 3072) or (w is not None and w.data_ptr() % 16):
         return splits
     return library().pae_stream_ranges(M, N, K) or splits
 
@@ -705,7 +706,7 @@ def _compute_units() -> int:
     return _UNITS
 
 
-def residual_splits(N: int, K: int, M: int = 1) -> int:
+def residual_splits(N: int, K: int, M: int = 1, w: Optional[torch.Tensor] = None) -> int:
     """k ranges for a product that adds itself into the residual (EPI_RESIDUAL).  Up to 16 rows from
     the product's sizes alone: a row's sums are the same bits whatever it is batched with, launched by
     itself or as a phase of a decode program.  Four ranges run side by side in one workgroup of sixteen
@@ -724,7 +725,7 @@ def residual_splits(N: int, K: int, M: int = 1) -> int:
         # workgroups: 15.6 / 17.9 us against 16.8 / 19.9 with four ranges; 3B down, 64 x 4: 18.5 / 22.9 against
         # 21.8 / 28.4 with five; 7B down: eight, 35 / 47 us; 14B: six, 33 / 44; 14B O: six, 19 / 27 against 27 / 37
         # with two)
-        return skinny_splits(N, K, M)
+        return skinny_splits(N, K, M, w)
     tiles = -(-N // 16)
     # one such workgroup fills a compute unit, so the tiles should fill the chip's units a whole number of
     # times, or nearly (14B/32B down: 320 tiles are a full round and a quarter of one; 32B at 8 rows 86.7 us
@@ -1005,7 +1006,7 @@ def _launch_ticketed(counters, call) -> None:
         raise
 
 
-def whole_sum_splits(N: int, K: int, M: int) -> int:
+def whole_sum_splits(N: int, K: int, M: int, w: Optional[torch.Tensor] = None) -> int:
     """k ranges for a product whose epilogue needs whole sums (gate, rotation, bias), which the
     kernel then adds up itself.  That costs a trip to memory, and pays with more than 8 rows of
     activations where workgroups are few (measured at the 1.5B to 72B layer sizes):
@@ -1013,8 +1014,9 @@ def whole_sum_splits(N: int, K: int, M: int) -> int:
       at 64 rows: 85 -> 72 us; with more weight rows, or somewhat fewer, one range is as fast or faster);
     * few weight rows (the QKV products): ranges of about 1,280 (7B at 64 rows 26 -> 22 us in three,
       14B 37 -> 31 us in four, 72B 87 -> 54 us in six);
-    * not with very few weight rows, where the rows of activations are shared out instead."""
-    tiles, groups = -(-N // 32), -(-N // 128)
+    * not with very few weight rows, where the rows of activations are shared out instead.
+    Most products of more than 16 rows are streamed, with ranges of that kernel's own (`_streamed_splits`, `w` as there);
+    the rules here are for k that is no multiple of 64 and weights off 16 bytes, and for what that kernel leaves."""
     if M <= SAME_ORDER_MAX_ROWS:
         # from the sizes alone, so that a row's sums do not depend on the batch (as `residual_splits`): one
         # range at every size (QKV from HBM at 1 / 8 / 16 rows, one range against the best of two to six: 72B
@@ -1022,30 +1024,33 @@ def whole_sum_splits(N: int, K: int, M: int) -> int:
         # 15.2 / 20.4 against 13.1 / 14.1 / 20.9; gate/up likewise at all seven widths)
         return 1
     waves = -(-(-(-N // 16)) // 256)  # wavefronts of 16 weight rows a workgroup for at most 256 workgroups
-    if 32 < M <= SKINNY_MAX_ROWS and N > 3072:
-        return _streamed_splits(N, K, M, 1)
-    if 5 <= waves <= 8 and -(-(-(-N // 16)) // waves) >= 216:
+    one_a_unit = 5 <= waves <= 8 and -(-(-(-N // 16)) // waves) >= 216
+    if one_a_unit and M <= 32:
         # one workgroup per compute unit, nearly all units busy: one range (the launcher then takes the
-        # kernel of `waves` wavefronts; 1.5B gate/up at 32 rows 19.1 -> 16.7 us, at 64 rows 23.4 -> 22.2)
+        # kernel of `waves` wavefronts; 1.5B gate/up at 32 rows 19.1 -> 16.7 us)
         return 1
+    return _streamed_splits(N, K, M, 1 if one_a_unit else _whole_sum_ranges(N, K, M), w)
+
+
+def _whole_sum_ranges(N: int, K: int, M: int) -> int:
+    """The ranges of `whole_sum_splits` for more than 16 rows in the kernels that do not stream."""
+    tiles, groups = -(-N // 32), -(-N // 128)
     if 128 <= groups < 256:
         # a couple of workgroups of 32 weight rows per compute unit: three ranges from 32
         # rows on (1.5B gate/up at 64 rows 27.2 -> 23.3 us, at 32 rows 20.2 -> 19.0 us; below, one range is ahead)
-        return _streamed_splits(N, K, M, 3 if M >= 32 and K >= 1536 else 1)
-    if tiles <= 96:
+        return 3 if M >= 32 and K >= 1536 else 1
+    if tiles <= 96 or groups >= 384:
         return 1
-    if groups >= 384:
-        return _streamed_splits(N, K, M, 1)
     if groups >= 256:
         wanted = -(-(768 if M > 48 else 512) // groups)
         if K // wanted < 512:
-            return _streamed_splits(N, K, M, 1)
+            return 1
     else:
         # (and no more than make about a thousand 32-row workgroups: 72B QKV at 32 / 64 rows, 320 tiles, six
         # ranges 44.6 / 56.8 us, three 40.3 / 52.9)
         wanted = min(8, max(1, (K + 640) // 1280), max(1, round(1000 / tiles)))
     k_per = -(-(-(-K // wanted)) // 128) * 128
-    return _streamed_splits(N, K, M, -(-K // k_per))
+    return -(-K // k_per)
 
 
 def skinny_rope_supported(a: torch.Tensor, w: torch.Tensor, hd: int, rot: int) -> bool:

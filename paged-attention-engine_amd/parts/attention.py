@@ -315,7 +315,7 @@ class PagedAttention(Part):
         if x.dtype == torch.bfloat16 and K.skinny_rope_supported(x, linear.weight, s.head_dim, rot):
             # up to 64 rows: one kernel projects, rotates and stores
             q = torch.empty((x.shape[0], s.num_heads * s.head_dim), dtype=x.dtype, device=x.device)
-            splits = K.whole_sum_splits(linear.out_features, linear.in_features, x.shape[0])
+            splits = K.whole_sum_splits(linear.out_features, linear.in_features, x.shape[0], linear.weight)
             K.gemm_skinny_rope(q, x, linear.weight, linear.bias, s.num_heads, nkv, s.head_dim, rot, cos_sin,
                                ctx.positions, ctx.tok_seq, table, bs, k_cache, v_cache, splits,
                                row_scale=owed.row_scale if owed is not None else None)

@@ -97,7 +97,7 @@ class Linear:
             plain = Linear(self.weight)
             return BranchTerms([(plain.branch(x), 1.0), (self.bias, 1.0)])
         if x.dtype == torch.bfloat16 and self.bias is None and x.shape[0] and K.skinny_supported(x, self.weight):
-            splits = K.skinny_splits(self.out_features, self.in_features, x.shape[0])
+            splits = K.skinny_splits(self.out_features, self.in_features, x.shape[0], self.weight)
             fold = sink.folded(x.shape[0]) if sink is not None else None
             residual = sink.stream.residual if sink is not None else None
             if (fold is not None and residual.dtype == torch.float32
@@ -106,7 +106,7 @@ class Linear:
                 rows = torch.empty((x.shape[0], self.out_features), dtype=torch.bfloat16, device=x.device)
                 stats = torch.empty((x.shape[0], K.stat_tiles(self.out_features)), dtype=torch.float32, device=x.device)
                 K.gemm_skinny(residual, x, self.weight, None, K.EPI_RESIDUAL,
-                              K.residual_splits(self.out_features, self.in_features, x.shape[0]),
+                              K.residual_splits(self.out_features, self.in_features, x.shape[0], self.weight),
                               following=(rows, weight, stats))
                 sink.deliver(OwedRows(rows, stats, eps))
                 return None
@@ -116,7 +116,7 @@ class Linear:
         if x.dtype == torch.bfloat16 and x.shape[0] and K.skinny_supported(x, self.weight):
             out = torch.empty((x.shape[0], self.out_features), dtype=x.dtype, device=x.device)
             K.gemm_skinny(out, x, self.weight, self.bias, K.EPI_BF16,
-                          K.whole_sum_splits(self.out_features, self.in_features, x.shape[0]))
+                          K.whole_sum_splits(self.out_features, self.in_features, x.shape[0], self.weight))
             return out
         plan = K.wide_plan(x, self.weight, K.WIDE_SUMS, ranges=True) if sink is not None and self.bias is None else None
         if plan is not None and plan >> 8 > 1:

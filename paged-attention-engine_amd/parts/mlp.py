@@ -65,12 +65,12 @@ class SwiGLU(Part):
         plan = (K.wide_plan(x, self.gate_up.weight, K.WIDE_GATED, self.spec.activation)
                 if self.block and not isinstance(x, OwedRows) else None)
         if self.silu and self.block and x.shape[0] and K.skinny_supported(rows, self.gate_up.weight):
-            splits = K.whole_sum_splits(2 * self.spec.intermediate_size, self.spec.hidden_size, x.shape[0])
+            splits = K.whole_sum_splits(2 * self.spec.intermediate_size, self.spec.hidden_size, x.shape[0], self.gate_up.weight)
             K.gemm_skinny(act, rows, self.gate_up.weight, None, K.EPI_SWIGLU, splits,
                           row_scale=x.row_scale if isinstance(x, OwedRows) else None)
         elif self.block and x.shape[0] and K.skinny_supported(rows, self.gate_up.weight) and not isinstance(x, OwedRows):
             # another activation: the same product and layout, the activation by name in its epilogue
-            splits = K.whole_sum_splits(2 * self.spec.intermediate_size, self.spec.hidden_size, x.shape[0])
+            splits = K.whole_sum_splits(2 * self.spec.intermediate_size, self.spec.hidden_size, x.shape[0], self.gate_up.weight)
             K.gemm_skinny_gated(act, rows, self.gate_up.weight, self.spec.activation, splits)
         elif plan is not None:
             K.gemm_wide(act, x, self.gate_up.weight, plan, kind=self.spec.activation, mode=K.WIDE_GATED)
@@ -120,7 +120,7 @@ class DenseFeedForward(Part):
         plan = K.wide_plan(x, self.up.weight, K.WIDE_PLAIN, self.spec.activation, bias=self.up.bias)
         if x.shape[0] and K.skinny_supported(x, self.up.weight):
             act = torch.empty((x.shape[0], self.spec.intermediate_size), dtype=x.dtype, device=x.device)
-            splits = K.whole_sum_splits(self.spec.intermediate_size, self.spec.hidden_size, x.shape[0])
+            splits = K.whole_sum_splits(self.spec.intermediate_size, self.spec.hidden_size, x.shape[0], self.up.weight)
             K.gemm_skinny_act(act, x, self.up.weight, self.spec.activation, splits, self.up.bias)
         elif plan is not None:
             act = torch.empty((x.shape[0], self.spec.intermediate_size), dtype=x.dtype, device=x.device)

@@ -146,3 +146,16 @@ def test_the_plain_entry_of_wide_products_refuses_rotated_heads():
     assert "entry point of their own" in lib.pae_last_error().decode()
     for hd in (0, 32, 80):
         assert lib.pae_gemm_wide_rope(plan, 1 << 20, 256, 1 << 20, 128, 1 << 20, None, 0, 128, 128, 2, 0, hd, 0, None, None, None, None, 0, 16, None, None, None) != 0
+
+
+@pytest.mark.parametrize("M,N,k,ranges", [(64, 4608, 3592, 3), (64, 37888, 3592, 3), (48, 37888, 3592, 2), (33, 10240, 18952, 3), (64, 17920, 1544, 1),
+                                          (64, 16384, 1544, 3), (32, 16384, 1544, 3), (31, 16384, 1544, 1), (64, 2048, 3592, 1), (16, 4608, 3592, 1)])
+def test_ranges_of_products_that_are_not_streamed(M, N, k, ranges):
+    """k that is no multiple of 64, and weights off 16 bytes, which leave the streamed products' ranges to the other kernels' own rule."""
+    assert K.whole_sum_splits(N, k, M) == ranges
+    off = torch.empty(8, dtype=torch.bfloat16)[1:]
+    assert off.data_ptr() % 16
+    assert K.whole_sum_splits(N, k // 64 * 64, M, off) == K.whole_sum_splits(N, k // 64 * 64 + 8, M)
+    assert K.skinny_splits(N, k, M, off) == K.skinny_splits(N, k, M) and K.residual_splits(2048, k, M, off) == K.residual_splits(2048, k, M)
+    streamed = K.library().pae_stream_ranges(M, 4608, 3584)
+    assert K.whole_sum_splits(4608, 3584, M) == (streamed or 1)
