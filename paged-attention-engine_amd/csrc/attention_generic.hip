@@ -479,12 +479,13 @@ static int rows_of_a_workgroup(int num_tokens, int nh, int nkv, int& heads_each,
 // chip idle and the chunks are three or more (a token at 60 keys 9.5 and 11.3; 14 heads of 64 at 75 about 8 and 9): 12 heads over 2 of
 // 128, in us, walked and shared: three tokens at 200 keys 20.7 and 12.1, eight at 1,000 71 and 13.4, at
 // 4,000 278 and 49, 64 at 1,000 77 and 71 (128 workgroups), 40 tokens behind 2,000 142 and 85 (80); but a prompt of 200 tokens (400)
-// 33 and 44, 600 tokens 111 and 173: a workgroup's start and end, 5 us, then come once a chunk.
+// 33 and 44, 600 tokens 111 and 173: a workgroup's start and end, 5 us, then come once a chunk.  (All with a token a workgroup: where several
+// share one, from 512 such workgroups on, they walk.)
 static int split_chunks(int num_tokens, int nh, int nkv, int vd, int max_blocks, int bs) {
   int heads_each, parts;
-  const int toks = rows_of_a_workgroup(num_tokens, nh, nkv, heads_each, parts);
+  rows_of_a_workgroup(num_tokens, nh, nkv, heads_each, parts);
   const int64_t chunks = ((int64_t)max_blocks * bs + PAE_WAVE - 1) / PAE_WAVE;
-  const int64_t groups = (int64_t)((num_tokens + toks - 1) / toks) * nkv * parts;
+  const int64_t groups = (int64_t)num_tokens * nkv * parts;
   if (chunks < 3 || chunks > 65535 || groups > SPLIT_GROUPS || (int64_t)num_tokens * nh * chunks * (vd + 2) > SPLIT_FLOATS) return 1;
   return (int)chunks;
 }

@@ -114,7 +114,9 @@ def test_ranges_of_streamed_products_fit_their_scratch(M):
 
 
 @pytest.mark.parametrize("T,nh,nkv,hd,vd,blocks,bs", [(1, 12, 2, 128, 128, 64, 16), (64, 12, 2, 128, 128, 64, 16), (65, 12, 2, 128, 128, 64, 16),
-                                                      (3, 40, 1, 64, 64, 5, 16), (8, 16, 16, 64, 200, 3, 64), (1, 1, 1, 4, 4, 8, 16), (2, 8, 2, 256, 256, 6000, 16)])
+                                                      (3, 40, 1, 64, 64, 5, 16), (8, 16, 16, 64, 200, 3, 64), (43, 12, 12, 64, 64, 64, 16),
+                                                      (64, 16, 16, 64, 64, 64, 16), (520, 1, 1, 64, 64, 64, 16), (100, 16, 8, 64, 64, 64, 16),
+                                                      (9, 80, 1, 64, 64, 64, 16), (1, 1, 1, 4, 4, 8, 16), (2, 8, 2, 256, 256, 6000, 16)])
 def test_scratch_of_shared_out_chunks(T, nh, nkv, hd, vd, blocks, bs):
     """Every chunk's sums have room, within 64 MiB; what is not asked of the library has none; other types and pools use none."""
     scratch = lambda *args: K.library().pae_paged_attention_scratch(*args)
