@@ -419,6 +419,13 @@ int run_shape(int shape, const Product& p, hipStream_t stream) {
 
 }  // namespace
 
+// Microseconds of a projection by the platform's library and the kernel that rotates and stores behind it, where the rule below leaves the
+// product to the library: met within 11 % (root mean square) over 187 such products of 12 widths of heads (768 to 12,288 rows of W, k 2,048 to
+// 8,192) by 65 to 6,030 rows.
+static double library_and_rotation_time(int M, int N, int K) {
+  return 12.8 + 0.80e-9 * M * N * K + 0.72e-6 * N * K + 2.3e-6 * M * N + 1.8e-6 * M * K;
+}
+
 // The shape for a product, in the low byte, and its ranges of k behind that.  `mode` as for pae_gemm_wide; `ranges` != 0: the
 // product may leave float32 sums of ranges of k for a caller that reads them again (counted at 3.6 TB/s against one bfloat16
 // result).  -1: the platform library, which shares a product out over k, for one without an activation that no shape here fills
@@ -428,12 +435,17 @@ int run_shape(int shape, const Product& p, hipStream_t stream) {
 // to 64 tiles 0.84 to 1.83 times its time, 1.30 on average, and up to 128 0.85 to 1.26, 1.04 on average (128 x 896 x 4,864 23.9 against 13.1
 // us, 300 x 256 x 4,096 18.6 against 11.2, 65 x 16 x 8,192 22.4 against 8.3).  Up to 35 stages as few tiles are ahead (65 x 1,536 x 2,240 8.8
 // against 11.4), and so are 128 to 256 of them (0.84 on average).
+// Heads that are rotated (mode 3) leave the library its products only where that and a rotation behind it are ahead by their times: over
+// those 187 products the tiles with the rotation in them take 0.94 of its time with this rule and 1.01 without, 1.09 at worst and
+// 1.71 (us, tiles and library: 65 x 1,536 x 8,192 35.2 and 20.9, 127 x 768 x 4,096 22.6 and 15.6, 993 x 1,536 x 8,192 67.6 and 52.5, 240 x
+// 5,120 x 6,144 64.0 and 51.3, which go to the library; 993 x 4,608 x 3,584 56.8 and 63.6, 385 x 7,168 x 5,120 44.4 and 65.6, 127 x 10,240 x 8,192
+// 80.9 and 74.3, which do not).
 extern "C" int pae_gemm_wide_plan(int mode, int act, int M, int N, int K, int ranges) {
   static const int CUTS[] = {2, 3, 4, 5, 6, 8};
   int best = SHAPE_LARGE, cuts = 1;
   double least = 1e30;
   for (int shape = 0; shape < SHAPES; ++shape) {
-    if ((shape == SHAPE_128_96 && mode == wide_gemm::GATED) || (shape == SHAPE_LARGE && K < 128)) continue;
+    if ((shape == SHAPE_128_96 && (mode == wide_gemm::GATED || mode == wide_gemm::ROTATED)) || (shape == SHAPE_LARGE && K < 128)) continue;
     const double t = shape_time(shape, M, N, K, 1);
     if (t < least) least = t, best = shape;
   }
@@ -445,6 +457,9 @@ extern "C" int pae_gemm_wide_plan(int mode, int act, int M, int N, int K, int ra
     }
   if (mode == wide_gemm::PLAIN && act == NO_ACT &&
       ((least > 30.0 && 2.0 * M * N * K / least < 0.95e9) || (K >= 48 * 64 && tiles_of(M, N, 64, 64) <= UNITS / 2)))
+    return -1;
+  if (mode == wide_gemm::ROTATED && pae_gemm_wide_plan(wide_gemm::PLAIN, NO_ACT, M, N, K, 0) < 0 &&
+      1.05 * least + 1.3 + 0.9e-6 * M * N > 0.95 * library_and_rotation_time(M, N, K))
     return -1;
   return best | cuts << 8;
 }
@@ -499,7 +514,7 @@ static int wide_product(int mode, int act, int plan, void* out, int64_t ldc, con
 
 // A W^T + bias, W [(nh + 2 nkv) hd, K] the projections to query, key and value heads: query heads, their first `rot` features rotated in pairs
 // (i, i + rot / 2), to out [M, nh hd], key heads rotated likewise and value heads to their places in the pages, as pae_rope_kv_write
-// puts them.  `plan` as pae_gemm_wide_plan gives it for mode 1.  nkv may be 0: only queries.
+// puts them.  `plan` as pae_gemm_wide_plan gives it for mode 3.  nkv may be 0: only queries.
 extern "C" int pae_gemm_wide_rope(int plan, void* out, int64_t ldc, const void* a, int64_t lda, const void* w, const void* bias, int b_is_f32,
                                   int M, int K, int nh, int nkv, int hd, int rot, const float* cos_sin, const int* positions, const int* tok_seq,
                                   const int* block_tables, int max_blocks, int bs, void* k_cache, void* v_cache, hipStream_t stream) {

@@ -837,7 +837,7 @@ CHECK_TICKET_SUMS = os.environ.get("PAE_CHECK_TICKETS", "") == "sums"
 
 
 # Products of more rows than the few-row kernels take (csrc/gemm_wide.hip).  `plan`: how one is made, as `wide_plan` gives it.
-WIDE_PLAIN, WIDE_GATED, WIDE_SUMS = 0, 1, 2
+WIDE_PLAIN, WIDE_GATED, WIDE_SUMS, WIDE_ROTATED = 0, 1, 2, 3
 WIDE_ACTIVATIONS = {WIDE_PLAIN: ("gelu", "relu2"), WIDE_GATED: ("gelu_tanh", "silu")}  # those that the product's epilogue knows
 _WIDE_STRIDE = 1 << 22
 
@@ -884,10 +884,11 @@ def gemm_wide(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, plan: int, bi
 
 def wide_rope_plan(a: torch.Tensor, w: torch.Tensor, hd: int, rot: int, bias: Optional[torch.Tensor] = None, cos_sin: Optional[torch.Tensor] = None,
                    k_cache: Optional[torch.Tensor] = None) -> Optional[int]:
-    """How `gemm_wide_rope` makes this projection, or None: sizes or operands that it does not take."""
+    """How `gemm_wide_rope` makes this projection, or None: sizes or operands that it does not take, or that the platform's library and a
+    kernel behind it are ahead at."""
     if hd % 64 or rot % 64 or any(t is not None and t.data_ptr() % 16 for t in (cos_sin, k_cache)) or (256 + hd) * a.shape[-1] >= 1 << 31:
         return None
-    return wide_plan(a, w, WIDE_GATED, bias=bias)
+    return wide_plan(a, w, WIDE_ROTATED, bias=bias)
 
 
 def gemm_wide_rope(q_out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], plan: int, nh: int, nkv: int, hd: int,

@@ -161,3 +161,13 @@ def test_ranges_of_products_that_are_not_streamed(M, N, k, ranges):
     assert K.skinny_splits(N, k, M, off) == K.skinny_splits(N, k, M) and K.residual_splits(2048, k, M, off) == K.residual_splits(2048, k, M)
     streamed = K.library().pae_stream_ranges(M, 4608, 3584)
     assert K.whole_sum_splits(4608, 3584, M) == (streamed or 1)
+
+
+def test_projections_that_the_library_is_ahead_at_are_not_rotated_in_tiles():
+    """Few tiles with much of k, as for plain products, go to the library and a rotation behind it; elsewhere the tiles are those of gated products."""
+    plan = K.library().pae_gemm_wide_plan
+    for M, N, k in ((65, 1536, 8192), (127, 768, 4096), (240, 768, 4096), (993, 1536, 8192), (240, 5120, 6144), (127, 1280, 3072)):
+        assert plan(K.WIDE_ROTATED, -1, M, N, k, 0) == plan(K.WIDE_PLAIN, -1, M, N, k, 0) == -1, (M, N, k)
+    for M, N, k in ((65, 1152, 896), (2048, 2048, 1536), (2500, 2560, 2048), (993, 4608, 3584), (6030, 4608, 3584), (385, 7168, 5120), (300, 12288, 4096),
+                    (6000, 1536, 8192), (700, 768, 4096), (70, 2048, 64)):
+        assert plan(K.WIDE_ROTATED, -1, M, N, k, 0) == plan(K.WIDE_GATED, -1, M, N, k, 0) >= 0, (M, N, k)
