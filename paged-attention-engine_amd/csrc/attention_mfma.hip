@@ -705,6 +705,9 @@ extern "C" int pae_attn_decode_bf16(void* out, int64_t out_stride, const void* q
 //   * 32-token workgroups that are one round of the chip and meet about a thousand keys: the kernel above, which has no
 //     LDS to fill before its first product (12 heads, 128 tokens: 7.7, two query groups 8.9; 512 tokens 10.5 and 11.3; 1,024
 //     tokens, 384 workgroups, 19.2 and 14.6; 64 tokens behind 3,000 28.4 and 25.3).
+//     A round as launched, counting the 32-token parts that a run does not have: where more are launched, those that wait for a unit
+//     cost a second start unless enough parts are empty (12 heads, runs of 90: five, 240 launched, 7.2 and 8.4, six, 288, 12.0 and 8.5; six of
+//     60 7.1 and 8.2; 28 heads, three of 90 11.8 and 8.6).  Heads of 64 fit a unit twice (20 heads, six of 60 6.0 and 6.1).
 //   * else two query groups where 64-token workgroups are one round, and for heads of 64 always (two of its workgroups fit a
 //     compute unit: 14 heads, 4,096 tokens 47.2, four groups 49.2);
 //   * else whichever ends sooner as a row of workgroups of (start and end + keys) dealt to 256 compute units, longest
@@ -716,7 +719,7 @@ static int route_of(int nh, int hd, int vd, int bs, int num_tiles, int tokens, i
   const double few = nh * fmin(4 * runs, tokens / 32.0 + runs / 2), two = nh * fmin(2 * runs, tokens / 64.0 + runs / 2), four = nh * runs;
   double keys = 16.0 * max_blocks;
   if (window > 0) keys = fmin(keys, window + (double)PREFILL_RUN);
-  if (few <= 288 && keys <= 1024) return 0;
+  if ((4 * nh * runs <= 256 || few <= (hd == 64 ? 288 : 232)) && keys <= 1024) return 0;
   if (hd == 64 || two <= 256) return 2;
   const double mean = tokens < keys ? keys - 0.5 * tokens : 0.5 * keys;
   auto time = [&](double groups, double start, double per_key) {
@@ -742,14 +745,16 @@ static int check_route(const char* what, int route, int hd, int vd, int bs, cons
 
 // tiles[t] = (table row of the sequence, first flat token, number of tokens <= 128), heaviest runs
 // first: workgroups start in the order of the grid, and the last to finish sets the time.
-// `tokens`: the step's rows, as many as the runs have or a few more.  `route`: what `route_of` says, or -1 to ask it.
+// `tokens`: the step's rows, as many as the runs have or a few more.  `keys`: the most keys that a run sees, or 0: the tables' width (a step's
+// tables are as wide as its longest sequence, which may be one that brings a single token and is not among the runs).  `route`: what
+// `route_of` says, or -1 to ask it.
 static int attn_prefill_any(void* out, int64_t out_stride, const void* q, int64_t q_stride,
                                           const void* k_cache, const void* v_cache, const int* tiles,
                                           int num_tiles, const int* positions, const int* block_tables,
                                           int max_blocks, int bs, int nh, int nkv, int hd, float scale, int window,
                                           float cap, const float* sinks, bool biased, int chunked, const float* slopes,
                                           const void* gate, int64_t gate_stride, const void* head_gate,
-                                          int64_t head_gate_stride, int tokens, int route, hipStream_t stream) {
+                                          int64_t head_gate_stride, int tokens, int keys, int route, hipStream_t stream) {
   if (int rc = check_common("attn_prefill", nh, nkv, hd, bs, max_blocks, window)) return rc;
   PAE_REQUIRE(!biased || cap == 0.f, "attn_prefill: a bias by distance and a score cap together are not built");
   PAE_REQUIRE(!biased || !slopes || scale > 0.f, "attn_prefill: a bias by distance needs a positive scale");
@@ -764,7 +769,7 @@ static int attn_prefill_any(void* out, int64_t out_stride, const void* q, int64_
   PAE_REQUIRE(cap >= 0.f && (cap == 0.f || scale > 0.f), "attn_prefill: bad score cap %g (scale %g)", (double)cap, (double)scale);
   const float cap_over_scale = cap > 0.f ? cap / scale : 0.f, scale_over_cap = cap > 0.f ? scale / cap : 0.f;
   // (pages that do not start on 16 bytes, which the loads to LDS need, stay here)
-  if (route < 0) route = ((uintptr_t)k_cache | (uintptr_t)v_cache) % 16 ? 0 : route_of(nh, hd, hd, bs, num_tiles, tokens, max_blocks, window);
+  if (route < 0) route = ((uintptr_t)k_cache | (uintptr_t)v_cache) % 16 ? 0 : route_of(nh, hd, hd, bs, num_tiles, tokens, keys > 0 ? (keys + 15) / 16 : max_blocks, window);
   if (route > 0) {
     const PrefillArgs args = {(bf16_t*)out, out_stride, (const bf16_t*)q, q_stride, (const bf16_t*)k_cache, (const bf16_t*)v_cache,
                               tiles, num_tiles, positions, block_tables, max_blocks, nh, nkv, scale_log2, window, cap_over_scale,
@@ -815,10 +820,10 @@ extern "C" int pae_attn_prefill_capped_bf16(void* out, int64_t out_stride, const
                                           int num_tiles, const int* positions, const int* block_tables,
                                           int max_blocks, int bs, int nh, int nkv, int hd, float scale, int window,
                                           float cap, const float* sinks, const void* head_gate, int64_t head_gate_stride,
-                                          int tokens, int route, hipStream_t stream) {
+                                          int tokens, int keys, int route, hipStream_t stream) {
   return attn_prefill_any(out, out_stride, q, q_stride, k_cache, v_cache, tiles, num_tiles, positions, block_tables,
                           max_blocks, bs, nh, nkv, hd, scale, window, cap, sinks, false, 0, nullptr, nullptr, 0, head_gate,
-                          head_gate_stride, tokens, route, stream);
+                          head_gate_stride, tokens, keys, route, stream);
 }
 
 extern "C" int pae_attn_prefill_biased_bf16(void* out, int64_t out_stride, const void* q, int64_t q_stride,
@@ -826,10 +831,10 @@ extern "C" int pae_attn_prefill_biased_bf16(void* out, int64_t out_stride, const
                                           int num_tiles, const int* positions, const int* block_tables,
                                           int max_blocks, int bs, int nh, int nkv, int hd, float scale, int window,
                                           int chunked, const float* slopes, const void* gate, int64_t gate_stride,
-                                          int tokens, int route, hipStream_t stream) {
+                                          int tokens, int keys, int route, hipStream_t stream) {
   return attn_prefill_any(out, out_stride, q, q_stride, k_cache, v_cache, tiles, num_tiles, positions, block_tables,
                           max_blocks, bs, nh, nkv, hd, scale, window, 0.f, nullptr, true, chunked, slopes, gate, gate_stride,
-                          nullptr, 0, tokens, route, stream);
+                          nullptr, 0, tokens, keys, route, stream);
 }
 
 extern "C" int pae_attn_prefill_bf16(void* out, int64_t out_stride, const void* q, int64_t q_stride,
@@ -838,7 +843,7 @@ extern "C" int pae_attn_prefill_bf16(void* out, int64_t out_stride, const void* 
                                      int nkv, int hd, float scale, int window, hipStream_t stream) {
   return pae_attn_prefill_capped_bf16(out, out_stride, q, q_stride, k_cache, v_cache, tiles, num_tiles, positions,
                                       block_tables, max_blocks, bs, nh, nkv, hd, scale, window, 0.f, nullptr, nullptr, 0,
-                                      num_tiles * PREFILL_RUN, -1, stream);
+                                      num_tiles * PREFILL_RUN, 0, -1, stream);
 }
 
 // Key widths `hd` (multiples of 32 up to 256) built for values `vd` wide: the smallest that holds `width` features, or 0.

@@ -136,9 +136,9 @@ def _declare(lib) -> None:
         "pae_attn_decode_bf16": [P, L, P, L, P, P, P, I, P, I, I, I, I, I, F, I, P, P, P],
         "pae_attn_decode_split": [],
         "pae_attn_decode_biased_bf16": [P, L, P, L, P, P, P, I, P, I, I, I, I, I, F, I, I, P, P, L, P, P, P],
-        "pae_attn_prefill_biased_bf16": [P, L, P, L, P, P, P, I, P, P, I, I, I, I, I, F, I, I, P, P, L, I, I, P],
+        "pae_attn_prefill_biased_bf16": [P, L, P, L, P, P, P, I, P, P, I, I, I, I, I, F, I, I, P, P, L, I, I, I, P],
         "pae_attn_decode_capped_bf16": [P, L, P, L, P, P, P, I, P, I, I, I, I, I, F, I, F, P, P, L, P, P, P],
-        "pae_attn_prefill_capped_bf16": [P, L, P, L, P, P, P, I, P, P, I, I, I, I, I, F, I, F, P, P, L, I, I, P],
+        "pae_attn_prefill_capped_bf16": [P, L, P, L, P, P, P, I, P, P, I, I, I, I, I, F, I, F, P, P, L, I, I, I, P],
         "pae_attn_prefill_bf16": [P, L, P, L, P, P, P, I, P, P, I, I, I, I, I, F, I, P],
         "pae_program_phase_bytes": [],
         "pae_program_barrier_bytes": [],
@@ -2188,13 +2188,14 @@ def attn_prefill(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v_ca
                  tiles: torch.Tensor, positions: torch.Tensor, block_tables: torch.Tensor,
                  nh: int, nkv: int, hd: int, scale: float, window: int, softcap: float = 0.0,
                  sinks: Optional[torch.Tensor] = None, chunked: bool = False, slopes: Optional[torch.Tensor] = None,
-                 gate: Optional[torch.Tensor] = None, head_gate: Optional[torch.Tensor] = None, route: int = -1) -> None:
+                 gate: Optional[torch.Tensor] = None, head_gate: Optional[torch.Tensor] = None, route: int = -1, keys: int = 0) -> None:
     """Attention of runs of consecutive tokens; tiles[t] = (table row of the sequence, first
     flat token, number of tokens <= PREFILL_TILE).  Workgroups per run and head, whose
     wavefronts share out the keys, start in the order of `tiles`, so the runs with
     the most keys should come first.  `softcap`, `sinks`, `chunked`, `slopes`, `gate` and `head_gate` as in `attn_decode`.
     `route`: -1 lets the sizes choose the kernel; 0 is the one for any shape, 2 and 4 share the keys through LDS between as
-    many groups of 32 tokens (heads of 128, 2 also of 64, pages of 16)."""
+    many groups of 32 tokens (heads of 128, 2 also of 64, pages of 16).  `keys`: the most keys that a run sees, for that choice (0: as
+    many as the tables hold, which is more where a sequence that is not among the runs is longer)."""
     _not_while_recording("attn_prefill")
     _gpu(out, q, k_cache, v_cache, tiles, positions, block_tables, sinks, slopes, gate, head_gate)
     if head_gate is not None:
@@ -2215,13 +2216,13 @@ def attn_prefill(out: torch.Tensor, q: torch.Tensor, k_cache: torch.Tensor, v_ca
         _check(library().pae_attn_prefill_biased_bf16(
             out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0), k_cache.data_ptr(), v_cache.data_ptr(),
             tiles.data_ptr(), tiles.shape[0], positions.data_ptr(), block_tables.data_ptr(), block_tables.shape[1],
-            bs, nh, nkv, hd, float(scale), int(window), 1 if chunked else 0, _ptr(slopes), gp, gs, q.shape[0], int(route), _stream()))
+            bs, nh, nkv, hd, float(scale), int(window), 1 if chunked else 0, _ptr(slopes), gp, gs, q.shape[0], int(keys), int(route), _stream()))
         return
     _check(library().pae_attn_prefill_capped_bf16(
         out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0), k_cache.data_ptr(), v_cache.data_ptr(),
         tiles.data_ptr(), tiles.shape[0], positions.data_ptr(), block_tables.data_ptr(), block_tables.shape[1],
         bs, nh, nkv, hd, float(scale), int(window), float(softcap), _ptr(sinks), _ptr(head_gate),
-        head_gate.stride(0) if head_gate is not None else 0, q.shape[0], int(route), _stream()))
+        head_gate.stride(0) if head_gate is not None else 0, q.shape[0], int(keys), int(route), _stream()))
 
 
 def sample(tokens: torch.Tensor, logits: torch.Tensor, temperature: Optional[torch.Tensor],

@@ -54,6 +54,7 @@ from .delta import sequence_runs
 from .linear import Linear, rows_a_graph_may_hold
 
 WORK_LISTS = ("paged attention work lists", K.PREFILL_TILE)
+MOST_KEYS = "the most keys a run of tokens sees"  # the key of a step's memo for `most_keys`
 SOURCE_VALUES = "values of the layer that others mix in"  # the key of a step's memo under which they wait
 CONV_LISTS = ("paged attention work lists and sequence runs", K.PREFILL_TILE)
 
@@ -76,18 +77,26 @@ def attention_work_lists(shape: StepShape):
     return {"decode_work": (decode_work, 4), "prefill_tiles": ([x for _, tile in runs for x in tile], 3)}
 
 
+def most_keys(ctx) -> int:
+    """The most keys that a run of several tokens sees in this step (its tables are as wide as its longest sequence)."""
+    if MOST_KEYS not in ctx.memo:
+        ctx.memo[MOST_KEYS] = max((past + n for n, past in zip(ctx.q_lens, ctx.past_lens) if n > 1), default=0)
+    return ctx.memo[MOST_KEYS]
+
+
 def attend_paged(attn, q, k_cache, v_cache, positions, tok_seq, table, work, num_heads: int, num_kv_heads: int,
-                 head_dim: int, value_dim: int, scale: float, window: int, softcap: float, sinks, head_gate=None) -> None:
+                 head_dim: int, value_dim: int, scale: float, window: int, softcap: float, sinks, head_gate=None,
+                 keys: int = 0) -> None:
     """Attention of a step's queries over the paged cache into `attn`: with `work` (the device lists of
     `attention_work_lists`) on the matrix cores, single tokens by the decode kernel and runs of tokens by
-    the prefill kernel; without, by the kernel that takes any shape and precision."""
+    the prefill kernel; without, by the kernel that takes any shape and precision.  `keys`: the most that a run sees, if known."""
     if work is not None:
         geometry = (num_heads, num_kv_heads, head_dim, scale, window, softcap, sinks)
         decode_work, prefill_tiles = work["decode_work"], work["prefill_tiles"]
         if decode_work.numel():
             K.attn_decode(attn, q, k_cache, v_cache, decode_work, table, *geometry, head_gate=head_gate)
         if prefill_tiles.numel():
-            K.attn_prefill(attn, q, k_cache, v_cache, prefill_tiles, positions, table, *geometry, head_gate=head_gate)
+            K.attn_prefill(attn, q, k_cache, v_cache, prefill_tiles, positions, table, *geometry, head_gate=head_gate, keys=keys)
     elif head_gate is not None:
         K.paged_attention_masked(attn, q, k_cache, v_cache, positions, tok_seq, table, num_heads, num_kv_heads,
                                  head_dim, value_dim, scale, window, softcap=softcap, sinks=sinks, head_gate=head_gate)
@@ -372,7 +381,7 @@ class PagedAttention(Part):
         attn = torch.empty((qkv.shape[0], s.num_heads * s.v_dim), dtype=qkv.dtype, device=qkv.device)
         work = ctx.memo.get(WORK_LISTS) if self._matrix_cores(ctx.cache.block_size) else None
         attend_paged(attn, qkv, pages["k"], pages["v"], ctx.positions, ctx.tok_seq, table, work, s.num_heads,
-                     s.num_kv_heads, s.head_dim, s.v_dim, s.scale, s.window or 0, s.softcap or 0.0, self.sinks, gate)
+                     s.num_kv_heads, s.head_dim, s.v_dim, s.scale, s.window or 0, s.softcap or 0.0, self.sinks, gate, most_keys(ctx))
         return self.out.branch(attn, ctx.sink)
 
     def _forward_convolved(self, ctx, x):
@@ -405,7 +414,8 @@ class PagedAttention(Part):
             if lists["decode_work"].numel():
                 K.attn_decode(attn, q, pages["k"], pages["v"], lists["decode_work"], table, *geometry)
             if lists["prefill_tiles"].numel():
-                K.attn_prefill(attn, q, pages["k"], pages["v"], lists["prefill_tiles"], ctx.positions, table, *geometry)
+                K.attn_prefill(attn, q, pages["k"], pages["v"], lists["prefill_tiles"], ctx.positions, table, *geometry,
+                               keys=most_keys(ctx))
         else:
             K.paged_attention_masked(attn, q, pages["k"], pages["v"], ctx.positions, ctx.tok_seq, table, s.num_heads,
                                      s.num_kv_heads, s.head_dim, s.v_dim, s.scale, s.window or 0, chunked, self.slopes, gate)
@@ -430,7 +440,7 @@ class PagedAttention(Part):
             if decode_work.numel():
                 K.attn_decode(attn, qkv, k_cache, v_cache, decode_work, table, *geometry)
             if prefill_tiles.numel():
-                K.attn_prefill(attn, qkv, k_cache, v_cache, prefill_tiles, ctx.positions, table, *geometry)
+                K.attn_prefill(attn, qkv, k_cache, v_cache, prefill_tiles, ctx.positions, table, *geometry, keys=most_keys(ctx))
         else:
             K.paged_attention_generic(attn, qkv, k_cache, v_cache, ctx.positions, ctx.tok_seq, table, *geometry)
         return self.out.branch(attn, ctx.sink)

@@ -154,3 +154,22 @@ def test_formed_heads_with_sinks(R, V, window, pad):
     # the roundings of weights, their sum and the result as above; the keys' and values' own, which the oracle repeats, fall on the other
     # side of a tie where the product's sum in 32 bits does: 2^-8 of one of 128 terms of a score, and of a value
     assert ((out.cpu().double() - want).abs() <= 2.0 ** -8 * (2 * sizes + 2 * want.abs()) + 1e-3).all()
+
+
+def test_runs_choose_a_kernel_by_the_keys_they_see():
+    """In tables that a longer sequence made wide: the bits of tables as wide as the run, if the run's keys are told."""
+    nh, nkv, hd, n = 12, 2, 128, 100
+    q, k, v, table, _, _ = inputs([(0, n)], nh, nkv, hd, hd, 5, [0])
+    tiles, at = torch.tensor([[0, 0, n]], dtype=torch.int32, device=DEV), torch.arange(n, dtype=torch.int32, device=DEV)
+    wide = torch.full((1, 256), -1, dtype=torch.int32)
+    wide[:, :table.shape[1]] = table
+
+    def run(table, **how):
+        out = torch.empty(n, nh * hd, dtype=torch.bfloat16, device=DEV)
+        K.attn_prefill(out, q.to(DEV), k.to(DEV), v.to(DEV), tiles, at, table.to(DEV), nh, nkv, hd, hd ** -0.5, 0, **how)
+        return out
+
+    routes = K.library().pae_attn_prefill_route
+    assert routes(nh, hd, hd, 16, 1, n, table.shape[1], 0) == 0 and routes(nh, hd, hd, 16, 1, n, 256, 0) == 2
+    assert torch.equal(run(wide, keys=n), run(table)) and torch.equal(run(wide, keys=n), run(wide, route=0))
+    assert torch.equal(run(wide), run(wide, route=2))

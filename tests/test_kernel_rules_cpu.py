@@ -171,3 +171,16 @@ def test_projections_that_the_library_is_ahead_at_are_not_rotated_in_tiles():
     for M, N, k in ((65, 1152, 896), (2048, 2048, 1536), (2500, 2560, 2048), (993, 4608, 3584), (6030, 4608, 3584), (385, 7168, 5120), (300, 12288, 4096),
                     (6000, 1536, 8192), (700, 768, 4096), (70, 2048, 64)):
         assert plan(K.WIDE_ROTATED, -1, M, N, k, 0) == plan(K.WIDE_GATED, -1, M, N, k, 0) >= 0, (M, N, k)
+
+
+def test_short_runs_beside_a_long_context_choose_by_their_own_keys():
+    """The tables are as wide as the longest sequence of a step, which may bring a single token."""
+    from paged_attention_engine_amd.parts.attention import most_keys
+    from paged_attention_engine_amd.parts.base import StepContext
+
+    step = lambda lens, past: StepContext(torch.bfloat16, torch.device("cpu"), sum(lens), len(lens), None, None, {}, None, None, q_lens=lens, past_lens=past)
+    ctx = step([1, 128, 1, 40], [4000, 0, 9, 200])
+    assert most_keys(ctx) == most_keys(ctx) == 240 and most_keys(step([1, 1], [70, 3])) == 0
+    route = lambda runs, tokens, keys, nh=12: K.library().pae_attn_prefill_route(nh, 128, 128, 16, runs, tokens, -(-keys // 16), 0)
+    assert route(2, 168, 240) == 0 and route(2, 168, 4001) == 2
+    assert [route(n, 90 * n, 90) for n in (1, 5, 6)] == [0, 0, 2] and route(6, 360, 60) == 0 and route(3, 270, 90, 28) == 2
