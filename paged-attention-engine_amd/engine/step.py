@@ -66,8 +66,14 @@ class StepRunner:
     logits are dropped."""
 
     TABLE_ROUND = 64    # block tables of captured steps are padded to a multiple of this many pages,
-    SHORT_CONTEXT = 128  # but in float32 those of sequences up to so many tokens to this: its attention, which shares out keys by the
-    # tables' width, then sees that they are few (bfloat16's splits keys at fixed places, whatever the width)
+    # but in float32 those of sequences up to so many tokens to this: its attention, which shares out keys by the tables' width, then sees
+    # that they are few (bfloat16's splits keys at fixed places, whatever the width).  A count of rows is then recorded twice, once more
+    # when its sequences pass that many tokens (4 to 5 ms once); a step before that is 3.5 % faster for it at 0.5B with four requests,
+    # 1.8 % with one (1.632 -> 1.579 and 1.471 -> 1.446 ms), and as fast at 1.5B (2.48, with eight 2.91).
+    SHORT_CONTEXT = 128
+    # Recordings kept: the counts of rows up to 64 that `padded_rows` gives and some for longer tables; in float32 twice as many, for both
+    # widths of a count.  A recording keeps its step's tensors: up to 40 MB of logits, and in float32 the attention's sums over chunks
+    # of keys (64 MiB at most; 6 MB for 64 rows by 1,024 keys at 1.5B).
     MAX_GRAPHS = 24
 
     def __init__(self, model: Model, cache: CacheManager, use_graphs: bool = True,
@@ -79,6 +85,8 @@ class StepRunner:
         self.use_graphs = use_graphs and model.graph_safe
         self.graph_max_rows = model.graph_max_rows
         self._list_parts = model.step_list_parts(cache.block_size)
+        if model.dtype == torch.float32:
+            self.MAX_GRAPHS = 2 * self.MAX_GRAPHS
         self._graphs: Dict[tuple, _CapturedStep] = {}
         self.graph_replays = 0
         self.graph_recordings = 0

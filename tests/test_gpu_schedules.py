@@ -112,6 +112,27 @@ def test_more_step_shapes_than_recordings_are_kept(tmp_path, dtype):
         assert a.shape == b.shape and torch.equal(a, b)
 
 
+def test_short_and_longer_contexts_of_every_row_count_stay_recorded(tmp_path):
+    """float32 records a count of rows for contexts up to 128 tokens and for longer ones; there is room for both of every count up to 64."""
+    folder = helpers.make_model_folder(tmp_path, "D")
+    model = pae.load_model(folder, "float32")
+    cache = model.new_cache(16, 64 * (4 + 13) + 8, 128)
+    runner = pae.StepRunner(model, cache)
+    held = [20] * 64 + [140] * 64
+    for s, n in enumerate(held):
+        cache.create_sequence(s)
+        cache.reserve(s, n)
+        runner.run([pae.StepEntry(s, tuple(tokens_of(helpers.TINY_D, n, s)), ())])
+    counts = sorted({padded_rows(n) for n in range(1, 65)})
+    for again in range(2):
+        for n in counts:
+            for first in (0, 64):
+                for s in range(first, first + n):
+                    cache.reserve(s, 1)
+                runner.run([pae.StepEntry(s, (7,), (0,)) for s in range(first, first + n)])
+        assert runner.graph_recordings == 2 * len(counts)
+
+
 def snapshot(cache):
     return {(g.index, name): pool.clone() for g in cache.groups for name, pool in g.pools.items()}
 
