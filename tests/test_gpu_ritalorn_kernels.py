@@ -449,6 +449,27 @@ def test_runs_under_a_window_meet_no_numbers_of_another_run(window):
     assert torch.isfinite(got[0].float()).all() and torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
 
 
+@pytest.fixture
+def pieces_of_a_step(monkeypatch):
+    """`expanded_runs` cuts runs as the mixer asks for, into up to PREFILL_TILE tokens."""
+    import functools
+
+    from paged_attention_engine_amd.parts import latent
+
+    monkeypatch.setattr(latent, "expanded_runs", functools.partial(latent.expanded_runs, piece=_K().PREFILL_TILE))
+
+
+@pytest.mark.parametrize("H,D,R,V,C", [(3, 64, 32, 64, 64), (2, 128, 64, 128, 512)])
+@pytest.mark.parametrize("window", [0, 33, 200])
+def test_latent_attention_over_long_runs_in_the_pieces_of_a_step(H, D, R, V, C, window, pieces_of_a_step):
+    test_latent_attention_over_long_runs_under_a_window(H, D, R, V, C, window)
+
+
+@pytest.mark.parametrize("window", [1, 17, 18, 190, 200])
+def test_runs_in_the_pieces_of_a_step_meet_no_numbers_of_another_run(window, pieces_of_a_step):
+    test_runs_under_a_window_meet_no_numbers_of_another_run(window)
+
+
 @pytest.mark.parametrize("bs,window", [(16, 17), (16, 100), (32, 100)])
 @pytest.mark.parametrize("chunked,slopes", [(False, False), (True, True), (False, True)])
 def test_prompts_under_a_window_meet_no_numbers_of_the_pool_s_first_page(bs, window, chunked, slopes):
