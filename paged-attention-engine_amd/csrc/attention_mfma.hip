@@ -19,13 +19,15 @@
 //          page is read once for all of them.  Four wavefronts take pages in turn
 //          and merge in LDS; a second small kernel merges the splits.  Splits
 //          start at multiples of the split length from position 0.
-// prefill: one workgroup per (up to 64 consecutive tokens of a sequence, query head), whose
+// prefill: runs of up to 128 consecutive tokens of a sequence, a workgroup per (32 or 64 of them, query head), whose
 //          wavefronts share out the keys (see there); most runs of more than a few hundred tokens go to
 //          attention_prefill.hip, which shares them through LDS (`route_of` below has the rule).
 //
 // Masking is the reference's rule (engine/attention.py:474-487: key j visible iff
-// j <= position of the query) plus an optional window.  A column's result depends
-// only on its own position: fully masked pages add exact zeros.
+// j <= position of the query) plus an optional window.  In one kernel a column's result depends
+// only on its own position: fully masked pages add exact zeros.  Which prefill kernel runs, though, follows from the step's
+// runs (`route_of`): the three deal keys to wavefronts in their own ways, and four query groups divide by the sum of the rounded
+// weights, so that a token of a prompt has the same bits in two steps only where these take the same one.
 //
 // For designs that have them (the BIASED instantiations): the window read as a chunk length
 // (`chunked`: position p sees the keys from p - p % window on), a bias by distance,

@@ -16,11 +16,10 @@
 //     2,048 x  2,048 x  1,536           19                                   15
 //     6,030 x 37,888 x  3,584        1,209 and 117 for the gate              1,176 with the gate
 //     6,030 x  3,584 x 18,944        1,041                                   600
-//       601 x  1,536 x  8,960           36                                   24 in three ranges of k
-//   With the norm that adds the ranges' sums, before them and now in tiles of 256 x 256 too:
-//     2,048 x  1,536 x  8,960           77.7                                 69.4 in five ranges
-//     2,500 x  2,048 x 11,008          134                                  107 in three
+//       601 x  1,536 x  8,960           36                                   24 in ranges of k
 //       200 x  1,536 x  1,536           20                                   8
+// With the norm that adds the ranges' sums, without ranges in the tiles of 256 x 256 and with them: 2,048 x 1,536 x 8,960 77.7 and, in five
+// ranges, 69.4; 2,500 x 2,048 x 11,008 134 and, in three, 107.
 #include "wide_gemm.h"
 #include "api.h"
 

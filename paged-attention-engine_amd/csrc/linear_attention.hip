@@ -77,7 +77,8 @@ __global__ __launch_bounds__(128) void gla_prepare_kernel(const T* __restrict__ 
 //
 // What is infinite or NaN in a token's row reaches its own read-out and those behind it, as token by token.
 constexpr int GLA_CHUNK = 16;
-// Steps whose runs have that many tokens on average go by chunks; the host knows no run's length.  Both ways in us, 12 heads of 128:
+// Steps whose runs have that many tokens on average go by chunks: the launch is given counts of tokens and runs, their lengths lie on the
+// device (a long run beside many single tokens stays token by token).  Both ways in us, 12 heads of 128:
 // one run of 96 24.7 and 26.6, 128 30.6 and 29.1, 160 36.5 and 31.7; 8 runs of 100 57.3 and 60.3, of 138 71.0 and 68.3; 28 heads, two
 // runs of 128 45.3 and 47.8; 300 tokens beside 63 single ones 63 and 94.  Heads of up to 32 features have less to share out: 16
 // features, one run of 160 21.0 and 24.0, of 200 25.2 and 26.1, 16 runs of 250 55 and 43.
