@@ -213,15 +213,12 @@ static int best_tiles(int M, int N, int K, int splits, double& least) {
 }
 
 // Which products go here.  Few weight rows in one range stay with the kernel that shares out the rows of A (2,048 x 1,536 at 64 rows
-// 5.7 us, here 7.4; 896 x 4,864 9.1 and 10.1; 2,048 x 2,048 8.3 and 8.9), and up to 32 rows the one workgroup a unit of that launcher's is
-// level (17,920 x 1,536 at 32 and 20 rows 16.1 and 15.8 us, here 16.6 and 16.0; 22,016 x 2,048 24.4 and 22.7, here 24.3 and 23.0).
+// 5.7 us, here 7.4; 896 x 4,864 9.1 and 10.1; 2,048 x 2,048 8.3 and 8.9), and some of many weight rows with that launcher's one workgroup a
+// unit (`pae_one_workgroup_a_unit`).
 int stream_tiles(int epilogue, const void* a, const void* w, int M, int N, int K, int64_t lda, int splits) {
   if (((uintptr_t)a | (uintptr_t)w) % 16 || M <= 16 || M > 64 || K % 64 || K > 1 << 20 || lda >= 1 << 24 || (splits > 1 && epilogue != EPI_F32 && N > 131072)) return 0;
   if (splits == 1 && N <= 3072) return 0;
-  const int tiles = (N + 15) / 16, waves = (tiles + 255) / 256;
-  if (M <= 32 && splits == 1 && waves >= 5 && waves <= 8 && (tiles + waves - 1) / waves >= 216 &&
-      (epilogue == EPI_BF16 || epilogue == EPI_SWIGLU))
-    return 0;
+  if (splits == 1 && (epilogue == EPI_BF16 || epilogue == EPI_SWIGLU) && pae_one_workgroup_a_unit(M, N, K)) return 0;
   double least;
   return best_tiles(M, N, K, splits, least);
 }
@@ -238,6 +235,21 @@ extern "C" int pae_stream_ranges(int M, int N, int K) {
     if (best_tiles(M, N, K, splits, t) && t < least) least = t, best = splits;
   }
   return best;
+}
+
+// Whether a product of 17 to 64 rows, with whole sums, takes one range of k in workgroups of 5 to 8 wavefronts of 16 weight rows, one a compute unit and
+// nearly all units busy (gemm_skinny.hip), although it could be streamed.  Over 12 counts of weight rows (17,408 to 32,768) by 7 of k (1,024 to
+// 8,192) at 33 to 64 rows the choice is 0.965 of that kernel's time and 1.08 at worst, streaming all of them 0.985 and 1.18.
+//   * up to 32 rows always: level (17,920 x 1,536 at 32 and 20 rows 16.1 and 15.8 us, streamed 16.6 and 16.0; 22,016 x 2,048 24.4 and 22.7, 24.3 and 23.0);
+//   * up to 48 with seven wavefronts and more (48 rows, 27,648 x 5,120 52.8, streamed 56.4; 28,672 x 4,096 51.2 and 55.4; but 24,576 x 3,072, six, 28.7 and
+//     27.2), or where streaming would cut k in three ranges, or in two from 8,192 on (48 rows, 21,504 x 5,120 44.1 and 47.1, 17,920 x 8,192 64.9 and
+//     70.8; but 17,920 x 4,096 32.2 and 31.6);
+//   * beyond that with seven and more and k from 4,096 on (64 rows, 28,672 x 4,096 52.9 and 56.2; 28,672 x 2,048 0.99 of it streamed).
+extern "C" int pae_one_workgroup_a_unit(int M, int N, int K) {
+  const int tiles = (N + 15) / 16, waves = (tiles + 255) / 256;
+  if (M <= 16 || M > 64 || waves < 5 || waves > 8 || (tiles + waves - 1) / waves < 216) return 0;
+  if (M <= 32) return 1;
+  return waves >= 7 ? M <= 48 || K >= 4096 : M <= 48 && pae_stream_ranges(M, N, K) > (K >= 8192 ? 1 : 2);
 }
 
 int stream_ticket_slots(int M, int N) { return M > 16 && N <= 131072 ? (N + 31) / 32 * 8 : 0; }

@@ -71,6 +71,7 @@ def _declare(lib) -> None:
         "pae_scaled_rows": [P, P, P, I, F, I, I, P],
         "pae_skinny_ticket_slots": [I, I],
         "pae_stream_ranges": [I, I, I],
+        "pae_one_workgroup_a_unit": [I, I, I],
         "pae_gemm_skinny_act": [P, L, P, L, P, P, I, I, I, I, I, P, P, I, P],
         "pae_gemm_plain_shared": [I, I, P, L, L, P, L, L, P, L, P, I, I, I, I, I, P, P],
         "pae_gemm_skinny_gated": [P, L, P, L, P, I, I, I, I, P, P, I, P],
@@ -1024,18 +1025,19 @@ def whole_sum_splits(N: int, K: int, M: int, w: Optional[torch.Tensor] = None) -
         # 37.2 / 43.7 / 52.0 us against 36.4 / 42.8 / 59.6; 14B 18.7 / 23.3 / 29.4 against 20.7 / 24.1 / 30.3; 7B 13.1 /
         # 15.2 / 20.4 against 13.1 / 14.1 / 20.9; gate/up likewise at all seven widths)
         return 1
-    waves = -(-(-(-N // 16)) // 256)  # wavefronts of 16 weight rows a workgroup for at most 256 workgroups
-    one_a_unit = 5 <= waves <= 8 and -(-(-(-N // 16)) // waves) >= 216
-    if one_a_unit and M <= 32:
-        # one workgroup per compute unit, nearly all units busy: one range (the launcher then takes the
-        # kernel of `waves` wavefronts; 1.5B gate/up at 32 rows 19.1 -> 16.7 us)
+    if library().pae_one_workgroup_a_unit(M, N, K):
         return 1
-    return _streamed_splits(N, K, M, 1 if one_a_unit else _whole_sum_ranges(N, K, M), w)
+    return _streamed_splits(N, K, M, _whole_sum_ranges(N, K, M), w)
 
 
 def _whole_sum_ranges(N: int, K: int, M: int) -> int:
     """The ranges of `whole_sum_splits` for more than 16 rows in the kernels that do not stream."""
     tiles, groups = -(-N // 32), -(-N // 128)
+    waves = -(-(-(-N // 16)) // 256)  # wavefronts of 16 weight rows a workgroup for at most 256 workgroups
+    if 5 <= waves <= 8 and -(-(-(-N // 16)) // waves) >= 216:
+        # one workgroup per compute unit, nearly all units busy: one range (the launcher then takes the
+        # kernel of `waves` wavefronts; 1.5B gate/up at 32 rows 19.1 -> 16.7 us, at 64 rows 23.4 -> 22.2)
+        return 1
     if 128 <= groups < 256:
         # a couple of workgroups of 32 weight rows per compute unit: three ranges from 32
         # rows on (1.5B gate/up at 64 rows 27.2 -> 23.3 us, at 32 rows 20.2 -> 19.0 us; below, one range is ahead)

@@ -184,3 +184,16 @@ def test_short_runs_beside_a_long_context_choose_by_their_own_keys():
     route = lambda runs, tokens, keys, nh=12: K.library().pae_attn_prefill_route(nh, 128, 128, 16, runs, tokens, -(-keys // 16), 0)
     assert route(2, 168, 240) == 0 and route(2, 168, 4001) == 2
     assert [route(n, 90 * n, 90) for n in (1, 5, 6)] == [0, 0, 2] and route(6, 360, 60) == 0 and route(3, 270, 90, 28) == 2
+
+
+def test_products_of_one_workgroup_a_unit_that_are_ahead_are_not_streamed():
+    """Workgroups of seven and eight wavefronts up to 48 rows, and beyond that with much of k; five and six where streaming would cut k
+    often or k is long."""
+    one = K.library().pae_one_workgroup_a_unit
+    for M, N, k in ((17, 17920, 1536), (32, 22016, 2048), (33, 28672, 4096), (48, 27648, 5120), (64, 28672, 4096), (64, 32768, 8192), (48, 17920, 8192), (40, 28672, 1024),
+                    (48, 21504, 5120)):
+        assert one(M, N, k) and K.whole_sum_splits(N, k, M) == 1, (M, N, k)
+    for M, N, k in ((16, 17920, 1536), (65, 28672, 4096), (33, 17920, 1536), (64, 17920, 1536), (64, 22016, 2048), (48, 24576, 3072), (64, 28672, 2048),
+                    (64, 17920, 8192), (48, 17920, 4096), (32, 16384, 1536), (20, 37888, 3584)):
+        assert not one(M, N, k), (M, N, k)
+        assert M == 16 or M == 65 or K.whole_sum_splits(N, k, M) == K.library().pae_stream_ranges(M, N, k) > 0
