@@ -214,10 +214,14 @@ static int best_tiles(int M, int N, int K, int splits, double& least) {
 
 // Which products go here.  Few weight rows in one range stay with the kernel that shares out the rows of A (2,048 x 1,536 at 64 rows
 // 5.7 us, here 7.4; 896 x 4,864 9.1 and 10.1; 2,048 x 2,048 8.3 and 8.9), and some of many weight rows with that launcher's one workgroup a
-// unit (`pae_one_workgroup_a_unit`).
+// unit (`pae_one_workgroup_a_unit`).  Neither come here few and short weight rows, for which the start alone, about 4 us, is more than the other kernels take
+// (with the norm that adds the ranges, at 20 / 48 rows: 640 x 3,072 7.6 / 7.7 us in two ranges there, 8.6 / 9.9 in three here, 1,024 x 4,096 8.8 / 10.7 and
+// 9.5 / 11.0, 896 x 4,864 9.8 / 11.6 and 10.2 / 11.9; but 1,280 x 4,096 0.95 / 0.99 of it here, 1,024 x 6,144 0.95 / 0.97, 1,536 x 3,072 level).
+static bool few_and_short(int N, int K) { return N <= 1280 && (int64_t)N * K < 4500000; }
+
 int stream_tiles(int epilogue, const void* a, const void* w, int M, int N, int K, int64_t lda, int splits) {
   if (((uintptr_t)a | (uintptr_t)w) % 16 || M <= 16 || M > 64 || K % 64 || K > 1 << 20 || lda >= 1 << 24 || (splits > 1 && epilogue != EPI_F32 && N > 131072)) return 0;
-  if (splits == 1 && N <= 3072) return 0;
+  if ((splits == 1 && N <= 3072) || few_and_short(N, K)) return 0;
   if (splits == 1 && (epilogue == EPI_BF16 || epilogue == EPI_SWIGLU) && pae_one_workgroup_a_unit(M, N, K)) return 0;
   double least;
   return best_tiles(M, N, K, splits, least);
@@ -225,7 +229,7 @@ int stream_tiles(int epilogue, const void* a, const void* w, int M, int N, int K
 
 // k ranges for a product of 17 to 64 rows that this kernel takes, 0 for one that it does not.
 extern "C" int pae_stream_ranges(int M, int N, int K) {
-  if (M <= 16 || M > 64 || K % 64 || K > 1 << 20) return 0;
+  if (M <= 16 || M > 64 || K % 64 || K > 1 << 20 || few_and_short(N, K)) return 0;
   int best = 0;
   double least = 1e29;
   for (int splits = N <= 3072 ? 2 : 1; splits <= 8 && (splits == 1 || K / splits >= 384); ++splits) {

@@ -56,6 +56,13 @@ def test_streamed_products(M, N, K_, splits):
 
 
 @pytest.mark.parametrize("M", [17, 33, 64])
+@pytest.mark.parametrize("N,K_,splits", [(1288, 1536, 3), (1272, 3584, 5), (16, 281344, 8), (1272, 1536, 3)])
+def test_streamed_products_of_few_weight_rows(M, N, K_, splits):
+    """At the line between few weight rows that are streamed and those that are not; ranges as they are cut, the last one shorter."""
+    test_streamed_products(M, N, K_, splits)
+
+
+@pytest.mark.parametrize("M", [17, 33, 64])
 @pytest.mark.parametrize("nh,nkv,hd,rot,splits", [(28, 4, 128, 128, 3), (36, 8, 80, 32, 1), (50, 4, 96, 96, 1), (12, 2, 128, 64, 2)])
 def test_streamed_projections_rotate_and_store(M, nh, nkv, hd, rot, splits):
     width, bs, N = 640, 16, (nh + 2 * nkv) * hd

@@ -197,3 +197,12 @@ def test_products_of_one_workgroup_a_unit_that_are_ahead_are_not_streamed():
                     (64, 17920, 8192), (48, 17920, 4096), (32, 16384, 1536), (20, 37888, 3584)):
         assert not one(M, N, k), (M, N, k)
         assert M == 16 or M == 65 or K.whole_sum_splits(N, k, M) == K.library().pae_stream_ranges(M, N, k) > 0
+
+
+@pytest.mark.parametrize("M", [17, 32, 48, 64])
+def test_few_and_short_weight_rows_are_not_streamed(M):
+    """A product whose weights are read in less time than a streamed product starts in keeps the ranges of the other kernels."""
+    for N, k in ((640, 3072), (640, 6144), (896, 4864), (1024, 4096), (1280, 3072), (16, 65536)):
+        assert K.library().pae_stream_ranges(M, N, k) == 0 and K.skinny_splits(N, k, M) == K.skinny_splits(N, k + 8, M), (N, k)
+    for N, k in ((640, 12288), (1024, 6144), (1536, 2240), (1536, 8960), (1296, 3072)):
+        assert K.library().pae_stream_ranges(M, N, k) > 1, (N, k)
