@@ -56,6 +56,7 @@ int pae_gemm_skinny_act(void* out, int64_t ldc, const void* A, int64_t lda, cons
 int pae_gemm_skinny_gated(void* out, int64_t ldc, const void* A, int64_t lda, const void* W, int M, int N, int K, int splits,
                           float* ticket_parts, int* ticket_counters, int act, hipStream_t stream);
 int pae_stream_ranges(int M, int N, int K);
+int pae_stream_part_ranges(int M, int N, int K);
 int pae_one_workgroup_a_unit(int M, int N, int K);
 int pae_skinny_ticket_slots(int M, int N);
 int64_t pae_skinny_ticket_floats(int M, int N, int splits);

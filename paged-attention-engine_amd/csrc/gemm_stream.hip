@@ -190,14 +190,15 @@ int launch_epilogue(const StreamProduct& p, int splits, hipStream_t stream) {
 }  // namespace
 
 // Microseconds, by the fit above, of workgroups of `nt` tiles.  (A unit holds two workgroups, of 10 tiles one: those only where one
-// round of the chip takes them all; and ranges by ticket only where all workgroups are there at once.)  Ranges cost the same where they leave
-// partial sums, which the kernel behind reads: 64 rows of 3,584 numbers, written and read once, are 1.8 MB, 0.4 us, a range.
+// round of the chip takes them all; and ranges by ticket only where all workgroups are there at once.)
+constexpr double TICKETS = 0.7, EACH_TICKET = 0.5;
+
 static double stream_time(int M, int N, int K, int nt, int splits) {
   const int mt = (M + 15) / 16, range = ((K + splits - 1) / splits + 127) / 128 * 128;
   const int64_t groups = (int64_t)((N + 16 * nt - 1) / (16 * nt)) * splits;
   if ((mt == 2 && nt % 2) || (nt == 10 && groups > 256) || (splits > 1 && groups > 512)) return 1e30;
   const double rounds = groups <= 512 ? (groups + 255) / 256 : groups / 256.0;
-  return 3.9 + rounds * (mt + nt) * 32.0 * range / 88e3 + (double)N * K * 2 / 6.5e6 + (splits > 1 ? 0.7 + 0.5 * splits : 0.0);
+  return 3.9 + rounds * (mt + nt) * 32.0 * range / 88e3 + (double)N * K * 2 / 6.5e6 + (splits > 1 ? TICKETS + EACH_TICKET * splits : 0.0);
 }
 
 static const int TILES[] = {2, 3, 4, 5, 6, 8, 10};
@@ -237,6 +238,25 @@ extern "C" int pae_stream_ranges(int M, int N, int K) {
     if ((int64_t)range * (splits - 1) >= K) continue;
     double t;
     if (best_tiles(M, N, K, splits, t) && t < least) least = t, best = splits;
+  }
+  return best;
+}
+
+// The same for partial sums that the kernel behind adds, where one range would be taken: a range costs less there, 0.2 us and its sums' way to memory
+// and back at 4.5 TB/s (with the norm, one range and these: 32 rows, 8,192 x 4,096 26.2 and 21.8 us, 4,096 x 2,048 12.6 and 10.8; of 416 sizes 25 change,
+// 0.93 of the time on average, 1.09 at worst: 20 rows, 6,144 x 3,072 17.6 and 19.1).  Several ranges by ticket stay as they are: counted anew they would be
+// 0.99 of the time on average and 1.10 at worst.
+extern "C" int pae_stream_part_ranges(int M, int N, int K) {
+  const int ticketed = pae_stream_ranges(M, N, K);
+  if (ticketed != 1 || N > 10240 || K < 1536) return ticketed;  // (as far as was measured)
+  int best = 1;
+  double least = 1e30;
+  for (int splits = 1; splits <= 8 && (splits == 1 || K / splits >= 384); ++splits) {
+    const int range = ((K + splits - 1) / splits + 127) / 128 * 128;
+    double t;
+    if ((int64_t)range * (splits - 1) >= K || !best_tiles(M, N, K, splits, t)) continue;
+    if (splits > 1) t += splits * (0.2 + 8.0 * M * N / 4.5e6) - TICKETS - EACH_TICKET * splits;
+    if (t < least) least = t, best = splits;
   }
   return best;
 }

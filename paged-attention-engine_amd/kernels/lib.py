@@ -71,6 +71,7 @@ def _declare(lib) -> None:
         "pae_scaled_rows": [P, P, P, I, F, I, I, P],
         "pae_skinny_ticket_slots": [I, I],
         "pae_stream_ranges": [I, I, I],
+        "pae_stream_part_ranges": [I, I, I],
         "pae_one_workgroup_a_unit": [I, I, I],
         "pae_gemm_skinny_act": [P, L, P, L, P, P, I, I, I, I, I, P, P, I, P],
         "pae_gemm_plain_shared": [I, I, P, L, L, P, L, L, P, L, P, I, I, I, I, I, P, P],
@@ -651,6 +652,11 @@ def skinny_splits(N: int, K: int, M: int = 1, w: Optional[torch.Tensor] = None) 
     """k ranges for a product whose consumer adds float32 partials: enough workgroups to fill the
     chip (a workgroup takes 16 weight rows, or 32 and more with more than 8 rows of activations).
     `w`: the weights, where they are at hand (see `_streamed_splits`)."""
+    return _streamed_splits(N, K, M, _part_ranges(N, K, M), w, parts=True)
+
+
+def _part_ranges(N: int, K: int, M: int) -> int:
+    """The ranges of `skinny_splits` in the kernels that do not stream."""
     rows = 32 if M > 8 else 16
     tiles = -(-N // rows)
     # (ranges of at least 1,024 of k: the 0.5B sizes at 8 rows, O 5.3 us in three ranges and 3.9 in one, down
@@ -686,15 +692,17 @@ def skinny_splits(N: int, K: int, M: int = 1, w: Optional[torch.Tensor] = None) 
         if M > SAME_ORDER_MAX_ROWS and 4 <= one_round <= 8 and K // one_round >= 1024:
             wanted = one_round
     k_per = -(-(-(-K // wanted)) // 128) * 128
-    return _streamed_splits(N, K, M, -(-K // k_per), w)
+    return -(-K // k_per)
 
 
-def _streamed_splits(N: int, K: int, M: int, splits: int, w: Optional[torch.Tensor]) -> int:
+def _streamed_splits(N: int, K: int, M: int, splits: int, w: Optional[torch.Tensor], parts: bool = False) -> int:
     """k ranges of a product of more than 16 rows that csrc/gemm_stream.hip takes (several ranges, or many weight rows), by its
-    times; else, also for weights off 16 bytes, `splits`, which suit the other kernels."""
+    times; else, also for weights off 16 bytes, `splits`, which suit the other kernels.  `parts`: the ranges' sums are left for the
+    consumer to add."""
     if M <= SAME_ORDER_MAX_ROWS or (splits == 1 and N <= 3072) or (w is not None and w.data_ptr() % 16):
         return splits
-    return library().pae_stream_ranges(M, N, K) or splits
+    lib = library()
+    return (lib.pae_stream_part_ranges if parts else lib.pae_stream_ranges)(M, N, K) or splits
 
 
 _UNITS = 0
@@ -726,7 +734,7 @@ def residual_splits(N: int, K: int, M: int = 1, w: Optional[torch.Tensor] = None
         # workgroups: 15.6 / 17.9 us against 16.8 / 19.9 with four ranges; 3B down, 64 x 4: 18.5 / 22.9 against
         # 21.8 / 28.4 with five; 7B down: eight, 35 / 47 us; 14B: six, 33 / 44; 14B O: six, 19 / 27 against 27 / 37
         # with two)
-        return skinny_splits(N, K, M, w)
+        return _streamed_splits(N, K, M, _part_ranges(N, K, M), w)
     tiles = -(-N // 16)
     # one such workgroup fills a compute unit, so the tiles should fill the chip's units a whole number of
     # times, or nearly (14B/32B down: 320 tiles are a full round and a quarter of one; 32B at 8 rows 86.7 us
@@ -735,7 +743,7 @@ def residual_splits(N: int, K: int, M: int = 1, w: Optional[torch.Tensor] = None
     rounds_full = tiles <= units or tiles % units == 0 or tiles % units >= 3 * units // 4
     if K >= 1024 and (tiles >= 192 or 32 * K <= 65536) and rounds_full:
         return -(-K // (-(-(-(-K // 4)) // 128) * 128))  # four, as the rounding to 128 leaves them
-    splits = skinny_splits(N, K, 1)
+    splits = _part_ranges(N, K, 1)
     if splits == 4 and K >= 1024 and (tiles >= 192 or 32 * K <= 65536):
         # four would be taken side by side (the same sums, slower here)
         return 5 if K // 5 >= 256 else 3

@@ -206,3 +206,16 @@ def test_few_and_short_weight_rows_are_not_streamed(M):
         assert K.library().pae_stream_ranges(M, N, k) == 0 and K.skinny_splits(N, k, M) == K.skinny_splits(N, k + 8, M), (N, k)
     for N, k in ((640, 12288), (1024, 6144), (1536, 2240), (1536, 8960), (1296, 3072)):
         assert K.library().pae_stream_ranges(M, N, k) > 1, (N, k)
+
+
+@pytest.mark.parametrize("M", [16, 17, 32, 33, 64])
+def test_ranges_of_partial_sums_cost_less_than_tickets(M):
+    """Only where a streamed product would take one range; those cover k, and products that add themselves into the residual keep theirs."""
+    lib = K.library()
+    for N in (16, 640, 1536, 3072, 3088, 3584, 4096, 8192, 10240):
+        for k in (64, 384, 768, 1536, 2048, 4096, 8960, 18944):
+            one, part = lib.pae_stream_ranges(M, N, k), lib.pae_stream_part_ranges(M, N, k)
+            assert part == one or (one == 1 and part <= 8 and (-(-(-(-k // part)) // 128) * 128) * (part - 1) < k and k // part >= 384), (N, k)
+            if M > 16 and N > 3072:
+                assert K.skinny_splits(N, k, M) == part and K.residual_splits(N, k, M) == one, (N, k)
+    assert lib.pae_stream_part_ranges(32, 8192, 4096) > 1 == lib.pae_stream_ranges(32, 8192, 4096)
