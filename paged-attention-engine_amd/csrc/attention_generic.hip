@@ -33,16 +33,16 @@
 #include "common.h"
 #include "api.h"
 
-// What weights are taken relative to where `m` is the largest score: itself, or zero where all scores are minus infinity (numbers that
-// overflowed, or a bias that hides a key), whose weights are then zero as they are beside a score that is a number.
-__device__ __forceinline__ float reference_of(float m) { return m == -INFINITY ? 0.f : m; }
+// What a chunk's weights are taken relative to: its largest score, or the least number there is where all its scores are minus infinity (numbers that
+// overflowed, or a bias that hides a key), whose weights are then zero as they are beside a score that is a number.  (Once a chunk and not
+// where chunks are added: there it cost 2.5 % of a prompt of 1,500 tokens.)
+__device__ __forceinline__ float reference_of(float largest) { return fmaxf(largest, -3.402823466e38f); }
 
 // A chunk's sums (its largest score, the sum of its weights, the weighted values) onto those of the chunks before it.
 template <int MAXD>
 __device__ __forceinline__ void add_chunk(float (&acc)[MAXD], float& m, float& l, const float (&sum)[MAXD], float m_chunk, float l_chunk) {
   const float m_new = fmaxf(m, m_chunk);
-  const float ref = reference_of(m_new);
-  const float before = expf(m - ref), now = expf(m_chunk - ref);  // 0 and 1 on the first chunk (m = -inf)
+  const float before = expf(m - m_new), now = expf(m_chunk - m_new);  // 0 and 1 on the first chunk (m = -inf)
   l = l * before + l_chunk * now;
   m = m_new;
 #pragma unroll
@@ -115,8 +115,8 @@ __global__ void paged_attention_generic_kernel(
       if (slopes) s -= slope * (float)(pos - key);
       if (cap > 0.f) s = cap * tanhf(s / cap);
     }
-    const float m_chunk = wave_max(s);
-    const float p = valid ? expf(s - reference_of(m_chunk)) : 0.f;
+    const float m_chunk = reference_of(wave_max(s));
+    const float p = valid ? expf(s - m_chunk) : 0.f;
     const float l_chunk = wave_sum(p);
     p_lds[lane] = p;
     __syncthreads();
@@ -333,11 +333,11 @@ __global__ __launch_bounds__(PAE_WAVE * PAE_ROWS_WAVES) void paged_attention_row
         if (slopes) sc[i] -= slopes[head[i]] * (float)(pos[i] - key);
         if (cap > 0.f) sc[i] = cap * tanhf(sc[i] / cap);
         if (!(key >= start[i] && key <= pos[i])) sc[i] = -INFINITY;
-        m_chunk[i] = wave_max(sc[i]);
+        m_chunk[i] = reference_of(wave_max(sc[i]));
       }
 #pragma unroll
       for (int i = 0; i < EACH; ++i) {  // the rows' reductions side by side; rows that are not on keep what they have
-        p[i] = key >= start[i] && key <= pos[i] ? expf(sc[i] - reference_of(m_chunk[i])) : 0.f;
+        p[i] = key >= start[i] && key <= pos[i] ? expf(sc[i] - m_chunk[i]) : 0.f;
         l_chunk[i] = wave_sum(p[i]);
       }
 #pragma unroll
