@@ -16,7 +16,7 @@
 // chunks' sums are added in order, in float32 (`add_chunk`).  What a
 // (token, head) computes therefore depends on nothing but its own position:
 // not on how the step was cut, nor on what else is in the batch, nor on whether a workgroup walks the chunks or
-// each chunk has one of its own (few tokens at many keys: `split_chunks`).
+// several share them out (few tokens at many keys: `split_chunks`).
 //
 // Three things beyond the reference's attention, each switched by a parameter: values of their own
 // width `vd` (keys and queries stay `hd` wide), a cap on the scores (s <- cap * tanh(s / cap),
@@ -170,10 +170,12 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 #define PAE_ROWS_EACH 2
 #define PAE_ROWS_MOST (PAE_ROWS_WAVES * PAE_ROWS_EACH)
 #define SPLIT_GROUPS 128         // up to so many workgroups' chunks are shared out
+#define SPLIT_UNITS 256          // over so many workgroups
 #define SPLIT_FLOATS (16 << 20)  // numbers that their sums may take: 64 MiB
 
-// SPLIT: blockIdx.z is the only chunk of 64 keys the workgroup looks at, and every row's sums over it go to
-// `chunk_sums` [(token, head)][chunk][vd] and `chunk_ml` [(token, head)][chunk][2], for the kernel below to add up in the order of the chunks.
+// SPLIT: the workgroup looks at every gridDim.z-th chunk of 64 keys from chunk blockIdx.z on, and every row's sums over each go to
+// `chunk_sums` [(token, head)][chunk][vd] and `chunk_ml` [(token, head)][chunk][2], for the kernel below to add up in the order of the chunks
+// (`chunks` is how many the tables have room for).
 template <int MAXD, int EACH, bool SPLIT>  // keys and values at most 64 * MAXD wide; rows of a wavefront: one where eight rows are all there are
 __global__ __launch_bounds__(PAE_WAVE * PAE_ROWS_WAVES) void paged_attention_rows_kernel(
     float* __restrict__ out, int64_t out_stride, const float* __restrict__ q, int64_t q_stride,
@@ -181,7 +183,7 @@ __global__ __launch_bounds__(PAE_WAVE * PAE_ROWS_WAVES) void paged_attention_row
     const int* __restrict__ tok_seq, const int* __restrict__ block_tables, int max_blocks, int bs, int num_tokens,
     int nh, int nkv, int hd, int vd, float scale, int window, float cap, const float* __restrict__ sinks,
     int chunked, const float* __restrict__ slopes, const float* __restrict__ gate, int64_t gate_stride,
-    int gate_per_head, int toks, int heads_each, float* __restrict__ chunk_sums, float* __restrict__ chunk_ml) {
+    int gate_per_head, int toks, int heads_each, int chunks, float* __restrict__ chunk_sums, float* __restrict__ chunk_ml) {
   constexpr int FOURS = 16 * MAXD / PAE_ROWS_WAVES;  // that a thread brings of a chunk's keys, and of its values
   extern __shared__ float lds[];
   const int kst = hd + 4, vst = vd + 4;  // row strides that spread a quad's reads and writes over the banks
@@ -275,13 +277,22 @@ __global__ __launch_bounds__(PAE_WAVE * PAE_ROWS_WAVES) void paged_attention_row
       for (int u = 0; u < FOURS; ++u)
         v_reg[u] = *(const f32x4*)(v_cache + (((int64_t)v_page[u] * nkv + kvh) * vd + v_dim[u]) * bs + off0 + v_key[u] % span);
     };
-    const int base0 = SPLIT ? blockIdx.z * PAE_WAVE : (low / PAE_WAVE) * PAE_WAVE;
-    if (SPLIT && (base0 > high || base0 + PAE_WAVE <= low)) {
-      at = next;
-      continue;
+    const int step = SPLIT ? gridDim.z * PAE_WAVE : PAE_WAVE;
+    int base0 = (low / PAE_WAVE) * PAE_WAVE;
+    if (SPLIT) {
+      base0 = blockIdx.z * PAE_WAVE;
+      if (base0 + PAE_WAVE <= low) base0 += (low - base0) / step * step;
+      if (base0 + PAE_WAVE <= low) base0 += step;  // the first of the workgroup's chunks with a key in sight
+      if (base0 > high) {
+        at = next;
+        continue;
+      }
     }
-    fetch(base0);
-    for (int base = base0; SPLIT ? base == base0 : base <= high; base += PAE_WAVE) {
+    // (shared out, heads of more than 192 have no registers for the chunk after this one: eight tokens at 1,000 keys 25.4 us with it, 21 without)
+    constexpr bool AHEAD = !SPLIT || MAXD < 4;
+    if (AHEAD) fetch(base0);
+    for (int base = base0; base <= high; base += step) {
+      if (!AHEAD) fetch(base);
       __syncthreads();  // the chunk before has been read
 #pragma unroll
       for (int u = 0; u < FOURS; ++u) *(f32x4*)(k_lds + k_key[u] * kst + k_dim[u]) = k_reg[u];
@@ -294,7 +305,7 @@ __global__ __launch_bounds__(PAE_WAVE * PAE_ROWS_WAVES) void paged_attention_row
         v[3 * vst] = v_reg[u].w;
       }
       __syncthreads();
-      if (!SPLIT && base + PAE_WAVE <= high) fetch(base + PAE_WAVE);
+      if (AHEAD && base + step <= high) fetch(base + step);
       bool on[EACH];
       bool any = false, whole = true;
 #pragma unroll
@@ -409,7 +420,7 @@ __global__ __launch_bounds__(PAE_WAVE * PAE_ROWS_WAVES) void paged_attention_row
           add_chunk<MAXD>(acc[i], m[i], l[i], sum[i], m_chunk[i], l_chunk[i]);
           continue;
         }
-        const int64_t part = ((int64_t)tok[i] * nh + head[i]) * gridDim.z + blockIdx.z;
+        const int64_t part = ((int64_t)tok[i] * nh + head[i]) * chunks + base / PAE_WAVE;
         if (lane == 0) *reinterpret_cast<float2*>(chunk_ml + 2 * part) = make_float2(m_chunk[i], l_chunk[i]);
 #pragma unroll
         for (int d = 0; d < MAXD; ++d)
@@ -475,12 +486,14 @@ static int rows_of_a_workgroup(int num_tokens, int nh, int nkv, int& heads_each,
   return (int64_t)num_tokens * nkv * parts >= 512 ? PAE_ROWS_MOST / heads_each : 1;
 }
 
-// Chunks of keys that get workgroups of their own, or 1: a workgroup walks them.  Shared out where the walks would leave most of the
-// chip idle and the chunks are three or more (a token at 60 keys 9.5 and 11.3; 14 heads of 64 at 75 about 8 and 9): 12 heads over 2 of
-// 128, in us, walked and shared: three tokens at 200 keys 20.7 and 12.1, eight at 1,000 71 and 13.4, at
-// 4,000 278 and 49, 64 at 1,000 77 and 71 (128 workgroups), 40 tokens behind 2,000 142 and 85 (80); but a prompt of 200 tokens (400)
-// 33 and 44, 600 tokens 111 and 173: a workgroup's start and end, 5 us, then come once a chunk.  (All with a token a workgroup: where several
-// share one, from 512 such workgroups on, they walk.)
+// Chunks of keys that are shared out, or 1: a workgroup walks them all.  Shared out where the walks would leave half the chip idle and more
+// and the tables have room for three chunks (a token at 60 keys 10.0 and 12.1; 14 heads of 64 at 75 about 8 and 9), over one workgroup a compute unit
+// in all: a count by the tables' room would launch one for every chunk that a longer sequence or a rounded width makes room for, which costs its
+// start also where it finds no key.  12 heads over 2 of 128, in us, walked, shared, and with a workgroup for every chunk in the tables: three
+// tokens at 200 keys of 1,024 21.4, 12.8 and 12.7; eight at 1,000 73, 14.6 and 14.6, at 4,000 278, 42 and 53; 32 at 200 21.6, 13.2 and 22.3; 64 at
+// 130 17.9, 16.0 and 37.6, at 1,000 78, 49 and 70; one at 2,000 beside 63 at 130 143, 80 and 99.  Over 783 such calls (9 kinds of heads) 0.473 of the walk's
+// time and 1.36 at worst (60 keys), by the tables' room 0.523 and 3.1, with two workgroups a unit 0.49 and 1.5.  Prompts walk (200 tokens, 400 workgroups, 33 us,
+// by chunks 44).  (All with a token a workgroup: where several share one, from 512 such workgroups on, they walk.)
 static int split_chunks(int num_tokens, int nh, int nkv, int vd, int max_blocks, int bs) {
   int heads_each, parts;
   rows_of_a_workgroup(num_tokens, nh, nkv, heads_each, parts);
@@ -500,8 +513,8 @@ static int launch_rows(float* out, int64_t out_stride, const float* q, int64_t q
   const int chunks = scratch ? split_chunks(num_tokens, nh, nkv, vd, max_blocks, bs) : 1;
   float* part_ml = scratch;
   float* part_sums = scratch ? scratch + (int64_t)2 * num_tokens * nh * chunks : nullptr;
-  const dim3 grid((num_tokens + toks - 1) / toks, nkv * parts, chunks);
   const size_t lds = (size_t)(PAE_WAVE * (hd + 4 + vd + 4) + PAE_ROWS_MOST * (PAE_WAVE + hd)) * sizeof(float);
+  const dim3 grid((num_tokens + toks - 1) / toks, nkv * parts, chunks > 1 ? min(chunks, SPLIT_UNITS / (num_tokens * nkv * parts)) : 1);
 #define PAE_LAUNCH_EACH(MAXD, EACH, SPLIT)                                                                            \
   do {                                                                                                                \
     if (lds > 65536) {                                                                                                \
@@ -512,7 +525,7 @@ static int launch_rows(float* out, int64_t out_stride, const float* q, int64_t q
     paged_attention_rows_kernel<MAXD, EACH, SPLIT><<<grid, PAE_WAVE * PAE_ROWS_WAVES, lds, stream>>>(                 \
         out, out_stride, q, q_stride, k_cache, v_cache, positions, tok_seq, block_tables, max_blocks, bs, num_tokens, \
         nh, nkv, hd, vd, scale, window, cap, sinks, chunked, slopes, gate, gate_stride, gate_per_head, toks, heads_each, \
-        part_sums, part_ml);                                                                                          \
+        chunks, part_sums, part_ml);                                                                                          \
   } while (0)
 #define PAE_LAUNCH(MAXD)                                                                                              \
   do {                                                                                                                \

@@ -1089,3 +1089,33 @@ def test_float32_attention_with_a_chunk_of_scores_of_minus_infinity(nh, nkv, hd,
                                         torch.arange(pages, dtype=torch.int32, device=DEV)[None], nh, nkv, hd, hd ** -0.5, 0)
             outs.append(out.cpu()[seen])
         assert torch.equal(outs[0], outs[1]) and float((outs[0].double() - want[seen]).abs().max()) < 2e-5, (n, new)
+
+
+@pytest.mark.parametrize("window,chunked", [(0, False), (100, False), (192, True)])
+@pytest.mark.parametrize("nh,nkv,hd,T", [(12, 2, 64, 64), (12, 2, 64, 43), (6, 3, 128, 11), (20, 1, 192, 50)])
+def test_shared_out_chunks_of_sequences_of_many_lengths(nh, nkv, hd, T, window, chunked):
+    """Workgroups that take every second to seventh chunk of 64 keys of a token, beside tokens that have fewer chunks than workgroups: the bits of the
+    kernel with a wavefront per (token, head), which takes pools off 16 bytes.  Keys and values that nobody may see are NaN."""
+    bs, gen = 16, torch.Generator().manual_seed(nh + T)
+    lengths = [1, 64, 65, 128, 700] + torch.randint(1, 701, (T - 5,), generator=gen).tolist()
+    pages = [-(-n // bs) for n in lengths]
+    tables, at = torch.full((T, 48), -1, dtype=torch.int32), 1
+    k_pool, v_pool = (torch.full((sum(pages) + 1, nkv, *shape), float("nan")) for shape in ((bs, hd), (hd, bs)))
+    for s, (n, count) in enumerate(zip(lengths, pages)):
+        first = (n - 1) // window * window if chunked else max(0, n - window) if window else 0
+        tables[s, first // bs:count] = torch.arange(at + first // bs, at + count, dtype=torch.int32)
+        inside = torch.arange(count * bs).view(count, bs) < n
+        k_pool[at:at + count] = torch.randn(count, nkv, bs, hd, generator=gen).masked_fill(~inside[:, None, :, None], float("nan"))
+        v_pool[at:at + count] = torch.randn(count, nkv, hd, bs, generator=gen).masked_fill(~inside[:, None, None], float("nan"))
+        at += count
+    assert K().library().pae_paged_attention_scratch(0, 256, 512, 48, bs, T, nh, nkv, hd, hd, 0) > 0
+    q, positions = torch.randn(T, nh * hd, generator=gen).to(DEV), torch.tensor(lengths, dtype=torch.int32, device=DEV) - 1
+    outs = []
+    for shift in (0, 1):
+        kc = torch.empty(k_pool.numel() + 4, device=DEV)[shift:shift + k_pool.numel()].view(k_pool.shape).copy_(k_pool)
+        vc = torch.empty(v_pool.numel() + 4, device=DEV)[shift:shift + v_pool.numel()].view(v_pool.shape).copy_(v_pool)
+        out = torch.full((T, nh * hd), float("nan"), device=DEV)
+        K().paged_attention_masked(out, q, kc, vc, positions, torch.arange(T, dtype=torch.int32, device=DEV), tables.to(DEV), nh, nkv, hd, hd,
+                                   hd ** -0.5, window, chunked)
+        outs.append(out)
+    assert bool(torch.isfinite(outs[1]).all()) and torch.equal(outs[0], outs[1])
