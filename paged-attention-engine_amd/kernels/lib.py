@@ -10,6 +10,7 @@ functions raise.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 from ctypes import c_char_p, c_float, c_int, c_int64, c_void_p
 from typing import Optional
@@ -652,7 +653,21 @@ def skinny_splits(N: int, K: int, M: int = 1, w: Optional[torch.Tensor] = None) 
     """k ranges for a product whose consumer adds float32 partials: enough workgroups to fill the
     chip (a workgroup takes 16 weight rows, or 32 and more with more than 8 rows of activations).
     `w`: the weights, where they are at hand (see `_streamed_splits`)."""
-    return _streamed_splits(N, K, M, _part_ranges(N, K, M), w, parts=True)
+    return _skinny_splits(N, K, M, _off_16_bytes(w))
+
+
+def _off_16_bytes(w: Optional[torch.Tensor]) -> bool:
+    return w is not None and w.data_ptr() % 16 != 0
+
+
+# The rules for k ranges follow from sizes alone, and a step that is not recorded asks them six times a layer: worked out on each call they were
+# 12 us of the host's 110 a layer (1.5B; short prompts are bound by the host), 1 us looked up.  A model has some ten products by 64 counts of rows.
+_rule_of_sizes = functools.lru_cache(maxsize=4096)
+
+
+@_rule_of_sizes
+def _skinny_splits(N: int, K: int, M: int, off: bool) -> int:
+    return _streamed_splits(N, K, M, _part_ranges(N, K, M), off, parts=True)
 
 
 def _part_ranges(N: int, K: int, M: int) -> int:
@@ -695,11 +710,11 @@ def _part_ranges(N: int, K: int, M: int) -> int:
     return -(-K // k_per)
 
 
-def _streamed_splits(N: int, K: int, M: int, splits: int, w: Optional[torch.Tensor], parts: bool = False) -> int:
+def _streamed_splits(N: int, K: int, M: int, splits: int, off: bool, parts: bool = False) -> int:
     """k ranges of a product of more than 16 rows that csrc/gemm_stream.hip takes (several ranges, or many weight rows), by its
-    times; else, also for weights off 16 bytes, `splits`, which suit the other kernels.  `parts`: the ranges' sums are left for the
-    consumer to add."""
-    if M <= SAME_ORDER_MAX_ROWS or (splits == 1 and N <= 3072) or (w is not None and w.data_ptr() % 16):
+    times; else, also for weights off 16 bytes (`off`), `splits`, which suit the other kernels.  `parts`: the ranges' sums are left
+    for the consumer to add."""
+    if M <= SAME_ORDER_MAX_ROWS or (splits == 1 and N <= 3072) or off:
         return splits
     lib = library()
     return (lib.pae_stream_part_ranges if parts else lib.pae_stream_ranges)(M, N, K) or splits
@@ -723,6 +738,11 @@ def residual_splits(N: int, K: int, M: int = 1, w: Optional[torch.Tensor] = None
     workgroups fill the chip or have little to read (1.5B O at 8 rows 7.2 -> 5.9 us, 7B down 38.3 -> 36.1
     us, 72B down 111 -> 107.5 us); a few workgroups with much to read each want ticketed ranges (1.5B
     down: 96 workgroups of 287 KB, 17.4 us in one workgroup each, 12.5 in five ranges)."""
+    return _residual_splits(N, K, M, _off_16_bytes(w))
+
+
+@_rule_of_sizes
+def _residual_splits(N: int, K: int, M: int, off: bool) -> int:
     if M > SAME_ORDER_MAX_ROWS:
         # Where norms are folded beyond that many rows (all from HBM, at 24 and 64 rows):
         groups32 = -(-N // 32)
@@ -734,7 +754,7 @@ def residual_splits(N: int, K: int, M: int = 1, w: Optional[torch.Tensor] = None
         # workgroups: 15.6 / 17.9 us against 16.8 / 19.9 with four ranges; 3B down, 64 x 4: 18.5 / 22.9 against
         # 21.8 / 28.4 with five; 7B down: eight, 35 / 47 us; 14B: six, 33 / 44; 14B O: six, 19 / 27 against 27 / 37
         # with two)
-        return _streamed_splits(N, K, M, _part_ranges(N, K, M), w)
+        return _streamed_splits(N, K, M, _part_ranges(N, K, M), off)
     tiles = -(-N // 16)
     # one such workgroup fills a compute unit, so the tiles should fill the chip's units a whole number of
     # times, or nearly (14B/32B down: 320 tiles are a full round and a quarter of one; 32B at 8 rows 86.7 us
@@ -1027,6 +1047,11 @@ def whole_sum_splits(N: int, K: int, M: int, w: Optional[torch.Tensor] = None) -
     * not with very few weight rows, where the rows of activations are shared out instead.
     Most products of more than 16 rows are streamed, with ranges of that kernel's own (`_streamed_splits`, `w` as there);
     the rules here are for k that is no multiple of 64 and weights off 16 bytes, and for what that kernel leaves."""
+    return _whole_sum_splits(N, K, M, _off_16_bytes(w))
+
+
+@_rule_of_sizes
+def _whole_sum_splits(N: int, K: int, M: int, off: bool) -> int:
     if M <= SAME_ORDER_MAX_ROWS:
         # from the sizes alone, so that a row's sums do not depend on the batch (as `residual_splits`): one
         # range at every size (QKV from HBM at 1 / 8 / 16 rows, one range against the best of two to six: 72B
@@ -1035,7 +1060,7 @@ def whole_sum_splits(N: int, K: int, M: int, w: Optional[torch.Tensor] = None) -
         return 1
     if library().pae_one_workgroup_a_unit(M, N, K):
         return 1
-    return _streamed_splits(N, K, M, _whole_sum_ranges(N, K, M), w)
+    return _streamed_splits(N, K, M, _whole_sum_ranges(N, K, M), off)
 
 
 def _whole_sum_ranges(N: int, K: int, M: int) -> int:

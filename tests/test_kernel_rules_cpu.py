@@ -163,6 +163,19 @@ def test_ranges_of_products_that_are_not_streamed(M, N, k, ranges):
     assert K.whole_sum_splits(4608, 3584, M) == (streamed or 1)
 
 
+def test_rules_of_sizes_are_worked_out_once(monkeypatch):
+    """A step that is not recorded asks them for every product of every layer, and the host bounds a short prompt's."""
+    off = torch.empty(8, dtype=torch.bfloat16)[1:]
+    asked = [(rule, N, k, M, w) for rule in (K.whole_sum_splits, K.residual_splits, K.skinny_splits) for M in (1, 16, 17, 40, 64)
+             for N, k in ((2048, 1536), (37888, 3584), (3584, 18944), (4608, 3592)) for w in (None, off)]
+    before = [rule(N, k, M, w) for rule, N, k, M, w in asked]
+    monkeypatch.setattr(K, "library", None)
+    monkeypatch.setattr(K, "_part_ranges", None)
+    monkeypatch.setattr(K, "_whole_sum_ranges", None)
+    assert [rule(N, k, M, w) for rule, N, k, M, w in asked] == before
+    assert any(a != b for a, b in zip(before[0::2], before[1::2]))  # weights off 16 bytes have their own
+
+
 def test_projections_that_the_library_is_ahead_at_are_not_rotated_in_tiles():
     """Few tiles with much of k, as for plain products, go to the library and a rotation behind it; elsewhere the tiles are those of gated products."""
     plan = K.library().pae_gemm_wide_plan
