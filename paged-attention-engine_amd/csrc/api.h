@@ -49,7 +49,7 @@ int pae_gemm_skinny(int epilogue, void* out, int64_t ldc, const void* A, int64_t
                     const void* bias, int b_is_f32, int M, int N, int K, int splits, int64_t part_stride,
                     float* ticket_parts, int* ticket_counters, const float* row_stats, int row_stat_tiles,
                     float row_eps, void* next_rows, int64_t ld_next, const void* next_w, int next_w_is_f32,
-                    float* next_stats, hipStream_t stream);
+                    float* next_stats, int next_stat_tiles, hipStream_t stream);
 int pae_gemm_skinny_act(void* out, int64_t ldc, const void* A, int64_t lda, const void* W, const void* bias,
                         int b_is_f32, int M, int N, int K, int splits, float* ticket_parts, int* ticket_counters,
                         int act, hipStream_t stream);
@@ -279,7 +279,7 @@ int pae_program_put_product(void* phases, int index, int epilogue, void* out, in
                             const void* W, const void* bias, int b_is_f32, int M, int N, int K, int splits,
                             float* ticket_parts, int* ticket_counters, const float* row_stats, int row_stat_tiles,
                             float row_eps, void* next_rows, int64_t ld_next, const void* next_w, int next_w_is_f32,
-                            float* next_stats, const SkinnyRope* rope);
+                            float* next_stats, int next_stat_tiles, const SkinnyRope* rope);
 int pae_program_put_product_rope(void* phases, int index, void* q_out, int64_t ldq, const void* A, int64_t lda,
                                  const void* W, const void* bias, int b_is_f32, int M, int K, int nh, int nkv, int hd,
                                  int rot, const float* cos_sin, const int* positions, const int* tok_seq,

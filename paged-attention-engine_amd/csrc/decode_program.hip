@@ -9,9 +9,9 @@
 // "quads" of four wavefronts) and meet at a barrier of their own between phases.
 //
 // Phases are the existing kernels' work, cut into items that the quads take in turn:
-//   product    one item = 16 weight rows x one k range, the quad's wavefronts taking 32-wide k
-//              steps in turn exactly as gemm_skinny_kernel<1, 1, EPI, 4> does (the same sums in the
-//              same order, bit for bit), k ranges added up by ticket, any of that kernel's epilogues;
+//   product    one item = 16 weight rows x one k range, the quad's wavefronts taking 128-wide k
+//              steps in turn exactly as gemm_rows.hip's kernels do (the same sums in the
+//              same order, bit for bit), k ranges added up by ticket, any of those kernels' epilogues;
 //   attention  one item = (token, key/value head, split of 128 keys) as attn_decode_kernel;
 //   merge      one item = 64 (head, four features) of a (token, key/value head): its splits' partial
 //              results added in attn_decode_merge_kernel's order, four groups of splits.
@@ -41,6 +41,7 @@
 #define PROG_THREADS (PROG_QUADS * 4 * PAE_WAVE)
 #define PROG_MAX_ROWS 16
 #define PROG_SPLIT 128    // keys per split of the attention phase: pae_attn_decode_split()
+#define PROG_SUMS (4 * 4 * 4 * 16)  // numbers in one set of a quad's sums: [wavefront][fragment][four rows][16]
 #define PROG_STAMPS 8        // numbers a workgroup may leave per phase in a trace (see pae_program_run)
 
 struct ProgPhase {
@@ -68,7 +69,7 @@ struct ProgPhase {
   int64_t q_stride, out_stride;
   int num_dec, max_splits, max_blocks, bs, nh, nkv, hd, window;
   float scale_log2;
-  int pad_[3];
+  int pad_[1];
 };
 static_assert(sizeof(ProgPhase) % 16 == 0, "phases are copied as 16-byte pieces");
 
@@ -143,33 +144,35 @@ __device__ __forceinline__ bool grid_barrier(ProgBarrier* bar, unsigned& epoch, 
 // k range (workgroup b the range b % splits; with fewer workgroups than ranges, several in turn): it
 // reads the activations of that range once, with device-scope loads, into LDS, in the order in which the
 // matrix instruction wants its B operand, and its quads then take the range's tiles in turn, streaming
-// only weights.  A quad's four wavefronts take the 32-wide k steps of the range in turn and their sums
-// are added in wavefront order through LDS, exactly as gemm_skinny_kernel<1, 1, EPI, 4> adds them.
+// only weights.  A quad's four wavefronts take the 128-wide k steps of the range in turn and their sums
+// are added in wavefront order through LDS, exactly as gemm_rows.hip's kernels add them.
 //
 // Weights do not depend on what a barrier waits for, so a wavefront always has its next chunk of them
-// (up to PROG_S of its k steps, 14 KB a wavefront) on the way: the next tile's while it multiplies the
+// (up to PROG_S of its k steps, 12 KB a wavefront) on the way: the next tile's while it multiplies the
 // current one, and, across the barrier, the first PROG_AHEAD steps of its first tile of the next phase.
 // `coming` carries them from one phase to the next.
-#define PROG_S 14  // most k steps of a wavefront whose weights are asked for together (a chunk)
-#define PROG_AHEAD 4  // steps of its first chunk of the next phase that a wavefront asks for before the barrier
+#define PROG_S 3  // most k steps of a wavefront whose weights are asked for together (a chunk): four fragments each
+#define PROG_AHEAD 1  // steps of its first chunk of the next phase that a wavefront asks for before the barrier
+#define PROG_STEP (4 * 128)  // from one k step of a wavefront to its next
 
-// Where a wavefront's chunk of weights lies: `steps` steps of 32 from k = kb on, 128 apart, of this
-// lane's weight row of width K.  The places past `steps` are asked for from the last step's address
+// Where a wavefront's chunk of weights lies: `steps` steps of 128 from k = kb on, PROG_STEP apart, of this
+// lane's weight rows (one a fragment) of width K.  The places past `steps` are asked for from the last step's address
 // again (a load that is not made would need a branch, and branches between loads make the compiler
 // wait for all of them).
 struct Chunk {
-  const bf16_t* row;
+  const bf16_t* row[4];
   int kb, K, steps;
 };
 
 template <int S, int FROM = 0>
-__device__ __forceinline__ void ask_chunk(bf16x8 (&frag)[PROG_S], const Chunk& c) {
-  const int lkg = threadIdx.x % 4;
+__device__ __forceinline__ void ask_chunk(bf16x8 (&frag)[PROG_S][4], const Chunk& c) {
+  const int piece = piece_of(threadIdx.x % PAE_WAVE);
 #pragma unroll
   for (int u = FROM; u < S; ++u) {
     const int uu = u < c.steps ? u : (c.steps > 0 ? c.steps - 1 : 0);
-    const int k = c.kb + 128 * uu + 8 * lkg;
-    frag[u] = *reinterpret_cast<const bf16x8*>(c.row + (k < c.K - 8 ? k : c.K - 8));
+    const int k = c.kb + PROG_STEP * uu + 8 * piece;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) frag[u][r] = *reinterpret_cast<const bf16x8*>(c.row[r] + (k < c.K - 8 ? k : c.K - 8));
   }
 }
 
@@ -193,28 +196,28 @@ __device__ __forceinline__ Share share_of(int splits, int range_turn, int quad) 
   return sh;
 }
 
-// This lane's weight row of a tile (row lane / 4, through the rotation's row order if any).
-__device__ __forceinline__ const bf16_t* weight_row(const ProgPhase& ph, int tile) {
-  const int lrow = threadIdx.x % PAE_WAVE / 4;
-  int n = 16 * tile + lrow;
+// This lane's weight row of a tile's fragment r (through the rotation's row order if any).
+__device__ __forceinline__ const bf16_t* weight_row(const ProgPhase& ph, int tile, int r) {
+  const int place = 4 * r + piece_row(threadIdx.x % PAE_WAVE);
+  int n = 16 * tile + place;
   if (ph.epilogue == EPI_ROPE) {
     const int per_head = ph.rope.hd / 16;
-    n = tile / per_head * ph.rope.hd + rope_feature(tile % per_head, lrow, ph.rope.rot);
+    n = tile / per_head * ph.rope.hd + rope_feature(tile % per_head, place, ph.rope.rot);
   }
   return in_memory(ph.W) + (int64_t)(n < ph.N ? n : ph.N - 1) * ph.K;  // rows past N are loaded from the last row and never stored
 }
 
-// k steps of 32 that one wavefront makes in a k range, at most, and whether its chunks are the short kind
-__device__ __forceinline__ int steps_of(const ProgPhase& ph) { return (min(ph.k_per_split, ph.K) + 127) / 128; }
-__device__ __forceinline__ bool short_chunks(const ProgPhase& ph) { return steps_of(ph) <= 4; }
+// k steps of 128 that one wavefront makes in a k range, at most, and whether its chunks are the short kind
+__device__ __forceinline__ int steps_of(const ProgPhase& ph) { return (min(ph.k_per_split, ph.K) + PROG_STEP - 1) / PROG_STEP; }
+__device__ __forceinline__ bool short_chunks(const ProgPhase& ph) { return steps_of(ph) <= 1; }
 
 // Chunk `c` of wavefront `wq` of a quad for `tile` in k range `range`.
 __device__ __forceinline__ Chunk chunk_of(const ProgPhase& ph, int tile, int range, int c, int wq) {
-  const int S = short_chunks(ph) ? 4 : PROG_S;
+  const int S = short_chunks(ph) ? 1 : PROG_S;
   const int k_lo = range * ph.k_per_split, k_hi = min(ph.K, k_lo + ph.k_per_split);
-  const int kb = k_lo + 32 * wq + 128 * S * c;
-  const int left = kb < k_hi ? (k_hi - kb + 127) / 128 : 0;
-  return Chunk{weight_row(ph, tile), kb, ph.K, left < S ? left : S};
+  const int kb = k_lo + 128 * wq + PROG_STEP * S * c;
+  const int left = kb < k_hi ? (k_hi - kb + PROG_STEP - 1) / PROG_STEP : 0;
+  return Chunk{{weight_row(ph, tile, 0), weight_row(ph, tile, 1), weight_row(ph, tile, 2), weight_row(ph, tile, 3)}, kb, ph.K, left < S ? left : S};
 }
 
 // The first chunk of this quad's first tile of phase `next`, if it is a product in which the quad has one.
@@ -227,16 +230,15 @@ __device__ __forceinline__ bool first_chunk_of(const ProgPhase* next, int quad, 
 }
 
 __device__ __forceinline__ void product_phase(const ProgPhase& ph, const ProgPhase* next, float* quad_lds, bf16x8* a_lds,
-                                              int& parity, bf16x8 (&coming)[PROG_S], bool& has_coming, long long* stamps) {
+                                              int& parity, bf16x8 (&coming)[PROG_S][4], bool& has_coming, long long* stamps) {
   const int lane = threadIdx.x % PAE_WAVE;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PAE_WAVE), quad = wave / 4, wq = wave % 4;
   const int M = ph.M, N = ph.N, K = ph.K, splits = ph.splits;
   const int tiles = (N + 15) / 16;
-  const int g4 = lane / 16;
-  const int fetch_from = ((lane % 16) * 4 + lane / 16) * 4;
+  const int g4 = lane / 16, piece = piece_of(lane), groups_of_rows = (M + 3) / 4;
   const bool brief = short_chunks(ph);  // the same in the whole grid
-  const int S = brief ? 4 : PROG_S, chunks_a_tile = (steps_of(ph) + S - 1) / S;
-  float* s_scale = quad_lds + 2 * 3 * 4 * PAE_WAVE;  // [16], behind the two sets of partial sums
+  const int S = brief ? 1 : PROG_S, chunks_a_tile = (steps_of(ph) + S - 1) / S;
+  float* s_scale = quad_lds + 2 * PROG_SUMS;  // [16], behind the two sets of partial sums
   const bf16x8 zero = {};
   const int groups = (int)gridDim.x, group = (int)blockIdx.x;
   const int range_turns = groups >= splits ? 1 : (splits - group + groups - 1) / groups;
@@ -249,7 +251,7 @@ __device__ __forceinline__ void product_phase(const ProgPhase& ph, const ProgPha
     c = chunk_of(ph, tile, sh.range, j % chunks_a_tile, wq);
     return true;
   };
-  const Chunk nothing = {in_memory(ph.W), 0, K, 1};  // asked for where a wavefront has nothing to ask for
+  const Chunk nothing = {{in_memory(ph.W), in_memory(ph.W), in_memory(ph.W), in_memory(ph.W)}, 0, K, 1};  // asked for where a wavefront has nothing to ask for
   // Of the first chunk only PROG_AHEAD steps were asked for before the barrier, as much as arrives while
   // the barrier is crossed and the activations are fetched; the rest is asked for once the activations are
   // there (asked for earlier, the weights that fast workgroups want fill the memory's queues in front of
@@ -260,10 +262,10 @@ __device__ __forceinline__ void product_phase(const ProgPhase& ph, const ProgPha
   for (int turn = 0; turn < range_turns; ++turn) {
     const Share sh = share_of(splits, turn, quad);
     const int k_lo = sh.range * ph.k_per_split, k_hi = min(K, k_lo + ph.k_per_split);
-    // the range's activations: chunk c of row m (8 elements at k_lo + 8 c) is what lane 16 (c % 4) + m of
-    // k step c / 4 multiplies; the last step's chunks past the range are zero (their weights are zeroed
+    // the range's activations, in fragments of (k step of 128, four rows): piece c of row m (8 elements at k_lo + 8 c) belongs to
+    // step c / 16 and to the lane whose row and piece it is; the last step's pieces past the range are zero (their weights are zeroed
     // too, but zero times whatever LDS held is not always zero)
-    const int chunks = (k_hi - k_lo) / 8, padded = (chunks + 3) / 4 * 4;
+    const int chunks = (k_hi - k_lo) / 8, padded = (chunks + 15) / 16 * 16;
     if (turn > 0) __syncthreads();  // the range before has been read
     const bf16_t* A = in_memory(ph.A);
     constexpr int AT_ONCE = 4;
@@ -278,7 +280,7 @@ __device__ __forceinline__ void product_phase(const ProgPhase& ph, const ProgPha
 #pragma unroll
       for (int q = 0; q < AT_ONCE; ++q) {
         const int idx = base + q * PROG_THREADS, m = idx / padded, c = idx % padded;
-        if (idx < M * padded) a_lds[(c / 4) * PAE_WAVE + (c % 4) * 16 + m] = v[q];
+        if (idx < M * padded) a_lds[(c / 16 * groups_of_rows + m / 4) * PAE_WAVE + c % 16 / 4 * 16 + m % 4 * 4 + c % 4] = v[q];
       }
     }
     __syncthreads();
@@ -286,7 +288,7 @@ __device__ __forceinline__ void product_phase(const ProgPhase& ph, const ProgPha
     if (rest_to_ask) {  // the same in the whole workgroup
       rest_to_ask = false;
       if (!has_coming) {
-        if (brief) ask_chunk<4>(coming, first_chunk);
+        if (brief) ask_chunk<1>(coming, first_chunk);
         else ask_chunk<PROG_S>(coming, first_chunk);
       } else if (!brief) {
         ask_chunk<PROG_S, PROG_AHEAD>(coming, first_chunk);
@@ -297,24 +299,29 @@ __device__ __forceinline__ void product_phase(const ProgPhase& ph, const ProgPha
     }
     const int rounds = (tiles + sh.stride - 1) / sh.stride;  // the same for the quads of a workgroup
     const int total = rounds * chunks_a_tile;
-    f32x4 acc[1][1] = {{(f32x4){0.f, 0.f, 0.f, 0.f}}};
+    f32x4 acc[4][4];
     EpilogueAhead<1> pre = {};
     for (int j = 0; j < total; ++j) {
-      bf16x8 cur[PROG_S];
+      bf16x8 cur[PROG_S][4];
 #pragma unroll
-      for (int u = 0; u < PROG_S; ++u) cur[u] = coming[u];
+      for (int u = 0; u < PROG_S; ++u)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) cur[u][r] = coming[u][r];
       // the chunk after this one, of this range or the next
       if (j + 1 < total || turn + 1 < range_turns) {
         Chunk c = nothing;
         if (j + 1 < total) in_turn(turn, j + 1, c);
         else in_turn(turn + 1, 0, c);
-        if (brief) ask_chunk<4>(coming, c);
+        if (brief) ask_chunk<1>(coming, c);
         else ask_chunk<PROG_S>(coming, c);
       }
       const int tile = sh.first + j / chunks_a_tile * sh.stride, c_in_tile = j % chunks_a_tile;
       const bool live = tile < tiles;  // the same in every lane of the quad
       if (c_in_tile == 0) {
-        acc[0][0] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int g = 0; g < 4; ++g) acc[r][g] = (f32x4){0.f, 0.f, 0.f, 0.f};
         // what the tile's epilogue reads beside the sums is asked for now (by the wavefront that runs it)
         if (live && wq == 0) {
           if (ph.epilogue == EPI_ROPE) ask_row<1, EPI_ROPE>(pre, M, in_memory(ph.rope));
@@ -323,47 +330,60 @@ __device__ __forceinline__ void product_phase(const ProgPhase& ph, const ProgPha
         }
       }
       if (live) {
-        const int kb = k_lo + 32 * wq + 128 * S * c_in_tile;
+        const int kb = k_lo + 128 * wq + PROG_STEP * S * c_in_tile;
         auto multiply = [&](auto steps) {
 #pragma unroll
           for (int u = 0; u < decltype(steps)::value; ++u) {
-            // four steps' operands at a time (read ahead for a whole chunk they would not fit the registers)
-            if (u % 4 == 0 && u > 0) asm volatile("" ::: "memory");
-            const int k = kb + 128 * u;  // this wavefront's step: k .. k + 31
-            const bool kok = k + 8 * g4 < k_hi;
+            // one step's operands at a time (read ahead for a whole chunk they would not fit the registers)
+            if (u > 0) asm volatile("" ::: "memory");
+            const int k = kb + PROG_STEP * u;  // this wavefront's step: k .. k + 127
+            const bool kok = k + 8 * piece < k_hi;
             // (past the range the step's place in LDS is the last one's: its weights are zero)
-            const bf16x8 a = a_lds[(min(k, k_hi - 1) - k_lo) / 32 * PAE_WAVE + lane];
-            const bf16x8 moved = to_mfma_order(cur[u], fetch_from);
-            acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kok ? moved : zero, a, acc[0][0], 0, 0, 0);
+            const bf16x8* at = a_lds + (min(k, k_hi - 1) - k_lo) / 128 * groups_of_rows * PAE_WAVE + lane;
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+              if (g >= groups_of_rows) break;
+              const bf16x8 a = at[g * PAE_WAVE];
+#pragma unroll
+              for (int r = 0; r < 4; ++r) acc[r][g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kok ? cur[u][r] : zero, a, acc[r][g], 0, 0, 0);
+            }
           }
         };
-        if (brief) multiply(std::integral_constant<int, 4>{});
+        if (brief) multiply(std::integral_constant<int, 1>{});
         else multiply(std::integral_constant<int, PROG_S>{});
       }
       if (stamps && threadIdx.x == 0 && turn == 0 && j == 0) stamps[3] = wall_clock64();
       if (c_in_tile + 1 < chunks_a_tile) continue;
       // the tile's sums: the four wavefronts' in wavefront order, then the k ranges', then the epilogue
-      float* s_part = quad_lds + parity * (3 * 4 * PAE_WAVE);  // [3][4][64]
+      float* s_part = quad_lds + parity * PROG_SUMS;  // [wavefront][fragment of weight rows][four rows of A][16]
       parity ^= 1;
-      if (live && wq > 0) {
+      if (live) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) s_part[((wq - 1) * 4 + i) * PAE_WAVE + lane] = acc[0][0][i];
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            const float sum = sum_of_parts(acc[r][g]);
+            if (lane % 4 == 0) s_part[((wq * 4 + r) * 4 + g) * 16 + lane / 4] = sum;
+          }
       }
       __syncthreads();
       if (stamps && threadIdx.x == 0 && turn == 0 && j + 1 == chunks_a_tile) stamps[4] = wall_clock64();
       if (!live || wq > 0) continue;
+      f32x4 sums[1][1];
 #pragma unroll
-      for (int w = 0; w < 3; ++w)
+      for (int i = 0; i < 4; ++i) {
+        const float* mine = s_part + (g4 * 4 + lane % 16 / 4) * 16 + 4 * i + lane % 4;
+        float sum = mine[0];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) acc[0][0][i] += s_part[(w * 4 + i) * PAE_WAVE + lane];
+        for (int w = 1; w < 4; ++w) sum += mine[w * 256];
+        sums[0][0][i] = sum;
+      }
       const float scale[1] = {s_scale[lane % 16]};
       if (ph.epilogue != EPI_F32 && splits > 1) {
-        f32x4 mine[1] = {acc[0][0]};
-        if (!add_up_k_ranges<1, 4>(mine, tile, sh.range, splits, SkinnyTickets{in_memory(ph.ticket_parts), in_memory(ph.ticket_counters)})) continue;
-        acc[0][0] = mine[0];
+        if (!add_up_k_ranges<1, 4>(sums[0], tile, sh.range, splits, SkinnyTickets{in_memory(ph.ticket_parts), in_memory(ph.ticket_counters)})) continue;
       }
 #define PROG_EPILOGUE(EPI)                                                                                          \
-  skinny_epilogue<1, 1, EPI, true>(acc, tile, -1, in_memory(ph.out), ph.ldc, in_memory(ph.bias), ph.b_is_f32, M, N, sh.range, \
+  skinny_epilogue<1, 1, EPI, true>(sums, tile, -1, in_memory(ph.out), ph.ldc, in_memory(ph.bias), ph.b_is_f32, M, N, sh.range, \
                                    (int64_t)M * N, in_memory(ph.rope), in_memory(ph.norm), scale, AHEAD)
       switch (ph.epilogue) {  // the one place where the epilogues part ways: the products above are the same code for all
 #define AHEAD nullptr
@@ -622,7 +642,7 @@ __global__ __launch_bounds__(PROG_THREADS) void decode_program_kernel(const Prog
   }
   __syncthreads();
   int parity = 0;
-  bf16x8 coming[PROG_S] = {};  // a wavefront's next chunk of weights, asked for ahead (see product_phase)
+  bf16x8 coming[PROG_S][4] = {};  // a wavefront's next chunk of weights, asked for ahead (see product_phase)
   bool has_coming = false;
   for (int p = 0; p < num_phases; ++p) {
     const ProgPhase& ph = s_phase[p % 3];
@@ -645,7 +665,9 @@ __global__ __launch_bounds__(PROG_THREADS) void decode_program_kernel(const Prog
       }
       has_coming = false;  // nothing is carried across an attention phase: the registers are free during it
 #pragma unroll
-      for (int u = 0; u < PROG_S; ++u) coming[u] = bf16x8{};
+      for (int u = 0; u < PROG_S; ++u)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) coming[u][r] = bf16x8{};
     }
     if (trace && threadIdx.x == 0) trace[((int64_t)p * gridDim.x + blockIdx.x) * PROG_STAMPS + 1] = wall_clock64();
     if (p + 1 == num_phases) break;
@@ -663,7 +685,7 @@ extern "C" int pae_program_phase_bytes() { return (int)sizeof(ProgPhase); }
 extern "C" int pae_program_barrier_bytes() { return (int)sizeof(ProgBarrier); }
 extern "C" int pae_program_max_rows() { return PROG_MAX_ROWS; }
 
-static int quad_bytes_of_product() { return (2 * 3 * 4 * PAE_WAVE + 16) * (int)sizeof(float); }
+static int quad_bytes_of_product() { return (2 * PROG_SUMS + 16) * (int)sizeof(float); }
 
 // Bytes of LDS that the activations of one k range of a product take in a workgroup: `rows` rows of one
 // range, whole k steps of 32.
@@ -671,8 +693,8 @@ extern "C" int pae_program_activation_bytes(int rows, int K, int splits) {
   if (rows < 1 || K < 1 || splits < 1) return 0;
   int k_per_split = (K + splits - 1) / splits;
   k_per_split = (k_per_split + 127) / 128 * 128;
-  if (k_per_split > K) k_per_split = (K + 31) / 32 * 32;
-  return k_per_split / 32 * PAE_WAVE * 16;
+  if (k_per_split > K) k_per_split = (K + 127) / 128 * 128;
+  return k_per_split / 128 * (PROG_MAX_ROWS / 4) * PAE_WAVE * 16;  // of the most rows: whether a phase fits does not depend on them
 }
 extern "C" int pae_program_lds_limit();
 
@@ -683,7 +705,8 @@ extern "C" int pae_program_put_product(void* phases, int index, int epilogue, vo
                                        int64_t lda, const void* W, const void* bias, int b_is_f32, int M, int N, int K,
                                        int splits, float* ticket_parts, int* ticket_counters, const float* row_stats,
                                        int row_stat_tiles, float row_eps, void* next_rows, int64_t ld_next,
-                                       const void* next_w, int next_w_is_f32, float* next_stats, const SkinnyRope* rope) {
+                                       const void* next_w, int next_w_is_f32, float* next_stats, int next_stat_tiles,
+                                       const SkinnyRope* rope) {
   PAE_REQUIRE(phases && index >= 0, "decode program: no room for phase %d", index);
   PAE_REQUIRE(M >= 1 && M <= PROG_MAX_ROWS, "decode program: a product of %d rows (1..%d are taken)", M, PROG_MAX_ROWS);
   PAE_REQUIRE(N > 0 && K > 0 && K % 8 == 0 && lda % 8 == 0, "decode program: N=%d K=%d lda=%lld (K and lda must be multiples of 8)",
@@ -697,6 +720,8 @@ extern "C" int pae_program_put_product(void* phases, int index, int epilogue, vo
   PAE_REQUIRE(!row_stats || row_stat_tiles > 0, "decode program: a row scale needs its shares of the sums of squares");
   PAE_REQUIRE(epilogue != EPI_RESIDUAL || (next_rows && next_w && next_stats && ld_next >= N && !bias),
               "decode program: the residual epilogue needs the next rows, the next norm's weight and room for its sums, and takes no bias");
+  PAE_REQUIRE(epilogue != EPI_RESIDUAL || next_stat_tiles == (N + 15) / 16 || next_stat_tiles == 2 * ((N + 15) / 16),
+              "decode program: %d shares of a row's sum of squares for %d columns", next_stat_tiles, N);
   PAE_REQUIRE(epilogue != EPI_SWIGLU || (N % 16 == 0 && ldc % 4 == 0), "decode program: gated epilogue needs N %% 16 == 0, got %d", N);
   PAE_REQUIRE(epilogue != EPI_ROPE || N % 16 == 0, "decode program: the rotating epilogue needs whole tiles, N=%d", N);
   int k_per_split = (K + splits - 1) / splits;
@@ -708,7 +733,7 @@ extern "C" int pae_program_put_product(void* phases, int index, int epilogue, vo
   ph.M = M; ph.N = N; ph.K = K; ph.splits = splits; ph.k_per_split = k_per_split; ph.b_is_f32 = b_is_f32;
   ph.W = (const bf16_t*)W; ph.bias = bias; ph.A = (const bf16_t*)A; ph.out = out;
   ph.lda = lda; ph.ldc = ldc;
-  ph.norm = SkinnyNorm{row_stats, row_stat_tiles, row_eps, (bf16_t*)next_rows, ld_next, next_w, next_w_is_f32, 0, next_stats};
+  ph.norm = SkinnyNorm{row_stats, row_stat_tiles, row_eps, (bf16_t*)next_rows, ld_next, next_w, next_w_is_f32, 0, next_stats, next_stat_tiles};
   if (rope) ph.rope = *rope;
   ph.ticket_parts = ticketed ? ticket_parts : nullptr;
   ph.ticket_counters = ticketed ? ticket_counters : nullptr;
@@ -735,7 +760,7 @@ extern "C" int pae_program_put_product_rope(void* phases, int index, void* q_out
                         nh, nkv, hd, rot, max_blocks, bs};
   return pae_program_put_product(phases, index, EPI_ROPE, q_out, ldq, A, lda, W, bias, b_is_f32, M, (nh + 2 * nkv) * hd, K,
                                  splits, ticket_parts, ticket_counters, row_stats, row_stat_tiles, row_eps, nullptr, 0,
-                                 nullptr, 0, nullptr, &rope);
+                                 nullptr, 0, nullptr, 0, &rope);
 }
 
 // Decode attention of num_dec tokens; arguments as pae_attn_decode_bf16.  Writes two phases, index and

@@ -20,27 +20,22 @@
 // makes a round trip through memory.
 #include "common.h"
 #include "api.h"
+#include "gemm_rows.h"
 #include "gemm_stream.h"
 
 // MT: column tiles of 16 rows of A; RT: tiles of 16 weight rows per workgroup; SKINNY_U: k steps
-// of a wavefront whose loads are in flight together.  With more
-// rows of A a workgroup takes more weight rows, so that the activations, which every
-// workgroup re-reads from L2, do not outweigh the weights.
-template <int MT, int RT, int EPI, int SKINNY_U, int NW = 4>
-__global__ __launch_bounds__(64 * NW) void gemm_skinny_kernel(void* __restrict__ out, int64_t ldc,
+// of a wavefront whose loads are in flight together.  With one column tile the rows of A are shared out over grid.z, 16 to a
+// workgroup.
+template <int MT, int RT, int EPI, int SKINNY_U>
+__global__ __launch_bounds__(256) void gemm_skinny_kernel(void* __restrict__ out, int64_t ldc,
                                                           const bf16_t* __restrict__ A, int64_t lda,
                                                           const bf16_t* __restrict__ W,
                                                           const void* __restrict__ bias, int b_is_f32, int M,
                                                           int N, int K, int k_per_split, int64_t part_stride,
                                                           SkinnyRope rope, SkinnyTickets tickets, SkinnyNorm norm) {
-  // NW == 16 (one column tile only): the workgroup holds four k ranges side by side, four wavefronts to
-  // each, and adds the ranges' sums in range order itself: the sums, bit for bit, of four workgroups
-  // with one range each whose results the last to finish adds up (grid.y == 4), without the tickets
-  // and the trip to memory.
-  static_assert(NW == 4 || (NW == 16 && MT == 1), "sixteen wavefronts only with one column tile");
-  __shared__ float s_part[MT == 1 ? NW - 1 : 4][RT * MT * 4][PAE_WAVE];
+  __shared__ float s_part[MT == 1 ? 3 : 4][RT * MT * 4][PAE_WAVE];
   __shared__ float s_scale[16 * MT];  // what the folded norm owes every row of A
-  if (MT == 1 && gridDim.z > 1) {  // the rows of A are shared out in tiles of 16: this workgroup's tile
+  if (MT == 1 && gridDim.z > 1) {  // this workgroup's tile of 16 rows
     const int m0 = blockIdx.z * 16;
     A += (int64_t)m0 * lda;
     out = (EPI == EPI_F32 || EPI == EPI_RESIDUAL) ? (void*)((float*)out + (int64_t)m0 * ldc)
@@ -49,7 +44,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_skinny_kernel(void* __restrict__
     if (norm.row_stats) norm.row_stats += (int64_t)m0 * norm.row_stat_tiles;
     if (EPI == EPI_RESIDUAL) {
       norm.next_rows += (int64_t)m0 * norm.ld_next;
-      norm.next_stats += (int64_t)m0 * ((N + 15) / 16);
+      norm.next_stats += (int64_t)m0 * norm.next_stat_tiles;
     }
     if (EPI == EPI_ROPE) {
       rope.positions += m0;
@@ -63,7 +58,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_skinny_kernel(void* __restrict__
   constexpr bool AHEAD = MT == 1 && (EPI == EPI_RESIDUAL || EPI == EPI_ROPE);
   EpilogueAhead<RT> ahead;
   const int n0 = blockIdx.x * 16 * RT;
-  const int k_lo = (NW == 16 ? wave / 4 : blockIdx.y) * k_per_split;
+  const int k_lo = blockIdx.y * k_per_split;
   const int k_hi = min(K, k_lo + k_per_split);
 
   // Loads are made with the lane order (row = lane / 4, k group = lane % 4): the four lanes of a
@@ -99,7 +94,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_skinny_kernel(void* __restrict__
   // addresses, and issued SKINNY_U steps ahead of their use; a lane past the end of
   // the k range zeroes its weight fragment (rows past N or M are simply not stored).
   const bf16x8 zero = {};
-  constexpr int KW = 128;  // a range's four wavefronts take 32-wide k steps in turn
+  constexpr int KW = 128;  // the four wavefronts take 32-wide k steps in turn
   struct Batch {  // SKINNY_U steps of a wavefront: k offsets kb + KW u
     bf16x8 wf[SKINNY_U][RT], af[SKINNY_U][MT];
   };
@@ -133,7 +128,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_skinny_kernel(void* __restrict__
     }
   };
   constexpr int STEP = KW * SKINNY_U;
-  int kb = k_lo + 32 * (wave % 4);  // the same in every lane of a wavefront: the branches on it are uniform
+  int kb = k_lo + 32 * (wave);  // the same in every lane of a wavefront: the branches on it are uniform
   {
     // Two batches take turns, so that a wavefront always has loads in flight: with one, every batch
     // waits out the memory's latency before the next is even asked for.  No load below stands under a
@@ -181,19 +176,6 @@ __global__ __launch_bounds__(64 * NW) void gemm_skinny_kernel(void* __restrict__
       for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc[rt][0][i] += s_part[w][rt * 4 + i][lane];
-    if (NW == 16) {  // the other three ranges: each added up in wavefront order, then onto the first in range order
-#pragma unroll
-      for (int range = 1; range < 4; ++range)
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            float sum = s_part[4 * range - 1][rt * 4 + i][lane];
-#pragma unroll
-            for (int w = 0; w < 3; ++w) sum += s_part[4 * range + w][rt * 4 + i][lane];
-            acc[rt][0][i] += sum;
-          }
-    }
   } else {
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
@@ -397,24 +379,16 @@ static int launch_skinny(int epilogue, void* out, int64_t ldc, const void* A, in
   PAE_REQUIRE(!norm.row_stats || norm.row_stat_tiles > 0, "gemm_skinny: a row scale needs its shares of the sums of squares");
   PAE_REQUIRE(epilogue != EPI_RESIDUAL || (norm.next_rows && norm.next_w && norm.next_stats && norm.ld_next >= N && !bias),
               "gemm_skinny: the residual epilogue needs the next rows, the next norm's weight and room for its sums, and takes no bias");
+  PAE_REQUIRE(epilogue != EPI_RESIDUAL || norm.next_stat_tiles == (N + 15) / 16 || norm.next_stat_tiles == 2 * ((N + 15) / 16),
+              "gemm_skinny: %d shares of a row's sum of squares for %d columns (one per 16 columns, or two)", norm.next_stat_tiles, N);
   PAE_REQUIRE(epilogue != EPI_SWIGLU || (N % 16 == 0 && ldc % 4 == 0), "gemm_skinny: gated epilogue needs N %% 16 == 0, got %d", N);
   if (M == 0) return 0;
-  // weight rows per workgroup: 16 for up to 8 rows of A, else 32, so that the activations, which every
-  // workgroup re-reads, stay behind the weights (9 to 16 rows with 32: 7B gate/up at 16 rows 70.6 -> 63.5 us,
-  // 32B 148.6 -> 135.8, 72B down 128.5 -> 108.6 us; at 8 rows and below 16 are as fast or faster at most
-  // sizes), unless that leaves too few workgroups (the QKV product of the 1.5B sizes at 16 rows: 64
-  // workgroups, 9.2 us).  5 to 8 rows with 32 only where there are very many weight rows (gate/up at 8
-  // rows: 7B, 1,184 such workgroups, 61.1 -> 57.9 us, 32B, 1,728, 129.0 -> 123.2; but 1.5B, 560, 14.2 -> 15.0,
-  // 14B, 864, 67.0 -> 67.6; at 4 rows and below never ahead; not with several k ranges: the 72B QKV product
-  // in four ranges, 1,280 such workgroups, 40.4 -> 60.2 us).  Never with k ranges of 8,192 and more: 72B
-  // gate/up, whose rows lie 16 KB apart, takes 195.9 us at 9 rows with 16 and 243.9 us with 32.
   const int mt = (M + 15) / 16;
-  const int64_t groups32 = (int64_t)((N + 31) / 32) * splits;
-  const bool long_ranges = (K + splits - 1) / splits >= 8192;
-  const int rt = mt >= 2 || (!long_ranges && ((M > 8 && groups32 >= 128) || (M > 4 && splits == 1 && groups32 >= 1024))) ? 2 : 1;
   int k_per_split = (K + splits - 1) / splits;
   k_per_split = (k_per_split + 127) / 128 * 128;
   PAE_REQUIRE((int64_t)k_per_split * (splits - 1) < K, "gemm_skinny: %d k ranges are too many for K=%d", splits, K);
+  const RowsProduct rows{epilogue, out, ldc, (const bf16_t*)A, lda, (const bf16_t*)W, bias, b_is_f32, M, N, K, splits, part_stride, rope, tickets, norm};
+  if (mt == 1) return launch_rows(rows, stream);
   if (const int tiles = stream_tiles(epilogue, A, W, M, N, K, lda, splits)) {
     const StreamProduct p{epilogue, out, ldc, (const bf16_t*)A, lda, (const bf16_t*)W, bias, b_is_f32, M, N, K, k_per_split,
                           part_stride, rope, tickets, norm};
@@ -431,8 +405,6 @@ static int launch_skinny(int epilogue, void* out, int64_t ldc, const void* A, in
   const bool only_narrow_fills = (int64_t)medium_groups * splits < 256 && (int64_t)narrow_groups * splits >= 384;
   const bool wide = !only_narrow_fills &&
                     (mt > 3 || (int64_t)medium_groups * splits >= 1024 || (int64_t)narrow_groups * splits < 512);
-  // (up to 16 rows every product takes the first kernel, whose order of adding the decode program shares:
-  // a row's sums are then the same bits alone, in a batch, in a program or launched by itself)
   // One k range and 16 W weight rows a workgroup (W = 5 to 8 wavefronts of 16 rows each) where that many
   // workgroups are nearly as many as the chip's 256 compute units: every unit then streams its share of
   // the weights once, with no partial sums to write and fetch back (1.5B gate/up, 224 workgroups of 80
@@ -480,7 +452,6 @@ static int launch_skinny(int epilogue, void* out, int64_t ldc, const void* A, in
                                                               bias, b_is_f32, M, N, K, k_per_split, part_stride, rope, tickets, norm)
 #define MEDIUM_BY_MT(EPI)                       \
   switch (mt) {                                 \
-    case 1: LAUNCH_MEDIUM(1, EPI); break;       \
     case 2: LAUNCH_MEDIUM(2, EPI); break;       \
     case 3: LAUNCH_MEDIUM(3, EPI); break;       \
     default: LAUNCH_MEDIUM(4, EPI); break;      \
@@ -498,16 +469,18 @@ static int launch_skinny(int epilogue, void* out, int64_t ldc, const void* A, in
     return pae_check_launch("gemm_medium");
   }
   // Very few weight rows (the QKV product of the 1.5B sizes: 64 workgroups of 32 rows): the rows of A are
-  // shared out too, 16 to a workgroup of the one-tile kernel, and the weights are read once from HBM and
-  // again from L2 (1.5B QKV at 64 rows 10.5 -> 6.7 us; from about 100 workgroups on it is slower).
-  if (mt >= 2 && !ticketed && (int64_t)((N + 31) / 32) * splits <= 96) {
+  // shared out too, 16 to a workgroup, and the weights are read once from HBM and
+  // again from L2 (1.5B QKV at 64 rows 10.5 -> 6.7 us; from about 100 workgroups on it is slower).  Plain float32 sums by the few
+  // rows' kernels, in whose order of adding a row is the same bits alone and in such a step (1.5B O at 17 / 64 rows 4.5 / 5.5 us either way);
+  // the other epilogues by the one-tile kernel, where those are behind (0.5B down 9.7 / 11.2 us against 15.6, 3B O 6.5 / 8.9 against 9.4 / 10.1).
+  if (!ticketed && (int64_t)((N + 31) / 32) * splits <= 96) {
+    if (epilogue == EPI_F32) return launch_rows(rows, stream);
     dim3 tiled((N + 15) / 16, splits, mt);
 #define LAUNCH_TILED(EPI)                                                                                        \
   gemm_skinny_kernel<1, 1, EPI, 4><<<tiled, 256, 0, stream>>>(out, ldc, (const bf16_t*)A, lda, (const bf16_t*)W, bias, \
                                                                b_is_f32, M, N, K, k_per_split, part_stride, rope, tickets, norm)
     switch (epilogue) {
       case EPI_BF16: LAUNCH_TILED(EPI_BF16); break;
-      case EPI_F32: LAUNCH_TILED(EPI_F32); break;
       case EPI_SWIGLU: LAUNCH_TILED(EPI_SWIGLU); break;
       case EPI_ROPE: LAUNCH_TILED(EPI_ROPE); break;
       case EPI_RESIDUAL: LAUNCH_TILED(EPI_RESIDUAL); break;
@@ -516,27 +489,16 @@ static int launch_skinny(int epilogue, void* out, int64_t ldc, const void* A, in
 #undef LAUNCH_TILED
     return pae_check_launch("gemm_skinny (rows of A in tiles)");
   }
-  if (epilogue == EPI_RESIDUAL && mt == 1 && splits == 4 && K >= 1024 && ((N + 15) / 16 >= 192 || 32 * (int64_t)K <= 65536)) {
-    // Four k ranges side by side in one workgroup of sixteen wavefronts: no tickets, no trip to memory
-    // for partial sums; few workgroups, but each keeps its compute unit's memory pipeline full.  Ahead
-    // wherever the 16-row workgroups fill the chip or have little to read each (1.5B O at 8 rows 7.2 ->
-    // 5.9 us, 7B down 38.3 -> 36.1 us); the same bits as the ticketed ranges (see the kernel).
-    gemm_skinny_kernel<1, 1, EPI_RESIDUAL, 4, 16><<<dim3((N + 15) / 16, 1), 1024, 0, stream>>>(
-        out, ldc, (const bf16_t*)A, lda, (const bf16_t*)W, bias, b_is_f32, M, N, K, k_per_split, part_stride, rope,
-        SkinnyTickets{nullptr, nullptr}, norm);
-    return pae_check_launch("gemm_skinny (sixteen wavefronts)");
-  }
-  dim3 grid((N + 16 * rt - 1) / (16 * rt), splits);
-  // four k steps of loads in flight per wavefront: deeper prefetch costs registers and measured slower
-#define LAUNCH(MT, RT, EPI)                                                                                  \
-  gemm_skinny_kernel<MT, RT, EPI, (MT == 1 ? 4 : 2)><<<grid, 256, 0, stream>>>(out, ldc, (const bf16_t*)A, lda, (const bf16_t*)W, \
-                                                               bias, b_is_f32, M, N, K, k_per_split, part_stride, rope, tickets, norm)
-#define BY_MT(EPI)                                                   \
-  switch (mt) {                                                      \
-    case 1: if (rt == 2) { LAUNCH(1, 2, EPI); } else { LAUNCH(1, 1, EPI); } break; \
-    case 2: LAUNCH(2, 2, EPI); break;                                \
-    case 3: LAUNCH(3, 2, EPI); break;                                \
-    default: LAUNCH(4, 2, EPI); break;                               \
+  dim3 grid((N + 31) / 32, splits);
+  // two k steps of loads in flight per wavefront: deeper prefetch costs registers and measured slower
+#define LAUNCH(MT, EPI)                                                                                      \
+  gemm_skinny_kernel<MT, 2, EPI, 2><<<grid, 256, 0, stream>>>(out, ldc, (const bf16_t*)A, lda, (const bf16_t*)W, \
+                                                              bias, b_is_f32, M, N, K, k_per_split, part_stride, rope, tickets, norm)
+#define BY_MT(EPI)                 \
+  switch (mt) {                    \
+    case 2: LAUNCH(2, EPI); break; \
+    case 3: LAUNCH(3, EPI); break; \
+    default: LAUNCH(4, EPI); break; \
   }
   switch (epilogue) {
     case EPI_BF16: BY_MT(EPI_BF16); break;
@@ -555,7 +517,7 @@ static int launch_skinny(int epilogue, void* out, int64_t ldc, const void* A, in
 // by its root mean square; row_stats[m][0 .. row_stat_tiles) add up to sum(x^2) and the sums of row m
 // are multiplied by rsqrt(that / K + row_eps).  Epilogue 4 adds the sums into the float32 `out`
 // (the residual) in place and leaves bfloat16(out * next_w) in next_rows and the shares of the new
-// rows' sums of squares in next_stats[M][(N + 15) / 16].
+// rows' sums of squares in next_stats[M][next_stat_tiles]: (N + 15) / 16 of 16 columns each, or twice as many of 8.
 // Several k ranges with an epilogue other than float32 partial sums are added up inside the kernel:
 // ticket_parts is scratch of pae_skinny_ticket_floats(M, N, splits) floats and ticket_counters holds
 // pae_skinny_ticket_slots(M, N) ints that are zero before the call and zero after it.  Launches that
@@ -565,9 +527,10 @@ extern "C" int pae_gemm_skinny(int epilogue, void* out, int64_t ldc, const void*
                                int64_t part_stride, float* ticket_parts, int* ticket_counters,
                                const float* row_stats, int row_stat_tiles, float row_eps, void* next_rows,
                                int64_t ld_next, const void* next_w, int next_w_is_f32, float* next_stats,
-                               hipStream_t stream) {
+                               int next_stat_tiles, hipStream_t stream) {
   PAE_REQUIRE(epilogue != EPI_ROPE, "gemm_skinny: the rotating epilogue has an entry point of its own");
-  const SkinnyNorm norm{row_stats, row_stat_tiles, row_eps, (bf16_t*)next_rows, ld_next, next_w, next_w_is_f32, 0, next_stats};
+  const SkinnyNorm norm{row_stats, row_stat_tiles, row_eps, (bf16_t*)next_rows, ld_next, next_w, next_w_is_f32, 0, next_stats,
+                        next_stat_tiles};
   return launch_skinny(epilogue, out, ldc, A, lda, W, bias, b_is_f32, M, N, K, splits, part_stride, SkinnyRope{},
                        SkinnyTickets{ticket_parts, ticket_counters}, norm, stream);
 }
@@ -578,7 +541,7 @@ extern "C" int pae_gemm_skinny_act(void* out, int64_t ldc, const void* A, int64_
                                    int b_is_f32, int M, int N, int K, int splits, float* ticket_parts,
                                    int* ticket_counters, int act, hipStream_t stream) {
   PAE_REQUIRE(act >= 0 && act <= PAE_LAST_ACTIVATION, "gemm_skinny_act: unknown activation %d", act);
-  const SkinnyNorm norm{nullptr, 0, 0.f, nullptr, 0, nullptr, 0, act + 1, nullptr};
+  const SkinnyNorm norm{nullptr, 0, 0.f, nullptr, 0, nullptr, 0, act + 1, nullptr, 0};
   return launch_skinny(EPI_BF16, out, ldc, A, lda, W, bias, b_is_f32, M, N, K, splits, 0, SkinnyRope{},
                        SkinnyTickets{ticket_parts, ticket_counters}, norm, stream);
 }
@@ -589,7 +552,7 @@ extern "C" int pae_gemm_skinny_gated(void* out, int64_t ldc, const void* A, int6
                                      int splits, float* ticket_parts, int* ticket_counters, int act, hipStream_t stream) {
   PAE_REQUIRE(act >= 0 && act <= PAE_LAST_ACTIVATION, "gemm_skinny_gated: unknown activation %d", act);
   PAE_REQUIRE(N % 16 == 0 && ldc % 4 == 0, "gemm_skinny_gated: gated epilogue needs N %% 16 == 0, got %d", N);
-  const SkinnyNorm norm{nullptr, 0, 0.f, nullptr, 0, nullptr, 0, act + 1, nullptr};
+  const SkinnyNorm norm{nullptr, 0, 0.f, nullptr, 0, nullptr, 0, act + 1, nullptr, 0};
   return launch_skinny(EPI_SWIGLU, out, ldc, A, lda, W, nullptr, 0, M, N, K, splits, 0, SkinnyRope{},
                        SkinnyTickets{ticket_parts, ticket_counters}, norm, stream);
 }
@@ -626,7 +589,7 @@ extern "C" int pae_gemm_skinny_rope(void* q_out, int64_t ldq, const void* A, int
               "gemm_skinny_rope: the cache write needs tables and pools");
   SkinnyRope rope{cos_sin, positions, tok_seq, block_tables, (bf16_t*)k_cache, (bf16_t*)v_cache,
                   nh, nkv, hd, rot, max_blocks, bs};
-  const SkinnyNorm norm{row_stats, row_stat_tiles, row_eps, nullptr, 0, nullptr, 0, 0, nullptr};
+  const SkinnyNorm norm{row_stats, row_stat_tiles, row_eps, nullptr, 0, nullptr, 0, 0, nullptr, 0};
   return launch_skinny(EPI_ROPE, q_out, ldq, A, lda, W, bias, b_is_f32, M, (nh + 2 * nkv) * hd, K, splits, 0, rope,
                        SkinnyTickets{ticket_parts, ticket_counters}, norm, stream);
 }

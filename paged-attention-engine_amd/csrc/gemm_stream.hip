@@ -144,7 +144,7 @@ __global__ __launch_bounds__(512, 4) void gemm_stream_kernel(StreamProduct p) {
   void* out = (EPI == EPI_F32 || EPI == EPI_RESIDUAL) ? (void*)((float*)p.out + m0 * p.ldc) : (void*)((bf16_t*)p.out + m0 * p.ldc);
   if (EPI == EPI_RESIDUAL) {
     p.norm.next_rows += m0 * p.norm.ld_next;
-    p.norm.next_stats += (int64_t)m0 * ((p.N + 15) / 16);
+    p.norm.next_stats += (int64_t)m0 * p.norm.next_stat_tiles;
   }
   if (EPI == EPI_ROPE) {
     p.rope.positions += m0;

@@ -22,7 +22,8 @@ typedef __attribute__((ext_vector_type(4))) short s16x4;
 // Producer (EPI_RESIDUAL, the product that ends a residual branch): the sums of all k ranges are
 // added into the float32 residual in place; the same tile is written again as
 // bfloat16(residual * w_next), the rows the next product multiplies, and the tile's share of every
-// row's sum of squares goes to next_stats[m][16-column tile].
+// row's sum of squares goes to next_stats[m][16-column tile], or its two halves' shares to [m][8-column half]: up to
+// 16 rows a product may be shared out in halves of tiles.
 // Consumer (any epilogue): `row_stats` holds those shares for the rows of A; every lane adds up
 // its row's shares in a fixed order (the same in every workgroup, so all columns of a row get the
 // same scale) and multiplies its sums by rsqrt(total / K + eps) before bias, rotation or gate.
@@ -35,7 +36,8 @@ struct SkinnyNorm {
   const void* next_w;      // [N] weight of the norm that follows
   int next_w_is_f32;
   int act;                 // EPI_BF16: 0, or 1 + the code of an activation (see act_of) that the sums pass before they are rounded
-  float* next_stats;       // [M][(N + 15) / 16]
+  float* next_stats;       // [M][next_stat_tiles]
+  int next_stat_tiles;     // (N + 15) / 16, one share per 16 columns, or twice that, one per 8
 };
 
 // A pointer that a kernel has read from a description in LDS (not taken as a kernel argument) is a
@@ -128,6 +130,29 @@ struct RowShares {
   }
 };
 
+// The sum over 4 or 16 neighbouring lanes in all of them: every lane meets the lane 1, 2, 4 and 8 away (once a quad's lanes agree, the
+// lane at the mirrored place of the eight, or of the sixteen, holds what the one 4, or 8, away does).  Within the vector pipe: a shuffle
+// goes through LDS.
+template <int LANES>
+__device__ __forceinline__ float sum_over(float v) {
+  static_assert(LANES == 4 || LANES == 16, "a quad or a row of lanes");
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, true));
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, true));
+  if (LANES == 4) return v;
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xf, 0xf, true));
+  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xf, 0xf, true));
+}
+
+// The number of the lane 32, or 16, away, likewise.
+__device__ __forceinline__ float from_32_away(float v) {
+  const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(threadIdx.x % PAE_WAVE < 32 ? both[1] : both[0]);
+}
+__device__ __forceinline__ float from_16_away(float v) {
+  const auto both = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(threadIdx.x % 32 < 16 ? both[1] : both[0]);
+}
+
 // The scales into s_scale[16 MT] (1 without a folded norm).  Threads t >= 256 do nothing.  The
 // caller puts a workgroup barrier between this and the first read of s_scale.  `before_sum`: called
 // between asking and adding (the place for loads that should be on their way meanwhile).  AT_ONCE:
@@ -154,8 +179,7 @@ __device__ __forceinline__ void row_scales_to_lds(float* s_scale, const SkinnyNo
     more.ask(norm, M, t, base);
     sum = more.add_to(sum);
   }
-#pragma unroll
-  for (int step = 1; step < PER_ROW; step *= 2) sum += __shfl_xor(sum, step);
+  sum = sum_over<PER_ROW>(sum);
   if (t % PER_ROW == 0) s_scale[t / PER_ROW] = rsqrtf(sum / (float)K + norm.eps);
 }
 
@@ -173,7 +197,7 @@ struct SkinnyRope {
 
 __device__ __forceinline__ SkinnyNorm in_memory(const SkinnyNorm& n) {
   return SkinnyNorm{in_memory(n.row_stats), n.row_stat_tiles, n.eps, in_memory(n.next_rows), n.ld_next,
-                    in_memory(n.next_w), n.next_w_is_f32, n.act, in_memory(n.next_stats)};
+                    in_memory(n.next_w), n.next_w_is_f32, n.act, in_memory(n.next_stats), n.next_stat_tiles};
 }
 __device__ __forceinline__ SkinnyRope in_memory(const SkinnyRope& r) {
   return SkinnyRope{in_memory(r.cos_sin), in_memory(r.positions), in_memory(r.tok_seq), in_memory(r.block_tables),
@@ -185,6 +209,22 @@ __device__ __forceinline__ SkinnyRope in_memory(const SkinnyRope& r) {
 // tiles past it hold 16 consecutive features that pass through.
 __device__ __forceinline__ int rope_feature(int j, int r, int rot) {
   return 16 * j < rot ? (r < 8 ? 8 * j + r : rot / 2 + 8 * j + r - 8) : 16 * j + r;
+}
+
+// Products of up to 16 rows (gemm_rows_kernel.h, which says why): a fragment of weights or activations is four rows by the 16 pieces of 16
+// bytes of a 128-wide k step, multiplied as it was loaded.  A lane's row of the four, and its piece:
+__device__ __forceinline__ int piece_row(int lane) { return lane % 16 / 4; }
+__device__ __forceinline__ int piece_of(int lane) { return lane % 4 + 4 * (lane / 16); }
+
+template <int FROM>
+__device__ __forceinline__ float of_quad_lane(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), FROM * 0x55, 0xf, 0xf, true));
+}
+// In the first lane of every quad: the sum over the parts of k (part p: pieces p, p + 4, p + 8, p + 12), in order.  A lane holds column
+// (row of A, part) = lane % 16 and, in register i, line (weight row lane / 16, part i) of the 16 x 16 tile; equal parts, which alone
+// mean something, stand in register p of the quad's lane p.
+__device__ __forceinline__ float sum_of_parts(f32x4 v) {
+  return ((v[0] + of_quad_lane<1>(v[1])) + of_quad_lane<2>(v[2])) + of_quad_lane<3>(v[3]);
 }
 
 // A fragment loaded as (row = lane / 4, k group = lane % 4) moved to (row = lane % 16, k group = lane / 16).
@@ -253,14 +293,14 @@ __device__ __forceinline__ void ask_row(EpilogueAhead<RT>& pre, int M, const Ski
   }
 }
 
-// (after ask_row)
+// (after ask_row; `live`: see skinny_epilogue)
 template <int RT, int EPI, bool THROUGH>
 __device__ __forceinline__ void ask_epilogue(EpilogueAhead<RT>& pre, int tile_base, const void* out, int64_t ldc,
-                                             int M, int N, const SkinnyRope& rope, const SkinnyNorm& norm) {
+                                             int M, int N, const SkinnyRope& rope, const SkinnyNorm& norm, bool live = true) {
   const int lane = threadIdx.x % PAE_WAVE;
   const int r = lane % 16, g4 = lane / 16;
   const int mc = r < M ? r : M - 1;
-  if (EPI == EPI_RESIDUAL) {
+  if (EPI == EPI_RESIDUAL && live) {
     const float* res = (const float*)out + (int64_t)mc * ldc;
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
@@ -305,13 +345,16 @@ __device__ __forceinline__ void ask_epilogue(EpilogueAhead<RT>& pre, int tile_ba
 // What a wavefront does with finished sums: acc[rt][mt] is the 16 x 16 tile of weight rows
 // 16 (tile_base + rt) .. (through the rotation's row order, if any) by rows 16 mt .. of A; a lane
 // holds row m = 16 mt + lane % 16 of A and weight rows 4 (lane / 16) + i.  only_mt >= 0: just
-// that column tile (the others belong to other wavefronts).
+// that column tile (the others belong to other wavefronts).  `live`: false in lanes whose weight rows are another
+// workgroup's, where a tile is shared out in halves (rows 0-3 and 8-11 against the others for the gate and the rotation, which join row r
+// with row r + 8; rows 0-7 against 8-15 for the rest).
 template <int MT, int RT, int EPI, bool THROUGH = false>
 __device__ __forceinline__ void skinny_epilogue(const f32x4 (&acc)[RT][MT], int tile_base, int only_mt,
                                                 void* __restrict__ out, int64_t ldc, const void* __restrict__ bias,
                                                 int b_is_f32, int M, int N, int split, int64_t part_stride,
                                                 const SkinnyRope& rope, const SkinnyNorm& norm,
-                                                const float (&scale)[MT], const EpilogueAhead<RT>* pre = nullptr) {
+                                                const float (&scale)[MT], const EpilogueAhead<RT>* pre = nullptr,
+                                                bool live = true) {
   const int lane = threadIdx.x % PAE_WAVE;
   const int r = lane % 16, g4 = lane / 16;
   if (EPI == EPI_ROPE) {
@@ -338,7 +381,7 @@ __device__ __forceinline__ void skinny_epilogue(const f32x4 (&acc)[RT][MT], int 
           // the projection is rounded to bfloat16 before the rotation, as where the two are separate kernels
           const float own = __bfloat162float(__float2bfloat16(
               acc[rt][mt][i] * scale[mt] + ((bias && n + i < N) ? load_param(bias, b_is_f32, n + i) : 0.f)));
-          const float other = __shfl_xor(own, 32);  // in every lane
+          const float other = from_32_away(own);  // in every lane
           float o = own;
           if (rotated) {
             const float* angle = rope.cos_sin + ((int64_t)mc * (rope.rot / 2) + 8 * j + (4 * g4 + i) % 8) * 2;
@@ -347,7 +390,7 @@ __device__ __forceinline__ void skinny_epilogue(const f32x4 (&acc)[RT][MT], int 
           }
           res[i] = to_bf16_bits(o);
         }
-        if (m >= M || n >= N) continue;
+        if (m >= M || n >= N || !live) continue;
         if (head < rope.nh) {
           put<THROUGH>(reinterpret_cast<s16x4*>((bf16_t*)out + (int64_t)m * ldc + n), res);
           continue;
@@ -385,11 +428,11 @@ __device__ __forceinline__ void skinny_epilogue(const f32x4 (&acc)[RT][MT], int 
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const float own = acc[rt][mt][i] * scale[mt];
-          const float up = __shfl_xor(own, 32);  // in every lane (the same row of A, so the same scale)
+          const float up = from_32_away(own);  // in every lane (the same row of A, so the same scale)
           // the gate's activation: SiLU, or the one the caller named (1 + its code, see act_of)
           v[i] = to_bf16_bits((norm.act ? act_of(own, norm.act - 1) : own / (1.0f + expf(-own))) * up);
         }
-        if (g4 < 2 && j < N / 2)  // N counts gate and up rows
+        if (g4 < 2 && j < N / 2 && live)  // N counts gate and up rows
           put<THROUGH>(reinterpret_cast<s16x4*>((bf16_t*)out + (int64_t)m * ldc + j), v);
       }
     } else if (EPI == EPI_RESIDUAL) {
@@ -399,7 +442,7 @@ __device__ __forceinline__ void skinny_epilogue(const f32x4 (&acc)[RT][MT], int 
       for (int rt = 0; rt < RT; ++rt) {
         const int n = 16 * (tile_base + rt) + 4 * g4;
         float ss = 0.f;
-        if (n < N) {
+        if (n < N && live) {
           float v[4];
           s16x4 p;
 #pragma unroll
@@ -420,16 +463,20 @@ __device__ __forceinline__ void skinny_epilogue(const f32x4 (&acc)[RT][MT], int 
             }
           }
         }
-        ss += __shfl_xor(ss, 16);  // the four lanes that hold this row's 16 columns
-        ss += __shfl_xor(ss, 32);
-        if (g4 == 0 && 16 * (tile_base + rt) < N)
-          put<THROUGH>(norm.next_stats + (int64_t)m * ((N + 15) / 16) + tile_base + rt, ss);
+        ss += from_16_away(ss);  // the four lanes that hold this row's 16 columns, two to a half
+        float* shares = norm.next_stats + (int64_t)m * norm.next_stat_tiles;
+        if (norm.next_stat_tiles > (N + 15) / 16) {
+          if (g4 % 2 == 0 && live && 16 * (tile_base + rt) < N) put<THROUGH>(shares + 2 * (tile_base + rt) + g4 / 2, ss);
+        } else {
+          ss += from_32_away(ss);
+          if (g4 == 0 && 16 * (tile_base + rt) < N) put<THROUGH>(shares + tile_base + rt, ss);
+        }
       }
     } else {
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) {
         const int n = 16 * (tile_base + rt) + 4 * g4;
-        if (n >= N) continue;
+        if (n >= N || !live) continue;
         float v[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i)

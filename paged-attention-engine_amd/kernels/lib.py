@@ -63,7 +63,7 @@ def _declare(lib) -> None:
         "pae_rope_table": [P, P, P, I, I, P],
         "pae_rope_kv_write": [I, P, L, I, I, I, I, I, P, I, P, P, P, P, I, I, P, P, I, P],
         "pae_swiglu": [I, P, P, I, I, I, P],
-        "pae_gemm_skinny": [I, P, L, P, L, P, P, I, I, I, I, I, L, P, P, P, I, F, P, L, P, I, P, P],
+        "pae_gemm_skinny": [I, P, L, P, L, P, P, I, I, I, I, I, L, P, P, P, I, F, P, L, P, I, P, I, P],
         "pae_gemm_skinny_rope": [P, L, P, L, P, P, I, I, I, I, I, I, I, P, P, P, P, I, I, P, P, I, P, P, P, I, F, P],
         "pae_gemm_wide_plan": [I, I, I, I, I, I],
         "pae_gemm_wide": [I, I, I, P, L, P, L, P, P, I, I, I, I, P],
@@ -147,7 +147,7 @@ def _declare(lib) -> None:
         "pae_program_barrier_bytes": [],
         "pae_program_max_rows": [],
         "pae_program_max_groups": [],
-        "pae_program_put_product": [P, I, I, P, L, P, L, P, P, I, I, I, I, I, P, P, P, I, F, P, L, P, I, P, P],
+        "pae_program_put_product": [P, I, I, P, L, P, L, P, P, I, I, I, I, I, P, P, P, I, F, P, L, P, I, P, I, P],
         "pae_program_put_product_rope": [P, I, P, L, P, L, P, P, I, I, I, I, I, I, I, P, P, P, P, I, I, P, P, I, P, P, P,
                                          I, F],
         "pae_program_put_attention": [P, I, P, L, P, L, P, P, P, I, P, I, I, I, I, I, F, I, P, P],
@@ -600,6 +600,13 @@ def stat_tiles(width: int) -> int:
     return -(-width // 16)
 
 
+def fine_stat_tiles(width: int, rows: int = 1) -> int:
+    """The same in halves, one per 8 columns, which products that add themselves into the residual may be asked for: with up to 16
+    rows their workgroups may then take 8 weight rows each.  Wider and more rows keep one per 16: their workgroups are many, and every
+    workgroup of the product behind reads all rows' shares (64 rows of 1,536 in shares of 8: 2,160 -> 2,283 us a step)."""
+    return 2 * stat_tiles(width) if width <= 3072 and rows <= SAME_ORDER_MAX_ROWS else stat_tiles(width)
+
+
 def _row_scale(row_scale, M: int, K: int):
     """(pointer, tiles, eps) of the shares of the rows' sums of squares, for a product whose rows
     are still to be divided by their root mean square; (None, 0, 0) for plain rows."""
@@ -607,7 +614,7 @@ def _row_scale(row_scale, M: int, K: int):
         return None, 0, 0.0
     stats, eps = row_scale
     assert stats.is_cuda and stats.dtype == torch.float32 and stats.is_contiguous()
-    assert stats.dim() == 2 and stats.shape[0] >= M and stats.shape[1] == stat_tiles(K)
+    assert stats.dim() == 2 and stats.shape[0] >= M and stats.shape[1] in (stat_tiles(K), fine_stat_tiles(K))
     return stats.data_ptr(), stats.shape[1], float(eps)
 
 
@@ -636,7 +643,8 @@ def scaled_rows(rows: torch.Tensor, stats: torch.Tensor, eps: float) -> torch.Te
     _gpu(rows, stats)
     M, H = rows.shape
     assert rows.dtype == torch.bfloat16 and rows.is_contiguous()
-    assert stats.dtype == torch.float32 and stats.shape == (M, stat_tiles(H)) and stats.is_contiguous()
+    assert stats.dtype == torch.float32 and stats.is_contiguous()
+    assert tuple(stats.shape) in ((M, stat_tiles(H)), (M, fine_stat_tiles(H)))
     out = torch.empty_like(rows)
     _check(library().pae_scaled_rows(out.data_ptr(), rows.data_ptr(), stats.data_ptr(), stats.shape[1], float(eps),
                                      M, H, _stream()))
@@ -650,8 +658,8 @@ def skinny_supported(a: torch.Tensor, w: torch.Tensor) -> bool:
 
 
 def skinny_splits(N: int, K: int, M: int = 1, w: Optional[torch.Tensor] = None) -> int:
-    """k ranges for a product whose consumer adds float32 partials: enough workgroups to fill the
-    chip (a workgroup takes 16 weight rows, or 32 and more with more than 8 rows of activations).
+    """k ranges for a product whose consumer adds float32 partials: one up to 16 rows (1.5B down with the norm behind it
+    at 8 rows in five ranges 8.7 + 4.1 us, in one 9.4 + 3.3), beyond that enough workgroups to fill the chip.
     `w`: the weights, where they are at hand (see `_streamed_splits`)."""
     return _skinny_splits(N, K, M, _off_16_bytes(w))
 
@@ -667,45 +675,38 @@ _rule_of_sizes = functools.lru_cache(maxsize=4096)
 
 @_rule_of_sizes
 def _skinny_splits(N: int, K: int, M: int, off: bool) -> int:
+    if M <= SAME_ORDER_MAX_ROWS:
+        return 1
     return _streamed_splits(N, K, M, _part_ranges(N, K, M), off, parts=True)
 
 
 def _part_ranges(N: int, K: int, M: int) -> int:
-    """The ranges of `skinny_splits` in the kernels that do not stream."""
-    rows = 32 if M > 8 else 16
-    tiles = -(-N // rows)
-    # (ranges of at least 1,024 of k: the 0.5B sizes at 8 rows, O 5.3 us in three ranges and 3.9 in one, down
-    # 8.0 us in eight and 7.4 in four)
-    wanted = max(1, min(512 // tiles, K // 1024, 8))
-    if M <= 8 and tiles >= 200 and tiles * wanted < 640 and K >= 4096:
-        # one or two workgroups per compute unit, each with a long way to go (14B down at 8 rows:
-        # 320 workgroups over 13,824 of k take 48 us with the norm, three ranges 35 us)
-        wanted = min(8, -(-960 // tiles))
-    if M > 8:
-        # every range costs its partial sums a trip to memory and back in the norm that adds them, so a
-        # workgroup wants about 128 KB of weights before another range pays (with the norm, at 64 rows:
-        # 1.5B O one range 9.8 us, six 11.5; 1.5B down four 21.0, eight 22.9; 7B O two 18.2, four 19.8)
-        wanted = max(1, min(8, round(rows * K * 2 / 131072)))
-        # enough ranges of at least 1024 for the many-weight-rows kernel (128 rows a workgroup) to fill
-        # the chip twice, where that many exist (72B down at 64 rows: 2 ranges 177 us, 8 ranges 115 us)
-        groups = -(-N // 128)
-        many = min(12, -(-512 // groups))
-        while many > 1 and K // many < 1024:
-            many -= 1
-        if groups * many >= 256:
-            wanted = max(wanted, many)
-        # or fewer, longer ranges for that kernel's 64-row workgroups, where those fill the chip and the
-        # 128-row ones do not (7B down at 48 rows: 12 ranges 47 us, 8 ranges of 64-row workgroups 42 us)
-        # (ranges down to 768 of k: 14B/32B O, 5,120 x 5,120, at 24 / 64 rows from HBM with the norm: two ranges
-        # 28.2 / 38.0 us, six 22.7 / 27.6)
-        fewer = -(-448 // -(-N // 64))
-        if fewer <= 8 and K // fewer >= 768 and groups * fewer < 256:
-            wanted = fewer
-        # or, with few weight rows, as many ranges as make one round of 32-row workgroups over the chip (3B
-        # down, 64 x 4: 19.9 / 23.7 us with the norm against 23.1 / 29.0 with five ranges; 1.5B down, 48 x 5)
-        one_round = _compute_units() // -(-N // 32)
-        if M > SAME_ORDER_MAX_ROWS and 4 <= one_round <= 8 and K // one_round >= 1024:
-            wanted = one_round
+    """The ranges of `skinny_splits` for more than 16 rows in the kernels that do not stream."""
+    rows = 32
+    # every range costs its partial sums a trip to memory and back in the norm that adds them, so a
+    # workgroup wants about 128 KB of weights before another range pays (with the norm, at 64 rows:
+    # 1.5B O one range 9.8 us, six 11.5; 1.5B down four 21.0, eight 22.9; 7B O two 18.2, four 19.8)
+    wanted = max(1, min(8, round(rows * K * 2 / 131072)))
+    # enough ranges of at least 1024 for the many-weight-rows kernel (128 rows a workgroup) to fill
+    # the chip twice, where that many exist (72B down at 64 rows: 2 ranges 177 us, 8 ranges 115 us)
+    groups = -(-N // 128)
+    many = min(12, -(-512 // groups))
+    while many > 1 and K // many < 1024:
+        many -= 1
+    if groups * many >= 256:
+        wanted = max(wanted, many)
+    # or fewer, longer ranges for that kernel's 64-row workgroups, where those fill the chip and the
+    # 128-row ones do not (7B down at 48 rows: 12 ranges 47 us, 8 ranges of 64-row workgroups 42 us)
+    # (ranges down to 768 of k: 14B/32B O, 5,120 x 5,120, at 24 / 64 rows from HBM with the norm: two ranges
+    # 28.2 / 38.0 us, six 22.7 / 27.6)
+    fewer = -(-448 // -(-N // 64))
+    if fewer <= 8 and K // fewer >= 768 and groups * fewer < 256:
+        wanted = fewer
+    # or, with few weight rows, as many ranges as make one round of 32-row workgroups over the chip (3B
+    # down, 64 x 4: 19.9 / 23.7 us with the norm against 23.1 / 29.0 with five ranges; 1.5B down, 48 x 5)
+    one_round = _compute_units() // -(-N // 32)
+    if 4 <= one_round <= 8 and K // one_round >= 1024:
+        wanted = one_round
     k_per = -(-(-(-K // wanted)) // 128) * 128
     return -(-K // k_per)
 
@@ -733,11 +734,10 @@ def _compute_units() -> int:
 def residual_splits(N: int, K: int, M: int = 1, w: Optional[torch.Tensor] = None) -> int:
     """k ranges for a product that adds itself into the residual (EPI_RESIDUAL).  Up to 16 rows from
     the product's sizes alone: a row's sums are the same bits whatever it is batched with, launched by
-    itself or as a phase of a decode program.  Four ranges run side by side in one workgroup of sixteen
-    wavefronts, with no tickets and no trip to memory for partial sums, and are ahead wherever the 16-row
-    workgroups fill the chip or have little to read (1.5B O at 8 rows 7.2 -> 5.9 us, 7B down 38.3 -> 36.1
-    us, 72B down 111 -> 107.5 us); a few workgroups with much to read each want ticketed ranges (1.5B
-    down: 96 workgroups of 287 KB, 17.4 us in one workgroup each, 12.5 in five ranges)."""
+    itself or as a phase of a decode program.  Two or four ranges run side by side in one workgroup of eight or sixteen
+    wavefronts, with no tickets and no trip to memory for partial sums: what a workgroup of few weight rows and much of k has to
+    read then comes to more wavefronts (1.5B down at 1 / 8 / 16 rows in one range 7.4 / 8.7 / 11.9 us, in four 6.9 / 8.8 / 10.6;
+    7B down 24.9 / 30.4 / 41.5, in two 24.9 / 25.2 / 31.7, in four 24.5 / 26.6 / 37.1; sums alone)."""
     return _residual_splits(N, K, M, _off_16_bytes(w))
 
 
@@ -755,19 +755,8 @@ def _residual_splits(N: int, K: int, M: int, off: bool) -> int:
         # 21.8 / 28.4 with five; 7B down: eight, 35 / 47 us; 14B: six, 33 / 44; 14B O: six, 19 / 27 against 27 / 37
         # with two)
         return _streamed_splits(N, K, M, _part_ranges(N, K, M), off)
-    tiles = -(-N // 16)
-    # one such workgroup fills a compute unit, so the tiles should fill the chip's units a whole number of
-    # times, or nearly (14B/32B down: 320 tiles are a full round and a quarter of one; 32B at 8 rows 86.7 us
-    # side by side, ticketed ranges are ahead)
-    units = _compute_units()
-    rounds_full = tiles <= units or tiles % units == 0 or tiles % units >= 3 * units // 4
-    if K >= 1024 and (tiles >= 192 or 32 * K <= 65536) and rounds_full:
-        return -(-K // (-(-(-(-K // 4)) // 128) * 128))  # four, as the rounding to 128 leaves them
-    splits = _part_ranges(N, K, 1)
-    if splits == 4 and K >= 1024 and (tiles >= 192 or 32 * K <= 65536):
-        # four would be taken side by side (the same sums, slower here)
-        return 5 if K // 5 >= 256 else 3
-    return splits  # (four ticketed ranges where the launcher keeps them apart: 3B down at 8 rows 14.7 us, five 16.5)
+    wanted = 4 if N <= 3072 and K >= 4096 else 2 if N <= 4096 and K >= 512 else 1
+    return -(-K // (-(-(-(-K // wanted)) // 128) * 128))
 
 
 def gemm_skinny(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
@@ -784,13 +773,13 @@ def gemm_skinny(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, bias: Optio
     and row m's sums are multiplied by rsqrt(that / K + eps) before the epilogue.
     EPI_RESIDUAL: `out` is the float32 residual [M, N], to which the product is added in place;
     `following = (next_rows, next_w, next_stats)` receives bfloat16(out * next_w) [M, N] and the
-    shares [M, stat_tiles(N)] of the new rows' sums of squares, for the product after the next norm."""
+    shares [M, stat_tiles(N)] or [M, fine_stat_tiles(N)] of the new rows' sums of squares, for the product after the next norm."""
     _gpu(out, a, w, bias)
     M, K_ = a.shape
     N = w.shape[0]
     assert skinny_supported(a, w) and w.shape == (N, K_) and w.is_contiguous() and out.is_contiguous()
     nr = nw = ns = None
-    nwf, ld_next = 0, 0
+    nwf, ld_next, nst = 0, 0, 0
     if epilogue == EPI_SWIGLU:
         assert out.shape == (M, N // 2) and out.dtype == torch.bfloat16 and bias is None
     elif epilogue == EPI_F32:
@@ -801,9 +790,10 @@ def gemm_skinny(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, bias: Optio
         next_rows, next_w, next_stats = following
         _gpu(next_rows, next_w, next_stats)
         assert next_rows.dtype == torch.bfloat16 and next_rows.shape == (M, N) and next_rows.stride(1) == 1
-        assert next_stats.dtype == torch.float32 and next_stats.shape == (M, stat_tiles(N)) and next_stats.is_contiguous()
+        assert next_stats.dtype == torch.float32 and next_stats.is_contiguous()
+        assert tuple(next_stats.shape) in ((M, stat_tiles(N)), (M, fine_stat_tiles(N)))
         assert next_w.numel() == N
-        nr, ns, ld_next = next_rows.data_ptr(), next_stats.data_ptr(), next_rows.stride(0)
+        nr, ns, ld_next, nst = next_rows.data_ptr(), next_stats.data_ptr(), next_rows.stride(0), next_stats.shape[1]
         nw, nwf = _param(next_w)
     else:
         assert out.shape == (M, N) and out.dtype == torch.bfloat16
@@ -814,14 +804,14 @@ def gemm_skinny(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, bias: Optio
         _RECORDING.add(library().pae_program_put_product(
             _RECORDING.host_ptr, _RECORDING.count, epilogue, out.data_ptr(), out.stride(-2), a.data_ptr(), a.stride(0),
             w.data_ptr(), bp, bf, M, N, K_, splits, _ptr(parts), _ptr(counters), sp, st, se, nr, ld_next, nw, nwf, ns,
-            None), out, a, w, bias, parts, row_scale, following,
+            nst, None), out, a, w, bias, parts, row_scale, following,
             activation_bytes=library().pae_program_activation_bytes(M, K_, splits))
         return
     checking = (parts is not None and CHECK_TICKET_SUMS and not torch.cuda.is_current_stream_capturing())
     before = out.clone() if checking and epilogue == EPI_RESIDUAL else None
     _launch_ticketed(counters, lambda: library().pae_gemm_skinny(
         epilogue, out.data_ptr(), out.stride(-2), a.data_ptr(), a.stride(0), w.data_ptr(), bp, bf, M, N, K_, splits,
-        M * N, _ptr(parts), _ptr(counters), sp, st, se, nr, ld_next, nw, nwf, ns, _stream()))
+        M * N, _ptr(parts), _ptr(counters), sp, st, se, nr, ld_next, nw, nwf, ns, nst, _stream()))
     if checking:
         _check_ticket_sums(out, before, a, w, bias, epilogue, splits, row_scale, following)
 

@@ -104,7 +104,7 @@ class Linear:
                     and residual.is_contiguous() and tuple(residual.shape) == (x.shape[0], self.out_features)):
                 weight, eps = fold
                 rows = torch.empty((x.shape[0], self.out_features), dtype=torch.bfloat16, device=x.device)
-                stats = torch.empty((x.shape[0], K.stat_tiles(self.out_features)), dtype=torch.float32, device=x.device)
+                stats = torch.empty((x.shape[0], K.fine_stat_tiles(self.out_features, x.shape[0])), dtype=torch.float32, device=x.device)
                 K.gemm_skinny(residual, x, self.weight, None, K.EPI_RESIDUAL,
                               K.residual_splits(self.out_features, self.in_features, x.shape[0], self.weight),
                               following=(rows, weight, stats))
