@@ -17,6 +17,8 @@
 //                      first token to its last; the lanes of a group share out the D rows.
 //   delta_gated_norm   o / sqrt(mean_V(o^2) + eps) * w * silu(gate), rounded to the activation type.
 //
+// A step of single tokens does all four in one launch, with the same bits (recurrent_tokens.hip).
+//
 // For designs that have them, each switched by a parameter: a decay per head and key channel instead of one
 // per head (`channel_decay`: the decay's input and dt_bias are then H x D wide and row d of a head's S is
 // multiplied by its own number); beta, the decay's input and the gate read from rows of their own instead of
@@ -30,9 +32,7 @@
 // prompt was cut into steps or on what else the step holds.
 #include "common.h"
 #include "api.h"
-
-__device__ __forceinline__ float silu_f(float z) { return z / (1.0f + expf(-z)); }
-__device__ __forceinline__ float softplus_f(float z) { return z > 20.f ? z : log1pf(expf(z)); }
+#include "recurrent_tokens.h"
 
 // seq_runs[s] = (first flat row, rows in this step, tokens held before the step, unused)
 // One workgroup of 128 threads per (token, segment): segments 0 .. G-1 are the q heads, G .. 2G-1 the
@@ -194,21 +194,12 @@ __global__ __launch_bounds__(256) void delta_recurrence_kernel(
 // bounds it now is the issue of a step's 52 vector instructions by the one wavefront a SIMD has.  Measured, 12 heads
 // of 128 x 128: 2,048 tokens of one sequence 544 -> 307 us (the same bits).
 //
-// Steps in which no run can hold a whole chunk (decoding) have a kernel without the unrolled part (WHOLE off): that takes 130 to 148
+// Steps in which no run can hold a whole chunk have a kernel without the unrolled part (WHOLE off): that takes 130 to 148
 // registers where the loop by tokens takes 75 to 90, and with many sequences, whose states' way from memory and back is the
 // time, wavefronts are then missing (the whole delta step for 64 sequences of one token 48.8 us with it, 43.0 without; with 28 heads
 // 91 and 75).  The host knows a step's tokens and sequences, not its longest run: many runs of 3 to 15 tokens side by side pay for the
 // chunk that none of them fills (64 of three 46 -> 55 us).  Unrolling two or four tokens at a time takes 111 to 130
 // registers and half of what a long run gains (2,048 tokens 352 us all 16, 434 four, 442 two, 611 before).
-template <int L>
-__device__ __forceinline__ float group_sum(float v) {
-  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xB1, 0xF, 0xF, true));  // lanes (1, 0, 3, 2) of a quad
-  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4E, 0xF, 0xF, true));  // lanes (2, 3, 0, 1)
-  if (L >= 8) v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x141, 0xF, 0xF, true));   // 8 lanes mirrored
-  if (L >= 16) v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x140, 0xF, 0xF, true));  // 16 lanes mirrored
-  return v;
-}
-
 template <int R, int L, int CH, bool CHANNEL, bool DELTA, bool WHOLE>
 __global__ __launch_bounds__(16 * L) void delta_recurrence_group_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v, const float* __restrict__ beta,
@@ -510,6 +501,13 @@ extern "C" int pae_delta_rule_step(int dtype, const void* proj, int64_t row_stri
   PAE_REQUIRE(gate_in && b_in && a_in, "delta rule: the gate's, beta's and the decay's rows are needed");
   PAE_REQUIRE(dtype == PAE_F32 || dtype == PAE_BF16, "delta rule: unknown dtype code %d", dtype);
   if (num_tokens <= 0 || num_seqs <= 0) return 0;
+  if (takes_tokens_step(num_tokens, num_seqs, G, H, D, V, state, state_slot_stride)) {
+    const TokensStep p = {proj, row_stride, (const int4*)seq_runs, slots, state, state_slot_stride, G, H, D, V, a_in, a_stride,
+                          gate_in, gate_stride, gate_sigmoid, norm_w, w_is_f32, norm_eps, out, conv_w, conv_tail, tail_slot_stride, taps,
+                          a_log, dt_bias, unit_eps, b_in, b_stride, nullptr, 0, 0.f};
+    launch_tokens_step(channel_decay ? TOKENS_CHANNEL_DELTA : TOKENS_DELTA, dtype, p, num_seqs, stream);
+    return pae_check_launch("delta_rule_step (single tokens)");
+  }
   // work: q [T][G][D], k [T][G][D], v [T][H][V], beta [T][H], decay [T][H] or [T][H][D], o [T][H][V]
   // (every part starts on a 16-byte boundary: the recurrence reads k, q and channel decays four at a time)
   float* q = work;

@@ -15,13 +15,15 @@
 //   read-before-write: a column of S stays in the registers of a group of lanes over the whole step
 //   the delta rule's gated norm
 //
-// Steps whose runs are long on average go by chunks of 16 tokens instead of the first two (see below).
+// Steps whose runs are long on average go by chunks of 16 tokens instead of the first two (see below); a step of single tokens does
+// all three in one launch, with the same bits (recurrent_tokens.hip).
 //
 // Everything but the projected rows, z and the gate's rows is float32: the decay and its logarithm, the state,
 // the read-out and the norm.  Token by token the order in which a column's sums are formed depends on D alone; by chunks it
 // depends on where in its run a token stands, and which of the two is taken on the step.
 #include "common.h"
 #include "api.h"
+#include "recurrent_tokens.h"
 
 void pae_launch_recurrence(const float* q, const float* k, const float* v, const float* beta, const float* decay,
                            const int4* runs, const int* slots, float* state, int64_t state_slot_stride, int G, int H,
@@ -29,8 +31,6 @@ void pae_launch_recurrence(const float* q, const float* k, const float* v, const
 int pae_launch_gated_norm(int dtype, const float* o, const void* gates, int64_t gate_stride, int gate_sigmoid,
                           const void* weight, int w_is_f32, float eps, int num_tokens, int H, int V, void* out,
                           hipStream_t stream);
-
-__device__ __forceinline__ float gla_log_sigmoid(float z) { return fminf(z, 0.f) - log1pf(expf(-fabsf(z))); }
 
 // One workgroup of 128 threads per (token, head).
 template <typename T>
@@ -351,6 +351,13 @@ extern "C" int pae_linear_attention_step(int dtype, const void* proj, int64_t ro
   PAE_REQUIRE(z_in && gate_in, "linear attention: the decay's and the gate's rows are needed");
   PAE_REQUIRE(dtype == PAE_F32 || dtype == PAE_BF16, "linear attention: unknown dtype code %d", dtype);
   if (num_tokens <= 0 || num_seqs <= 0) return 0;
+  if (takes_tokens_step(num_tokens, num_seqs, H, H, D, V, state, state_slot_stride)) {
+    const TokensStep p = {proj, row_stride, (const int4*)seq_runs, slots, state, state_slot_stride, H, H, D, V, z_in, z_stride,
+                          gate_in, gate_stride, gate_sigmoid, norm_w, w_is_f32, norm_eps, out, nullptr, nullptr, 0, 0,
+                          nullptr, nullptr, 0.f, nullptr, 0, z_bias, bias_is_f32, 1.0f / tau};
+    launch_tokens_step(TOKENS_LINEAR, dtype, p, num_seqs, stream);
+    return pae_check_launch("linear_attention_step (single tokens)");
+  }
   // work: q [T][H][D], k [T][H][D], decay [T][H][D], v [T][H][V], ones [T][H] (by chunks: near [T][H][16]), o [T][H][V], each on a
   // 16-byte boundary
   const int64_t T = num_tokens;
