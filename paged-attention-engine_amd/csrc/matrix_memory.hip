@@ -36,6 +36,7 @@
 #define MM_VS 64     // value features of a workgroup in the chunk kernels
 #define MM_STEPS 4   // tokens the serial kernel stages at a time
 #define MM_FEW 16    // tokens the serial gates take at a time
+#define MM_TOKEN_COLUMNS 2  // columns of the memory a lane holds rows of, where a step is single tokens
 
 __device__ __forceinline__ float log_sigmoid_f(float z) { return fminf(z, 0.f) - log1pf(expf(-fabsf(z))); }
 
@@ -50,6 +51,26 @@ struct MemoryGates {
 };
 
 // ---------------------------------------------------------------------------------------------- gates, few tokens
+// One gate's sum of a token, by a wavefront.  wide: rows of whole 16-byte pieces at multiples of 16 bytes.
+template <typename T>
+__device__ __forceinline__ float gate_sum(const T* row, const T* w, int hidden, int wide) {
+  constexpr int VEC = 16 / sizeof(T);
+  struct alignas(16) Chunk { T v[VEC]; };
+  const int lane = threadIdx.x % PAE_WAVE;
+  float z = 0.f;
+  if (wide) {
+    for (int k = lane * VEC; k < hidden; k += PAE_WAVE * VEC) {
+      const Chunk a = *reinterpret_cast<const Chunk*>(row + k);
+      const Chunk b = *reinterpret_cast<const Chunk*>(w + k);
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) z = fmaf(to_f32(a.v[e]), to_f32(b.v[e]), z);
+    }
+  } else {
+    for (int k = lane; k < hidden; k += PAE_WAVE) z = fmaf(to_f32(row[k]), to_f32(w[k]), z);
+  }
+  return wave_sum(z);
+}
+
 // runs[i] = (table row of the sequence, first flat row, rows, unused); one workgroup of four wavefronts per (run, head).
 // Without `gate_logits` the two sums of every token are formed here from the mixer's input: a wavefront a sum.
 template <typename T>
@@ -59,8 +80,6 @@ __global__ __launch_bounds__(256) void memory_gates_few_kernel(const float* __re
                                                                const int4* __restrict__ runs, const int* __restrict__ slots,
                                                                float* __restrict__ maximum, int64_t max_slot_stride, int H,
                                                                float cap, MemoryGates gates) {
-  constexpr int VEC = 16 / sizeof(T);
-  struct alignas(16) Chunk { T v[VEC]; };
   __shared__ float s_log[2][MM_FEW];  // the gates' logarithms: input, forget
   const int4 run = runs[blockIdx.x];
   const int h = blockIdx.y, wave = threadIdx.x / PAE_WAVE, lane = threadIdx.x % PAE_WAVE;
@@ -75,19 +94,7 @@ __global__ __launch_bounds__(256) void memory_gates_few_kernel(const float* __re
       if (gate_logits) {
         z = gate_logits[t * 2 * H + which * H + h];
       } else {
-        const T* row = x + t * ldx;
-        const T* w = gate_w + (int64_t)(which * H + h) * hidden;
-        if (wide) {
-          for (int k = lane * VEC; k < hidden; k += PAE_WAVE * VEC) {
-            const Chunk a = *reinterpret_cast<const Chunk*>(row + k);
-            const Chunk b = *reinterpret_cast<const Chunk*>(w + k);
-#pragma unroll
-            for (int e = 0; e < VEC; ++e) z = fmaf(to_f32(a.v[e]), to_f32(b.v[e]), z);
-          }
-        } else {
-          for (int k = lane; k < hidden; k += PAE_WAVE) z = fmaf(to_f32(row[k]), to_f32(w[k]), z);
-        }
-        z = wave_sum(z) + gate_b[which * H + h];
+        z = gate_sum(x + t * ldx, gate_w + (int64_t)(which * H + h) * hidden, hidden, wide) + gate_b[which * H + h];
       }
       z = cap * tanhf(z / cap);
       if (lane == 0) s_log[which][j] = which ? log_sigmoid_f(z) : z;
@@ -261,6 +268,135 @@ __global__ __launch_bounds__(256) void memory_serial_kernel(const T* __restrict_
         if (d + e < D) column[d + e] = S[r][e];
     }
   }
+}
+
+// ---------------------------------------------------------------------------------------------- single tokens
+// Steps without a run in chunks and with as many runs as tokens (decoding; a run of several beside empty ones is worked on
+// token by token): the gates, the recurrence and what follows it, three launches otherwise, in one.  What bounds such a step is the
+// launches, 5 us each beside 66 KB of state a head each way.  A workgroup of 16 wavefronts takes a (run, head): the first two form the
+// gates' sums, the others bring the token's numbers, the state is asked for before either.  16 lanes share a column as in memory_serial_kernel, a lane
+// holds its rows of two; the column n is held by every group of 16, which so has the divisor itself.  Every sum is formed in the
+// separate kernels' order: the same bits.
+// In a recorded graph, three launches and one, us for 1 / 8 / 64 sequences: 12 heads of 128 by 128 9.2 / 10.2 / 27.8 and 5.6 / 6.2 / 25.6; 28 heads for
+// 1 / 8 / 24 9.5 / 12.8 / 25.8 and 5.6 / 7.8 / 23.3; 14 heads of 64 for 1 / 32 8.9 / 11.8 and 5.2 / 9.4.
+template <typename T, int R>
+__global__ __launch_bounds__(1024) void memory_tokens_kernel(const T* __restrict__ proj, int64_t row_stride, const float* __restrict__ gate_logits,
+                                                             const T* __restrict__ x, int64_t ldx, const T* __restrict__ gate_w,
+                                                             const float* __restrict__ gate_b, int hidden, int wide, const int4* __restrict__ runs,
+                                                             const int* __restrict__ slots, float* __restrict__ state, int64_t slot_stride,
+                                                             float* __restrict__ maximum, int64_t max_slot_stride, int H, int D, int V, float cap,
+                                                             const T* __restrict__ gates, int64_t gate_stride, const void* __restrict__ weight,
+                                                             int w_is_f32, float eps, float floor_eps, int pairs, T* __restrict__ out) {
+  constexpr int DP = R * 64, COLUMNS = MM_TOKEN_COLUMNS, EACH = 64;
+  __shared__ __attribute__((aligned(16))) float s_q[DP], s_k[DP];
+  __shared__ float s_v[COLUMNS * EACH], s_out[COLUMNS * EACH], s_log[2];
+  const int4 run = runs[blockIdx.x];
+  const int h = blockIdx.y, tid = threadIdx.x, wave = tid / PAE_WAVE, lane = tid % PAE_WAVE, sub = tid % 16, column = tid / 16;
+  const int slot = slots[run.x];
+  if (run.z <= 0) return;
+  float* held = state + (int64_t)slot * slot_stride + (int64_t)h * (V + 1) * D;
+  float* m_at = maximum + (int64_t)slot * max_slot_stride + h;
+  float S[COLUMNS][R][4], n[R][4];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int d = 64 * r + 4 * sub;
+    const f32x4 y = *reinterpret_cast<const f32x4*>(held + (uint32_t)(V * D + min(d, D - 4)));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) n[r][e] = d < D ? y[e] : 0.f;
+#pragma unroll
+    for (int c = 0; c < COLUMNS; ++c) {
+      const f32x4 z = *reinterpret_cast<const f32x4*>(held + (uint32_t)(min(c * EACH + column, V - 1) * D + min(d, D - 4)));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) S[c][r][e] = d < D ? z[e] : 0.f;
+    }
+  }
+  float m = *m_at;
+  const float q_scale = 1.0f / sqrtf((float)D), w = load_param(weight, w_is_f32, h * V + min(tid, V - 1));
+  for (int i = 0; i < run.z; ++i) {
+    const int64_t t = run.y + i;
+    const T* row = proj + t * row_stride;
+    const float gate = to_f32(gates[t * gate_stride + h * V + min(tid, V - 1)]);
+    if (wave < 2) {  // the input gate's sum, and the forget gate's
+      float z = 0.f;
+      if (gate_logits) {
+        z = gate_logits[t * 2 * H + wave * H + h];
+      } else {
+        z = gate_sum(x + t * ldx, gate_w + (int64_t)(wave * H + h) * hidden, hidden, wide) + gate_b[wave * H + h];
+      }
+      z = cap * tanhf(z / cap);
+      if (lane == 0) s_log[wave] = wave ? log_sigmoid_f(z) : z;
+    } else {
+      for (int e = tid - 128; e < 2 * DP + V; e += 1024 - 128) {
+        if (e < 2 * DP) {
+          const int which = e / DP, d = e % DP;
+          const float a = d < D ? to_f32(row[(which * H + h) * (int64_t)D + d]) : 0.f;
+          if (which) s_k[d] = a;
+          else s_q[d] = a * q_scale;
+        } else {
+          s_v[e - 2 * DP] = to_f32(row[2 * H * (int64_t)D + h * V + e - 2 * DP]);
+        }
+      }
+    }
+    __syncthreads();
+    const float li = s_log[0], lf = s_log[1], next = fmaxf(lf + m, li);
+    const float keep = expf(lf + m - next), take = expf(li - next), floors = expf(-next);
+    m = next;
+    float k[R][4], q[R][4], nq = 0.f;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const f32x4 k4 = *reinterpret_cast<const f32x4*>(s_k + 64 * r + 4 * sub), q4 = *reinterpret_cast<const f32x4*>(s_q + 64 * r + 4 * sub);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        k[r][e] = k4[e];
+        q[r][e] = q4[e];
+        n[r][e] = fmaf(k[r][e], take * 1.f, keep * n[r][e]);
+        nq = fmaf(n[r][e], q[r][e], nq);
+      }
+    }
+    nq = sum16(nq);
+    const float denom = fmaxf(fabsf(nq), floors) + floor_eps;
+#pragma unroll
+    for (int c = 0; c < COLUMNS; ++c) {
+      const int col = c * EACH + column;
+      const float v = take * s_v[min(col, V - 1)];
+      float o = 0.f;
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          S[c][r][e] = fmaf(k[r][e], v, keep * S[c][r][e]);
+          o = fmaf(S[c][r][e], q[r][e], o);
+        }
+      o = sum16(o);
+      if (sub == 0) s_out[col] = o;
+    }
+    __syncthreads();
+    if (tid < (V + PAE_WAVE - 1) / PAE_WAVE * PAE_WAVE) {  // whole wavefronts
+      float ss = 0.f;
+      const int each = pairs ? 2 : 1;  // a lane's neighbours, as in memory_finish_kernel
+      for (int u = lane * each; u < V; u += PAE_WAVE * each)
+        for (int e = 0; e < each; ++e) {
+          const float y = s_out[u + e] / denom;
+          ss = fmaf(y, y, ss);
+        }
+      ss = wave_sum(ss);
+      const float inv = 1.0f / sqrtf(ss / (float)V + eps);
+      const float g = 1.0f / (1.0f + expf(-gate));
+      if (tid < V) out[(t * H + h) * V + tid] = from_f32<T>(s_out[tid] / denom * inv * w * g);
+    }
+    // (what the next token writes: s_log, s_q, s_k and s_v were read before the last barrier, s_out is written behind the next)
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int d = 64 * r + 4 * sub;
+    if (d >= D) continue;
+    if (column == 0) *reinterpret_cast<f32x4*>(held + (uint32_t)(V * D + d)) = f32x4{n[r][0], n[r][1], n[r][2], n[r][3]};
+#pragma unroll
+    for (int c = 0; c < COLUMNS; ++c)
+      if (c * EACH + column < V)
+        *reinterpret_cast<f32x4*>(held + (uint32_t)((c * EACH + column) * D + d)) = f32x4{S[c][r][0], S[c][r][1], S[c][r][2], S[c][r][3]};
+  }
+  if (tid == 0) *m_at = m;
 }
 
 // ---------------------------------------------------------------------------------------------- chunks
@@ -575,14 +711,32 @@ struct MemoryStep {
   float *sums, *o, *nq;
 };
 
+// Rows that the gates' sums may read in 16-byte pieces.
+template <typename T>
+static int wide_gates(const MemoryStep& a) {
+  const int vec = 16 / (int)sizeof(T);
+  return a.x && a.hidden % vec == 0 && a.ldx % vec == 0 && (uintptr_t)a.x % 16 == 0 && (uintptr_t)a.gate_w % 16 == 0;
+}
+
+template <typename T>
+static void memory_tokens(const T* proj, const MemoryStep& a, const void* gate_in, const void* norm_w, int w_is_f32, float norm_eps,
+                          float floor_eps, bool pairs, void* out, hipStream_t stream) {
+#define MEMORY_TOKENS(R)                                                                                                            \
+  memory_tokens_kernel<T, R><<<dim3(a.num_serial, a.H), 1024, 0, stream>>>(                                                         \
+      proj, a.row_stride, a.gate_logits, (const T*)a.x, a.ldx, (const T*)a.gate_w, a.gate_b, a.hidden, wide_gates<T>(a), a.serial,  \
+      a.slots, a.state, a.state_slot_stride, a.maximum, a.max_slot_stride, a.H, a.D, a.V, a.cap, (const T*)gate_in, a.gate_stride, \
+      norm_w, w_is_f32, norm_eps, floor_eps, pairs, (T*)out)
+  if (a.D <= 64) MEMORY_TOKENS(1);
+  else MEMORY_TOKENS(2);
+#undef MEMORY_TOKENS
+}
+
 template <typename T>
 static void memory_launch(const T* proj, const MemoryStep& a, hipStream_t stream) {
   const int H = a.H, D = a.D, V = a.V;
   if (a.num_serial > 0) {
-    const int vec = 16 / (int)sizeof(T);
-    const int wide = a.x && a.hidden % vec == 0 && a.ldx % vec == 0 && (uintptr_t)a.x % 16 == 0 && (uintptr_t)a.gate_w % 16 == 0;
     memory_gates_few_kernel<T><<<dim3(a.num_serial, H), 256, 0, stream>>>(a.gate_logits, (const T*)a.x, a.ldx, (const T*)a.gate_w,
-                                                                          a.gate_b, a.hidden, wide, a.serial, a.slots, a.maximum,
+                                                                          a.gate_b, a.hidden, wide_gates<T>(a), a.serial, a.slots, a.maximum,
                                                                           a.max_slot_stride, H, a.cap, a.gates);
     dim3 grid(a.num_serial, H, (V + 16) / 16);
 #define MEMORY_SERIAL(R)                                                                                                \
@@ -648,6 +802,17 @@ extern "C" int pae_matrix_memory_step(int dtype, const void* proj, int64_t row_s
   a.serial = (const int4*)serial; a.chunks = (const int4*)chunks; a.scans = (const int4*)scans;
   a.num_tokens = num_tokens; a.num_serial = num_serial; a.num_chunks = num_chunks; a.num_scans = num_scans;
   a.slots = slots; a.H = H; a.D = D; a.V = V; a.cap = gate_cap; a.state = state; a.maximum = maximum;
+  const int size = dtype == PAE_F32 ? 4 : 2;
+  const bool pairs = V % 2 == 0 && gate_stride % 2 == 0 && (uintptr_t)gate_in % (2 * size) == 0 && (uintptr_t)out % (2 * size) == 0;
+  // Single tokens: one launch, for what a workgroup's lanes hold, where four rows of a column may be read together, and up to about three
+  // workgroups a compute unit, which holds one at a time (28 heads of 128 for 24 / 32 / 48 sequences 23.3 / 30.4 / 42.1 us against 25.8 / 30.2 / 39.6, 14 of 64
+  // for 48 / 64 13.2 / 16.6 against 13.7 / 15.5).
+  if ((int64_t)num_serial * H <= 768 && num_chunks == 0 && num_serial == num_tokens && D <= 128 && D % 4 == 0 && V <= MM_TOKEN_COLUMNS * 64 && state_slot_stride % 4 == 0 &&
+      (uintptr_t)state % 16 == 0) {
+    if (dtype == PAE_F32) memory_tokens<float>((const float*)proj, a, gate_in, norm_w, w_is_f32, norm_eps, floor_eps, pairs, out, stream);
+    else memory_tokens<bf16_t>((const bf16_t*)proj, a, gate_in, norm_w, w_is_f32, norm_eps, floor_eps, pairs, out, stream);
+    return pae_check_launch("matrix_memory_step (single tokens)");
+  }
   // work: o [T][H][V], sums [num_chunks][H][V + 1][D], each from a 16-byte boundary on; then seven of [T][H]
   a.o = work;
   a.sums = a.o + (TH * V + 3) / 4 * 4;
@@ -655,8 +820,6 @@ extern "C" int pae_matrix_memory_step(int dtype, const void* proj, int64_t row_s
   a.nq = rest;
   a.gates = MemoryGates{rest + TH, rest + 2 * TH, rest + 3 * TH, rest + 4 * TH, rest + 5 * TH, rest + 6 * TH};
   dim3 token_heads(num_tokens, (H + 3) / 4);
-  const int size = dtype == PAE_F32 ? 4 : 2;
-  const bool pairs = V % 2 == 0 && gate_stride % 2 == 0 && (uintptr_t)gate_in % (2 * size) == 0 && (uintptr_t)out % (2 * size) == 0;
 #define MEMORY_FINISH(T, W)                                                                                              \
   memory_finish_kernel<T, W><<<token_heads, 256, 0, stream>>>(a.o, a.nq, a.gates.floors, (const T*)gate_in, gate_stride,  \
                                                               norm_w, w_is_f32, norm_eps, floor_eps, H, V, (T*)out)

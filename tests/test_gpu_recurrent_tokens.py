@@ -1,5 +1,5 @@
-"""Steps of single tokens through the gated delta rule and gated linear attention in one launch (recurrent_tokens.hip) against the separate
-kernels, which take a step with an empty run beside them: the same bits in the read-outs, the states and the convolution's inputs.  Widths
+"""Steps of single tokens through the gated delta rule, gated linear attention (recurrent_tokens.hip) and the matrix memory
+(matrix_memory.hip) in one launch against the separate kernels, which take a step with an empty run beside them: the same bits in the read-outs, the states and the convolution's inputs.  Widths
 at the edges of lanes, columns and wavefronts; one to three value heads a key head; no, few and many taps; runs of two tokens beside empty ones."""
 
 import pytest
@@ -68,6 +68,30 @@ def test_linear_attention(dtype, bias, H, D, V):
             out, st = torch.full((T, H * V), float("nan"), dtype=dtype, device=DEV), state.clone()
             K.linear_attention_step(proj, decay, decay_bias, 16.0, gate, out, runs, slots, st, norm_w, H, D, V, 1e-5, "silu" if bias else "sigmoid")
             got.append((out, st))
+        for one, many in zip(*got):
+            assert torch.equal(one, many), lengths
+        assert not torch.equal(got[0][1], state) and bool(torch.isfinite(got[0][0].float()).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("formed", [False, True])
+@pytest.mark.parametrize("H,D,V,hidden", [(1, 4, 1, 64), (4, 64, 128, 1536), (12, 128, 128, 1536), (3, 100, 72, 100), (2, 68, 65, 1030)])
+def test_matrix_memory(dtype, formed, H, D, V, hidden):
+    gen = torch.Generator().manual_seed(D + V)
+    for lengths in RUNS:
+        T, S = sum(lengths), len(lengths)
+        proj, gate = normal(gen, T, 2 * H * D + H * V).to(dtype), normal(gen, T, H * V).to(dtype)
+        x, gate_w, gate_b = normal(gen, T, hidden).to(dtype), (normal(gen, 2 * H, hidden) * 0.1).to(dtype), normal(gen, 2 * H) * 3.0
+        logits = None if formed else normal(gen, T, 2 * H) * 6.0
+        state, maximum, norm_w = normal(gen, 2 * S + 4, H, V + 1, D), normal(gen, 2 * S + 4, H), normal(gen, H * V)
+        empty, got = torch.zeros(0, 4, dtype=torch.int32, device=DEV), []
+        for spare in (False, True):
+            runs, slots = runs_of(lengths, spare)
+            serial = torch.stack([torch.arange(len(runs), dtype=torch.int32, device=DEV), runs[:, 0], runs[:, 1], runs[:, 2]], 1).contiguous()
+            out, st, top = torch.full((T, H * V), float("nan"), dtype=dtype, device=DEV), state.clone(), maximum.clone()
+            K.matrix_memory_step(proj, gate, logits, out, serial, empty, empty, slots, st, top, norm_w, H, D, V, 15.0, 1e-5, 1e-6,
+                                 gates_from=(x, gate_w, gate_b) if formed else None)
+            got.append((out, st, top))
         for one, many in zip(*got):
             assert torch.equal(one, many), lengths
         assert not torch.equal(got[0][1], state) and bool(torch.isfinite(got[0][0].float()).all())
