@@ -484,7 +484,7 @@ __global__ void swiglu_kernel(T* __restrict__ out, const T* __restrict__ x, int 
   const int64_t ui = block ? gi + block : (int64_t)inter + j;
   const float g = to_f32(x[t * 2 * inter + gi]);
   const float u = to_f32(x[t * 2 * inter + ui]);
-  out[idx] = from_f32<T>(g / (1.0f + expf(-g)) * u);
+  out[idx] = from_f32<T>(act_to<T>(g, 2) * u);
 }
 
 // Eight bfloat16 outputs per thread (16-byte loads and stores): used when the width and
@@ -506,8 +506,8 @@ __global__ void swiglu_vec8_kernel(bf16_t* __restrict__ out, const bf16_t* __res
   for (int k = 0; k < 4; ++k) {
     const float g0 = __uint_as_float(gw[k] << 16), g1 = __uint_as_float(gw[k] & 0xffff0000u);
     const float u0 = __uint_as_float(uw[k] << 16), u1 = __uint_as_float(uw[k] & 0xffff0000u);
-    const bf16_t o0 = __float2bfloat16(g0 / (1.0f + expf(-g0)) * u0);
-    const bf16_t o1 = __float2bfloat16(g1 / (1.0f + expf(-g1)) * u1);
+    const bf16_t o0 = __float2bfloat16(silu_to_bf16(g0) * u0);
+    const bf16_t o1 = __float2bfloat16(silu_to_bf16(g1) * u1);
     ow[k] = (unsigned)(*reinterpret_cast<const unsigned short*>(&o0)) |
             ((unsigned)(*reinterpret_cast<const unsigned short*>(&o1)) << 16);
   }
@@ -524,7 +524,7 @@ __global__ void gated_act_kernel(T* __restrict__ out, const T* __restrict__ x, i
   const int j = (int)(idx % inter);
   const int64_t gi = block ? (int64_t)(j / block) * 2 * block + j % block : j;
   const int64_t ui = block ? gi + block : (int64_t)inter + j;
-  out[idx] = from_f32<T>(act_of(to_f32(x[t * 2 * inter + gi]), kind) * to_f32(x[t * 2 * inter + ui]));
+  out[idx] = from_f32<T>(act_to<T>(to_f32(x[t * 2 * inter + gi]), kind) * to_f32(x[t * 2 * inter + ui]));
 }
 
 // Eight bfloat16 outputs per thread (16-byte loads and stores), for widths and blocks in multiples of 8.
@@ -545,8 +545,8 @@ __global__ void gated_act_vec8_kernel(bf16_t* __restrict__ out, const bf16_t* __
   for (int k = 0; k < 4; ++k) {
     const float g0 = __uint_as_float(gw[k] << 16), g1 = __uint_as_float(gw[k] & 0xffff0000u);
     const float u0 = __uint_as_float(uw[k] << 16), u1 = __uint_as_float(uw[k] & 0xffff0000u);
-    const bf16_t o0 = __float2bfloat16(act_of(g0, kind) * u0);
-    const bf16_t o1 = __float2bfloat16(act_of(g1, kind) * u1);
+    const bf16_t o0 = __float2bfloat16(act_to<bf16_t>(g0, kind) * u0);
+    const bf16_t o1 = __float2bfloat16(act_to<bf16_t>(g1, kind) * u1);
     ow[k] = (unsigned)(*reinterpret_cast<const unsigned short*>(&o0)) |
             ((unsigned)(*reinterpret_cast<const unsigned short*>(&o1)) << 16);
   }

@@ -111,7 +111,7 @@ __device__ __forceinline__ void finish(const Product& p, const f32x4 (&acc)[MT][
 #pragma unroll
       for (int x = 0; x < X; x += 2)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[2 * x + e] = (__bf16)(act_of(rounded(acc[i][x][e]), ACT) * rounded(acc[i][x + 1][e]));
+        for (int e = 0; e < 4; ++e) v[2 * x + e] = (__bf16)(act_to<bf16_t>(rounded(acc[i][x][e]), ACT) * rounded(acc[i][x + 1][e]));
       if constexpr (X == 4) *reinterpret_cast<bf16x8*>(o) = *reinterpret_cast<const bf16x8*>(v);
       else *reinterpret_cast<bf16x4*>(o) = *reinterpret_cast<const bf16x4*>(v);
     }

@@ -549,7 +549,7 @@ __global__ __launch_bounds__(256) void moe_tiles_gate_up_kernel(bf16_t* __restri
       bf16_t* o = act + (int64_t)(tile.y + r) * inter + f;
 #pragma unroll
       for (int i = 0; i < 4; ++i)
-        if (f + i < inter) o[i] = __float2bfloat16(act_of(gs[mt][nt][i], act_kind) * us[mt][nt][i]);
+        if (f + i < inter) o[i] = __float2bfloat16(act_to<bf16_t>(gs[mt][nt][i], act_kind) * us[mt][nt][i]);
     }
   }
 }
@@ -755,7 +755,7 @@ __global__ __launch_bounds__(256) void moe_few_tiles_kernel(bf16_t* __restrict__
         bf16_t* o = act_out + (int64_t)sorted * N + n;
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          if (n + i < N) o[i] = __float2bfloat16(act_of(s1[i], act_kind) * s2[i]);
+          if (n + i < N) o[i] = __float2bfloat16(act_to<bf16_t>(s1[i], act_kind) * s2[i]);
       } else {
         const float weight = weights[pair];
         float* o = y + ((int64_t)(pair % top) * num_tokens + pair / top) * N + n;
@@ -840,7 +840,7 @@ __global__ __launch_bounds__(512, 1) void moe_big_tiles_kernel(bf16_t* __restric
       if (f < N) {
         bf16_t eight[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) eight[i] = __float2bfloat16(act_of(acc[mt][i / 4][i % 4], act_kind) * acc[mt][2 + i / 4][i % 4]);
+        for (int i = 0; i < 8; ++i) eight[i] = __float2bfloat16(act_to<bf16_t>(acc[mt][i / 4][i % 4], act_kind) * acc[mt][2 + i / 4][i % 4]);
         *reinterpret_cast<uint4*>(act_out + (int64_t)(tile.y + r) * N + f) = *reinterpret_cast<const uint4*>(eight);
       }
     } else {
