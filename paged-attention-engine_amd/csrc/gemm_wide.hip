@@ -11,10 +11,10 @@
 // 160 and 45.6, 177 in one.  What the epilogue adds is the angles' and pages' way and the values' stores of 2 bytes.
 //
 // Measured beside the platform library's product (weights from memory, us; rows x features x k):
-//     2,048 x 17,920 x  1,536   library 111 and 22 for the gate behind it    here with the gate 100
+//     2,048 x 17,920 x  1,536   library 111 and 22 for the gate behind it    here with the gate 96
 //     2,048 x  1,536 x  8,960           71                                   66
 //     2,048 x  2,048 x  1,536           19                                   15
-//     6,030 x 37,888 x  3,584        1,209 and 117 for the gate              1,176 with the gate
+//     6,030 x 37,888 x  3,584        1,209 and 117 for the gate              1,143 with the gate
 //     6,030 x  3,584 x 18,944        1,041                                   600
 //       601 x  1,536 x  8,960           36                                   24 in ranges of k
 //       200 x  1,536 x  1,536           20                                   8
@@ -282,42 +282,59 @@ __global__ __launch_bounds__(512, 2) void wide_large_kernel(Product p) {
   const int lane = threadIdx.x % PAE_WAVE;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PAE_WAVE);
   int tm, tn;
-  if (PARTS > 1 && (int)blockIdx.x >= p.whole) {
-    const int rest = (p.row_tiles * p.col_tiles - p.whole) * PARTS, at = in_row(blockIdx.x - p.whole, rest);
+  const int ranges = MODE == wide_gemm::SUMS ? p.whole * p.splits : p.whole, together = min(ranges, UNITS);
+  if (PARTS > 1 && (int)blockIdx.x >= together) {
+    const int rest = (p.row_tiles * p.col_tiles - p.whole) * PARTS, at = in_row(blockIdx.x - together, rest);
     place_of(p.whole + at / PARTS, p.row_tiles, p.col_tiles, p.strip, tm, tn);
     const int m0 = tm * 256 + at % PARTS / (PARTS / 2) * 128, n0 = tn * 256 + (PARTS == 4 ? at % 2 * 128 : 0);
     if (m0 >= p.M || n0 >= p.N) return;
     small_tile<MODE, ACT, typename std::conditional<PARTS == 4, Quarter, Half>::type>(p, wide_lds, m0, n0, 0, p.stages, 0);
     return;
   }
-  int id = in_row(blockIdx.x, MODE == wide_gemm::SUMS ? p.whole * p.splits : p.whole), split = 0, first = 0, stages = p.stages;
-  if (MODE == wide_gemm::SUMS) {  // the ranges of k lie one after another
-    split = id / p.whole;
-    id -= split * p.whole;
-    first = (int)((int64_t)p.stages * split / p.splits);
-    stages = (int)((int64_t)p.stages * (split + 1) / p.splits) - first;
-  }
-  place_of(id, p.row_tiles, p.col_tiles, p.strip, tm, tn);
-  const int m0 = tm * 256, n0 = tn * 256;
+  // A unit's workgroup takes one tile after another (the ones that it would be given one by one), and asks for the next one's first stages
+  // before it leaves a tile's results: what a tile needs beside its stages, some 11 of 39 us at k 1,536, is the way of its first stage, its epilogue and
+  // a workgroup's start (gated, us, a workgroup a tile and this: 8,192 x 17,920 x 1,536 350 and 338, 2,048 98.7 and 96.4, 8,192 x 22,016 x 2,048 541 and
+  // 527, 8,192 x 9,728 x 896 127 and 117; 6,030 x 37,888 x 3,584 1,149 and 1,143).
   Large::Source src;
-  src.a = p.a + m0 * p.lda + (int64_t)first * wide_gemm::ROW_BYTES;
-  const int w0 = first_w_row<MODE>(p, n0);
-  src.w = p.w + w0 * p.ldw + (int64_t)first * wide_gemm::ROW_BYTES;
-#pragma unroll
-  for (int h = 0; h < 2; ++h)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int q = (wave * 2 + j) * 8 + lane / 8;
-      src.a_off[h][j] = (uint32_t)min(Large::a_row(h, q), p.M - 1 - m0) * (uint32_t)p.lda + wide_gemm::piece_of(lane, q);
-      src.w_off[h][j] = (uint32_t)(w_row_of<MODE>(p, min(n0 + Large::w_row<MODE>(h, q), p.N - 1)) - w0) * (uint32_t)p.ldw + wide_gemm::piece_of(lane, q);
+  int m0, n0, split, stages;
+  auto begin = [&](int i) {
+    int id = in_row(i, ranges), first = 0;
+    split = 0;
+    stages = p.stages;
+    if (MODE == wide_gemm::SUMS) {  // the ranges of k lie one after another
+      split = id / p.whole;
+      id -= split * p.whole;
+      first = (int)((int64_t)p.stages * split / p.splits);
+      stages = (int)((int64_t)p.stages * (split + 1) / p.splits) - first;
     }
-  f32x4 acc[Large::MT][Large::X];
+    place_of(id, p.row_tiles, p.col_tiles, p.strip, tm, tn);
+    m0 = tm * 256;
+    n0 = tn * 256;
+    src.a = p.a + m0 * p.lda + (int64_t)first * wide_gemm::ROW_BYTES;
+    const int w0 = first_w_row<MODE>(p, n0);
+    src.w = p.w + w0 * p.ldw + (int64_t)first * wide_gemm::ROW_BYTES;
 #pragma unroll
-  for (int i = 0; i < Large::MT; ++i)
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
-    for (int x = 0; x < Large::X; ++x) acc[i][x] = f32x4{0.f, 0.f, 0.f, 0.f};
-  Large::run(acc, wide_lds, src, stages);
-  finish<MODE, ACT>(p, acc, m0 + wave / Large::WN * Large::PM, n0 + wave % Large::WN * Large::PN, split);
+      for (int j = 0; j < 2; ++j) {
+        const int q = (wave * 2 + j) * 8 + lane / 8;
+        src.a_off[h][j] = (uint32_t)min(Large::a_row(h, q), p.M - 1 - m0) * (uint32_t)p.lda + wide_gemm::piece_of(lane, q);
+        src.w_off[h][j] = (uint32_t)(w_row_of<MODE>(p, min(n0 + Large::w_row<MODE>(h, q), p.N - 1)) - w0) * (uint32_t)p.ldw + wide_gemm::piece_of(lane, q);
+      }
+    Large::begin(wide_lds, src);
+  };
+  begin(blockIdx.x);
+  for (int i = blockIdx.x; i < ranges; i += together) {
+    f32x4 acc[Large::MT][Large::X];
+#pragma unroll
+    for (int j = 0; j < Large::MT; ++j)
+#pragma unroll
+      for (int x = 0; x < Large::X; ++x) acc[j][x] = f32x4{0.f, 0.f, 0.f, 0.f};
+    Large::run(acc, wide_lds, src, stages);
+    const int row0 = m0 + wave / Large::WN * Large::PM, col0 = n0 + wave % Large::WN * Large::PN, of = split;
+    if (i + together < ranges) begin(i + together);
+    finish<MODE, ACT>(p, acc, row0, col0, of);
+  }
 }
 
 // One shape of smaller tiles throughout; the ranges of k lie one after another.  (Never all 512 registers for a wavefront: the
@@ -353,6 +370,9 @@ int launch_small(Product p, hipStream_t stream) {
   return launch(wide_small_kernel<MODE, ACT, T>, p, (int64_t)p.row_tiles * p.col_tiles * p.splits, T::WAVES * 64, T::LDS_BYTES, stream);
 }
 
+// Workgroups of tiles of 256 x 256: one a unit.
+int64_t together(int64_t tiles) { return tiles < UNITS ? tiles : UNITS; }
+
 template <int MODE, int ACT>
 int launch_large(Product p, hipStream_t stream) {
   p.row_tiles = (p.M + 255) / 256;
@@ -363,15 +383,15 @@ int launch_large(Product p, hipStream_t stream) {
   if constexpr (MODE == wide_gemm::SUMS) {
     p.whole = (int)tiles;
     PAE_REQUIRE(tiles * p.splits < (1ll << 30), "wide product: too many tiles");
-    return launch(wide_large_kernel<MODE, ACT, 1>, p, tiles * p.splits, 512, Large::LDS_BYTES, stream);
+    return launch(wide_large_kernel<MODE, ACT, 1>, p, together(tiles * p.splits), 512, Large::LDS_BYTES, stream);
   }
   const int rest = (int)(tiles % UNITS), parts = rest == 0 || rest > UNITS / 2 ? 1 : rest > UNITS / 4 ? 2 : 4;
   p.whole = (int)(parts == 1 ? tiles : tiles - rest);
   constexpr int LDS = Large::LDS_BYTES > Half::LDS_BYTES ? Large::LDS_BYTES : Half::LDS_BYTES;
   static_assert(Quarter::LDS_BYTES <= LDS, "room for every part");
-  if (parts == 1) return launch(wide_large_kernel<MODE, ACT, 1>, p, tiles, 512, Large::LDS_BYTES, stream);
-  if (parts == 2) return launch(wide_large_kernel<MODE, ACT, 2>, p, p.whole + 2 * rest, 512, LDS, stream);
-  return launch(wide_large_kernel<MODE, ACT, 4>, p, p.whole + 4 * rest, 512, LDS, stream);
+  if (parts == 1) return launch(wide_large_kernel<MODE, ACT, 1>, p, together(tiles), 512, Large::LDS_BYTES, stream);
+  if (parts == 2) return launch(wide_large_kernel<MODE, ACT, 2>, p, together(p.whole) + 2 * rest, 512, LDS, stream);
+  return launch(wide_large_kernel<MODE, ACT, 4>, p, together(p.whole) + 4 * rest, 512, LDS, stream);
 }
 
 enum { SHAPE_LARGE, SHAPE_128_256, SHAPE_128_128, SHAPE_128_96, SHAPE_64_128, SHAPE_64_64, SHAPES };

@@ -222,20 +222,41 @@ struct Large {
   template <int MODE>
   static __device__ __forceinline__ int w_row(int h, int q) { return (q / 32) * PN + dealt_row<MODE, X>(h * 2 + (q / 16) % 2, q % 16); }
 
-  // `stages` >= 2
+  static __device__ __forceinline__ uint32_t lds_at(const char* lds) {
+    return __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)lds);
+  }
+  static __device__ __forceinline__ void load_a(uint32_t lds0, const Source& src, int h, uint32_t stage) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PAE_WAVE);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) load_to_lds(lds0 + stage + h * HALF + (wave * 2 + j) * 1024, src.a_off[h][j], src.a);
+  }
+  static __device__ __forceinline__ void load_w(uint32_t lds0, const Source& src, int h, uint32_t stage) {
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PAE_WAVE);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) load_to_lds(lds0 + stage + (2 + h) * HALF + (wave * 2 + j) * 1024, src.w_off[h][j], src.w);
+  }
+  // The first loads of a tile; no wavefront reads `lds` any more (as when `run` is through).
+  static __device__ __forceinline__ void begin(char* lds, Source& src) {
+    const uint32_t lds0 = lds_at(lds);
+    load_w(lds0, src, 0, 0);
+    load_a(lds0, src, 0, 0);
+    load_w(lds0, src, 1, 0);
+    load_a(lds0, src, 1, 0);
+    src.a += ROW_BYTES;
+    src.w += ROW_BYTES;
+    load_w(lds0, src, 0, STAGE_BYTES);
+    load_a(lds0, src, 0, STAGE_BYTES);
+    load_w(lds0, src, 1, STAGE_BYTES);
+  }
+
+  // Behind `begin`; `stages` >= 2.  Loads and stores that came between are waited for with its loads.
   static __device__ __forceinline__ void run(f32x4 (&acc)[MT][X], char* lds, Source& src, int stages) {
     const int lane = threadIdx.x % PAE_WAVE, col = lane % 16, kg = lane / 16;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PAE_WAVE);
     const int wm = wave / WN, wn = wave % WN;
-    const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds);
-    auto load_a = [&](int h, uint32_t stage) {
-#pragma unroll
-      for (int j = 0; j < 2; ++j) load_to_lds(lds0 + stage + h * HALF + (wave * 2 + j) * 1024, src.a_off[h][j], src.a);
-    };
-    auto load_w = [&](int h, uint32_t stage) {
-#pragma unroll
-      for (int j = 0; j < 2; ++j) load_to_lds(lds0 + stage + (2 + h) * HALF + (wave * 2 + j) * 1024, src.w_off[h][j], src.w);
-    };
+    const uint32_t lds0 = lds_at(lds);
+    auto load_a = [&](int h, uint32_t stage) { Large::load_a(lds0, src, h, stage); };
+    auto load_w = [&](int h, uint32_t stage) { Large::load_w(lds0, src, h, stage); };
     uint32_t a_at[2], w_at[2];
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
@@ -272,14 +293,6 @@ struct Large {
       src.a += ROW_BYTES;
       src.w += ROW_BYTES;
     };
-    load_w(0, 0);
-    load_a(0, 0);
-    load_w(1, 0);
-    load_a(1, 0);
-    forward();
-    load_w(0, STAGE_BYTES);
-    load_a(0, STAGE_BYTES);
-    load_w(1, STAGE_BYTES);
     asm volatile("s_waitcnt vmcnt(6)" ::: "memory");  // the first stage: all but the last three halves, of two loads each
     meet();
     if (wm == 1) meet();

@@ -253,3 +253,16 @@ def test_silu_of_every_bfloat16_number():
         got = out[0].cpu().double()
         assert ((got - exact).abs()[finite] <= (2.0 ** -8 * 1.01 * exact.abs() + 2.0 ** -133 + 3e-37 * (z < -88.5))[finite]).all()
         assert torch.equal(got.isnan(), exact.isnan()) and got[z == float("inf")] == float("inf")
+
+
+@pytest.mark.parametrize("M,N,mode,ranges", [(2048, 8448, K.WIDE_PLAIN, 1), (2300, 9472, K.WIDE_GATED, 1), (1000, 9216, K.WIDE_SUMS, 4), (4097, 8208, K.WIDE_PLAIN, 1)])
+def test_more_tiles_of_256_than_units(M, N, mode, ranges):
+    """A workgroup then takes one tile after another: what its first tile gives and its last, with whole tiles, cut ones and ranges of k,
+    is what tiles of 128 x 128 give, bit for bit."""
+    a, w = operands(M, N, 512, 9)
+    shape = {K.WIDE_PLAIN: (M, N), K.WIDE_GATED: (M, N // 2), K.WIDE_SUMS: (ranges, M, N)}[mode]
+    kind = "silu" if mode == K.WIDE_GATED else None
+    got = [torch.full(shape, float("nan"), device="cuda", dtype=torch.float32 if mode == K.WIDE_SUMS else torch.bfloat16) for _ in range(2)]
+    for out, tile in zip(got, (0, 2)):
+        K.gemm_wide(out, a, w, tile | ranges << 8, kind=kind, mode=mode)
+    assert -(-M // 256) * -(-N // 256) * ranges > 256 and torch.equal(*got)
