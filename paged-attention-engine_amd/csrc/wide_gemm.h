@@ -249,8 +249,9 @@ struct Large {
     load_w(lds0, src, 1, STAGE_BYTES);
   }
 
-  // Behind `begin`; `stages` >= 2.  Loads and stores that came between are waited for with its loads.
-  static __device__ __forceinline__ void run(f32x4 (&acc)[MT][X], char* lds, Source& src, int stages) {
+  // Behind `begin`; `stages` >= 2.  Loads and stores that came between are waited for with its loads, but for STORES if `stored`: that many were.
+  template <int STORES>
+  static __device__ __forceinline__ void run(f32x4 (&acc)[MT][X], char* lds, Source& src, int stages, bool stored) {
     const int lane = threadIdx.x % PAE_WAVE, col = lane % 16, kg = lane / 16;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PAE_WAVE);
     const int wm = wave / WN, wn = wave % WN;
@@ -293,7 +294,9 @@ struct Large {
       src.a += ROW_BYTES;
       src.w += ROW_BYTES;
     };
-    asm volatile("s_waitcnt vmcnt(6)" ::: "memory");  // the first stage: all but the last three halves, of two loads each
+    // the first stage: all but the last three halves, of two loads each
+    if (STORES > 0 && stored) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(6 + STORES) : "memory");
+    else asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
     meet();
     if (wm == 1) meet();
     // ONE, TWO: stages t + 1 and t + 2 there are
