@@ -234,7 +234,7 @@ template <typename T>
 __global__ void activation_kernel(T* __restrict__ x, int64_t n, int kind, const void* __restrict__ bias, int b_is_f32,
                                   int width) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) x[i] = from_f32<T>(act_of(to_f32(x[i]) + (bias ? load_param(bias, b_is_f32, i % width) : 0.f), kind));
+  if (i < n) x[i] = from_f32<T>(act_to<T>(to_f32(x[i]) + (bias ? load_param(bias, b_is_f32, i % width) : 0.f), kind));
 }
 
 // eight bfloat16 numbers a thread (one 16-byte load and store), for sizes that are multiples of eight
@@ -245,8 +245,8 @@ __global__ void activation_bf16x8_kernel(uint4* __restrict__ x, int64_t nvec, in
   unsigned* w = reinterpret_cast<unsigned*>(&v);
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    const bf16_t lo = __float2bfloat16(act_of(__uint_as_float(w[j] << 16), kind));
-    const bf16_t hi = __float2bfloat16(act_of(__uint_as_float(w[j] & 0xffff0000u), kind));
+    const bf16_t lo = __float2bfloat16(act_to<bf16_t>(__uint_as_float(w[j] << 16), kind));
+    const bf16_t hi = __float2bfloat16(act_to<bf16_t>(__uint_as_float(w[j] & 0xffff0000u), kind));
     w[j] = (unsigned)*reinterpret_cast<const unsigned short*>(&lo) | ((unsigned)*reinterpret_cast<const unsigned short*>(&hi) << 16);
   }
   x[i] = v;
@@ -265,8 +265,8 @@ __global__ __launch_bounds__(256) void activation_bias_bf16x8_kernel(uint4* __re
     unsigned* w = reinterpret_cast<unsigned*>(&v);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const bf16_t lo = __float2bfloat16(act_of(__uint_as_float(w[j] << 16) + b[2 * j], kind));
-      const bf16_t hi = __float2bfloat16(act_of(__uint_as_float(w[j] & 0xffff0000u) + b[2 * j + 1], kind));
+      const bf16_t lo = __float2bfloat16(act_to<bf16_t>(__uint_as_float(w[j] << 16) + b[2 * j], kind));
+      const bf16_t hi = __float2bfloat16(act_to<bf16_t>(__uint_as_float(w[j] & 0xffff0000u) + b[2 * j + 1], kind));
       w[j] = (unsigned)*reinterpret_cast<const unsigned short*>(&lo) | ((unsigned)*reinterpret_cast<const unsigned short*>(&hi) << 16);
     }
     x[(int64_t)r * row_vecs + c] = v;

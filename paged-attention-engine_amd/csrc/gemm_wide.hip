@@ -231,7 +231,7 @@ __device__ __forceinline__ void finish(const Product& p, const f32x4 (&acc)[MT][
 #pragma unroll
       for (int x = 0; x < X; ++x)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[4 * x + e] = (__bf16)(ACT == NO_ACT ? z[x][e] : act_of(z[x][e], ACT));
+        for (int e = 0; e < 4; ++e) v[4 * x + e] = (__bf16)(ACT == NO_ACT ? z[x][e] : act_to<bf16_t>(z[x][e], ACT));
 #pragma unroll
       for (int x = 0; x < X; x += 2) {
         const int n = n0 + 16 * x + (x + 1 < X ? 8 : 4) * kg;

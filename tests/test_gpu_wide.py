@@ -237,21 +237,27 @@ def test_projections_rotate_and_store(M, nh, nkv, hd, rot, bs, bias, k):
         assert bool((pools[0].cpu().transpose(1, 2)[kept] == 7.0).all()) and bool((pools[1].cpu().permute(0, 3, 1, 2)[kept] == 7.0).all())
 
 
-def test_silu_of_every_bfloat16_number():
-    """The gate of bfloat16 results is worked out by the unit's own exponential and reciprocal: within bfloat16's rounding, 2^-8
-    of the result and a part in 100 more, of SiLU in float64; zero, as before, from where exp(-z) passes float32's largest number (-88.72: 3e-37 and
-    less are left out); what is not finite stays so."""
+@pytest.mark.parametrize("kind", ["silu", "gelu_tanh", "gelu"])
+def test_activations_of_every_bfloat16_number(kind):
+    """Activations of bfloat16 results are worked out by the unit's own exponential and reciprocal: within bfloat16's rounding, 2^-8 of the
+    result and a part in 100 more, of the activation in float64.  Left out is what the unit gives as zero: results below 3e-37, from where
+    exp(-z) passes float32's largest number (-88.72) or exp(-z^2 / 2) its least.  What is not finite stays so."""
     z = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
     x = torch.zeros(1, 2 * 65536, dtype=torch.bfloat16)
     x[0, :65536], x[0, 65536:] = z, 1.0
-    x = x.to("cuda")
-    exact = z.double() / (1 + torch.exp(-z.double()))
+    x, d = x.to("cuda"), z.double()
+    if kind == "gelu":
+        exact = 0.5 * d * torch.special.erfc(-d * 0.5 ** 0.5)
+    else:
+        exact = d / (1 + torch.exp(-d if kind == "silu" else -2 * (2 / torch.pi) ** 0.5 * (d + 0.044715 * d ** 3)))
     finite = z.isfinite()
-    for call in (lambda out, t: K.swiglu(out, t), lambda out, t: K.gated_act(out, t, "silu")):
+    calls = [lambda out: K.gated_act(out, x, kind)]
+    calls += {"silu": [lambda out: K.swiglu(out, x)], "gelu": [lambda out: K.activation(out.copy_(x[:, :65536]), kind)], "gelu_tanh": []}[kind]
+    for call in calls:
         out = torch.empty(1, 65536, dtype=torch.bfloat16, device="cuda")
-        call(out, x)
+        call(out)
         got = out[0].cpu().double()
-        assert ((got - exact).abs()[finite] <= (2.0 ** -8 * 1.01 * exact.abs() + 2.0 ** -133 + 3e-37 * (z < -88.5))[finite]).all()
+        assert ((got - exact).abs() <= 2.0 ** -8 * 1.01 * exact.abs() + 2.0 ** -133 + 3e-37 * (exact.abs() < 3e-37))[finite].all()
         assert torch.equal(got.isnan(), exact.isnan()) and got[z == float("inf")] == float("inf")
 
 
