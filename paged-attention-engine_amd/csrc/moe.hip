@@ -778,11 +778,13 @@ __global__ __launch_bounds__(256) void moe_few_tiles_kernel(bf16_t* __restrict__
 // one workgroup's features after another 594 and 298 us; four wavefronts of 64 x 128 through LDS 382 and 172; with an expert's
 // tiles side by side on one die 318 and 140 (three quarters of the lines from L2); with the loads spread among
 // the products 306 and 127 us (540 and 650 TFLOP/s); eight wavefronts of 64 x 64, two a
-// SIMD, 243 and 121 us (680 TFLOP/s both).
+// SIMD, 243 and 121 us (680 TFLOP/s both); the activation as an argument of the template, and worked out as act_to does, both products 384 -> 354 us
+// (373 with its code looked at for every number).
 typedef wide_gemm::Tile<128, 256, 2, 4, 3> MoeTile;
 #define MOE_BIG_ROWS MoeTile::BM
 #define MOE_BIG_K wide_gemm::BK
-template <bool GATED>
+// ACT: the activation's code, an argument of the template as in gemm_wide.hip's epilogue; -1: any, by `act_kind`.
+template <bool GATED, int ACT>
 __global__ __launch_bounds__(512, 1) void moe_big_tiles_kernel(bf16_t* __restrict__ act_out, float* __restrict__ y,
                                                                const bf16_t* __restrict__ a_rows, int64_t lda,
                                                                const bf16_t* __restrict__ w_first, const bf16_t* __restrict__ w_second,
@@ -840,7 +842,7 @@ __global__ __launch_bounds__(512, 1) void moe_big_tiles_kernel(bf16_t* __restric
       if (f < N) {
         bf16_t eight[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) eight[i] = __float2bfloat16(act_to<bf16_t>(acc[mt][i / 4][i % 4], act_kind) * acc[mt][2 + i / 4][i % 4]);
+        for (int i = 0; i < 8; ++i) eight[i] = __float2bfloat16(act_to<bf16_t>(acc[mt][i / 4][i % 4], ACT < 0 ? act_kind : ACT) * acc[mt][2 + i / 4][i % 4]);
         *reinterpret_cast<uint4*>(act_out + (int64_t)(tile.y + r) * N + f) = *reinterpret_cast<const uint4*>(eight);
       }
     } else {
@@ -930,16 +932,16 @@ extern "C" int pae_moe_experts_tiles(float* y, const void* x, int64_t ldx, const
   else {
     const int64_t up_grid = (int64_t)max_tiles * ((inter + 127) / 128) + 7, down_grid = (int64_t)max_tiles * ((hidden + 255) / 256) + 7;
     PAE_REQUIRE(up_grid < (1ll << 31) && down_grid < (1ll << 31), "experts: widths %d, %d exceed the grid", hidden, inter);
-    for (const void* kernel : {(const void*)moe_big_tiles_kernel<true>, (const void*)moe_big_tiles_kernel<false>}) {
+    auto up = act_kind == 2 ? moe_big_tiles_kernel<true, 2> : act_kind == 1 ? moe_big_tiles_kernel<true, 1> : moe_big_tiles_kernel<true, -1>;
+    auto down = moe_big_tiles_kernel<false, -1>;
+    for (const void* kernel : {(const void*)up, (const void*)down}) {
       const hipError_t err = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, MoeTile::LDS_BYTES);
       PAE_REQUIRE(err == hipSuccess, "experts: %d bytes of LDS refused: %s", MoeTile::LDS_BYTES, hipGetErrorString(err));
     }
-    moe_big_tiles_kernel<true><<<up_grid, 512, MoeTile::LDS_BYTES, stream>>>((bf16_t*)act, nullptr, (const bf16_t*)x, ldx, (const bf16_t*)gate_w,
-                                                            (const bf16_t*)up_w, order, weights, (const int4*)tiles, max_tiles, top,
-                                                            num_tokens, hidden, inter, act_kind);
-    moe_big_tiles_kernel<false><<<down_grid, 512, MoeTile::LDS_BYTES, stream>>>(nullptr, y, (const bf16_t*)act, inter, (const bf16_t*)down_w,
-                                                               nullptr, order, weights, (const int4*)tiles, max_tiles, top, num_tokens,
-                                                               inter, hidden, act_kind);
+    up<<<up_grid, 512, MoeTile::LDS_BYTES, stream>>>((bf16_t*)act, nullptr, (const bf16_t*)x, ldx, (const bf16_t*)gate_w, (const bf16_t*)up_w,
+                                                     order, weights, (const int4*)tiles, max_tiles, top, num_tokens, hidden, inter, act_kind);
+    down<<<down_grid, 512, MoeTile::LDS_BYTES, stream>>>(nullptr, y, (const bf16_t*)act, inter, (const bf16_t*)down_w, nullptr, order, weights,
+                                                         (const int4*)tiles, max_tiles, top, num_tokens, inter, hidden, act_kind);
   }
 #undef MOE_TILES
   return pae_check_launch("moe_experts_tiles");
