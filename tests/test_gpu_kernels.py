@@ -1119,3 +1119,22 @@ def test_shared_out_chunks_of_sequences_of_many_lengths(nh, nkv, hd, T, window, 
                                    hd ** -0.5, window, chunked)
         outs.append(out)
     assert bool(torch.isfinite(outs[1]).all()) and torch.equal(outs[0], outs[1])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T,H", [(65, 4), (65, 260), (70, 1536), (66, 4096)])
+def test_norm_of_many_rows_has_the_bits_of_few(dtype, T, H):
+    """More than 64 rows are normed with all partial sums asked for at once, by number of parts; up to 64 in a loop."""
+    gen = torch.Generator().manual_seed(H)
+    res, w = torch.randn(T, H, generator=gen).to(DEV), torch.randn(H, generator=gen).to(DEV)
+    for parts in (0, 1, 2, 3, 4, 5, 6, 7, 8, 9):
+        delta = torch.randn(parts, T, H, generator=gen).to(DEV) if parts else torch.randn(T, H, generator=gen).to(dtype).to(DEV)
+        weight = w.to(dtype) if parts % 2 else w
+        many, few = res.clone(), res.clone()
+        out = [torch.full((T, H), float("nan"), dtype=dtype, device=DEV) for _ in range(2)]
+        K().add_rmsnorm(many, delta, weight, 1e-6, out[0])
+        for i in range(0, T, 40):
+            part = few[i:i + 40].clone()
+            K().add_rmsnorm(part, (delta[:, i:i + 40] if parts else delta[i:i + 40]).contiguous(), weight, 1e-6, out[1][i:i + 40])
+            few[i:i + 40] = part
+        assert torch.equal(many, few) and torch.equal(*out) and not torch.equal(many, res)
