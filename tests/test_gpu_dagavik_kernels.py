@@ -440,6 +440,18 @@ def test_few_features_summed_in_float32(dtype):
     close(got, a.double() @ w.double().T + bias.double(), 1e-5, "float32 sums")
 
 
+@pytest.mark.parametrize("M,N,width", [(2000, 1, 8), (2003, 33, 512), (2001, 5, 520), (2050, 32, 1536), (2002, 40, 2040), (2000, 3, 2048), (2000, 3, 2056)])
+def test_few_features_of_many_rows_have_the_bits_of_few(M, N, width):
+    """From 2,000 rows on a workgroup takes four; below it takes one.  Widths of one to four stretches of 512, whole and ragged, and one wider."""
+    gen = torch.Generator().manual_seed(width)
+    a = torch.randn((M, width + 8), generator=gen).to(torch.bfloat16).to(DEV)[:, :width]
+    w, bias = torch.randn((N, width), generator=gen).to(torch.bfloat16).to(DEV), torch.randn(N, generator=gen).to(DEV)
+    for b in (None, bias):
+        many = K().project_f32(a, w, b)
+        assert torch.equal(many, torch.cat([K().project_f32(a[i:i + 300], w, b) for i in range(0, M, 300)]))
+    assert torch.allclose(many.cpu().double(), a.cpu().double() @ w.cpu().double().T + bias.cpu().double(), atol=1e-4)
+
+
 @pytest.mark.parametrize("H,F", [(64, 64), (128, 192), (192, 128), (256, 320), (320, 64), (64, 256), (576, 448)])
 def test_experts_of_prompts_on_large_tiles(H, F):
     """Steps of over 4,096 pairs at widths in multiples of 64: one to nine stages of 64 of k in either product, features that end
