@@ -54,25 +54,33 @@ __device__ __forceinline__ float act_of(float z, int kind) {
   return z / (1.0f + expf(-z));
 }
 
-// The same where the result is rounded to bfloat16: SiLU by the unit's own exponential and reciprocal (good to 1e-6 of the result up to |z| = 10
-// and 8e-6 up to 88, of which bfloat16 keeps 2e-3) in 7 instructions instead of about 24.  The epilogue of a product's 256 x 256 tile forms 64 a
-// lane while no matrix core works (with the gate in it, us: 2,048 x 17,920 x 1,536 101.9 -> 98.7, 8,192 of it 368 -> 350, 6,030 x 37,888 x 3,584
-// 1,191 -> 1,149, with results half as wide now ahead of the product without a gate, 353 to 370 and 1,151 to 1,176).  The reciprocal of up to 2^128 is a number below 2^-126, which the unit does not give: it is taken of a
-// 2^32nd.
+// The same where the result is rounded to bfloat16, by the unit's own exponential and reciprocal with what they round away put back.  Their error
+// against 64 bits before that rounding is no larger than act_of's (normally distributed z, 2-norm of the error over that of the results, act_of
+// and here: SiLU 3.94e-8 and 3.94e-8, GELU by tanh 3.75e-8 and 2.72e-8, by erf 3.85e-8 and 2.92e-8), in 13, 13 and 24 vector instructions beside
+// those two instead of 24, about 40 and about 40.  The epilogue of a product's 256 x 256 tile forms 64 a lane while no matrix core works: us with act_of and
+// with these, SiLU with the gate in it 2,048 x 17,920 x 1,536 104.7 and 100.6, 8,192 of it 363 and 347, 6,030 x 37,888 x 3,584 1,182 and 1,161; GELU by tanh 8,192 x
+// 17,920 x 1,536 403 and 367 (with tiles one after another as well); by erf 2,048 x 8,960 x 1,536 68.3 and 60.6, 300 rows 21.1 and 17.5.  (SiLU without what puts
+// the roundings back: 96.4, 334 and 1,130, 1e-6 of the result off at z = -8 and 8e-6 at -88.)
+
+// z / d for d from 1 on, infinity too: q z's product with the reciprocal r, `left` what that leaves of z.  The reciprocal is taken of a 2^32nd: of up
+// to 2^128 it is a number below 2^-126, which the unit does not give.
+__device__ __forceinline__ float over_one(float d) { return __builtin_amdgcn_rcpf(d * 0x1p-32f) * 0x1p-32f; }
+__device__ __forceinline__ float quotient(float left, float r, float q, float z, float d) { return __builtin_amdgcn_div_fixupf(fmaf(left, r, q), d, z); }
 __device__ __forceinline__ float silu_to_bf16(float z) {
-  const float d = 1.0f + __builtin_amdgcn_exp2f(z * -1.44269504088896341f);
-  return z * (__builtin_amdgcn_rcpf(d * 0x1p-32f) * 0x1p-32f);
+  const float c = __builtin_amdgcn_fmed3f(z, -126.f, 126.f), n = rintf(c * -1.44269504088896341f);
+  const float f = fmaf(c, -1.925963033500e-8f, fmaf(c, -1.44269504088896341f, -n));  // log2(e) in two parts
+  const float d = 1.0f + ldexpf(__builtin_amdgcn_exp2f(f), (int)n), r = over_one(d), q = z * r;
+  return quotient(fmaf(-q, d, z), r, q, z, d);
 }
-// GELU by tanh likewise (gated, 8,192 x 17,920 x 1,536 412 -> 372 us, 5,000 rows 254 -> 224; by erf below, 2,048 x 8,960 x 1,536 71.1 -> 62.3, 300 rows
-// 22.6 -> 17.7): half of 1 + tanh(u) is 1 / (1 + exp(-2 u)).  (The tanh's form takes 1 + tanh apart where it is small: at z = -4 it is
-// 4e-4 of the result off, this 2e-6.)
+// Half of 1 + tanh(u) is 1 / (1 + exp(-2 u)).  (The tanh's form takes 1 + tanh apart where it is small: at z = -4 it is 4e-4 of the result off.)  What
+// is rounded off the sum counts in what is left.
 __device__ __forceinline__ float gelu_tanh_to_bf16(float z) {
-  const float d = 1.0f + __builtin_amdgcn_exp2f(-2.30220819813f * (z + 0.044715f * z * z * z));
-  return z * (__builtin_amdgcn_rcpf(d * 0x1p-32f) * 0x1p-32f);
+  const float e = __builtin_amdgcn_exp2f(-2.30220819813f * fmaf(0.044715f * z * z, z, z)), d = 1.0f + e, r = over_one(d), q = z * r;
+  return quotient(fmaf(-q, (1.0f - d) + e, fmaf(-q, d, z)), r, q, z, d);
 }
-// GELU by the complementary error function of x = |z| / sqrt(2): erfc(x) = exp(-x^2) (1 + s q(s)), s = 0.35 x / (1 + 0.35 x), q of degree 8 fitted to
+// By the complementary error function of x = |z| / sqrt(2): erfc(x) = exp(-x^2) (1 + s q(s)), s = 0.35 x / (1 + 0.35 x), q of degree 8 fitted to
 // exp(x^2) erfc(x) over 0 <= x <= 9.4 for the least largest relative error (Lawson's iteration), 1.5e-8, 1.4e-7 with the numbers below.  What is rounded
-// in q counts by s: at z = 0 nothing of it does.  Normally distributed z, 2-norm of the error in float32 over that of the results: 2.92e-8, 1 + erf 3.85e-8.
+// in q counts by s: at z = 0 nothing of it does.
 __device__ __forceinline__ float gelu_to_bf16(float z) {
   const float a = fminf(fabsf(z), 1e30f);  // (at infinity, where half is 0, a product with it would be no number)
   const float x = 0.247487373f * a, s = x * __builtin_amdgcn_rcpf(1.0f + x);
