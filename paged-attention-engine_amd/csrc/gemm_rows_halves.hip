@@ -14,8 +14,10 @@ void launch_rows_halves(const RowsProduct& p, int side_by_side, int k_per_range,
     ROWS_HALVES(16, 1, 1, 1)
   } else if (side_by_side == 2) {
     ROWS_HALVES(8, 2, 2, 1)
-  } else {
+  } else if (grid.x <= 256) {  // a workgroup a unit: more under way in each
     ROWS_HALVES(4, 2, 2, 2)
+  } else {  // (288 tiles of 3,584 of k at 4 / 8 / 12 rows 10.4 / 11.2 / 12.3 us, in batches of two steps 10.9 / 11.8 / 13.3)
+    ROWS_HALVES(4, 1, 1, 1)
   }
 #undef ROWS_HALVES
 }

@@ -15,11 +15,12 @@
 //
 // In a recorded graph, weights from HBM, microseconds at 1 / 8 / 16 rows, before (a kernel that loaded 16 rows by 64 bytes and moved
 // every fragment to the instruction's order through LDS) and now:
-//   1.5B gate/up with the gate   13.8 / 15.1 / 17.8   11.7 / 13.4 / 16.3      0.5B gate/up   7.0 / 7.2 / 9.1     6.5 / 6.9 / 9.3
-//   1.5B down onto the residual  10.9 / 11.3 / 12.7    8.3 /  9.3 / 11.7      0.5B down      7.4 / 7.4 / 7.7     5.4 / 6.5 / 7.8
-//   1.5B QKV                      4.7 /  4.9 /  5.2    3.8 /  4.2 /  4.7      7B gate/up    50.6 / 57.0 / 64.4  45.5 / 48.5 / 67.2
-//   1.5B O onto the residual      4.8 /  5.1 /  5.6    3.9 /  4.2 /  4.8      7B down       31.3 / 37.3 / 44.1  25.2 / 26.8 / 31.2
-//   LM head of 1,536 columns       75 /   97 /  108     75 /   83 /   99
+//   0.5B gate/up with the gate    7.0 /  7.2 /  9.0    6.5 /  6.9 /  7.9      0.5B down      6.8 /  7.0 /  7.2    4.9 /  5.9 /  7.2
+//   1.5B gate/up                 13.7 / 15.5 / 18.1   12.1 / 13.1 / 14.6      1.5B down     10.1 / 10.8 / 11.8    7.6 /  9.1 / 11.3
+//   1.5B QKV                      5.8 /  6.1 /  6.8    5.0 /  5.3 /  5.9      1.5B O         4.7 /  5.0 /  5.7    3.7 /  4.0 /  4.7
+//   3B gate/up                   20.8 / 22.9 / 24.6   17.9 / 20.4 / 23.2      3B QKV         6.6 /  7.0 /  7.6    6.0 /  6.6 /  7.4
+//   7B gate/up                   52.2 / 59.2 / 64.2   48.2 / 49.8 / 60.5      7B down       33.5 / 39.0 / 44.8   26.1 / 27.0 / 32.4
+//   14B gate/up                  57.9 / 69.2 / 78.1   50.8 / 53.0 / 69.0      72B gate/up    181 /  198 /  230    163 /  172 /  196
 // (55 MB, the 1.5B gate/up's weights, are read in 10.9 us by a kernel that does nothing else.  At 16 rows the fragments of A are as many
 // as the weights', which is what is left there.)
 #pragma once
@@ -29,30 +30,22 @@
 
 // R: fragments of four weight rows a wavefront (R = 2: half of a tile of 16); MG: groups of four rows of A; NW: wavefronts, four to a
 // k range; U: steps asked for together.  Two batches of U steps take turns; ONE: a wavefront has at most U steps, all asked for at once.
+// Wavefronts a SIMD are asked for where the compiler would give sums registers twice over (16 rows: 196, two wavefronts, instead of 136 to 160;
+// at 16 rows 7B gate/up 68.3 -> 60.5 us, 0.5B 9.4 -> 7.9, 72B 218 -> 197).
 template <int R, int MG, int EPI, int NW, int U, bool ONE>
-__global__ __launch_bounds__(64 * NW) void gemm_rows_kernel(RowsProduct p, int k_per_range) {
+__global__ __launch_bounds__(64 * NW, NW > 4 ? NW / 4 : U == 4 ? 2 : MG == 4 || (ONE && MG >= 2) ? 3 : 1) void gemm_rows_kernel(RowsProduct p, int k_per_range) {
   static_assert((R == 4 || R == 2) && (NW == 4 || NW == 8 || NW == 16), "a tile of 16 weight rows or half of one; one range, two or four");
   constexpr bool PAIRS = EPI == EPI_SWIGLU || EPI == EPI_ROPE;  // the epilogue joins row r of a tile with row r + 8
   constexpr bool AHEAD = EPI == EPI_RESIDUAL || EPI == EPI_ROPE;
   __shared__ float s_part[NW][R * MG][16];
   __shared__ float s_scale[16];
   int M = p.M;
-  if (gridDim.z > 1) {  // the rows of A are shared out: this workgroup's 4 MG
+  if (EPI == EPI_F32 && gridDim.z > 1) {  // the rows of A are shared out: this workgroup's 4 MG
     const int m0 = blockIdx.z * 4 * MG;
     p.A += (int64_t)m0 * p.lda;
-    p.out = (EPI == EPI_F32 || EPI == EPI_RESIDUAL) ? (void*)((float*)p.out + (int64_t)m0 * p.ldc)
-                                                    : (void*)((bf16_t*)p.out + (int64_t)m0 * p.ldc);
+    p.out = (float*)p.out + (int64_t)m0 * p.ldc;
     M = min(4 * MG, M - m0);
     if (p.norm.row_stats) p.norm.row_stats += (int64_t)m0 * p.norm.row_stat_tiles;
-    if (EPI == EPI_RESIDUAL) {
-      p.norm.next_rows += (int64_t)m0 * p.norm.ld_next;
-      p.norm.next_stats += (int64_t)m0 * p.norm.next_stat_tiles;
-    }
-    if (EPI == EPI_ROPE) {
-      p.rope.positions += m0;
-      if (p.rope.tok_seq) p.rope.tok_seq += m0;
-      if (p.rope.cos_sin) p.rope.cos_sin += (int64_t)m0 * p.rope.rot;
-    }
   }
   const int N = p.N, K = p.K;
   const int tid = threadIdx.x, lane = tid % PAE_WAVE, wave = tid / PAE_WAVE;
@@ -178,13 +171,24 @@ __global__ __launch_bounds__(64 * NW) void gemm_rows_kernel(RowsProduct p, int k
                              AHEAD ? &ahead : nullptr, live);
 }
 
-// One wavefront's steps of a range decide how its loads are asked for: two or three steps at once, more in batches of U that take turns.
+// One wavefront's steps of a range decide how its loads are asked for: two to four steps at once, more in batches of U that take turns.
+// (Four at once, k of 1,537 to 2,048, us at 1 / 8 / 16 rows: 22,016 weight rows 18.2 / 21.1 / 25.5 -> 17.7 / 20.4 / 23.6, 2,560 6.5 / 7.2 / 8.3 -> 6.0 / 6.6 / 7.4;
+// three, at 8 rows, 17,920 weight rows 14.0 -> 13.2.)
 template <int R, int MG, int NW, int U, int EPI>
 void launch_rows_as(const RowsProduct& p, int k_per_range, dim3 grid, hipStream_t stream) {
   const int steps = (k_per_range + 511) / 512;
-  if (steps == 2) gemm_rows_kernel<R, MG, EPI, NW, 2, true><<<grid, 64 * NW, 0, stream>>>(p, k_per_range);
-  else if (steps == 3 && NW == 4 && !(R == 4 && MG == 2)) gemm_rows_kernel<R, MG, EPI, NW, 3, true><<<grid, 64 * NW, 0, stream>>>(p, k_per_range);
-  else gemm_rows_kernel<R, MG, EPI, NW, U, false><<<grid, 64 * NW, 0, stream>>>(p, k_per_range);
+  if (steps == 2) {
+    gemm_rows_kernel<R, MG, EPI, NW, 2, true><<<grid, 64 * NW, 0, stream>>>(p, k_per_range);
+    return;
+  }
+  if constexpr (NW == 4) {
+    if (steps == 3 || steps == 4) {
+      if (steps == 3) gemm_rows_kernel<R, MG, EPI, NW, 3, true><<<grid, 64 * NW, 0, stream>>>(p, k_per_range);
+      else gemm_rows_kernel<R, MG, EPI, NW, 4, true><<<grid, 64 * NW, 0, stream>>>(p, k_per_range);
+      return;
+    }
+  }
+  gemm_rows_kernel<R, MG, EPI, NW, U, false><<<grid, 64 * NW, 0, stream>>>(p, k_per_range);
 }
 
 template <int R, int MG, int NW, int U>

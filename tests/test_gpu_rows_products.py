@@ -20,7 +20,7 @@ def operands(M, N, K_, seed):
 
 
 @pytest.mark.parametrize("M", [1, 4, 5, 9, 13, 16])
-@pytest.mark.parametrize("N,K_", [(8, 8), (24, 136), (1000, 1032), (72, 2048), (6400, 392), (10272, 264), (10272, 1544), (3344, 648)])
+@pytest.mark.parametrize("N,K_", [(8, 8), (24, 136), (1000, 1032), (72, 2048), (6400, 392), (10272, 264), (10272, 1544), (3344, 648), (2568, 2048), (9736, 1536), (4616, 2568)])
 def test_plain_and_float32_sums(M, N, K_):
     """Also several ranges: tickets (bfloat16) and partial sums (float32)."""
     a, w, want, gen = operands(M, N, K_, M + N + K_)
