@@ -658,8 +658,12 @@ def skinny_supported(a: torch.Tensor, w: torch.Tensor) -> bool:
 
 
 def skinny_splits(N: int, K: int, M: int = 1, w: Optional[torch.Tensor] = None) -> int:
-    """k ranges for a product whose consumer adds float32 partials: one up to 16 rows (1.5B down with the norm behind it
-    at 8 rows in five ranges 8.7 + 4.1 us, in one 9.4 + 3.3), beyond that enough workgroups to fill the chip.
+    """k ranges for a product whose consumer adds float32 partials.  Up to 16 rows from the sizes alone: two workgroups a unit of 1,536 of k or
+    more, and four ranges of what one range would give some units twice as much of as others (with the norm behind it, us at 1 / 8 / 16 rows, one
+    range and what is taken: 0.5B down 8.1 / 9.5 / 11.3 and 8.1 / 8.9 / 9.5 in three, 1.5B down 11.1 / 12.8 / 16.2 and 11.6 / 12.4 / 13.5 in five, 3B down 14.2 /
+    15.7 / 19.5 and 14.4 / 15.2 / 17.7 in four, 7B down 30.3 / 31.2 / 52.4 and 30.7 / 32.5 / 41.8 in two, 14B down 32.9 / 37.3 / 42.8 and 33.2 / 34.4 / 38.9 in four, 32B
+    down 59 / 68 / 84 and 58 / 59 / 74 in four; but 3B O 7.0 / 7.6 / 8.1 and 7.3 / 8.0 / 8.4 in two, 6,144 x 16,384 44 / 46 / 56 and 51 / 49 / 54 in four).
+    Beyond that enough workgroups to fill the chip.
     `w`: the weights, where they are at hand (see `_streamed_splits`)."""
     return _skinny_splits(N, K, M, _off_16_bytes(w))
 
@@ -676,8 +680,20 @@ _rule_of_sizes = functools.lru_cache(maxsize=4096)
 @_rule_of_sizes
 def _skinny_splits(N: int, K: int, M: int, off: bool) -> int:
     if M <= SAME_ORDER_MAX_ROWS:
-        return 1
+        tiles = -(-N // 16)
+        wanted = max(1, min(512 // tiles, K // 1536, 8)) if tiles <= 256 else 4 if K >= 8192 and _evens_out(tiles, 4) else 1
+        return _whole_ranges(K, wanted)
     return _streamed_splits(N, K, M, _part_ranges(N, K, M), off, parts=True)
+
+
+def _whole_ranges(K: int, wanted: int) -> int:
+    """`wanted` ranges of k as the rounding of their length to 128 leaves them."""
+    return -(-K // (-(-(-(-K // wanted)) // 128) * 128))
+
+
+def _evens_out(tiles: int, ranges: int) -> bool:
+    """Whether that many ranges of k take a third or more off what the busiest of 256 compute units has of workgroups of 16 weight rows."""
+    return 3 * -(-ranges * tiles // 256) <= 2 * ranges * -(-tiles // 256)
 
 
 def _part_ranges(N: int, K: int, M: int) -> int:
@@ -737,7 +753,10 @@ def residual_splits(N: int, K: int, M: int = 1, w: Optional[torch.Tensor] = None
     itself or as a phase of a decode program.  Two or four ranges run side by side in one workgroup of eight or sixteen
     wavefronts, with no tickets and no trip to memory for partial sums: what a workgroup of few weight rows and much of k has to
     read then comes to more wavefronts (1.5B down at 1 / 8 / 16 rows in one range 7.4 / 8.7 / 11.9 us, in four 6.9 / 8.8 / 10.6;
-    7B down 24.9 / 30.4 / 41.5, in two 24.9 / 25.2 / 31.7, in four 24.5 / 26.6 / 37.1; sums alone)."""
+    7B down 26.0 / 27.6 / 40.0, in two 25.1 / 26.2 / 31.0; sums alone).  Wider ones, in one range or, where that leaves some units twice the
+    workgroups of others, in three by ticket (14B down, 320 workgroups of 16 weight rows, one 31.9 / 34.9 / 38.0, two side by side 30.3 / 33.9 / 41.4,
+    three 29.4 / 29.8 / 34.6; 32B down 60 / 66 / 79, 60 / 65 / 77, 53 / 55 / 70; 14B O 13.7 / 14.9 / 17.8, 12.9 / 15.2 / 18.1, 13.7 / 14.2 / 17.3; 72B down, 512
+    workgroups, 86 / 89 / 99, 86 / 89 / 100, 89 / 92 / 103; 72B O 28.0 / 29.0 / 31.8, 27.9 / 30.5 / 33.1, 29.6 / 30.2 / 32.2)."""
     return _residual_splits(N, K, M, _off_16_bytes(w))
 
 
@@ -755,8 +774,8 @@ def _residual_splits(N: int, K: int, M: int, off: bool) -> int:
         # 21.8 / 28.4 with five; 7B down: eight, 35 / 47 us; 14B: six, 33 / 44; 14B O: six, 19 / 27 against 27 / 37
         # with two)
         return _streamed_splits(N, K, M, _part_ranges(N, K, M), off)
-    wanted = 4 if N <= 3072 and K >= 4096 else 2 if N <= 4096 and K >= 512 else 1
-    return -(-K // (-(-(-(-K // wanted)) // 128) * 128))
+    wanted = 4 if N <= 3072 and K >= 4096 else 2 if N <= 4096 and K >= 512 else 3 if K >= 4096 and _evens_out(-(-N // 16), 3) else 1
+    return _whole_ranges(K, wanted)
 
 
 def gemm_skinny(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,

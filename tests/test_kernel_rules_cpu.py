@@ -253,3 +253,13 @@ def test_the_polynomial_of_gelu_is_the_one_that_was_fitted():
     for c in at[1:]:
         value = value * s + c
     assert len(q) == 9 and ((2 * (0.5 + s * value) / torch.special.erfcx(x) - 1).abs() < 3e-7).all()
+
+
+@pytest.mark.parametrize("N,K_", [(896, 4864), (1536, 8960), (3200, 8640), (3584, 18944), (5120, 5120), (5120, 13824), (5120, 27648), (8192, 29568), (9216, 300)])
+def test_ranges_of_few_rows_follow_from_the_weights_alone(N, K_):
+    """Up to 16 rows a row's sums are the same bits whatever it is batched with; no range is empty."""
+    for rule in (K.residual_splits, K.skinny_splits):
+        ranges = {rule(N, K_, M) for M in range(1, 17)}
+        assert len(ranges) == 1
+        r = ranges.pop()
+        assert 1 <= r <= 8 and (r - 1) * (-(-(-(-K_ // r)) // 128) * 128) < K_
