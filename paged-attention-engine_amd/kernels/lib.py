@@ -775,7 +775,20 @@ def _residual_splits(N: int, K: int, M: int, off: bool) -> int:
         # with two)
         return _streamed_splits(N, K, M, _part_ranges(N, K, M), off)
     wanted = 4 if N <= 3072 and K >= 4096 else 2 if N <= 4096 and K >= 512 else 3 if K >= 4096 and _evens_out(-(-N // 16), 3) else 1
+    # layers whose other products a decode program has the LDS for: as many ranges, by ticket, as it has the LDS for this one's as well
+    # (at most four of the wider, else what two workgroups a unit come to)
+    longest = _program_range()
+    if N <= longest and longest * wanted < K <= longest * (4 if N > 3072 else min(8, 512 // -(-N // 16))):
+        wanted = -(-K // longest)
     return _whole_ranges(K, wanted)
+
+
+def _program_range() -> int:
+    """The longest range of k whose activations a decode program has the LDS for."""
+    steps = 1
+    while program_takes_product(SAME_ORDER_MAX_ROWS, 128 * (steps + 1), 1):
+        steps += 1
+    return 128 * steps
 
 
 def gemm_skinny(out: torch.Tensor, a: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,

@@ -255,6 +255,20 @@ def test_the_polynomial_of_gelu_is_the_one_that_was_fitted():
     assert len(q) == 9 and ((2 * (0.5 + s * value) / torch.special.erfcx(x) - 1).abs() < 3e-7).all()
 
 
+def test_ranges_of_k_leave_a_decode_program_the_layers_that_it_took():
+    """A program's LDS holds a range's activations: the down product of a layer whose gate product fits has ranges that fit too, up to eight of
+    them, or four of wider ones."""
+    fits = lambda k, splits: K.program_takes_product(16, k, splits)
+    longest = max(k for k in range(128, 8192, 128) if fits(k, 1))
+    assert K._program_range() == longest and fits(longest, 1) and not fits(longest + 128, 1)
+    for hidden in range(64, longest + 1, 64):
+        tiles = -(-hidden // 16)
+        most = 4 if hidden > 3072 else min(8, 512 // tiles)
+        for ff in {longest * most, longest * most - 8, 4 * hidden, 8 * hidden // 3 // 8 * 8, 5 * hidden, 8960}:
+            if ff <= longest * most:
+                assert fits(ff, K.residual_splits(hidden, ff, 16)), (hidden, ff)
+
+
 @pytest.mark.parametrize("N,K_", [(896, 4864), (1536, 8960), (3200, 8640), (3584, 18944), (5120, 5120), (5120, 13824), (5120, 27648), (8192, 29568), (9216, 300)])
 def test_ranges_of_few_rows_follow_from_the_weights_alone(N, K_):
     """Up to 16 rows a row's sums are the same bits whatever it is batched with; no range is empty."""
