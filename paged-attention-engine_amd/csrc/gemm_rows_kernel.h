@@ -28,6 +28,8 @@
 #include "api.h"
 #include "gemm_rows.h"
 
+#include <type_traits>
+
 // R: fragments of four weight rows a wavefront (R = 2: half of a tile of 16); MG: groups of four rows of A; NW: wavefronts, four to a
 // k range; U: steps asked for together.  Two batches of U steps take turns; ONE: a wavefront has at most U steps, all asked for at once.
 // Wavefronts a SIMD are asked for where the compiler would give sums registers twice over (16 rows: 196, two wavefronts, instead of 136 to 160;
@@ -40,12 +42,24 @@ __global__ __launch_bounds__(64 * NW, NW > 4 ? NW / 4 : U == 4 ? 2 : MG == 4 || 
   __shared__ float s_part[NW][R * MG][16];
   __shared__ float s_scale[16];
   int M = p.M;
-  if (EPI == EPI_F32 && gridDim.z > 1) {  // the rows of A are shared out: this workgroup's 4 MG
+  // Rows of A shared out: this workgroup's 4 MG.  (Only float32 sums are asked for so.  The residual's and the rotation's arguments are then fetched with
+  // the others at the start and not, one trip more, behind the products: 1.5B O at 1 row 3.9 -> 3.7 us; the gate's kernel is better off without, 0.5B at
+  // 8 rows 6.9 -> 6.7.)
+  if ((AHEAD || EPI == EPI_F32) && gridDim.z > 1) {
     const int m0 = blockIdx.z * 4 * MG;
     p.A += (int64_t)m0 * p.lda;
-    p.out = (float*)p.out + (int64_t)m0 * p.ldc;
+    p.out = EPI == EPI_ROPE ? (void*)((bf16_t*)p.out + (int64_t)m0 * p.ldc) : (void*)((float*)p.out + (int64_t)m0 * p.ldc);
     M = min(4 * MG, M - m0);
     if (p.norm.row_stats) p.norm.row_stats += (int64_t)m0 * p.norm.row_stat_tiles;
+    if (EPI == EPI_RESIDUAL) {
+      p.norm.next_rows += (int64_t)m0 * p.norm.ld_next;
+      p.norm.next_stats += (int64_t)m0 * p.norm.next_stat_tiles;
+    }
+    if (EPI == EPI_ROPE) {
+      p.rope.positions += m0;
+      if (p.rope.tok_seq) p.rope.tok_seq += m0;
+      if (p.rope.cos_sin) p.rope.cos_sin += (int64_t)m0 * p.rope.rot;
+    }
   }
   const int N = p.N, K = p.K;
   const int tid = threadIdx.x, lane = tid % PAE_WAVE, wave = tid / PAE_WAVE;
@@ -77,7 +91,8 @@ __global__ __launch_bounds__(64 * NW, NW > 4 ? NW / 4 : U == 4 ? 2 : MG == 4 || 
     for (int g = 0; g < MG; ++g) acc[r][g] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
   // Loads are unconditional, from clamped addresses (the compiler counts the loads in flight behind the one it waits for, and where one
-  // may or may not have been issued it waits for all); a lane past the end of the range zeroes its weights.
+  // may or may not have been issued it waits for all); a lane past the end of the range zeroes its weights, and, where a wavefront's last batch may
+  // hold whole steps behind it, its numbers of A (zero times an infinite one would be no number).
   constexpr int KW = 128 * 4, STEP = KW * U;
   const bf16x8 zero = {};
   struct Batch {
@@ -94,18 +109,23 @@ __global__ __launch_bounds__(64 * NW, NW > 4 ? NW / 4 : U == 4 ? 2 : MG == 4 || 
       for (int g = 0; g < MG; ++g) b.af[u][g] = *reinterpret_cast<const bf16x8*>(arow[g] + kc);
     }
   };
-  auto multiply = [&](Batch& b, int kb) {
+  auto multiply = [&](const Batch& b, int kb, auto last) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const bool in = kb + KW * u + 8 * piece < k_hi;  // K and the bounds are multiples of 8: a lane's eight numbers are all in or all out
+      bf16x8 a[MG];
+#pragma unroll
+      for (int g = 0; g < MG; ++g) a[g] = in || U == 1 || !decltype(last)::value ? b.af[u][g] : zero;
 #pragma unroll
       for (int r = 0; r < R; ++r) {
         const bf16x8 w = in ? b.wf[u][r] : zero;
 #pragma unroll
-        for (int g = 0; g < MG; ++g) acc[r][g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, b.af[u][g], acc[r][g], 0, 0, 0);
+        for (int g = 0; g < MG; ++g) acc[r][g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, a[g], acc[r][g], 0, 0, 0);
       }
     }
   };
+  const std::false_type inside;
+  const std::true_type last;
   int kb = k_lo + 128 * (wave % 4);  // the same in every lane of a wavefront: the branches on it are uniform
   // what the epilogue reads beside the sums, and the rows' shares of the sums of squares, are asked for before the first batch is waited for
   EpilogueAhead<1> ahead;
@@ -116,24 +136,24 @@ __global__ __launch_bounds__(64 * NW, NW > 4 ? NW / 4 : U == 4 ? 2 : MG == 4 || 
   row_scales_to_lds<1>(s_scale, p.norm, M, K, tid, [&] { load(b0, kb); });
   if (AHEAD && wave == 0) ask_epilogue<1, EPI, false>(ahead, tile, p.out, p.ldc, M, N, p.rope, p.norm, live);
   if (ONE) {
-    multiply(b0, kb);
+    multiply(b0, kb, last);
   } else {
     Batch b1;
     int batches = kb < k_hi ? (k_hi - kb + STEP - 1) / STEP : 0;  // of this wavefront
     while (batches >= 3) {
       load(b1, kb + STEP);
-      multiply(b0, kb);
+      multiply(b0, kb, inside);
       load(b0, kb + 2 * STEP);
-      multiply(b1, kb + STEP);
+      multiply(b1, kb + STEP, inside);
       kb += 2 * STEP;
       batches -= 2;
     }
     if (batches == 2) {
       load(b1, kb + STEP);
-      multiply(b0, kb);
-      multiply(b1, kb + STEP);
+      multiply(b0, kb, inside);
+      multiply(b1, kb + STEP, last);
     } else if (batches == 1) {
-      multiply(b0, kb);
+      multiply(b0, kb, last);
     }
   }
 #pragma unroll

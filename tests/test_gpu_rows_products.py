@@ -94,3 +94,24 @@ def test_a_row_is_the_same_bits_in_either_share_of_weight_rows(M):
     K.gemm_skinny(alone, a[M - 1:], many.to(DEV), None, K.EPI_F32)
     K.gemm_skinny(among, a, many.to(DEV), None, K.EPI_F32)
     assert torch.equal(alone[0], among[M - 1])
+
+
+@pytest.mark.parametrize("M", [1, 8, 12, 16])
+@pytest.mark.parametrize("N,K_,ranges", [(2048, 1536, 1), (2560, 2048, 1), (72, 896, 1), (9736, 1536, 1), (40, 1536, 3), (4616, 2560, 1), (1536, 1536, 2), (3584, 3584, 2), (1544, 8960, 4)])
+def test_an_infinite_number_of_a_row_is_added_once(M, N, K_, ranges):
+    """Steps that reach past a range of k multiply nothing there: what stands at the row's end, or in another range, does not come in as zero times it."""
+    a, w, _, _ = operands(M, N, K_, M)
+    w[w == 0] = 0.1
+    want = torch.zeros(M, N, dtype=torch.float64)
+    for m, at in enumerate((K_ - 1, 0, K_ - 8, K_ // 2 + 1, K_ // 2 - 130)):
+        if m < M:
+            a[m, at] = float("inf")
+            want[m] = w[:, at].double().sign() * float("inf")
+    d_a, d_w = a.to(DEV), w.to(DEV)
+    out = torch.zeros(M, N, device=DEV)
+    if ranges == 1:
+        K.gemm_skinny(out, d_a, d_w, None, K.EPI_F32)
+    else:
+        K.gemm_skinny(out, d_a, d_w, None, K.EPI_RESIDUAL, ranges, following=(torch.empty(M, N, dtype=torch.bfloat16, device=DEV), torch.ones(N, device=DEV),
+                                                                              torch.empty(M, K.fine_stat_tiles(N, M), device=DEV)))
+    assert torch.equal(out.cpu().double()[: min(M, 5)], want[: min(M, 5)]) and bool(out[5:].isfinite().all())
