@@ -148,10 +148,12 @@ __device__ __forceinline__ bool grid_barrier(ProgBarrier* bar, unsigned& epoch, 
 // are added in wavefront order through LDS, exactly as gemm_rows.hip's kernels add them.
 //
 // Weights do not depend on what a barrier waits for, so a wavefront always has its next chunk of them
-// (up to PROG_S of its k steps, 12 KB a wavefront) on the way: the next tile's while it multiplies the
-// current one, and, across the barrier, the first PROG_AHEAD steps of its first tile of the next phase.
-// `coming` carries them from one phase to the next.
-#define PROG_S 3  // most k steps of a wavefront whose weights are asked for together (a chunk): four fragments each
+// (up to PROG_S of its k steps, 8 KB a wavefront) on the way, step by step in the places of the one that it multiplies, and, across the barrier, the first PROG_AHEAD steps of its first tile of the next phase.
+// `coming` carries them from one phase to the next.  (Sixteen rows' sums are 64 registers, a step's weights 16: with three steps 33 registers go to
+// memory and back, with a second set of places for the next chunk and a form of its own for short ranges 158.  A decode step as a program, 0.5B at one
+// request / 1.5B at 8, us: that 2,789 / 4,512, three steps 1,534 / 2,800, two 1,424 / 2,688; 16 rows by 64 bytes a load, moved to the
+// instruction's order, before it 1,694 / 2,797.)
+#define PROG_S 2  // most k steps of a wavefront whose weights are asked for together (a chunk): four fragments each
 #define PROG_AHEAD 1  // steps of its first chunk of the next phase that a wavefront asks for before the barrier
 #define PROG_STEP (4 * 128)  // from one k step of a wavefront to its next
 
@@ -164,16 +166,16 @@ struct Chunk {
   int kb, K, steps;
 };
 
+__device__ __forceinline__ void ask_step(bf16x8 (&frag)[4], const Chunk& c, int u) {
+  const int uu = u < c.steps ? u : (c.steps > 0 ? c.steps - 1 : 0);
+  const int k = c.kb + PROG_STEP * uu + 8 * piece_of(threadIdx.x % PAE_WAVE);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) frag[r] = *reinterpret_cast<const bf16x8*>(c.row[r] + (k < c.K - 8 ? k : c.K - 8));
+}
 template <int S, int FROM = 0>
 __device__ __forceinline__ void ask_chunk(bf16x8 (&frag)[PROG_S][4], const Chunk& c) {
-  const int piece = piece_of(threadIdx.x % PAE_WAVE);
 #pragma unroll
-  for (int u = FROM; u < S; ++u) {
-    const int uu = u < c.steps ? u : (c.steps > 0 ? c.steps - 1 : 0);
-    const int k = c.kb + PROG_STEP * uu + 8 * piece;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) frag[u][r] = *reinterpret_cast<const bf16x8*>(c.row[r] + (k < c.K - 8 ? k : c.K - 8));
-  }
+  for (int u = FROM; u < S; ++u) ask_step(frag[u], c, u);
 }
 
 // Which tiles of which k range quad `quad` of this workgroup takes: tile first, first + stride, ...
@@ -207,13 +209,12 @@ __device__ __forceinline__ const bf16_t* weight_row(const ProgPhase& ph, int til
   return in_memory(ph.W) + (int64_t)(n < ph.N ? n : ph.N - 1) * ph.K;  // rows past N are loaded from the last row and never stored
 }
 
-// k steps of 128 that one wavefront makes in a k range, at most, and whether its chunks are the short kind
+// k steps of 128 that one wavefront makes in a k range, at most
 __device__ __forceinline__ int steps_of(const ProgPhase& ph) { return (min(ph.k_per_split, ph.K) + PROG_STEP - 1) / PROG_STEP; }
-__device__ __forceinline__ bool short_chunks(const ProgPhase& ph) { return steps_of(ph) <= 1; }
 
 // Chunk `c` of wavefront `wq` of a quad for `tile` in k range `range`.
 __device__ __forceinline__ Chunk chunk_of(const ProgPhase& ph, int tile, int range, int c, int wq) {
-  const int S = short_chunks(ph) ? 1 : PROG_S;
+  constexpr int S = PROG_S;
   const int k_lo = range * ph.k_per_split, k_hi = min(ph.K, k_lo + ph.k_per_split);
   const int kb = k_lo + 128 * wq + PROG_STEP * S * c;
   const int left = kb < k_hi ? (k_hi - kb + PROG_STEP - 1) / PROG_STEP : 0;
@@ -235,10 +236,11 @@ __device__ __forceinline__ void product_phase(const ProgPhase& ph, const ProgPha
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PAE_WAVE), quad = wave / 4, wq = wave % 4;
   const int M = ph.M, N = ph.N, K = ph.K, splits = ph.splits;
   const int tiles = (N + 15) / 16;
-  const int g4 = lane / 16, piece = piece_of(lane), groups_of_rows = (M + 3) / 4;
-  const bool brief = short_chunks(ph);  // the same in the whole grid
-  const int S = brief ? 1 : PROG_S, chunks_a_tile = (steps_of(ph) + S - 1) / S;
+  const int g4 = lane / 16, piece = piece_of(lane);
+  constexpr int S = PROG_S;
+  const int chunks_a_tile = (steps_of(ph) + S - 1) / S;
   float* s_scale = quad_lds + 2 * PROG_SUMS;  // [16], behind the two sets of partial sums
+  constexpr int ROW_GROUPS = PROG_MAX_ROWS / 4;
   const bf16x8 zero = {};
   const int groups = (int)gridDim.x, group = (int)blockIdx.x;
   const int range_turns = groups >= splits ? 1 : (splits - group + groups - 1) / groups;
@@ -280,7 +282,7 @@ __device__ __forceinline__ void product_phase(const ProgPhase& ph, const ProgPha
 #pragma unroll
       for (int q = 0; q < AT_ONCE; ++q) {
         const int idx = base + q * PROG_THREADS, m = idx / padded, c = idx % padded;
-        if (idx < M * padded) a_lds[(c / 16 * groups_of_rows + m / 4) * PAE_WAVE + c % 16 / 4 * 16 + m % 4 * 4 + c % 4] = v[q];
+        if (idx < M * padded) a_lds[(c / 16 * ROW_GROUPS + m / 4) * PAE_WAVE + c % 16 / 4 * 16 + m % 4 * 4 + c % 4] = v[q];
       }
     }
     __syncthreads();
@@ -288,9 +290,8 @@ __device__ __forceinline__ void product_phase(const ProgPhase& ph, const ProgPha
     if (rest_to_ask) {  // the same in the whole workgroup
       rest_to_ask = false;
       if (!has_coming) {
-        if (brief) ask_chunk<1>(coming, first_chunk);
-        else ask_chunk<PROG_S>(coming, first_chunk);
-      } else if (!brief) {
+        ask_chunk<PROG_S>(coming, first_chunk);
+      } else {
         ask_chunk<PROG_S, PROG_AHEAD>(coming, first_chunk);
       }
       // what the folded norm owes the rows: the quad's threads together, into the quad's LDS (read after the
@@ -299,29 +300,20 @@ __device__ __forceinline__ void product_phase(const ProgPhase& ph, const ProgPha
     }
     const int rounds = (tiles + sh.stride - 1) / sh.stride;  // the same for the quads of a workgroup
     const int total = rounds * chunks_a_tile;
-    f32x4 acc[4][4];
+    f32x4 acc[4][ROW_GROUPS];
     EpilogueAhead<1> pre = {};
     for (int j = 0; j < total; ++j) {
-      bf16x8 cur[PROG_S][4];
-#pragma unroll
-      for (int u = 0; u < PROG_S; ++u)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) cur[u][r] = coming[u][r];
-      // the chunk after this one, of this range or the next
-      if (j + 1 < total || turn + 1 < range_turns) {
-        Chunk c = nothing;
-        if (j + 1 < total) in_turn(turn, j + 1, c);
-        else in_turn(turn + 1, 0, c);
-        if (brief) ask_chunk<1>(coming, c);
-        else ask_chunk<PROG_S>(coming, c);
-      }
+      // the chunk after this one, of this range or the next, is asked for step by step in the places of this one's
+      Chunk c = nothing;
+      if (j + 1 < total) in_turn(turn, j + 1, c);
+      else in_turn(turn + 1, 0, c);
       const int tile = sh.first + j / chunks_a_tile * sh.stride, c_in_tile = j % chunks_a_tile;
       const bool live = tile < tiles;  // the same in every lane of the quad
       if (c_in_tile == 0) {
 #pragma unroll
         for (int r = 0; r < 4; ++r)
 #pragma unroll
-          for (int g = 0; g < 4; ++g) acc[r][g] = (f32x4){0.f, 0.f, 0.f, 0.f};
+          for (int g = 0; g < ROW_GROUPS; ++g) acc[r][g] = (f32x4){0.f, 0.f, 0.f, 0.f};
         // what the tile's epilogue reads beside the sums is asked for now (by the wavefront that runs it)
         if (live && wq == 0) {
           if (ph.epilogue == EPI_ROPE) ask_row<1, EPI_ROPE>(pre, M, in_memory(ph.rope));
@@ -329,29 +321,26 @@ __device__ __forceinline__ void product_phase(const ProgPhase& ph, const ProgPha
           if (ph.epilogue == EPI_RESIDUAL) ask_epilogue<1, EPI_RESIDUAL, true>(pre, tile, in_memory(ph.out), ph.ldc, M, N, SkinnyRope{}, in_memory(ph.norm));
         }
       }
-      if (live) {
-        const int kb = k_lo + 128 * wq + PROG_STEP * S * c_in_tile;
-        auto multiply = [&](auto steps) {
+      const int kb = k_lo + 128 * wq + PROG_STEP * S * c_in_tile;
+      auto multiply = [&](auto steps) {
 #pragma unroll
-          for (int u = 0; u < decltype(steps)::value; ++u) {
-            // one step's operands at a time (read ahead for a whole chunk they would not fit the registers)
-            if (u > 0) asm volatile("" ::: "memory");
-            const int k = kb + PROG_STEP * u;  // this wavefront's step: k .. k + 127
-            const bool kok = k + 8 * piece < k_hi;
-            // (past the range the step's place in LDS is the last one's: its weights are zero)
-            const bf16x8* at = a_lds + (min(k, k_hi - 1) - k_lo) / 128 * groups_of_rows * PAE_WAVE + lane;
+        for (int u = 0; u < decltype(steps)::value; ++u) {
+          // one step's operands at a time (read ahead for a whole chunk they would not fit the registers)
+          if (u > 0) asm volatile("" ::: "memory");
+          const int k = kb + PROG_STEP * u;  // this wavefront's step: k .. k + 127
+          const bool kok = k + 8 * piece < k_hi;
+          // (past the range the step's place in LDS is the last one's: weights and numbers of A are zero)
+          const bf16x8* at = a_lds + (min(k, k_hi - 1) - k_lo) / 128 * ROW_GROUPS * PAE_WAVE + lane;
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-              if (g >= groups_of_rows) break;
-              const bf16x8 a = at[g * PAE_WAVE];
+          for (int g = 0; g < ROW_GROUPS; ++g) {  // (rows past M are whatever LDS held, and are not stored)
+            const bf16x8 a = kok ? at[g * PAE_WAVE] : zero;
 #pragma unroll
-              for (int r = 0; r < 4; ++r) acc[r][g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kok ? cur[u][r] : zero, a, acc[r][g], 0, 0, 0);
-            }
+            for (int r = 0; r < 4; ++r) acc[r][g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kok ? coming[u][r] : zero, a, acc[r][g], 0, 0, 0);
           }
-        };
-        if (brief) multiply(std::integral_constant<int, 1>{});
-        else multiply(std::integral_constant<int, PROG_S>{});
-      }
+          ask_step(coming[u], c, u);
+        }
+      };
+      multiply(std::integral_constant<int, PROG_S>{});
       if (stamps && threadIdx.x == 0 && turn == 0 && j == 0) stamps[3] = wall_clock64();
       if (c_in_tile + 1 < chunks_a_tile) continue;
       // the tile's sums: the four wavefronts' in wavefront order, then the k ranges', then the epilogue
@@ -688,7 +677,7 @@ extern "C" int pae_program_max_rows() { return PROG_MAX_ROWS; }
 static int quad_bytes_of_product() { return (2 * PROG_SUMS + 16) * (int)sizeof(float); }
 
 // Bytes of LDS that the activations of one k range of a product take in a workgroup: `rows` rows of one
-// range, whole k steps of 32.
+// range, whole k steps of 128.
 extern "C" int pae_program_activation_bytes(int rows, int K, int splits) {
   if (rows < 1 || K < 1 || splits < 1) return 0;
   int k_per_split = (K + splits - 1) / splits;

@@ -89,8 +89,8 @@ def test_a_decode_program_at_the_real_layer_widths_and_sixteen_rows(tmp_path):
 
 
 def test_a_decode_program_whose_wavefronts_take_a_tile_in_several_chunks():
-    """With a width of 2,560 and 6,912 between, a k range is longer than the 14 k steps a wavefront asks
-    for at once (20 for QKV and gate/up, 18 for down's three ranges): a tile's weights then come in two
+    """With a width of 2,560 and 6,912 between, a k range is longer than the two k steps of 512 a wavefront asks
+    for at once (five for QKV and gate/up, four for down's four ranges): a tile's weights then come in three or two
     chunks, the next always on the way.  (Wider still, and a range's activations no longer fit LDS beside
     the attention's: the 7B widths are refused, and run kernel by kernel.)"""
     wider = dict(WIDE, num_hidden_layers=1, hidden_size=2560, num_attention_heads=20, num_key_value_heads=4,
