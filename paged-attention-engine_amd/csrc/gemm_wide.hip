@@ -275,6 +275,11 @@ __device__ __forceinline__ void small_tile(const Product& p, char* lds, int m0, 
 using Half = Tile<128, 256, 2, 4, 3>;     // of a tile of 256 x 256, by the same eight wavefronts
 using Quarter = Tile<128, 128, 2, 4, 4>;
 
+// Whether a workgroup takes one tile of 256 x 256 after another (see below).  Not with rotated heads, whose epilogue has no registers left for it: 28 bytes
+// a lane went to memory and back, and it gained nothing (us, in turns and not: 6,030 x 4,608 x 3,584 165.6 and 165.2, 8,192 x 7,168 x 5,120 427 and 427).
+template <int MODE>
+constexpr bool in_turns() { return MODE != wide_gemm::ROTATED; }
+
 // parts: into how many each tile behind the whole ones is cut (1, 2 or 4)
 template <int MODE, int ACT, int PARTS>
 __global__ __launch_bounds__(512, 2) void wide_large_kernel(Product p) {
@@ -282,7 +287,7 @@ __global__ __launch_bounds__(512, 2) void wide_large_kernel(Product p) {
   const int lane = threadIdx.x % PAE_WAVE;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PAE_WAVE);
   int tm, tn;
-  const int ranges = MODE == wide_gemm::SUMS ? p.whole * p.splits : p.whole, together = min(ranges, UNITS);
+  const int ranges = MODE == wide_gemm::SUMS ? p.whole * p.splits : p.whole, together = in_turns<MODE>() ? min(ranges, UNITS) : ranges;
   if (PARTS > 1 && (int)blockIdx.x >= together) {
     const int rest = (p.row_tiles * p.col_tiles - p.whole) * PARTS, at = in_row(blockIdx.x - together, rest);
     place_of(p.whole + at / PARTS, p.row_tiles, p.col_tiles, p.strip, tm, tn);
@@ -337,8 +342,9 @@ __global__ __launch_bounds__(512, 2) void wide_large_kernel(Product p) {
     Large::run<STORES>(acc, wide_lds, src, stages, stored);
     stored = m0 + 256 <= p.M && n0 + 256 <= p.N;
     const int row0 = m0 + wave / Large::WN * Large::PM, col0 = n0 + wave % Large::WN * Large::PN, of = split;
-    if (i + together < ranges) begin(i + together);
+    if (in_turns<MODE>() && i + together < ranges) begin(i + together);
     finish<MODE, ACT>(p, acc, row0, col0, of);
+    if (!in_turns<MODE>()) return;
   }
 }
 
@@ -375,8 +381,9 @@ int launch_small(Product p, hipStream_t stream) {
   return launch(wide_small_kernel<MODE, ACT, T>, p, (int64_t)p.row_tiles * p.col_tiles * p.splits, T::WAVES * 64, T::LDS_BYTES, stream);
 }
 
-// Workgroups of tiles of 256 x 256: one a unit.
-int64_t together(int64_t tiles) { return tiles < UNITS ? tiles : UNITS; }
+// Workgroups of tiles of 256 x 256.
+template <int MODE>
+int64_t together(int64_t tiles) { return in_turns<MODE>() && tiles > UNITS ? UNITS : tiles; }
 
 template <int MODE, int ACT>
 int launch_large(Product p, hipStream_t stream) {
@@ -388,15 +395,15 @@ int launch_large(Product p, hipStream_t stream) {
   if constexpr (MODE == wide_gemm::SUMS) {
     p.whole = (int)tiles;
     PAE_REQUIRE(tiles * p.splits < (1ll << 30), "wide product: too many tiles");
-    return launch(wide_large_kernel<MODE, ACT, 1>, p, together(tiles * p.splits), 512, Large::LDS_BYTES, stream);
+    return launch(wide_large_kernel<MODE, ACT, 1>, p, together<MODE>(tiles * p.splits), 512, Large::LDS_BYTES, stream);
   }
   const int rest = (int)(tiles % UNITS), parts = rest == 0 || rest > UNITS / 2 ? 1 : rest > UNITS / 4 ? 2 : 4;
   p.whole = (int)(parts == 1 ? tiles : tiles - rest);
   constexpr int LDS = Large::LDS_BYTES > Half::LDS_BYTES ? Large::LDS_BYTES : Half::LDS_BYTES;
   static_assert(Quarter::LDS_BYTES <= LDS, "room for every part");
-  if (parts == 1) return launch(wide_large_kernel<MODE, ACT, 1>, p, together(tiles), 512, Large::LDS_BYTES, stream);
-  if (parts == 2) return launch(wide_large_kernel<MODE, ACT, 2>, p, together(p.whole) + 2 * rest, 512, LDS, stream);
-  return launch(wide_large_kernel<MODE, ACT, 4>, p, together(p.whole) + 4 * rest, 512, LDS, stream);
+  if (parts == 1) return launch(wide_large_kernel<MODE, ACT, 1>, p, together<MODE>(tiles), 512, Large::LDS_BYTES, stream);
+  if (parts == 2) return launch(wide_large_kernel<MODE, ACT, 2>, p, together<MODE>(p.whole) + 2 * rest, 512, LDS, stream);
+  return launch(wide_large_kernel<MODE, ACT, 4>, p, together<MODE>(p.whole) + 4 * rest, 512, LDS, stream);
 }
 
 enum { SHAPE_LARGE, SHAPE_128_256, SHAPE_128_128, SHAPE_128_96, SHAPE_64_128, SHAPE_64_64, SHAPES };

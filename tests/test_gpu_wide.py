@@ -261,17 +261,42 @@ def test_activations_of_every_bfloat16_number(kind):
         assert torch.equal(got.isnan(), exact.isnan()) and got[z == float("inf")] == float("inf")
 
 
-@pytest.mark.parametrize("M,N,mode,ranges", [(2048, 8448, K.WIDE_PLAIN, 1), (2300, 9472, K.WIDE_GATED, 1), (1000, 9216, K.WIDE_SUMS, 4), (4097, 8208, K.WIDE_PLAIN, 1)])
-def test_more_tiles_of_256_than_units(M, N, mode, ranges):
+def run_whole(M, N, ranges=1):
+    """How many tiles of 256 x 256 are run as such: what is left over behind whole rounds of 256 is cut where it is half a round or less."""
+    tiles = -(-M // 256) * -(-N // 256)
+    return tiles * ranges if ranges > 1 or tiles % 256 > 128 else tiles - tiles % 256
+
+
+@pytest.mark.parametrize("M,N,mode,ranges,kind", [
+    (4097, 8208, K.WIDE_PLAIN, 1, None), (2048, 17920, K.WIDE_GATED, 1, "silu"), (2300, 11504, K.WIDE_GATED, 1, "silu"),
+    (2300, 11504, K.WIDE_GATED, 1, "gelu_tanh"), (2300, 11504, K.WIDE_PLAIN, 1, "gelu"), (2100, 11504, K.WIDE_PLAIN, 1, None), (1000, 9216, K.WIDE_SUMS, 4, None)])
+def test_more_tiles_of_256_than_units(M, N, mode, ranges, kind):
     """A workgroup then takes one tile after another: what its first tile gives and its last, with whole tiles, cut ones and ranges of k,
-    is what tiles of 128 x 128 give, bit for bit."""
+    is what tiles of 128 x 128 give, bit for bit; all workgroups two (2,048 rows, gated), or some of them."""
     a, w = operands(M, N, 512, 9)
+    bias = torch.randn(N, device="cuda") if mode == K.WIDE_PLAIN else None
     shape = {K.WIDE_PLAIN: (M, N), K.WIDE_GATED: (M, N // 2), K.WIDE_SUMS: (ranges, M, N)}[mode]
-    kind = "silu" if mode == K.WIDE_GATED else None
     got = [torch.full(shape, float("nan"), device="cuda", dtype=torch.float32 if mode == K.WIDE_SUMS else torch.bfloat16) for _ in range(2)]
     for out, tile in zip(got, (0, 2)):
-        K.gemm_wide(out, a, w, tile | ranges << 8, kind=kind, mode=mode)
-    assert -(-M // 256) * -(-N // 256) * ranges > 256 and torch.equal(*got)
+        K.gemm_wide(out, a, w, tile | ranges << 8, bias, kind=kind, mode=mode)
+    assert run_whole(M, N, ranges) > 256 and torch.equal(*got)
+
+
+def test_more_tiles_of_256_than_units_of_heads():
+    """A workgroup a tile here; queries, keys and values are those of tiles of 128 x 128."""
+    M, nh, nkv, hd, bs = 5408, 28, 4, 128, 16
+    a, w = operands(M, (nh + 2 * nkv) * hd, 256, 3)
+    assert run_whole(M, (nh + 2 * nkv) * hd) > 256
+    positions, tok_seq = torch.arange(M, device="cuda", dtype=torch.int32), torch.zeros(M, device="cuda", dtype=torch.int32)
+    tables = torch.randperm(M // bs, device="cuda").int()[None].contiguous()
+    angles = torch.randn(M, hd // 2, 2, device="cuda")
+    got = []
+    for tile in (0, 2):
+        q = torch.empty(M, nh * hd, device="cuda", dtype=torch.bfloat16)
+        pools = [torch.empty(M // bs, nkv, *s, device="cuda", dtype=torch.bfloat16) for s in ((bs, hd), (hd, bs))]
+        K.gemm_wide_rope(q, a, w, None, tile | 1 << 8, nh, nkv, hd, hd, angles, positions, tok_seq, tables, bs, *pools)
+        got.append((q, *pools))
+    assert all(torch.equal(x, y) for x, y in zip(*got)) and bool(got[0][1].float().isfinite().all())
 
 
 @pytest.mark.parametrize("kind,low,bound", [("silu", -88.0, 3e-7), ("gelu_tanh", -1.0, 3.5e-7), ("gelu", -1.0, 4.5e-7)])
