@@ -144,6 +144,7 @@ int pae_norm_scale_add(int dtype, float* residual, const void* y, int parts, int
                        int w_is_f32, float eps, float scale, void* next, int num_rows, int hidden, hipStream_t stream);
 int pae_activation(int dtype, void* x, int64_t n, int kind, const void* bias, int b_is_f32, int width, hipStream_t stream);
 // the gated delta rule over a step's projected rows: see delta_rule.hip
+int pae_tokens_step_pays(int num_seqs, int G, int H);  // whether a step of single tokens takes one launch, by its sizes
 int pae_delta_rule_step(int dtype, const void* proj, int64_t row_stride, int num_tokens, int num_seqs, const int* tok_seq,
                         const int* positions, const int* seq_runs, const int* slots, const float* conv_w,
                         float* conv_tail, int64_t tail_slot_stride, int taps, int G, int H, int D, int V,

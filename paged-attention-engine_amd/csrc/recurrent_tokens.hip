@@ -12,6 +12,7 @@
 // and 7.9 / 8.7 / 24.1, with channel decays 12.7 / 15.1 / 43.3 and 8.5 / 9.5 / 26.1; 28 heads 12.3 / 21.5 / 73.0 and 8.0 / 10.2 / 48.6; linear attention with 12
 // heads 8.9 / 11.4 / 37.9 and 4.3 / 5.2 / 20.5, 14 heads of 64 8.4 / 8.8 / 17.8 and 3.9 / 4.4 / 13.9.  What is left of the delta rule's 8 us is
 // a chain: the run and its slot, the convolution's inputs, the unit vectors' sums, the state's products, the norm's sum.
+#include "api.h"
 #include "recurrent_tokens.h"
 
 namespace {
@@ -237,13 +238,19 @@ void launch_of(int kind, const TokensStep& p, int num_seqs, hipStream_t stream) 
 
 }  // namespace
 
-// As many tokens as sequences: single tokens (a run of several beside empty ones is worked on token by token here), at any count of them (above:
-// ahead from 1 to 64 sequences).  The other
+// Whether a step of that many single tokens is ahead in one launch.  A workgroup takes the value heads of its key head one after another, 2 us each:
+// always up to four of them, beyond that where workgroups are so many that the units are busy anyway (us, separate kernels and one launch, heads of 128 by
+// 128: 4 key and 16 value heads for 1 / 8 / 64 sequences 12.2 / 16.2 / 49.3 and 11.6 / 12.7 / 26.4; 2 and 16 for 1 / 16 / 32 / 64 12.2 / 21.8 / 33.1 / 48.7 and
+// 19.9 / 21.9 / 29.0 / 34.6; 1 and 16 for 1 / 64 / 128 11.9 / 48.7 / 78.3 and 35.1 / 52.4 / 61.3; 2 and 28 of 64 by 64 for 32 / 64 21.0 / 30.7 and 24.1 / 29.9).
+extern "C" int pae_tokens_step_pays(int num_seqs, int G, int H) { return H <= 4 * G || (int64_t)num_seqs * G * G >= 8 * (int64_t)H; }
+
+// As many tokens as sequences: single tokens (a run of several beside empty ones is worked on token by token here).  The other
 // bounds are what a workgroup holds, lanes of 8 rows by two columns and what the value heads of a key head have in LDS, and that four rows of
 // a column are read at a time.
 bool takes_tokens_step(int num_tokens, int num_seqs, int G, int H, int D, int V, const float* state, int64_t slot_stride) {
   const int lanes = D <= 64 ? 8 : 16;
-  return num_tokens == num_seqs && D % 4 == 0 && slot_stride % 4 == 0 && (uintptr_t)state % 16 == 0 && D > 32 && D <= 128 && V <= COLUMNS * THREADS / lanes && (int64_t)(H / G) * (V + lanes * R) <= MOST_VALUES;
+  return num_tokens == num_seqs && pae_tokens_step_pays(num_seqs, G, H) && D % 4 == 0 && slot_stride % 4 == 0 && (uintptr_t)state % 16 == 0 && D > 32 &&
+         D <= 128 && V <= COLUMNS * THREADS / lanes && (int64_t)(H / G) * (V + lanes * R) <= MOST_VALUES;
 }
 
 void launch_tokens_step(int kind, int dtype, const TokensStep& p, int num_seqs, hipStream_t stream) {

@@ -102,6 +102,7 @@ def _declare(lib) -> None:
         "pae_rows_from_residual": [I, P, P, L, P],
         "pae_norm_scale_add": [I, P, P, I, L, P, I, F, F, P, I, I, P],
         "pae_activation": [I, P, L, I, P, I, I, P],
+        "pae_tokens_step_pays": [I, I, I],
         "pae_delta_rule_step": [I, P, L, I, I, P, P, P, P, P, P, L, I, I, I, I, I, P, P, F, P, L, P, I, F, P, P,
                                 P, L, I, P, L, P, L, I, P],
         "pae_matrix_memory_step": [I, P, L, P, L, P, P, L, P, P, I, I, P, I, P, I, P, I, P, I, I, I, F, P, L, P, L, P, I, F, F, P,

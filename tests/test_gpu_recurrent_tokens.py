@@ -28,7 +28,7 @@ def normal(gen, *shape):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("channel", [False, True])
-@pytest.mark.parametrize("G,H,D,V,taps", [(1, 1, 36, 1, 1), (2, 4, 64, 256, 4), (6, 12, 128, 128, 4), (2, 6, 100, 72, 7), (3, 3, 68, 65, 2), (1, 2, 40, 200, 5)])
+@pytest.mark.parametrize("G,H,D,V,taps", [(1, 1, 36, 1, 1), (2, 4, 64, 256, 4), (6, 12, 128, 128, 4), (2, 6, 100, 72, 7), (3, 3, 68, 65, 2), (1, 2, 40, 200, 5), (2, 8, 64, 40, 3), (1, 5, 36, 16, 4)])
 def test_delta_rule(dtype, channel, G, H, D, V, taps):
     gen = torch.Generator().manual_seed(D + V)
     C = 2 * G * D + H * V

@@ -277,3 +277,12 @@ def test_ranges_of_few_rows_follow_from_the_weights_alone(N, K_):
         assert len(ranges) == 1
         r = ranges.pop()
         assert 1 <= r <= 8 and (r - 1) * (-(-(-(-K_ // r)) // 128) * 128) < K_
+
+
+def test_single_tokens_of_many_value_heads_a_key_head_take_one_launch_only_where_they_are_many():
+    """A workgroup takes a key head's value heads one after another: few sequences of many value heads go by the separate kernels, whose heads run beside
+    each other."""
+    pays = lambda seqs, G, H: bool(K.library().pae_tokens_step_pays(seqs, G, H))
+    assert all(pays(seqs, G, H) for seqs in (1, 8, 1000) for G, H in ((1, 1), (12, 12), (6, 12), (4, 16), (28, 28)))
+    assert not any((pays(1, 1, 16), pays(64, 1, 16), pays(1, 2, 16), pays(8, 2, 16), pays(4, 4, 32), pays(32, 2, 28), pays(8, 1, 8)))
+    assert all((pays(128, 1, 16), pays(32, 2, 16), pays(16, 4, 32), pays(64, 2, 28), pays(64, 1, 8), pays(60000, 1000, 64000)))
