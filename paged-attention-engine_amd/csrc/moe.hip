@@ -122,14 +122,14 @@ extern "C" int pae_project_f32(int dtype, float* out, int64_t ldo, const void* A
   if (M <= 0) return 0;
   const int vec = dtype == PAE_F32 ? 4 : 8;
   const bool wide = K % vec == 0 && lda % vec == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0;
-  // (from where its workgroups are two a unit: 3,001 x 32 x 1,536 23.5 -> 17.5 us, 8,192 54.8 -> 38.6, 2,047 x 24 x 2,048 16.3 -> 12.4; but 1,500 x 33 13.7 and 14.4)
-  if (wide && dtype == PAE_BF16 && M >= 2000 && K <= 4 * 512) {
+  // (from where its workgroups are two a unit, and there are outputs enough for the held rows: 3,001 x 32 x 1,536 20.4 -> 16.0 us, 8,192 49.1 -> 35.0, 2,000 x
+  // 16 x 896 6.5 -> 6.4, x 2,048 10.7 -> 9.1; but 3,001 x 2 x 2,048 3.8 and 5.9, 2,000 x 32 x 256 7.5 and 8.3, 1,500 x 33 x 1,536 13.7 and 14.4)
+  if (wide && dtype == PAE_BF16 && M >= 2000 && N >= 16 && K > 512 && K <= 4 * 512) {
     constexpr int rows = 4;
     const int groups = (M + rows - 1) / rows;
 #define PROJECT_ROWS(STEPS) \
   project_f32_rows_kernel<STEPS, rows><<<groups, 256, 0, stream>>>(out, ldo, (const bf16_t*)A, lda, (const bf16_t*)W, bias, b_is_f32, M, N, K)
-    if (K <= 512) PROJECT_ROWS(1);
-    else if (K <= 1024) PROJECT_ROWS(2);
+    if (K <= 1024) PROJECT_ROWS(2);
     else if (K <= 1536) PROJECT_ROWS(3);
     else PROJECT_ROWS(4);
 #undef PROJECT_ROWS

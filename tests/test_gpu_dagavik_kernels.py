@@ -440,9 +440,11 @@ def test_few_features_summed_in_float32(dtype):
     close(got, a.double() @ w.double().T + bias.double(), 1e-5, "float32 sums")
 
 
-@pytest.mark.parametrize("M,N,width", [(2000, 1, 8), (2003, 33, 512), (2001, 5, 520), (2050, 32, 1536), (2002, 40, 2040), (2000, 3, 2048), (2000, 3, 2056)])
+@pytest.mark.parametrize("M,N,width", [(2000, 1, 8), (2003, 33, 512), (2001, 5, 520), (2003, 17, 520), (2001, 16, 1032), (2050, 32, 1536), (2002, 40, 2040),
+                                       (2000, 19, 2048), (2000, 3, 2048), (2000, 17, 2056)])
 def test_few_features_of_many_rows_have_the_bits_of_few(M, N, width):
-    """From 2,000 rows on a workgroup takes four; below it takes one.  Widths of one to four stretches of 512, whole and ragged, and one wider."""
+    """From 2,000 rows and 16 features on a workgroup takes four rows; below it takes one.  Widths of two to four stretches of 512, whole and ragged, and
+    shorter and wider ones."""
     gen = torch.Generator().manual_seed(width)
     a = torch.randn((M, width + 8), generator=gen).to(torch.bfloat16).to(DEV)[:, :width]
     w, bias = torch.randn((N, width), generator=gen).to(torch.bfloat16).to(DEV), torch.randn(N, generator=gen).to(DEV)
