@@ -11,10 +11,10 @@
 // 160 and 45.6, 177 in one.  What the epilogue adds is the angles' and pages' way and the values' stores of 2 bytes.
 //
 // Measured beside the platform library's product (weights from memory, us; rows x features x k):
-//     2,048 x 17,920 x  1,536   library 111 and 22 for the gate behind it    here with the gate 96
+//     2,048 x 17,920 x  1,536   library 111 and 22 for the gate behind it    here with the gate 101
 //     2,048 x  1,536 x  8,960           71                                   66
 //     2,048 x  2,048 x  1,536           19                                   15
-//     6,030 x 37,888 x  3,584        1,209 and 117 for the gate              1,143 with the gate
+//     6,030 x 37,888 x  3,584        1,209 and 117 for the gate              1,175 with the gate
 //     6,030 x  3,584 x 18,944        1,041                                   600
 //       601 x  1,536 x  8,960           36                                   24 in ranges of k
 //       200 x  1,536 x  1,536           20                                   8
@@ -275,10 +275,12 @@ __device__ __forceinline__ void small_tile(const Product& p, char* lds, int m0, 
 using Half = Tile<128, 256, 2, 4, 3>;     // of a tile of 256 x 256, by the same eight wavefronts
 using Quarter = Tile<128, 128, 2, 4, 4>;
 
-// Whether a workgroup takes one tile of 256 x 256 after another (see below).  Not with rotated heads, whose epilogue has no registers left for it: 28 bytes
-// a lane went to memory and back, and it gained nothing (us, in turns and not: 6,030 x 4,608 x 3,584 165.6 and 165.2, 8,192 x 7,168 x 5,120 427 and 427).
-template <int MODE>
-constexpr bool in_turns() { return MODE != wide_gemm::ROTATED; }
+// Whether a workgroup takes one tile of 256 x 256 after another (see below): where an activation makes the epilogue long.  Without one a workgroup a tile
+// is ahead (us, in turns and not: sums of ranges 6,030 x 1,536 x 8,960 in three 146.7 and 141.7, 2,500 x 2,048 x 11,008 in five 114.0 and 111.9; 2,048 x 37,888 x
+// 3,584 410.8 and 405.4), and the epilogue of rotated heads has no registers left for it, 28 bytes a lane went to memory and back (6,030 x 4,608 x 3,584 165.6
+// and 165.2).  With one: by erf 8,192 x 8,960 x 1,536 211.6 and 217.6.
+template <int MODE, int ACT>
+constexpr bool in_turns() { return ACT != NO_ACT; }
 
 // parts: into how many each tile behind the whole ones is cut (1, 2 or 4)
 template <int MODE, int ACT, int PARTS>
@@ -287,7 +289,7 @@ __global__ __launch_bounds__(512, 2) void wide_large_kernel(Product p) {
   const int lane = threadIdx.x % PAE_WAVE;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PAE_WAVE);
   int tm, tn;
-  const int ranges = MODE == wide_gemm::SUMS ? p.whole * p.splits : p.whole, together = in_turns<MODE>() ? min(ranges, UNITS) : ranges;
+  const int ranges = MODE == wide_gemm::SUMS ? p.whole * p.splits : p.whole, together = in_turns<MODE, ACT>() ? min(ranges, UNITS) : ranges;
   if (PARTS > 1 && (int)blockIdx.x >= together) {
     const int rest = (p.row_tiles * p.col_tiles - p.whole) * PARTS, at = in_row(blockIdx.x - together, rest);
     place_of(p.whole + at / PARTS, p.row_tiles, p.col_tiles, p.strip, tm, tn);
@@ -298,8 +300,8 @@ __global__ __launch_bounds__(512, 2) void wide_large_kernel(Product p) {
   }
   // A unit's workgroup takes one tile after another (the ones that it would be given one by one), and asks for the next one's first stages
   // before it leaves a tile's results: what a tile needs beside its stages, some 11 of 39 us at k 1,536, is the way of its first stage, its epilogue and
-  // a workgroup's start (gated, us, a workgroup a tile and this: 8,192 x 17,920 x 1,536 350 and 338, 2,048 98.7 and 96.4, 8,192 x 22,016 x 2,048 541 and
-  // 527, 8,192 x 9,728 x 896 127 and 117; 6,030 x 37,888 x 3,584 1,149 and 1,143).
+  // a workgroup's start (gated, us, a workgroup a tile and this: 8,192 x 17,920 x 1,536 356 and 349, 6,030 271 and 263, 2,048 102.2 and 100.7, 8,192 x 22,016 x
+  // 2,048 552 and 539, 8,192 x 9,728 x 896 132 and 127; 6,030 x 37,888 x 3,584 1,178 and 1,175).
   Large::Source src;
   int m0, n0, split, stages;
   auto begin = [&](int i) {
@@ -330,8 +332,8 @@ __global__ __launch_bounds__(512, 2) void wide_large_kernel(Product p) {
   };
   begin(blockIdx.x);
   // Stores of a whole tile's results by a wavefront, 16 bytes a lane each and none under a condition then: the next tile's first stage is
-  // waited for and they are not (gated, us, waited for and not: 8,192 x 17,920 x 1,536 338 and 334, 2,048 96.4 and 95.5, 8,192 x 9,728 x 896 117 and 113).
-  constexpr int STORES = MODE == wide_gemm::GATED ? Large::MT : MODE == wide_gemm::SUMS ? Large::MT * Large::X : MODE == wide_gemm::PLAIN ? Large::MT * Large::X / 2 : 0;
+  // waited for and they are not (gated, us, waited for and not, with a SiLU of half the instructions: 8,192 x 17,920 x 1,536 338 and 334, 2,048 96.4 and 95.5, 8,192 x 9,728 x 896 117 and 113).
+  constexpr int STORES = !in_turns<MODE, ACT>() ? 0 : MODE == wide_gemm::GATED ? Large::MT : Large::MT * Large::X / 2;
   bool stored = false;
   for (int i = blockIdx.x; i < ranges; i += together) {
     f32x4 acc[Large::MT][Large::X];
@@ -342,9 +344,9 @@ __global__ __launch_bounds__(512, 2) void wide_large_kernel(Product p) {
     Large::run<STORES>(acc, wide_lds, src, stages, stored);
     stored = m0 + 256 <= p.M && n0 + 256 <= p.N;
     const int row0 = m0 + wave / Large::WN * Large::PM, col0 = n0 + wave % Large::WN * Large::PN, of = split;
-    if (in_turns<MODE>() && i + together < ranges) begin(i + together);
+    if (in_turns<MODE, ACT>() && i + together < ranges) begin(i + together);
     finish<MODE, ACT>(p, acc, row0, col0, of);
-    if (!in_turns<MODE>()) return;
+    if (!in_turns<MODE, ACT>()) return;
   }
 }
 
@@ -382,8 +384,8 @@ int launch_small(Product p, hipStream_t stream) {
 }
 
 // Workgroups of tiles of 256 x 256.
-template <int MODE>
-int64_t together(int64_t tiles) { return in_turns<MODE>() && tiles > UNITS ? UNITS : tiles; }
+template <int MODE, int ACT>
+int64_t together(int64_t tiles) { return in_turns<MODE, ACT>() && tiles > UNITS ? UNITS : tiles; }
 
 template <int MODE, int ACT>
 int launch_large(Product p, hipStream_t stream) {
@@ -395,15 +397,15 @@ int launch_large(Product p, hipStream_t stream) {
   if constexpr (MODE == wide_gemm::SUMS) {
     p.whole = (int)tiles;
     PAE_REQUIRE(tiles * p.splits < (1ll << 30), "wide product: too many tiles");
-    return launch(wide_large_kernel<MODE, ACT, 1>, p, together<MODE>(tiles * p.splits), 512, Large::LDS_BYTES, stream);
+    return launch(wide_large_kernel<MODE, ACT, 1>, p, together<MODE, ACT>(tiles * p.splits), 512, Large::LDS_BYTES, stream);
   }
   const int rest = (int)(tiles % UNITS), parts = rest == 0 || rest > UNITS / 2 ? 1 : rest > UNITS / 4 ? 2 : 4;
   p.whole = (int)(parts == 1 ? tiles : tiles - rest);
   constexpr int LDS = Large::LDS_BYTES > Half::LDS_BYTES ? Large::LDS_BYTES : Half::LDS_BYTES;
   static_assert(Quarter::LDS_BYTES <= LDS, "room for every part");
-  if (parts == 1) return launch(wide_large_kernel<MODE, ACT, 1>, p, together<MODE>(tiles), 512, Large::LDS_BYTES, stream);
-  if (parts == 2) return launch(wide_large_kernel<MODE, ACT, 2>, p, together<MODE>(p.whole) + 2 * rest, 512, LDS, stream);
-  return launch(wide_large_kernel<MODE, ACT, 4>, p, together<MODE>(p.whole) + 4 * rest, 512, LDS, stream);
+  if (parts == 1) return launch(wide_large_kernel<MODE, ACT, 1>, p, together<MODE, ACT>(tiles), 512, Large::LDS_BYTES, stream);
+  if (parts == 2) return launch(wide_large_kernel<MODE, ACT, 2>, p, together<MODE, ACT>(p.whole) + 2 * rest, 512, LDS, stream);
+  return launch(wide_large_kernel<MODE, ACT, 4>, p, together<MODE, ACT>(p.whole) + 4 * rest, 512, LDS, stream);
 }
 
 enum { SHAPE_LARGE, SHAPE_128_256, SHAPE_128_128, SHAPE_128_96, SHAPE_64_128, SHAPE_64_64, SHAPES };
