@@ -18,7 +18,7 @@ struct RowsProduct {
   SkinnyNorm norm;
 };
 
-// M <= 16, or (float32 sums) more: 16 rows a workgroup, shared out over grid.z.
+// M <= 16, or (float32 sums) more: 16 or 8 rows a workgroup, shared out over grid.z.
 int launch_rows(const RowsProduct& p, hipStream_t stream);
 
 // The part of it that takes eight weight rows a workgroup: `side_by_side` k ranges in a workgroup (1, 2 or 4).
