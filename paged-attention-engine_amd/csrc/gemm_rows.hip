@@ -2,13 +2,16 @@
 #include "gemm_rows_kernel.h"
 
 // Whether workgroups take eight weight rows instead of 16: by the rows of W and A that the busiest of the 256 compute units has to take in, which bounds
-// these products.  Eights count for less, 0.85: more of them are under way beside each other.  Us at 4 / 8 / 16 rows, eights and sixteens: 128
-// tiles of 1,536 of k 5.1 / 5.3 / 5.9 and 5.5 / 5.8 / 6.5, 160 of 2,048 6.5 / 7.0 / 7.9 and 6.3 / 6.6 / 7.4, 288 of 3,584 10.4 / 11.2 / 13.8 and 11.2 / 11.9 / 13.7,
-// 448 of 5,120 17.5 / 20.1 / 24.5 and 16.9 / 18.3 / 20.6, 608 of 896 6.5 / 6.9 / 8.0 and 6.9 / 7.1 / 7.9, 1,120 of 1,536 12.3 / 13.8 / 17.6 and 12.6 / 13.2 /
-// 15.0, 1,376 of 2,048 18.1 / 20.4 / 25.1 and 19.6 / 20.4 / 23.6.
-static bool takes_halves(int tiles, int groups) {
+// these products.  Eights count for less, 0.85, as more of them are under way beside each other, 0.75 where all of k is asked for at once in four steps;
+// and with one workgroup a unit and batches of steps (k above 2,048) eights always have more under way.  Measured with the gate at five k from 896 to 3,584
+// by 16 numbers of tiles from 96 to 2,368 and 1 to 16 rows, the rule is 0.2 % behind the faster of the two on average and 8.5 % at worst.  Us at 4 / 8 / 16
+// rows, eights and sixteens: 96 tiles of 1,536 of k 3.9 / 3.9 / 4.1 and 4.0 / 4.1 / 4.7, 192 of 1,536 5.2 / 5.4 / 6.1 and 5.0 / 5.1 / 5.6, 192 of 3,584 7.5 / 7.9 /
+// 9.9 and 7.5 / 7.8 / 11.5, 320 of 3,584 10.1 / 10.6 / 12.6 and 10.9 / 11.1 / 13.9, 512 of 2,048 8.9 / 9.1 / 11.0 and 9.5 / 9.6 / 10.4, 1,120 of 1,536 12.3 /
+// 13.1 / 16.4 and 12.7 / 12.6 / 14.1, 2,368 of 3,584 48.4 / 51.5 / 65.5 and 49.5 / 50.0 / 57.8.
+static bool takes_halves(int tiles, int groups, int K) {
+  if (tiles <= 256 && K > 2048) return true;
   const int64_t of_a = 4 * groups, whole = (tiles + 255) / 256 * (16 + of_a), halves = (2 * (int64_t)tiles + 255) / 256 * (8 + of_a);
-  return 17 * halves <= 20 * whole;
+  return (K > 1536 && K <= 2048 ? 15 : 17) * halves <= 20 * whole;
 }
 
 int launch_rows(const RowsProduct& p, hipStream_t stream) {
@@ -32,7 +35,7 @@ int launch_rows(const RowsProduct& p, hipStream_t stream) {
     }
     return pae_check_launch("gemm_rows (ranges side by side)");
   }
-  if (p.splits == 1 && p.M <= 16 && !whole_tiles && takes_halves(tiles, groups)) {
+  if (p.splits == 1 && p.M <= 16 && !whole_tiles && takes_halves(tiles, groups, p.K)) {
     launch_rows_halves(p, 1, k_per_range, dim3(2 * tiles), stream);
   } else {
     // more than 16 rows are shared out by 16, or by 8 where workgroups are few even so (1,536 x 1,536 at 17 rows 4.65 -> 4.46 us, 896 x 896 3.63 -> 3.24)
