@@ -347,7 +347,6 @@ extern "C" int pae_add_rmsnorm(int dtype, void* residual, const void* delta, int
       RMS_PARTS(T, 5) RMS_PARTS(T, 6) RMS_PARTS(T, 7) RMS_PARTS(T, 8)                                         \
     }                                                                                                         \
   } else if (vec)                                                                                             \
-                                                                                                    \
     add_rmsnorm_vec_kernel<T><<<num_rows, threads, 0, stream>>>((float*)residual, delta, parts, part_stride,  \
                                                                 weight, w_is_f32, eps, rows, (T*)out, hidden, \
                                                                 write_residual);                              \

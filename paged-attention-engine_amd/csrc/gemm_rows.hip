@@ -2,7 +2,7 @@
 #include "gemm_rows_kernel.h"
 
 // Whether workgroups take eight weight rows instead of 16: by the rows of W and A that the busiest of the 256 compute units has to take in, which bounds
-// these products.  Eights count for less, 0.85, as more of them are under way beside each other, 0.75 where all of k is asked for at once in four steps;
+// these products.  Eights count for less, 0.85, as more of them are under way beside each other, 0.75 where all of k is asked for at once in four steps and units have two or more;
 // and with one workgroup a unit and batches of steps (k above 2,048) eights always have more under way.  Measured with the gate at five k from 896 to 3,584
 // by 16 numbers of tiles from 96 to 2,368 and 1 to 16 rows, the rule is 0.2 % behind the faster of the two on average and 8.5 % at worst.  Us at 4 / 8 / 16
 // rows, eights and sixteens: 96 tiles of 1,536 of k 3.9 / 3.9 / 4.1 and 4.0 / 4.1 / 4.7, 192 of 1,536 5.2 / 5.4 / 6.1 and 5.0 / 5.1 / 5.6, 192 of 3,584 7.5 / 7.9 /
@@ -11,7 +11,7 @@
 static bool takes_halves(int tiles, int groups, int K) {
   if (tiles <= 256 && K > 2048) return true;
   const int64_t of_a = 4 * groups, whole = (tiles + 255) / 256 * (16 + of_a), halves = (2 * (int64_t)tiles + 255) / 256 * (8 + of_a);
-  return (K > 1536 && K <= 2048 ? 15 : 17) * halves <= 20 * whole;
+  return (K > 1536 && K <= 2048 && tiles > 192 ? 15 : 17) * halves <= 20 * whole;
 }
 
 int launch_rows(const RowsProduct& p, hipStream_t stream) {

@@ -840,8 +840,8 @@ __global__ __launch_bounds__(256) void moe_few_tiles_kernel(bf16_t* __restrict__
 // one workgroup's features after another 594 and 298 us; four wavefronts of 64 x 128 through LDS 382 and 172; with an expert's
 // tiles side by side on one die 318 and 140 (three quarters of the lines from L2); with the loads spread among
 // the products 306 and 127 us (540 and 650 TFLOP/s); eight wavefronts of 64 x 64, two a
-// SIMD, 243 and 121 us (680 TFLOP/s both); the activation as an argument of the template, and worked out as act_to does, both products 384 -> 354 us
-// (373 with its code looked at for every number).
+// SIMD, 243 and 121 us (680 TFLOP/s both); the activation as an argument of the template, and worked out as act_to does, both products 384 -> 359 us
+// (378 with its code looked at for every number).
 typedef wide_gemm::Tile<128, 256, 2, 4, 3> MoeTile;
 #define MOE_BIG_ROWS MoeTile::BM
 #define MOE_BIG_K wide_gemm::BK
